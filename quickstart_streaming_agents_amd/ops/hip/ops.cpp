@@ -94,7 +94,9 @@ extern "C" void qsa_hash_build_launch(const long long*, const long long*,
 extern "C" void qsa_hash_probe_launch(const long long*,
                                       const unsigned long long*,
                                       const unsigned long long*, int*, int,
-                                      unsigned int, long long, hipStream_t);
+                                      unsigned int, long long, int,
+                                      hipStream_t);
+extern "C" int qsa_topk_block_docs(long long);
 extern "C" void qsa_topk_launch(const float*, const float*, float*, int*,
                                 float*, int*, int, int, int, int, int,
                                 hipStream_t);
@@ -457,13 +459,15 @@ std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
   const int Q = queries.size(0), D = queries.size(1), N = docs.size(0);
   TORCH_CHECK(docs.size(1) == D, "dim mismatch");
   TORCH_CHECK(k >= 1 && k <= 16, "k in [1,16]");
-  const int nblk = std::max(1, (N + 2047) / 2048);
+  const int per = qsa_topk_block_docs(N);
+  const int nblk = std::max(1, (N + per - 1) / per);
   auto opts_f = queries.options();
   auto opts_i = queries.options().dtype(at::kInt);
   auto cand_s = torch::empty({Q, nblk, k}, opts_f);
   auto cand_i = torch::empty({Q, nblk, k}, opts_i);
   auto out_s = torch::empty({Q, k}, opts_f);
   auto out_i = torch::empty({Q, k}, opts_i);
+  if (Q == 0) return {out_s, out_i};
   qsa_topk_launch(queries.data_ptr<float>(), docs.data_ptr<float>(),
                   cand_s.data_ptr<float>(), cand_i.data_ptr<int>(),
                   out_s.data_ptr<float>(), out_i.data_ptr<int>(), Q, N, D,

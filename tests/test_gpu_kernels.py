@@ -151,6 +151,35 @@ def test_topk_cosine(ext):
     assert torch.equal(i.cpu(), ri)
 
 
+@pytest.mark.parametrize("Q,N,D,k", [
+    (1, 1, 4, 1), (3, 2, 30, 5), (1, 15, 33, 16), (16, 17, 64, 3),
+    (17, 65, 36, 4), (2, 1000, 1536, 10), (5, 32_767, 40, 16),
+    (9, 32_768, 28, 3), (16, 32_801, 31, 1), (33, 70_001, 32, 2)])
+def test_topk_cosine_edges(ext, Q, N, D, k):
+    """Small whole numbers: every score is exact, so scores, documents and the
+    order of equal scores (ascending document) are pinned without tolerance.
+    Scores of -2 and less are never reported."""
+    g = torch.Generator().manual_seed(Q * 1000 + N + D)
+    docs = torch.randint(-2, 3, (N, D), generator=g).float()
+    qs = torch.randint(-2, 3, (Q, D), generator=g).float()
+    if N > 3:
+        docs[2] = float("nan")
+        docs[3] = torch.where(qs[0] >= 0, 1.0, -1.0) * float("inf")
+    s, i = ext.topk_cosine(qs.to(dev()), docs.to(dev()), k)
+    full = (qs.double() @ docs.double().T).nan_to_num(
+        -9e9, float("inf"), -9e9)        # an infinite score comes first
+    order = torch.sort(full, dim=1, descending=True, stable=True)[1][:, :k]
+    want_s = torch.full((Q, k), -2.0)
+    want_i = torch.full((Q, k), -1, dtype=torch.int32)
+    top = full.gather(1, order)
+    ok = top > -2
+    m = order.shape[1]
+    want_s[:, :m][ok] = top[ok].float()
+    want_i[:, :m][ok] = order[ok].int()
+    assert torch.equal(s.cpu(), want_s)
+    assert torch.equal(i.cpu(), want_i)
+
+
 def test_window_agg(ext):
     torch.manual_seed(6)
     n, nkeys, nwin = 50000, 7, 288
