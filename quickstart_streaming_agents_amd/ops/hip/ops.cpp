@@ -88,7 +88,6 @@ extern "C" void qsa_gemm_fp8_batch_launch(const unsigned short*,
                                           float*, int, int, long long,
                                           long long, int, hipStream_t);
 extern "C" void qsa_hash_build_launch(const long long*, const long long*,
-                                      unsigned long long*,
                                       unsigned long long*, int, unsigned int,
                                       hipStream_t);
 extern "C" void qsa_hash_probe_launch(const long long*,
@@ -102,8 +101,9 @@ extern "C" void qsa_topk_launch(const float*, const float*, float*, int*,
                                 hipStream_t);
 extern "C" void qsa_window_agg_launch(const long long*, const int*,
                                       const float*, int*, float*, long long,
-                                      long long, int, long long, int,
+                                      long long, int, int, long long, int*,
                                       hipStream_t);
+extern "C" long long qsa_window_workspace(long long);
 void register_avro(pybind11::module_&);  // avro_codec.cpp
 extern "C" void qsa_anomaly_batch_launch(const float*, const int*, float*,
                                          float*, int*, int, int, int,
@@ -389,15 +389,13 @@ std::vector<torch::Tensor> hash_build(torch::Tensor keys,
   TORCH_CHECK(n < (1 << 24), "hash_build: <= 2^24 rows per batch");
   long long cap = 64;
   while (cap < 2 * n) cap <<= 1;
-  auto opts = keys.options();
-  auto tkeys = torch::full({cap}, -1, opts);   // all-ones bits == EMPTY
-  auto tpay = torch::zeros({cap}, opts);
+  // slots of (key, payload) pairs, handed out as two strided views
+  auto slots = torch::empty({cap, 2}, keys.options());
   qsa_hash_build_launch((const long long*)keys.data_ptr<int64_t>(),
                         (const long long*)ts.data_ptr<int64_t>(),
-                        (unsigned long long*)tkeys.data_ptr<int64_t>(),
-                        (unsigned long long*)tpay.data_ptr<int64_t>(),
+                        (unsigned long long*)slots.data_ptr<int64_t>(),
                         (int)n, (unsigned int)(cap - 1), cur_stream());
-  return {tkeys, tpay};
+  return {slots.select(1, 0), slots.select(1, 1)};
 }
 
 torch::Tensor hash_probe(torch::Tensor tkeys, torch::Tensor tpay,
@@ -409,11 +407,20 @@ torch::Tensor hash_probe(torch::Tensor tkeys, torch::Tensor tpay,
   const long long cap = tkeys.numel();
   TORCH_CHECK((cap & (cap - 1)) == 0, "table capacity must be pow2");
   auto out = torch::empty({m}, keys.options().dtype(torch::kInt32));
+  const int64_t* words = tkeys.data_ptr<int64_t>();
+  const bool paired = tkeys.stride(0) == 2 && tpay.stride(0) == 2 &&
+                      tpay.data_ptr<int64_t>() == words + 1 &&
+                      (reinterpret_cast<uintptr_t>(words) & 15) == 0;
+  if (!paired) {
+    tkeys = tkeys.contiguous();
+    tpay = tpay.contiguous();
+  }
   qsa_hash_probe_launch((const long long*)keys.data_ptr<int64_t>(),
                         (const unsigned long long*)tkeys.data_ptr<int64_t>(),
                         (const unsigned long long*)tpay.data_ptr<int64_t>(),
                         out.data_ptr<int>(), (int)m,
-                        (unsigned int)(cap - 1), min_ts, cur_stream());
+                        (unsigned int)(cap - 1), min_ts, paired,
+                        cur_stream());
   return out;
 }
 
@@ -482,18 +489,26 @@ std::vector<torch::Tensor> window_agg(torch::Tensor ts, torch::Tensor key,
   CHK_DEV(ts); CHK_CONT(ts); CHK_I32(key);
   TORCH_CHECK(ts.scalar_type() == at::kLong, "ts must be i64");
   const long long n = ts.numel();
-  auto counts = torch::zeros({nkeys, nwin}, key.options());
-  auto sums = torch::zeros({nkeys, nwin}, ts.options().dtype(at::kFloat));
+  // one buffer: the two tables are cleared by one fill
+  auto cells = torch::zeros({2, nkeys, nwin}, key.options());
+  auto counts = cells[0];
+  auto sums = cells[1].view(at::kFloat);
   const float* vptr = nullptr;
   if (value.has_value()) {
     CHK_F32(value.value());
     vptr = value.value().data_ptr<float>();
   }
-  const int blocks = (int)std::min<long long>((n + 255) / 256, 4096);
+  const long long words = qsa_window_workspace(n);
+  torch::Tensor ws;
+  int* wptr = nullptr;
+  if (words) {
+    ws = torch::empty({words}, key.options());
+    wptr = ws.data_ptr<int>();
+  }
   qsa_window_agg_launch(reinterpret_cast<const long long*>(ts.data_ptr<int64_t>()),
                         key.data_ptr<int>(), vptr,
                         counts.data_ptr<int>(), sums.data_ptr<float>(), t0,
-                        win_ms, (int)nwin, n, std::max(blocks, 1),
+                        win_ms, (int)nwin, (int)nkeys, n, wptr,
                         cur_stream());
   return {counts, sums};
 }

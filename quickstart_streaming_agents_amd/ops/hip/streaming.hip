@@ -1,25 +1,178 @@
 // Streaming-analytics kernels: batched windowed aggregation (K7) and the
 // batched per-key AR anomaly scorer (K3).
+#include <algorithm>
+
 #include "common.h"
 
 // ---------------------------------------------------------------------------
 // Windowed aggregation: segmented count/sum by (key, window) over an event
 // batch.  window = (ts - t0) / win_ms; out slot = key * nwin + window.
 // The reference shape: TUMBLE(...) GROUP BY key (LAB3:99-133, LAB4:127-141).
+//
+// Bound by atomics, not bytes: those of different dies meet behind the L2s, at
+// some 12 G/s whether they collide or not (two per event: 307 us for 2M
+// events, 1000 keys, 288 windows; one pair per touched cell of a 4096-event
+// chunk: 81 us).  So blocks count CHUNKS of consecutive events, which in a
+// stream span a few windows, in LDS and leave (windows spanned) * nkeys cells
+// in a workspace; qsa_window_merge adds them up, without atomics and in a fixed
+// order (42 us together).  A chunk whose span does not fit goes to the output
+// with atomics, as do batches of a few chunks, where a second launch costs
+// more than their cells.
 // ---------------------------------------------------------------------------
+#define QSA_AGG_CELLS 6144             // 48 KiB of LDS: three blocks per CU
+#define QSA_AGG_CHUNK 4096
+#define QSA_AGG_BLOCKS 2048            // most chunks, 96 MiB of workspace
+#define QSA_AGG_DIRECT 16              // chunks that need no workspace
+
+__device__ __forceinline__ int qsa_window_of(long long ts, long long t0,
+                                             long long win_ms, int nwin) {
+  const long long w = (ts - t0) / win_ms;
+  return w >= 0 && w < nwin ? (int)w : -1;
+}
+
 __global__ void __launch_bounds__(256)
 qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
                const float* __restrict__ value,  // nullptr -> count only
                int* __restrict__ counts, float* __restrict__ sums,
-               long long t0, long long win_ms, int nwin, long long n) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) {
-    const long long w = (ts[i] - t0) / win_ms;
-    if (w < 0 || w >= nwin) continue;
-    const long long slot = (long long)key[i] * nwin + w;
-    atomicAdd(counts + slot, 1);
-    if (value && sums) atomicAdd(sums + slot, value[i]);
+               long long t0, long long win_ms, int nwin, int nkeys,
+               long long n, long long chunk,
+               int2* __restrict__ span,          // [blocks] {first, windows}
+               int* __restrict__ ws) {           // [blocks, 2, CELLS] or null
+  __shared__ int cnt[QSA_AGG_CELLS];
+  __shared__ float sum[QSA_AGG_CELLS];
+  __shared__ int lo_s, hi_s;
+  const int tid = threadIdx.x;
+  const long long first = (long long)blockIdx.x * chunk;
+  const long long end = min(first + chunk, n);
+  if (tid == 0) {
+    lo_s = 0x7fffffff;
+    hi_s = -1;
+  }
+  __syncthreads();
+  int lo = 0x7fffffff, hi = -1;
+#pragma unroll 4
+  for (long long i = first + tid; i < end; i += 256) {
+    const int w = qsa_window_of(ts[i], t0, win_ms, nwin);
+    if (w >= 0) {
+      lo = min(lo, w);
+      hi = max(hi, w);
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    lo = min(lo, __shfl_xor(lo, o, QSA_WAVE));
+    hi = max(hi, __shfl_xor(hi, o, QSA_WAVE));
+  }
+  if ((tid & 63) == 0) {
+    atomicMin(&lo_s, lo);
+    atomicMax(&hi_s, hi);
+  }
+  __syncthreads();
+  lo = lo_s;
+  hi = hi_s;
+  const long long cells = hi < 0 ? 0 : (long long)(hi - lo + 1) * nkeys;
+  const bool local = cells <= QSA_AGG_CELLS;     // uniform over the block
+  if (ws && tid == 0)
+    span[blockIdx.x] = make_int2(lo, local && hi >= 0 ? hi - lo + 1 : 0);
+  if (cells == 0) return;              // no event of the chunk counts
+  if (local) {
+    for (int c = tid; c < (int)cells; c += 256) {
+      cnt[c] = 0;
+      sum[c] = 0.f;
+    }
+    __syncthreads();
+  }
+#pragma unroll 4
+  for (long long i = first + tid; i < end; i += 256) {
+    const int w = qsa_window_of(ts[i], t0, win_ms, nwin);
+    const int kk = key[i];
+    const float v = value ? value[i] : 0.f;
+    if (w < 0 || kk < 0 || kk >= nkeys) continue;
+    if (local) {
+      const int c = (w - lo) * nkeys + kk;
+      atomicAdd(cnt + c, 1);
+      if (value) unsafeAtomicAdd(sum + c, v);
+    } else {
+      const long long slot = (long long)kk * nwin + w;
+      atomicAdd(counts + slot, 1);
+      if (value) unsafeAtomicAdd(sums + slot, v);
+    }
+  }
+  if (!local) return;
+  __syncthreads();
+  if (ws) {
+    int* wc = ws + (long long)blockIdx.x * 2 * QSA_AGG_CELLS;
+    float* wf = reinterpret_cast<float*>(wc + QSA_AGG_CELLS);
+    for (int c = tid; c < (int)cells; c += 256) {
+      wc[c] = cnt[c];
+      if (value) wf[c] = sum[c];
+    }
+    return;
+  }
+  for (int c = tid; c < (int)cells; c += 256) {
+    if (cnt[c] == 0) continue;
+    const long long slot = (long long)(c % nkeys) * nwin + lo + c / nkeys;
+    atomicAdd(counts + slot, cnt[c]);
+    if (value) unsafeAtomicAdd(sums + slot, sum[c]);
+  }
+}
+
+// Block = 8 windows x 64 keys, a wave per two windows: the chunks that reach
+// these windows, in order, added to what other chunks left in the output.
+__global__ void __launch_bounds__(256)
+qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
+                 int blocks, int* __restrict__ counts,
+                 float* __restrict__ sums, int has_value, int nwin,
+                 int nkeys) {
+  __shared__ int list[QSA_AGG_BLOCKS];
+  __shared__ int2 range[QSA_AGG_BLOCKS];
+  __shared__ int wave_n[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int w0 = blockIdx.x * 8, k = blockIdx.y * 64 + lane;
+  int total = 0;
+  for (int base = 0; base < blocks; base += 256) {
+    const int b = base + tid;
+    const int2 s = b < blocks ? span[b] : make_int2(0, 0);
+    const bool in = s.y > 0 && s.x < w0 + 8 && s.x + s.y > w0;
+    const unsigned long long m = __ballot(in);
+    if (lane == 0) wave_n[wave] = __popcll(m);
+    __syncthreads();
+    int at = total + __popcll(m & ((1ull << lane) - 1));
+    for (int w = 0; w < 4; ++w) {
+      if (w < wave) at += wave_n[w];
+      total += wave_n[w];
+    }
+    if (in) {
+      list[at] = b;
+      range[at] = s;
+    }
+    __syncthreads();
+  }
+  const bool live = k < nkeys;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int w = w0 + wave * 2 + u;
+    int c = 0;
+    float v = 0.f;
+#pragma unroll 4
+    for (int j = 0; j < total; ++j) {
+      const int2 s = range[j];
+      const bool in = live && w >= s.x && w < s.x + s.y;
+      // outside its span a chunk lends its first cell, which counts for none
+      const int* p = ws + (long long)list[j] * 2 * QSA_AGG_CELLS +
+                     (in ? (w - s.x) * nkeys + k : 0);
+      const int pc = *p;
+      c += in ? pc : 0;
+      if (has_value) {
+        const float pv = __int_as_float(p[QSA_AGG_CELLS]);
+        v += in ? pv : 0.f;
+      }
+    }
+    if (live && w < nwin) {
+      const long long slot = (long long)k * nwin + w;
+      counts[slot] += c;
+      if (has_value) sums[slot] += v;
+    }
   }
 }
 
@@ -28,6 +181,11 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
 // Mirrors runtime/anomaly.py ar_forecast(): centered lag design, ridge
 // lambda = 0.3 * tr(G)/p, prediction se with leverage.  p <= 4.
 // series: [K, Tmax] f32 (ragged via lengths[]); outputs per key.
+//
+// Bound by latency: three passes over a series that L1 holds after the first.
+// All lanes share every pass and solve the padded 4x4 system in registers
+// (rows beyond p are the identity).  1000 series of 288: 171 us with the
+// solve and the residuals on one lane, 11 us here.
 // ---------------------------------------------------------------------------
 #define QSA_AR_MAXP 4
 
@@ -109,61 +267,66 @@ qsa_anomaly_batch(const float* __restrict__ series, const int* __restrict__ leng
     for (int c = 0; c < QSA_AR_MAXP; ++c) G[a][c] = wave_reduce_sum(G[a][c]);
   }
 
-  // lane 0: ridge solve (G + lam I) coef = b, Gauss-Jordan on p<=4;
-  // also invert for the leverage term.
-  if (lane == 0) {
-    float tr = 0.f;
-    for (int a = 0; a < p; ++a) tr += G[a][a];
-    const float lam = 0.3f * (tr / p + 1e-12f);
-    // augmented [A | I | b]
-    float A[QSA_AR_MAXP][2 * QSA_AR_MAXP + 1];
-    for (int a = 0; a < p; ++a) {
-      for (int c = 0; c < p; ++c) A[a][c] = G[a][c] + (a == c ? lam : 0.f);
-      for (int c = 0; c < p; ++c) A[a][p + c] = (a == c) ? 1.f : 0.f;
-      A[a][2 * p] = bb[a];
-    }
-    for (int col = 0; col < p; ++col) {
-      // partial pivot
-      int piv = col;
-      for (int rr2 = col + 1; rr2 < p; ++rr2)
-        if (fabsf(A[rr2][col]) > fabsf(A[piv][col])) piv = rr2;
-      if (piv != col)
-        for (int c = 0; c <= 2 * p; ++c) {
-          float tmp = A[col][c]; A[col][c] = A[piv][c]; A[piv][c] = tmp;
-        }
-      const float d = A[col][col];
-      const float dinv = (fabsf(d) > 1e-30f) ? 1.f / d : 0.f;
-      for (int c = 0; c <= 2 * p; ++c) A[col][c] *= dinv;
-      for (int rr2 = 0; rr2 < p; ++rr2) {
-        if (rr2 == col) continue;
-        const float f = A[rr2][col];
-        for (int c = 0; c <= 2 * p; ++c) A[rr2][c] -= f * A[col][c];
+  // ridge solve (G + lam I) [coef | y] = [b | x_next] by Gauss-Jordan, every
+  // lane the same; x_next' y is the leverage of the newest lags
+  float tr = 0.f;
+#pragma unroll
+  for (int a = 0; a < QSA_AR_MAXP; ++a) tr += G[a][a];   // 0 beyond p
+  const float lam = 0.3f * (tr / p + 1e-12f);
+  constexpr int W = QSA_AR_MAXP + 2;
+  float A[QSA_AR_MAXP][W], xn[QSA_AR_MAXP];
+#pragma unroll
+  for (int a = 0; a < QSA_AR_MAXP; ++a) {
+    xn[a] = a < p ? h[n - 1 - a] - xm[a] : 0.f;
+#pragma unroll
+    for (int c = 0; c < QSA_AR_MAXP; ++c)
+      A[a][c] = G[a][c] + (a == c ? (a < p ? lam : 1.f) : 0.f);
+    A[a][QSA_AR_MAXP] = bb[a];
+    A[a][QSA_AR_MAXP + 1] = xn[a];
+  }
+#pragma unroll
+  for (int col = 0; col < QSA_AR_MAXP; ++col) {
+#pragma unroll
+    for (int row = col + 1; row < QSA_AR_MAXP; ++row) {
+      const bool swap = fabsf(A[row][col]) > fabsf(A[col][col]);
+#pragma unroll
+      for (int c = 0; c < W; ++c) {
+        const float u = A[col][c], v = A[row][c];
+        A[col][c] = swap ? v : u;
+        A[row][c] = swap ? u : v;
       }
     }
-    float coef[QSA_AR_MAXP];
-    for (int a = 0; a < p; ++a) coef[a] = A[a][2 * p];
-    // residual variance: (yc'yc - 2 coef'b + coef'G coef) / dof
-    // recompute yc'yc quickly (lane 0 serial over n-p; n <= 7000 ok)
-    float yy = 0.f;
-    for (int t = p; t < n; ++t) {
-      const float yc = h[t] - ym;
-      float pred = 0.f;
-      for (int j = 0; j < p; ++j) pred = fmaf(coef[j], h[t - 1 - j] - xm[j], pred);
-      const float r = yc - pred;
-      yy = fmaf(r, r, yy);
+    const float d = A[col][col];
+    const float dinv = (fabsf(d) > 1e-30f) ? 1.f / d : 0.f;
+#pragma unroll
+    for (int c = 0; c < W; ++c) A[col][c] *= dinv;
+#pragma unroll
+    for (int row = 0; row < QSA_AR_MAXP; ++row) {
+      if (row == col) continue;
+      const float f = A[row][col];
+#pragma unroll
+      for (int c = 0; c < W; ++c) A[row][c] -= f * A[col][c];
     }
+  }
+  float rr = 0.f;                      // residual sum of squares
+#pragma unroll 4
+  for (int t = p + lane; t < n; t += QSA_WAVE) {
+    float pred = 0.f;
+#pragma unroll
+    for (int j = 0; j < QSA_AR_MAXP; ++j)
+      if (j < p) pred = fmaf(A[j][QSA_AR_MAXP], h[t - 1 - j] - xm[j], pred);
+    const float r = h[t] - ym - pred;
+    rr = fmaf(r, r, rr);
+  }
+  rr = wave_reduce_sum(rr);
+  if (lane == 0) {
     const int dof = max(m - (p + 1), 1);
-    const float resid_var = yy / dof;
-    // x_next, leverage via inverse block
-    float xn[QSA_AR_MAXP];
-    for (int j = 0; j < p; ++j) xn[j] = h[n - 1 - j] - xm[j];
-    float fc = ym;
-    for (int j = 0; j < p; ++j) fc = fmaf(coef[j], xn[j], fc);
-    float lever = 1.f / m;
-    for (int a = 0; a < p; ++a) {
-      float tmp = 0.f;
-      for (int c = 0; c < p; ++c) tmp = fmaf(A[a][p + c], xn[c], tmp);
-      lever = fmaf(xn[a], tmp, lever);
+    const float resid_var = rr / dof;
+    float fc = ym, lever = 1.f / m;
+#pragma unroll
+    for (int j = 0; j < QSA_AR_MAXP; ++j) {
+      fc = fmaf(A[j][QSA_AR_MAXP], xn[j], fc);
+      lever = fmaf(A[j][QSA_AR_MAXP + 1], xn[j], lever);
     }
     forecast[kidx] = fc;
     pred_se[kidx] =
@@ -173,13 +336,37 @@ qsa_anomaly_batch(const float* __restrict__ series, const int* __restrict__ leng
   }
 }
 
+extern "C" long long qsa_window_chunk(long long n) {
+  return std::max<long long>(
+      QSA_AGG_CHUNK, (n + QSA_AGG_BLOCKS - 1) / QSA_AGG_BLOCKS);
+}
+
+// words of workspace for n events, 0 for none
+extern "C" long long qsa_window_workspace(long long n) {
+  const long long chunk = qsa_window_chunk(n), blocks = (n + chunk - 1) / chunk;
+  return blocks <= QSA_AGG_DIRECT ? 0 : blocks * (2 + 2 * QSA_AGG_CELLS);
+}
+
 extern "C" void qsa_window_agg_launch(const long long* ts, const int* key,
                                       const float* value, int* counts,
                                       float* sums, long long t0,
-                                      long long win_ms, int nwin, long long n,
-                                      int blocks, hipStream_t stream) {
+                                      long long win_ms, int nwin, int nkeys,
+                                      long long n, int* ws,
+                                      hipStream_t stream) {
+  if (n == 0 || nwin <= 0 || nkeys <= 0) return;
+  // without a workspace, short chunks: a few thousand events on as many CUs
+  const long long chunk = ws ? qsa_window_chunk(n) : 256;
+  const int blocks = (int)((n + chunk - 1) / chunk);
+  int2* span = reinterpret_cast<int2*>(ws);
+  int* cells = ws ? ws + 2 * blocks : nullptr;
   hipLaunchKernelGGL(qsa_window_agg, dim3(blocks), dim3(256), 0, stream, ts,
-                     key, value, counts, sums, t0, win_ms, nwin, n);
+                     key, value, counts, sums, t0, win_ms, nwin, nkeys, n,
+                     chunk, span, cells);
+  if (ws)
+    hipLaunchKernelGGL(qsa_window_merge,
+                       dim3((nwin + 7) / 8, (nkeys + 63) / 64), dim3(256), 0,
+                       stream, span, cells, blocks, counts, sums,
+                       value ? 1 : 0, nwin, nkeys);
 }
 
 extern "C" void qsa_anomaly_batch_launch(const float* series,

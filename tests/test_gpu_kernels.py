@@ -194,6 +194,69 @@ def test_window_agg(ext):
     torch.testing.assert_close(sums.cpu(), rs, atol=1e-1, rtol=1e-4)
 
 
+@pytest.mark.parametrize("n,nkeys,nwin,shuffle", [
+    (1, 1, 1, False), (255, 3, 2, True), (257, 6144, 1, False),
+    (5000, 6145, 2, False),              # one key more than a block's cells
+    (140_000, 40, 300, False), (140_000, 40, 300, True),
+    (300_001, 1000, 7, False)])
+def test_window_agg_edges(ext, n, nkeys, nwin, shuffle):
+    """Chunks counted in LDS and chunks that go to memory directly; events
+    before and behind the windows.  Whole values: sums are exact."""
+    g = torch.Generator().manual_seed(n)
+    win, t0 = 1000, 5000
+    ts = torch.randint(t0 - 2 * win, t0 + (nwin + 1) * win, (n,), generator=g)
+    if not shuffle:
+        ts = ts.sort()[0]
+    key = torch.randint(0, nkeys, (n,), generator=g, dtype=torch.int32)
+    val = torch.randint(-8, 9, (n,), generator=g).float()
+    w = torch.div(ts - t0, win, rounding_mode="trunc")
+    ok = (w >= 0) & (w < nwin)
+    at = (key.long() * nwin + w)[ok]
+    counts = torch.zeros(nkeys * nwin, dtype=torch.int32).index_add_(
+        0, at, torch.ones_like(at, dtype=torch.int32)).view(nkeys, nwin)
+    sums = torch.zeros(nkeys * nwin).index_add_(0, at, val[ok]) \
+        .view(nkeys, nwin)
+    args = (t0, win, nwin, nkeys)
+    c, s = ext.window_agg(ts.to(dev()), key.to(dev()), val.to(dev()), *args)
+    assert torch.equal(c.cpu(), counts) and torch.equal(s.cpu(), sums)
+    c, s = ext.window_agg(ts.to(dev()), key.to(dev()), None, *args)
+    assert torch.equal(c.cpu(), counts) and not s.any()
+
+
+@pytest.mark.parametrize("n", [1, 5, 6, 9, 12, 20, 63, 64, 69, 288, 7000])
+def test_anomaly_batch_lengths(ext, n):
+    """Every order of the fit (0 to 4 lags) at lengths around the wave."""
+    from quickstart_streaming_agents_amd.runtime.anomaly import ar_forecast
+    rng = np.random.default_rng(n)
+    x = rng.normal(100, 10, (5, n + 3)).astype(np.float32)
+    x[:, n:] = 1e9                       # beyond the length: never read
+    fc, se, dof = ext.anomaly_batch(
+        torch.from_numpy(x).to(dev()),
+        torch.full((5,), n, dtype=torch.int32, device=dev()), 4)
+    for i in range(5):
+        f, e, d = ar_forecast(x[i, :n].astype(np.float64), 4)
+        # f32 sums over n values about 100: the centred products keep 5 digits
+        assert abs(float(fc[i]) - f) < 1e-3 * abs(f)
+        assert abs(float(se[i]) - e) < 2e-3 * e
+        assert int(dof[i]) == d
+
+
+def test_hash_table_as_two_arrays(ext):
+    """A table's words may be kept as separate arrays."""
+    keys = torch.arange(1000, dtype=torch.int64, device=dev()) * 7919
+    ts = torch.arange(1000, dtype=torch.int64, device=dev()) - 5
+    k, p = ext.hash_build(keys, ts)
+    probe = torch.cat([keys.flip(0), keys + 1])
+    for cut in (-1, 3, 1 << 50):
+        rows = ext.hash_probe(k, p, probe, cut)
+        assert torch.equal(rows, ext.hash_probe(k.clone(), p.clone(), probe,
+                                                cut))
+        want = torch.where(ts.clamp(min=0) >= cut,
+                           torch.arange(1000, device=dev()), -1).flip(0)
+        assert torch.equal(rows[:1000].long(), want)
+        assert (rows[1000:] == -1).all()
+
+
 def test_anomaly_batch_matches_cpu(ext):
     from quickstart_streaming_agents_amd.runtime.anomaly import ar_forecast
     rng = np.random.default_rng(0)
