@@ -200,13 +200,13 @@ def bench_kernels(reps: int = 8) -> None:
         bt = torch.arange(n_seq * np_, device=dev, dtype=torch.int32) \
             .view(n_seq, np_).contiguous()
         q3 = q.view(T, H, Dm)
-        item16 = i.repeat_interleave(n // 16).contiguous()
-        t16 = (torch.arange(n // 16, device=dev, dtype=torch.int32) * 16) \
+        item32 = i.repeat_interleave(n // 32).contiguous()
+        t32 = (torch.arange(n // 32, device=dev, dtype=torch.int32) * 32) \
             .repeat(n_seq).contiguous()
         _report("llama paged_attn_prefill", _graph_time([
-            lambda: ext().paged_attn_prefill(q3, kc, vc, bt, item16, t16,
+            lambda: ext().paged_attn_prefill(q3, kc, vc, bt, item32, t32,
                                              i * n, zero, lens, 0.1,
-                                             True)] * 2),
+                                             True, 32)] * 2),
             T * (2 * H + 2 * KVH) * Dm * 2, 4.0 * pairs * H * Dm,
             shape=[n_seq, n, H, KVH, Dm])
 

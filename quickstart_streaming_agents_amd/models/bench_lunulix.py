@@ -181,12 +181,12 @@ def _attention() -> None:
             shape=[n_seq, n, H, KVH, DH])
         kc, vc = k.view(-1, KVH, DH // 8, 64, 8), v.view(-1, KVH, DH, 64)
         q3 = q.view(T, H, DH)
-        _, item16, t16 = _portions(n_seq, n, 16)
-        t16 = t16.contiguous()
+        _, item32, t32 = _portions(n_seq, n, 32)
+        t32 = t32.contiguous()
         _report("llama paged_attn_prefill", _graph_time([
-            lambda: ext().paged_attn_prefill(q3, kc, vc, bt, item16, t16,
+            lambda: ext().paged_attn_prefill(q3, kc, vc, bt, item32, t32,
                                              i * n, zero, lens, 0.1,
-                                             True)] * 2),
+                                             True, 32)] * 2),
             T * (2 * H + 2 * KVH) * DH * 2, flops,
             shape=[n_seq, n, H, KVH, DH])
 

@@ -85,6 +85,8 @@ class EmbeddingEncoder:
         self._use_hip = str(device).startswith("cuda")
 
     # -- varlen attention plumbing (GPU path) ------------------------------
+    QROWS = 64      # query tokens per attention block: one 16-row tile a wave
+
     def _attn_maps(self, n: int, L: int, lens: torch.Tensor):
         """Page table / q-block maps for the bidirectional varlen kernel.
         Items sit at padded offsets i*L; pages are preallocated per item
@@ -108,7 +110,7 @@ class EmbeddingEncoder:
         qb_item, qb_pos0 = [], []
         lens_l = lens.tolist()
         for i in range(n):
-            for p0 in range(0, max(int(lens_l[i]), 1), 16):
+            for p0 in range(0, max(int(lens_l[i]), 1), self.QROWS):
                 qb_item.append(i)
                 qb_pos0.append(p0)
         dev = self.device
@@ -180,7 +182,7 @@ class EmbeddingEncoder:
                 attn = D.ext().paged_attn_prefill(
                     q, kc, vc, maps["block_table"], maps["qb_item"],
                     maps["qb_pos0"], maps["item_off"], maps["item_start"],
-                    maps["item_len"], self.scale, False)
+                    maps["item_len"], self.scale, False, self.QROWS)
                 attn = attn.contiguous()
             else:
                 # [n*heads, L, D] padded bmm reference

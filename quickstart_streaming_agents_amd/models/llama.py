@@ -389,15 +389,20 @@ class LlamaModel:
                     torch.zeros(padn, dtype=torch.int32, device=dev)
                 ]).contiguous()
         if use_hip_prefill:
-            # varlen flash prefill over the paged cache: per-q-block maps
-            # (one WAVE per 16 q rows x head in the kernel)
-            qb_item, qb_pos0 = [], []
-            for i, n in enumerate(lens):
-                for p0 in range(0, n, 16):
-                    qb_item.append(i)
-                    qb_pos0.append(p0)
-            qb_item_t = torch.tensor(qb_item, dtype=torch.int32, device=dev)
-            qb_pos0_t = torch.tensor(qb_pos0, dtype=torch.int32, device=dev)
+            # varlen flash prefill over the paged cache: maps of blocks of
+            # qrows query tokens, which with their R heads fill the kernel's
+            # 128 rows; 64 where 128 would leave CUs without two blocks
+            qrows = max(1, 128 // R)
+            if sum(-(-n // qrows) for n in lens) * self.n_kv < 512:
+                qrows = max(1, 64 // R)
+            blocks = [(i, p0) for i, n in enumerate(lens)
+                      for p0 in range(0, n, qrows)]
+            # the ones with most keys first: the last to start are short
+            blocks.sort(key=lambda b: -int(items[b[0]][2]) - b[1])
+            qb_item_t = torch.tensor([b[0] for b in blocks],
+                                     dtype=torch.int32, device=dev)
+            qb_pos0_t = torch.tensor([b[1] for b in blocks],
+                                     dtype=torch.int32, device=dev)
             off_t = torch.tensor(offs[:-1], dtype=torch.int32, device=dev)
             start_t = torch.tensor([int(s) for _, _, s in items],
                                    dtype=torch.int32, device=dev)
@@ -445,7 +450,7 @@ class LlamaModel:
                 # gather/pad/score materialization
                 attn = D.ext().paged_attn_prefill(
                     q, kv.k[li], kv.v[li], bt_t, qb_item_t, qb_pos0_t,
-                    off_t, start_t, len_t, self.scale, True)
+                    off_t, start_t, len_t, self.scale, True, qrows)
             else:
                 # padded q: [nb*nmax, n_q, D] -> [nb*KVH, R*nmax, D]
                 q_pad = torch.zeros(nb * nmax, self.n_q, c.d_head,

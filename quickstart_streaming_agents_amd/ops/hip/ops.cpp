@@ -50,7 +50,7 @@ extern "C" void qsa_kv_append_launch(const unsigned short*,
 extern "C" void qsa_paged_attn_prefill_launch(
     const unsigned short*, const unsigned short*, const unsigned short*,
     const int*, const int*, const int*, const int*, const int*, const int*,
-    unsigned short*, float, int, int, int, int, int, long long, int,
+    unsigned short*, float, int, int, int, int, int, long long, int, int,
     hipStream_t);
 extern "C" void qsa_rope_kv_append_launch(unsigned short*,
                                           const unsigned short*,
@@ -253,7 +253,8 @@ torch::Tensor paged_attn_prefill(torch::Tensor q, torch::Tensor kc,
                                  torch::Tensor item_off,
                                  torch::Tensor item_start,
                                  torch::Tensor item_len, double scale,
-                                 bool causal) {
+                                 bool causal, long rows) {
+  // rows: query tokens per block of the maps (qb_item, qb_pos0)
   CHK_DEV(q); CHK_BF16(q); CHK_BF16(kc); CHK_BF16(vc);
   CHK_CONT(kc); CHK_CONT(vc); CHK_I32(block_table); CHK_CONT(block_table);
   CHK_I32(qb_item); CHK_I32(qb_pos0); CHK_I32(item_off);
@@ -263,8 +264,8 @@ torch::Tensor paged_attn_prefill(torch::Tensor q, torch::Tensor kc,
   const int KVH = kc.size(1);
   TORCH_CHECK(D == 128 || D == 64, "D must be 64/128");
   TORCH_CHECK(QH % KVH == 0 && QH / KVH <= 16, "GQA ratio <= 16");
-  TORCH_CHECK(QH % 4 == 0, "QH % 4 == 0 (4 head-waves per workgroup "
-              "lockstep on a shared page stream)");
+  TORCH_CHECK(QH % 4 == 0, "QH % 4 == 0");
+  TORCH_CHECK(rows >= 1 && rows <= 4096, "rows in [1,4096]");
   TORCH_CHECK(vc.size(2) == D && vc.size(3) == 64, "V layout [P,KVH,D,64]");
   const int QB = qb_item.numel();
   const int npmax = block_table.size(1);
@@ -274,7 +275,7 @@ torch::Tensor paged_attn_prefill(torch::Tensor q, torch::Tensor kc,
       qb_item.data_ptr<int>(), qb_pos0.data_ptr<int>(),
       item_off.data_ptr<int>(), item_start.data_ptr<int>(),
       item_len.data_ptr<int>(), u16m(out), (float)scale, QB, QH, KVH, npmax,
-      D, q.stride(0), causal ? 1 : 0, cur_stream());
+      D, q.stride(0), causal ? 1 : 0, (int)rows, cur_stream());
   return out;
 }
 
@@ -539,7 +540,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("scores"), py::arg("col_offset") = 0, py::arg("causal") = false,
         py::arg("row_mod") = 0, py::arg("row_limits") = py::none());
   m.def("paged_attn_prefill", &paged_attn_prefill,
-        "varlen flash prefill attention over the paged cache");
+        "varlen flash prefill attention over the paged cache",
+        py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("block_table"),
+        py::arg("qb_item"), py::arg("qb_pos0"), py::arg("item_off"),
+        py::arg("item_start"), py::arg("item_len"), py::arg("scale"),
+        py::arg("causal"), py::arg("rows") = 16);
   m.def("paged_attn_decode", &paged_attn_decode,
         "paged-attention decode (bf16, GQA, page=64)");
   m.def("kv_append", &kv_append, "append one step's k/v to the paged cache");

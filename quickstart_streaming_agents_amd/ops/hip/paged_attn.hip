@@ -23,7 +23,9 @@
 //
 // The online softmax runs per head-column in registers: column max/sum
 // reduce with two shfl_xor hops (the 4 hi-lane groups of a column).
-#include "common.h"
+#include <type_traits>
+
+#include "lm_common.h"
 
 #define QSA_PAGE 64
 
@@ -401,25 +403,35 @@ extern "C" void qsa_kv_scatter_launch(const unsigned short* knew,
 }
 
 // ---------------------------------------------------------------------------
-// Varlen flash PREFILL attention over the paged cache (K4 prefill path).
+// Varlen flash PREFILL attention over the paged cache (K4 prefill path), and
+// with CAUSAL=false the encoder's bidirectional attention (K1).
 //
-// One WAVE per (16-row q-block, q head): streams the sequence's K/V pages
-// directly from the paged cache (K [P,KVH,D/8,64,8], V^T [P,KVH,D,64] —
-// the same coalesced MFMA fragment reads as the decode kernel), online
-// softmax per q-row column, causal masking against the row's absolute
-// position (cached prefix start + row).  No K/V gather, no padding, no
-// materialized score matrix: each KV byte is read once per wave and the
-// bmm+softmax+bmm chain collapses into one kernel per layer.
+// Host passes maps of blocks of `rows` consecutive query tokens (item id,
+// first token) plus per-item row offset / cached start / new length and the
+// page table.
 //
-// Host passes per-q-block maps (item id, first q position) plus per-item
-// row offset / cached start / new length and the padded page table.
-//
-// CAUSAL=false is the ENCODER path (K1, models/encoder.py): bidirectional
-// attention over the full item — every row attends to every valid key —
-// with the same varlen layout and paged K/V fragment reads.
+// Block = (token block, kv head): the R query heads of a kv head share its
+// keys, so its tokens and heads together form the rows (row = token * R + head)
+// of 16-row tiles, QT per wave, four waves.  Short portions thus fill tiles
+// with heads, and K and V are read once per kv head.  Key heads run fastest
+// over the blocks: with 8 of them a die's L2 keeps one.
+// Each K and V page goes through LDS once per block; the next page is fetched
+// into registers meanwhile.  Scores come out transposed (row = key, column =
+// query row): softmax state and rescale are lane-local, and the keys are dealt
+// to the score tiles so that a lane ends up with 8 consecutive ones, which is
+// the operand layout of the second product and of 16-byte V reads.  V's 16-byte
+// groups are swizzled by row, so that 8 rows of a tile read all banks once.
+// The bound is LDS reads (each K/V fragment serves QT tiles; at QT = 2 they
+// take as long as the matrix cores) beside exp2, so rescaling is left out when
+// no maximum of the wave moved.
+// 1 x 8192 tokens, 32/8 heads of 128: 3128 us with one wave per 16 rows and
+// head reading K and V through L1, 787 us here (700 TFLOP/s); 64 x 700: 1757 ->
+// 523 us.
 // ---------------------------------------------------------------------------
-template <int D, bool CAUSAL>
-__global__ void __launch_bounds__(256)
+#define QSA_NEG (-3.0e38f)
+
+template <int D, int QT, bool CAUSAL>
+__global__ void __launch_bounds__(256, 2)
 qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] strided
                        const unsigned short* __restrict__ kc,
                        const unsigned short* __restrict__ vc,
@@ -430,177 +442,223 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
                        const int* __restrict__ item_start,     // [nb] cached
                        const int* __restrict__ item_len,       // [nb] new rows
                        unsigned short* __restrict__ out,       // [T, QH*D]
-                       float scale, int QB, int QH, int KVH, int npmax,
-                       long long qstride) {
-  constexpr int KSTEPS = D / 32;
-  constexpr int DTILES = D / 16;
-  const int lane = threadIdx.x & 63;
-  const int gw = blockIdx.x * 4 + (threadIdx.x >> 6);  // global wave id
-  // the 4 waves of a workgroup are 4 consecutive heads of the SAME
-  // q-block (and, at R>=4, the same kv head): they stream identical
-  // K/V pages, so keeping them in lockstep (per-page barrier below)
-  // turns 3 of the 4 streams into L1 hits
-  const bool live = gw < QB * QH;
-  const int gws = live ? gw : QB * QH - 1;   // dead waves shadow the last
-  const int qb = gws / QH;
-  const int qh = gws % QH;
+                       float scale2, int QH, int KVH, int npmax,
+                       long long qstride, int rows, int subs) {
+  constexpr int KS = D / 32;           // k-steps of a score tile
+  constexpr int ET = D / 16;           // tiles of value columns
+  constexpr int L = D / 32;            // 16 B loads per thread, K and V each
+  __shared__ __attribute__((aligned(16))) unsigned short kt[64 * D];
+  __shared__ __attribute__((aligned(16))) unsigned short vt[64 * D];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 15, hi = lane >> 4;
   const int R = QH / KVH;
-  const int kvh = qh / R;
-  const int item = qb_item[qb];
-  const int pos0 = qb_pos0[qb];          // first new-row index in the item
-  const int n_i = item_len[item];
-  const int start = item_start[item];
-  const int off = item_off[item];
-  const int col = lane & 15;             // q-row column in the score tiles
-  const int hi = lane >> 4;
+  const int g = blockIdx.x % KVH;
+  const int qb = blockIdx.x / KVH / subs, sub = blockIdx.x / KVH % subs;
+  const int item = qb_item[qb], pos0 = qb_pos0[qb];
+  const int n = item_len[item], start = item_start[item];
+  const int v0 = pos0 * R + sub * 64 * QT;
+  const int vend = min(pos0 + rows, n) * R;
+  if (v0 >= vend) return;              // uniform over the block
+  const long long off = item_off[item];
+  // last key that any row of the block / of this wave sees
+  const int last = start + (CAUSAL ? (min(v0 + 64 * QT, vend) - 1) / R : n - 1);
+  const int w0 = v0 + wave * 16 * QT;
+  const int wfirst = start + min(w0, vend - 1) / R;
+  const int wlast = w0 >= vend ? -1
+      : CAUSAL ? start + (min(w0 + 16 * QT, vend) - 1) / R : last;
 
-  // ---- Q B-fragments: lane holds Q[row pos0+col][k = ks*32 + hi*8+e] --
-  const int qrow_l = min(pos0 + col, n_i - 1);   // clamp pad rows
-  const unsigned short* qrow =
-      q + (long long)(off + qrow_l) * qstride + (long long)qh * D;
-  bf16x8_a qf[KSTEPS];
+  // maxima are taken before the scale, which therefore has to be positive
+  const bool negative = scale2 < 0.f;
+  scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  bf16x8_v qf[QT][KS];
+  int qpos[QT];
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks)
-    qf[ks] = *reinterpret_cast<const bf16x8_a*>(qrow + ks * 32 + hi * 8);
-
-  float m = -3.0e38f, lsum = 0.f;
-  f32x4_a o_acc[DTILES];
+  for (int u = 0; u < QT; ++u) {
+    const int v = min(w0 + u * 16 + col, vend - 1);
+    const int tok = v / R;
+    qpos[u] = CAUSAL ? start + tok : last;
+    const unsigned short* qrow =
+        q + (off + tok) * qstride + (long long)(g * R + v - tok * R) * D;
 #pragma unroll
-  for (int dt = 0; dt < DTILES; ++dt)
-    o_acc[dt] = (f32x4_a){0.f, 0.f, 0.f, 0.f};
-
-  // attention horizon: causal -> the block's LAST row's position;
-  // bidirectional -> the whole item
-  const int max_abs = CAUSAL ? start + min(pos0 + 15, n_i - 1)
-                             : start + n_i - 1;
-  const int npages = (max_abs + QSA_PAGE) / QSA_PAGE;  // ceil(max_abs+1/64)
-  const int* btab = block_table + (long long)item * npmax;
-
-  for (int pi = 0; pi < npages; ++pi) {
-    __syncthreads();   // lockstep the 4 head-waves on the shared page
-    const int page = btab[pi];
-    const unsigned short* kbase =
-        kc + ((((long long)page * KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
-    const unsigned short* vbase =
-        vc + (((long long)page * KVH + kvh) * D) * QSA_PAGE;
-    const int nvalid = min(max_abs + 1 - pi * QSA_PAGE, QSA_PAGE);
-
-    f32x4_a sc[4];
-#pragma unroll
-    for (int pt = 0; pt < 4; ++pt) {
-      f32x4_a acc = {0.f, 0.f, 0.f, 0.f};
-      const int pos = pt * 16 + col;
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        const bf16x8_a kf = *reinterpret_cast<const bf16x8_a*>(
-            kbase + (((long long)(ks * 4 + hi) * QSA_PAGE) + pos) * 8);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], acc,
-                                                      0, 0, 0);
-      }
-      sc[pt] = acc;
-    }
-    // mask: kpos (abs) must be <= start + qrow (abs) and < nvalid bound;
-    // C layout row kpos = pt*16 + hi*4 + r, col = q-row
-    const int qabs = start + pos0 + col;          // this column's row
-    float pagemax = -3.0e38f;
-#pragma unroll
-    for (int pt = 0; pt < 4; ++pt) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kpos = pt * 16 + hi * 4 + r;
-        const int kabs = pi * QSA_PAGE + kpos;
-        const bool ok = (kpos < nvalid) && (!CAUSAL || kabs <= qabs) &&
-                        (pos0 + col < n_i);
-        float v = ok ? sc[pt][r] * scale : -3.0e38f;
-        sc[pt][r] = v;
-        pagemax = fmaxf(pagemax, v);
-      }
-    }
-    pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 16, QSA_WAVE));
-    pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 32, QSA_WAVE));
-    // skip only when EVERY column is masked: the skip must be
-    // wave-uniform — MFMA reads all 64 lanes' source registers
-    // regardless of EXEC, so divergence around the PV MFMAs corrupts
-    // active lanes' products
-    if (__all(pagemax <= -3.0e38f)) continue;
-    const float m_new = fmaxf(m, pagemax);
-    float alpha = __expf(m - m_new);
-    if (m <= -3.0e38f) alpha = 0.f;
-    m = m_new;
-    // o_acc element (dt, r) belongs to OUTPUT ROW hi*4 + r (the PV
-    // C-layout), while alpha lives per score COLUMN (this lane's l&15):
-    // fetch each row's own alpha from the lane holding that column —
-    // using the lane's own alpha zeroes/mis-scales other rows' history
-    // whenever per-row maxima diverge across pages
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float alpha_r = __shfl(alpha, hi * 4 + r, 16);
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) o_acc[dt][r] *= alpha_r;
-    }
-    unsigned int ppk[8];
-    float psum = 0.f;
-#pragma unroll
-    for (int pt = 0; pt < 4; ++pt) {
-      float p0f = 0.f, p1f = 0.f, p2f = 0.f, p3f = 0.f;
-      if (sc[pt][0] > -1.0e38f) p0f = __expf(sc[pt][0] - m_new);
-      if (sc[pt][1] > -1.0e38f) p1f = __expf(sc[pt][1] - m_new);
-      if (sc[pt][2] > -1.0e38f) p2f = __expf(sc[pt][2] - m_new);
-      if (sc[pt][3] > -1.0e38f) p3f = __expf(sc[pt][3] - m_new);
-      psum += p0f + p1f + p2f + p3f;
-      ppk[pt * 2] = f32x2_to_bf16x2(p0f, p1f);
-      ppk[pt * 2 + 1] = f32x2_to_bf16x2(p2f, p3f);
-    }
-    psum += __shfl_xor(psum, 16, QSA_WAVE);
-    psum += __shfl_xor(psum, 32, QSA_WAVE);
-    lsum = lsum * alpha + psum;
-
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int src_a = col + (((2 * hi) & 3) << 4);
-      const int src_b = col + (((2 * hi + 1) & 3) << 4);
-      const int tA = half * 2;
-      const int tB = half * 2 + 1;
-      const unsigned int a0A = __shfl(ppk[tA * 2], src_a, QSA_WAVE);
-      const unsigned int a1A = __shfl(ppk[tA * 2 + 1], src_a, QSA_WAVE);
-      const unsigned int b0A = __shfl(ppk[tA * 2], src_b, QSA_WAVE);
-      const unsigned int b1A = __shfl(ppk[tA * 2 + 1], src_b, QSA_WAVE);
-      const unsigned int a0B = __shfl(ppk[tB * 2], src_a, QSA_WAVE);
-      const unsigned int a1B = __shfl(ppk[tB * 2 + 1], src_a, QSA_WAVE);
-      const unsigned int b0B = __shfl(ppk[tB * 2], src_b, QSA_WAVE);
-      const unsigned int b1B = __shfl(ppk[tB * 2 + 1], src_b, QSA_WAVE);
-      const bool lo = hi < 2;
-      bf16x8_a pa;
-      unsigned int* pa_u = reinterpret_cast<unsigned int*>(&pa);
-      pa_u[0] = lo ? a0A : a0B;
-      pa_u[1] = lo ? a1A : a1B;
-      pa_u[2] = lo ? b0A : b0B;
-      pa_u[3] = lo ? b1A : b1B;
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) {
-        const bf16x8_a vf = *reinterpret_cast<const bf16x8_a*>(
-            vbase + ((long long)(dt * 16 + col) * QSA_PAGE) + half * 32 +
-            hi * 8);
-        o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vf,
-                                                            o_acc[dt],
-                                                            0, 0, 0);
-      }
+    for (int s = 0; s < KS; ++s) {
+      qf[u][s] = *reinterpret_cast<const bf16x8_v*>(qrow + s * 32 + hi * 8);
+      if (negative) qf[u][s] ^= (short)0x8000;
     }
   }
+  f32x4_v acc[QT][ET];
+  float m[QT], l[QT];
+#pragma unroll
+  for (int u = 0; u < QT; ++u) {
+    m[u] = QSA_NEG;
+    l[u] = 0.f;
+#pragma unroll
+    for (int t = 0; t < ET; ++t) acc[u][t] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  }
 
-  // ---- epilogue: O C-layout row = q-row = hi*4 + r, col = dim ----------
-  // per-row 1/l lives in the lanes of its COLUMN; fetch via shfl
+  // LDS places.  K [D/8][64 keys][8]: key 32s + 8h + 4p + r of a page stands
+  // where row h*4 + r of score tile 2s + p reads it.  V [D][64 keys]: group j
+  // of 8 keys of column e stands at j ^ sw(e), sw = e&3 | (e>>3 & 1) << 2.
+  int kdst[L], vdst[L];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int qr = hi * 4 + r;               // q-row this lane holds
-    const float lr = __shfl(lsum, qr, 16);   // lanes 0-15 hold cols 0-15
-    const float inv = (lr > 0.f) ? 1.f / lr : 0.f;
-    if (pos0 + qr < n_i) {
-      unsigned short* orow =
-          out + (long long)(off + pos0 + qr) * (QH * D) + (long long)qh * D;
+  for (int u = 0; u < L; ++u) {
+    const int i = tid + u * 256, key = i & 63;
+    kdst[u] = ((i & ~63) + (key >> 5) * 32 + ((key >> 2) & 1) * 16 +
+               ((key >> 3) & 3) * 4 + (key & 3)) * 8;
+    const int e = i >> 3;
+    vdst[u] = (e * 8 + ((i & 7) ^ ((e & 3) | ((e >> 1) & 4)))) * 8;
+  }
+  const int* bt = block_table + (long long)item * npmax;
+  u32x4_v kr[L], vr[L];
+  auto fetch = [&](int page) {
+    const long long tile = ((long long)page * KVH + g) * (D * QSA_PAGE);
+    const u32x4_v* kp = reinterpret_cast<const u32x4_v*>(kc + tile) + tid;
+    const u32x4_v* vp = reinterpret_cast<const u32x4_v*>(vc + tile) + tid;
 #pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt)
-        orow[dt * 16 + col] = f32_to_bf16(o_acc[dt][r] * inv);
+    for (int u = 0; u < L; ++u) {
+      kr[u] = kp[u * 256];
+      vr[u] = vp[u * 256];
+    }
+  };
+  const int pages = last / QSA_PAGE + 1;
+  fetch(bt[0]);
+  int next = pages > 1 ? bt[1] : 0;
+  for (int pg = 0; pg < pages; ++pg) {
+    const int have = last - pg * QSA_PAGE;        // keys 0..have count
+    lds_barrier();
+    if (have < QSA_PAGE - 1) {
+      // slots nobody has written yet may hold anything, NaN too
+      const int k0 = (tid & 7) * 8;
+#pragma unroll
+      for (int u = 0; u < L; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = k0 + 2 * e;
+          const unsigned int w = vr[u][e];
+          vr[u][e] = k > have ? 0u : k + 1 > have ? w & 0xffffu : w;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < L; ++u) {
+      *reinterpret_cast<u32x4_v*>(kt + kdst[u]) = kr[u];
+      *reinterpret_cast<u32x4_v*>(vt + vdst[u]) = vr[u];
+    }
+    lds_barrier();
+    if (pg + 1 < pages) {
+      fetch(next);
+      next = pg + 2 < pages ? bt[pg + 2] : 0;
+    }
+    if (pg * QSA_PAGE > wlast) continue;          // nothing for this wave
+
+    f32x4_v sc[QT][4];
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt) {
+#pragma unroll
+      for (int u = 0; u < QT; ++u) sc[u][pt] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const bf16x8_v a = *reinterpret_cast<const bf16x8_v*>(
+            kt + ((s * 4 + hi) * 64 + pt * 16 + col) * 8);
+#pragma unroll
+        for (int u = 0; u < QT; ++u)
+          sc[u][pt] = mfma_bf16(a, qf[u][s], sc[u][pt]);
+      }
+    }
+    bf16x8_v pf[QT][2];
+    float alpha[QT], psum[QT], top[QT];
+    bool moved = false;
+    auto softmax = [&](auto edge, auto guard) {
+#pragma unroll
+      for (int u = 0; u < QT; ++u) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if constexpr (edge.value) {
+              const int p = pg * QSA_PAGE + (pt >> 1) * 32 + hi * 8 +
+                            (pt & 1) * 4 + r;
+              if (p > qpos[u]) sc[u][pt][r] = -INFINITY;
+            }
+            if constexpr (guard.value)
+              sc[u][pt][r] = fmaxf(sc[u][pt][r], -INFINITY);
+            mx = fmaxf(mx, sc[u][pt][r]);
+          }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
+        const float mn = fmaxf(m[u], mx * scale2);
+        moved |= mn > m[u];
+        alpha[u] = __builtin_amdgcn_exp2f(m[u] - mn);
+        psum[u] = 0.f;
+        uint2 pk[4];
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt) {
+          float p[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            p[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][pt][r], scale2, -mn));
+            psum[u] += p[r];
+          }
+          pk[pt] = make_uint2(cvt_bf16x2(p[0], p[1]), cvt_bf16x2(p[2], p[3]));
+        }
+        top[u] = mn;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          pf[u][s] = __builtin_bit_cast(
+              bf16x8_v, make_uint4(pk[2 * s].x, pk[2 * s].y, pk[2 * s + 1].x,
+                                   pk[2 * s + 1].y));
+      }
+    };
+    if (pg * QSA_PAGE + QSA_PAGE - 1 > (CAUSAL ? wfirst : last))
+      softmax(std::true_type{}, std::false_type{});
+    else
+      softmax(std::false_type{}, std::false_type{});
+    bool bad = false;
+#pragma unroll
+    for (int u = 0; u < QT; ++u) bad |= !(psum[u] <= 64.f);
+    // a NaN score counts as no key: masked ones are -inf by now
+    if (__any(bad)) softmax(std::false_type{}, std::true_type{});
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      m[u] = top[u];
+      l[u] = l[u] * alpha[u] + psum[u];
+    }
+    if (__any(moved)) {
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+#pragma unroll
+        for (int t = 0; t < ET; ++t) acc[u][t] *= alpha[u];
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int t = 0; t < ET; ++t) {
+        // row i of tile t is column 32(t/2) + 8(i/4) + 4(t%2) + i%4: a lane
+        // collects 8 consecutive columns over two tiles
+        const int e = (t >> 1) * 32 + (col >> 2) * 8 + (t & 1) * 4 + (col & 3);
+        const bf16x8_v a = *reinterpret_cast<const bf16x8_v*>(
+            vt + (e * 8 + ((s * 4 + hi) ^ ((col & 3) | (col & 4)))) * 8);
+#pragma unroll
+        for (int u = 0; u < QT; ++u)
+          acc[u][t] = mfma_bf16(a, pf[u][s], acc[u][t]);
+      }
+  }
+
+#pragma unroll
+  for (int u = 0; u < QT; ++u) {
+    l[u] += __shfl_xor(l[u], 16, QSA_WAVE);
+    l[u] += __shfl_xor(l[u], 32, QSA_WAVE);
+    const float inv = l[u] > 0.f ? 1.f / l[u] : 0.f;
+    const int v = w0 + u * 16 + col;
+    if (v >= vend) continue;
+    const int tok = v / R;
+    unsigned short* orow = out + (off + tok) * ((long long)QH * D) +
+                           (long long)(g * R + v - tok * R) * D;
+#pragma unroll
+    for (int t = 0; t < ET; t += 2) {
+      const f32x4_v a = acc[u][t] * inv, b = acc[u][t + 1] * inv;
+      *reinterpret_cast<uint4*>(orow + t * 16 + hi * 8) =
+          make_uint4(cvt_bf16x2(a[0], a[1]), cvt_bf16x2(a[2], a[3]),
+                     cvt_bf16x2(b[0], b[1]), cvt_bf16x2(b[2], b[3]));
     }
   }
 }
@@ -610,19 +668,25 @@ extern "C" void qsa_paged_attn_prefill_launch(
     const unsigned short* vc, const int* block_table, const int* qb_item,
     const int* qb_pos0, const int* item_off, const int* item_start,
     const int* item_len, unsigned short* out, float scale, int QB, int QH,
-    int KVH, int npmax, int D, long long qstride, int causal,
+    int KVH, int npmax, int D, long long qstride, int causal, int rows,
     hipStream_t stream) {
-  const long long waves = (long long)QB * QH;
-  dim3 grid((unsigned)((waves + 3) / 4));
-#define QSA_PREFILL_CASE(DD, CC)                                          \
-  if (D == DD && causal == (int)CC) {                                     \
-    hipLaunchKernelGGL((qsa_paged_attn_prefill<DD, CC>), grid, dim3(256), \
-                       0, stream, q, kc, vc, block_table, qb_item,        \
-                       qb_pos0, item_off, item_start, item_len, out,      \
-                       scale, QB, QH, KVH, npmax, qstride);               \
-    return;                                                               \
+  const float scale2 = scale * 1.4426950408889634f;
+  // two tiles per wave as soon as a block's rows fill more than one each
+  const int vrows = rows * (QH / KVH), qt = vrows > 64 ? 2 : 1;
+  const int subs = (vrows + 64 * qt - 1) / (64 * qt);
+  const dim3 grid((unsigned)((long long)QB * KVH * subs));
+  if (grid.x == 0) return;
+#define QSA_PREFILL_CASE(DD, QQ, CC)                                          \
+  if (D == DD && qt == QQ && causal == (int)CC) {                             \
+    hipLaunchKernelGGL((qsa_paged_attn_prefill<DD, QQ, CC>), grid, dim3(256), \
+                       0, stream, q, kc, vc, block_table, qb_item, qb_pos0,   \
+                       item_off, item_start, item_len, out, scale2, QH, KVH,  \
+                       npmax, qstride, rows, subs);                           \
+    return;                                                                   \
   }
-  QSA_PREFILL_CASE(128, true) QSA_PREFILL_CASE(128, false)
-  QSA_PREFILL_CASE(64, true) QSA_PREFILL_CASE(64, false)
+  QSA_PREFILL_CASE(128, 1, true) QSA_PREFILL_CASE(128, 1, false)
+  QSA_PREFILL_CASE(64, 1, true) QSA_PREFILL_CASE(64, 1, false)
+  QSA_PREFILL_CASE(128, 2, true) QSA_PREFILL_CASE(128, 2, false)
+  QSA_PREFILL_CASE(64, 2, true) QSA_PREFILL_CASE(64, 2, false)
 #undef QSA_PREFILL_CASE
 }

@@ -524,6 +524,59 @@ def test_varlen_attention_noncausal_matches_torch():
             assert rel < 2e-2, f"causal={causal} item {i}: rel {rel}"
 
 
+@pytest.mark.parametrize("D,QH,KVH,rows,causal", [
+    (128, 32, 8, 32, True), (128, 32, 8, 16, True), (128, 28, 4, 18, True),
+    (64, 8, 8, 128, False), (64, 8, 8, 64, False), (64, 32, 8, 16, False),
+    (64, 16, 1, 8, True), (128, 4, 4, 40, True)])
+def test_paged_attn_prefill_blocks(ext, D, QH, KVH, rows, causal):
+    """Token blocks of every shape over ragged portions with a cached prefix;
+    slots that were never written hold NaN."""
+    from quickstart_streaming_agents_amd.ops import dispatch as disp
+    g = torch.Generator().manual_seed(D + QH + rows)
+    items = [(0, 1), (63, 1), (64, 2), (5, 59), (0, 64), (100, 33), (1, 191),
+             (700, 17)]
+    lens = [n for _, n in items]
+    np_ = [-(-(a + n) // 64) for a, n in items]
+    P, cap = sum(np_), max(np_)
+    kc = torch.full((P, KVH, D // 8, 64, 8), float("nan")).bfloat16().to(dev())
+    vc = torch.full((P, KVH, D, 64), float("nan")).bfloat16().to(dev())
+    pages = torch.randperm(P, generator=g).int()
+    bt = torch.zeros(len(items), cap, dtype=torch.int32)
+    T = sum(lens)
+    q = torch.randn(T, QH, D, generator=g).bfloat16().to(dev())
+    kv, at, offs = [], 0, []
+    for i, (a, n) in enumerate(items):
+        bt[i, :np_[i]] = pages[at:at + np_[i]]
+        at += np_[i]
+        offs.append(sum(lens[:i]))
+        k = torch.randn(a + n, KVH, D, generator=g).bfloat16().to(dev())
+        v = torch.randn(a + n, KVH, D, generator=g).bfloat16().to(dev())
+        pos = torch.arange(a + n)
+        slots = (bt[i][pos // 64] * 64 + pos % 64).int().to(dev())
+        disp.kv_scatter(k, v, kc, vc, slots)
+        kv.append((k.double(), v.double()))
+    blocks = [(i, p) for i, n in enumerate(lens) for p in range(0, n, rows)]
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=dev())
+    out = ext.paged_attn_prefill(
+        q, kc, vc, bt.to(dev()), mk([b[0] for b in blocks]),
+        mk([b[1] for b in blocks]), mk(offs), mk([a for a, _ in items]),
+        mk(lens), D ** -0.5, causal, rows)
+    R = QH // KVH
+    for i, (a, n) in enumerate(items):
+        k, v = (t.repeat_interleave(R, 1).transpose(0, 1) for t in kv[i])
+        qi = q[offs[i]:offs[i] + n].double().transpose(0, 1)
+        s = qi @ k.transpose(1, 2).contiguous() * D ** -0.5
+        if causal:
+            j = torch.arange(a + n, device=dev())
+            s = s.masked_fill(j[None] > j[a:, None], float("-inf"))
+        ref = (s.softmax(-1) @ v).transpose(0, 1).reshape(n, QH * D)
+        got = out[offs[i]:offs[i] + n].double()
+        # probabilities and the result are rounded to bf16: 2^-9 each of
+        # values up to the largest |v|, and independent over the keys
+        assert (got - ref).norm() <= 5e-3 * ref.norm(), i
+        assert (got - ref).abs().max() <= 2 ** -7 * v.abs().max(), i
+
+
 def test_hash_join_gpu_matches_cpu_semantics():
     """K8 hash build/probe on GPU vs the CPU dispatch fallback: random
     keys with duplicates, latest-event-time-wins, TTL cutoff."""
