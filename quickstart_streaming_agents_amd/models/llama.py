@@ -267,6 +267,8 @@ class LlamaModel:
         token (its k/v is appended at position seq_lens-1)."""
         c = self.cfg
         B = tokens.shape[0]
+        if tokens.is_cuda and 1 <= B <= 32 and self._streams_fp8():
+            return self._decode_fp8(tokens, kv, block_table, seq_lens)
         res = self.embed.index_select(0, tokens).contiguous()
         h = None
         mlp_out = None
@@ -278,27 +280,66 @@ class LlamaModel:
                                        c.norm_eps)
             qkv = self._linear(h, L["wqkv"], L.get("wqkv_f"),
                                L.get("wqkv_f8"))
-            if "bqkv" in L:
-                qkv = qkv + L["bqkv"]
-            # strided [B, H, D] views straight into the fused qkv buffer —
-            # the kernels take row strides, no contiguous() copies
-            qd = self.n_q * c.d_head
-            kd = self.n_kv * c.d_head
-            q = qkv[:, :qd].view(B, self.n_q, c.d_head)
-            k = qkv[:, qd:qd + kd].view(B, self.n_kv, c.d_head)
-            v = qkv[:, qd + kd:].view(B, self.n_kv, c.d_head)
-            D.rope_kv_append(q, k, v, kv.k[li], kv.v[li], self.rope_cos,
-                             self.rope_sin, block_table, seq_lens)
-            attn = D.paged_attn_decode(q, kv.k[li], kv.v[li], block_table,
-                                       seq_lens, self.scale)
+            attn = self._decode_attention(qkv, L, li, kv, block_table,
+                                          seq_lens).view(B, -1)
             o = self._tp_all_reduce(
-                self._linear(attn.view(B, -1), L["wo"], L.get("wo_f"),
-                             L.get("wo_f8")))
+                self._linear(attn, L["wo"], L.get("wo_f"), L.get("wo_f8")))
             h = D.rmsnorm_residual(o, res, L["mlp_norm"], c.norm_eps)
             mlp_out = self._ffn(L, h)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)
         return self._linear(final_h, self.lm_head, self.lm_head_f,
                             self.lm_head_f8)
+
+    def _decode_attention(self, qkv: torch.Tensor, L: dict, li: int,
+                          kv: PagedKVCache, block_table: torch.Tensor,
+                          seq_lens: torch.Tensor,
+                          step: bool = False) -> torch.Tensor:
+        """One token per row: rotation, cache append, attention."""
+        if "bqkv" in L:
+            qkv = qkv + L["bqkv"]
+        # strided [B, H, D] views straight into the fused qkv buffer —
+        # the kernels take row strides, no contiguous() copies
+        q, k, v = self._split_qkv(qkv, qkv.shape[0])
+        return D.paged_attn_step(q, k, v, kv.k[li], kv.v[li], self.rope_cos,
+                                 self.rope_sin, block_table, seq_lens,
+                                 self.scale, step)
+
+    def _streams_fp8(self) -> bool:
+        """Whether _decode_fp8 serves this model: every projection packed,
+        dense feed-forwards, and nothing to reduce between ranks."""
+        return self.tp_size == 1 and self.lm_head_f8 is not None and \
+            type(self)._ffn is LlamaModel._ffn and \
+            self.ffn_local % 32 == 0 and self.cfg.hidden % 32 == 0 and all(
+                key + "_f8" in L for L in self.layers
+                for key in ("wqkv", "wo", "wgu", "wdown"))
+
+    def _decode_fp8(self, tokens: torch.Tensor, kv: PagedKVCache,
+                    block_table: torch.Tensor,
+                    seq_lens: torch.Tensor) -> torch.Tensor:
+        """A step of at most 32 rows on the fp8 weight streams: the
+        projections norm their input, gate and add to the residual, so a
+        layer is four of them and the attention."""
+        B, eps = tokens.shape[0], self.cfg.norm_eps
+        parts = self.cfg.hidden // 16        # of a row's sum of squares
+        norms = [L["attn_norm"] for L in self.layers] + [self.final_norm]
+        res, x, ss = D.embed_rows(self.embed, tokens, norms[0])
+        n = 1
+        for li, L in enumerate(self.layers):
+            qkv = D.norm_linear_fp8(x, ss, n, B, eps, L["wqkv_f8"],
+                                    *L["wqkv"].shape)
+            attn = self._decode_attention(qkv, L, li, kv, block_table,
+                                          seq_lens, step=True)
+            x, ss = D.linear_residual_fp8(
+                attn if attn.dim() == 4 else attn.view(B, -1), L["wo_f8"],
+                *L["wo"].shape, res, L["mlp_norm"])
+            n = parts
+            act = D.norm_linear_fp8(x, ss, n, B, eps, L["wgu_f8"],
+                                    *L["wgu"].shape, glu=True)
+            x, ss = D.linear_residual_fp8(act, L["wdown_f8"],
+                                          *L["wdown"].shape, res,
+                                          norms[li + 1])
+        return D.norm_linear_fp8(x, ss, n, B, eps, self.lm_head_f8,
+                                 *self.lm_head.shape)
 
     def _ffn(self, L: dict, h: torch.Tensor) -> torch.Tensor:
         """Dense SwiGLU FFN (TP row/col-parallel). Mixtral overrides with

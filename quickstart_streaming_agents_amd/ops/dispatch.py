@@ -159,6 +159,18 @@ def paged_attn_decode(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
                           scale).to(q.dtype)
 
 
+def paged_attn_step(q, k, v, kc, vc, cos_t, sin_t, block_table, seq_lens,
+                    scale: float, step: bool = False) -> torch.Tensor:
+    """One token per row: q and k rotated to position seq_lens - 1, k and v
+    appended to the cache, attention -> [B, QH, D].  `step` (GPU) returns step
+    rows for linear_residual_fp8 instead."""
+    if _cuda(q):
+        return ext().paged_attn_step(q, k, v, kc, vc, cos_t, sin_t,
+                                     block_table, seq_lens, scale, step)
+    rope_kv_append(q, k, v, kc, vc, cos_t, sin_t, block_table, seq_lens)
+    return paged_attn_decode(q, kc, vc, block_table, seq_lens, scale)
+
+
 # ---- skinny decode GEMM ---------------------------------------------------
 
 def can_pack_weight(n: int, k: int) -> bool:
@@ -222,6 +234,33 @@ def skinny_linear_fp8(x: torch.Tensor, qf: torch.Tensor,
         return ext().skinny_gemm_fp8(x, qf, scale, n, k)
     w = unpack_weight_fp8(qf, scale, n, k)
     return (x.float() @ w.T).to(x.dtype)
+
+
+# Decoding steps of up to 32 rows: norm, activation and residual are done by
+# the projections (GPU; ops/hip/skinny_stream.h).  Rows pass between them as
+# "step rows", whose layout depends on their number, with the sums of squares
+# `ss` in `parts` parts.
+
+def embed_rows(embed: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor):
+    """(residual, step rows of the norm with weight w before 1/rms, ss)."""
+    return ext().embed_rows(embed, tokens, w)
+
+
+def norm_linear_fp8(x: torch.Tensor, ss: torch.Tensor, parts: int, rows: int,
+                    eps: float, packed: tuple, n: int, k: int,
+                    glu: bool = False) -> torch.Tensor:
+    """Normed step rows through a packed fp8 weight: [rows, n].  With `glu`
+    its rows are [gate; up] and the result is silu(gate) * up, step rows."""
+    return ext().skinny_gemm_fp8_norm(x, ss, parts, rows, eps, packed[0],
+                                      packed[1], n, k, glu)
+
+
+def linear_residual_fp8(x: torch.Tensor, packed: tuple, n: int, k: int,
+                        res: torch.Tensor, w: torch.Tensor):
+    """res <- res + step rows x through a packed fp8 weight, in place; returns
+    the step rows of the norm with weight w that follows, and ss."""
+    return ext().skinny_gemm_fp8_residual(x, packed[0], packed[1], n, k, res,
+                                          w)
 
 
 # ---- mixer decoders (qsa_lm_hip) ------------------------------------------

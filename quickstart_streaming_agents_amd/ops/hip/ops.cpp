@@ -38,10 +38,12 @@ extern "C" void qsa_softmax_rows_launch(float*, int, int, int, int, int,
                                         const int*, hipStream_t);
 extern "C" void qsa_softmax_rows_bf16_launch(unsigned short*, long long, int,
                                              float, const int*, hipStream_t);
+extern "C" void qsa_paged_attn_split(int, int, int, int, int, int*, int*);
 extern "C" void qsa_paged_attn_mfma_launch(
     const unsigned short*, const unsigned short*, const unsigned short*,
-    const int*, const int*, float*, float*, unsigned short*, float, int, int,
-    int, int, int, long long, int, hipStream_t);
+    unsigned short*, unsigned short*, const float*, const float*, const int*,
+    const int*, float*, float*, unsigned short*, float, int, int, int, int,
+    int, long long, long long, int, int, int, hipStream_t);
 extern "C" void qsa_kv_append_launch(const unsigned short*,
                                      const unsigned short*, unsigned short*,
                                      unsigned short*, const int*, const int*,
@@ -68,20 +70,23 @@ extern "C" void qsa_skinny_gemm_launch(const unsigned short*,
                                        const unsigned short*, unsigned short*,
                                        int, int, long long, long long,
                                        hipStream_t);
-extern "C" void qsa_skinny_gemm_probe_launch(const unsigned short*,
-                                             const unsigned short*,
-                                             unsigned short*, int, int,
-                                             long long, long long, int, int,
-                                             int, hipStream_t);
-extern "C" void qsa_skinny_gemm_fp8_launch(const unsigned short*,
-                                           const unsigned char*,
-                                           const float*, unsigned short*,
-                                           int, int, long long, long long,
-                                           hipStream_t);
-extern "C" void qsa_skinny_gemm_fp8_probe_launch(
+extern "C" int qsa_skinny_gemm_probe_launch(const unsigned short*,
+                                            const unsigned short*,
+                                            unsigned short*, int, int,
+                                            long long, long long, int, int,
+                                            hipStream_t);
+extern "C" void qsa_skinny_gemm_fp8_launch(
+    const unsigned short*, const unsigned char*, const float*,
+    unsigned short*, unsigned short*, int, int, long long, long long, int,
+    const unsigned short*, const float*, int, float, int, float*, hipStream_t);
+extern "C" int qsa_skinny_gemm_fp8_probe_launch(
     const unsigned short*, const unsigned char*, const float*,
     unsigned short*, int, int, long long, long long, int, int, int,
     hipStream_t);
+extern "C" void qsa_embed_rows_launch(const unsigned short*, const long long*,
+                                      const unsigned short*, unsigned short*,
+                                      unsigned short*, float*, int, int,
+                                      long long, int, hipStream_t);
 extern "C" void qsa_gemm_fp8_batch_launch(const unsigned short*,
                                           const unsigned char*,
                                           const float*, unsigned short*,
@@ -198,9 +203,22 @@ void softmax_rows_bf16_(torch::Tensor scores, double scale,
                                row_limits.data_ptr<int>(), cur_stream());
 }
 
-torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor kc,
-                                torch::Tensor vc, torch::Tensor block_table,
-                                torch::Tensor seq_lens, double scale) {
+// ---- activations of a decoding step ---------------------------------------
+// Up to 4 rows are kept row-major [M, K], more of them packed in fragments
+// [K/32, row tiles, 64, 8] (skinny_stream.h).
+static int step_tiles(long M) { return M <= 4 ? 0 : M <= 16 ? 1 : 2; }
+
+static torch::Tensor step_rows(long M, long K, torch::TensorOptions opts) {
+  const int mt = step_tiles(M);
+  return mt ? torch::empty({K / 32, mt, 64, 8}, opts)
+            : torch::empty({M, K}, opts);
+}
+
+static torch::Tensor decode_attention(
+    const torch::Tensor& q, const torch::Tensor* k, const torch::Tensor* v,
+    torch::Tensor& kc, torch::Tensor& vc, const float* cos_t,
+    const float* sin_t, const torch::Tensor& block_table,
+    const torch::Tensor& seq_lens, double scale, bool step) {
   CHK_DEV(q); CHK_BF16(q); CHK_BF16(kc); CHK_BF16(vc);
   CHK_CONT(kc); CHK_CONT(vc); CHK_I32(block_table); CHK_I32(seq_lens);
   CHK_CONT(block_table);
@@ -214,23 +232,60 @@ torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor kc,
               "K cache layout [P, KVH, D/8, 64, 8]");
   TORCH_CHECK(vc.size(2) == D && vc.size(3) == 64,
               "V cache layout [P, KVH, D, 64] (transposed)");
+  TORCH_CHECK(!step || (B >= 1 && B <= 32), "step rows: B in [1,32]");
   const int max_pages = block_table.size(1);
-  auto out = torch::empty({B, QH, D}, q.options());
-  // flash-decoding split count: fill the 256-CU chip (one WAVE per
-  // (b, kvh, split); 4 splits share a workgroup)
-  int ns = (int)std::min<long long>(32, std::max<long long>(
-      1, (2048 + (long long)B * KVH - 1) / ((long long)B * KVH)));
-  if (ns > 1) ns = std::max(ns, 4);   // fill all 4 waves per workgroup
-  ns = std::min(ns, std::max(1, max_pages));
-  auto opts_f = q.options().dtype(at::kFloat);
-  auto part_o = torch::empty({B, QH, ns, D}, opts_f);
-  auto part_ml = torch::empty({B, QH, ns, 2}, opts_f);
+  const int mt = step ? step_tiles(B) : 0;
+  auto out = mt ? step_rows(B, (long)QH * D, q.options())
+                : torch::empty({B, QH, D}, q.options());
+  int waves, ns;
+  qsa_paged_attn_split(B, QH, KVH, max_pages, D, &waves, &ns);
+  torch::Tensor part_o, part_ml;
+  if (ns > 1) {
+    auto opts_f = q.options().dtype(at::kFloat);
+    part_o = torch::empty({B, QH, ns, D}, opts_f);
+    part_ml = torch::empty({B, QH, ns, 2}, opts_f);
+  }
   qsa_paged_attn_mfma_launch(
-      u16(q), u16(kc), u16(vc), block_table.data_ptr<int>(),
-      seq_lens.data_ptr<int>(), part_o.data_ptr<float>(),
-      part_ml.data_ptr<float>(), u16m(out), (float)scale, B, QH, KVH,
-      max_pages, D, q.stride(0), ns, cur_stream());
+      u16(q), k ? u16(*k) : nullptr, v ? u16(*v) : nullptr, u16m(kc), u16m(vc),
+      cos_t, sin_t, block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
+      ns > 1 ? part_o.data_ptr<float>() : nullptr,
+      ns > 1 ? part_ml.data_ptr<float>() : nullptr, u16m(out), (float)scale, B,
+      QH, KVH, max_pages, D, q.stride(0), k ? k->stride(0) : 0, waves, ns, mt,
+      cur_stream());
   return out;
+}
+
+torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor kc,
+                                torch::Tensor vc, torch::Tensor block_table,
+                                torch::Tensor seq_lens, double scale) {
+  return decode_attention(q, nullptr, nullptr, kc, vc, nullptr, nullptr,
+                          block_table, seq_lens, scale, false);
+}
+
+torch::Tensor paged_attn_step(torch::Tensor q, torch::Tensor k,
+                              torch::Tensor v, torch::Tensor kc,
+                              torch::Tensor vc, torch::Tensor cos_t,
+                              torch::Tensor sin_t, torch::Tensor block_table,
+                              torch::Tensor seq_lens, double scale,
+                              bool step) {
+  // rope_kv_append and paged_attn_decode in one; q, k and v stay as they
+  // are.  step: the result as step rows instead of [B, QH, D]
+  CHK_BF16(k); CHK_BF16(v); CHK_F32(cos_t); CHK_F32(sin_t);
+  CHK_CONT(cos_t); CHK_CONT(sin_t);
+  const int D = q.size(2);
+  chk_hd_strided(k, D, "k"); chk_hd_strided(v, D, "v");
+  TORCH_CHECK(k.size(0) == q.size(0) && k.size(1) == kc.size(1) &&
+                  v.sizes() == k.sizes(), "k/v [B, KVH, D]");
+  TORCH_CHECK(k.stride(0) == v.stride(0), "k/v strides must match");
+  TORCH_CHECK(q.stride(0) % 8 == 0 && k.stride(0) % 8 == 0 &&
+                  ((reinterpret_cast<uintptr_t>(q.data_ptr()) |
+                    reinterpret_cast<uintptr_t>(k.data_ptr())) & 15) == 0,
+              "q and k rows must be 16-byte aligned");
+  TORCH_CHECK(cos_t.size(-1) == D / 2 && sin_t.size(-1) == D / 2,
+              "cos/sin [positions, D/2]");
+  return decode_attention(q, &k, &v, kc, vc, cos_t.data_ptr<float>(),
+                          sin_t.data_ptr<float>(), block_table, seq_lens,
+                          scale, step);
 }
 
 void kv_append(torch::Tensor knew, torch::Tensor vnew, torch::Tensor kc,
@@ -337,13 +392,17 @@ torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor wf, long N, long K) {
 }
 
 torch::Tensor skinny_gemm_probe(torch::Tensor a, torch::Tensor wf, long N,
-                                long K, long waves, long nt, long variant) {
+                                long K, long waves, long tiles) {
   CHK_DEV(a); CHK_BF16(a); CHK_BF16(wf); CHK_CONT(wf);
   const int M = a.size(0);
+  TORCH_CHECK(M >= 1 && M <= 32 && N % (16 * tiles) == 0 && K % 64 == 0 &&
+                  wf.numel() == (long long)N * K && a.size(1) == K,
+              "skinny_gemm_probe: shapes");
   auto out = torch::empty({M, (long long)N}, a.options());
-  qsa_skinny_gemm_probe_launch(u16(a), u16(wf), u16m(out), M, (int)N, K,
-                               a.stride(0), (int)waves, (int)nt,
-                               (int)variant, cur_stream());
+  TORCH_CHECK(qsa_skinny_gemm_probe_launch(u16(a), u16(wf), u16m(out), M,
+                                           (int)N, K, a.stride(0), (int)waves,
+                                           (int)tiles, cur_stream()),
+              "skinny_gemm_probe: no such block shape");
   return out;
 }
 
@@ -425,38 +484,136 @@ torch::Tensor hash_probe(torch::Tensor tkeys, torch::Tensor tpay,
   return out;
 }
 
-torch::Tensor skinny_gemm_fp8(torch::Tensor a, torch::Tensor qf,
-                              torch::Tensor scale, long N, long K) {
-  // C[M,N] = a @ (scale[N] * dequant(Q))^T; Q pre-packed fp8 e4m3 in the
-  // fragment-pair-major stream layout (skinny_gemm_fp8.hip header).
-  CHK_DEV(a); CHK_BF16(a); CHK_CONT(qf);
+static void chk_fp8_weight(const torch::Tensor& qf, const torch::Tensor& scale,
+                           long N, long K) {
+  CHK_DEV(qf); CHK_CONT(qf);
   TORCH_CHECK(qf.scalar_type() == torch::kUInt8, "qf must be uint8 (fp8)");
   TORCH_CHECK(scale.scalar_type() == torch::kFloat32 && scale.is_cuda() &&
                   scale.is_contiguous() && scale.numel() == N,
               "scale must be f32 [N] on device");
+  TORCH_CHECK(K % 256 == 0 && N % 16 == 0, "K%256==0, N%16==0");
+  TORCH_CHECK(qf.numel() == (long long)N * K, "qf size");
+}
+
+static int chk_skinny_fp8(const torch::Tensor& a, const torch::Tensor& qf,
+                          const torch::Tensor& scale, long N, long K) {
+  CHK_DEV(a); CHK_BF16(a);
   TORCH_CHECK(a.dim() == 2 && a.stride(1) == 1, "a rows must be contiguous");
   const int M = a.size(0);
   TORCH_CHECK(M >= 1 && M <= 32, "skinny_gemm_fp8: M in [1,32]");
   TORCH_CHECK(a.size(1) == K, "K mismatch");
-  TORCH_CHECK(K % 256 == 0 && N % 16 == 0, "K%256==0, N%16==0");
-  TORCH_CHECK(qf.numel() == (long long)N * K, "qf size");
+  chk_fp8_weight(qf, scale, N, K);
+  return M;
+}
+
+torch::Tensor skinny_gemm_fp8(torch::Tensor a, torch::Tensor qf,
+                              torch::Tensor scale, long N, long K) {
+  // C[M,N] = a @ (scale[N] * dequant(Q))^T; Q pre-packed fp8 e4m3 in the
+  // fragment-pair-major stream layout (skinny_gemm_fp8.hip header).
+  const int M = chk_skinny_fp8(a, qf, scale, N, K);
   auto out = torch::empty({M, (long long)N}, a.options());
   qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
-                             scale.data_ptr<float>(), u16m(out), M, (int)N,
-                             K, a.stride(0), cur_stream());
+                             scale.data_ptr<float>(), u16m(out), nullptr, M,
+                             (int)N, K, a.stride(0), 0, nullptr, nullptr, 0,
+                             0.f, 0, nullptr, cur_stream());
   return out;
 }
 
+// step rows, their sums of squares being [32, parts4] (parts rounded up to 4)
+static void chk_step_rows(const torch::Tensor& a, long M, long K) {
+  CHK_DEV(a); CHK_BF16(a); CHK_CONT(a);
+  TORCH_CHECK(M >= 1 && M <= 32, "step rows: M in [1,32]");
+  const int mt = step_tiles(M);
+  TORCH_CHECK(mt ? a.dim() == 4 && a.size(1) == mt &&
+                       a.numel() == (long long)K * mt * 16
+                 : a.dim() == 2 && a.size(0) == M && a.size(1) == K,
+              "step rows: shape");
+}
+
+torch::Tensor skinny_gemm_fp8_norm(torch::Tensor a, torch::Tensor ss,
+                                   long parts, long M, double eps,
+                                   torch::Tensor qf, torch::Tensor scale,
+                                   long N, long K, bool glu) {
+  // a: rows x * w of an rms norm; 1/rms from the rows' sums of squares.
+  // glu: Q's rows are [gate; up], returns silu(gate) * up as step rows.
+  chk_step_rows(a, M, K);
+  chk_fp8_weight(qf, scale, N, K);
+  CHK_DEV(ss); CHK_F32(ss); CHK_CONT(ss);
+  TORCH_CHECK(parts >= 1 && ss.numel() == 32 * ((parts + 3) & ~3L),
+              "sums of squares [32, parts4]");
+  TORCH_CHECK(!glu || N % 64 == 0, "gate and up: N % 64 == 0");
+  auto out = glu ? step_rows(M, N / 2, a.options())
+                 : torch::empty({(long long)M, (long long)N}, a.options());
+  qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
+                             scale.data_ptr<float>(), u16m(out), nullptr,
+                             (int)M, (int)N, K, K, step_tiles(M) > 0, nullptr,
+                             ss.data_ptr<float>(), (int)parts, (float)eps,
+                             glu ? 1 : 0, nullptr, cur_stream());
+  return out;
+}
+
+std::vector<torch::Tensor> skinny_gemm_fp8_residual(
+    torch::Tensor a, torch::Tensor qf, torch::Tensor scale, long N, long K,
+    torch::Tensor res, torch::Tensor w) {
+  // res [M, N] <- res + the product; returns the rows of the norm with weight
+  // w that follows (before 1/rms) and the sums of squares in N/16 parts
+  CHK_DEV(res); CHK_BF16(res); CHK_CONT(res);
+  TORCH_CHECK(res.dim() == 2 && res.size(1) == N, "residual [M, N]");
+  const long M = res.size(0);
+  chk_step_rows(a, M, K);
+  chk_fp8_weight(qf, scale, N, K);
+  CHK_DEV(w); CHK_BF16(w); CHK_CONT(w);
+  TORCH_CHECK(w.numel() == N && N % 32 == 0, "norm weight [N], N % 32 == 0");
+  auto next = step_rows(M, N, a.options());
+  auto ss = torch::empty({32, (N / 16 + 3) & ~3L},
+                         a.options().dtype(at::kFloat));
+  qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
+                             scale.data_ptr<float>(), u16m(res), u16m(next),
+                             (int)M, (int)N, K, K, step_tiles(M) > 0, u16(w),
+                             nullptr, 0, 0.f, 0, ss.data_ptr<float>(),
+                             cur_stream());
+  return {next, ss};
+}
+
+std::vector<torch::Tensor> embed_rows(torch::Tensor embed,
+                                      torch::Tensor tokens,
+                                      torch::Tensor w) {
+  // (embed[tokens], the rows of the norm with weight w that follows, the
+  // sums of squares in one part)
+  CHK_DEV(embed); CHK_BF16(embed); CHK_CONT(embed); CHK_DEV(tokens);
+  TORCH_CHECK(tokens.scalar_type() == torch::kInt64 &&
+                  tokens.is_contiguous() && tokens.dim() == 1,
+              "tokens must be contiguous i64 [M]");
+  const long M = tokens.size(0), H = embed.size(1);
+  TORCH_CHECK(M >= 1 && M <= 32 && H % 32 == 0, "M in [1,32], H % 32 == 0");
+  CHK_DEV(w); CHK_BF16(w); CHK_CONT(w);
+  TORCH_CHECK(w.numel() == H, "norm weight [H]");
+  auto res = torch::empty({M, H}, embed.options());
+  auto next = step_rows(M, H, embed.options());
+  auto ss = torch::empty({32, 4}, embed.options().dtype(at::kFloat));
+  qsa_embed_rows_launch(u16(embed),
+                        (const long long*)tokens.data_ptr<int64_t>(), u16(w),
+                        u16m(res), u16m(next), ss.data_ptr<float>(), (int)M,
+                        (int)H, embed.size(0), step_tiles(M), cur_stream());
+  return {res, next, ss};
+}
+
 torch::Tensor skinny_gemm_fp8_probe(torch::Tensor a, torch::Tensor qf,
-                                    torch::Tensor scale, long N, long K,
-                                    long waves, long tiles, long nt) {
-  CHK_DEV(a); CHK_BF16(a); CHK_CONT(qf);
-  const int M = a.size(0);
-  auto out = torch::empty({M, (long long)N}, a.options());
-  qsa_skinny_gemm_fp8_probe_launch(u16(a), qf.data_ptr<unsigned char>(),
-                                   scale.data_ptr<float>(), u16m(out), M,
-                                   (int)N, K, a.stride(0), (int)waves,
-                                   (int)tiles, (int)nt, cur_stream());
+                                    torch::Tensor scale, long M, long N,
+                                    long K, long waves, long tiles) {
+  // a: [M, K], or packed fragments
+  chk_fp8_weight(qf, scale, N, K);
+  CHK_DEV(a); CHK_BF16(a); CHK_CONT(a);
+  const bool pack = a.dim() == 4;
+  TORCH_CHECK(M >= 1 && M <= 32 && N % (16 * tiles) == 0 &&
+                  a.numel() == (pack ? (M <= 16 ? 16 : 32) : M) * (long long)K,
+              "skinny_gemm_fp8_probe: shapes");
+  auto out = torch::empty({(long long)M, (long long)N}, a.options());
+  TORCH_CHECK(qsa_skinny_gemm_fp8_probe_launch(
+                  u16(a), qf.data_ptr<unsigned char>(),
+                  scale.data_ptr<float>(), u16m(out), (int)M, (int)N, K, K,
+                  pack, (int)waves, (int)tiles, cur_stream()),
+              "skinny_gemm_fp8_probe: no such block shape");
   return out;
 }
 
@@ -547,6 +704,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("causal"), py::arg("rows") = 16);
   m.def("paged_attn_decode", &paged_attn_decode,
         "paged-attention decode (bf16, GQA, page=64)");
+  m.def("paged_attn_step", &paged_attn_step,
+        "a decoding step's rotation, cache append and attention");
   m.def("kv_append", &kv_append, "append one step's k/v to the paged cache");
   m.def("rope_kv_append", &rope_kv_append,
         "fused decode rope + paged-cache append");
@@ -556,13 +715,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm,
         "decode-batch GEMM (M<=32) on the packed weight stream");
   m.def("skinny_gemm_probe", &skinny_gemm_probe,
-        "ablation probe: waves/nt/variant sweep");
+        "tuning probe: waves, tiles");
   m.def("skinny_gemm_fp8", &skinny_gemm_fp8,
         "fp8-weight decode GEMM (M<=32): half the weight stream");
   m.def("gemm_fp8_batch", &gemm_fp8_batch,
         "batched-M (<=256) fp8 weight-stream GEMM with optional split-K");
   m.def("skinny_gemm_fp8_probe", &skinny_gemm_fp8_probe,
-        "fp8 ablation probe: waves/tiles/nt sweep");
+        "fp8 tuning probe: waves, tiles");
+  m.def("skinny_gemm_fp8_norm", &skinny_gemm_fp8_norm,
+        "fp8-weight decode GEMM of rms-normed rows, optionally gated");
+  m.def("skinny_gemm_fp8_residual", &skinny_gemm_fp8_residual,
+        "fp8-weight decode GEMM added to the residual stream");
+  m.def("embed_rows", &embed_rows,
+        "a step's first rows and their sums of squares");
   m.def("topk_cosine", &topk_cosine, "exact cosine top-k over the HBM index");
   m.def("hash_build", &hash_build,
         "build latest-per-key hash table from (keys, event ts)");

@@ -4,25 +4,30 @@
 // terraform/core/main.tf:461) with on-GPU batched decode attention over a
 // paged KV cache resident in 288 GB HBM3E.
 //
-// Design (flash-decoding, one WAVE per (batch b, kv head, context split)):
+// Design (flash decoding; a block of NW waves per (row b, kv head, share of the
+// pages), a wave per page in turn):
 //   - All R GQA query heads of a kv head compute TOGETHER on the matrix
 //     cores: scores via mfma_f32_16x16x32_bf16 with A = K-tile
 //     [16 pos x 32 k] and B = Q [32 k x 16 heads] (heads pad to 16), PV
 //     via A = P [16 heads x 32 pos] (packed bf16, redistributed with 8
-//     cross-lane shuffles) and B = V^T [32 pos x 16 dims].  A VALU
-//     decode kernel pays ~16 VALU per 16 B of KV; this pays ~1 MFMA per
-//     1 KiB plus the online-softmax tail.
-//   - K cache layout [page, kvh, D/8, 64, 8] (d-major x8): the A-fragment
-//     read (lane = pos x k-slice) is one fully coalesced 1 KiB wave load.
-//   - V cache layout [page, kvh, D, 64] (TRANSPOSED, pos minor): the PV
-//     B-fragment read (lane = dim x pos-slice) is also one coalesced 1 KiB
-//     wave load.  Every KV byte is read exactly ONCE per (b, kvh) — the
-//     per-head VALU design re-read it R times.
-//   - Context splits fill the chip (grid = B*KVH*NS >= ~2k waves);
-//     unnormalized partials (o, m, l) merge in qsa_attn_reduce.
+//     cross-lane shuffles) and B = V^T [32 pos x 16 dims].  Every KV byte is
+//     read exactly once.
+//   - K cache layout [page, kvh, D/8, 64, 8] (d-major x8) and V cache layout
+//     [page, kvh, D, 64] (transposed, pos minor): both fragment reads are
+//     coalesced 1 KiB wave loads.  The values of a page and the keys of the
+//     next one are under way while its scores are computed: 32 KiB a wave.
+//   - The waves of a block merge in LDS.  One block per (row, kv head) stores
+//     the result; several leave (o, m, l) for qsa_attn_reduce.
+//   - FUSE is a decoding step's attention: q is rotated in registers, and the
+//     wave with the last page first writes the rotated new key and the new
+//     value to the cache, so that no launch has to come before.
+// 192 rows of 400-1000 keys, 32/8 heads of 128: rotation 11, attention 172,
+// merge 7 us as separate kernels with a wave per share, 130 us here (4.2 TB/s); 16
+// rows of 1536-2048: 5 + 35 + 9, 29 + 5.
 //
 // The online softmax runs per head-column in registers: column max/sum
 // reduce with two shfl_xor hops (the 4 hi-lane groups of a column).
+#include <algorithm>
 #include <type_traits>
 
 #include "lm_common.h"
@@ -32,53 +37,62 @@
 using bf16x8_a = __attribute__((ext_vector_type(8))) short;
 using f32x4_a = __attribute__((ext_vector_type(4))) float;
 
-template <int D>
-__global__ void __launch_bounds__(256)
-qsa_paged_attn_mfma(const unsigned short* __restrict__ q,   // [B, QH, D]
-                    const unsigned short* __restrict__ kc,  // [P, KVH, D/8, 64, 8]
-                    const unsigned short* __restrict__ vc,  // [P, KVH, D, 64]
-                    const int* __restrict__ block_table,    // [B, max_pages]
-                    const int* __restrict__ seq_lens,       // [B]
-                    float* __restrict__ part_o,              // [B, QH, NS, D]
-                    float* __restrict__ part_ml,             // [B, QH, NS, 2]
-                    float scale, int B, int QH, int KVH, int max_pages,
-                    long long qstride, int NS) {
+// place of element k of a step's row in packed activations (skinny_stream.h)
+__device__ __forceinline__ long long qsa_step_at(int row, int k, int mt) {
+  return ((long long)(k >> 5) * mt + (row >> 4)) * 512 +
+         ((row & 15) + ((k >> 3) & 3) * 16) * 8 + (k & 7);
+}
+
+struct DecodeArgs {
+  const unsigned short* q;             // [B, QH, D], row stride qstride
+  const unsigned short* kc;            // [P, KVH, D/8, 64, 8]
+  const unsigned short* vc;            // [P, KVH, D, 64]
+  const int* block_table;              // [B, max_pages]
+  const int* seq_lens;                 // [B]
+  float* part_o;                       // [B, QH, NS, D]
+  float* part_ml;                      // [B, QH, NS, 2]
+  unsigned short* out;                 // NS == 1: [B, QH, D], or packed rows
+  // FUSE
+  const unsigned short* k;             // [B, KVH, D], row stride kvstride
+  const unsigned short* v;
+  unsigned short* kw;                  // the caches again, to write
+  unsigned short* vw;
+  const float* cos_t;                  // [positions, D/2]
+  const float* sin_t;
+  float scale;
+  int QH, KVH, max_pages, NS, mt;      // mt: row tiles of packed rows, or 0
+  long long qstride, kvstride;
+};
+
+// rotate elements k0.. and k0 + D/2.. of a row held in two fragments
+__device__ __forceinline__ void rotate_pair(bf16x8_a& a, bf16x8_a& b,
+                                            const float* c, const float* s) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x = bf16_to_f32((unsigned short)a[e]);
+    const float y = bf16_to_f32((unsigned short)b[e]);
+    a[e] = (short)f32_to_bf16(x * c[e] - y * s[e]);
+    b[e] = (short)f32_to_bf16(x * s[e] + y * c[e]);
+  }
+}
+
+template <int D, int NW, bool FUSE>
+__global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
+qsa_paged_attn_mfma(DecodeArgs p) {
   constexpr int KSTEPS = D / 32;      // QK^T k-steps (4 for D=128)
   constexpr int DTILES = D / 16;      // PV d-tiles (8 for D=128)
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int nsb = (NS + 3) / 4;       // split-blocks per (b, kvh)
-  const int bk = blockIdx.x / nsb;
-  const int split = (blockIdx.x % nsb) * 4 + wave;
-  const int b = bk / KVH;
-  const int kvh = bk % KVH;
-  const int R = QH / KVH;
-  if (split >= NS) return;
-
-  const int seqlen = seq_lens[b];
+  extern __shared__ float smem[];     // [NW][R][D] o, [NW][16] m, [NW][16] l
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int split = blockIdx.x % p.NS;
+  const int bk = blockIdx.x / p.NS;
+  const int b = bk / p.KVH;
+  const int kvh = bk % p.KVH;
+  const int R = p.QH / p.KVH;
+  const int seqlen = p.seq_lens[b];
   const int npages = (seqlen + QSA_PAGE - 1) / QSA_PAGE;
-  const int chunk = (npages + NS - 1) / NS;
-  const int p0 = split * chunk;
-  const int p1 = min(npages, p0 + chunk);
   const int col = lane & 15;          // head col (scores) / dim col (PV)
   const int hi = lane >> 4;           // 4 hi-lane groups
-
-  // every (head) slot writes its partial, real or empty
-  float* pml_base = part_ml + (((long long)b * QH + kvh * R) * NS + split) * 2;
-  if (seqlen <= 0 || p0 >= npages) {
-    if (lane < R)
-      *reinterpret_cast<float2*>(pml_base + (long long)lane * NS * 2) =
-          make_float2(-3.0e38f, 0.f);
-    return;
-  }
-
-  // ---- Q B-fragments: lane holds Q[head=col][k = ks*32 + hi*8 + e] ----
-  const int qh_l = kvh * R + min(col, R - 1);   // clamp: pad heads compute
-  const unsigned short* qrow = q + (long long)b * qstride + (long long)qh_l * D;
-  bf16x8_a qf[KSTEPS];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks)
-    qf[ks] = *reinterpret_cast<const bf16x8_a*>(qrow + ks * 32 + hi * 8);
 
   float m = -3.0e38f, lsum = 0.f;
   f32x4_a o_acc[DTILES];
@@ -86,193 +100,303 @@ qsa_paged_attn_mfma(const unsigned short* __restrict__ q,   // [B, QH, D]
   for (int dt = 0; dt < DTILES; ++dt)
     o_acc[dt] = (f32x4_a){0.f, 0.f, 0.f, 0.f};
 
-  const int* btab = block_table + (long long)b * max_pages;
-  for (int pi = p0; pi < p1; ++pi) {
-    const int page = btab[pi];
-    const unsigned short* kbase =
-        kc + ((((long long)page * KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
-    const unsigned short* vbase =
-        vc + (((long long)page * KVH + kvh) * D) * QSA_PAGE;
-    const int nvalid = min(seqlen - pi * QSA_PAGE, QSA_PAGE);
-
-    // ---- scores: 4 pos-tiles x KSTEPS MFMAs ---------------------------
-    // A-frag: lane holds K[pos = pt*16 + col][k = ks*32 + hi*8 + e];
-    // K layout element (pos, k) at ((k/8)*64 + pos)*8 + k%8 ->
-    // 16 B at ((ks*4 + hi)*64 + pos)*8.
-    f32x4_a sc[4];
+  const int first = split * NW + wave, step = NW * p.NS;
+  if (first < npages) {               // uniform over the wave
+    // ---- Q B-fragments: lane holds Q[head=col][k = ks*32 + hi*8 + e] ----
+    const int qh_l = kvh * R + min(col, R - 1);   // clamp: pad heads compute
+    const unsigned short* qrow =
+        p.q + (long long)b * p.qstride + (long long)qh_l * D;
+    bf16x8_a qf[KSTEPS];
 #pragma unroll
-    for (int pt = 0; pt < 4; ++pt) {
-      f32x4_a acc = {0.f, 0.f, 0.f, 0.f};
-      const int pos = pt * 16 + col;
+    for (int ks = 0; ks < KSTEPS; ++ks)
+      qf[ks] = *reinterpret_cast<const bf16x8_a*>(qrow + ks * 32 + hi * 8);
+    const int* btab = p.block_table + (long long)b * p.max_pages;
+    if constexpr (FUSE) {
+      const long long at = (long long)(seqlen - 1) * (D / 2) + hi * 8;
 #pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        const bf16x8_a kf = *reinterpret_cast<const bf16x8_a*>(
-            kbase + (((long long)(ks * 4 + hi) * QSA_PAGE) + pos) * 8);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], acc,
-                                                      0, 0, 0);
+      for (int ks = 0; ks < KSTEPS / 2; ++ks) {
+        float c[8], s[8];
+        ldv<float, 8>(p.cos_t + at + ks * 32, c);
+        ldv<float, 8>(p.sin_t + at + ks * 32, s);
+        rotate_pair(qf[ks], qf[ks + KSTEPS / 2], c, s);
       }
-      sc[pt] = acc;
-    }
-    // scale + mask invalid positions; C layout: row pos = hi*4 + r,
-    // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
-    float pagemax = -3.0e38f;
+      if ((npages - 1 - first) % step == 0) {     // the last page is this wave's
+        const int pin = (seqlen - 1) % QSA_PAGE;  // the new token's slot
+        const long long tile =
+            ((long long)btab[npages - 1] * p.KVH + kvh) * D * QSA_PAGE;
+        const long long row = (long long)b * p.kvstride + (long long)kvh * D;
+        const int d = lane * 8;
+        if (d < D / 2) {              // lane: keys d.. and d + D/2..
+          bf16x8_a x = *reinterpret_cast<const bf16x8_a*>(p.k + row + d);
+          bf16x8_a y =
+              *reinterpret_cast<const bf16x8_a*>(p.k + row + d + D / 2);
+          const long long t = (long long)(seqlen - 1) * (D / 2) + d;
+          float c[8], s[8];
+          ldv<float, 8>(p.cos_t + t, c);
+          ldv<float, 8>(p.sin_t + t, s);
+          rotate_pair(x, y, c, s);
+          unsigned short* kp = p.kw + tile + (lane * QSA_PAGE + pin) * 8;
+          *reinterpret_cast<bf16x8_a*>(kp) = x;
+          *reinterpret_cast<bf16x8_a*>(kp + D / 2 * QSA_PAGE) = y;
+        }
 #pragma unroll
-    for (int pt = 0; pt < 4; ++pt) {
+        for (int i = 0; i < D; i += 64)
+          p.vw[tile + (long long)(i + lane) * QSA_PAGE + pin] =
+              p.v[row + i + lane];
+        // the page is read by this wave alone: its stores come first
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+      }
+    }
+
+    auto load_k = [&](int page, bf16x8_a (&kf)[4][KSTEPS]) {
+      const unsigned short* kbase =
+          p.kc + ((((long long)page * p.KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks)
+          kf[pt][ks] = *reinterpret_cast<const bf16x8_a*>(
+              kbase + ((ks * 4 + hi) * QSA_PAGE + pt * 16 + col) * 8);
+    };
+    bf16x8_a kf[4][KSTEPS];
+    int page = btab[first];
+    load_k(page, kf);
+    for (int pi = first; pi < npages; pi += step) {
+      const bool more = pi + step < npages;
+      const int next = more ? btab[pi + step] : 0;
+      const long long head = (long long)page * p.KVH + kvh;
+      const unsigned short* vbase = p.vc + head * D * QSA_PAGE;
+      const int nvalid = min(seqlen - pi * QSA_PAGE, QSA_PAGE);
+      bf16x8_a vf[2][DTILES];
+      // B-frag: lane holds V^T[pos = half*32 + hi*8 + e][d = dt*16+col]
+      auto load_v = [&](int half) {
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt)
+          vf[half][dt] = *reinterpret_cast<const bf16x8_a*>(
+              vbase + (dt * 16 + col) * QSA_PAGE + half * 32 + hi * 8);
+      };
+      load_v(0);
+      // ---- scores: 4 pos-tiles x KSTEPS MFMAs ---------------------------
+      // A-frag: lane holds K[pos = pt*16 + col][k = ks*32 + hi*8 + e]
+      f32x4_a sc[4];
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt) {
+        f32x4_a acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[pt][ks], qf[ks],
+                                                        acc, 0, 0, 0);
+        sc[pt] = acc;
+      }
+      load_v(1);
+      if (more) load_k(next, kf);
+      // scale + mask invalid positions; C layout: row pos = hi*4 + r,
+      // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
+      float pagemax = -3.0e38f;
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int pos = pt * 16 + hi * 4 + r;
+          float v = (pos < nvalid) ? sc[pt][r] * p.scale : -3.0e38f;
+          sc[pt][r] = v;
+          pagemax = fmaxf(pagemax, v);
+        }
+      }
+      // column (per-head) max across the 4 hi groups
+      pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 16, QSA_WAVE));
+      pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 32, QSA_WAVE));
+      const float m_new = fmaxf(m, pagemax);
+      float alpha = __expf(m - m_new);
+      if (m <= -3.0e38f) alpha = 0.f;
+      m = m_new;
+      // o_acc element (dt, r) belongs to OUTPUT ROW hi*4 + r (the PV
+      // C-layout), while alpha lives per score COLUMN (this lane's l&15):
+      // fetch each row's own alpha from the lane holding that column
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int pos = pt * 16 + hi * 4 + r;
-        float v = (pos < nvalid) ? sc[pt][r] * scale : -3.0e38f;
-        sc[pt][r] = v;
-        pagemax = fmaxf(pagemax, v);
+        const float alpha_r = __shfl(alpha, hi * 4 + r, 16);
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt) o_acc[dt][r] *= alpha_r;
       }
-    }
-    // column (per-head) max across the 4 hi groups
-    pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 16, QSA_WAVE));
-    pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 32, QSA_WAVE));
-    const float m_new = fmaxf(m, pagemax);
-    float alpha = __expf(m - m_new);
-    if (m <= -3.0e38f) alpha = 0.f;
-    m = m_new;
-    // o_acc element (dt, r) belongs to OUTPUT ROW hi*4 + r (the PV
-    // C-layout), while alpha lives per score COLUMN (this lane's l&15):
-    // fetch each row's own alpha from the lane holding that column —
-    // using the lane's own alpha zeroes/mis-scales other rows' history
-    // whenever per-row maxima diverge across pages
+      // P = exp(sc - m) (invalid -> 0), packed bf16x2 per tile quad
+      unsigned int ppk[8];   // tile pt -> 2 uints (4 bf16 = quads r0..3)
+      float psum = 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float alpha_r = __shfl(alpha, hi * 4 + r, 16);
+      for (int pt = 0; pt < 4; ++pt) {
+        float pr[4];
 #pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) o_acc[dt][r] *= alpha_r;
-    }
-    // P = exp(sc - m) (invalid -> 0), packed bf16x2 per tile quad
-    unsigned int ppk[8];   // tile pt -> 2 uints (4 bf16 = quads r0..3)
-    float psum = 0.f;
-#pragma unroll
-    for (int pt = 0; pt < 4; ++pt) {
-      float p0f = 0.f, p1f = 0.f, p2f = 0.f, p3f = 0.f;
-      if (sc[pt][0] > -1.0e38f) p0f = __expf(sc[pt][0] - m_new);
-      if (sc[pt][1] > -1.0e38f) p1f = __expf(sc[pt][1] - m_new);
-      if (sc[pt][2] > -1.0e38f) p2f = __expf(sc[pt][2] - m_new);
-      if (sc[pt][3] > -1.0e38f) p3f = __expf(sc[pt][3] - m_new);
-      psum += p0f + p1f + p2f + p3f;
-      ppk[pt * 2] = f32x2_to_bf16x2(p0f, p1f);
-      ppk[pt * 2 + 1] = f32x2_to_bf16x2(p2f, p3f);
-    }
-    psum += __shfl_xor(psum, 16, QSA_WAVE);
-    psum += __shfl_xor(psum, 32, QSA_WAVE);
-    lsum = lsum * alpha + psum;
+        for (int r = 0; r < 4; ++r) {
+          pr[r] = sc[pt][r] > -1.0e38f ? __expf(sc[pt][r] - m_new) : 0.f;
+          psum += pr[r];
+        }
+        ppk[pt * 2] = cvt_bf16x2(pr[0], pr[1]);
+        ppk[pt * 2 + 1] = cvt_bf16x2(pr[2], pr[3]);
+      }
+      psum += __shfl_xor(psum, 16, QSA_WAVE);
+      psum += __shfl_xor(psum, 32, QSA_WAVE);
+      lsum = lsum * alpha + psum;
 
-    // ---- PV: two 32-pos halves ---------------------------------------
-    // A-frag needs lane (head=col, hi) to hold P[head][pos = hi*8 + e]:
-    // packed pairs come from source lanes (same col) with hi' = (2*hi)&3
-    // and (2*hi+1)&3, tile = half*2 + (hi>>1).
+      // ---- PV: two 32-pos halves ---------------------------------------
+      // A-frag needs lane (head=col, hi) to hold P[head][pos = hi*8 + e]:
+      // packed pairs come from source lanes (same col) with hi' = (2*hi)&3
+      // and (2*hi+1)&3, tile = half*2 + (hi>>1).  __shfl evaluates its value
+      // in EACH lane and a register index has to be a constant: shuffle both
+      // candidate tiles' registers and select by hi.
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      // lane (col, hi) needs P[head=col][pos = half*32 + hi*8 + e]:
-      // tile T = half*2 + (hi>>1), quads (hi&1)*2 and (hi&1)*2+1 — i.e.
-      // source lanes (col, g) with g = (2*hi)&3 and (2*hi+1)&3.  __shfl
-      // evaluates the value expression in EACH lane, so the register
-      // index must be compile-time: shuffle both candidate tiles'
-      // packed regs and select by hi (guide rule 20: runtime-indexed
-      // arrays spill to scratch; and a runtime index would read the
-      // SOURCE lane's differently-computed tile).
-      const int src_a = col + (((2 * hi) & 3) << 4);
-      const int src_b = col + (((2 * hi + 1) & 3) << 4);
-      const int tA = half * 2;           // tile for hi 0,1
-      const int tB = half * 2 + 1;       // tile for hi 2,3
-      const unsigned int a0A = __shfl(ppk[tA * 2], src_a, QSA_WAVE);
-      const unsigned int a1A = __shfl(ppk[tA * 2 + 1], src_a, QSA_WAVE);
-      const unsigned int b0A = __shfl(ppk[tA * 2], src_b, QSA_WAVE);
-      const unsigned int b1A = __shfl(ppk[tA * 2 + 1], src_b, QSA_WAVE);
-      const unsigned int a0B = __shfl(ppk[tB * 2], src_a, QSA_WAVE);
-      const unsigned int a1B = __shfl(ppk[tB * 2 + 1], src_a, QSA_WAVE);
-      const unsigned int b0B = __shfl(ppk[tB * 2], src_b, QSA_WAVE);
-      const unsigned int b1B = __shfl(ppk[tB * 2 + 1], src_b, QSA_WAVE);
-      const bool lo = hi < 2;
-      bf16x8_a pa;
-      unsigned int* pa_u = reinterpret_cast<unsigned int*>(&pa);
-      pa_u[0] = lo ? a0A : a0B;
-      pa_u[1] = lo ? a1A : a1B;
-      pa_u[2] = lo ? b0A : b0B;
-      pa_u[3] = lo ? b1A : b1B;
+      for (int half = 0; half < 2; ++half) {
+        const int src_a = col + (((2 * hi) & 3) << 4);
+        const int src_b = col + (((2 * hi + 1) & 3) << 4);
+        const int tA = half * 2;           // tile for hi 0,1
+        const int tB = half * 2 + 1;       // tile for hi 2,3
+        const unsigned int a0A = __shfl(ppk[tA * 2], src_a, QSA_WAVE);
+        const unsigned int a1A = __shfl(ppk[tA * 2 + 1], src_a, QSA_WAVE);
+        const unsigned int b0A = __shfl(ppk[tA * 2], src_b, QSA_WAVE);
+        const unsigned int b1A = __shfl(ppk[tA * 2 + 1], src_b, QSA_WAVE);
+        const unsigned int a0B = __shfl(ppk[tB * 2], src_a, QSA_WAVE);
+        const unsigned int a1B = __shfl(ppk[tB * 2 + 1], src_a, QSA_WAVE);
+        const unsigned int b0B = __shfl(ppk[tB * 2], src_b, QSA_WAVE);
+        const unsigned int b1B = __shfl(ppk[tB * 2 + 1], src_b, QSA_WAVE);
+        const bool lo = hi < 2;
+        const u32x4_v pu = {lo ? a0A : a0B, lo ? a1A : a1B, lo ? b0A : b0B,
+                            lo ? b1A : b1B};
+        const bf16x8_a pa = __builtin_bit_cast(bf16x8_a, pu);
 #pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) {
-        // B-frag: lane holds V^T[pos = half*32 + hi*8 + e][d = dt*16+col]
-        // = vc[.., d, pos]: 16 B at (d*64 + half*32 + hi*8)
-        const bf16x8_a vf = *reinterpret_cast<const bf16x8_a*>(
-            vbase + ((long long)(dt * 16 + col) * QSA_PAGE) + half * 32 +
-            hi * 8);
-        o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vf,
-                                                            o_acc[dt],
-                                                            0, 0, 0);
+        for (int dt = 0; dt < DTILES; ++dt)
+          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              pa, vf[half][dt], o_acc[dt], 0, 0, 0);
       }
+      page = next;
     }
   }
 
-  // ---- store partials: O C-layout row = head = hi*4 + r, col = dim ----
-  // lane (hi, col): holds O[head hi*4+r][d = dt*16 + col]
+  // ---- the waves of the block meet: O C-layout row = head = hi*4 + r -----
+  float* ml = smem + NW * R * D;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int head = hi * 4 + r;
-    if (head < R) {
-      float* po = part_o +
-          (((long long)b * QH + kvh * R + head) * NS + split) * D;
+    if (head < R)
 #pragma unroll
       for (int dt = 0; dt < DTILES; ++dt)
-        po[dt * 16 + col] = o_acc[dt][r];
+        smem[(wave * R + head) * D + dt * 16 + col] = o_acc[dt][r];
+  }
+  if (lane < 16) {
+    ml[wave * 16 + lane] = m;
+    ml[NW * 16 + wave * 16 + lane] = lsum;
+  }
+  __syncthreads();
+  for (int i = tid; i < R * D; i += NW * 64) {
+    const int head = i / D, d = i % D;
+    float M = -3.0e38f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml[w * 16 + head]);
+    float L = 0.f, acc = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float ls = ml[NW * 16 + w * 16 + head];
+      // a wave without keys: no weight, whatever M is
+      const float f = ls > 0.f ? __expf(ml[w * 16 + head] - M) : 0.f;
+      L += f * ls;
+      acc += f * smem[(w * R + head) * D + d];
+    }
+    const int qh = kvh * R + head;
+    if (p.NS == 1) {
+      const unsigned short v = cvt_bf16(L > 0.f ? acc / L : 0.f);
+      if (p.mt)
+        p.out[qsa_step_at(b, qh * D + d, p.mt)] = v;
+      else
+        p.out[((long long)b * p.QH + qh) * D + d] = v;
+    } else {
+      const long long at = ((long long)b * p.QH + qh) * p.NS + split;
+      p.part_o[at * D + d] = acc;
+      if (d == 0)
+        *reinterpret_cast<float2*>(p.part_ml + at * 2) = make_float2(M, L);
     }
   }
-  if (lane < R)
-    *reinterpret_cast<float2*>(pml_base + (long long)lane * NS * 2) =
-        make_float2(m, lsum);
 }
 
 template <int D>
 __global__ void __launch_bounds__(128)
 qsa_attn_reduce(const float* __restrict__ part_o,   // [rows, NS, D]
                 const float* __restrict__ part_ml,  // [rows, NS, 2]
-                unsigned short* __restrict__ out,   // [rows, D]
-                int NS) {
+                unsigned short* __restrict__ out,   // [rows, D], or packed
+                int NS, int QH, int mt) {
   const long long row = blockIdx.x;
   const int d = threadIdx.x;  // D threads
   const float* ml = part_ml + row * NS * 2;
   float M = -3.0e38f;
+#pragma unroll 4
   for (int s = 0; s < NS; ++s)
     if (ml[2 * s + 1] > 0.f) M = fmaxf(M, ml[2 * s]);
   float L = 0.f, acc = 0.f;
+#pragma unroll 4
   for (int s = 0; s < NS; ++s) {
     const float ls = ml[2 * s + 1];
-    if (ls <= 0.f) continue;
-    const float w = __expf(ml[2 * s] - M);
+    const float o = part_o[(row * NS + s) * D + d];
+    const float w = ls > 0.f ? __expf(ml[2 * s] - M) : 0.f;
     L += w * ls;
-    acc += w * part_o[(row * NS + s) * D + d];
+    acc += w * o;
   }
-  const float v = (L > 0.f) ? acc / L : 0.f;
-  out[row * D + d] = f32_to_bf16(v);
+  const unsigned short v = cvt_bf16((L > 0.f) ? acc / L : 0.f);
+  if (mt)
+    out[qsa_step_at((int)(row / QH), (int)(row % QH) * D + d, mt)] = v;
+  else
+    out[row * D + d] = v;
+}
+
+// Waves of a block and blocks per (row, kv head): one block of four waves where
+// the rows alone give every CU two, one of eight for few pages (a second launch
+// would cost more than it spreads); otherwise blocks of four until there are
+// 2048 waves.
+extern "C" void qsa_paged_attn_split(int B, int QH, int KVH, int max_pages,
+                                     int D, int* waves, int* splits) {
+  const long long heads = (long long)B * KVH;
+  const int lds = QH / KVH * D * 4;    // bytes per wave
+  *waves = 4;
+  *splits = 1;
+  if (heads >= 512) return;
+  if (max_pages <= 16 && 8 * lds <= 60 * 1024) {
+    *waves = max_pages <= 4 ? 4 : 8;
+    return;
+  }
+  const long long want = (2048 + 4 * heads - 1) / (4 * heads);
+  *splits = (int)std::max<long long>(
+      1, std::min<long long>(want, (max_pages + 3) / 4));
 }
 
 extern "C" void qsa_paged_attn_mfma_launch(
-    const unsigned short* q, const unsigned short* kc,
-    const unsigned short* vc, const int* block_table, const int* seq_lens,
+    const unsigned short* q, const unsigned short* k, const unsigned short* v,
+    unsigned short* kc, unsigned short* vc, const float* cos_t,
+    const float* sin_t, const int* block_table, const int* seq_lens,
     float* part_o, float* part_ml, unsigned short* out, float scale, int B,
-    int QH, int KVH, int max_pages, int D, long long qstride, int NS,
-    hipStream_t stream) {
-  const int nsb = (NS + 3) / 4;
-  dim3 grid(B * KVH * nsb);
-  dim3 block(256);
-  if (D == 128) {
-    hipLaunchKernelGGL((qsa_paged_attn_mfma<128>), grid, block, 0, stream,
-                       q, kc, vc, block_table, seq_lens, part_o, part_ml,
-                       scale, B, QH, KVH, max_pages, qstride, NS);
-    hipLaunchKernelGGL((qsa_attn_reduce<128>), dim3(B * QH), dim3(128), 0,
-                       stream, part_o, part_ml, out, NS);
-  } else if (D == 64) {
-    hipLaunchKernelGGL((qsa_paged_attn_mfma<64>), grid, block, 0, stream,
-                       q, kc, vc, block_table, seq_lens, part_o, part_ml,
-                       scale, B, QH, KVH, max_pages, qstride, NS);
-    hipLaunchKernelGGL((qsa_attn_reduce<64>), dim3(B * QH), dim3(64), 0,
-                       stream, part_o, part_ml, out, NS);
+    int QH, int KVH, int max_pages, int D, long long qstride,
+    long long kvstride, int waves, int NS, int mt, hipStream_t stream) {
+  const DecodeArgs p{q, kc, vc, block_table, seq_lens, part_o, part_ml, out,
+                     k, v, kc, vc, cos_t, sin_t, scale, QH, KVH, max_pages,
+                     NS, mt, qstride, kvstride};
+  const dim3 grid((unsigned)((long long)B * KVH * NS)), block(waves * 64);
+  if (grid.x == 0) return;
+  const size_t lds = sizeof(float) * waves * ((size_t)QH / KVH * D + 32);
+#define QSA_DECODE(DD, NW)                                                  \
+  if (D == DD && waves == NW) {                                             \
+    if (k)                                                                  \
+      hipLaunchKernelGGL((qsa_paged_attn_mfma<DD, NW, true>), grid, block,  \
+                         lds, stream, p);                                   \
+    else                                                                    \
+      hipLaunchKernelGGL((qsa_paged_attn_mfma<DD, NW, false>), grid, block, \
+                         lds, stream, p);                                   \
   }
+  QSA_DECODE(128, 4) QSA_DECODE(128, 8) QSA_DECODE(64, 4) QSA_DECODE(64, 8)
+#undef QSA_DECODE
+  if (NS == 1) return;
+  if (D == 128)
+    hipLaunchKernelGGL((qsa_attn_reduce<128>), dim3(B * QH), dim3(128), 0,
+                       stream, part_o, part_ml, out, NS, QH, mt);
+  else
+    hipLaunchKernelGGL((qsa_attn_reduce<64>), dim3(B * QH), dim3(64), 0,
+                       stream, part_o, part_ml, out, NS, QH, mt);
 }
 
 // ---------------------------------------------------------------------------
@@ -449,7 +573,9 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
   constexpr int L = D / 32;            // 16 B loads per thread, K and V each
   __shared__ __attribute__((aligned(16))) unsigned short kt[64 * D];
   __shared__ __attribute__((aligned(16))) unsigned short vt[64 * D];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // a scalar: branches on it skip MFMAs, which ignore disabled lanes
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
   const int R = QH / KVH;
   const int g = blockIdx.x % KVH;

@@ -1,0 +1,237 @@
+// Weight-streaming decode GEMM for CDNA4 (gfx950), shared by the bf16 and the
+// fp8 form: C[M,N] = A[M,K] @ W[N,K]^T for M <= 32 rows.
+//
+// The projections of a decoding step read every weight once, so the weight
+// stream is the bound and the rest has to stay out of its way:
+//   * W is packed once into MFMA fragments (layouts in skinny_gemm.hip and
+//     skinny_gemm_fp8.hip): a wave instruction reads 1 KiB in a row.
+//   * A block owns TILES tiles of 16 columns; its waves take the 64-deep steps
+//     of K in turn, so that the block reads its stream front to back, and keep
+//     two groups of U steps in flight.  They meet in LDS at the end.
+//   * A is tiny and L2 holds it, but a row-major fragment touches 16 lines
+//     where W's takes 8, and at 16 rows those lookups, not the weights, set
+//     the pace (a tile per block: 28672 x 4096 fp8 in 25 us at 1 row, 38 us at
+//     16).  From 5 rows on the decoder keeps its activations packed in
+//     fragments like W (PACK: [K/32, MT, 64 lanes, 8]); producers store them
+//     so.  MT row tiles of 16: one for up to 16 rows, two above.
+//   * Row-major rows beyond M shadow row M-1, packed ones are whatever the
+//     buffer holds; they meet no other row and are never stored.
+// What surrounds a projection in the decoder is done on the way, since every
+// launch costs a few microseconds of a step that is made of hundreds:
+//   NORM  A is x * w of an rms norm; the row factor 1/rms meets the sums at the
+//         end.  The sum of squares of a row comes in parts from whoever wrote
+//         the row (ss_in [32, parts4], parts4 = parts rounded up to 4).
+//   GLU   W's rows are [gate; up]: a block takes the same columns of both and
+//         stores silu(gate) * up, packed if A is.
+//   RES   the result is added to the residual stream in place; the next norm's
+//         operand (new row * norm_w, packed if A is) goes to `next`, the
+//         sums of squares of the new rows to ss_out, one part per tile.
+// (Multiplying by w on the way in instead cost 20 us of 25 at 28672 x 4096:
+// every block redoes it, and its loads take the place of the stream's.)
+#pragma once
+
+#include "lm_common.h"
+
+struct SkinnyArgs {
+  const bf16_t* A;
+  const u32x4_v* W;
+  const float* scale;                  // fp8: per output column
+  bf16_t* C;                           // result, or the residual stream
+  bf16_t* next;
+  const bf16_t* norm_w;
+  const float* ss_in;
+  float* ss_out;
+  int M, N, parts;
+  long long K, lda;
+  float eps;
+};
+
+// 8 fp8 bytes (as 2 dwords) -> bf16x8 fragment, exact: every e4m3 value is a
+// bf16 value, so cutting the f32 down loses nothing
+__device__ __forceinline__ bf16x8_v fp8x8_to_bf16x8(unsigned int a,
+                                                    unsigned int b) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  const f32x2 f0 = __builtin_amdgcn_cvt_pk_f32_fp8(a, false);
+  const f32x2 f1 = __builtin_amdgcn_cvt_pk_f32_fp8(a, true);
+  const f32x2 f2 = __builtin_amdgcn_cvt_pk_f32_fp8(b, false);
+  const f32x2 f3 = __builtin_amdgcn_cvt_pk_f32_fp8(b, true);
+  auto high = [](f32x2 f) {
+    return __builtin_amdgcn_perm(__float_as_uint(f.y), __float_as_uint(f.x),
+                                 0x07060302u);
+  };
+  const u32x4_v u = {high(f0), high(f1), high(f2), high(f3)};
+  return __builtin_bit_cast(bf16x8_v, u);
+}
+
+// place of element k of a row in packed activations
+__device__ __forceinline__ long long packed_at(int row, int k, int mt) {
+  return ((long long)(k >> 5) * mt + (row >> 4)) * 512 +
+         ((row & 15) + ((k >> 3) & 3) * 16) * 8 + (k & 7);
+}
+
+template <int WAVES, int TILES, int MT, bool FP8, bool PACK, bool NORM,
+          bool GLU, bool RES>
+__device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
+  constexpr int WL = FP8 ? 1 : 2;      // 16 B loads of a tile per step
+  constexpr int PER = TILES * WL * 4 + MT * 8;
+  constexpr int U = PER <= 12 ? 4 : PER <= 24 ? 2 : 1;
+  __shared__ float red[WAVES][TILES * MT * 4][64];
+  __shared__ float inv_s[32];
+  const int tid = threadIdx.x, lane = tid & 63;
+  // the wave's number as a scalar: branches on it must skip MFMAs, which
+  // would otherwise run with no lane enabled and still add up
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, hi = lane >> 4;
+  const int steps = (int)(p.K >> 6);   // K % 64 == 0
+
+  // row factors: the parts' loads go ahead of the stream, a row per wave
+  constexpr int NR = NORM ? MT * 16 / WAVES : 1;
+  f32x4_v sv[NR];
+  const int p4 = (p.parts + 3) & ~3;
+  if constexpr (NORM)
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int row = wave + i * WAVES;
+      sv[i] = *reinterpret_cast<const f32x4_v*>(
+          p.ss_in + (row < p.M ? row : 0) * p4 + (lane * 4 < p4 ? lane * 4 : 0));
+    }
+
+  // GLU: tiles 2j and 2j+1 are gate and up of the same 16 columns
+  auto tile_of = [&](int t) {
+    return GLU ? (int)blockIdx.x * (TILES / 2) + t / 2 +
+                     (t & 1) * (p.N >> 5)
+               : (int)blockIdx.x * TILES + t;
+  };
+  const u32x4_v* wp[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t)
+    wp[t] = p.W + (long long)tile_of(t) * steps * (64 * WL) + col * 4 + hi;
+  const bf16_t* ap[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    ap[m] = PACK ? p.A + m * 512 + lane * 8
+                 : p.A + (long long)min(m * 16 + col, p.M - 1) * p.lda +
+                       hi * 8;
+
+  struct Group {
+    u32x4_v w[U][TILES][WL];
+    bf16x8_v a[U][MT][2];
+  };
+  f32x4_v acc[TILES][MT];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+
+  auto load = [&](Group& g, int base) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long s = min(base + u * WAVES, steps - 1);
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int i = 0; i < WL; ++i)
+          g.w[u][t][i] = wp[t][s * (64 * WL) + i * 64];
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          g.a[u][m][i] = *reinterpret_cast<const bf16x8_v*>(
+              ap[m] + (PACK ? (s * 2 + i) * (MT * 512) : s * 64 + i * 32));
+    }
+  };
+  auto compute = [&](Group& g, int base) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (base + u * WAVES >= steps) break;       // uniform over the wave
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          bf16x8_v w;
+          if constexpr (FP8)
+            w = fp8x8_to_bf16x8(g.w[u][t][0][2 * i], g.w[u][t][0][2 * i + 1]);
+          else
+            w = __builtin_bit_cast(bf16x8_v, g.w[u][t][i]);
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            acc[t][m] = mfma_bf16(g.a[u][m][i], w, acc[t][m]);
+        }
+    }
+  };
+
+  Group g0, g1;
+  constexpr int ROUND = WAVES * U;
+  load(g0, wave);
+  load(g1, wave + ROUND);
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int row = wave + i * WAVES;
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += lane * 4 + e < p.parts ? sv[i][e] : 0.f;
+      for (int k = 256 + lane; k < p.parts; k += 64)
+        s += p.ss_in[(row < p.M ? row : 0) * p4 + k];
+      s = wave_reduce_sum(s);
+      if (lane == 0) inv_s[row] = rsqrtf(s / (float)p.K + p.eps);
+    }
+  }
+  for (int base = wave; base < steps; base += 2 * ROUND) {
+    compute(g0, base);
+    if (base + 2 * ROUND < steps) load(g0, base + 2 * ROUND);
+    compute(g1, base + ROUND);
+    if (base + 3 * ROUND < steps) load(g1, base + 3 * ROUND);
+  }
+
+#pragma unroll
+  for (int t = 0; t < TILES; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave][(t * MT + m) * 4 + r][lane] = acc[t][m][r];
+  __syncthreads();
+
+  constexpr int OUT = (GLU ? TILES / 2 : TILES) * MT * 256;
+  for (int idx = tid; idx < OUT; idx += WAVES * 64) {
+    const int r = (idx >> 6) & 3, m = (idx >> 8) % MT, j = (idx >> 8) / MT;
+    const int row = m * 16 + (lane >> 4) * 4 + r;
+    auto total = [&](int t) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) v += red[w][(t * MT + m) * 4 + r][lane];
+      if constexpr (FP8) v *= p.scale[tile_of(t) * 16 + col];
+      return v;
+    };
+    const float inv = NORM ? inv_s[row] : 1.f;
+    const int ncol = tile_of(GLU ? 2 * j : j) * 16 + col;
+    const bool live = row < p.M;
+    auto place = [&](int width) {
+      return PACK ? packed_at(row, ncol, MT) : (long long)row * width + ncol;
+    };
+    if constexpr (GLU) {
+      const float g = total(2 * j) * inv, u = total(2 * j + 1) * inv;
+      if (live)
+        p.C[place(p.N >> 1)] = cvt_bf16(g / (1.f + __expf(-g)) * u);
+    } else if constexpr (RES) {
+      bf16_t* at = p.C + (long long)(live ? row : 0) * p.N + ncol;
+      const float v = bf16_to_f32(*at) + total(j);
+      const bf16_t b = cvt_bf16(v);
+      if (live) {
+        *at = b;
+        p.next[place(p.N)] = cvt_bf16(bf16_to_f32(b) *
+                                      bf16_to_f32(p.norm_w[ncol]));
+      }
+      float q = v * v;
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) q += __shfl_xor(q, o, 16);
+      const int parts = p.N >> 4;
+      if (live && col == 0)
+        p.ss_out[row * ((parts + 3) & ~3) + (ncol >> 4)] = q;
+    } else {
+      const float v = total(j) * inv;
+      if (live) p.C[(long long)row * p.N + ncol] = cvt_bf16(v);
+    }
+  }
+}

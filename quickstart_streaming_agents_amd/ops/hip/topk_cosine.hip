@@ -59,7 +59,8 @@ qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
               int* __restrict__ cand_ids,         // [Q, nblk, k]
               int Qn, int N, int D, int k) {
   __shared__ float part[4][16 * T][QSA_TOPK_QG + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
   const int doc0 = blockIdx.x * 16 * T, q0 = blockIdx.y * QSA_TOPK_QG;
 

@@ -446,6 +446,142 @@ def test_skinny_gemm_fp8_gpu_pack_matches_cpu_pack():
     assert frac_diff < 0.02, f"packs differ on {frac_diff:.1%} of bytes"
 
 
+def _step_rows(x):
+    """[M, K] in the layout that decoding steps pass between projections."""
+    M, K = x.shape
+    if M <= 4:
+        return x.contiguous()
+    mt = 1 if M <= 16 else 2
+    p = torch.full((mt * 16, K), float("nan"), dtype=x.dtype, device=x.device)
+    p[:M] = x
+    return p.view(mt, 16, K // 32, 4, 8).permute(2, 0, 3, 1, 4) \
+        .reshape(K // 32, mt, 64, 8).contiguous()
+
+
+def _from_step_rows(x, M):
+    if x.dim() == 2:
+        return x
+    kb, mt = x.shape[:2]
+    return x.view(kb, mt, 4, 16, 8).permute(1, 3, 0, 2, 4) \
+        .reshape(mt * 16, kb * 32)[:M]
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(64, 256), (192, 768), (4096, 8448),
+                                 (65_600, 512), (6208, 2304)])
+def test_skinny_fp8_forms(M, N, K):
+    """Plain, normed, gated and residual forms against f64 on the
+    dequantized weights; rows that do not exist hold NaN."""
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    from quickstart_streaming_agents_amd.ops import ext
+    torch.manual_seed(M + N + K)
+    w = torch.randn(N, K, device=dev(), dtype=torch.bfloat16) * K ** -0.5
+    packed = D.pack_weight_fp8(w)
+    W = D.unpack_weight_fp8(*packed, N, K).double()
+    x = torch.randn(M, K + 64, device=dev(), dtype=torch.bfloat16)[:, :K]
+    # operands are exact here; results are rounded to bf16 (2^-9 each)
+    tol = 2 ** -8
+
+    def close(got, want):
+        err = (got.double() - want).norm() / want.norm()
+        assert err < tol, float(err)
+
+    y = x.double() @ W.T
+    close(ext().skinny_gemm_fp8(x, *packed, N, K), y)
+    xs = _step_rows(x)
+    eps = 1e-5
+    for parts in (1, 3, 260):
+        p4 = (parts + 3) // 4 * 4
+        ss = torch.full((32, p4), float("nan"), device=dev())
+        share = torch.rand(M, parts, device=dev())
+        ss[:M, :parts] = share / share.sum(1, keepdim=True) \
+            * x.float().square().sum(1, keepdim=True)
+        h = y * torch.rsqrt(x.double().square().mean(1, keepdim=True) + eps)
+        close(D.norm_linear_fp8(xs, ss, parts, M, eps, packed, N, K), h)
+        g, u = h.chunk(2, 1)
+        act = D.norm_linear_fp8(xs, ss, parts, M, eps, packed, N, K, glu=True)
+        close(_from_step_rows(act, M), torch.nn.functional.silu(g) * u)
+    res = torch.randn(M, N, device=dev(), dtype=torch.bfloat16)
+    nw = (1 + 0.2 * torch.randn(N, device=dev())).bfloat16()
+    want = res.double() + y
+    nxt, out = D.linear_residual_fp8(xs, packed, N, K, res, nw)
+    close(res, want)
+    assert torch.equal(_from_step_rows(nxt, M),
+                       (res.float() * nw.float()).bfloat16())
+    sums = out[:M, :N // 16].double().sum(1)
+    assert ((sums - want.square().sum(1)).abs()
+            < tol * want.square().sum(1)).all()
+
+
+@pytest.mark.parametrize("B,QH,KVH,D,longest", [
+    (1, 32, 8, 64, 700), (1, 32, 8, 128, 60), (4, 32, 8, 128, 1100),
+    (5, 32, 8, 128, 900), (17, 16, 1, 64, 2000), (32, 28, 4, 128, 300),
+    (70, 32, 8, 128, 400), (3, 4, 4, 64, 4500)])
+def test_paged_attn_step(ext, B, QH, KVH, D, longest):
+    """Rotation, append and attention in one against the separate ones, at
+    page edges; a row not in use leaves everything alone."""
+    g = torch.Generator().manual_seed(B + longest)
+    lens = torch.randint(1, longest + 1, (B,), generator=g)
+    lens[:3] = torch.tensor([longest, 64, 65])[:B].clamp(max=longest)
+    if B > 3:
+        lens[3] = 0
+    kc, vc, bt = _make_paged_kv(B, KVH, D, lens.tolist(),
+                                sum(-(-n // 64) for n in lens.tolist()) + 1)
+    kc2, vc2 = kc.clone(), vc.clone()
+    rot = torch.rand(longest + 1, D // 2, generator=g) * 6.28
+    cos, sin = rot.cos().to(dev()), rot.sin().to(dev())
+    qkv = torch.randn(B, (QH + 2 * KVH) * D, generator=g).bfloat16().to(dev())
+    sl = lens.int().to(dev())
+
+    def split(t):
+        q, k, v = t.split([QH * D, KVH * D, KVH * D], 1)
+        return (q.view(B, QH, D), k.view(B, KVH, D), v.view(B, KVH, D))
+
+    kept = qkv.clone()
+    out = ext.paged_attn_step(*split(qkv), kc, vc, cos, sin, bt, sl,
+                              D ** -0.5, False)
+    assert torch.equal(qkv, kept)
+    q, k, v = split(qkv)
+    ext.rope_kv_append(q, k, v, kc2, vc2, cos, sin, bt, sl)
+    assert torch.equal(vc, vc2)
+    # products of the rotation may be fused differently: one bf16 step
+    assert ((kc.float() - kc2.float()).abs()
+            <= 2 ** -7 * kc2.float().abs() + 1e-6).all()
+    ref = cpu_ref.paged_attn_ref(q.cpu(), kc2.cpu(), vc2.cpu(), bt.cpu(),
+                                 sl.cpu(), D ** -0.5)
+    torch.testing.assert_close(out.float().cpu(), ref, atol=2e-2, rtol=2e-2)
+    if B <= 32:
+        q, k, v = split(kept)
+        step = ext.paged_attn_step(q, k, v, kc, vc, cos, sin, bt, sl,
+                                   D ** -0.5, True)
+        step = step.view(B, -1) if step.dim() == 3 else step
+        assert torch.equal(_from_step_rows(step, B), out.view(B, -1))
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(16, 256), (48, 768), (4096, 8192)])
+def test_skinny_bf16_rows(ext, M, N, K):
+    torch.manual_seed(M + N)
+    a = torch.randn(M, K, device=dev(), dtype=torch.bfloat16)
+    w = torch.randn(N, K, device=dev(), dtype=torch.bfloat16) * K ** -0.5
+    out = ext.skinny_gemm(a, ext.pack_weight_frag(w), N, K)
+    want = a.double() @ w.double().T
+    # exact products, f32 sums; the result is rounded to bf16
+    assert (out.double() - want).norm() < 2 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 17])
+def test_embed_rows(ext, M):
+    embed = torch.randn(100, 288, device=dev(), dtype=torch.bfloat16)
+    w = torch.randn(288, device=dev()).bfloat16()
+    tok = torch.tensor([0, 99, 7, 7, 31] * 4, device=dev())[:M]
+    res, nxt, ss = ext.embed_rows(embed, tok, w)
+    assert torch.equal(res, embed[tok])
+    assert torch.equal(_from_step_rows(nxt, M),
+                       (res.float() * w.float()).bfloat16())
+    torch.testing.assert_close(ss[:M, 0], res.float().square().sum(1))
+
+
 def test_llama_decode_uses_fp8_path():
     """The flagship decode path must run the fp8 kernel by default (the
     driver's native-code check: no silent bf16/rocBLAS fallback)."""

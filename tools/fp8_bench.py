@@ -53,16 +53,14 @@ def main():
         t_bf = timeit(lambda: ext().skinny_gemm(a, wf, N, K))
         t_f8 = timeit(lambda: ext().skinny_gemm_fp8(a, qf, s, N, K))
         if os.environ.get("QSA_FP8_SWEEP") == "1":
-            for waves, tiles, ntl in [(8, 1, 0), (8, 1, 1), (8, 2, 0),
-                                      (8, 4, 0), (8, 4, 1), (8, 8, 0),
-                                      (16, 1, 0), (16, 2, 0), (16, 4, 0),
-                                      (4, 4, 0), (4, 8, 0), (2, 8, 0)]:
+            for waves, tiles in [(4, 1), (8, 1), (16, 1), (4, 2), (8, 2),
+                                 (2, 4), (4, 4), (8, 4)]:
                 if N % (16 * tiles):
                     continue
                 try:
                     t = timeit(lambda: ext().skinny_gemm_fp8_probe(
-                        a, qf, s, N, K, waves, tiles, ntl), reps=20)
-                    print(f"    probe {name} w{waves} t{tiles} nt{ntl}: "
+                        a, qf, s, N, K, waves, tiles), reps=20)
+                    print(f"    probe {name} w{waves} t{tiles}: "
                           f"{t:.1f} us ({(N*K)/(t*1e-6)/1e9:.0f} GB/s)",
                           file=sys.stderr)
                 except Exception as e:
