@@ -87,43 +87,117 @@ class EmbeddingEncoder:
     # -- varlen attention plumbing (GPU path) ------------------------------
     QROWS = 64      # query tokens per attention block: one 16-row tile a wave
 
-    def _attn_maps(self, n: int, L: int, lens: torch.Tensor):
-        """Page table / q-block maps for the bidirectional varlen kernel.
-        Items sit at padded offsets i*L; pages are preallocated per item
-        over the PADDED length (pad slots are never read: item_len bounds
-        the key range)."""
+    def _embed_rows(self, enc: list[list[int]]) -> torch.Tensor:
+        """Mean-pooled final states [n, hidden] f32 of the token lists, all
+        rows in one concatenation without padding.  Keys and values go to
+        scratch pages, preallocated per item (slots nobody writes are never
+        used: item_len bounds the key range)."""
+        import numpy as np
+
+        from .layers import ints_to_device
+        c, dev = self.cfg, self.device
+        lens = np.array([len(x) for x in enc])
+        n, T = len(enc), int(lens.sum())
+        off = np.cumsum(lens) - lens
+        item = np.repeat(np.arange(n), lens)
+        pos = np.arange(T) - off[item]
+        ppi = -(-int(lens.max()) // 64)      # pages per item
+        nqb = -(-lens // self.QROWS)
+        qb_item = np.repeat(np.arange(n), nqb)
+        qb_pos0 = (np.arange(int(nqb.sum()))
+                   - (np.cumsum(nqb) - nqb)[qb_item]) * self.QROWS
+        (toks, positions, slots, bt, qb_item, qb_pos0, off, lens_t,
+         start) = ints_to_device(
+            dev, np.concatenate(enc), pos, item * ppi * 64 + pos,
+            np.arange(n * ppi), qb_item, qb_pos0, off, lens, np.zeros(n))
+        bt = bt.view(n, ppi)
+        kc = torch.empty(n * ppi, c.n_heads, c.d_head // 8, 64, 8,
+                         dtype=self.dtype, device=dev)
+        vc = torch.empty(n * ppi, c.n_heads, c.d_head, 64, dtype=self.dtype,
+                         device=dev)
+        res = self.tok_embed.index_select(0, toks)
+        mlp_out = None
+        for Ly in self.layers:
+            if mlp_out is None:
+                h = D.rmsnorm(res, Ly["attn_norm"], c.norm_eps)
+            else:
+                h = D.rmsnorm_residual(mlp_out, res, Ly["attn_norm"],
+                                       c.norm_eps)
+            q, k, v = F.linear(h, Ly["wqkv"]) \
+                .view(T, 3, c.n_heads, c.d_head).unbind(1)
+            D.rope_kv_scatter(q, k, v, kc, vc, self.rope_cos, self.rope_sin,
+                              positions, slots)
+            # bidirectional varlen MFMA flash attention (CAUSAL=false)
+            attn = D.ext().paged_attn_prefill(
+                q, kc, vc, bt, qb_item, qb_pos0, off, start, lens_t,
+                self.scale, False, self.QROWS)
+            o = F.linear(attn, Ly["wo"])
+            h = D.rmsnorm_residual(o, res, Ly["mlp_norm"], c.norm_eps)
+            gu = F.linear(h, Ly["wgu"])
+            act = D.swiglu(gu[:, :c.ffn], gu[:, c.ffn:])
+            mlp_out = F.linear(act, Ly["wdown"])
+        final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm,
+                                     c.norm_eps)
+        return D.ext().mean_rows(final_h, off, lens_t)
+
+    def _embed_padded(self, enc: list[list[int]]) -> torch.Tensor:
+        """The same by a padded batch and a materialized softmax (CPU)."""
         c = self.cfg
-        ppi = (L + 63) // 64            # pages per item
-        bt = (torch.arange(n * ppi, dtype=torch.int32, device=self.device)
-              .reshape(n, ppi).contiguous())
-        # pad rows scatter to a TRASH page no block_table references:
-        # their k/v are downstream of an unwritten attention-output row
-        # (possibly NaN), and the PV MFMA reads FULL 64-slot pages before
-        # masking — 0 * NaN would poison valid rows from layer 2 on
-        j = torch.arange(L, device=self.device).unsqueeze(0).expand(n, L)
-        lens_d = lens.to(self.device).unsqueeze(1)
-        base = (torch.arange(n, device=self.device) * ppi * 64) \
-            .unsqueeze(1) + j
-        trash = n * ppi * 64
-        slots = torch.where(j < lens_d, base, trash) \
-            .to(torch.int32).reshape(-1).contiguous()
-        qb_item, qb_pos0 = [], []
-        lens_l = lens.tolist()
-        for i in range(n):
-            for p0 in range(0, max(int(lens_l[i]), 1), self.QROWS):
-                qb_item.append(i)
-                qb_pos0.append(p0)
-        dev = self.device
-        mk = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
-        return {
-            "n_pages": n * ppi + 1,     # +1 trash page for pad rows
-            "block_table": bt,
-            "slots": slots,
-            "qb_item": mk(qb_item), "qb_pos0": mk(qb_pos0),
-            "item_off": mk([i * L for i in range(n)]),
-            "item_start": mk([0] * n),
-            "item_len": mk([max(int(x), 1) for x in lens_l]),
-        }
+        n = len(enc)
+        L = max(len(x) for x in enc)
+        T = n * L
+        toks = torch.zeros(n, L, dtype=torch.int64, device=self.device)
+        for i, x in enumerate(enc):
+            toks[i, :len(x)] = torch.tensor(x, dtype=torch.int64)
+        lens = torch.tensor([len(x) for x in enc], dtype=torch.int32,
+                            device=self.device)
+        positions = torch.arange(L, dtype=torch.int32, device=self.device) \
+            .repeat(n).contiguous()
+        # per-row score limits: row = (seq, head, qpos) -> seq len
+        row_limits = lens.repeat_interleave(c.n_heads * L).contiguous()
+        res = self.tok_embed.index_select(0, toks.reshape(-1)).contiguous()
+        h = None
+        mlp_out = None
+        for li, Ly in enumerate(self.layers):
+            if li == 0:
+                h = D.rmsnorm(res, Ly["attn_norm"], c.norm_eps)
+            else:
+                h = D.rmsnorm_residual(mlp_out, res, Ly["attn_norm"],
+                                       c.norm_eps)
+            qkv = F.linear(h, Ly["wqkv"])
+            A = c.attn_dim
+            q = qkv[:, :A].reshape(T, c.n_heads, c.d_head).contiguous()
+            k = qkv[:, A:2 * A].reshape(T, c.n_heads, c.d_head).contiguous()
+            v = qkv[:, 2 * A:].reshape(T, c.n_heads, c.d_head).contiguous()
+            D.rope_inplace(q, k, self.rope_cos, self.rope_sin, positions)
+            # [n*heads, L, D] padded bmm reference
+            qh = q.reshape(n, L, c.n_heads, c.d_head).permute(0, 2, 1, 3) \
+                .reshape(n * c.n_heads, L, c.d_head)
+            kh = k.reshape(n, L, c.n_heads, c.d_head).permute(0, 2, 1, 3) \
+                .reshape(n * c.n_heads, L, c.d_head)
+            vh = v.reshape(n, L, c.n_heads, c.d_head).permute(0, 2, 1, 3) \
+                .reshape(n * c.n_heads, L, c.d_head)
+            scores = (torch.bmm(qh.float(), kh.float().transpose(1, 2))
+                      * self.scale).reshape(n * c.n_heads * L, L) \
+                .contiguous()
+            D.softmax_rows_(scores, 0, False, 0, row_limits)
+            attn = torch.bmm(scores.reshape(n * c.n_heads, L, L),
+                             vh.float())
+            attn = attn.reshape(n, c.n_heads, L, c.d_head) \
+                .permute(0, 2, 1, 3).reshape(T, A).to(self.dtype) \
+                .contiguous()
+            o = F.linear(attn, Ly["wo"])
+            h = D.rmsnorm_residual(o, res, Ly["mlp_norm"], c.norm_eps)
+            gu = F.linear(h, Ly["wgu"])
+            act = D.swiglu(gu[:, :c.ffn], gu[:, c.ffn:])
+            mlp_out = F.linear(act, Ly["wdown"])
+        final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm,
+                                     c.norm_eps)
+        hs = final_h.reshape(n, L, c.hidden).float()
+        valid = (torch.arange(L, device=self.device).unsqueeze(0)
+                 < lens.unsqueeze(1)).unsqueeze(-1)
+        hs = torch.where(valid, hs, torch.zeros((), device=self.device))
+        return hs.sum(dim=1) / valid.float().sum(dim=1).clamp(min=1)
 
     @torch.no_grad()
     def embed_batch(self, texts: list[str]):
@@ -133,88 +207,10 @@ class EmbeddingEncoder:
         c = self.cfg
         enc = [self.tokenizer.encode(t)[: c.max_pos] or [BpeTokenizer.BOS]
                for t in texts]
-        n = len(enc)
-        L = max(len(x) for x in enc)
-        toks = torch.zeros(n, L, dtype=torch.int64, device=self.device)
-        lens = torch.zeros(n, dtype=torch.int32)
-        for i, x in enumerate(enc):
-            toks[i, :len(x)] = torch.tensor(x, dtype=torch.int64,
-                                            device=self.device)
-            lens[i] = len(x)
-        lens_dev = lens.to(self.device)
-        positions = torch.arange(L, dtype=torch.int32, device=self.device) \
-            .repeat(n).contiguous()
-        T = n * L
-
+        # mean over the tokens, project, L2-normalize
         from ..ops import have_ext
-        use_hip = self._use_hip and have_ext()
-        if use_hip:
-            maps = self._attn_maps(n, L, lens)
-            # zeros, not empty: the attention kernel's MFMAs read FULL
-            # 64-slot pages before masking; garbage V in never-scattered
-            # tail slots would 0*inf=NaN the PV accumulate
-            kc = torch.zeros(maps["n_pages"], c.n_heads, c.d_head // 8, 64,
-                             8, dtype=self.dtype, device=self.device)
-            vc = torch.zeros(maps["n_pages"], c.n_heads, c.d_head, 64,
-                             dtype=self.dtype, device=self.device)
-        else:
-            # per-row score limits: row = (seq, head, qpos) -> seq len
-            row_limits = lens_dev.repeat_interleave(c.n_heads * L) \
-                .contiguous()
-
-        res = self.tok_embed.index_select(0, toks.reshape(-1)).contiguous()
-        h = None
-        mlp_out = None
-        for li, Ly in enumerate(self.layers):
-            if li == 0:
-                h = D.rmsnorm(res, Ly["attn_norm"], c.norm_eps)
-            else:
-                h = D.rmsnorm_residual(mlp_out, res, Ly["attn_norm"], c.norm_eps)
-            qkv = F.linear(h, Ly["wqkv"])
-            A = c.attn_dim
-            q = qkv[:, :A].reshape(T, c.n_heads, c.d_head).contiguous()
-            k = qkv[:, A:2 * A].reshape(T, c.n_heads, c.d_head).contiguous()
-            v = qkv[:, 2 * A:].reshape(T, c.n_heads, c.d_head).contiguous()
-            D.rope_inplace(q, k, self.rope_cos, self.rope_sin, positions)
-            if use_hip:
-                # bidirectional varlen MFMA flash attention (CAUSAL=false)
-                D.kv_scatter(k, v, kc, vc, maps["slots"])
-                attn = D.ext().paged_attn_prefill(
-                    q, kc, vc, maps["block_table"], maps["qb_item"],
-                    maps["qb_pos0"], maps["item_off"], maps["item_start"],
-                    maps["item_len"], self.scale, False, self.QROWS)
-                attn = attn.contiguous()
-            else:
-                # [n*heads, L, D] padded bmm reference
-                qh = q.reshape(n, L, c.n_heads, c.d_head).permute(0, 2, 1, 3) \
-                    .reshape(n * c.n_heads, L, c.d_head)
-                kh = k.reshape(n, L, c.n_heads, c.d_head).permute(0, 2, 1, 3) \
-                    .reshape(n * c.n_heads, L, c.d_head)
-                vh = v.reshape(n, L, c.n_heads, c.d_head).permute(0, 2, 1, 3) \
-                    .reshape(n * c.n_heads, L, c.d_head)
-                scores = (torch.bmm(qh.float(), kh.float().transpose(1, 2))
-                          * self.scale).reshape(n * c.n_heads * L, L) \
-                    .contiguous()
-                D.softmax_rows_(scores, 0, False, 0, row_limits)
-                attn = torch.bmm(scores.reshape(n * c.n_heads, L, L),
-                                 vh.float())
-                attn = attn.reshape(n, c.n_heads, L, c.d_head) \
-                    .permute(0, 2, 1, 3).reshape(T, A).to(self.dtype) \
-                    .contiguous()
-            o = F.linear(attn, Ly["wo"])
-            h = D.rmsnorm_residual(o, res, Ly["mlp_norm"], c.norm_eps)
-            gu = F.linear(h, Ly["wgu"])
-            act = D.swiglu(gu[:, :c.ffn], gu[:, c.ffn:])
-            mlp_out = F.linear(act, Ly["wdown"])
-        final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)
-        # mean-pool valid positions, project, L2-normalize.  Pad rows are
-        # never written by the varlen kernel (garbage bf16): zero them
-        # with where() before pooling so inf*0 cannot NaN the pool.
-        hs = final_h.reshape(n, L, c.hidden).float()
-        valid = (torch.arange(L, device=self.device).unsqueeze(0)
-                 < lens_dev.unsqueeze(1)).unsqueeze(-1)
-        hs = torch.where(valid, hs, torch.zeros((), device=self.device))
-        pooled = hs.sum(dim=1) / valid.float().sum(dim=1).clamp(min=1)
+        pooled = self._embed_rows(enc) if self._use_hip and have_ext() \
+            else self._embed_padded(enc)
         out = F.linear(pooled.to(self.dtype), self.proj).float()
         out = out / out.norm(dim=-1, keepdim=True).clamp(min=1e-9)
         return out.cpu().numpy()

@@ -484,8 +484,13 @@ class LlamaModel:
                                        c.norm_eps)
             qkv = F.linear(h, L["wqkv"], L.get("bqkv"))
             q, k, v = self._split_qkv(qkv, T_pad)
-            D.rope_inplace(q, k, self.rope_cos, self.rope_sin, positions)
-            D.kv_scatter(k[:T], v[:T], kv.k[li], kv.v[li], slots)
+            if use_hip_prefill:
+                D.rope_kv_scatter(q[:T], k[:T], v[:T], kv.k[li], kv.v[li],
+                                  self.rope_cos, self.rope_sin,
+                                  positions[:T], slots)
+            else:
+                D.rope_inplace(q, k, self.rope_cos, self.rope_sin, positions)
+                D.kv_scatter(k[:T], v[:T], kv.k[li], kv.v[li], slots)
             if use_hip_prefill:
                 # ONE varlen flash kernel: streams K/V pages directly, no
                 # gather/pad/score materialization

@@ -148,6 +148,16 @@ def kv_scatter(knew: torch.Tensor, vnew: torch.Tensor, kc: torch.Tensor,
         vc[page, :, :, off] = vnew[t]
 
 
+def rope_kv_scatter(q, k, v, kc, vc, cos_t, sin_t, pos, slots) -> None:
+    """rope_inplace of q and k and kv_scatter in one (on the GPU k is rotated
+    on its way to the cache only)."""
+    if _cuda(q):
+        ext().rope_kv_scatter(q, k, v, kc, vc, cos_t, sin_t, pos, slots)
+        return
+    rope_inplace(q, k, cos_t, sin_t, pos)
+    kv_scatter(k, v, kc, vc, slots)
+
+
 def paged_attn_decode(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
                       block_table: torch.Tensor, seq_lens: torch.Tensor,
                       scale: float) -> torch.Tensor:

@@ -169,6 +169,47 @@ qsa_swiglu_kernel(const unsigned short* __restrict__ gate,
 }
 
 // ---------------------------------------------------------------------------
+// Mean of each item's rows: out[i] = mean(x[off[i] : off[i] + len[i]]), f32.
+// Block = (item, 512 columns): lanes take 8 columns, waves every fourth row.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256)
+qsa_mean_rows(const unsigned short* __restrict__ x, const int* __restrict__ off,
+              const int* __restrict__ len, float* __restrict__ out, int H) {
+  __shared__ float part[4][512];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = blockIdx.y * 512 + lane * 8;
+  const int n = len[blockIdx.x];
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (c < H) {
+    const unsigned short* p = x + (long long)off[blockIdx.x] * H + c;
+#pragma unroll 4
+    for (int r = wave; r < n; r += 4) {
+      const uint4 v = *reinterpret_cast<const uint4*>(p + (long long)r * H);
+      const unsigned int u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float2 f = bf16x2_to_f32x2(u[j]);
+        s[2 * j] += f.x;
+        s[2 * j + 1] += f.y;
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) part[wave][lane * 8 + j] = s[j];
+  __syncthreads();
+  for (int i = threadIdx.x; i < 512 && blockIdx.y * 512 + i < H; i += 256)
+    out[(long long)blockIdx.x * H + blockIdx.y * 512 + i] =
+        ((part[0][i] + part[1][i]) + (part[2][i] + part[3][i])) / max(n, 1);
+}
+
+extern "C" void qsa_mean_rows_launch(const unsigned short* x, const int* off,
+                                     const int* len, float* out, int n, int H,
+                                     hipStream_t stream) {
+  hipLaunchKernelGGL(qsa_mean_rows, dim3(n, (H + 511) / 512), dim3(256), 0,
+                     stream, x, off, len, out, H);
+}
+
+// ---------------------------------------------------------------------------
 // RoPE (llama-style half-rotation), in-place on q [B, QH, D] and k [B, KVH, D]
 // cos/sin table [max_pos, D/2] f32; positions [B].
 // One block of D/2 threads per (b, head); heads 0..QH-1 are q, rest are k.

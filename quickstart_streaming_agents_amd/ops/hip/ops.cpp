@@ -54,6 +54,13 @@ extern "C" void qsa_paged_attn_prefill_launch(
     const int*, const int*, const int*, const int*, const int*, const int*,
     unsigned short*, float, int, int, int, int, int, long long, int, int,
     hipStream_t);
+extern "C" void qsa_rope_kv_scatter_launch(
+    unsigned short*, const unsigned short*, const unsigned short*,
+    unsigned short*, unsigned short*, const float*, const float*, const int*,
+    const int*, int, int, int, int, long long, long long, hipStream_t);
+extern "C" void qsa_mean_rows_launch(const unsigned short*, const int*,
+                                     const int*, float*, int, int,
+                                     hipStream_t);
 extern "C" void qsa_rope_kv_append_launch(unsigned short*,
                                           const unsigned short*,
                                           const unsigned short*,
@@ -352,6 +359,56 @@ void rope_kv_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                             seq_lens.data_ptr<int>(), B, QH, KVH, D,
                             (int)block_table.size(1), q.stride(0),
                             k.stride(0), cur_stream());
+}
+
+void rope_kv_scatter(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                     torch::Tensor kc, torch::Tensor vc, torch::Tensor cos_t,
+                     torch::Tensor sin_t, torch::Tensor pos,
+                     torch::Tensor slots) {
+  // rope_inplace on q, and k rotated and v written to the pages; k and v stay
+  CHK_DEV(q); CHK_BF16(q); CHK_BF16(k); CHK_BF16(v);
+  CHK_BF16(kc); CHK_BF16(vc); CHK_CONT(kc); CHK_CONT(vc);
+  CHK_F32(cos_t); CHK_F32(sin_t); CHK_CONT(cos_t); CHK_CONT(sin_t);
+  CHK_I32(pos); CHK_I32(slots); CHK_CONT(pos); CHK_CONT(slots);
+  const int T = q.size(0), QH = q.size(1), D = q.size(2);
+  const int KVH = k.size(1);
+  TORCH_CHECK(D == 128 || D == 64, "D must be 64/128");
+  TORCH_CHECK(QH % KVH == 0, "GQA requires QH % KVH == 0");
+  TORCH_CHECK(k.size(0) == T && k.size(2) == D && v.sizes() == k.sizes() &&
+                  pos.numel() == T && slots.numel() == T, "k/v/pos/slots [T]");
+  TORCH_CHECK(kc.dim() == 5 && kc.size(1) == KVH && kc.size(2) == D / 8 &&
+                  kc.size(3) == 64 && kc.size(4) == 8 && vc.dim() == 4 &&
+                  vc.size(1) == KVH && vc.size(2) == D && vc.size(3) == 64,
+              "cache layouts [P, KVH, D/8, 64, 8], [P, KVH, D, 64]");
+  TORCH_CHECK(cos_t.size(-1) == D / 2 && sin_t.size(-1) == D / 2,
+              "cos/sin [positions, D/2]");
+  chk_hd_strided(q, D, "q"); chk_hd_strided(k, D, "k");
+  chk_hd_strided(v, D, "v");
+  TORCH_CHECK(k.stride(0) == v.stride(0), "k/v strides must match");
+  TORCH_CHECK(q.stride(0) % 8 == 0 && k.stride(0) % 8 == 0 &&
+                  ((reinterpret_cast<uintptr_t>(q.data_ptr()) |
+                    reinterpret_cast<uintptr_t>(k.data_ptr()) |
+                    reinterpret_cast<uintptr_t>(v.data_ptr())) & 15) == 0,
+              "q, k and v rows must be 16-byte aligned");
+  if (T == 0) return;
+  qsa_rope_kv_scatter_launch(u16m(q), u16(k), u16(v), u16m(kc), u16m(vc),
+                             cos_t.data_ptr<float>(), sin_t.data_ptr<float>(),
+                             pos.data_ptr<int>(), slots.data_ptr<int>(), T, QH,
+                             KVH, D, q.stride(0), k.stride(0), cur_stream());
+}
+
+torch::Tensor mean_rows(torch::Tensor x, torch::Tensor off,
+                        torch::Tensor len) {
+  CHK_DEV(x); CHK_BF16(x); CHK_CONT(x); CHK_I32(off); CHK_I32(len);
+  CHK_CONT(off); CHK_CONT(len);
+  TORCH_CHECK(x.dim() == 2 && x.size(1) % 8 == 0, "x [T, H], H % 8 == 0");
+  TORCH_CHECK(off.numel() == len.numel(), "off and len per item");
+  const int n = off.numel(), H = x.size(1);
+  auto out = torch::empty({n, H}, x.options().dtype(at::kFloat));
+  if (n)
+    qsa_mean_rows_launch(u16(x), off.data_ptr<int>(), len.data_ptr<int>(),
+                         out.data_ptr<float>(), n, H, cur_stream());
+  return out;
 }
 
 void kv_scatter(torch::Tensor knew, torch::Tensor vnew, torch::Tensor kc,
@@ -709,6 +766,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", &kv_append, "append one step's k/v to the paged cache");
   m.def("rope_kv_append", &rope_kv_append,
         "fused decode rope + paged-cache append");
+  m.def("rope_kv_scatter", &rope_kv_scatter,
+        "prefill rotation and paged-cache write");
+  m.def("mean_rows", &mean_rows, "mean of each item's rows (f32)");
   m.def("kv_scatter", &kv_scatter, "scatter prefill k/v by slot ids");
   m.def("pack_weight_frag", &pack_weight_frag,
         "repack [N,K] bf16 into MFMA-fragment-major for skinny_gemm");

@@ -527,6 +527,103 @@ extern "C" void qsa_kv_scatter_launch(const unsigned short* knew,
 }
 
 // ---------------------------------------------------------------------------
+// Prefill rotation and cache write in one pass: q is rotated in place, k on its
+// way to the pages, v transposed into them through LDS.
+//
+// Block = (64 tokens, kv head): its R query heads, its key and its value.  A
+// lane owns 8 dims and their rotation partners of one token, so angles are read
+// once for all heads, and every access is 16 bytes wide; the page's K groups
+// and V columns of neighbouring tokens lie together.  Bound by memory:
+// 45k tokens, 32/8 heads of 128: 468 (rotation) + 292 us (scatter by elements)
+// before, 234 us here (4.7 TB/s, what a copy reaches).
+// ---------------------------------------------------------------------------
+template <int D>
+__global__ void __launch_bounds__(256)
+qsa_rope_kv_scatter(unsigned short* __restrict__ q,        // [T, QH, D] strided
+                    const unsigned short* __restrict__ k,  // [T, KVH, D]
+                    const unsigned short* __restrict__ v,
+                    unsigned short* __restrict__ kc,
+                    unsigned short* __restrict__ vc,
+                    const float* __restrict__ cos_t,
+                    const float* __restrict__ sin_t,
+                    const int* __restrict__ pos,           // [T]
+                    const int* __restrict__ slots,         // [T], < 0: none
+                    int T, int QH, int KVH, long long qstride,
+                    long long kvstride) {
+  constexpr int LT = D / 16;           // lanes per token
+  constexpr int TB = 256 / LT;         // tokens per pass of the block
+  constexpr int VP = D + 8;
+  __shared__ __attribute__((aligned(16))) unsigned short vt[64 * VP];
+  const int g = blockIdx.x % KVH;
+  const long long t0 = (long long)(blockIdx.x / KVH) * 64;
+  const int tid = threadIdx.x, R = QH / KVH;
+  const int d = (tid % LT) * 8;
+#pragma unroll
+  for (int p = 0; p < 64; p += TB) {
+    const int i = p + tid / LT;
+    const long long t = t0 + i;
+    if (t >= T) break;
+    const long long at = (long long)pos[t] * (D / 2) + d;
+    float c[8], s[8];
+    ldv<float, 8>(cos_t + at, c);
+    ldv<float, 8>(sin_t + at, s);
+    unsigned short* qp = q + t * qstride + (long long)g * R * D + d;
+    for (int h = 0; h < R; ++h, qp += D) {
+      bf16x8_a x = *reinterpret_cast<bf16x8_a*>(qp);
+      bf16x8_a y = *reinterpret_cast<bf16x8_a*>(qp + D / 2);
+      rotate_pair(x, y, c, s);
+      *reinterpret_cast<bf16x8_a*>(qp) = x;
+      *reinterpret_cast<bf16x8_a*>(qp + D / 2) = y;
+    }
+    const long long row = t * kvstride + (long long)g * D + d;
+    bf16x8_a x = *reinterpret_cast<const bf16x8_a*>(k + row);
+    bf16x8_a y = *reinterpret_cast<const bf16x8_a*>(k + row + D / 2);
+    rotate_pair(x, y, c, s);
+    const int slot = slots[t];
+    if (slot >= 0) {
+      const long long tile =
+          ((long long)(slot / QSA_PAGE) * KVH + g) * D * QSA_PAGE;
+      unsigned short* kp =
+          kc + tile + ((d / 8) * QSA_PAGE + slot % QSA_PAGE) * 8;
+      *reinterpret_cast<bf16x8_a*>(kp) = x;
+      *reinterpret_cast<bf16x8_a*>(kp + D / 2 * QSA_PAGE) = y;
+    }
+    *reinterpret_cast<bf16x8_a*>(vt + i * VP + d) =
+        *reinterpret_cast<const bf16x8_a*>(v + row);
+    *reinterpret_cast<bf16x8_a*>(vt + i * VP + d + D / 2) =
+        *reinterpret_cast<const bf16x8_a*>(v + row + D / 2);
+  }
+  __syncthreads();
+  // lane = token: a wave's store is one column of the page's value tile
+  const int lane = tid & 63;
+  const long long t = t0 + lane;
+  const int slot = t < T ? slots[t] : -1;
+  if (slot < 0) return;
+  unsigned short* vp =
+      vc + ((long long)(slot / QSA_PAGE) * KVH + g) * D * QSA_PAGE +
+      slot % QSA_PAGE;
+#pragma unroll 8
+  for (int e = tid >> 6; e < D; e += 4) vp[e * QSA_PAGE] = vt[lane * VP + e];
+}
+
+extern "C" void qsa_rope_kv_scatter_launch(
+    unsigned short* q, const unsigned short* k, const unsigned short* v,
+    unsigned short* kc, unsigned short* vc, const float* cos_t,
+    const float* sin_t, const int* pos, const int* slots, int T, int QH,
+    int KVH, int D, long long qstride, long long kvstride,
+    hipStream_t stream) {
+  const dim3 grid((unsigned)((long long)((T + 63) / 64) * KVH));
+  if (D == 128)
+    hipLaunchKernelGGL(qsa_rope_kv_scatter<128>, grid, dim3(256), 0, stream, q,
+                       k, v, kc, vc, cos_t, sin_t, pos, slots, T, QH, KVH,
+                       qstride, kvstride);
+  else
+    hipLaunchKernelGGL(qsa_rope_kv_scatter<64>, grid, dim3(256), 0, stream, q,
+                       k, v, kc, vc, cos_t, sin_t, pos, slots, T, QH, KVH,
+                       qstride, kvstride);
+}
+
+// ---------------------------------------------------------------------------
 // Varlen flash PREFILL attention over the paged cache (K4 prefill path), and
 // with CAUSAL=false the encoder's bidirectional attention (K1).
 //

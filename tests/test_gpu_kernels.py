@@ -713,6 +713,51 @@ def test_paged_attn_prefill_blocks(ext, D, QH, KVH, rows, causal):
         assert (got - ref).abs().max() <= 2 ** -7 * v.abs().max(), i
 
 
+@pytest.mark.parametrize("T,QH,KVH,D", [
+    (1, 8, 8, 64), (63, 4, 2, 128), (65, 32, 8, 128), (200, 28, 4, 128),
+    (130, 16, 1, 64)])
+def test_rope_kv_scatter(ext, T, QH, KVH, D):
+    """One pass against rotation and scatter apart; tokens in any slots."""
+    g = torch.Generator().manual_seed(T + D)
+    P = T // 64 + 3
+    kc = torch.randn(P, KVH, D // 8, 64, 8, generator=g).bfloat16().to(dev())
+    vc = torch.randn(P, KVH, D, 64, generator=g).bfloat16().to(dev())
+    kc2, vc2 = kc.clone(), vc.clone()
+    slots = torch.randperm(P * 64, generator=g)[:T].int().to(dev())
+    pos = torch.randint(0, 500, (T,), generator=g).int().to(dev())
+    rot = torch.rand(500, D // 2, generator=g) * 6.28
+    cos, sin = rot.cos().to(dev()), rot.sin().to(dev())
+    qkv = torch.randn(T, (QH + 2 * KVH) * D, generator=g).bfloat16().to(dev())
+    twin = qkv.clone()
+
+    def split(t):
+        q, k, v = t.split([QH * D, KVH * D, KVH * D], 1)
+        return (q.view(T, QH, D), k.view(T, KVH, D), v.view(T, KVH, D))
+
+    q, k, v = split(qkv)
+    ext.rope_kv_scatter(q, k, v, kc, vc, cos, sin, pos, slots)
+    q2, k2, v2 = split(twin)
+    ext.rope_inplace(q2, k2, cos, sin, pos)
+    ext.kv_scatter(k2, v2, kc2, vc2, slots)
+    assert torch.equal(vc, vc2)
+    # products of the rotation may be fused differently: one bf16 step
+    for a, b in ((q, q2), (kc, kc2)):
+        assert ((a.float() - b.float()).abs()
+                <= 2 ** -7 * b.float().abs() + 1e-6).all()
+
+
+def test_mean_rows(ext):
+    lens = [1, 3, 4, 5, 700]
+    x = torch.randn(sum(lens), 520, device=dev()).bfloat16()
+    off = np.cumsum(lens) - lens
+    got = ext.mean_rows(x, torch.tensor(off, dtype=torch.int32, device=dev()),
+                        torch.tensor(lens, dtype=torch.int32, device=dev()))
+    want = torch.stack([x[o:o + n].double().mean(0)
+                        for o, n in zip(off, lens)])
+    # f32 sums of up to 175 values in four parts
+    torch.testing.assert_close(got.double(), want, rtol=1e-5, atol=1e-6)
+
+
 def test_hash_join_gpu_matches_cpu_semantics():
     """K8 hash build/probe on GPU vs the CPU dispatch fallback: random
     keys with duplicates, latest-event-time-wins, TTL cutoff."""
