@@ -107,12 +107,28 @@ class TokenSide:
                                      self.col0, self.act))
 
 
+def upload(a: np.ndarray, device) -> torch.Tensor:
+    """A host array on the device.  To a GPU it goes through pinned memory and
+    without waiting: a pageable copy would first wait for everything queued,
+    and the GPU then idles while the host prepares and launches the step."""
+    t = torch.from_numpy(a)
+    if a.size and torch.device(device).type == "cuda":
+        return t.pin_memory().to(device, non_blocking=True)
+    return t.to(device)
+
+
 def ints_to_device(device, *arrays: np.ndarray) -> list[torch.Tensor]:
     """Several int32 arrays in one host-to-device copy."""
     sizes = [len(a) for a in arrays]
     flat = np.concatenate([np.asarray(a, dtype=np.int32) for a in arrays]) \
         if arrays else np.zeros(0, np.int32)
-    return list(torch.from_numpy(flat).to(device).split(sizes))
+    return list(upload(flat, device).split(sizes))
+
+
+def tokens_to_device(device, lists: list[list[int]]) -> list[torch.Tensor]:
+    """Token lists as i64 tensors, in one host-to-device copy."""
+    flat = np.fromiter((t for x in lists for t in x), dtype=np.int64)
+    return list(upload(flat, device).split([len(x) for x in lists]))
 
 
 class AttnRows:

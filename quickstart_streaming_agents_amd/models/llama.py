@@ -35,11 +35,13 @@ from __future__ import annotations
 
 from dataclasses import dataclass
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
 from ..ops import dispatch as D
 from .kv_cache import PagedKVCache
+from .layers import ints_to_device
 
 
 @dataclass
@@ -381,30 +383,55 @@ class LlamaModel:
         """
         c = self.cfg
         dev = self.device
-        lens = [int(t.shape[0]) for t, _, _ in items]
-        offs = [0]
-        for t in lens:
-            offs.append(offs[-1] + t)
-        T = offs[-1]
+        nb = len(items)
+        lens = np.array([int(t.shape[0]) for t, _, _ in items])
+        starts = np.array([int(s) for _, _, s in items])
+        offs = np.cumsum(lens) - lens
+        T = int(lens.sum())
         tokens = torch.cat([t for t, _, _ in items])
-        positions = torch.cat([
-            torch.arange(s, s + n, dtype=torch.int32, device=dev)
-            for (_, _, s), n in zip(items, lens)]).contiguous()
-        slots = torch.cat([
-            kv.slot_ids(sid, s, n)
-            for (_, sid, s), n in zip(items, lens)]).contiguous()
+        row_item = np.repeat(np.arange(nb), lens)
+        pos = starts[row_item] + np.arange(T) - offs[row_item]
+        # page table of all items, up to the last position of this step
+        npmax = int((starts + lens + kv.PAGE - 1).max()) // kv.PAGE
+        table = np.zeros((nb, npmax), dtype=np.int32)
+        for i, (_, sid, _) in enumerate(items):
+            pages = kv._seq_pages[sid][:npmax]
+            if len(pages) * kv.PAGE < starts[i] + lens[i]:
+                raise IndexError(f"sequence {sid}: {starts[i] + lens[i]} "
+                                 f"positions on {len(pages)} pages")
+            table[i, :len(pages)] = pages
+        slots = table[row_item, pos // kv.PAGE] * kv.PAGE + pos % kv.PAGE
+        if want is None:
+            want = [[n - 1] for n in lens]
+        last = [o + w for o, ws in zip(offs, want) for w in ws]
+        host = [pos, slots, last]
 
         # ---- attention prep (once per prefill call) ---------------------
         R = self.n_q // self.n_kv
-        nb = len(items)
-        nmax = max(lens)
-        npmax = max((int(items[i][2]) + lens[i] + kv.PAGE - 1) // kv.PAGE
-                    for i in range(nb))
+        nmax = int(lens.max())
         ctxp = npmax * kv.PAGE
         import os as _os
         use_hip_prefill = str(dev).startswith("cuda") and \
             self.cfg.d_head in (64, 128) and self.n_q % 4 == 0 and \
             _os.environ.get("QSA_NO_HIP_PREFILL") != "1"
+        if use_hip_prefill:
+            # varlen flash prefill over the paged cache: maps of blocks of
+            # qrows query tokens, which with their R heads fill the kernel's
+            # 128 rows; 64 where 128 would leave CUs without two blocks
+            qrows = max(1, 128 // R)
+            if int((-(-lens // qrows)).sum()) * self.n_kv < 512:
+                qrows = max(1, 64 // R)
+            nqb = -(-lens // qrows)
+            qb_item = np.repeat(np.arange(nb), nqb)
+            qb_pos0 = (np.arange(int(nqb.sum()))
+                       - (np.cumsum(nqb) - nqb)[qb_item]) * qrows
+            # the ones with most keys first: the last to start are short
+            heavy = np.argsort(-(starts[qb_item] + qb_pos0), kind="stable")
+            host += [qb_item[heavy], qb_pos0[heavy], offs, starts, lens]
+        # everything the step needs, in one copy
+        positions, slots, last, bt_t, *maps = ints_to_device(
+            dev, *host[:3], table.reshape(-1), *host[3:])
+        bt_t = bt_t.view(nb, npmax)
         # optional token-dim bucketing (QSA_PREFILL_PAD=1): pad the
         # concatenated batch to a bucket with TunableOp-tuned GEMM
         # entries (data/tunableop_mi355x.csv).  Pad rows run the
@@ -429,43 +456,14 @@ class LlamaModel:
                     positions,
                     torch.zeros(padn, dtype=torch.int32, device=dev)
                 ]).contiguous()
-        if use_hip_prefill:
-            # varlen flash prefill over the paged cache: maps of blocks of
-            # qrows query tokens, which with their R heads fill the kernel's
-            # 128 rows; 64 where 128 would leave CUs without two blocks
-            qrows = max(1, 128 // R)
-            if sum(-(-n // qrows) for n in lens) * self.n_kv < 512:
-                qrows = max(1, 64 // R)
-            blocks = [(i, p0) for i, n in enumerate(lens)
-                      for p0 in range(0, n, qrows)]
-            # the ones with most keys first: the last to start are short
-            blocks.sort(key=lambda b: -int(items[b[0]][2]) - b[1])
-            qb_item_t = torch.tensor([b[0] for b in blocks],
-                                     dtype=torch.int32, device=dev)
-            qb_pos0_t = torch.tensor([b[1] for b in blocks],
-                                     dtype=torch.int32, device=dev)
-            off_t = torch.tensor(offs[:-1], dtype=torch.int32, device=dev)
-            start_t = torch.tensor([int(s) for _, _, s in items],
-                                   dtype=torch.int32, device=dev)
-            len_t = torch.tensor(lens, dtype=torch.int32, device=dev)
-            bt = torch.zeros(nb, npmax, dtype=torch.int32)
-            for i, (_, sid, _) in enumerate(items):
-                pages = kv._seq_pages[sid][:npmax]
-                bt[i, :len(pages)] = torch.tensor(pages, dtype=torch.int32)
-            bt_t = bt.to(dev)
-        else:
+        if not use_hip_prefill:
             # CPU reference: padded-batch bmm pair + masked softmax.
             # Per-row limits (start_i + qpos + 1, or 0 on pad rows) give
             # exact causal + ragged masking.
             dst_idx = torch.tensor(
                 [i * nmax + p for i, n in enumerate(lens) for p in range(n)],
                 dtype=torch.int64, device=dev)
-            page_idx = torch.zeros(nb, npmax, dtype=torch.int64)
-            for i, (_, sid, _) in enumerate(items):
-                pages = kv._seq_pages[sid][:npmax]
-                page_idx[i, :len(pages)] = torch.tensor(pages,
-                                                        dtype=torch.int64)
-            flat_pages = page_idx.reshape(-1).to(dev)
+            flat_pages = bt_t.reshape(-1).long()
             limits = torch.zeros(nb, self.n_q, nmax, dtype=torch.int32)
             for i, ((_, _, start), n) in enumerate(zip(items, lens)):
                 lim = torch.arange(start + 1, start + n + 1,
@@ -495,8 +493,8 @@ class LlamaModel:
                 # ONE varlen flash kernel: streams K/V pages directly, no
                 # gather/pad/score materialization
                 attn = D.ext().paged_attn_prefill(
-                    q, kv.k[li], kv.v[li], bt_t, qb_item_t, qb_pos0_t,
-                    off_t, start_t, len_t, self.scale, True, qrows)
+                    q, kv.k[li], kv.v[li], bt_t, *maps, self.scale, True,
+                    qrows)
             else:
                 # padded q: [nb*nmax, n_q, D] -> [nb*KVH, R*nmax, D]
                 q_pad = torch.zeros(nb * nmax, self.n_q, c.d_head,
@@ -528,10 +526,6 @@ class LlamaModel:
             h = D.rmsnorm_residual(o, res, L["mlp_norm"], c.norm_eps)
             mlp_out = self._ffn(L, h)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)
-        if want is None:
-            want = [[n - 1] for n in lens]
-        last = torch.tensor([offs[i] + w for i, ws in enumerate(want)
-                             for w in ws], dtype=torch.int64, device=dev)
         if not last.numel():
             return final_h.new_empty(0, c.vocab_size)
         return self._linear(final_h.index_select(0, last), self.lm_head,

@@ -28,6 +28,7 @@ from dataclasses import dataclass, field
 import torch
 
 from ..ops import dispatch as D
+from .layers import tokens_to_device
 
 
 @dataclass
@@ -475,7 +476,6 @@ class Engine:
         self.pending.sort(
             key=lambda s: (s.cached_len > 0,
                            -(len(s.prompt) - s.cached_len)))
-        batch_items: list[tuple[torch.Tensor, int, int]] = []
         admitted: list[Sequence] = []
         new_tokens = 0
         while self.pending and len(self.running) + len(admitted) < self.max_batch:
@@ -487,16 +487,13 @@ class Engine:
             if not self.kv.can_admit(seq.seq_id, need):
                 break
             delta = len(seq.prompt) - seq.cached_len
-            if batch_items and new_tokens + delta > self.prefill_batch_tokens:
+            if admitted and new_tokens + delta > self.prefill_batch_tokens:
                 break
             self.pending.pop(0)
             if seq.cached_len:
                 self.kv.extend(seq.seq_id, len(seq.prompt))
             else:
                 self.kv.allocate(seq.seq_id, len(seq.prompt))
-            toks = torch.tensor(seq.prompt[seq.cached_len:],
-                                dtype=torch.int64, device=self.model.device)
-            batch_items.append((toks, seq.seq_id, seq.cached_len))
             admitted.append(seq)
             new_tokens += delta
             self.stats.prefill_tokens += delta
@@ -504,6 +501,10 @@ class Engine:
             self.stats.prefills += 1
         if not admitted:
             return
+        toks = tokens_to_device(self.model.device,
+                                [s.prompt[s.cached_len:] for s in admitted])
+        batch_items = [(t, s.seq_id, s.cached_len)
+                       for t, s in zip(toks, admitted)]
         if _TIMING:
             torch.cuda.synchronize()
             _t0 = time.perf_counter()
@@ -570,8 +571,8 @@ class Engine:
             if rows == list(range(len(entries))):
                 return logits
             return logits[torch.tensor(rows, dtype=torch.int64, device=dev)]
-        items = [(torch.tensor(e.tokens, dtype=torch.int64, device=dev),
-                  e.seq_id, e.start) for e in entries]
+        items = [(t, e.seq_id, e.start) for t, e in zip(
+            tokens_to_device(dev, [e.tokens for e in entries]), entries)]
         return self.model.forward_prefill_batch(
             items, self.kv, want=[e.want for e in entries])
 
