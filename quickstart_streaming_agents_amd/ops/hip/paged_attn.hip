@@ -111,6 +111,28 @@ qsa_paged_attn_mfma(DecodeArgs p) {
     for (int ks = 0; ks < KSTEPS; ++ks)
       qf[ks] = *reinterpret_cast<const bf16x8_a*>(qrow + ks * 32 + hi * 8);
     const int* btab = p.block_table + (long long)b * p.max_pages;
+    auto load_k = [&](int page, bf16x8_a (&kf)[4][KSTEPS]) {
+      const unsigned short* kbase =
+          p.kc + ((((long long)page * p.KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks)
+          kf[pt][ks] = *reinterpret_cast<const bf16x8_a*>(
+              kbase + ((ks * 4 + hi) * QSA_PAGE + pt * 16 + col) * 8);
+    };
+    // the last page is read by this wave alone, after its own stores
+    auto stores_done = [&] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    bf16x8_a kf[4][KSTEPS];
+    int page = btab[first];
+    // keys of the first page are under way before anything else, unless the
+    // new one still has to get there
+    const bool wait_first = FUSE && first == npages - 1;
+    if (!wait_first) load_k(page, kf);
     if constexpr (FUSE) {
       const long long at = (long long)(seqlen - 1) * (D / 2) + hi * 8;
 #pragma unroll
@@ -143,26 +165,13 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         for (int i = 0; i < D; i += 64)
           p.vw[tile + (long long)(i + lane) * QSA_PAGE + pin] =
               p.v[row + i + lane];
-        // the page is read by this wave alone: its stores come first
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
       }
     }
 
-    auto load_k = [&](int page, bf16x8_a (&kf)[4][KSTEPS]) {
-      const unsigned short* kbase =
-          p.kc + ((((long long)page * p.KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
-#pragma unroll
-      for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks)
-          kf[pt][ks] = *reinterpret_cast<const bf16x8_a*>(
-              kbase + ((ks * 4 + hi) * QSA_PAGE + pt * 16 + col) * 8);
-    };
-    bf16x8_a kf[4][KSTEPS];
-    int page = btab[first];
-    load_k(page, kf);
+    if (wait_first) {
+      stores_done();
+      load_k(page, kf);
+    }
     for (int pi = first; pi < npages; pi += step) {
       const bool more = pi + step < npages;
       const int next = more ? btab[pi + step] : 0;
@@ -191,7 +200,10 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         sc[pt] = acc;
       }
       load_v(1);
-      if (more) load_k(next, kf);
+      if (more) {
+        if (FUSE && pi + step == npages - 1) stores_done();
+        load_k(next, kf);
+      }
       // scale + mask invalid positions; C layout: row pos = hi*4 + r,
       // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
       float pagemax = -3.0e38f;
