@@ -15,7 +15,7 @@
 // chunk: 81 us).  So blocks count CHUNKS of consecutive events, which in a
 // stream span a few windows, in LDS and leave (windows spanned) * nkeys cells
 // in a workspace; qsa_window_merge adds them up, without atomics and in a fixed
-// order (42 us together).  A chunk whose span does not fit goes to the output
+// order (33 us together).  A chunk whose span does not fit goes to the output
 // with atomics, as do batches of a few chunks, where a second launch costs
 // more than their cells.
 // ---------------------------------------------------------------------------
@@ -30,6 +30,21 @@ __device__ __forceinline__ int qsa_window_of(long long ts, long long t0,
   return w >= 0 && w < nwin ? (int)w : -1;
 }
 
+// The same for win_ms > 0 without a 64-bit division (some 130 instructions):
+// a quotient below 2^31 from the reciprocal is off by one at most.
+// limit = nwin * win_ms, inv = 1 / win_ms.
+__device__ __forceinline__ int qsa_window_by(long long ts, long long t0,
+                                             long long win_ms, long long limit,
+                                             double inv) {
+  const long long d = ts - t0;
+  if (d <= -win_ms || d >= limit) return -1;
+  int w = (int)((double)d * inv);
+  const long long r = d - w * win_ms;
+  w += r >= win_ms ? 1 : r < 0 ? -1 : 0;
+  return max(w, 0);                    // the quotient is cut towards zero
+}
+
+template <bool FAST>                   // chunk == QSA_AGG_CHUNK, win_ms > 0
 __global__ void __launch_bounds__(256)
 qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
                const float* __restrict__ value,  // nullptr -> count only
@@ -50,12 +65,40 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
   }
   __syncthreads();
   int lo = 0x7fffffff, hi = -1;
+  // FAST: every load of the chunk is under way before the first is used, and
+  // an event's window is found once
+  constexpr int PER = QSA_AGG_CHUNK / 256;
+  int win[FAST ? PER : 1], ek[FAST ? PER : 1];
+  float ev[FAST ? PER : 1];
+  if constexpr (FAST) {
+    long long et[PER];
+    const long long limit = win_ms > 0x7fffffffffffffffll / nwin
+                                ? 0x7fffffffffffffffll : win_ms * nwin;
+    const double inv = 1.0 / (double)win_ms;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const long long i = min(first + tid + j * 256, n - 1);
+      et[j] = ts[i];
+      ek[j] = key[i];
+      ev[j] = value ? value[i] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      win[j] = first + tid + j * 256 < end
+                   ? qsa_window_by(et[j], t0, win_ms, limit, inv) : -1;
+      if (win[j] >= 0) {
+        lo = min(lo, win[j]);
+        hi = max(hi, win[j]);
+      }
+    }
+  } else {
 #pragma unroll 4
-  for (long long i = first + tid; i < end; i += 256) {
-    const int w = qsa_window_of(ts[i], t0, win_ms, nwin);
-    if (w >= 0) {
-      lo = min(lo, w);
-      hi = max(hi, w);
+    for (long long i = first + tid; i < end; i += 256) {
+      const int w = qsa_window_of(ts[i], t0, win_ms, nwin);
+      if (w >= 0) {
+        lo = min(lo, w);
+        hi = max(hi, w);
+      }
     }
   }
 #pragma unroll
@@ -82,12 +125,8 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
     }
     __syncthreads();
   }
-#pragma unroll 4
-  for (long long i = first + tid; i < end; i += 256) {
-    const int w = qsa_window_of(ts[i], t0, win_ms, nwin);
-    const int kk = key[i];
-    const float v = value ? value[i] : 0.f;
-    if (w < 0 || kk < 0 || kk >= nkeys) continue;
+  auto count = [&](int w, int kk, float v) {
+    if (w < 0 || kk < 0 || kk >= nkeys) return;
     if (local) {
       const int c = (w - lo) * nkeys + kk;
       atomicAdd(cnt + c, 1);
@@ -97,6 +136,15 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
       atomicAdd(counts + slot, 1);
       if (value) unsafeAtomicAdd(sums + slot, v);
     }
+  };
+  if constexpr (FAST) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) count(win[j], ek[j], ev[j]);
+  } else {
+#pragma unroll 4
+    for (long long i = first + tid; i < end; i += 256)
+      count(qsa_window_of(ts[i], t0, win_ms, nwin), key[i],
+            value ? value[i] : 0.f);
   }
   if (!local) return;
   __syncthreads();
@@ -154,18 +202,37 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
     const int w = w0 + wave * 2 + u;
     int c = 0;
     float v = 0.f;
-#pragma unroll 4
-    for (int j = 0; j < total; ++j) {
-      const int2 s = range[j];
-      const bool in = live && w >= s.x && w < s.x + s.y;
-      // outside its span a chunk lends its first cell, which counts for none
-      const int* p = ws + (long long)list[j] * 2 * QSA_AGG_CELLS +
-                     (in ? (w - s.x) * nkeys + k : 0);
-      const int pc = *p;
-      c += in ? pc : 0;
-      if (has_value) {
-        const float pv = __int_as_float(p[QSA_AGG_CELLS]);
-        v += in ? pv : 0.f;
+    // four chunks at a time, their loads together; in a stream most groups
+    // do not reach this window
+    for (int j0 = 0; j0 < total; j0 += 4) {
+      bool any = false, in[4];
+      int at[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = min(j0 + j, total - 1);
+        const int2 s = range[i];
+        in[j] = j0 + j < total && w >= s.x && w < s.x + s.y;
+        at[j] = in[j] ? i : -1;
+        any |= in[j];
+      }
+      if (!any) continue;              // uniform over the wave
+      int pc[4];
+      float pv[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        pc[j] = 0;
+        pv[j] = 0.f;
+        if (in[j] && live) {
+          const int* p = ws + (long long)list[at[j]] * 2 * QSA_AGG_CELLS +
+                         (w - range[at[j]].x) * nkeys + k;
+          pc[j] = *p;
+          if (has_value) pv[j] = __int_as_float(p[QSA_AGG_CELLS]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        c += pc[j];
+        v += pv[j];
       }
     }
     if (live && w < nwin) {
@@ -359,9 +426,14 @@ extern "C" void qsa_window_agg_launch(const long long* ts, const int* key,
   const int blocks = (int)((n + chunk - 1) / chunk);
   int2* span = reinterpret_cast<int2*>(ws);
   int* cells = ws ? ws + 2 * blocks : nullptr;
-  hipLaunchKernelGGL(qsa_window_agg, dim3(blocks), dim3(256), 0, stream, ts,
-                     key, value, counts, sums, t0, win_ms, nwin, nkeys, n,
-                     chunk, span, cells);
+  if (chunk == QSA_AGG_CHUNK && win_ms > 0)
+    hipLaunchKernelGGL(qsa_window_agg<true>, dim3(blocks), dim3(256), 0,
+                       stream, ts, key, value, counts, sums, t0, win_ms, nwin,
+                       nkeys, n, chunk, span, cells);
+  else
+    hipLaunchKernelGGL(qsa_window_agg<false>, dim3(blocks), dim3(256), 0,
+                       stream, ts, key, value, counts, sums, t0, win_ms, nwin,
+                       nkeys, n, chunk, span, cells);
   if (ws)
     hipLaunchKernelGGL(qsa_window_merge,
                        dim3((nwin + 7) / 8, (nkeys + 63) / 64), dim3(256), 0,

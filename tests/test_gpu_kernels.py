@@ -203,7 +203,7 @@ def test_window_agg_edges(ext, n, nkeys, nwin, shuffle):
     """Chunks counted in LDS and chunks that go to memory directly; events
     before and behind the windows.  Whole values: sums are exact."""
     g = torch.Generator().manual_seed(n)
-    win, t0 = 1000, 5000
+    win, t0 = 1000 + n % 7, 5000 - (n % 3) * (1 << 40)
     ts = torch.randint(t0 - 2 * win, t0 + (nwin + 1) * win, (n,), generator=g)
     if not shuffle:
         ts = ts.sort()[0]
