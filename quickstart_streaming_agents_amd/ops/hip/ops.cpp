@@ -107,7 +107,7 @@ extern "C" void qsa_hash_probe_launch(const long long*,
                                       const unsigned long long*, int*, int,
                                       unsigned int, long long, int,
                                       hipStream_t);
-extern "C" int qsa_topk_block_docs(long long);
+extern "C" int qsa_topk_block_docs(long long, long long);
 extern "C" void qsa_topk_launch(const float*, const float*, float*, int*,
                                 float*, int*, int, int, int, int, int,
                                 hipStream_t);
@@ -681,7 +681,7 @@ std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
   const int Q = queries.size(0), D = queries.size(1), N = docs.size(0);
   TORCH_CHECK(docs.size(1) == D, "dim mismatch");
   TORCH_CHECK(k >= 1 && k <= 16, "k in [1,16]");
-  const int per = qsa_topk_block_docs(N);
+  const int per = qsa_topk_block_docs(Q, N);
   const int nblk = std::max(1, (N + per - 1) / per);
   auto opts_f = queries.options();
   auto opts_i = queries.options().dtype(at::kInt);

@@ -6,19 +6,18 @@
 //
 // Bound by one read of the index.  A block scores 16*T documents against 16
 // queries at once on the f32 matrix cores (16x16x4, f32 products and sums), so
-// up to 16 queries cost one read of the matrix; its four waves split the
-// vector dimension and meet in LDS, so a block needs no query staging and
-// small indexes still spread over the chip.  T = 4 keeps 8 KiB of documents
+// up to 16 queries (32 with QT = 2) cost one read of the matrix; its four waves
+// split the vector dimension and meet in LDS, so a block needs no query staging
+// and small indexes still spread over the chip.  T = 4 keeps 8 KiB of documents
 // per wave in flight while the previous step multiplies; T = 1 serves indexes
 // whose 64-document blocks would leave CUs idle.
 // 100,000 x 1536, 8 queries, k = 3: 4490 us with one dot product per wave and
-// a pass per query, before; 146 us here (4.2 TB/s), and 13 us of merge.
+// a pass per query, before; 145 us here (4.2 TB/s), and 7 us of merge.
 //
 // Results: scores > -2 in descending order, equal scores by ascending
 // document; what k asks for beyond them is (-2, -1).  NaN scores never enter.
 #include "common.h"
 
-#define QSA_TOPK_QG 16                 // queries per block
 
 using f32x4_t = __attribute__((ext_vector_type(4))) float;
 
@@ -51,141 +50,180 @@ __device__ __forceinline__ void qsa_row8(const float* __restrict__ row, int k,
   }
 }
 
-template <int T, bool VEC>
-__global__ void __launch_bounds__(256)
+template <int T, int QT, bool VEC>     // 16*T documents, 16*QT queries
+__global__ void __launch_bounds__(256, 2)
 qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
               const float* __restrict__ docs,     // [N, D] L2-normalized
               float* __restrict__ cand_scores,    // [Q, nblk, k]
               int* __restrict__ cand_ids,         // [Q, nblk, k]
               int Qn, int N, int D, int k) {
-  __shared__ float part[4][16 * T][QSA_TOPK_QG + 1];
+  __shared__ float part[4][16 * T][17];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
-  const int doc0 = blockIdx.x * 16 * T, q0 = blockIdx.y * QSA_TOPK_QG;
+  const int doc0 = blockIdx.x * 16 * T, q0 = blockIdx.y * 16 * QT;
 
   // rows beyond the end shadow the last one; nothing of theirs is kept
-  const float* qrow = queries + (long long)min(q0 + col, Qn - 1) * D;
+  const float* qrow[QT];
+#pragma unroll
+  for (int u = 0; u < QT; ++u)
+    qrow[u] = queries + (long long)min(q0 + u * 16 + col, Qn - 1) * D;
   const float* drow[T];
 #pragma unroll
   for (int t = 0; t < T; ++t)
     drow[t] = docs + (long long)min(doc0 + t * 16 + col, N - 1) * D;
 
-  double total[T][4];
+  double total[T][QT][4];
 #pragma unroll
   for (int t = 0; t < T; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) total[t][r] = 0.0;
+    for (int u = 0; u < QT; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) total[t][u][r] = 0.0;
 
   const int steps = (D + 31) / 32;     // 32 floats of every row, 8 per lane
-  float qn[8], dn[T][8];
+  float qn[QT][8], dn[T][8];
   auto fetch = [&](int s) {
     const int kk = s * 32 + hi * 8;
-    qsa_row8<VEC>(qrow, kk, D, qn);
+#pragma unroll
+    for (int u = 0; u < QT; ++u) qsa_row8<VEC>(qrow[u], kk, D, qn[u]);
 #pragma unroll
     for (int t = 0; t < T; ++t) qsa_row8<VEC>(drow[t], kk, D, dn[t]);
   };
   if (wave < steps) fetch(wave);
   for (int s = wave; s < steps; s += 4) {
-    float qc[8], dc[T][8];
+    float qc[QT][8], dc[T][8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      qc[e] = qn[e];
+#pragma unroll
+      for (int u = 0; u < QT; ++u) qc[u][e] = qn[u][e];
 #pragma unroll
       for (int t = 0; t < T; ++t) dc[t][e] = dn[t][e];
     }
     if (s + 4 < steps) fetch(s + 4);
     // sums of 32 products, added up in f64: one f32 chain over the row would
     // double the rounding of a score
-    f32x4_t acc[T];
+    f32x4_t acc[T][QT];
 #pragma unroll
-    for (int t = 0; t < T; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int u = 0; u < QT; ++u) acc[t][u] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int e = 0; e < 8; ++e)
 #pragma unroll
       for (int t = 0; t < T; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(dc[t][e], qc[e], acc[t],
-                                                      0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < QT; ++u)
+          acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              dc[t][e], qc[u][e], acc[t][u], 0, 0, 0);
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) total[t][r] += (double)acc[t][r];
+      for (int u = 0; u < QT; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) total[t][u][r] += (double)acc[t][u][r];
   }
-#pragma unroll
-  for (int t = 0; t < T; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      part[wave][t * 16 + hi * 4 + r][col] = (float)total[t][r];
-  __syncthreads();
 
-  // 16 lanes per query, T documents each: k rounds of best-of-the-rest
-  const int q = tid >> 4, sub = tid & 15;
-  float sc[T];
 #pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const int d = t * 16 + sub;
-    const float v = (float)(((double)part[0][d][q] + part[1][d][q]) +
-                            ((double)part[2][d][q] + part[3][d][q]));
-    sc[t] = doc0 + d < N && v > -2.0f ? v : -INFINITY;
-  }
-  const bool live = q0 + q < Qn;
-  const long long at =
-      ((long long)(q0 + q) * gridDim.x + blockIdx.x) * k;
-  for (int r = 0; r < k; ++r) {
-    float bs = sc[0];
-    int bi = doc0 + sub;
-#pragma unroll
-    for (int t = 1; t < T; ++t)
-      if (sc[t] > bs) {
-        bs = sc[t];
-        bi = doc0 + t * 16 + sub;
-      }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-      const float os = __shfl_xor(bs, o, 16);
-      const int oi = __shfl_xor(bi, o, 16);
-      if (qsa_better(os, oi, bs, bi)) {
-        bs = os;
-        bi = oi;
-      }
-    }
+  for (int u = 0; u < QT; ++u) {       // 16 queries at a time
+    if (u) __syncthreads();
 #pragma unroll
     for (int t = 0; t < T; ++t)
-      if (doc0 + t * 16 + sub == bi) sc[t] = -INFINITY;
-    if (live && sub == 0) {
-      const bool some = bs > -INFINITY;
-      cand_scores[at + r] = some ? bs : -2.0f;
-      cand_ids[at + r] = some ? bi : -1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        part[wave][t * 16 + hi * 4 + r][col] = (float)total[t][u][r];
+    __syncthreads();
+    // 16 lanes per query, T documents each: k rounds of best-of-the-rest
+    const int q = tid >> 4, sub = tid & 15, qi = q0 + u * 16 + q;
+    float sc[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int d = t * 16 + sub;
+      const float v = (float)(((double)part[0][d][q] + part[1][d][q]) +
+                              ((double)part[2][d][q] + part[3][d][q]));
+      sc[t] = doc0 + d < N && v > -2.0f ? v : -INFINITY;
+    }
+    const bool live = qi < Qn;
+    const long long at =
+        ((long long)qi * gridDim.x + blockIdx.x) * k;
+    for (int r = 0; r < k; ++r) {
+      float bs = sc[0];
+      int bi = doc0 + sub;
+#pragma unroll
+      for (int t = 1; t < T; ++t)
+        if (sc[t] > bs) {
+          bs = sc[t];
+          bi = doc0 + t * 16 + sub;
+        }
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) {
+        const float os = __shfl_xor(bs, o, 16);
+        const int oi = __shfl_xor(bi, o, 16);
+        if (qsa_better(os, oi, bs, bi)) {
+          bs = os;
+          bi = oi;
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        if (doc0 + t * 16 + sub == bi) sc[t] = -INFINITY;
+      if (live && sub == 0) {
+        const bool some = bs > -INFINITY;
+        cand_scores[at + r] = some ? bs : -2.0f;
+        cand_ids[at + r] = some ? bi : -1;
+      }
     }
   }
 }
 
 // One block per query: k rounds, each the best candidate behind the last one.
-// The few thousand candidates stay in L2 between rounds.
-__global__ void __launch_bounds__(1024)
-qsa_topk_merge(const float* __restrict__ cand_scores,  // [Q, n]
+// A scan block's candidates are sorted, so a thread keeps the heads of HEADS of
+// their lists and a round compares heads only; lists beyond HEADS per thread
+// (indexes of 262,144 documents and more) are searched whole.
+#define QSA_MERGE_THREADS 512
+#define QSA_MERGE_HEADS 8
+
+__global__ void __launch_bounds__(QSA_MERGE_THREADS)
+qsa_topk_merge(const float* __restrict__ cand_scores,  // [Q, lists, k]
                const int* __restrict__ cand_ids,
                float* __restrict__ out_scores,         // [Q, k]
-               int* __restrict__ out_ids, int n, int k) {
-  __shared__ float ws[16];
-  __shared__ int wi[16];
+               int* __restrict__ out_ids, int lists, int k) {
+  constexpr int NT = QSA_MERGE_THREADS, NH = QSA_MERGE_HEADS, NW = NT / 64;
+  __shared__ float ws[NW];
+  __shared__ int wi[NW];
   const int tid = threadIdx.x, wave = tid >> 6;
-  const float* cs = cand_scores + (long long)blockIdx.x * n;
-  const int* ci = cand_ids + (long long)blockIdx.x * n;
+  const float* cs = cand_scores + (long long)blockIdx.x * lists * k;
+  const int* ci = cand_ids + (long long)blockIdx.x * lists * k;
+  float hs[NH];
+  int hd[NH], at[NH];                  // id -1: the list is used up
+#pragma unroll
+  for (int j = 0; j < NH; ++j) {
+    at[j] = (tid + j * NT) * k;
+    const bool in = tid + j * NT < lists;
+    hd[j] = in ? ci[at[j]] : -1;
+    hs[j] = in ? cs[at[j]] : 0.f;
+  }
   float last_s = INFINITY;
   int last_i = -1;
   for (int r = 0; r < k; ++r) {
     float bs = -INFINITY;
     int bi = 0x7fffffff;
-    for (int c = tid; c < n; c += 1024) {
-      const float s = cs[c];
-      const int i = ci[c];
-      if (i >= 0 && qsa_better(last_s, last_i, s, i) &&
-          qsa_better(s, i, bs, bi)) {
-        bs = s;
-        bi = i;
+#pragma unroll
+    for (int j = 0; j < NH; ++j)
+      if (hd[j] >= 0 && qsa_better(hs[j], hd[j], bs, bi)) {
+        bs = hs[j];
+        bi = hd[j];
       }
-    }
+    for (int c = (tid + NH * NT) * k; c < lists * k; c += NT * k)
+      for (int e = 0; e < k; ++e) {
+        const float s = cs[c + e];
+        const int i = ci[c + e];
+        if (i >= 0 && qsa_better(last_s, last_i, s, i) &&
+            qsa_better(s, i, bs, bi)) {
+          bs = s;
+          bi = i;
+        }
+      }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const float os = __shfl_xor(bs, o, QSA_WAVE);
@@ -203,7 +241,8 @@ qsa_topk_merge(const float* __restrict__ cand_scores,  // [Q, n]
     __syncthreads();
     last_s = ws[0];
     last_i = wi[0];
-    for (int w = 1; w < 16; ++w)
+#pragma unroll
+    for (int w = 1; w < NW; ++w)
       if (qsa_better(ws[w], wi[w], last_s, last_i)) {
         last_s = ws[w];
         last_i = wi[w];
@@ -213,34 +252,51 @@ qsa_topk_merge(const float* __restrict__ cand_scores,  // [Q, n]
       out_scores[(long long)blockIdx.x * k + r] = some ? last_s : -2.0f;
       out_ids[(long long)blockIdx.x * k + r] = some ? last_i : -1;
     }
+#pragma unroll
+    for (int j = 0; j < NH; ++j)
+      if (hd[j] >= 0 && hd[j] == last_i) {        // its owner moves on
+        ++at[j];
+        const bool in = at[j] < (tid + j * NT + 1) * k;
+        hd[j] = in ? ci[at[j]] : -1;
+        hs[j] = in ? cs[at[j]] : 0.f;
+      }
   }
 }
 
-// Documents per block.  64 as soon as that gives every CU two blocks.
-extern "C" int qsa_topk_block_docs(long long N) {
-  return N >= 64 * 512 ? 64 : 16;
+// Documents per block: 16 for small indexes; 64 as soon as that gives every CU
+// two blocks, or 32 beside twice the queries (17 and more of them: 32 queries
+// in one read of the index, 222 us where two reads took 296).
+extern "C" int qsa_topk_block_docs(long long Q, long long N) {
+  return N < 64 * 512 ? 16 : Q > 16 ? 32 : 64;
 }
 
 extern "C" void qsa_topk_launch(const float* queries, const float* docs,
                                 float* cand_scores, int* cand_ids,
                                 float* out_scores, int* out_ids, int Q, int N,
                                 int D, int k, int nblk, hipStream_t stream) {
-  const dim3 grid(nblk, (Q + QSA_TOPK_QG - 1) / QSA_TOPK_QG);
   const bool vec = D % 4 == 0 && ((reinterpret_cast<uintptr_t>(queries) |
                                    reinterpret_cast<uintptr_t>(docs)) &
                                   15) == 0;
-#define QSA_SCAN(T, V)                                                       \
-  hipLaunchKernelGGL((qsa_topk_scan<T, V>), grid, dim3(256), 0, stream,      \
-                     queries, docs, cand_scores, cand_ids, Q, N, D, k)
+#define QSA_SCAN(T, QT)                                                      \
+  {                                                                          \
+    const dim3 grid(nblk, (Q + 16 * QT - 1) / (16 * QT));                    \
+    if (vec)                                                                 \
+      hipLaunchKernelGGL((qsa_topk_scan<T, QT, true>), grid, dim3(256), 0,   \
+                         stream, queries, docs, cand_scores, cand_ids, Q, N, \
+                         D, k);                                              \
+    else                                                                     \
+      hipLaunchKernelGGL((qsa_topk_scan<T, QT, false>), grid, dim3(256), 0,  \
+                         stream, queries, docs, cand_scores, cand_ids, Q, N, \
+                         D, k);                                              \
+  }
   if (N > 0) {
-    if (qsa_topk_block_docs(N) == 64) {
-      if (vec) QSA_SCAN(4, true); else QSA_SCAN(4, false);
-    } else {
-      if (vec) QSA_SCAN(1, true); else QSA_SCAN(1, false);
-    }
+    const int per = qsa_topk_block_docs(Q, N);
+    if (per == 64) QSA_SCAN(4, 1)
+    else if (per == 32) QSA_SCAN(2, 2)
+    else QSA_SCAN(1, 1)
   }
 #undef QSA_SCAN
-  hipLaunchKernelGGL(qsa_topk_merge, dim3(Q), dim3(1024), 0, stream,
-                     cand_scores, cand_ids, out_scores, out_ids,
-                     N > 0 ? nblk * k : 0, k);
+  hipLaunchKernelGGL(qsa_topk_merge, dim3(Q), dim3(QSA_MERGE_THREADS), 0,
+                     stream, cand_scores, cand_ids, out_scores, out_ids,
+                     N > 0 ? nblk : 0, k);
 }

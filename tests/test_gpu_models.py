@@ -205,6 +205,39 @@ def test_vector_index_gpu_search_matches_cpu():
         assert {h.document_id for h in g_hits} <= set(idx.ids)
 
 
+@pytest.mark.parametrize("rows,queries,k", [
+    (40_000, 17, 3), (40_000, 37, 16), (40_000, 38, 16), (500, 16, 17),
+    (500, 200, 5)])
+def test_vector_index_batches(rows, queries, k):
+    """The kernel and the matmul on either side of the rule between them; 40
+    numbers a row, so a score's error stays under 40 roundings of f32."""
+    import numpy as np
+    from quickstart_streaming_agents_amd.vector.index import VectorIndex
+    rng = np.random.default_rng(rows + queries)
+    m = rng.standard_normal((rows, 40)).astype(np.float32)
+    m /= np.linalg.norm(m, axis=1, keepdims=True)
+    idx = VectorIndex(dim=40)
+    idx._vecs, idx.metadata = list(m), [{}] * rows
+    idx.ids = [str(i) for i in range(rows)]
+    idx.chunks = idx.ids
+    q = rng.standard_normal((queries, 40)).astype(np.float32)
+    q[3] = m[rows - 1]
+    want = q.astype(np.float64)
+    want /= np.linalg.norm(want, axis=1, keepdims=True)
+    want = want @ m.astype(np.float64).T
+    tol = 40 * 2.0 ** -24
+    for i, hits in enumerate(idx.search_batch_gpu(q, k, device="cuda:0")):
+        top = np.sort(want[i])[::-1][:k]
+        assert len(hits) == k and len({h.document_id for h in hits}) == k
+        for h, best in zip(hits, top):
+            assert abs(h.score - best) < tol
+            assert abs(h.score - want[i, int(h.document_id)]) < tol
+    q[5] = np.nan                      # a query without an answer
+    hits = idx.search_batch_gpu(q, k, device="cuda:0")
+    assert all(np.isnan(h.score) for h in hits[5]) and \
+        hits[3][0].document_id == str(rows - 1)
+
+
 def test_lab3_lab4_gpu_anomaly_matches_cpu_and_invariants():
     """The batched GPU anomaly path must reproduce the sequential CPU
     reference on the real lab datagen — and hence the determinism
