@@ -113,9 +113,20 @@ extern "C" void qsa_gqa_rows_launch(
 // lane-local (column = query head), V passes through the wave's own LDS tile
 // for the transposing read.  A wave goes 32 positions at a time; the next
 // keys are fetched once the scores are done, the next values once these are
-// in LDS.
+// in LDS.  Bound by the read of the pages.
+// MERGE: a block's four waves are the shares of one (row, key head, heads) and
+// finish it in LDS; without, shares meet in qsa_gqa_merge (64 rows of 600-1400
+// keys, 16 heads on 8 of 128: 68 + 6 us so, 69 us here, 3.9 TB/s).
 // ---------------------------------------------------------------------------
-template <int KS, int ET>  // D <= 32*KS, E <= 16*ET
+struct GqaFinish {
+  const float* sink;
+  const bf16_t* gate;
+  bf16_t* out;
+  long long gstride, ostride;
+  float out_scale;
+};
+
+template <int KS, int ET, bool MERGE>  // D <= 32*KS, E <= 16*ET
 __global__ void __launch_bounds__(256, KS <= 4 && ET <= 8 ? 2 : 1)
 qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                   const bf16_t* __restrict__ vc,
@@ -124,13 +135,13 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                   const int* __restrict__ row_len,
                   float* __restrict__ part_o, float* __restrict__ part_ml,
                   int H, int G, int D, int E, float scale2, int NS,
-                  int units) {
+                  int units, GqaFinish fin) {
   constexpr int VP = 16 * ET + 16;
   constexpr int VG = 2 * ET;                      // 16 B groups per V row
   __shared__ __attribute__((aligned(16))) bf16_t vt_all[4][32 * VP];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int unit = blockIdx.x * 4 + wave;
-  if (unit >= units) return;
+  if (unit >= units) return;                      // MERGE: never
   bf16_t* vt = vt_all[wave];
   const int RG = H / G, HT = (RG + 15) / 16;
   const int split = unit % NS;
@@ -256,6 +267,56 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
     l += __shfl_xor(l, 16, QSA_WAVE);
     l += __shfl_xor(l, 32, QSA_WAVE);
   }
+  if constexpr (MERGE) {
+    // [16 heads][E] of every wave where its values were
+    __shared__ float ml[4][16][2];
+    float* mine = reinterpret_cast<float*>(vt);
+    __builtin_amdgcn_wave_barrier();
+    if (hi == 0) {
+      ml[wave][col][0] = m;
+      ml[wave][col][1] = l;
+    }
+#pragma unroll
+    for (int t = 0; t < ET; ++t)
+      *reinterpret_cast<f32x4_v*>(mine + col * (16 * ET) + t * 16 + hi * 4) =
+          acc[t];
+    __syncthreads();
+    const int heads = min(16, RG - ht * 16);
+    for (int i = threadIdx.x; i < heads * (E / 2); i += 256) {
+      const int hd = i / (E / 2), e = i % (E / 2) * 2;
+      const int h = g * RG + ht * 16 + hd;
+      const float sk = fin.sink ? fin.sink[h] * LOG2E : NEG_BIG;
+      float top = sk;
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        if (ml[w][hd][1] > 0.f) top = fmaxf(top, ml[w][hd][0]);
+      float den = fin.sink ? exp2_hw(sk - top) : 0.f, a0 = 0.f, a1 = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        if (!(ml[w][hd][1] > 0.f)) continue;      // a share without keys
+        const float f = exp2_hw(ml[w][hd][0] - top);
+        den = fmaf(f, ml[w][hd][1], den);
+        const float2 v = *reinterpret_cast<const float2*>(
+            reinterpret_cast<const float*>(vt_all[w]) + hd * (16 * ET) + e);
+        a0 = fmaf(f, v.x, a0);
+        a1 = fmaf(f, v.y, a1);
+      }
+      const float inv = den > 0.f ? fin.out_scale / den : 0.f;
+      a0 *= inv;
+      a1 *= inv;
+      if (fin.gate) {
+        const float2 gv = bf16x2_to_f32x2(
+            *reinterpret_cast<const unsigned int*>(
+                fin.gate + row * fin.gstride + (long long)h * E + e));
+        a0 /= 1.f + __expf(-gv.x);
+        a1 /= 1.f + __expf(-gv.y);
+      }
+      *reinterpret_cast<unsigned int*>(fin.out + row * fin.ostride +
+                                       (long long)h * E + e) =
+          cvt_bf16x2(a0, a1);
+    }
+    return;
+  }
   if (hg < RG) {
     const long long o = (row * H + head) * NS + split;
     if (hi == 0) {
@@ -356,21 +417,30 @@ extern "C" void qsa_gqa_rows_mfma_launch(
   const int units = R * G * ((H / G + 15) / 16) * NS;
   dim3 grid((unsigned)((units + 3) / 4));
   const float scale2 = scale * LOG2E;
+  const GqaFinish fin{sink, gate, out, gstride, ostride, out_scale};
 #define QSA_GM(K, V)                                                          \
-  hipLaunchKernelGGL((qsa_gqa_rows_mfma<K, V>), grid, dim3(256), 0, st, q,    \
-                     kc, vc, block_table, max_pages, row_item, row_len,       \
-                     part_o, part_ml, H, G, D, E, scale2, NS, units)
+  if (part_o)                                                                 \
+    hipLaunchKernelGGL((qsa_gqa_rows_mfma<K, V, false>), grid, dim3(256), 0,  \
+                       st, q, kc, vc, block_table, max_pages, row_item,       \
+                       row_len, part_o, part_ml, H, G, D, E, scale2, NS,      \
+                       units, fin);                                           \
+  else                                                                        \
+    hipLaunchKernelGGL((qsa_gqa_rows_mfma<K, V, true>), grid, dim3(256), 0,   \
+                       st, q, kc, vc, block_table, max_pages, row_item,       \
+                       row_len, part_o, part_ml, H, G, D, E, scale2, NS,      \
+                       units, fin)
 #define QSA_GM_E(K)                                                           \
-  if (E <= 32) QSA_GM(K, 2);                                                  \
-  else if (E <= 64) QSA_GM(K, 4);                                             \
-  else if (E <= 128) QSA_GM(K, 8);                                            \
-  else QSA_GM(K, 16)
+  if (E <= 32) { QSA_GM(K, 2); }                                              \
+  else if (E <= 64) { QSA_GM(K, 4); }                                         \
+  else if (E <= 128) { QSA_GM(K, 8); }                                        \
+  else { QSA_GM(K, 16); }
   if (D <= 32) { QSA_GM_E(1); }
   else if (D <= 64) { QSA_GM_E(2); }
   else if (D <= 128) { QSA_GM_E(4); }
   else { QSA_GM_E(8); }
 #undef QSA_GM_E
 #undef QSA_GM
+  if (!part_o) return;
   const long long total = (long long)R * H;
   if (NS > 8)
     hipLaunchKernelGGL((qsa_gqa_merge<4>), dim3((unsigned)total), dim3(256),

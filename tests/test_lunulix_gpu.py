@@ -277,6 +277,46 @@ def test_grouped_attention(H, G, Dm, E, dtype):
             close(out, ref[start:start + n], dtype)
 
 
+@pytest.mark.parametrize("R,H,G,Dm,E", [
+    (64, 16, 8, 128, 128), (129, 34, 2, 40, 24), (513, 1, 1, 256, 136)])
+def test_grouped_attention_many_rows(R, H, G, Dm, E):
+    """Enough rows for a block to finish its own: lengths without keys for
+    some of its four shares, none at all, ends of pages."""
+    g = gen(R)
+    T, scale = 700, 0.8 * Dm ** -0.5
+    q, k, v = (rnd(g, n, m, d, dtype=BF)
+               for n, m, d in ((T, H, Dm), (T, G, Dm), (T, G, E)))
+    sink, gate = rnd(g, H) + 1.0, rnd(g, T, H * E, dtype=BF)
+    pages = [7, 2, 9, 4, 1, 3, 10, 0, 5, 8, 6]
+    kc = torch.full((11, G, 64, Dm), 50.0, dtype=BF)
+    vc = torch.full((11, G, 64, E), float("nan"), dtype=BF)
+    for t in range(T):
+        kc[pages[t // 64], :, t % 64] = k[t]
+        vc[pages[t // 64], :, t % 64] = v[t]
+    bt = torch.tensor([pages], dtype=torch.int32, device=DEV)
+    edge = torch.tensor([0, 31, 63, 64, 127, 128, 191, 256, 699])
+    idx = torch.cat([edge, torch.randint(0, T, (R - len(edge),),
+                                         generator=g)])
+    qf = q.reshape(T, -1)[idx].to(DEV)
+    length = (idx + 1).int().to(DEV)
+    length[-1] = 0
+    for s, gt, mult in ((sink, gate, 0.7),
+                        (torch.full((H,), -1e30), None, 1.0)):
+        want = O.sink_attention(q.double(), k.double(), v.double(), scale,
+                                s.double()).reshape(T, -1)
+        if gt is not None:
+            want = want * O.sigmoid(gt.double()) * mult
+        want = want[idx]
+        want[-1] = 0.0
+        out = torch.zeros(R, H * E + 8, dtype=BF, device=DEV)
+        D.gqa_rows(qf, kc.to(DEV), vc.to(DEV), bt, i32(*[0] * R), length,
+                   s.to(DEV) if gt is not None else None,
+                   None if gt is None else gt[idx].to(DEV),
+                   out[:, :H * E], H, scale, mult)
+        close(out[:, :H * E], want, BF)
+        assert not out[:, H * E:].any()
+
+
 def test_portions_of_several_sequences():
     """One launch over portions of two sequences, rows behind each other."""
     g = gen(9)
