@@ -1,6 +1,6 @@
 // FP8 (OCP e4m3) weight-streaming decode GEMM for CDNA4 (gfx950):
 // C[M,N] = A[M,K] @ (s[N] * Q[N,K])^T, M <= 32, A bf16, Q fp8, C bf16.
-// Serves the K4 agent-LLM decode projections.
+// Serves the decode projections of the agents' language models.
 //
 // The bf16 skinny kernel (skinny_gemm.hip) is HBM-bound on the WEIGHT
 // stream (PMC: ~3% MFMA util); its ceiling is W bytes / 6.3 TB/s.  FP8

@@ -102,6 +102,27 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
                      (t & 1) * (p.N >> 5)
                : (int)blockIdx.x * TILES + t;
   };
+  // what the results need besides the sums is fetched ahead of the stream: at
+  // the end each of these would be a memory latency of its own (2048 x 2048
+  // fp8, 1 row: 4.5 -> 4.1 us; 4096 x 14336: 15.0 -> 14.3)
+  constexpr int OUT = (GLU ? TILES / 2 : TILES) * MT * 256;
+  constexpr int NI = (OUT + WAVES * 64 - 1) / (WAVES * 64);
+  float sc[NI][GLU ? 2 : 1];
+  bf16_t old[NI], nw[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int idx = min(tid + i * WAVES * 64, OUT - 1);
+    const int r = (idx >> 6) & 3, m = (idx >> 8) % MT, j = (idx >> 8) / MT;
+    if constexpr (FP8)
+#pragma unroll
+      for (int e = 0; e < (GLU ? 2 : 1); ++e)
+        sc[i][e] = p.scale[tile_of(GLU ? 2 * j + e : j) * 16 + col];
+    if constexpr (RES) {
+      const int row = m * 16 + hi * 4 + r, c = tile_of(j) * 16 + col;
+      old[i] = p.C[(long long)(row < p.M ? row : 0) * p.N + c];
+      nw[i] = p.norm_w[c];
+    }
+  }
   const u32x4_v* wp[TILES];
 #pragma unroll
   for (int t = 0; t < TILES; ++t)
@@ -193,15 +214,17 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
         red[wave][(t * MT + m) * 4 + r][lane] = acc[t][m][r];
   __syncthreads();
 
-  constexpr int OUT = (GLU ? TILES / 2 : TILES) * MT * 256;
-  for (int idx = tid; idx < OUT; idx += WAVES * 64) {
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int idx = tid + i * WAVES * 64;
+    if (OUT % (WAVES * 64) != 0 && idx >= OUT) break;
     const int r = (idx >> 6) & 3, m = (idx >> 8) % MT, j = (idx >> 8) / MT;
     const int row = m * 16 + (lane >> 4) * 4 + r;
-    auto total = [&](int t) {
+    auto total = [&](int t, int e) {
       float v = 0.f;
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) v += red[w][(t * MT + m) * 4 + r][lane];
-      if constexpr (FP8) v *= p.scale[tile_of(t) * 16 + col];
+      if constexpr (FP8) v *= sc[i][e];
       return v;
     };
     const float inv = NORM ? inv_s[row] : 1.f;
@@ -211,17 +234,16 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
       return PACK ? packed_at(row, ncol, MT) : (long long)row * width + ncol;
     };
     if constexpr (GLU) {
-      const float g = total(2 * j) * inv, u = total(2 * j + 1) * inv;
+      const float g = total(2 * j, 0) * inv, u = total(2 * j + 1, GLU) * inv;
       if (live)
         p.C[place(p.N >> 1)] = cvt_bf16(g / (1.f + __expf(-g)) * u);
     } else if constexpr (RES) {
-      bf16_t* at = p.C + (long long)(live ? row : 0) * p.N + ncol;
-      const float v = bf16_to_f32(*at) + total(j);
+      const float v = bf16_to_f32(old[i]) + total(j, 0);
       const bf16_t b = cvt_bf16(v);
       if (live) {
-        *at = b;
+        p.C[(long long)row * p.N + ncol] = b;
         p.next[place(p.N)] = cvt_bf16(bf16_to_f32(b) *
-                                      bf16_to_f32(p.norm_w[ncol]));
+                                      bf16_to_f32(nw[i]));
       }
       float q = v * v;
 #pragma unroll
@@ -230,7 +252,7 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
       if (live && col == 0)
         p.ss_out[row * ((parts + 3) & ~3) + (ncol >> 4)] = q;
     } else {
-      const float v = total(j) * inv;
+      const float v = total(j, 0) * inv;
       if (live) p.C[(long long)row * p.N + ncol] = cvt_bf16(v);
     }
   }
