@@ -19,8 +19,10 @@
 //   - The waves of a block merge in LDS.  One block per (row, kv head) stores
 //     the result; several leave (o, m, l) for qsa_attn_reduce.
 //   - FUSE is a decoding step's attention: q is rotated in registers, and the
-//     wave with the last page first writes the rotated new key and the new
-//     value to the cache, so that no launch has to come before.
+//     wave with the last page writes the rotated new key and the new value to
+//     the cache, so that no launch has to come before.  It reads the page
+//     beside that and fills their place in from LDS: waiting for its own
+//     stores cost a round trip to memory.
 // 192 rows of 400-1000 keys, 32/8 heads of 128: rotation 11, attention 172,
 // merge 7 us as separate kernels with a wave per share, 130 us here (4.2 TB/s); 16
 // rows of 1536-2048: 5 + 35 + 9, 29 + 5.
@@ -82,6 +84,8 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   constexpr int KSTEPS = D / 32;      // QK^T k-steps (4 for D=128)
   constexpr int DTILES = D / 16;      // PV d-tiles (8 for D=128)
   extern __shared__ float smem[];     // [NW][R][D] o, [NW][16] m, [NW][16] l
+  // the new key and value: one wave of a block has the last page
+  __shared__ __attribute__((aligned(16))) unsigned short fresh[FUSE ? 2 * D : 8];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int split = blockIdx.x % p.NS;
@@ -121,18 +125,9 @@ qsa_paged_attn_mfma(DecodeArgs p) {
           kf[pt][ks] = *reinterpret_cast<const bf16x8_a*>(
               kbase + ((ks * 4 + hi) * QSA_PAGE + pt * 16 + col) * 8);
     };
-    // the last page is read by this wave alone, after its own stores
-    auto stores_done = [&] {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    };
     bf16x8_a kf[4][KSTEPS];
     int page = btab[first];
-    // keys of the first page are under way before anything else, unless the
-    // new one still has to get there
-    const bool wait_first = FUSE && first == npages - 1;
-    if (!wait_first) load_k(page, kf);
+    load_k(page, kf);                 // under way before anything else
     if constexpr (FUSE) {
       const long long at = (long long)(seqlen - 1) * (D / 2) + hi * 8;
 #pragma unroll
@@ -160,19 +155,24 @@ qsa_paged_attn_mfma(DecodeArgs p) {
           unsigned short* kp = p.kw + tile + (lane * QSA_PAGE + pin) * 8;
           *reinterpret_cast<bf16x8_a*>(kp) = x;
           *reinterpret_cast<bf16x8_a*>(kp + D / 2 * QSA_PAGE) = y;
+          *reinterpret_cast<bf16x8_a*>(fresh + d) = x;
+          *reinterpret_cast<bf16x8_a*>(fresh + d + D / 2) = y;
         }
 #pragma unroll
-        for (int i = 0; i < D; i += 64)
-          p.vw[tile + (long long)(i + lane) * QSA_PAGE + pin] =
-              p.v[row + i + lane];
+        for (int i = 0; i < D; i += 64) {
+          const unsigned short x = p.v[row + i + lane];
+          p.vw[tile + (long long)(i + lane) * QSA_PAGE + pin] = x;
+          fresh[D + i + lane] = x;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
       }
     }
 
-    if (wait_first) {
-      stores_done();
-      load_k(page, kf);
-    }
-    for (int pi = first; pi < npages; pi += step) {
+    // patch: the row's last page, which came from memory with or without the
+    // new token, gets its place filled in from LDS
+    auto walk = [&](int pi, auto patch) {
       const bool more = pi + step < npages;
       const int next = more ? btab[pi + step] : 0;
       const long long head = (long long)page * p.KVH + kvh;
@@ -187,6 +187,16 @@ qsa_paged_attn_mfma(DecodeArgs p) {
               vbase + (dt * 16 + col) * QSA_PAGE + half * 32 + hi * 8);
       };
       load_v(0);
+      if constexpr (patch.value) {
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          const bf16x8_a x = *reinterpret_cast<const bf16x8_a*>(
+              fresh + ks * 32 + hi * 8);
+#pragma unroll
+          for (int pt = 0; pt < 4; ++pt)
+            if (pt * 16 + col == nvalid - 1) kf[pt][ks] = x;
+        }
+      }
       // ---- scores: 4 pos-tiles x KSTEPS MFMAs ---------------------------
       // A-frag: lane holds K[pos = pt*16 + col][k = ks*32 + hi*8 + e]
       f32x4_a sc[4];
@@ -200,10 +210,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         sc[pt] = acc;
       }
       load_v(1);
-      if (more) {
-        if (FUSE && pi + step == npages - 1) stores_done();
-        load_k(next, kf);
-      }
+      if (more) load_k(next, kf);
       // scale + mask invalid positions; C layout: row pos = hi*4 + r,
       // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
       float pagemax = -3.0e38f;
@@ -251,6 +258,23 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       psum += __shfl_xor(psum, 32, QSA_WAVE);
       lsum = lsum * alpha + psum;
 
+      if constexpr (patch.value) {
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt) {
+          const unsigned int x = fresh[D + dt * 16 + col];
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            const int e = nvalid - 1 - half * 32 - hi * 8;
+            u32x4_v u = __builtin_bit_cast(u32x4_v, vf[half][dt]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              if (e == 2 * i) u[i] = (u[i] & 0xffff0000u) | x;
+              if (e == 2 * i + 1) u[i] = (u[i] & 0xffffu) | x << 16;
+            }
+            vf[half][dt] = __builtin_bit_cast(bf16x8_a, u);
+          }
+        }
+      }
       // ---- PV: two 32-pos halves ---------------------------------------
       // A-frag needs lane (head=col, hi) to hold P[head][pos = hi*8 + e]:
       // packed pairs come from source lanes (same col) with hi' = (2*hi)&3
@@ -281,7 +305,11 @@ qsa_paged_attn_mfma(DecodeArgs p) {
               pa, vf[half][dt], o_acc[dt], 0, 0, 0);
       }
       page = next;
-    }
+    };
+    int pi = first;
+    for (; pi < npages - (FUSE ? 1 : 0); pi += step)
+      walk(pi, std::false_type{});
+    if (FUSE && pi == npages - 1) walk(pi, std::true_type{});
   }
 
   // ---- the waves of the block meet: O C-layout row = head = hi*4 + r -----

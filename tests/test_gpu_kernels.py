@@ -527,6 +527,10 @@ def test_paged_attn_step(ext, B, QH, KVH, D, longest):
         lens[3] = 0
     kc, vc, bt = _make_paged_kv(B, KVH, D, lens.tolist(),
                                 sum(-(-n // 64) for n in lens.tolist()) + 1)
+    for i, n in enumerate(lens.tolist()):         # the new token's place
+        if n:
+            kc[bt[i, (n - 1) // 64], :, :, (n - 1) % 64] = float("nan")
+            vc[bt[i, (n - 1) // 64], :, :, (n - 1) % 64] = float("nan")
     kc2, vc2 = kc.clone(), vc.clone()
     rot = torch.rand(longest + 1, D // 2, generator=g) * 6.28
     cos, sin = rot.cos().to(dev()), rot.sin().to(dev())
