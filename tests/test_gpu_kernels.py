@@ -32,6 +32,31 @@ def test_rmsnorm(ext):
     torch.testing.assert_close(y.float().cpu(), ref, atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("rows", [1, 4, 7])
+@pytest.mark.parametrize("H", [8, 384, 512, 520, 1024, 1032])
+def test_rmsnorm_narrow(ext, rows, H):
+    """Rows of one wave, up to one and two groups and just beyond; a rounding
+    to bf16 of the result and of the residual each."""
+    g = torch.Generator().manual_seed(H + rows)
+    x, res, w = (torch.randn(*s, generator=g).bfloat16()
+                 for s in ((rows, H), (rows, H), (H,)))
+
+    def norm(t):
+        t = t.double()
+        return t * (t.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * \
+            w.double()
+
+    y = ext.rmsnorm(x.to(dev()), w.to(dev()), 1e-5).cpu().double()
+    assert ((y - norm(x)).abs() <= 2 ** -8 * norm(x).abs() + 1e-6).all()
+    r = res.to(dev())
+    y = ext.rmsnorm_residual(x.to(dev()), r, w.to(dev()), 1e-5).cpu().double()
+    total = (x.float() + res.float()).bfloat16()
+    assert torch.equal(r.cpu(), total)
+    want = norm(total)
+    # the mean square is the exact sums': 2**-9 of rounding either way
+    assert ((y - want).abs() <= 2 ** -7 * want.abs() + 1e-6).all()
+
+
 def test_rmsnorm_residual(ext):
     torch.manual_seed(1)
     x = torch.randn(17, 4096, dtype=torch.bfloat16, device=dev())
