@@ -294,8 +294,8 @@ class LlamaModel:
 
     def _decode_attention(self, qkv: torch.Tensor, L: dict, li: int,
                           kv: PagedKVCache, block_table: torch.Tensor,
-                          seq_lens: torch.Tensor,
-                          step: bool = False) -> torch.Tensor:
+                          seq_lens: torch.Tensor, step: bool = False,
+                          warm: tuple = ()) -> torch.Tensor:
         """One token per row: rotation, cache append, attention."""
         if "bqkv" in L:
             qkv = qkv + L["bqkv"]
@@ -304,7 +304,7 @@ class LlamaModel:
         q, k, v = self._split_qkv(qkv, qkv.shape[0])
         return D.paged_attn_step(q, k, v, kv.k[li], kv.v[li], self.rope_cos,
                                  self.rope_sin, block_table, seq_lens,
-                                 self.scale, step)
+                                 self.scale, step, warm)
 
     def _streams_fp8(self) -> bool:
         """Whether _decode_fp8 serves this model: every projection packed,
@@ -330,7 +330,8 @@ class LlamaModel:
             qkv = D.norm_linear_fp8(x, ss, n, B, eps, L["wqkv_f8"],
                                     *L["wqkv"].shape)
             attn = self._decode_attention(qkv, L, li, kv, block_table,
-                                          seq_lens, step=True)
+                                          seq_lens, True,
+                                          (L["wdown_f8"][0], L["wo_f8"][0]))
             x, ss = D.linear_residual_fp8(
                 attn if attn.dim() == 4 else attn.view(B, -1), L["wo_f8"],
                 *L["wo"].shape, res, L["mlp_norm"])

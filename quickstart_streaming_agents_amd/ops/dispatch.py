@@ -170,13 +170,17 @@ def paged_attn_decode(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
 
 
 def paged_attn_step(q, k, v, kc, vc, cos_t, sin_t, block_table, seq_lens,
-                    scale: float, step: bool = False) -> torch.Tensor:
+                    scale: float, step: bool = False,
+                    warm: list = ()) -> torch.Tensor:
     """One token per row: q and k rotated to position seq_lens - 1, k and v
     appended to the cache, attention -> [B, QH, D].  `step` (GPU) returns step
-    rows for linear_residual_fp8 instead."""
+    rows for linear_residual_fp8 instead.  `warm`: up to two tensors that the
+    launches behind read, for compute units that a small step leaves idle to
+    fetch towards the last-level cache."""
     if _cuda(q):
         return ext().paged_attn_step(q, k, v, kc, vc, cos_t, sin_t,
-                                     block_table, seq_lens, scale, step)
+                                     block_table, seq_lens, scale, step,
+                                     list(warm))
     rope_kv_append(q, k, v, kc, vc, cos_t, sin_t, block_table, seq_lens)
     return paged_attn_decode(q, kc, vc, block_table, seq_lens, scale)
 

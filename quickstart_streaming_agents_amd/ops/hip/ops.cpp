@@ -43,7 +43,8 @@ extern "C" void qsa_paged_attn_mfma_launch(
     const unsigned short*, const unsigned short*, const unsigned short*,
     unsigned short*, unsigned short*, const float*, const float*, const int*,
     const int*, float*, float*, unsigned short*, float, int, int, int, int,
-    int, long long, long long, int, int, int, hipStream_t);
+    int, long long, long long, int, int, int, const void* const*,
+    const long long*, hipStream_t);
 extern "C" void qsa_kv_append_launch(const unsigned short*,
                                      const unsigned short*, unsigned short*,
                                      unsigned short*, const int*, const int*,
@@ -225,7 +226,8 @@ static torch::Tensor decode_attention(
     const torch::Tensor& q, const torch::Tensor* k, const torch::Tensor* v,
     torch::Tensor& kc, torch::Tensor& vc, const float* cos_t,
     const float* sin_t, const torch::Tensor& block_table,
-    const torch::Tensor& seq_lens, double scale, bool step) {
+    const torch::Tensor& seq_lens, double scale, bool step,
+    const std::vector<torch::Tensor>& warm = {}) {
   CHK_DEV(q); CHK_BF16(q); CHK_BF16(kc); CHK_BF16(vc);
   CHK_CONT(kc); CHK_CONT(vc); CHK_I32(block_table); CHK_I32(seq_lens);
   CHK_CONT(block_table);
@@ -252,13 +254,22 @@ static torch::Tensor decode_attention(
     part_o = torch::empty({B, QH, ns, D}, opts_f);
     part_ml = torch::empty({B, QH, ns, 2}, opts_f);
   }
+  TORCH_CHECK(warm.size() <= 2, "at most two tensors to read ahead");
+  const void* at[2] = {nullptr, nullptr};
+  long long bytes[2] = {0, 0};
+  for (size_t i = 0; i < warm.size(); ++i) {
+    CHK_DEV(warm[i]); CHK_CONT(warm[i]);
+    at[i] = warm[i].data_ptr();
+    bytes[i] = reinterpret_cast<uintptr_t>(at[i]) & 15
+        ? 0 : (long long)warm[i].nbytes();
+  }
   qsa_paged_attn_mfma_launch(
       u16(q), k ? u16(*k) : nullptr, v ? u16(*v) : nullptr, u16m(kc), u16m(vc),
       cos_t, sin_t, block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
       ns > 1 ? part_o.data_ptr<float>() : nullptr,
       ns > 1 ? part_ml.data_ptr<float>() : nullptr, u16m(out), (float)scale, B,
       QH, KVH, max_pages, D, q.stride(0), k ? k->stride(0) : 0, waves, ns, mt,
-      cur_stream());
+      at, bytes, cur_stream());
   return out;
 }
 
@@ -274,7 +285,7 @@ torch::Tensor paged_attn_step(torch::Tensor q, torch::Tensor k,
                               torch::Tensor vc, torch::Tensor cos_t,
                               torch::Tensor sin_t, torch::Tensor block_table,
                               torch::Tensor seq_lens, double scale,
-                              bool step) {
+                              bool step, std::vector<torch::Tensor> warm) {
   // rope_kv_append and paged_attn_decode in one; q, k and v stay as they
   // are.  step: the result as step rows instead of [B, QH, D]
   CHK_BF16(k); CHK_BF16(v); CHK_F32(cos_t); CHK_F32(sin_t);
@@ -292,7 +303,7 @@ torch::Tensor paged_attn_step(torch::Tensor q, torch::Tensor k,
               "cos/sin [positions, D/2]");
   return decode_attention(q, &k, &v, kc, vc, cos_t.data_ptr<float>(),
                           sin_t.data_ptr<float>(), block_table, seq_lens,
-                          scale, step);
+                          scale, step, warm);
 }
 
 void kv_append(torch::Tensor knew, torch::Tensor vnew, torch::Tensor kc,
@@ -762,7 +773,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attn_decode", &paged_attn_decode,
         "paged-attention decode (bf16, GQA, page=64)");
   m.def("paged_attn_step", &paged_attn_step,
-        "a decoding step's rotation, cache append and attention");
+        "a decoding step's rotation, cache append and attention",
+        py::arg("q"), py::arg("k"), py::arg("v"), py::arg("kc"),
+        py::arg("vc"), py::arg("cos"), py::arg("sin"), py::arg("block_table"),
+        py::arg("seq_lens"), py::arg("scale"), py::arg("step"),
+        py::arg("warm") = std::vector<torch::Tensor>());
   m.def("kv_append", &kv_append, "append one step's k/v to the paged cache");
   m.def("rope_kv_append", &rope_kv_append,
         "fused decode rope + paged-cache append");

@@ -64,7 +64,27 @@ struct DecodeArgs {
   float scale;
   int QH, KVH, max_pages, NS, mt;      // mt: row tiles of packed rows, or 0
   long long qstride, kvstride;
+  // blocks beyond the attention's read these (in 16 bytes)
+  int blocks;
+  const u32x4_v* warm[2];
+  long long warm_n[2];
 };
+
+// Reads memory for the launches that follow, towards the last-level cache.
+template <int THREADS>
+__device__ __forceinline__ void qsa_warm(const u32x4_v* at, long long n,
+                                         int block, int blocks) {
+  constexpr int U = 8;
+  for (long long i = (long long)block * THREADS * U + threadIdx.x; i < n;
+       i += (long long)blocks * THREADS * U) {
+    u32x4_v v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = at[min(i + u * THREADS, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) asm volatile("" ::"v"(v[u]));
+  }
+}
 
 // rotate elements k0.. and k0 + D/2.. of a row held in two fragments
 __device__ __forceinline__ void rotate_pair(bf16x8_a& a, bf16x8_a& b,
@@ -88,6 +108,12 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   __shared__ __attribute__((aligned(16))) unsigned short fresh[FUSE ? 2 * D : 8];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (FUSE && (int)blockIdx.x >= p.blocks) {
+    for (int i = 0; i < 2; ++i)
+      qsa_warm<NW * 64>(p.warm[i], p.warm_n[i], blockIdx.x - p.blocks,
+                        gridDim.x - p.blocks);
+    return;
+  }
   const int split = blockIdx.x % p.NS;
   const int bk = blockIdx.x / p.NS;
   const int b = bk / p.KVH;
@@ -412,12 +438,28 @@ extern "C" void qsa_paged_attn_mfma_launch(
     const float* sin_t, const int* block_table, const int* seq_lens,
     float* part_o, float* part_ml, unsigned short* out, float scale, int B,
     int QH, int KVH, int max_pages, int D, long long qstride,
-    long long kvstride, int waves, int NS, int mt, hipStream_t stream) {
-  const DecodeArgs p{q, kc, vc, block_table, seq_lens, part_o, part_ml, out,
-                     k, v, kc, vc, cos_t, sin_t, scale, QH, KVH, max_pages,
-                     NS, mt, qstride, kvstride};
-  const dim3 grid((unsigned)((long long)B * KVH * NS)), block(waves * 64);
+    long long kvstride, int waves, int NS, int mt, const void* const* warm,
+    const long long* warm_bytes, hipStream_t stream) {
+  DecodeArgs p{q, kc, vc, block_table, seq_lens, part_o, part_ml, out,
+               k, v, kc, vc, cos_t, sin_t, scale, QH, KVH, max_pages,
+               NS, mt, qstride, kvstride, 0, {nullptr, nullptr}, {0, 0}};
+  dim3 grid((unsigned)((long long)B * KVH * NS)), block(waves * 64);
   if (grid.x == 0) return;
+  p.blocks = (int)grid.x;
+  // Few blocks of few pages leave most of the chip idle for some 9 us: as much
+  // as memory delivers meanwhile, or nothing, since a projection whose weights
+  // are there in part waits for the rest.  2048-wide decoder, 16 layers, output
+  // and down projections of 21 MB: 1 row of 700 keys 618 -> 605 us a step, of
+  // 120 578 -> 552, 8 rows 715 -> 678; cut to 24 MB of a 4096-wide one's 75 it
+  // cost 1-2%.
+  const long long bytes = warm_bytes[0] + warm_bytes[1];
+  if (k && NS == 1 && grid.x <= 64 && bytes >= 16 && bytes <= 24 << 20) {
+    for (int i = 0; i < 2; ++i) {
+      p.warm[i] = static_cast<const u32x4_v*>(warm[i]);
+      p.warm_n[i] = warm_bytes[i] / 16;
+    }
+    grid.x = 256;
+  }
   const size_t lds = sizeof(float) * waves * ((size_t)QH / KVH * D + 32);
 #define QSA_DECODE(DD, NW)                                                  \
   if (D == DD && waves == NW) {                                             \

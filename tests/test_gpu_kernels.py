@@ -587,6 +587,31 @@ def test_paged_attn_step(ext, B, QH, KVH, D, longest):
         assert torch.equal(_from_step_rows(step, B), out.view(B, -1))
 
 
+@pytest.mark.parametrize("sizes", [(16,), (16 * 4097, 40), (1 << 20, 3),
+                                   (25 << 20, 16), (9, 7)])
+def test_paged_attn_step_reads_ahead(ext, sizes):
+    """What idle blocks read, ends included, changes nothing."""
+    g = torch.Generator().manual_seed(len(sizes))
+    lens = [300, 0, 65]
+    kc, vc, bt = _make_paged_kv(3, 4, 64, lens, 8)
+    rot = torch.rand(301, 32, generator=g)
+    qkv = torch.randn(3, 24 * 64, generator=g).bfloat16().to(dev())
+    q, k, v = (t.view(3, -1, 64) for t in qkv.split([1024, 256, 256], 1))
+    warm = [torch.ones(n, dtype=torch.uint8, device=dev()) for n in sizes]
+
+    def run(**more):
+        return ext.paged_attn_step(
+            q, k, v, kc, vc, rot.cos().to(dev()), rot.sin().to(dev()), bt,
+            torch.tensor(lens, dtype=torch.int32, device=dev()), 0.125, False,
+            **more)
+
+    out = run()
+    kept = kc.clone(), vc.clone()
+    assert torch.equal(out, run(warm=warm))
+    assert torch.equal(kept[0], kc) and torch.equal(kept[1], vc)
+    assert all((w == 1).all() for w in warm)
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(16, 256), (48, 768), (4096, 8192)])
 def test_skinny_bf16_rows(ext, M, N, K):
