@@ -15,7 +15,8 @@ from ..ops import dispatch as D
 class Linear:
     """y = x W^T.  On the GPU in bf16, decode-sized batches of the small
     shapes stream a packed copy of W (ops/hip/skinny_gemm.hip, the measured
-    winner there); everything else is a vendor GEMM."""
+    winner there) and larger ones of long K split it (ops/hip/rows_gemm.hip);
+    everything else is a vendor GEMM."""
 
     SKINNY_ROWS = 32
     SKINNY_MAX = 6144 * 4096
@@ -33,6 +34,8 @@ class Linear:
         if self.packed is not None and 1 <= x.shape[0] <= self.SKINNY_ROWS \
                 and x.stride(0) % 8 == 0:
             return D.skinny_linear(x, self.packed, n, k)
+        if D.rows_linear_ok(x, self.w):
+            return D.rows_linear(x, self.w)
         return F.linear(x, self.w)
 
 

@@ -216,7 +216,8 @@ class LlamaModel:
                 wf8: tuple | None = None) -> torch.Tensor:
         """Projection: decode-sized cuda batches go through the
         weight-streaming skinny GEMM — fp8 (W8A16, half the weight
-        stream) when packed, else bf16; everything else rocBLAS."""
+        stream) when packed, else bf16; batches beyond on a long K through
+        rows_gemm; everything else rocBLAS."""
         n, k = w.shape
         M = x.shape[0]
         if x.is_cuda and wf8 is not None:
@@ -241,6 +242,8 @@ class LlamaModel:
             # bf16 skinny wins only the small decode shapes (qkv/wo);
             # rocBLAS is at the bandwidth floor for the big-N ones
             return D.skinny_linear(x, wf, n, k)
+        if D.rows_linear_ok(x, w):
+            return D.rows_linear(x, w)
         return F.linear(x, w)
 
     def _tp_all_reduce(self, t: torch.Tensor) -> torch.Tensor:

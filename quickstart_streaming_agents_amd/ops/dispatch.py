@@ -197,6 +197,22 @@ def pack_weight_frag(w: torch.Tensor) -> torch.Tensor:
     return w.reshape(n // 16, 16, k // 32, 32).permute(0, 2, 1, 3).contiguous()
 
 
+def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x[M,K] @ W^T is rows_linear's: a decode batch beyond the skinny
+    kernels, and a long K beside few columns, where it beats the library at
+    every M (figures in ops/hip/rows_gemm.hip)."""
+    n, k = w.shape
+    return x.is_cuda and x.dim() == 2 and 32 < x.shape[0] <= 192 and \
+        k >= 3 * n and n * k >= 1 << 24 and n % 16 == 0 and k % 64 == 0 and \
+        x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and \
+        x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
+        (x.data_ptr() | w.data_ptr()) % 16 == 0
+
+
+def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    return lm_ext().rows_gemm(x, w)
+
+
 def skinny_linear(x: torch.Tensor, wf: torch.Tensor, n: int,
                   k: int) -> torch.Tensor:
     """x[M,K] @ W^T via the weight-streaming decode kernel (M <= 32)."""

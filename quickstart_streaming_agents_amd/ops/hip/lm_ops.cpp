@@ -126,6 +126,9 @@ extern "C" void qsa_window_attn_prefill_launch(const bf16_t*, long long,
     const int*, bf16_t*, int, int, int, int, int, float, hipStream_t);
 extern "C" void qsa_skinny_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     int, int, long long, long long, hipStream_t);
+extern "C" int qsa_rows_gemm_shares(int, int);
+extern "C" void qsa_rows_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
+    float*, int, int, int, long long, int, hipStream_t);
 
 // res [T, W] f32 updated in place; returns norm(res) * w (+ b), or res itself
 // in y's storage type when w is not given
@@ -880,6 +883,24 @@ Tensor skinny_gemm(Tensor a, Tensor wf, long N, long K) {
   return out;
 }
 
+// a @ w^T on W as it is stored, K split over the chip
+Tensor rows_gemm(Tensor a, Tensor w) {
+  CHK_DEV(a); chk_rows(a, "a"); CHK_CONT(w); CHK_SAME(a, w);
+  TORCH_CHECK(a.scalar_type() == at::kBFloat16, "bf16");
+  const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
+  TORCH_CHECK(M >= 1 && M <= 192 && a.size(1) == K, "M in [1, 192], K");
+  TORCH_CHECK(N >= 16 && N % 16 == 0 && K >= 64 && K % 64 == 0,
+              "N % 16, K % 64");
+  TORCH_CHECK(a.stride(0) % 8 == 0 && a.stride(0) < (1 << 24) &&
+                  aligned(a, 16) && aligned(w, 16), "alignment");
+  const int S = qsa_rows_gemm_shares(N, K);
+  auto out = torch::empty({M, N}, a.options());
+  auto part = torch::empty({S, M, N}, a.options().dtype(at::kFloat));
+  qsa_rows_gemm_launch(u16(a), u16(w), u16m(out), part.data_ptr<float>(), M,
+                       N, K, a.stride(0), S, cur_stream());
+  return out;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("residual_norm", &residual_norm,
         "f32 residual update (+ embedding row, + vector) and layer/rms norm");
@@ -912,4 +933,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "windowed flash attention with sink and gate (MFMA)");
   m.def("window_attn_ok", &window_attn_ok, "size support");
   m.def("skinny_gemm", &skinny_gemm, "packed-weight decode GEMM (M <= 32)");
+  m.def("rows_gemm", &rows_gemm, "long-K decode GEMM (M <= 192)");
 }

@@ -522,3 +522,20 @@ def test_preset_on_engine():
     assert len(out) == 2
     llm.release_all()
     assert llm.engine.kv.free_slots == llm.engine.kv.n_slots
+
+
+# ---- projections of larger decode batches -----------------------------------
+
+@pytest.mark.parametrize("M", [1, 33, 48, 49, 65, 97, 128, 129, 192])
+@pytest.mark.parametrize("N,K", [(16, 64), (144, 192), (2048, 8192)])
+def test_rows_gemm(M, N, K):
+    """Ends of row tiles, column blocks and shares of K; rows of a slice.  An
+    f32 sum of K products and a rounding to bf16."""
+    from quickstart_streaming_agents_amd.ops import lm_ext
+    g = gen(M + N)
+    x = rnd(g, M, K + 24, dtype=BF)[:, 8:K + 8].to(DEV)
+    w = rnd(g, N, K, dtype=BF).to(DEV)
+    got = lm_ext().rows_gemm(x, w).double()
+    a, b = x.double(), w.double()
+    bound = 2.0 ** -8 * (a @ b.T).abs() + K * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    assert ((got - a @ b.T).abs() <= bound).all()
