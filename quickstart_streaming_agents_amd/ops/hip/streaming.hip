@@ -15,7 +15,7 @@
 // chunk: 81 us).  So blocks count CHUNKS of consecutive events, which in a
 // stream span a few windows, in LDS and leave (windows spanned) * nkeys cells
 // in a workspace; qsa_window_merge adds them up, without atomics and in a fixed
-// order (33 us together).  A chunk whose span does not fit goes to the output
+// order (31 us together).  A chunk whose span does not fit goes to the output
 // with atomics, as do batches of a few chunks, where a second launch costs
 // more than their cells.
 // ---------------------------------------------------------------------------
@@ -165,20 +165,28 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
   }
 }
 
-// Block = 8 windows x 64 keys, a wave per two windows: the chunks that reach
-// these windows, in order, added to what other chunks left in the output.
-__global__ void __launch_bounds__(256)
+// Block = 8 windows x 64 keys, a wave per window: the chunks that reach it, in
+// order, added to what other chunks left in the output.  Bound by a chain of
+// latencies (spans, cells, output), so the output is fetched first and four
+// chunks' cells at a time: 288 x 1000 cells of 489 chunks 12.5 us with two
+// windows a wave, 10.6 here.
+__global__ void __launch_bounds__(512)
 qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
                  int blocks, int* __restrict__ counts,
                  float* __restrict__ sums, int has_value, int nwin,
                  int nkeys) {
   __shared__ int list[QSA_AGG_BLOCKS];
   __shared__ int2 range[QSA_AGG_BLOCKS];
-  __shared__ int wave_n[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int w0 = blockIdx.x * 8, k = blockIdx.y * 64 + lane;
+  __shared__ int wave_n[8];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w0 = blockIdx.x * 8, w = w0 + wave, k = blockIdx.y * 64 + lane;
+  const bool live = k < nkeys && w < nwin;
+  const long long slot = live ? (long long)k * nwin + w : 0;
+  int c = counts[slot];
+  float v = has_value ? sums[slot] : 0.f;
   int total = 0;
-  for (int base = 0; base < blocks; base += 256) {
+  for (int base = 0; base < blocks; base += 512) {
     const int b = base + tid;
     const int2 s = b < blocks ? span[b] : make_int2(0, 0);
     const bool in = s.y > 0 && s.x < w0 + 8 && s.x + s.y > w0;
@@ -186,9 +194,10 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
     if (lane == 0) wave_n[wave] = __popcll(m);
     __syncthreads();
     int at = total + __popcll(m & ((1ull << lane) - 1));
-    for (int w = 0; w < 4; ++w) {
-      if (w < wave) at += wave_n[w];
-      total += wave_n[w];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (i < wave) at += wave_n[i];
+      total += wave_n[i];
     }
     if (in) {
       list[at] = b;
@@ -196,50 +205,42 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
     }
     __syncthreads();
   }
-  const bool live = k < nkeys;
+  // in a stream most groups do not reach this window
+  int pc = 0;
+  float pv = 0.f;
+  for (int j0 = 0; j0 < total; j0 += 4) {
+    bool any = false, in[4];
+    int at[4];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int w = w0 + wave * 2 + u;
-    int c = 0;
-    float v = 0.f;
-    // four chunks at a time, their loads together; in a stream most groups
-    // do not reach this window
-    for (int j0 = 0; j0 < total; j0 += 4) {
-      bool any = false, in[4];
-      int at[4];
+    for (int j = 0; j < 4; ++j) {
+      at[j] = min(j0 + j, total - 1);
+      const int2 s = range[at[j]];
+      in[j] = j0 + j < total && w >= s.x && w < s.x + s.y;
+      any |= in[j];
+    }
+    if (!any) continue;                // uniform over the wave
+    int gc[4];
+    float gv[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int i = min(j0 + j, total - 1);
-        const int2 s = range[i];
-        in[j] = j0 + j < total && w >= s.x && w < s.x + s.y;
-        at[j] = in[j] ? i : -1;
-        any |= in[j];
-      }
-      if (!any) continue;              // uniform over the wave
-      int pc[4];
-      float pv[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        pc[j] = 0;
-        pv[j] = 0.f;
-        if (in[j] && live) {
-          const int* p = ws + (long long)list[at[j]] * 2 * QSA_AGG_CELLS +
-                         (w - range[at[j]].x) * nkeys + k;
-          pc[j] = *p;
-          if (has_value) pv[j] = __int_as_float(p[QSA_AGG_CELLS]);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        c += pc[j];
-        v += pv[j];
+    for (int j = 0; j < 4; ++j) {
+      gc[j] = 0;
+      gv[j] = 0.f;
+      if (in[j] && live) {
+        const int* p = ws + (long long)list[at[j]] * 2 * QSA_AGG_CELLS +
+                       (w - range[at[j]].x) * nkeys + k;
+        gc[j] = *p;
+        if (has_value) gv[j] = __int_as_float(p[QSA_AGG_CELLS]);
       }
     }
-    if (live && w < nwin) {
-      const long long slot = (long long)k * nwin + w;
-      counts[slot] += c;
-      if (has_value) sums[slot] += v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      pc += gc[j];
+      pv += gv[j];
     }
+  }
+  if (live) {
+    counts[slot] = c + pc;
+    if (has_value) sums[slot] = v + pv;
   }
 }
 
@@ -331,7 +332,8 @@ qsa_anomaly_batch(const float* __restrict__ series, const int* __restrict__ leng
   for (int a = 0; a < QSA_AR_MAXP; ++a) {
     bb[a] = wave_reduce_sum(bb[a]);
 #pragma unroll
-    for (int c = 0; c < QSA_AR_MAXP; ++c) G[a][c] = wave_reduce_sum(G[a][c]);
+    for (int c = 0; c < QSA_AR_MAXP; ++c)         // symmetric, to the last bit
+      G[a][c] = c < a ? G[c][a] : wave_reduce_sum(G[a][c]);
   }
 
   // ridge solve (G + lam I) [coef | y] = [b | x_next] by Gauss-Jordan, every
@@ -436,7 +438,7 @@ extern "C" void qsa_window_agg_launch(const long long* ts, const int* key,
                        nkeys, n, chunk, span, cells);
   if (ws)
     hipLaunchKernelGGL(qsa_window_merge,
-                       dim3((nwin + 7) / 8, (nkeys + 63) / 64), dim3(256), 0,
+                       dim3((nwin + 7) / 8, (nkeys + 63) / 64), dim3(512), 0,
                        stream, span, cells, blocks, counts, sums,
                        value ? 1 : 0, nwin, nkeys);
 }
