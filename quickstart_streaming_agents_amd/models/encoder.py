@@ -89,32 +89,20 @@ class EmbeddingEncoder:
 
     def _embed_rows(self, enc: list[list[int]]) -> torch.Tensor:
         """Mean-pooled final states [n, hidden] f32 of the token lists, all
-        rows in one concatenation without padding.  Keys and values go to
-        scratch pages, preallocated per item (slots nobody writes are never
-        used: item_len bounds the key range)."""
+        rows in one concatenation without padding."""
         import numpy as np
 
         from .layers import ints_to_device
         c, dev = self.cfg, self.device
         lens = np.array([len(x) for x in enc])
-        n, T = len(enc), int(lens.sum())
+        n = len(enc)
         off = np.cumsum(lens) - lens
-        item = np.repeat(np.arange(n), lens)
-        pos = np.arange(T) - off[item]
-        ppi = -(-int(lens.max()) // 64)      # pages per item
         nqb = -(-lens // self.QROWS)
         qb_item = np.repeat(np.arange(n), nqb)
         qb_pos0 = (np.arange(int(nqb.sum()))
                    - (np.cumsum(nqb) - nqb)[qb_item]) * self.QROWS
-        (toks, positions, slots, bt, qb_item, qb_pos0, off, lens_t,
-         start) = ints_to_device(
-            dev, np.concatenate(enc), pos, item * ppi * 64 + pos,
-            np.arange(n * ppi), qb_item, qb_pos0, off, lens, np.zeros(n))
-        bt = bt.view(n, ppi)
-        kc = torch.empty(n * ppi, c.n_heads, c.d_head // 8, 64, 8,
-                         dtype=self.dtype, device=dev)
-        vc = torch.empty(n * ppi, c.n_heads, c.d_head, 64, dtype=self.dtype,
-                         device=dev)
+        toks, qb_item, qb_pos0, off, lens_t = ints_to_device(
+            dev, np.concatenate(enc), qb_item, qb_pos0, off, lens)
         res = self.tok_embed.index_select(0, toks)
         mlp_out = None
         for Ly in self.layers:
@@ -123,14 +111,9 @@ class EmbeddingEncoder:
             else:
                 h = D.rmsnorm_residual(mlp_out, res, Ly["attn_norm"],
                                        c.norm_eps)
-            q, k, v = F.linear(h, Ly["wqkv"]) \
-                .view(T, 3, c.n_heads, c.d_head).unbind(1)
-            D.rope_kv_scatter(q, k, v, kc, vc, self.rope_cos, self.rope_sin,
-                              positions, slots)
-            # bidirectional varlen MFMA flash attention (CAUSAL=false)
-            attn = D.ext().paged_attn_prefill(
-                q, kc, vc, bt, qb_item, qb_pos0, off, start, lens_t,
-                self.scale, False, self.QROWS)
+            attn = D.ext().encoder_attn(
+                F.linear(h, Ly["wqkv"]), self.rope_cos, self.rope_sin, qb_item,
+                qb_pos0, off, lens_t, c.n_heads, self.scale)
             o = F.linear(attn, Ly["wo"])
             h = D.rmsnorm_residual(o, res, Ly["mlp_norm"], c.norm_eps)
             gu = F.linear(h, Ly["wgu"])

@@ -140,7 +140,7 @@ qsa_rmsnorm_kernel(const unsigned short* __restrict__ x,
 
 // The same for narrow rows, one wave each: no barrier, and every load of a row
 // is under way at once.  A block per row left most of its threads idle and was
-// bound by its latencies (6,600 x 384 with residual: 13.4 us, 8.0 here).
+// bound by its latencies (8,800 x 384 with residual: 13.4 us, 8.0 here).
 template <int GROUPS>                  // H <= 512 * GROUPS
 __global__ void __launch_bounds__(256)
 qsa_rmsnorm_narrow(const unsigned short* __restrict__ x,

@@ -108,6 +108,10 @@ extern "C" void qsa_hash_probe_launch(const long long*,
                                       const unsigned long long*, int*, int,
                                       unsigned int, long long, int,
                                       hipStream_t);
+extern "C" void qsa_encoder_attn_launch(
+    const unsigned short*, const float*, const float*, int, const int*,
+    const int*, const int*, const int*, unsigned short*, int, int, int, float,
+    hipStream_t);
 extern "C" int qsa_topk_block_docs(long long, long long);
 extern "C" void qsa_topk_launch(const float*, const float*, float*, int*,
                                 float*, int*, int, int, int, int, int,
@@ -685,6 +689,34 @@ torch::Tensor skinny_gemm_fp8_probe(torch::Tensor a, torch::Tensor qf,
   return out;
 }
 
+// rows of [q | k | v] of the items, blocks of 64 query rows -> [T, H*D]
+torch::Tensor encoder_attn(torch::Tensor qkv, torch::Tensor cos_t,
+                           torch::Tensor sin_t, torch::Tensor qb_item,
+                           torch::Tensor qb_t0, torch::Tensor off,
+                           torch::Tensor len, long heads, double scale) {
+  CHK_DEV(qkv); CHK_BF16(qkv); CHK_CONT(qkv);
+  CHK_F32(cos_t); CHK_F32(sin_t); CHK_CONT(cos_t); CHK_CONT(sin_t);
+  CHK_I32(qb_item); CHK_I32(qb_t0); CHK_I32(off); CHK_I32(len);
+  TORCH_CHECK(qkv.dim() == 2 && heads > 0 && heads % 4 == 0 &&
+                  qkv.size(1) % (3 * heads) == 0, "[T, 3 * heads * D]");
+  const long long A = qkv.size(1) / 3, D = A / heads;
+  TORCH_CHECK(D == 128 || D == 64, "D must be 64/128");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(qkv.data_ptr()) & 15) == 0,
+              "rows must be 16-byte aligned");
+  TORCH_CHECK(cos_t.dim() == 2 && cos_t.size(0) >= 1 &&
+                  cos_t.size(1) == D / 2 && sin_t.sizes() == cos_t.sizes(),
+              "cos/sin [positions, D/2]");
+  TORCH_CHECK(qb_item.numel() == qb_t0.numel() && off.numel() == len.numel(),
+              "maps");
+  auto out = torch::empty({qkv.size(0), A}, qkv.options());
+  qsa_encoder_attn_launch(
+      u16(qkv), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(),
+      (int)cos_t.size(0), qb_item.data_ptr<int>(), qb_t0.data_ptr<int>(),
+      off.data_ptr<int>(), len.data_ptr<int>(), u16m(out),
+      (int)qb_item.numel(), (int)heads, (int)D, (float)scale, cur_stream());
+  return out;
+}
+
 std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
                                        torch::Tensor docs, long k) {
   CHK_DEV(queries); CHK_CONT(queries); CHK_F32(queries); CHK_F32(docs);
@@ -783,6 +815,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fused decode rope + paged-cache append");
   m.def("rope_kv_scatter", &rope_kv_scatter,
         "prefill rotation and paged-cache write");
+  m.def("encoder_attn", &encoder_attn,
+        "rotation and bidirectional attention of projection rows");
   m.def("mean_rows", &mean_rows, "mean of each item's rows (f32)");
   m.def("kv_scatter", &kv_scatter, "scatter prefill k/v by slot ids");
   m.def("pack_weight_frag", &pack_weight_frag,

@@ -800,6 +800,41 @@ def test_rope_kv_scatter(ext, T, QH, KVH, D):
                 <= 2 ** -7 * b.float().abs() + 1e-6).all()
 
 
+@pytest.mark.parametrize("D,H", [(64, 8), (128, 4)])
+@pytest.mark.parametrize("lens", [[1], [64, 63, 65, 1, 130], [512, 3, 128]])
+def test_encoder_attn(ext, lens, D, H):
+    """Rows of q, k and v as the projection leaves them, items at tile edges,
+    blocks in any order; weights and results are rounded to bf16."""
+    g = torch.Generator().manual_seed(D + len(lens))
+    T, A = sum(lens), H * D
+    qkv = torch.randn(T, 3 * A, generator=g).bfloat16()
+    rot = torch.rand(512, D // 2, generator=g, dtype=torch.float64) * 6.28
+    cos, sin = rot.cos().float(), rot.sin().float()
+    off = np.cumsum(lens) - lens
+    blocks = [(i, t) for i, n in enumerate(lens) for t in range(0, n, 64)][::-1]
+    got = ext.encoder_attn(
+        qkv.to(dev()), cos.to(dev()), sin.to(dev()),
+        *(torch.tensor(x, dtype=torch.int32, device=dev())
+          for x in ([b[0] for b in blocks], [b[1] for b in blocks],
+                    off.tolist(), lens)), H, D ** -0.5).cpu().double()
+
+    def rotated(x, n):
+        a, b = x.float().chunk(2, -1)
+        c, s = cos[:n, None], sin[:n, None]
+        return torch.cat([a * c - b * s, a * s + b * c], -1).bfloat16() \
+            .double()
+
+    for o, n in zip(off, lens):
+        q, k, v = qkv[o:o + n].view(n, 3, H, D).unbind(1)
+        p = torch.einsum("ihd,jhd->hij", rotated(q, n), rotated(k, n))
+        p = (p * D ** -0.5).softmax(-1)
+        want = torch.einsum("hij,jhd->ihd", p, v.double()).reshape(n, A)
+        # of the weights 2**-9, of the result 2**-9, of a rotated number
+        # rounded the other way 2**-8 of some score of a few units
+        scale = torch.einsum("hij,jhd->ihd", p, v.double().abs()).reshape(n, A)
+        assert ((got[o:o + n] - want).abs() <= 2 ** -6 * scale + 1e-6).all()
+
+
 def test_mean_rows(ext):
     lens = [1, 3, 4, 5, 700]
     x = torch.randn(sum(lens), 520, device=dev()).bfloat16()
