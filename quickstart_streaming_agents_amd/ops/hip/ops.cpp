@@ -108,6 +108,10 @@ extern "C" void qsa_hash_probe_launch(const long long*,
                                       const unsigned long long*, int*, int,
                                       unsigned int, long long, int,
                                       hipStream_t);
+extern "C" void qsa_short_gemm_launch(const unsigned short*,
+                                      const unsigned short*, unsigned short*,
+                                      int, int, int, long long, int,
+                                      hipStream_t);
 extern "C" void qsa_encoder_attn_launch(
     const unsigned short*, const float*, const float*, int, const int*,
     const int*, const int*, const int*, unsigned short*, int, int, int, float,
@@ -689,6 +693,24 @@ torch::Tensor skinny_gemm_fp8_probe(torch::Tensor a, torch::Tensor qf,
   return out;
 }
 
+// a @ w^T, or with glu, w = [gate; up], silu(gate) * up of it
+torch::Tensor short_gemm(torch::Tensor a, torch::Tensor w, bool glu) {
+  CHK_DEV(a); CHK_DEV(w); CHK_BF16(a); CHK_BF16(w); CHK_CONT(w);
+  TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && a.stride(1) == 1 &&
+                  a.size(1) == w.size(1), "a [M, K], w [N, K]");
+  const long long M = a.size(0), N = w.size(0), K = w.size(1);
+  TORCH_CHECK(K >= 64 && K % 64 == 0 && N >= 32 && N % (glu ? 32 : 16) == 0,
+              "K % 64, N % 16");
+  TORCH_CHECK(M < (1 << 24) && N < (1 << 20) && a.stride(0) % 8 == 0 &&
+                  ((reinterpret_cast<uintptr_t>(a.data_ptr()) |
+                    reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0,
+              "sizes, alignment");
+  auto out = torch::empty({M, glu ? N / 2 : N}, a.options());
+  qsa_short_gemm_launch(u16(a), u16(w), u16m(out), (int)M, (int)N, (int)K,
+                        a.stride(0), glu, cur_stream());
+  return out;
+}
+
 // rows of [q | k | v] of the items, blocks of 64 query rows -> [T, H*D]
 torch::Tensor encoder_attn(torch::Tensor qkv, torch::Tensor cos_t,
                            torch::Tensor sin_t, torch::Tensor qb_item,
@@ -817,6 +839,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "prefill rotation and paged-cache write");
   m.def("encoder_attn", &encoder_attn,
         "rotation and bidirectional attention of projection rows");
+  m.def("short_gemm", &short_gemm, "GEMM of a short K, optionally gated");
   m.def("mean_rows", &mean_rows, "mean of each item's rows (f32)");
   m.def("kv_scatter", &kv_scatter, "scatter prefill k/v by slot ids");
   m.def("pack_weight_frag", &pack_weight_frag,

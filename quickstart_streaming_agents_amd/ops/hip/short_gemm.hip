@@ -1,0 +1,181 @@
+// GEMM of a short K for CDNA4 (gfx950): C[M,N] = A[M,K] @ W[N,K]^T, bf16 with f32
+// sums, and with GLU silu(gate) * up of it, W's rows being [gate; up]: the
+// encoder's projections (K 384 and 512, and 1536 for few rows).
+//
+// With a few steps of K a product is over before a deep pipeline is full; its
+// reads and writes and, for few rows, the host's way to a library's kernel (20
+// us a call, 4 here) count as much as the matrix cores.  So: tiles by the number
+// of blocks they leave, K in steps of 64 through two halves of LDS with the next
+// one in registers, whole 128-byte lines of every operand, a block row's columns
+// on one die, results through LDS to whole lines, and the gate's columns beside
+// the up's in a wave, so that the activation costs no pass over memory.
+// us, library -> here, at 100 / 1600 / 8800 rows: 1536 x 384 4.8 / 8.0 / 17.3 ->
+// 3.4 / 6.8 / 20.9, 384 x 512 5.0 / 6.1 / 9.4 -> 3.7 / 4.6 / 9.8, 384 x 1536 4.9
+// / 8.6 / 16.2 -> 7.1 / 9.5 / 22; 3072 x 384 with the activation (here a pass of
+// its own, 16 us at 8800) 5.1 / 10.0 / 57.2 without -> 4.3 / 11.0 / 35.4 with it.
+#include "lm_common.h"
+
+struct ShortArgs {
+  const bf16_t* A;                     // [M, K], row stride lda
+  const bf16_t* W;                     // [N, K]
+  bf16_t* C;                           // [M, N], or [M, N/2] with GLU
+  int M, N, K, NB;                     // NB: blocks along the columns
+  long long lda;
+};
+
+// 4 waves as 2 x 2; a wave has MT x NT tiles of 16 x 16
+template <int MT, int NT, bool GLU>
+__global__ void __launch_bounds__(256, 2)
+qsa_short_gemm(ShortArgs p) {
+  constexpr int BM = 32 * MT, BN = 32 * NT;
+  constexpr int AL = BM / 32, BL = BN / 32;       // 16 B loads of a thread
+  constexpr int OP = (GLU ? 8 : 16) * NT + 8;     // pitch of a wave's results
+  constexpr int TILE = (BM + BN) * 64;
+  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * TILE];
+  static_assert(4 * 16 * MT * OP <= 2 * TILE, "the results fit");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, hi = lane >> 4;
+  // a die keeps the rows of a block row: it has all their columns
+  const int mb = (blockIdx.x / 8 / p.NB) * 8 + blockIdx.x % 8;
+  const int nb = blockIdx.x / 8 % p.NB;
+  const int m0 = mb * BM;
+  if (m0 >= p.M) return;               // uniform over the block
+
+  // thread: 16 bytes of row tid/8 (+ 32 j), the eight of a row side by side
+  const int seg = tid & 7, r8 = tid >> 3;
+  const bf16_t* ap[AL];
+  const bf16_t* bp[BL];
+#pragma unroll
+  for (int j = 0; j < AL; ++j)
+    ap[j] = p.A + (long long)min(m0 + r8 + 32 * j, p.M - 1) * p.lda + seg * 8;
+#pragma unroll
+  for (int j = 0; j < BL; ++j) {
+    const int r = r8 + 32 * j;         // row of the tile
+    int n = nb * BN + r;
+    if (GLU)                           // tiles 2i and 2i + 1: gate, up
+      n = (r >> 4 & 1) * (p.N >> 1) + nb * (BN / 2) + (r >> 5) * 16 + (r & 15);
+    bp[j] = p.W + (long long)min(n, p.N - 1) * p.K + seg * 8;
+  }
+  // LDS: fragments [row tile][half of K][hi][16 rows][8], the rows of a group
+  // exchanged so that a row's eight segments go to different banks
+  auto place = [&](int row, int half, int h) {
+    return (((row >> 4) * 2 + half) * 64 + h * 16 +
+            ((row & 15) ^ (h << 1 | half << 3))) * 8;
+  };
+  u32x4_v ar[AL], br[BL];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int j = 0; j < AL; ++j)
+      ar[j] = *reinterpret_cast<const u32x4_v*>(ap[j] + k);
+#pragma unroll
+    for (int j = 0; j < BL; ++j)
+      br[j] = *reinterpret_cast<const u32x4_v*>(bp[j] + k);
+  };
+  auto store = [&](bf16_t* t) {
+#pragma unroll
+    for (int j = 0; j < AL; ++j)
+      *reinterpret_cast<u32x4_v*>(
+          t + place(r8 + 32 * j, seg >> 2, seg & 3)) = ar[j];
+#pragma unroll
+    for (int j = 0; j < BL; ++j)
+      *reinterpret_cast<u32x4_v*>(
+          t + BM * 64 + place(r8 + 32 * j, seg >> 2, seg & 3)) = br[j];
+  };
+  f32x4_v acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  const int wm = (wave >> 1) * MT, wn = (wave & 1) * NT;
+  const int steps = p.K >> 6;
+  load(0);
+  store(lds);
+  load(min(1, steps - 1) * 64);
+  for (int s = 0; s < steps; ++s) {
+    lds_barrier();
+    const bf16_t* t = lds + (s & 1) * TILE;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      bf16x8_v a[MT], b[NT];
+      const int at = h * 512 + (hi * 16 + (col ^ (hi << 1 | h << 3))) * 8;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        a[i] = *reinterpret_cast<const bf16x8_v*>(t + (wm + i) * 1024 + at);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        b[j] = *reinterpret_cast<const bf16x8_v*>(t + BM * 64 +
+                                                  (wn + j) * 1024 + at);
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = mfma_bf16(b[j], a[i], acc[i][j]);
+    }
+    if (s + 1 < steps) {
+      store(lds + ((s + 1) & 1) * TILE);
+      load(min(s + 2, steps - 1) * 64);
+    }
+  }
+  // results through LDS: a lane has 4 columns (hi*4..) of row col of each tile
+  lds_barrier();
+  bf16_t* o = lds + wave * (16 * MT * OP);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; j += GLU ? 2 : 1) {
+      f32x4_v v = acc[i][j];
+      if constexpr (GLU) {
+        const f32x4_v u = acc[i][j + 1];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = v[r] / (1.f + __expf(-v[r])) * u[r];
+      }
+      *reinterpret_cast<uint2*>(
+          o + (i * 16 + col) * OP + (GLU ? j / 2 : j) * 16 + hi * 4) =
+          make_uint2(cvt_bf16x2(v[0], v[1]), cvt_bf16x2(v[2], v[3]));
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+  constexpr int G = (GLU ? NT : 2 * NT);          // 16 B groups of a row
+  const int N = GLU ? p.N >> 1 : p.N;
+  const int c0 = (GLU ? nb * (BN / 2) : nb * BN) + (wave & 1) * G * 8;
+#pragma unroll
+  for (int i = lane; i < 16 * MT * G; i += 64) {
+    const int row = i / G, c = (i % G) * 8;
+    const int m = m0 + (wave >> 1) * 16 * MT + row;
+    if (m < p.M && c0 + c < N)                    // N % 8 == 0
+      *reinterpret_cast<u32x4_v*>(p.C + (long long)m * N + c0 + c) =
+          *reinterpret_cast<const u32x4_v*>(o + row * OP + c);
+  }
+}
+
+template <int MT, int NT>
+static void short_go(ShortArgs p, int glu, hipStream_t st) {
+  p.NB = (p.N + 32 * NT - 1) / (32 * NT);
+  const int mb = (p.M + 32 * MT - 1) / (32 * MT);
+  const dim3 grid((unsigned)((mb + 7) / 8 * 8 * p.NB));
+  if (glu)
+    hipLaunchKernelGGL((qsa_short_gemm<MT, NT, true>), grid, dim3(256), 0, st,
+                       p);
+  else
+    hipLaunchKernelGGL((qsa_short_gemm<MT, NT, false>), grid, dim3(256), 0, st,
+                       p);
+}
+
+// Tiles of 128 x 128 once two rounds of blocks are left, 64 x 64 while they
+// make half a round, 32 x 64 below (384 x 512 at 400 rows: 8.2 / 4.5 / 3.7 us;
+// 1536 x 384 at 1600: 7.9 / 6.8 / 8.0, at 8800: 20.9 / 23.0 / 28.4).
+extern "C" void qsa_short_gemm_launch(const bf16_t* A, const bf16_t* W,
+                                      bf16_t* C, int M, int N, int K,
+                                      long long lda, int glu,
+                                      hipStream_t st) {
+  if (M == 0) return;
+  const ShortArgs p{A, W, C, M, N, K, 0, lda};
+  auto blocks = [&](int b) {
+    return (long long)((M + b - 1) / b) * ((N + b - 1) / b);
+  };
+  if (blocks(128) >= 512) short_go<4, 4>(p, glu, st);
+  else if (blocks(64) >= 128) short_go<2, 2>(p, glu, st);
+  else short_go<1, 2>(p, glu, st);
+}

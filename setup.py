@@ -36,7 +36,7 @@ MODULES = {
     "qsa_hip": ["ops.cpp", "avro_codec.cpp", "elementwise.hip",
                 "paged_attn.hip", "skinny_gemm.hip", "skinny_gemm_fp8.hip",
                 "hash_join.hip", "gemm_fp8_batch.hip", "topk_cosine.hip",
-                "streaming.hip", "encoder_attn.hip"],
+                "streaming.hip", "encoder_attn.hip", "short_gemm.hip"],
     "qsa_lm_hip": ["lm_ops.cpp", "lm_elementwise.hip", "retention.hip",
                    "latent_attn.hip", "short_conv.hip", "gqa_attn.hip", "ssd.hip",
                    "skinny_gemm.hip", "rows_gemm.hip"],

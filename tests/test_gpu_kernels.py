@@ -835,6 +835,28 @@ def test_encoder_attn(ext, lens, D, H):
         assert ((got[o:o + n] - want).abs() <= 2 ** -6 * scale + 1e-6).all()
 
 
+@pytest.mark.parametrize("M", [1, 33, 65, 1000, 5600])
+@pytest.mark.parametrize("N,K,glu", [
+    (32, 64, False), (1536, 384, False), (400, 512, False), (96, 1536, False),
+    (3072, 384, True), (96, 192, True)])
+def test_short_gemm(ext, M, N, K, glu):
+    """Every tile shape, ragged ends of rows and columns, rows of a slice.  An
+    f32 sum of K products and a rounding to bf16; the activation's slope is
+    1.1 at most."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + 16, generator=g).bfloat16().to(dev())[:, 8:K + 8]
+    w = torch.randn(N, K, generator=g).mul(K ** -0.5).bfloat16().to(dev())
+    got = ext.short_gemm(x, w, glu).double()
+    a, b = x.double(), w.double()
+    want, err = a @ b.T, K * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    if glu:
+        z, u = want.chunk(2, 1)
+        want = torch.nn.functional.silu(z) * u
+        err = 1.1 * err[:, :N // 2] * u.abs() + z.abs() * err[:, N // 2:] + \
+            2.0 ** -20 * want.abs()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + err + 1e-30).all()
+
+
 def test_mean_rows(ext):
     lens = [1, 3, 4, 5, 700]
     x = torch.randn(sum(lens), 520, device=dev()).bfloat16()
