@@ -10,9 +10,9 @@
 // on one die, results through LDS to whole lines, and the gate's columns beside
 // the up's in a wave, so that the activation costs no pass over memory.
 // us, library -> here, at 100 / 1600 / 8800 rows: 1536 x 384 4.8 / 8.0 / 17.3 ->
-// 3.4 / 6.8 / 20.9, 384 x 512 5.0 / 6.1 / 9.4 -> 3.7 / 4.6 / 9.8, 384 x 1536 4.9
-// / 8.6 / 16.2 -> 7.1 / 9.5 / 22; 3072 x 384 with the activation (here a pass of
-// its own, 16 us at 8800) 5.1 / 10.0 / 57.2 without -> 4.3 / 11.0 / 35.4 with it.
+// 3.4 / 6.9 / 20.5, 384 x 512 5.0 / 6.1 / 9.4 -> 3.8 / 4.6 / 9.7, 384 x 1536 4.9
+// / 8.6 / 16.3 -> 7.4 / 9.5 / 23; 3072 x 384 with the activation (here a pass of
+// its own, 16 us at 8800) 5.1 / 10.0 / 39 without -> 3.6 / 10.8 / 35 with it.
 #include "lm_common.h"
 
 struct ShortArgs {
@@ -36,11 +36,19 @@ qsa_short_gemm(ShortArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
-  // a die keeps the rows of a block row: it has all their columns
-  const int mb = (blockIdx.x / 8 / p.NB) * 8 + blockIdx.x % 8;
-  const int nb = blockIdx.x / 8 % p.NB;
+  // a die keeps the rows of a block row: it has all their columns; fewer than
+  // eight block rows are spread over all dies
+  const int rows = (p.M + BM - 1) / BM;
+  int mb, nb;
+  if (rows < 8) {
+    mb = blockIdx.x % rows;
+    nb = blockIdx.x / rows;
+  } else {
+    mb = (blockIdx.x / 8 / p.NB) * 8 + blockIdx.x % 8;
+    nb = blockIdx.x / 8 % p.NB;
+    if (mb >= rows) return;            // uniform over the block
+  }
   const int m0 = mb * BM;
-  if (m0 >= p.M) return;               // uniform over the block
 
   // thread: 16 bytes of row tid/8 (+ 32 j), the eight of a row side by side
   const int seg = tid & 7, r8 = tid >> 3;
@@ -154,7 +162,7 @@ template <int MT, int NT>
 static void short_go(ShortArgs p, int glu, hipStream_t st) {
   p.NB = (p.N + 32 * NT - 1) / (32 * NT);
   const int mb = (p.M + 32 * MT - 1) / (32 * MT);
-  const dim3 grid((unsigned)((mb + 7) / 8 * 8 * p.NB));
+  const dim3 grid((unsigned)((mb < 8 ? mb : (mb + 7) / 8 * 8) * p.NB));
   if (glu)
     hipLaunchKernelGGL((qsa_short_gemm<MT, NT, true>), grid, dim3(256), 0, st,
                        p);
