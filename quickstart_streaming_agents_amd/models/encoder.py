@@ -9,12 +9,12 @@ Random-init weights (air-gapped): embeddings are deterministic and
 well-distributed; the retrieval CONTRACT (dims, cosine, top-k) is what the
 pipelines rely on.
 
-GPU attention runs the hand-written varlen MFMA flash kernel
-(ops/hip/paged_attn.hip, CAUSAL=false): per-layer K/V scatter into a
-paged scratch cache, then ONE bidirectional flash-attention kernel per
-layer streaming K/V fragments — no padded bmm, no materialized score
-matrix.  The CPU path keeps a padded bmm + masked-softmax reference of
-the same semantics (GPU-vs-CPU parity test in tests/test_gpu_models.py).
+On the GPU the tokens of a batch are rows without padding: the projections are
+ops/hip/short_gemm.hip's, the activation inside, and attention runs on the
+projection's rows as they are (ops/hip/encoder_attn.hip) — no padded bmm, no
+materialized score matrix.  The CPU path keeps a padded bmm + masked-softmax
+reference of the same semantics (GPU-vs-CPU parity test in
+tests/test_gpu_models.py).
 """
 
 from __future__ import annotations
