@@ -11,6 +11,8 @@
 //                                   (qsa_window_attn_prefill)
 // Window: position i sees j with 0 <= i - j < size.  The softmax sink adds
 // exp(sink_h) to the denominator: no key, no value, no scale.
+#include <type_traits>
+
 #include "lm_common.h"
 
 #define LPAGE 64
@@ -456,7 +458,11 @@ extern "C" void qsa_latent_rows_mfma_launch(
 // Block = (64-row query block, head): wave w owns 16 rows; 64-key tiles of K
 // and V go through LDS once per block.  O^T stays in accumulators (row =
 // value column, column = query row), so the softmax state, the rescale and
-// P^T (B operand of the second product) are all lane-local.
+// P^T (B operand of the second product) are all lane-local.  Beside LDS reads
+// the softmax's vector work bounds it: hidden keys are looked for only in tiles
+// that have some, maxima are taken before the scale, which joins the exponent in
+// one fma, and the output is rescaled only where a maximum moved (8192 tokens,
+// 32 heads of 128: 1358 us without, 1066 here; window 4096: 934, 747).
 //   q   [rows, H, D]           row stride qstride
 //   kv  [context rows, H*(D+E)]: k of head h at h*D, v at H*D + h*E
 //   portion it: rows off..off+len-1 at positions start..; its context rows
@@ -489,12 +495,16 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
   const int n = len[it], p0 = start[it], r0 = off[it];
   const int c_pos = ctx_pos[it];
   const long long c_off = ctx_off[it];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
   const int i = t0 + wave * 16 + col;             // row within the portion
   const int qpos = p0 + i;
   const long long qrow = r0 + min(i, n - 1);
 
+  // maxima are taken before the scale, which therefore has to be positive
+  const bool negative = scale2 < 0.f;
+  scale2 = fmaxf(fabsf(scale2), 1e-30f);
   const bf16x8_v zero = {0, 0, 0, 0, 0, 0, 0, 0};
   bf16x8_v qf[KS];
 #pragma unroll
@@ -502,6 +512,7 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
     const int d = s * 32 + hi * 8;                // D % 8 == 0
     bf16x8_v v = *reinterpret_cast<const bf16x8_v*>(
         q + qrow * qstride + (long long)h * D + (d < D ? d : 0));
+    if (negative) v ^= (short)0x8000;
     qf[s] = d < D ? v : zero;
   }
   f32x4_v acc[ET];
@@ -557,7 +568,6 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
     if (pos + 64 <= last) fetch(pos + 64);
     if (pos > wlast || pos + 63 < wfirst) continue;   // nothing for this wave
     f32x4_v s4[4];
-    float mx = NEG_BIG;
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt) {
       f32x4_v a4 = {0.f, 0.f, 0.f, 0.f};
@@ -567,34 +577,58 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
             &kt[(pt * 16 + col) * KP + s * 32 + hi * 8]);
         a4 = mfma_bf16(a, qf[s], a4);
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int p = pos + pt * 16 + hi * 4 + r;
-        const bool ok = p <= qpos && p <= last &&
-                        (window <= 0 || qpos - p < window);
-        a4[r] = ok ? a4[r] * scale2 : NEG_BIG;
-        mx = fmaxf(mx, a4[r]);
-      }
       s4[pt] = a4;
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
-    const float mn = fmaxf(m, mx);
-    const float alpha = m > NEG_BIG ? exp2f(m - mn) : 0.f;
-    m = mn;
-    float psum = 0.f;
     bf16x8_v pf[2];
+    float alpha;
+    bool moved;
+    auto softmax = [&](auto edge) {               // edge: some keys are hidden
+      float mx = -INFINITY;
 #pragma unroll
-    for (int pt = 0; pt < 4; ++pt)
+      for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = s4[pt][r] > NEG_BIG ? exp2f(s4[pt][r] - mn) : 0.f;
-        psum += p;
-        pf[pt >> 1][(pt & 1) * 4 + r] = (short)cvt_bf16(p);
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (edge.value) {
+            const int p = pos + pt * 16 + hi * 4 + r;
+            if (p > qpos || p > last || (window > 0 && qpos - p >= window))
+              s4[pt][r] = -INFINITY;
+          }
+          mx = fmaxf(mx, s4[pt][r]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
+      const float mn = fmaxf(m, mx * scale2);     // NEG_BIG: no key so far
+      moved = mn > m;
+      alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      float psum = 0.f;
+      uint2 pk[4];
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt) {
+        float p[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          p[r] = __builtin_amdgcn_exp2f(fmaf(s4[pt][r], scale2, -mn));
+          psum += p[r];
+        }
+        pk[pt] = make_uint2(cvt_bf16x2(p[0], p[1]), cvt_bf16x2(p[2], p[3]));
       }
-    l = l * alpha + psum;
 #pragma unroll
-    for (int t = 0; t < ET; ++t) acc[t] *= alpha;
+      for (int s = 0; s < 2; ++s)
+        pf[s] = __builtin_bit_cast(
+            bf16x8_v, make_uint4(pk[2 * s].x, pk[2 * s].y, pk[2 * s + 1].x,
+                                 pk[2 * s + 1].y));
+      l = l * alpha + psum;
+    };
+    if (pos + 63 > wlast - 15 || pos + 63 > last ||
+        (window > 0 && wlast - pos >= window))
+      softmax(std::true_type{});
+    else
+      softmax(std::false_type{});
+    if (__any(moved)) {                           // else every factor is 1
+#pragma unroll
+      for (int t = 0; t < ET; ++t) acc[t] *= alpha;
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
