@@ -580,9 +580,8 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
       s4[pt] = a4;
     }
     bf16x8_v pf[2];
-    float alpha;
-    bool moved;
-    auto softmax = [&](auto edge) {               // edge: some keys are hidden
+    float alpha, top, psum;
+    auto softmax = [&](auto edge, auto guard) {   // edge: some keys are hidden
       float mx = -INFINITY;
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt)
@@ -593,22 +592,21 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
             if (p > qpos || p > last || (window > 0 && qpos - p >= window))
               s4[pt][r] = -INFINITY;
           }
+          if constexpr (guard.value) s4[pt][r] = fmaxf(s4[pt][r], -INFINITY);
           mx = fmaxf(mx, s4[pt][r]);
         }
       mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
       mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
-      const float mn = fmaxf(m, mx * scale2);     // NEG_BIG: no key so far
-      moved = mn > m;
-      alpha = __builtin_amdgcn_exp2f(m - mn);
-      m = mn;
-      float psum = 0.f;
+      top = fmaxf(m, mx * scale2);                // NEG_BIG: no key so far
+      alpha = __builtin_amdgcn_exp2f(m - top);
+      psum = 0.f;
       uint2 pk[4];
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt) {
         float p[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p[r] = __builtin_amdgcn_exp2f(fmaf(s4[pt][r], scale2, -mn));
+          p[r] = __builtin_amdgcn_exp2f(fmaf(s4[pt][r], scale2, -top));
           psum += p[r];
         }
         pk[pt] = make_uint2(cvt_bf16x2(p[0], p[1]), cvt_bf16x2(p[2], p[3]));
@@ -618,13 +616,17 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
         pf[s] = __builtin_bit_cast(
             bf16x8_v, make_uint4(pk[2 * s].x, pk[2 * s].y, pk[2 * s + 1].x,
                                  pk[2 * s + 1].y));
-      l = l * alpha + psum;
     };
     if (pos + 63 > wlast - 15 || pos + 63 > last ||
         (window > 0 && wlast - pos >= window))
-      softmax(std::true_type{});
+      softmax(std::true_type{}, std::false_type{});
     else
-      softmax(std::false_type{});
+      softmax(std::false_type{}, std::false_type{});
+    // a NaN score counts as no key: hidden ones are -inf by now
+    if (__any(!(psum <= 64.f))) softmax(std::false_type{}, std::true_type{});
+    l = l * alpha + psum;
+    const bool moved = top > m;
+    m = top;
     if (__any(moved)) {                           // else every factor is 1
 #pragma unroll
       for (int t = 0; t < ET; ++t) acc[t] *= alpha;

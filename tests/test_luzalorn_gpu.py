@@ -230,6 +230,40 @@ def test_latent_attention_kernels(H, Dm, E, R, window, dtype):
         close(out, want[start:start + n], dtype)
 
 
+@pytest.mark.parametrize("window", [0, 100])
+@pytest.mark.parametrize("Dm,E", [(128, 128), (40, 24)])
+def test_window_attention_nan_scores(Dm, E, window):
+    """A NaN score counts as no key, in tiles with hidden keys and without; a
+    row that sees nothing else has the sink alone."""
+    g = gen(Dm + window)
+    n, H, scale = 230, 4, Dm ** -0.5
+    q, k = rnd(g, n, H, Dm, dtype=BF), rnd(g, n, H, Dm, dtype=BF)
+    v, gate = rnd(g, n, H, E, dtype=BF), rnd(g, n, H * E, dtype=BF)
+    sink = rnd(g, H, dtype=BF)
+    for j, h in ((0, 0), (31, 1), (64, 1), (127, 2), (200, 2), (229, 3)):
+        k[j, h, j % Dm] = float("nan")
+    i = torch.arange(n)
+    seen = i[:, None] >= i
+    if window:
+        seen &= i[:, None] - i < window
+    s = torch.einsum("ihd,jhd->hij", q.double(), k.double()) * scale
+    s = s.masked_fill(~seen | s.isnan(), float("-inf"))
+    top = torch.maximum(s.amax(-1), sink.double()[:, None])
+    e = (s - top[..., None]).exp()
+    den = e.sum(-1) + (sink.double()[:, None] - top).exp()
+    want = torch.einsum("hij,jhe->ihe", e / den[..., None], v.double()) \
+        .reshape(n, -1) * O.sigmoid(gate.double())
+    kv = torch.cat([k.reshape(n, -1), v.reshape(n, -1)], 1).to(DEV)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    out = torch.empty(n, H * E, dtype=BF, device=DEV)
+    D.window_attn_prefill(
+        q.reshape(n, -1).to(DEV), kv, gate.to(DEV), sink.to(DEV),
+        i32(0, 0, 0, 0), i32(0, 64, 128, 192), i32(0), i32(0), i32(n), i32(0),
+        i32(0), out, Dm, E, window, scale)
+    close(out, want, BF)
+    assert not out[0, :E].any()
+
+
 def test_latent_norm_store_and_slots():
     for dtype in (F32, BF):
         g = gen(5)
