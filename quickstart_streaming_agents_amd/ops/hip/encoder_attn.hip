@@ -125,7 +125,10 @@ qsa_encoder_attn(const bf16_t* __restrict__ qkv,      // [T, 3, H, D]
     if (w0 >= n) continue;             // nothing for this wave
 
     const int left = n - tile * ENC_KEYS;
-    auto keys = [&](auto edge) {       // edge: some are hidden
+    float alpha, top, psum;
+    uint2 pk[4];
+    // edge: some keys are hidden; guard: a NaN score counts as no key
+    auto weigh = [&](auto edge, auto guard) {
       f32x4_v sc[4];
       float mx = -INFINITY;
 #pragma unroll
@@ -141,43 +144,45 @@ qsa_encoder_attn(const bf16_t* __restrict__ qkv,      // [T, 3, H, D]
         for (int r = 0; r < 4; ++r) {
           if constexpr (edge.value)
             if (pt * 16 + hi * 4 + r >= left) sc[pt][r] = -INFINITY;
+          if constexpr (guard.value) sc[pt][r] = fmaxf(sc[pt][r], -INFINITY);
           mx = fmaxf(mx, sc[pt][r]);
         }
       }
       mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
       mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
-      const float mn = fmaxf(m, mx * scale2);
-      const float alpha = __builtin_amdgcn_exp2f(m - mn);
-      m = mn;
-      float psum = 0.f;
-      uint2 pk[4];
+      top = fmaxf(m, mx * scale2);
+      alpha = __builtin_amdgcn_exp2f(m - top);
+      psum = 0.f;
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt) {
         float p[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p[r] = __builtin_amdgcn_exp2f(fmaf(sc[pt][r], scale2, -mn));
+          p[r] = __builtin_amdgcn_exp2f(fmaf(sc[pt][r], scale2, -top));
           psum += p[r];
         }
         pk[pt] = make_uint2(cvt_bf16x2(p[0], p[1]), cvt_bf16x2(p[2], p[3]));
       }
-      l = l * alpha + psum;
-#pragma unroll
-      for (int t = 0; t < ET; ++t) acc[t] *= alpha;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const bf16x8_v pf = __builtin_bit_cast(
-            bf16x8_v, make_uint4(pk[2 * k].x, pk[2 * k].y, pk[2 * k + 1].x,
-                                 pk[2 * k + 1].y));
-#pragma unroll
-        for (int t = 0; t < ET; ++t)
-          acc[t] = mfma_bf16(lds_frag_tr(vt, VP, k * 32, k * 32 + 16,
-                                         t * 16, lane),
-                             pf, acc[t]);
-      }
     };
-    if (left >= ENC_KEYS) keys(std::false_type{});
-    else keys(std::true_type{});
+    if (left >= ENC_KEYS) weigh(std::false_type{}, std::false_type{});
+    else weigh(std::true_type{}, std::false_type{});
+    // once more from LDS: kept scores would take registers from every tile
+    if (__any(!(psum <= 64.f))) weigh(std::true_type{}, std::true_type{});
+    m = top;
+    l = l * alpha + psum;
+#pragma unroll
+    for (int t = 0; t < ET; ++t) acc[t] *= alpha;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const bf16x8_v pf = __builtin_bit_cast(
+          bf16x8_v, make_uint4(pk[2 * k].x, pk[2 * k].y, pk[2 * k + 1].x,
+                               pk[2 * k + 1].y));
+#pragma unroll
+      for (int t = 0; t < ET; ++t)
+        acc[t] = mfma_bf16(lds_frag_tr(vt, VP, k * 32, k * 32 + 16, t * 16,
+                                       lane),
+                           pf, acc[t]);
+    }
   }
   l += __shfl_xor(l, 16, QSA_WAVE);
   l += __shfl_xor(l, 32, QSA_WAVE);

@@ -835,6 +835,30 @@ def test_encoder_attn(ext, lens, D, H):
         assert ((got[o:o + n] - want).abs() <= 2 ** -6 * scale + 1e-6).all()
 
 
+def test_encoder_attn_nan_scores(ext):
+    """A NaN score counts as no key, in whole tiles and in the last one, as in
+    the paged kernel; a row that sees nothing else comes out as zero."""
+    g = torch.Generator().manual_seed(4)
+    H, D, lens, bad = 4, 64, [1, 150], (0, 1 + 10, 1 + 70, 1 + 149)
+    T = sum(lens)
+    qkv = torch.randn(T, 3, H, D, generator=g).bfloat16()
+    qkv[list(bad), 1, 2] = float("nan")
+    still = torch.ones(200, D // 2), torch.zeros(200, D // 2)
+    mk = lambda *x: torch.tensor(x, dtype=torch.int32, device=dev())
+    got = ext.encoder_attn(
+        qkv.view(T, -1).to(dev()), still[0].to(dev()), still[1].to(dev()),
+        mk(0, 1, 1, 1), mk(0, 0, 64, 128), mk(0, 1), mk(*lens), H,
+        D ** -0.5).cpu().double().view(T, H, D)
+    assert not got[0, 2].any()
+    q, k, v = qkv[1:].double().unbind(1)
+    s = torch.einsum("ihd,jhd->hij", q, k) * D ** -0.5
+    p = s.masked_fill(s.isnan(), float("-inf")).softmax(-1)
+    want = torch.einsum("hij,jhd->ihd", p, v)
+    scale = torch.einsum("hij,jhd->ihd", p, v.abs())
+    # weights and the result are rounded to bf16: 2**-9 each
+    assert ((got[1:] - want).abs() <= 2 ** -7 * scale + 1e-6).all()
+
+
 @pytest.mark.parametrize("M", [1, 33, 65, 1000, 5600])
 @pytest.mark.parametrize("N,K,glu", [
     (32, 64, False), (1536, 384, False), (400, 512, False), (96, 1536, False),
