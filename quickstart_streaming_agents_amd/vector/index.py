@@ -165,13 +165,12 @@ class VectorIndex:
         docs = self.to_torch(device)
         qt = torch.from_numpy(q).to(device=device, dtype=torch.float32)
         k_eff = min(k, len(self))
-        if len(q) >= 16 and (k_eff > 16 or
-                             len(q) > 32 and len(q) * len(self) > 1_500_000 or
-                             not np.isfinite(q).all()):
+        if k_eff > 16 or len(q) > 32 and len(q) * len(self) > 1_500_000 or \
+                not np.isfinite(q).all():
             # many queries are GEMM-shaped: a matmul over the HBM matrix and
             # a sort of the scores (48 queries: 165 us against 135 of the
-            # kernel at 30k rows, 189 against 245 at 60k).  The kernel has no
-            # answer for a query that is not a number.
+            # kernel at 30k rows, 189 against 245 at 60k).  The kernel keeps
+            # at most 16 hits and has none for a query that is not a number.
             scores_all = qt @ docs.T
             scores, idx = torch.topk(scores_all, k_eff, dim=1)
             idx = idx.int()
@@ -184,9 +183,10 @@ class VectorIndex:
         idx = idx.cpu().numpy()
         out = []
         for qi in range(len(q)):
+            # -1: fewer documents than k have a score
             out.append([SearchHit(self.ids[i], self.chunks[i],
                                   float(scores[qi, j]), self.metadata[i])
-                        for j, i in enumerate(idx[qi])])
+                        for j, i in enumerate(idx[qi]) if i >= 0])
         return out
 
     @staticmethod

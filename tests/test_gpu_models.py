@@ -238,6 +238,35 @@ def test_vector_index_batches(rows, queries, k):
         hits[3][0].document_id == str(rows - 1)
 
 
+@pytest.mark.parametrize("queries", [1, 15, 16])
+def test_vector_index_beyond_the_kernel(queries):
+    """More hits than the kernel keeps, a query that is not a number and
+    documents without a score, for every number of queries."""
+    import numpy as np
+    from quickstart_streaming_agents_amd.vector.index import VectorIndex
+    rng = np.random.default_rng(queries)
+    m = rng.standard_normal((50, 8)).astype(np.float32)
+    m /= np.linalg.norm(m, axis=1, keepdims=True)
+    idx = VectorIndex(dim=8)
+    idx._vecs, idx.metadata = list(m), [{}] * 50
+    idx.ids = [str(i) for i in range(50)]
+    idx.chunks = idx.ids
+    q = m[:queries].copy()
+    want = q.astype(np.float64) @ m.astype(np.float64).T
+    for i, hits in enumerate(idx.search_batch_gpu(q, 17, device="cuda:0")):
+        assert [h.document_id for h in hits] == \
+            [str(j) for j in np.argsort(-want[i])[:17]]
+    q[0] = np.nan
+    assert all(np.isnan(h.score) for h in
+               idx.search_batch_gpu(q, 3, device="cuda:0")[0])
+    short = VectorIndex(dim=8)
+    short._vecs = [m[0], np.full(8, np.nan, np.float32), m[1]]
+    short.ids = short.chunks = ["a", "b", "c"]
+    short.metadata = [{}] * 3
+    for hits in short.search_batch_gpu(m[:queries], 3, device="cuda:0"):
+        assert sorted(h.document_id for h in hits) == ["a", "c"]
+
+
 def test_lab3_lab4_gpu_anomaly_matches_cpu_and_invariants():
     """The batched GPU anomaly path must reproduce the sequential CPU
     reference on the real lab datagen — and hence the determinism
