@@ -657,9 +657,11 @@ std::vector<torch::Tensor> embed_rows(torch::Tensor embed,
   // (embed[tokens], the rows of the norm with weight w that follows, the
   // sums of squares in one part)
   CHK_DEV(embed); CHK_BF16(embed); CHK_CONT(embed); CHK_DEV(tokens);
-  TORCH_CHECK(tokens.scalar_type() == torch::kInt64 &&
-                  tokens.is_contiguous() && tokens.dim() == 1,
-              "tokens must be contiguous i64 [M]");
+  TORCH_CHECK((tokens.scalar_type() == torch::kInt64 ||
+               tokens.scalar_type() == torch::kInt32) && tokens.dim() == 1,
+              "tokens must be i64 or i32 [M]");
+  // as index_select takes them; the engine's are i64 and contiguous
+  tokens = tokens.to(torch::kInt64).contiguous();
   const long M = tokens.size(0), H = embed.size(1);
   TORCH_CHECK(M >= 1 && M <= 32 && H % 32 == 0, "M in [1,32], H % 32 == 0");
   CHK_DEV(w); CHK_BF16(w); CHK_CONT(w);

@@ -40,6 +40,29 @@ def test_prefill_decode_consistency(tiny):
     assert int(logits_a.argmax()) == int(logits_b.argmax())
 
 
+@pytest.mark.parametrize("rows", [1, 5, 33])
+def test_decode_takes_tokens_as_the_embedding_does(tiny, rows):
+    """i32 tokens and a strided column of them, on the fp8 streams and beyond
+    their 32 rows."""
+    assert tiny._streams_fp8()
+    g = torch.Generator().manual_seed(rows)
+    table = torch.randint(16, 2000, (rows, 3), generator=g).to("cuda:0")
+
+    def step(tokens):
+        kv = tiny.new_kv_cache(rows)
+        for i in range(rows):
+            kv.allocate(i, 1)
+        ids = list(range(rows))
+        lens = kv.seq_lens_tensor(ids)
+        return tiny.forward_decode(tokens, kv, kv.block_table(ids), lens,
+                                   lens - 1)
+
+    want = step(table[:, 1].contiguous())
+    assert torch.equal(step(table[:, 1]), want)
+    assert torch.equal(step(table[:, 1].int()), want)
+    assert torch.equal(step(table.int()[:, 1]), want)
+
+
 def test_engine_determinism_and_shapes(tiny):
     """Greedy decode is deterministic across engines; output lengths honor
     max_new_tokens.  (Exact solo-vs-batched token equality is NOT asserted:
