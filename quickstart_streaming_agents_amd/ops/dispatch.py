@@ -206,6 +206,7 @@ def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
         k >= 3 * n and n * k >= 1 << 24 and n % 16 == 0 and k % 64 == 0 and \
         x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and \
         x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
+        x.stride(0) < 1 << 24 and \
         (x.data_ptr() | w.data_ptr()) % 16 == 0 and not (
             torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
 

@@ -539,3 +539,18 @@ def test_rows_gemm(M, N, K):
     a, b = x.double(), w.double()
     bound = 2.0 ** -8 * (a @ b.T).abs() + K * 2.0 ** -24 * (a.abs() @ b.abs().T)
     assert ((got - a @ b.T).abs() <= bound).all()
+
+
+def test_linear_of_rows_far_apart():
+    """The kernel's offsets of a row have 32 bits; rows too far apart for them
+    are the library's."""
+    from quickstart_streaming_agents_amd.models.layers import Linear
+    K, far = 8192, 1 << 24
+    w = rnd(gen(1), 2048, K, dtype=BF).to(DEV)
+    store = torch.empty(32 * far + K, dtype=BF, device=DEV)
+    for step in (far - 8, far):
+        x = store.as_strided((33, K), (step, 1))
+        x.copy_(rnd(gen(2), 33, K, dtype=BF))
+        assert D.rows_linear_ok(x, w) == (step < far)
+        a, b = x.double(), w.double()
+        close(Linear(w)(x), (a @ b.T).cpu(), BF)
