@@ -11,6 +11,7 @@ CPU-only CI.  A CUDA tensor NEVER falls back to the CPU path.
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from . import ext, lm_ext
 
@@ -197,6 +198,20 @@ def pack_weight_frag(w: torch.Tensor) -> torch.Tensor:
     return w.reshape(n // 16, 16, k // 32, 32).permute(0, 2, 1, 3).contiguous()
 
 
+def _unobserved(*tensors: torch.Tensor) -> bool:
+    """Whether only the values of the tensors matter: derivatives in either
+    direction, function transforms, tracing, autocast, modes and subclasses
+    see the library's operations and would pass a kernel of our own by."""
+    return not (torch.is_grad_enabled() and
+                any(t.requires_grad for t in tensors)) and \
+        forward_ad._current_level < 0 and \
+        torch._C._functorch.peek_interpreter_stack() is None and \
+        torch._C._len_torch_dispatch_stack() == 0 and \
+        not torch.jit.is_tracing() and not torch.compiler.is_compiling() and \
+        not torch.is_autocast_enabled("cuda") and \
+        all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+
+
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether x[M,K] @ W^T is rows_linear's: a decode batch beyond the skinny
     kernels, and a long K beside few columns, where it beats the library at
@@ -206,9 +221,8 @@ def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
         k >= 3 * n and n * k >= 1 << 24 and n % 16 == 0 and k % 64 == 0 and \
         x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and \
         x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
-        x.stride(0) < 1 << 24 and \
-        (x.data_ptr() | w.data_ptr()) % 16 == 0 and not (
-            torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+        x.stride(0) < 1 << 24 and _unobserved(x, w) and \
+        (x.data_ptr() | w.data_ptr()) % 16 == 0
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
