@@ -124,7 +124,8 @@ extern "C" void qsa_window_agg_launch(const long long*, const int*,
                                       const float*, int*, float*, long long,
                                       long long, int, int, long long, int*,
                                       hipStream_t);
-extern "C" long long qsa_window_workspace(long long);
+extern "C" long long qsa_window_workspace(long long, long long, long long,
+                                          long long);
 void register_avro(pybind11::module_&);  // avro_codec.cpp
 extern "C" void qsa_anomaly_batch_launch(const float*, const int*, float*,
                                          float*, int*, int, int, int,
@@ -780,7 +781,7 @@ std::vector<torch::Tensor> window_agg(torch::Tensor ts, torch::Tensor key,
     CHK_F32(value.value());
     vptr = value.value().data_ptr<float>();
   }
-  const long long words = qsa_window_workspace(n);
+  const long long words = qsa_window_workspace(n, nkeys, nwin, win_ms);
   torch::Tensor ws;
   int* wptr = nullptr;
   if (words) {

@@ -10,19 +10,22 @@
 // The reference shape: TUMBLE(...) GROUP BY key (LAB3:99-133, LAB4:127-141).
 //
 // Bound by atomics, not bytes: those of different dies meet behind the L2s, at
-// some 12 G/s whether they collide or not (two per event: 307 us for 2M
-// events, 1000 keys, 288 windows; one pair per touched cell of a 4096-event
-// chunk: 81 us).  So blocks count CHUNKS of consecutive events, which in a
-// stream span a few windows, in LDS and leave (windows spanned) * nkeys cells
-// in a workspace; qsa_window_merge adds them up, without atomics and in a fixed
-// order (31 us together).  A chunk whose span does not fit goes to the output
-// with atomics, as do batches of a few chunks, where a second launch costs
-// more than their cells.
+// some 12 G/s whether they collide or not (two per event: 334 us for 2M
+// events, 1000 keys of uneven weight, 288 windows).  So blocks count chunks of
+// consecutive events, which in a stream span a few windows, in LDS, and a chunk
+// whose span does not fit goes to the output event by event.  How the cells of
+// a chunk reach the output is chosen by qsa_window_workspace:
+//   merged   chunks of 4096 leave (windows spanned) * nkeys cells in a
+//            workspace, qsa_window_merge adds them up, without atomics and in
+//            a fixed order (35 us)
+//   direct   chunks of 256 or 1024 add their cells to the output with atomics
+// More keys than fit in LDS have neither: an event at a time.
 // ---------------------------------------------------------------------------
 #define QSA_AGG_CELLS 6144             // 48 KiB of LDS: three blocks per CU
+#define QSA_AGG_FEW 2048               // of a chunk of 256: more cost more to
+                                       // clear and look through than to miss
 #define QSA_AGG_CHUNK 4096
 #define QSA_AGG_BLOCKS 2048            // most chunks, 96 MiB of workspace
-#define QSA_AGG_DIRECT 16              // chunks that need no workspace
 
 __device__ __forceinline__ int qsa_window_of(long long ts, long long t0,
                                              long long win_ms, int nwin) {
@@ -44,7 +47,26 @@ __device__ __forceinline__ int qsa_window_by(long long ts, long long t0,
   return max(w, 0);                    // the quotient is cut towards zero
 }
 
-template <bool FAST>                   // chunk == QSA_AGG_CHUNK, win_ms > 0
+// An event at a time, straight to the output.
+__global__ void __launch_bounds__(256)
+qsa_window_events(const long long* __restrict__ ts,
+                  const int* __restrict__ key,
+                  const float* __restrict__ value,  // nullptr -> count only
+                  int* __restrict__ counts, float* __restrict__ sums,
+                  long long t0, long long win_ms, int nwin, int nkeys,
+                  long long n) {
+  long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  for (; i < n; i += (long long)gridDim.x * 256) {
+    const int w = qsa_window_of(ts[i], t0, win_ms, nwin), k = key[i];
+    if (w < 0 || k < 0 || k >= nkeys) continue;
+    const long long slot = (long long)k * nwin + w;
+    atomicAdd(counts + slot, 1);
+    if (value) unsafeAtomicAdd(sums + slot, value[i]);
+  }
+}
+
+// PER events of a thread, chunk == 256 * PER; PER 0: any.  win_ms > 0.
+template <int PER, int CELLS>
 __global__ void __launch_bounds__(256)
 qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
                const float* __restrict__ value,  // nullptr -> count only
@@ -52,9 +74,9 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
                long long t0, long long win_ms, int nwin, int nkeys,
                long long n, long long chunk,
                int2* __restrict__ span,          // [blocks] {first, windows}
-               int* __restrict__ ws) {           // [blocks, 2, CELLS] or null
-  __shared__ int cnt[QSA_AGG_CELLS];
-  __shared__ float sum[QSA_AGG_CELLS];
+               int* __restrict__ ws) {           // [blocks, 2, QSA_AGG_CELLS]
+  __shared__ int cnt[CELLS];
+  __shared__ float sum[CELLS];
   __shared__ int lo_s, hi_s;
   const int tid = threadIdx.x;
   const long long first = (long long)blockIdx.x * chunk;
@@ -65,12 +87,11 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
   }
   __syncthreads();
   int lo = 0x7fffffff, hi = -1;
-  // FAST: every load of the chunk is under way before the first is used, and
+  // PER: every load of the chunk is under way before the first is used, and
   // an event's window is found once
-  constexpr int PER = QSA_AGG_CHUNK / 256;
-  int win[FAST ? PER : 1], ek[FAST ? PER : 1];
-  float ev[FAST ? PER : 1];
-  if constexpr (FAST) {
+  int win[PER ? PER : 1], ek[PER ? PER : 1];
+  float ev[PER ? PER : 1];
+  if constexpr (PER > 0) {
     long long et[PER];
     const long long limit = win_ms > 0x7fffffffffffffffll / nwin
                                 ? 0x7fffffffffffffffll : win_ms * nwin;
@@ -114,7 +135,7 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
   lo = lo_s;
   hi = hi_s;
   const long long cells = hi < 0 ? 0 : (long long)(hi - lo + 1) * nkeys;
-  const bool local = cells <= QSA_AGG_CELLS;     // uniform over the block
+  const bool local = cells <= CELLS;     // uniform over the block
   if (ws && tid == 0)
     span[blockIdx.x] = make_int2(lo, local && hi >= 0 ? hi - lo + 1 : 0);
   if (cells == 0) return;              // no event of the chunk counts
@@ -137,7 +158,7 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
       if (value) unsafeAtomicAdd(sums + slot, v);
     }
   };
-  if constexpr (FAST) {
+  if constexpr (PER > 0) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) count(win[j], ek[j], ev[j]);
   } else {
@@ -208,6 +229,7 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
   // in a stream most groups do not reach this window
   int pc = 0;
   float pv = 0.f;
+  bool reached = false;
   for (int j0 = 0; j0 < total; j0 += 4) {
     bool any = false, in[4];
     int at[4];
@@ -219,6 +241,7 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
       any |= in[j];
     }
     if (!any) continue;                // uniform over the wave
+    reached = true;
     int gc[4];
     float gv[4];
 #pragma unroll
@@ -238,7 +261,7 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
       pv += gv[j];
     }
   }
-  if (live) {
+  if (live && reached) {
     counts[slot] = c + pc;
     if (has_value) sums[slot] = v + pv;
   }
@@ -410,10 +433,26 @@ extern "C" long long qsa_window_chunk(long long n) {
       QSA_AGG_CHUNK, (n + QSA_AGG_BLOCKS - 1) / QSA_AGG_BLOCKS);
 }
 
-// words of workspace for n events, 0 for none
-extern "C" long long qsa_window_workspace(long long n) {
+// Words of workspace, 0 for the direct form.  Merging costs a second launch and
+// a pass over the output, 18 us for the smallest, so it takes 64 chunks (in
+// order, 400 keys, 288 windows, direct / merged: 200k events 17 / 21 us, 300k
+// 21 / 21, 500k 28 / 21), and it pays only where chunks fit in LDS.  In a stream
+// a chunk spans 4096 nwin / n windows and touches up to one more; where six in
+// ten would touch more than fit, or no chunk can, the direct form is ahead
+// (1000 keys, 288 windows, 200k events: 21 us against 40; 3000, 500k: 44 / 79;
+// 6000, 1M: 94 / 128; but 3000, 1M: 81 / 50 and 6000, 2M: 169 / 169).  Events in
+// no order have the merge in vain (7 us), except where the whole table fits:
+// there 17 chunks are enough (20 keys, 300 windows, 200k events: in order 8.6 /
+// 18, in none 62 / 29).
+extern "C" long long qsa_window_workspace(long long n, long long nkeys,
+                                          long long nwin, long long win_ms) {
   const long long chunk = qsa_window_chunk(n), blocks = (n + chunk - 1) / chunk;
-  return blocks <= QSA_AGG_DIRECT ? 0 : blocks * (2 + 2 * QSA_AGG_CELLS);
+  if (win_ms <= 0 || nkeys <= 0) return 0;
+  const long long fit = QSA_AGG_CELLS / nkeys;   // windows
+  if (fit == 0 || blocks <= (nwin <= fit ? 16 : 64) ||
+      10.0 * chunk * nwin > (double)n * (10 * fit - 4))
+    return 0;
+  return blocks * (2 + 2 * QSA_AGG_CELLS);
 }
 
 extern "C" void qsa_window_agg_launch(const long long* ts, const int* key,
@@ -423,19 +462,31 @@ extern "C" void qsa_window_agg_launch(const long long* ts, const int* key,
                                       long long n, int* ws,
                                       hipStream_t stream) {
   if (n == 0 || nwin <= 0 || nkeys <= 0) return;
-  // without a workspace, short chunks: a few thousand events on as many CUs
-  const long long chunk = ws ? qsa_window_chunk(n) : 256;
+  if (win_ms <= 0 || nkeys > QSA_AGG_CELLS) {
+    // 4096 blocks at most: 7000 keys, 8M events 832 us, 976 with a block for
+    // every 256
+    const unsigned grid =
+        (unsigned)std::min<long long>((n + 255) / 256, 4096);
+    hipLaunchKernelGGL(qsa_window_events, dim3(grid), dim3(256), 0, stream, ts,
+                       key, value, counts, sums, t0, win_ms, nwin, nkeys, n);
+    return;
+  }
+  // direct: chunks of 256 until they give every CU two blocks (1000 keys, 288
+  // windows, 100k events: 15.0 us, 15.8 with chunks of 1024; 200k: 22.7, 20.9)
+  const long long chunk = ws ? qsa_window_chunk(n)
+                             : n <= 512 * 256 ? 256 : 1024;
   const int blocks = (int)((n + chunk - 1) / chunk);
   int2* span = reinterpret_cast<int2*>(ws);
   int* cells = ws ? ws + 2 * blocks : nullptr;
-  if (chunk == QSA_AGG_CHUNK && win_ms > 0)
-    hipLaunchKernelGGL(qsa_window_agg<true>, dim3(blocks), dim3(256), 0,
-                       stream, ts, key, value, counts, sums, t0, win_ms, nwin,
-                       nkeys, n, chunk, span, cells);
-  else
-    hipLaunchKernelGGL(qsa_window_agg<false>, dim3(blocks), dim3(256), 0,
-                       stream, ts, key, value, counts, sums, t0, win_ms, nwin,
-                       nkeys, n, chunk, span, cells);
+#define QSA_AGG(PER, CELLS)                                                  \
+  hipLaunchKernelGGL((qsa_window_agg<PER, CELLS>), dim3(blocks), dim3(256),  \
+                     0, stream, ts, key, value, counts, sums, t0, win_ms,    \
+                     nwin, nkeys, n, chunk, span, cells)
+  if (chunk > QSA_AGG_CHUNK) QSA_AGG(0, QSA_AGG_CELLS);
+  else if (ws) QSA_AGG(QSA_AGG_CHUNK / 256, QSA_AGG_CELLS);
+  else if (chunk == 1024) QSA_AGG(4, QSA_AGG_CELLS);
+  else QSA_AGG(1, QSA_AGG_FEW);
+#undef QSA_AGG
   if (ws)
     hipLaunchKernelGGL(qsa_window_merge,
                        dim3((nwin + 7) / 8, (nkeys + 63) / 64), dim3(512), 0,

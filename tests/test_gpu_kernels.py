@@ -248,6 +248,35 @@ def test_window_agg_edges(ext, n, nkeys, nwin, shuffle):
     assert torch.equal(c.cpu(), counts) and not s.any()
 
 
+@pytest.mark.parametrize("n,nkeys,nwin", [
+    (131_072, 40, 200), (131_073, 40, 200),    # chunks of 256, of 1024
+    (140_000, 2049, 3), (262_144, 40, 154),
+    (262_145, 40, 154),                        # merged, 65 chunks
+    (65_536, 2048, 3), (65_537, 2048, 3),      # the whole table fits
+    (300_000, 6144, 44), (300_000, 6144, 43),  # six in ten chunks fit
+    (300_000, 6145, 1), (270_000, 4_200_000, 2),
+    (8_400_000, 10, 50)])                      # longer chunks
+def test_window_agg_forms(ext, n, nkeys, nwin):
+    """Both sides of the rule that chooses a form, events in order and not, and
+    more keys than a launch of the merge has rows for.  Whole values."""
+    g = torch.Generator().manual_seed(n + nkeys)
+    ts = torch.randint(-500, nwin * 1000 + 500, (n,), generator=g)
+    key = torch.randint(-1, nkeys + 1, (n,), generator=g, dtype=torch.int32)
+    key[:2] = torch.tensor([0, nkeys - 1])
+    val = torch.randint(-8, 9, (n,), generator=g).float()
+    for order in (ts.sort()[0], ts):
+        w = torch.div(order, 1000, rounding_mode="trunc")
+        ok = (w < nwin) & (key >= 0) & (key < nkeys)
+        at = (key.long() * nwin + w)[ok]
+        counts = torch.zeros(nkeys * nwin, dtype=torch.int32).index_add_(
+            0, at, torch.ones_like(at, dtype=torch.int32))
+        sums = torch.zeros(nkeys * nwin).index_add_(0, at, val[ok])
+        c, s = ext.window_agg(order.to(dev()), key.to(dev()), val.to(dev()),
+                              0, 1000, nwin, nkeys)
+        assert torch.equal(c.cpu().view(-1), counts)
+        assert torch.equal(s.cpu().view(-1), sums)
+
+
 @pytest.mark.parametrize("n", [1, 5, 6, 9, 12, 20, 63, 64, 69, 288, 7000])
 def test_anomaly_batch_lengths(ext, n):
     """Every order of the fit (0 to 4 lags) at lengths around the wave."""
