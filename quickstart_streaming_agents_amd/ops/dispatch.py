@@ -214,11 +214,18 @@ def _unobserved(*tensors: torch.Tensor) -> bool:
 
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether x[M,K] @ W^T is rows_linear's: a decode batch beyond the skinny
-    kernels, and a long K beside few columns, where it beats the library at
-    every M (figures in ops/hip/rows_gemm.hip)."""
+    kernels, and a long K beside few columns, where it beats the library
+    (figures in ops/hip/rows_gemm.hip; of 27 shapes at ten numbers of rows six
+    are up to 4% behind it, the others ahead, up to 3 times).  Small weights
+    leave little to split: up to 2560 x 8192 it takes K of five times the
+    columns, or of four and 64 rows (2560 x 8192 is behind by 8% at 33 to 48
+    rows and 13% at 192, 2048 x 8192 by 5% at 40 and ahead by 47% at 64)."""
     n, k = w.shape
-    return x.is_cuda and x.dim() == 2 and 32 < x.shape[0] <= 192 and \
-        k >= 3 * n and n * k >= 1 << 24 and n % 16 == 0 and k % 64 == 0 and \
+    m = x.shape[0]
+    small = n * k <= 5 << 22
+    return x.is_cuda and x.dim() == 2 and 32 < m <= 192 and \
+        n * k >= 1 << 24 and k >= (3 if not small else 4 if m >= 64 else 5) * n \
+        and n % 16 == 0 and k % 64 == 0 and \
         x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and \
         x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
         x.stride(0) < 1 << 24 and _unobserved(x, w) and \

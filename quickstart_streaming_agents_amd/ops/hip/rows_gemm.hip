@@ -9,11 +9,18 @@
 // for its four waves), and W goes from memory to the matrix cores' operands
 // directly, 32 columns a wave, 128 bytes of each at a time.  The shares' sums
 // meet in f32 in a second kernel.
-// us, library GEMM -> here (sums included), at 40 / 64 / 128 / 192 rows:
-// 4096 x 14336 36 / 40 / 75 / 62 -> 28 / 32 / 43 / 54, 2048 x 8192 13.9 / 22.4
-// / 21.2 / 26.6 -> 13.7 / 15.6 / 20.9 / 25.9.  With N nearer to K the library's
-// larger tiles win: 4096 x 4096 at 192 rows 20.5 against 25.6, 16384 x 2048
-// 27.2 against 36.
+// us, library GEMM -> here (sums included, weights from memory), at 40 / 64 /
+// 128 / 192 rows:
+//   2048 x  8192  14.1 / 22.6 / 21.1 / 26.5 -> 14.7 / 15.4 / 21.0 / 25.9
+//   2560 x  8192  16.3 / 23.1 / 41.8 / 26.9 -> 17.5 / 18.7 / 25.1 / 30.9
+//   1536 x 11264  20.8 / 31.0 / 27.2 / 38.2 -> 16.9 / 18.1 / 24.1 / 30.1
+//   2560 x 10240  20.9 / 30.5 / 55.8 / 36.7 -> 19.5 / 21.2 / 27.8 / 34.7
+//   4096 x 14336  36.7 / 41.2 / 76.2 / 64.3 -> 29.1 / 32.0 / 42.1 / 54.6
+//   4096 x 16384  38.8 / 42.5 / 82.4 / 115  -> 39.5 / 39.8 / 48.3 / 58.3
+//   5120 x 15360  49.7 / 53.9 / 82.8 / 112  -> 40.0 / 43.4 / 54.8 / 68.4
+//   8192 x 24576   113 /  130 /  181 /  210 ->  104 /  113 /  130 /  159
+// With N nearer to K the library's larger tiles win: 4096 x 4096 at 192 rows
+// 20.5 against 25.6, 16384 x 2048 27.2 against 36.
 #include "lm_common.h"
 
 struct RowsArgs {
@@ -142,10 +149,12 @@ qsa_rows_sum(const float* __restrict__ part, bf16_t* __restrict__ C,
       make_uint2(cvt_bf16x2(v[0], v[1]), cvt_bf16x2(v[2], v[3]));
 }
 
-// Shares of K: a block for each of the 256 CUs.
+// Shares of K: a block for each of the 256 CUs and none left over, which would
+// have some CUs do the work of two (2560 x 10240 with 13 shares, 260 blocks:
+// 28.8 us at 40 rows, 56.8 at 192; with 12: 19.5 and 34.7).
 extern "C" int qsa_rows_gemm_shares(int N, int K) {
   const int blocks = (N + 127) / 128, steps = K >> 6;
-  const int want = (256 + blocks - 1) / blocks;
+  const int want = blocks < 256 ? 256 / blocks : 1;
   return want < steps ? want : steps;
 }
 

@@ -541,12 +541,20 @@ def test_rows_gemm(M, N, K):
     assert ((got - a @ b.T).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M", [33, 192])
+@pytest.mark.parametrize("N,K", [(1280, 2112), (2576, 4160)])
+def test_rows_gemm_uneven_shares(M, N, K):
+    """Columns that divide the chip with a remainder, shares of unlike length
+    (33 steps of K in 25, 65 in 12)."""
+    test_rows_gemm(M, N, K)
+
+
 def test_linear_of_rows_far_apart():
     """The kernel's offsets of a row have 32 bits; rows too far apart for them
     are the library's."""
     from quickstart_streaming_agents_amd.models.layers import Linear
-    K, far = 8192, 1 << 24
-    w = rnd(gen(1), 2048, K, dtype=BF).to(DEV)
+    K, far = 16_384, 1 << 24
+    w = rnd(gen(1), 1024, K, dtype=BF).to(DEV)
     store = torch.empty(32 * far + K, dtype=BF, device=DEV)
     for step in (far - 8, far):
         x = store.as_strided((33, K), (step, 1))
@@ -562,7 +570,7 @@ def test_linear_under_observation():
     import torch.autograd.forward_ad as fwd
     from torch.fx.experimental.proxy_tensor import make_fx
     from quickstart_streaming_agents_amd.models.layers import Linear
-    M, N, K = 40, 2048, 8192
+    M, N, K = 40, 1024, 16_384
     x, t = (rnd(gen(s), M, K, dtype=BF).to(DEV) for s in (1, 2))
     w = rnd(gen(3), N, K, dtype=BF, scale=K ** -0.5).to(DEV)
     lin = Linear(w)
