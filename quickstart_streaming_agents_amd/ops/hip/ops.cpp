@@ -117,9 +117,11 @@ extern "C" void qsa_encoder_attn_launch(
     const int*, const int*, const int*, unsigned short*, int, int, int, float,
     hipStream_t);
 extern "C" int qsa_topk_block_docs(long long, long long);
-extern "C" void qsa_topk_launch(const float*, const float*, float*, int*,
-                                float*, int*, int, int, int, int, int,
-                                hipStream_t);
+extern "C" void qsa_topk_scan_launch(const float*, const float*, float*, int*,
+                                     int, int, int, int, int, hipStream_t);
+extern "C" int qsa_topk_groups(int);
+extern "C" void qsa_topk_merge_launch(const float*, const int*, float*, int*,
+                                      int, int, int, hipStream_t);
 extern "C" void qsa_window_agg_launch(const long long*, const int*,
                                       const float*, int*, float*, long long,
                                       long long, int, int, long long, int*,
@@ -750,19 +752,29 @@ std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
   TORCH_CHECK(docs.size(1) == D, "dim mismatch");
   TORCH_CHECK(k >= 1 && k <= 16, "k in [1,16]");
   const int per = qsa_topk_block_docs(Q, N);
-  const int nblk = std::max(1, (N + per - 1) / per);
+  int lists = (N + per - 1) / per;
   auto opts_f = queries.options();
   auto opts_i = queries.options().dtype(at::kInt);
-  auto cand_s = torch::empty({Q, nblk, k}, opts_f);
-  auto cand_i = torch::empty({Q, nblk, k}, opts_i);
-  auto out_s = torch::empty({Q, k}, opts_f);
-  auto out_i = torch::empty({Q, k}, opts_i);
-  if (Q == 0) return {out_s, out_i};
-  qsa_topk_launch(queries.data_ptr<float>(), docs.data_ptr<float>(),
-                  cand_s.data_ptr<float>(), cand_i.data_ptr<int>(),
-                  out_s.data_ptr<float>(), out_i.data_ptr<int>(), Q, N, D,
-                  (int)k, nblk, cur_stream());
-  return {out_s, out_i};
+  if (Q == 0)
+    return {torch::empty({Q, k}, opts_f), torch::empty({Q, k}, opts_i)};
+  auto s = torch::empty({Q, lists, k}, opts_f);
+  auto i = torch::empty({Q, lists, k}, opts_i);
+  qsa_topk_scan_launch(queries.data_ptr<float>(), docs.data_ptr<float>(),
+                       s.data_ptr<float>(), i.data_ptr<int>(), Q, N, D, (int)k,
+                       lists, cur_stream());
+  do {
+    const int groups = qsa_topk_groups(lists);
+    auto to_s = groups > 1 ? torch::empty({Q, groups, k}, opts_f)
+                           : torch::empty({Q, k}, opts_f);
+    auto to_i = torch::empty(to_s.sizes(), opts_i);
+    qsa_topk_merge_launch(s.data_ptr<float>(), i.data_ptr<int>(),
+                          to_s.data_ptr<float>(), to_i.data_ptr<int>(), Q,
+                          lists, (int)k, cur_stream());
+    s = to_s;
+    i = to_i;
+    lists = groups;
+  } while (lists > 1);
+  return {s, i};
 }
 
 std::vector<torch::Tensor> window_agg(torch::Tensor ts, torch::Tensor key,

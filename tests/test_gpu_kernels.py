@@ -219,6 +219,28 @@ def test_window_agg(ext):
     torch.testing.assert_close(sums.cpu(), rs, atol=1e-1, rtol=1e-4)
 
 
+@pytest.mark.parametrize("Q,N,k", [
+    (3, 262_144, 16), (3, 262_145, 16),      # 4096 and 4097 lists of 64
+    (17, 131_072, 5), (17, 131_073, 5),      # and of 32
+    (1, 900_001, 16)])
+def test_topk_cosine_many_lists(ext, Q, N, k):
+    """More lists than one merge holds; the best documents all in the last
+    list, in the first, in any.  Small whole numbers: exact."""
+    g = torch.Generator().manual_seed(N)
+    docs = torch.randint(-2, 3, (N, 4), generator=g).float()
+    qs = torch.randint(1, 3, (Q, 4), generator=g).float()
+    docs[-k:] = 3 + torch.arange(k).float()[:, None]
+    if Q > 1:
+        qs[1] = -qs[1]
+        docs[:k] = -4.0
+    s, i = ext.topk_cosine(qs.to(dev()), docs.to(dev()), k)
+    full = qs @ docs.T
+    full[full <= -2] = -float("inf")
+    top, order = torch.sort(full, dim=1, descending=True, stable=True)
+    assert torch.equal(s.cpu(), top[:, :k])
+    assert torch.equal(i.cpu(), order[:, :k].int())
+
+
 @pytest.mark.parametrize("n,nkeys,nwin,shuffle", [
     (1, 1, 1, False), (255, 3, 2, True), (257, 6144, 1, False),
     (5000, 6145, 2, False),              # one key more than a block's cells
