@@ -63,6 +63,20 @@ class HashingEmbedder:
             np.zeros((0, self.dim), dtype=np.float32)
 
 
+def _scan_wins(queries: int, rows: int, k: int) -> bool:
+    """Whether a search is the kernel's (ops/hip/topk_cosine.hip) or a matmul's
+    with a sort.  Measured at 1536 numbers a row (us, kernel / matmul): up to
+    16 queries are one read of the matrix (16, k = 16: 100k rows 194 / 312, 1M
+    1517 / 1536), up to 32 one and more work per row (32, k = 3: 100k 219 /
+    311, 200k 418 / 571, 300k 609 / 659, 500k 1001 / 924, 1M 1973 / 1556).
+    More are GEMM-shaped (48, k = 8: 26k 138 / 170, 45k 189 / 189, 100k 384 /
+    289)."""
+    if k > 16:                       # what the kernel keeps
+        return False
+    return queries <= 16 or \
+        queries * rows <= 1_500_000 or queries <= 32 and rows <= 262_144
+
+
 class VectorIndex:
     """Exact cosine top-k over L2-normalized rows.
 
@@ -165,19 +179,15 @@ class VectorIndex:
         docs = self.to_torch(device)
         qt = torch.from_numpy(q).to(device=device, dtype=torch.float32)
         k_eff = min(k, len(self))
-        if k_eff > 16 or len(q) > 32 and len(q) * len(self) > 1_500_000 or \
-                not np.isfinite(q).all():
-            # many queries are GEMM-shaped: a matmul over the HBM matrix and
-            # a sort of the scores (48 queries: 165 us against 135 of the
-            # kernel at 30k rows, 189 against 245 at 60k).  The kernel keeps
-            # at most 16 hits and has none for a query that is not a number.
+        if not _scan_wins(len(q), len(self), k_eff) or not (
+                np.isfinite(norms).all() or np.isfinite(q).all()):
+            # a matmul over the HBM matrix and a sort of the scores; the
+            # kernel has no answer for a query that is not a number
             scores_all = qt @ docs.T
             scores, idx = torch.topk(scores_all, k_eff, dim=1)
             idx = idx.int()
         else:
-            # the tiled cosine/top-k HIP kernel, up to 32 queries per read of
-            # the matrix (100k rows: 161 us against 322 at 16 queries, 222
-            # against 317 at 32)
+            # the tiled cosine/top-k HIP kernel
             scores, idx = D.topk_cosine(qt.contiguous(), docs, k_eff)
         scores = scores.cpu().numpy()
         idx = idx.cpu().numpy()

@@ -88,3 +88,13 @@ def test_add_documents_embeds_missing_and_keeps_metadata():
     hits = idx.search(emb.embed("flink joins"), k=1)
     assert hits[0].document_id == "b"
     assert hits[0].metadata["title"] == "Joins"
+
+
+def test_routes_of_gpu_searches():
+    """Which searches are the kernel's: few queries at any size, up to 32 until
+    the matmul is ahead, and no more hits than it keeps."""
+    from quickstart_streaming_agents_amd.vector.index import _scan_wins as w
+    assert w(1, 10 ** 7, 16) and w(16, 10 ** 7, 16) and not w(1, 10, 17)
+    assert w(17, 262_144, 16) and w(32, 262_144, 3)
+    assert not w(17, 262_145, 3) and not w(32, 10 ** 6, 1)
+    assert w(33, 45_454, 16) and not w(33, 45_455, 1) and w(1000, 1500, 3)
