@@ -675,6 +675,29 @@ def test_skinny_bf16_rows(ext, M, N, K):
     assert (out.double() - want).norm() < 2 ** -8 * want.norm()
 
 
+def test_fp8_block_sweep(ext):
+    """tools/fp8_bench.py times every block shape of the probe, and each of
+    them computes the product."""
+    import os
+    import sys
+    sys.path.insert(0, os.path.join(
+        os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tools"))
+    import fp8_bench
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    torch.manual_seed(5)
+    M, N, K = 24, 192, 768
+    a = torch.randn(M, K, device=dev(), dtype=torch.bfloat16)
+    packed = D.pack_weight_fp8(torch.randn(N, K, device=dev()).bfloat16())
+    assert [t[:2] for t in fp8_bench.sweep(a, *packed, N, K)] == \
+        fp8_bench.BLOCKS
+    want = a.double() @ D.unpack_weight_fp8(*packed, N, K).double().T
+    for waves, tiles in fp8_bench.BLOCKS:
+        out = ext.skinny_gemm_fp8_probe(a, *packed, M, N, K, waves, tiles)
+        assert (out.double() - want).norm() < 2 ** -8 * want.norm()
+    with pytest.raises(RuntimeError, match="no such block shape"):
+        ext.skinny_gemm_fp8_probe(a, *packed, M, N, K, 16, 1)
+
+
 @pytest.mark.parametrize("M", [1, 4, 5, 17])
 def test_embed_rows(ext, M):
     embed = torch.randn(100, 288, device=dev(), dtype=torch.bfloat16)

@@ -24,6 +24,8 @@ SHAPES = [  # (name, N, K) for llama3-8b decode projections
 ]
 M = 24
 REPS = 50
+# (waves, tiles of 16 columns) of a block that the probe is built for
+BLOCKS = [(4, 1), (8, 1), (4, 2), (8, 2), (4, 4), (8, 4)]
 
 
 def timeit(fn, reps=REPS):
@@ -35,6 +37,14 @@ def timeit(fn, reps=REPS):
         fn()
     torch.cuda.synchronize()
     return (time.perf_counter() - t0) / reps * 1e6  # us
+
+
+def sweep(a, qf, s, N, K):
+    """(waves, tiles, us) of every block shape that N divides into."""
+    for waves, tiles in BLOCKS:
+        if N % (16 * tiles) == 0:
+            yield waves, tiles, timeit(lambda: ext().skinny_gemm_fp8_probe(
+                a, qf, s, a.shape[0], N, K, waves, tiles), reps=20)
 
 
 def main():
@@ -53,19 +63,10 @@ def main():
         t_bf = timeit(lambda: ext().skinny_gemm(a, wf, N, K))
         t_f8 = timeit(lambda: ext().skinny_gemm_fp8(a, qf, s, N, K))
         if os.environ.get("QSA_FP8_SWEEP") == "1":
-            for waves, tiles in [(4, 1), (8, 1), (16, 1), (4, 2), (8, 2),
-                                 (2, 4), (4, 4), (8, 4)]:
-                if N % (16 * tiles):
-                    continue
-                try:
-                    t = timeit(lambda: ext().skinny_gemm_fp8_probe(
-                        a, qf, s, N, K, waves, tiles), reps=20)
-                    print(f"    probe {name} w{waves} t{tiles}: "
-                          f"{t:.1f} us ({(N*K)/(t*1e-6)/1e9:.0f} GB/s)",
-                          file=sys.stderr)
-                except Exception as e:
-                    print(f"    probe {name} w{waves} t{tiles}: {e}",
-                          file=sys.stderr)
+            for waves, tiles, t in sweep(a, qf, s, N, K):
+                print(f"    probe {name} w{waves} t{tiles}: "
+                      f"{t:.1f} us ({(N*K)/(t*1e-6)/1e9:.0f} GB/s)",
+                      file=sys.stderr)
         # correctness spot check
         ref = a.float() @ D.unpack_weight_fp8(qf, s, N, K).T
         out = ext().skinny_gemm_fp8(a, qf, s, N, K).float()
