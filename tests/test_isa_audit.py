@@ -45,7 +45,8 @@ def test_mixer_kernels(lm_stats):
     scratch, and no packed f32 arithmetic was formed."""
     for frag in ("retention_state", "retention_out", "latent_rows_mfma",
                  "window_attn_prefill", "head_matmul_mfma", "skinny_gemm",
-                 "gqa_rows_mfma", "gqa_portions", "ssd_state", "ssd_out"):
+                 "gqa_rows_mfma", "gqa_portions", "ssd_state", "ssd_out",
+                 "rows_gemm"):
         for name, st in _named(lm_stats, frag).items():
             assert st["mfma"] >= 4, f"{name}: only {st['mfma']} v_mfma"
     for name, st in lm_stats.items():
@@ -65,17 +66,25 @@ def test_matrix_kernels_use_mfma(stats):
     for frag in ("paged_attn_mfma", "paged_attn_prefill", "skinny_gemm"):
         for name, st in _named(stats, frag).items():
             assert st["mfma"] >= 8, f"{name}: only {st['mfma']} v_mfma"
+    for frag in ("encoder_attn", "short_gemm", "topk_scan"):
+        for name, st in _named(stats, frag).items():
+            assert st["mfma"] >= 4, f"{name}: only {st['mfma']} v_mfma"
 
 
 def test_no_spills_or_scratch_on_hot_kernels(stats):
     hot = ("paged_attn", "skinny_gemm", "rmsnorm", "rope", "swiglu",
-           "softmax", "kv_append", "kv_scatter", "topk")
+           "softmax", "kv_append", "kv_scatter", "topk", "encoder_attn",
+           "short_gemm", "embed_rows", "mean_rows", "window_agg",
+           "window_merge", "anomaly_batch")
     for frag in hot:
         for name, st in _named(stats, frag).items():
             assert st.get("vgpr_spill_count", 0) == 0, name
             assert st.get("sgpr_spill_count", 0) == 0, name
             assert st.get("private_segment_fixed_size", 0) == 0, \
                 f"{name}: scratch allocated"
+    for name, st in stats.items():
+        if name.startswith("_Z"):
+            assert st.get("packed_f32", 0) == 0, name
 
 
 def test_fp8_and_join_kernels_present_and_clean(stats):
