@@ -276,10 +276,11 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
       ml[wave][col][0] = m;
       ml[wave][col][1] = l;
     }
+    if (n > 0 && ia < ib)
 #pragma unroll
-    for (int t = 0; t < ET; ++t)
-      *reinterpret_cast<f32x4_v*>(mine + col * (16 * ET) + t * 16 + hi * 4) =
-          acc[t];
+      for (int t = 0; t < ET; ++t)
+        *reinterpret_cast<f32x4_v*>(mine + col * (16 * ET) + t * 16 + hi * 4) =
+            acc[t];
     __syncthreads();
     const int heads = min(16, RG - ht * 16);
     for (int i = threadIdx.x; i < heads * (E / 2); i += 256) {

@@ -652,6 +652,28 @@ static bool gqa_aligned(const Tensor& q, const OptTensor& gate,
 
 // q [R, H*D] rows -> rows of out; row_item: which block_table row a query row
 // uses (none: its own index); row_len: position + 1 (0: row not in use)
+// Rows that fill the chip with four shares each may be finished by the block,
+// which saves the partial results and a launch; where rows are so many or so
+// short that a wave each is enough, three of its four waves are in the way.  us,
+// shares and a merge kernel / in the block, heads of 128, keys 8:
+//    64 rows (512 tiles), 10-60 keys 10.5 /  7.4, 400-1000 37.5 / 34.1
+//   256 rows (2048)            14.0 / 20.9,                79.9 / 71.7
+//   1024 rows (8192)           39.6 / 71.6,                 264 / 250
+// 50-300 keys, a table of five pages: 192 rows 33.9 / 31.0, 512 50.5 / 60.4; of
+// heads of 64: 512 rows 29.7 / 26.7, 1024 49.9 / 50.6.  Heads beyond 128 leave
+// one block a CU: 17 heads on 1 of 256 / 136, 300 rows (600 tiles) of 50-300 34
+// / 41, 512 rows of 400-1000 100 / 109; 16 on 4 of 192 / 128, 128 rows of
+// 50-300 (512) 26.7 / 21.6, 192 of 400-1000 (768) 90 / 76, 512 (2048) 136 / 141.
+// mp: the table's columns, as the rows' lengths are on the device.
+static bool gqa_merge_in_block(long long tiles, int mp, int D, int E) {
+  if (tiles < 512) return false;
+  const int wide = std::max(D, E);
+  if (wide > 128)
+    return tiles == 512 || (mp >= 8 && tiles <= (E <= 128 ? 1600 : 800));
+  if (tiles <= 1024 || mp >= 8) return true;
+  return mp >= 4 && (wide <= 64 || tiles <= 2048);
+}
+
 void gqa_rows(Tensor q, Tensor kc, Tensor vc, Tensor block_table,
               OptTensor row_item, Tensor row_len, OptTensor sink,
               OptTensor gate, Tensor out, long H, double scale,
@@ -674,17 +696,14 @@ void gqa_rows(Tensor q, Tensor kc, Tensor vc, Tensor block_table,
   const void* gp = gate ? gate->data_ptr() : nullptr;
   const long long gs = gate ? gate->stride(0) : 0;
   if (!f32 && gqa_mfma_ok(d.D, d.E) && gqa_aligned(q, gate, out)) {
-    // two waves a SIMD fill the chip; no shares that differ by a page when
-    // they need not.  Rows that fill it with four shares each are finished by
-    // the block, which saves the partial results and a launch (64 rows of
-    // 600-1400, 16 heads on 8: 69 us against 68 + 6)
     const long long tiles =
         (long long)d.R * d.G * ((d.H / d.G + 15) / 16);
-    long long ns = (2048 + tiles - 1) / tiles;
-    const bool merge = ns <= 4;
-    if (merge) {
-      ns = 4;
-    } else {
+    // two waves a SIMD fill the chip; no shares that differ by a page when
+    // they need not
+    const bool merge = gqa_merge_in_block(tiles, mp, d.D, d.E);
+    long long ns = 4;
+    if (!merge) {
+      ns = (2048 + tiles - 1) / tiles;
       ns = std::max<long long>(1, std::min<long long>(ns, mp));
       const long long per = (mp + ns - 1) / ns;
       ns = (mp + per - 1) / per;

@@ -524,6 +524,34 @@ def test_preset_on_engine():
     assert llm.engine.kv.free_slots == llm.engine.kv.n_slots
 
 
+@pytest.mark.parametrize("R,H,G,Dm,E,pages", [
+    (129, 8, 8, 64, 64, 3), (129, 8, 8, 64, 64, 4),    # 1032 tiles
+    (257, 16, 8, 128, 128, 7), (257, 16, 8, 128, 128, 8),
+    (513, 2, 1, 200, 24, 7), (513, 2, 1, 200, 24, 8),
+    (801, 2, 1, 24, 136, 8), (64, 8, 8, 200, 200, 1)])
+def test_grouped_attention_forms(R, H, G, Dm, E, pages):
+    """Both sides of the rule between shares and a block's own rows, which
+    looks at rows, head sizes and the table's width: rows without keys, of one
+    key and of all."""
+    g = gen(R + pages)
+    kc, vc = rnd(g, pages, G, 64, Dm, dtype=BF), rnd(g, pages, G, 64, E,
+                                                     dtype=BF)
+    q = rnd(g, R, H * Dm, dtype=BF)
+    n = torch.randint(0, pages * 64 + 1, (R,), generator=g)
+    n[:3] = torch.tensor([0, 1, pages * 64])
+    bt = torch.randperm(pages, generator=g).int().repeat(R, 1)
+    out = torch.empty(R, H * E, dtype=BF, device=DEV)
+    D.gqa_rows(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), None,
+               n.int().to(DEV), None, None, out, H, Dm ** -0.5, 1.0)
+    k, v = (t[bt[0].long()].transpose(0, 1).reshape(G, pages * 64, -1)
+            .double().repeat_interleave(H // G, 0) for t in (kc, vc))
+    s = torch.einsum("rhd,hjd->rhj", q.double().view(R, H, Dm), k) * Dm ** -0.5
+    s = s.masked_fill(torch.arange(pages * 64) >= n[:, None, None],
+                      float("-inf"))
+    want = torch.einsum("rhj,hje->rhe", s.softmax(-1).nan_to_num(0.0), v)
+    close(out, want.reshape(R, -1), BF)
+
+
 # ---- projections of larger decode batches -----------------------------------
 
 @pytest.mark.parametrize("M", [1, 33, 48, 49, 65, 97, 128, 129, 192])
