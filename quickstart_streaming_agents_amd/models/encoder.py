@@ -87,10 +87,15 @@ class EmbeddingEncoder:
     def _linear(self, x: torch.Tensor, w: torch.Tensor,
                 glu: bool = False) -> torch.Tensor:
         """x W^T, with glu silu(gate) * up of it, w = [gate; up] (GPU).  Short
-        K goes to a kernel of our own, and so does longer K for rows so few
-        that the library's host path is the bound (384 x 1536, 16 us of it:
-        7 against 5 us of kernel at 100 rows, 9.5 against 8.6 at 1600; 22
-        against 16 at 8800, where the kernels are)."""
+        K goes to a kernel of our own at any number of rows: at some it is
+        behind the library's as a kernel (1536 x 384, 8800 rows: 19.7 us, 17.4),
+        but a call with those products from the library above 3500 rows is
+        never faster (12 layers, 3848 rows 870 us here, 1130 with; 6396 1186,
+        1241; 7744 1263, 1403; 10,325 1579, 1577; 12,868 1801, 2032; 20,870
+        2709, 2722), as its kernels are uneven and its host path is 16 us a
+        product.  That also bounds few rows of longer K (384 x 1536: 10.9 us
+        of kernel at 400 rows, 7.6 in the library; at 8800, where kernels
+        count, 22.6 and 16.9)."""
         n, k = w.shape
         if w.dtype == torch.bfloat16 and k % 64 == 0 and n % 32 == 0 and \
                 (k <= 512 or x.shape[0] <= 2048):

@@ -9,10 +9,14 @@
 // one in registers, whole 128-byte lines of every operand, a block row's columns
 // on one die, results through LDS to whole lines, and the gate's columns beside
 // the up's in a wave, so that the activation costs no pass over memory.
-// us, library -> here, at 100 / 1600 / 8800 rows: 1536 x 384 4.8 / 8.0 / 17.3 ->
-// 3.4 / 6.9 / 20.5, 384 x 512 5.0 / 6.1 / 9.4 -> 3.8 / 4.6 / 9.7, 384 x 1536 4.9
-// / 8.6 / 16.3 -> 7.4 / 9.5 / 23; 3072 x 384 with the activation (here a pass of
-// its own, 16 us at 8800) 5.1 / 10.0 / 39 without -> 3.6 / 10.8 / 35 with it.
+// us as kernels, library -> here, at 400 / 1600 / 4000 / 8800 / 16000 rows:
+//   1536 x 384  6.6 / 9.3 / 12.2 / 17.4 / 34.0 -> 5.3 / 7.2 / 12.3 / 19.7 / 29.1
+//   384 x 512   6.7 / 7.6 /  9.6 / 10.8 / 14.6 -> 5.3 / 5.7 /  6.7 / 10.3 / 15.3
+//   384 x 1536  7.6 / 9.6 / 13.1 / 16.9 / 23.4 -> 10.9 / 11.7 / 13.6 / 22.6 / 34
+//   3072 x 384 with the activation, there a pass of its own
+//               11.3 / 18.4 / 31.9 / 71 / 72.6 -> 6.3 / 11.3 / 17.9 / 34.1 / 56.9
+// The library is uneven in the rows (1536 x 384: 14.3 at 5470, 22.1 at 5817, 16.5
+// at 8246, 29 to 42 from 11000 to 12500).
 #include "lm_common.h"
 
 struct ShortArgs {
