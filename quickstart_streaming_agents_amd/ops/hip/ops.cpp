@@ -762,6 +762,8 @@ std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
   qsa_topk_scan_launch(queries.data_ptr<float>(), docs.data_ptr<float>(),
                        s.data_ptr<float>(), i.data_ptr<int>(), Q, N, D, (int)k,
                        lists, cur_stream());
+  // a single list is the result (5 rows, k = 5: 17.5 us with the merge)
+  if (lists == 1) return {s.view({Q, k}), i.view({Q, k})};
   do {
     const int groups = qsa_topk_groups(lists);
     auto to_s = groups > 1 ? torch::empty({Q, groups, k}, opts_f)
