@@ -2,7 +2,7 @@
 
 Extracts the .hip_fatbin bundles from the built extension, disassembles
 each gfx950 code object, and reports per-kernel instruction mix +
-resource metadata (the committed evidence in profiles/ comes from here).
+resource metadata (`isa_check.py profiles` writes the two tables there).
 Used by tests to guard two invariants:
   * matrix kernels (attention, skinny GEMM) issue v_mfma instructions
   * no hot kernel spills registers or allocates scratch
@@ -14,6 +14,7 @@ import glob
 import os
 import re
 import subprocess
+import sys
 import tempfile
 
 LLVM = "/opt/rocm/lib/llvm/bin"
@@ -74,6 +75,10 @@ def kernel_stats(hsacos: list[str]) -> dict[str, dict]:
                 continue
             if cur and "\t" in line:
                 stats[cur]["total"] += 1
+                for kind, start in (("lds", "ds_"), ("buf", "buffer_"),
+                                    ("glb", "global_")):
+                    if f"\t{start}" in line:
+                        stats[cur][kind] = stats[cur].get(kind, 0) + 1
                 if "v_mfma" in line:
                     stats[cur]["mfma"] += 1
                 elif re.search(r"v_pk_(add|mul|fma)_f32", line):
@@ -88,9 +93,11 @@ def kernel_stats(hsacos: list[str]) -> dict[str, dict]:
                 continue
             st = stats.setdefault(name.group(1), {"mfma": 0, "total": 0})
             for field in ("vgpr_spill_count", "sgpr_spill_count",
-                          "private_segment_fixed_size"):
+                          "private_segment_fixed_size", "vgpr_count",
+                          "sgpr_count", "group_segment_fixed_size"):
                 m = re.search(rf"\.{field}:\s*(\d+)", blk)
                 st[field] = int(m.group(1)) if m else 0
+            st["agpr_count"] = int(re.match(r"\s*(\d+)", blk).group(1))
     return stats
 
 
@@ -103,13 +110,27 @@ def main() -> int:
     for so in found:
         with tempfile.TemporaryDirectory() as wd:
             stats.update(kernel_stats(extract_hsacos(so, wd)))
+    mix, resources = [], []
     for name, st in sorted(stats.items()):
-        if st["total"] > 60:
-            print(f"{name[:64]:64s} instr={st['total']:5d} "
-                  f"mfma={st['mfma']:3d} "
-                  f"scratch={st.get('private_segment_fixed_size', 0)} "
-                  f"spills={st.get('vgpr_spill_count', 0)}"
-                  f"/{st.get('sgpr_spill_count', 0)}")
+        if not name.startswith("_Z") or "vgpr_count" not in st:
+            continue
+        mix.append(f"{name[:76]:76s} instr={st['total']:5d} "
+                   f"mfma={st['mfma']:3d} lds={st.get('lds', 0):3d} "
+                   f"buf={st.get('buf', 0):3d} glb={st.get('glb', 0):3d}")
+        resources.append(f"{name[:64]:64s} vgpr={st['vgpr_count']:3d} "
+                         f"agpr={st['agpr_count']:3d} "
+                         f"sgpr={st['sgpr_count']:3d} "
+                         f"lds={st['group_segment_fixed_size']:6d} "
+                         f"scratch={st['private_segment_fixed_size']:4d} "
+                         f"spills(v/s)={st['vgpr_spill_count']}"
+                         f"/{st['sgpr_spill_count']}")
+    if len(sys.argv) > 1:            # the two tables of profiles/
+        for file, lines in (("isa_instruction_mix_gfx950.txt", mix),
+                            ("kernel_resources_gfx950.txt", resources)):
+            with open(os.path.join(sys.argv[1], file), "w") as f:
+                f.write("\n".join(lines) + "\n")
+    else:
+        print("\n".join(mix + resources))
     return 0
 
 
