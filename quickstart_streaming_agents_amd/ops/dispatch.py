@@ -11,7 +11,6 @@ CPU-only CI.  A CUDA tensor NEVER falls back to the CPU path.
 from __future__ import annotations
 
 import torch
-from torch.autograd import forward_ad
 
 from . import ext, lm_ext
 
@@ -198,38 +197,12 @@ def pack_weight_frag(w: torch.Tensor) -> torch.Tensor:
     return w.reshape(n // 16, 16, k // 32, 32).permute(0, 2, 1, 3).contiguous()
 
 
-def _unobserved(*tensors: torch.Tensor) -> bool:
-    """Whether only the values of the tensors matter: derivatives in either
-    direction, function transforms, tracing, autocast, modes and subclasses
-    see the library's operations and would pass a kernel of our own by."""
-    return not (torch.is_grad_enabled() and
-                any(t.requires_grad for t in tensors)) and \
-        forward_ad._current_level < 0 and \
-        torch._C._functorch.peek_interpreter_stack() is None and \
-        torch._C._len_torch_dispatch_stack() == 0 and \
-        not torch.jit.is_tracing() and not torch.compiler.is_compiling() and \
-        not torch.is_autocast_enabled("cuda") and \
-        all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
-
-
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether x[M,K] @ W^T is rows_linear's: a decode batch beyond the skinny
-    kernels, and a long K beside few columns, where it beats the library
-    (figures in ops/hip/rows_gemm.hip; of 27 shapes at ten numbers of rows six
-    are up to 4% behind it, the others ahead, up to 3 times).  Small weights
-    leave little to split: up to 2560 x 8192 it takes K of five times the
-    columns, or of four and 64 rows (2560 x 8192 is behind by 8% at 33 to 48
-    rows and 13% at 192, 2048 x 8192 by 5% at 40 and ahead by 47% at 64)."""
-    n, k = w.shape
-    m = x.shape[0]
-    small = n * k <= 5 << 22
-    return x.is_cuda and x.dim() == 2 and 32 < m <= 192 and \
-        n * k >= 1 << 24 and k >= (3 if not small else 4 if m >= 64 else 5) * n \
-        and n % 16 == 0 and k % 64 == 0 and \
-        x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and \
-        x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
-        x.stride(0) < 1 << 24 and _unobserved(x, w) and \
-        (x.data_ptr() | w.data_ptr()) % 16 == 0
+    kernels on a long K, where nobody looks at the operation itself (the rules
+    are in ops/hip/lm_ops.cpp)."""
+    return x.is_cuda and type(x) is torch.Tensor and \
+        lm_ext().rows_gemm_ok(x, w) and not torch.compiler.is_compiling()
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -3,7 +3,10 @@
 // assume; the matrix-core variants are chosen here where the sizes fit them.
 #include <hip/hip_runtime.h>
 #include <torch/extension.h>
+#include <ATen/TracerMode.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/HIPContext.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 
 typedef unsigned short bf16_t;
 
@@ -902,6 +905,48 @@ Tensor skinny_gemm(Tensor a, Tensor wf, long N, long K) {
   return out;
 }
 
+// Whether only the values of a tensor matter: derivatives in either direction,
+// function transforms, traces, modes and autocast see the library's operations
+// and would pass a kernel of our own by.
+static bool unobserved(const Tensor& t) {
+  using K = c10::DispatchKey;
+  return !(at::GradMode::is_enabled() && t.requires_grad()) &&
+         !t._fw_grad(0).defined() &&
+         !t.key_set().has_any(c10::DispatchKeySet(
+             {K::Python, K::FuncTorchBatched, K::FuncTorchGradWrapper,
+              K::Batched, K::Functionalize, K::Conjugate, K::Negative,
+              K::ZeroTensor}));
+}
+
+static bool no_observer() {
+  return !c10::impl::tls_local_dispatch_key_set().included_.has(
+             c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+         !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+         !at::tracer::impl::is_dispatch_enabled() &&
+         !at::autocast::is_autocast_enabled(at::kCUDA);
+}
+
+// Whether a @ w^T is rows_gemm's: 33 to 192 rows and a long K beside few
+// columns, where it beats the library (figures in rows_gemm.hip; of 27 shapes at
+// ten numbers of rows six are up to 5% behind it at some, the others ahead, up to
+// 3 times, and a call that is not captured saves some 10 us of the library's
+// host path).  Small weights leave little to split: up to 2560 x 8192, itself
+// behind by 8% at 33 to 48 rows and 13% at 192, it takes K of four times the
+// columns.  The whole rule here: in Python the last part alone took 2 us of a
+// call, 2% of a step of 40 tokens.
+bool rows_gemm_ok(const Tensor& a, const Tensor& w) {
+  if (a.dim() != 2 || w.dim() != 2) return false;
+  const int64_t M = a.size(0), N = w.size(0), K = w.size(1);
+  return M > 32 && M <= 192 && N * K >= 1 << 24 &&
+         K >= (N * K <= 5 << 22 ? 4 : 3) * N && N % 16 == 0 && K % 64 == 0 &&
+         a.size(1) == K && a.is_cuda() && a.device() == w.device() &&
+         a.scalar_type() == at::kBFloat16 &&
+         w.scalar_type() == at::kBFloat16 && no_observer() && unobserved(a) &&
+         unobserved(w) && w.is_contiguous() && a.stride(1) == 1 &&
+         a.stride(0) % 8 == 0 && a.stride(0) < (1 << 24) && aligned(a, 16) &&
+         aligned(w, 16);
+}
+
 // a @ w^T on W as it is stored, K split over the chip
 Tensor rows_gemm(Tensor a, Tensor w) {
   CHK_DEV(a); chk_rows(a, "a"); CHK_CONT(w); CHK_SAME(a, w);
@@ -953,4 +998,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("window_attn_ok", &window_attn_ok, "size support");
   m.def("skinny_gemm", &skinny_gemm, "packed-weight decode GEMM (M <= 32)");
   m.def("rows_gemm", &rows_gemm, "long-K decode GEMM (M <= 192)");
+  m.def("rows_gemm_ok", &rows_gemm_ok, "whether a product is rows_gemm's");
 }
