@@ -189,15 +189,12 @@ class VectorIndex:
         else:
             # the tiled cosine/top-k HIP kernel
             scores, idx = D.topk_cosine(qt.contiguous(), docs, k_eff)
-        scores = scores.cpu().numpy()
-        idx = idx.cpu().numpy()
-        out = []
-        for qi in range(len(q)):
-            # -1: fewer documents than k have a score
-            out.append([SearchHit(self.ids[i], self.chunks[i],
-                                  float(scores[qi, j]), self.metadata[i])
-                        for j, i in enumerate(idx[qi]) if i >= 0])
-        return out
+        scores = scores.cpu().numpy().tolist()
+        idx = idx.cpu().numpy().tolist()
+        # -1: fewer documents than k have a score
+        return [[SearchHit(self.ids[i], self.chunks[i], s, self.metadata[i])
+                 for i, s in zip(ids, row) if i >= 0]
+                for ids, row in zip(idx, scores)]
 
     @staticmethod
     def mongo_score(cosine: float) -> float:
