@@ -7,7 +7,6 @@ import math
 
 import numpy as np
 import torch
-import torch.nn.functional as F
 
 from ..ops import dispatch as D
 
@@ -15,8 +14,8 @@ from ..ops import dispatch as D
 class Linear:
     """y = x W^T.  On the GPU in bf16, decode-sized batches of the small
     shapes stream a packed copy of W (ops/hip/skinny_gemm.hip, the measured
-    winner there) and larger ones of long K split it (ops/hip/rows_gemm.hip);
-    everything else is a vendor GEMM."""
+    winner there), all that do not fill a library's tiles are
+    ops/hip/rows_gemm.hip's, and the rest is a vendor GEMM."""
 
     SKINNY_ROWS = 32
     SKINNY_MAX = 6144 * 4096
@@ -30,13 +29,20 @@ class Linear:
             self.packed = D.pack_weight_frag(w)
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
-        n, k = self.w.shape
-        if self.packed is not None and 1 <= x.shape[0] <= self.SKINNY_ROWS \
-                and x.stride(0) % 8 == 0:
-            return D.skinny_linear(x, self.packed, n, k)
-        if D.rows_linear_ok(x, self.w):
-            return D.rows_linear(x, self.w)
-        return F.linear(x, self.w)
+        if self._skinny(x):
+            return D.skinny_linear(x, self.packed, *self.w.shape)
+        return D.linear(x, self.w)
+
+    def _skinny(self, x: torch.Tensor) -> bool:
+        return self.packed is not None and \
+            1 <= x.shape[0] <= self.SKINNY_ROWS and x.stride(0) % 8 == 0
+
+    def glu(self, x: torch.Tensor, act: str) -> torch.Tensor:
+        """act(gate) * up of y = [gate, up]."""
+        if not self._skinny(x) and D.glu_linear_ok(x, self.w):
+            return D.glu_linear(x, self.w, act)
+        y, half = self(x), self.w.shape[0] // 2
+        return D.glu(y[:, :half], y[:, half:], act)
 
 
 def rope_frequencies(dims: int, base: float,
@@ -86,13 +92,12 @@ class DenseGLU:
 
     def __init__(self, gate: torch.Tensor, up: torch.Tensor,
                  down: torch.Tensor, act: str = "silu"):
-        self.ff, self.act = gate.shape[0], act
+        self.act = act
         self.gate_up = Linear(torch.cat([gate, up]).contiguous())
         self.down = Linear(down)
 
     def __call__(self, h: torch.Tensor) -> torch.Tensor:
-        gu = self.gate_up(h)
-        return self.down(D.glu(gu[:, :self.ff], gu[:, self.ff:], self.act))
+        return self.down(self.gate_up.glu(h, self.act))
 
 
 class TokenSide:

@@ -216,8 +216,8 @@ class LlamaModel:
                 wf8: tuple | None = None) -> torch.Tensor:
         """Projection: decode-sized cuda batches go through the
         weight-streaming skinny GEMM — fp8 (W8A16, half the weight
-        stream) when packed, else bf16; batches beyond on a long K through
-        rows_gemm; everything else rocBLAS."""
+        stream) when packed, else bf16; what does not fill a library's tiles
+        through rows_gemm; everything else rocBLAS."""
         n, k = w.shape
         M = x.shape[0]
         if x.is_cuda and wf8 is not None:
@@ -242,9 +242,7 @@ class LlamaModel:
             # bf16 skinny wins only the small decode shapes (qkv/wo);
             # rocBLAS is at the bandwidth floor for the big-N ones
             return D.skinny_linear(x, wf, n, k)
-        if D.rows_linear_ok(x, w):
-            return D.rows_linear(x, w)
-        return F.linear(x, w)
+        return D.linear(x, w)
 
     def _tp_all_reduce(self, t: torch.Tensor) -> torch.Tensor:
         if self.tp_size > 1:
@@ -350,9 +348,13 @@ class LlamaModel:
     def _ffn(self, L: dict, h: torch.Tensor) -> torch.Tensor:
         """Dense SwiGLU FFN (TP row/col-parallel). Mixtral overrides with
         the routed MoE (models/mixtral.py)."""
-        gu = self._linear(h, L["wgu"], L.get("wgu_f"),
-                          L.get("wgu_f8"))
-        act = D.swiglu(gu[:, :self.ffn_local], gu[:, self.ffn_local:])
+        import os as _os
+        if h.shape[0] > 32 and _os.environ.get("QSA_FP8_BATCH") != "1" and \
+                D.glu_linear_ok(h, L["wgu"]):
+            act = D.glu_linear(h, L["wgu"])
+        else:
+            gu = self._linear(h, L["wgu"], L.get("wgu_f"), L.get("wgu_f8"))
+            act = D.swiglu(gu[:, :self.ffn_local], gu[:, self.ffn_local:])
         return self._tp_all_reduce(
             self._linear(act, L["wdown"], L.get("wdown_f"),
                          L.get("wdown_f8")))
@@ -484,7 +486,8 @@ class LlamaModel:
             else:
                 h = D.rmsnorm_residual(mlp_out, res, L["attn_norm"],
                                        c.norm_eps)
-            qkv = F.linear(h, L["wqkv"], L.get("bqkv"))
+            qkv = F.linear(h, L["wqkv"], L["bqkv"]) if "bqkv" in L \
+                else D.linear(h, L["wqkv"])
             q, k, v = self._split_qkv(qkv, T_pad)
             if use_hip_prefill:
                 D.rope_kv_scatter(q[:T], k[:T], v[:T], kv.k[li], kv.v[li],
@@ -526,7 +529,7 @@ class LlamaModel:
                     .permute(0, 3, 1, 2, 4) \
                     .reshape(nb * nmax, self.n_q * c.d_head) \
                     .index_select(0, dst_idx)
-            o = self._tp_all_reduce(F.linear(attn, L["wo"]))
+            o = self._tp_all_reduce(D.linear(attn, L["wo"]))
             h = D.rmsnorm_residual(o, res, L["mlp_norm"], c.norm_eps)
             mlp_out = self._ffn(L, h)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)

@@ -198,15 +198,35 @@ def pack_weight_frag(w: torch.Tensor) -> torch.Tensor:
 
 
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether x[M,K] @ W^T is rows_linear's: a decode batch beyond the skinny
-    kernels on a long K, where nobody looks at the operation itself (the rules
-    are in ops/hip/lm_ops.cpp)."""
+    """Whether x[M,K] @ W^T is rows_linear's: a product short of the sizes that
+    a library's tiles need, where nobody looks at the operation itself (the
+    rules are in ops/hip/lm_ops.cpp)."""
     return x.is_cuda and type(x) is torch.Tensor and \
         lm_ext().rows_gemm_ok(x, w) and not torch.compiler.is_compiling()
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return lm_ext().rows_gemm(x, w)
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ W^T for a weight as it is stored."""
+    if rows_linear_ok(x, w):
+        return rows_linear(x, w)
+    return torch.nn.functional.linear(x, w)
+
+
+def glu_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the activation is glu_linear's to apply: W's rows are [gate; up]
+    and both fit its kernel (the rules are beside rows_linear's)."""
+    return x.is_cuda and type(x) is torch.Tensor and \
+        lm_ext().rows_glu_ok(x, w) and not torch.compiler.is_compiling()
+
+
+def glu_linear(x: torch.Tensor, w: torch.Tensor,
+               act: str = "silu") -> torch.Tensor:
+    """act(x @ W_gate^T) * (x @ W_up^T) of W = [gate; up], in one kernel."""
+    return lm_ext().rows_glu(x, w, act == "gelu")
 
 
 def skinny_linear(x: torch.Tensor, wf: torch.Tensor, n: int,

@@ -82,6 +82,17 @@ __device__ __forceinline__ float sigmoid_f(float z) {
   return 1.f / (1.f + expf(-z));
 }
 
+// silu, or the tanh form of gelu
+#define QSA_ACT_SILU 0
+#define QSA_ACT_GELU 1
+
+template <bool EXACT, int ACT>
+__device__ __forceinline__ float act_f(float z) {
+  const float a = ACT == QSA_ACT_SILU
+      ? z : 1.5957691216057308f * fmaf(0.044715f * z * z, z, z);
+  return z / (1.f + (EXACT ? expf(-a) : __expf(-a)));
+}
+
 // x = hi + lo with both parts bf16: 16 mantissa bits survive, so a product
 // of two such pairs on the bf16 matrix cores (hi*hi + hi*lo + lo*hi) stays
 // at f32-like accuracy.

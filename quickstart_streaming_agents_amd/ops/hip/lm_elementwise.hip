@@ -220,16 +220,6 @@ extern "C" void qsa_residual_norm_launch(
 // act: silu, or the tanh form of gelu, z / (1 + exp(-2 sqrt(2/pi)
 // (z + 0.044715 z^3))).
 // ---------------------------------------------------------------------------
-#define QSA_ACT_SILU 0
-#define QSA_ACT_GELU 1
-
-template <bool EXACT, int ACT>
-__device__ __forceinline__ float act_f(float z) {
-  const float a = ACT == QSA_ACT_SILU
-      ? z : 1.5957691216057308f * fmaf(0.044715f * z * z, z, z);
-  return z / (1.f + (EXACT ? expf(-a) : __expf(-a)));
-}
-
 template <typename T, int VEC, int ACT>
 __global__ void __launch_bounds__(256)
 qsa_glu(const T* __restrict__ gate, const T* __restrict__ up,

@@ -129,9 +129,9 @@ extern "C" void qsa_window_attn_prefill_launch(const bf16_t*, long long,
     const int*, bf16_t*, int, int, int, int, int, float, hipStream_t);
 extern "C" void qsa_skinny_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     int, int, long long, long long, hipStream_t);
-extern "C" int qsa_rows_gemm_shares(int, int);
+extern "C" int qsa_rows_gemm_plan(int, int, int, int, int, int*);
 extern "C" void qsa_rows_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
-    float*, int, int, int, long long, int, hipStream_t);
+    float*, int, int, int, long long, int, int, int, hipStream_t);
 
 // res [T, W] f32 updated in place; returns norm(res) * w (+ b), or res itself
 // in y's storage type when w is not given
@@ -926,43 +926,79 @@ static bool no_observer() {
          !at::autocast::is_autocast_enabled(at::kCUDA);
 }
 
-// Whether a @ w^T is rows_gemm's: 33 to 192 rows and a long K beside few
-// columns, where it beats the library (figures in rows_gemm.hip; of 27 shapes at
-// ten numbers of rows six are up to 5% behind it at some, the others ahead, up to
-// 3 times, and a call that is not captured saves some 10 us of the library's
-// host path).  Small weights leave little to split: up to 2560 x 8192, itself
-// behind by 8% at 33 to 48 rows and 13% at 192, it takes K of four times the
-// columns.  The whole rule here: in Python the last part alone took 2 us of a
-// call, 2% of a step of 40 tokens.
-bool rows_gemm_ok(const Tensor& a, const Tensor& w) {
+// What rows_gemm.hip takes: bf16 with whole stages of K and column tiles, aligned
+// rows, and offsets within a block's rows (and from a gate's weights to its
+// up's) that fit 32 bits.
+static bool rows_gemm_fits(const Tensor& a, const Tensor& w, bool glu) {
   if (a.dim() != 2 || w.dim() != 2) return false;
-  const int64_t M = a.size(0), N = w.size(0), K = w.size(1);
-  return M > 32 && M <= 192 && N * K >= 1 << 24 &&
-         K >= (N * K <= 5 << 22 ? 4 : 3) * N && N % 16 == 0 && K % 64 == 0 &&
-         a.size(1) == K && a.is_cuda() && a.device() == w.device() &&
-         a.scalar_type() == at::kBFloat16 &&
-         w.scalar_type() == at::kBFloat16 && no_observer() && unobserved(a) &&
-         unobserved(w) && w.is_contiguous() && a.stride(1) == 1 &&
-         a.stride(0) % 8 == 0 && a.stride(0) < (1 << 24) && aligned(a, 16) &&
+  const int64_t M = a.size(0), N = w.size(0), K = w.size(1), ld = a.stride(0);
+  return M >= 1 && N >= 16 && K >= 64 && N % (glu ? 32 : 16) == 0 &&
+         K % 64 == 0 && a.size(1) == K && M < 1 << 24 && N < 1 << 24 &&
+         K < 1 << 24 && a.scalar_type() == at::kBFloat16 &&
+         w.scalar_type() == at::kBFloat16 && w.is_contiguous() &&
+         a.stride(1) == 1 && ld % 8 == 0 && ld >= 0 && ld < 1 << 24 &&
+         (std::min<int64_t>(M, 256) * ld + K) * 2 < (4ll << 30) &&
+         ((glu ? N / 2 : 0) + 257) * K * 2 < (4ll << 30) && aligned(a, 16) &&
          aligned(w, 16);
 }
 
-// a @ w^T on W as it is stored, K split over the chip
-Tensor rows_gemm(Tensor a, Tensor w) {
-  CHK_DEV(a); chk_rows(a, "a"); CHK_CONT(w); CHK_SAME(a, w);
-  TORCH_CHECK(a.scalar_type() == at::kBFloat16, "bf16");
+// Whether a @ w^T, with `glu` the gated activation of it, is rows_gemm's.  As
+// plain products of 26 pairs of N and K with M of 33 to 14000 it is 18 % faster
+// than the library's on average while M N is at most 9 million; beyond, the
+// library's 256 x 256 tiles fill the chip and reach 1.5 PFLOP/s, ours 1.3
+// (figures in rows_gemm.hip).  With K up to 768 they are not yet in their
+// stride: 8800 x 4096 x 512 takes 46 us for 75.  With the activation inside, a
+// pass over M N is saved, which is more than the library is ahead by up to K =
+// 3072 (13800 x 16384 x 2048: 735 us for 820) and at 4096 while the tiles are few
+// (1024 x 28672: 212 us for 211, 8192: 1450 for 1440, 44800: 1.6 % behind).  And
+// a call that is not captured is spared 15 us of the library's host path.  The
+// whole rule is here: in Python the last part alone took 2 us a call.
+static bool rows_gemm_rule(const Tensor& a, const Tensor& w, bool glu) {
+  if (a.dim() != 2 || w.dim() != 2) return false;
+  const int64_t MN = a.size(0) * w.size(0), K = w.size(1);
+  return (MN <= (glu ? 48000000 : 9000000) || K <= (glu ? 3072 : 768)) && a.is_cuda() &&
+         a.device() == w.device() && no_observer() && unobserved(a) &&
+         unobserved(w) && rows_gemm_fits(a, w, glu);
+}
+
+bool rows_gemm_ok(const Tensor& a, const Tensor& w) {
+  return rows_gemm_rule(a, w, false);
+}
+
+bool rows_glu_ok(const Tensor& a, const Tensor& w) {
+  return rows_gemm_rule(a, w, true);
+}
+
+static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act) {
+  CHK_DEV(a); CHK_SAME(a, w);
+  TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
+              "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
   const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
-  TORCH_CHECK(M >= 1 && M <= 192 && a.size(1) == K, "M in [1, 192], K");
-  TORCH_CHECK(N >= 16 && N % 16 == 0 && K >= 64 && K % 64 == 0,
-              "N % 16, K % 64");
-  TORCH_CHECK(a.stride(0) % 8 == 0 && a.stride(0) < (1 << 24) &&
-                  aligned(a, 16) && aligned(w, 16), "alignment");
-  const int S = qsa_rows_gemm_shares(N, K);
-  auto out = torch::empty({M, N}, a.options());
-  auto part = torch::empty({S, M, N}, a.options().dtype(at::kFloat));
-  qsa_rows_gemm_launch(u16(a), u16(w), u16m(out), part.data_ptr<float>(), M,
-                       N, K, a.stride(0), S, cur_stream());
+  int S;
+  const int tile = qsa_rows_gemm_plan(M, N, K, act, 0, &S);
+  auto out = torch::empty({M, act ? N / 2 : N}, a.options());
+  Tensor part;
+  if (S > 1) part = torch::empty({S, M, N}, a.options().dtype(at::kFloat));
+  qsa_rows_gemm_launch(u16(a), u16(w), u16m(out),
+                       S > 1 ? part.data_ptr<float>() : nullptr, M, N, K,
+                       a.stride(0), tile, S, act, cur_stream());
   return out;
+}
+
+// (tile, shares of K) that the rule in rows_gemm.hip takes
+std::tuple<int, int> rows_gemm_plan(int64_t M, int64_t N, int64_t K,
+                                    bool glu) {
+  int S;
+  const int tile = qsa_rows_gemm_plan((int)M, (int)N, (int)K, glu, 0, &S);
+  return {tile, S};
+}
+
+// a @ w^T on W as it is stored
+Tensor rows_gemm(Tensor a, Tensor w) { return rows_gemm_run(a, w, 0); }
+
+// act of the first half of a @ w^T's columns times the second
+Tensor rows_glu(Tensor a, Tensor w, bool gelu) {
+  return rows_gemm_run(a, w, gelu ? 2 : 1);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -997,6 +1033,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "windowed flash attention with sink and gate (MFMA)");
   m.def("window_attn_ok", &window_attn_ok, "size support");
   m.def("skinny_gemm", &skinny_gemm, "packed-weight decode GEMM (M <= 32)");
-  m.def("rows_gemm", &rows_gemm, "long-K decode GEMM (M <= 192)");
+  m.def("rows_gemm", &rows_gemm, "GEMM of decode batches and short prompts");
   m.def("rows_gemm_ok", &rows_gemm_ok, "whether a product is rows_gemm's");
+  m.def("rows_gemm_plan", &rows_gemm_plan, "tile and shares of a product");
+  m.def("rows_glu", &rows_glu, "the same with the gated activation inside");
+  m.def("rows_glu_ok", &rows_glu_ok, "whether a gated product is rows_glu's");
 }

@@ -1,139 +1,270 @@
-// Decode-batch GEMM on weights as they are stored, for a projection from many
-// columns to few: C[M,N] = A[M,K] @ W[N,K]^T, 32 < M <= 192 rows, K >= 3 N,
-// bf16 with f32 sums.
+// GEMM on weights as they are stored, for decode batches, short prompts and all
+// else that leaves a library's large tiles idle: C[M,N] = A[M,K] @ W[N,K]^T, bf16
+// with f32 sums, or act(gate) * up of it with W = [gate; up].
 //
-// Bound by the read of W; what stands in the way is that N alone makes too few
-// blocks, and that the rows, read again by every block, cost as much cache
-// bandwidth as W once there are many of them.  So K is split until every CU has
-// a block, each block keeps all rows of its share (A passes through LDS once
-// for its four waves), and W goes from memory to the matrix cores' operands
-// directly, 32 columns a wave, 128 bytes of each at a time.  The shares' sums
-// meet in f32 in a second kernel.
-// us, library GEMM -> here (sums included, weights from memory), at 40 / 64 /
-// 128 / 192 rows:
-//   2048 x  8192  14.1 / 22.6 / 21.1 / 26.5 -> 14.7 / 15.4 / 21.0 / 25.9
-//   2560 x  8192  16.3 / 23.1 / 41.8 / 26.9 -> 17.5 / 18.7 / 25.1 / 30.9
-//   1536 x 11264  20.8 / 31.0 / 27.2 / 38.2 -> 16.9 / 18.1 / 24.1 / 30.1
-//   2560 x 10240  20.9 / 30.5 / 55.8 / 36.7 -> 19.5 / 21.2 / 27.8 / 34.7
-//   4096 x 14336  36.7 / 41.2 / 76.2 / 64.3 -> 29.1 / 32.0 / 42.1 / 54.6
-//   4096 x 16384  38.8 / 42.5 / 82.4 / 115  -> 39.5 / 39.8 / 48.3 / 58.3
-//   5120 x 15360  49.7 / 53.9 / 82.8 / 112  -> 40.0 / 43.4 / 54.8 / 68.4
-//   8192 x 24576   113 /  130 /  181 /  210 ->  104 /  113 /  130 /  159
-// With N nearer to K the library's larger tiles win: 4096 x 4096 at 192 rows
-// 20.5 against 25.6, 16384 x 2048 27.2 against 36.
+// Up to some 200 rows it is bound by the read of W, then by the matrix cores.
+// Both operands go from memory straight into LDS (16 bytes a lane, whole lines),
+// two to five stages of K ahead, so the bytes under way do not cost registers;
+// the ring is as deep as the 160 KB of a CU allow.  A wave multiplies half a
+// stage while it reads the next half.  Tiles from 64 x 32 to 256 x 256 and
+// shares of K are chosen by what they should take (qsa_rows_gemm_plan); a tile's
+// LDS traffic per product falls with its sides, which is why the large ones are
+// the fast ones where the chip is full.  The activation
+// is that of the rounded products, so either way gives the same.
+// us, library -> here (sums of shares included, weights from memory):
+//   rows            33            64           128           192           768
+//   6144 x 4096  17.4 -> 15.6  17.9 -> 16.9  25.6 -> 21.0  34.1 -> 25.3  49 -> 47
+//   4096 x 4096  12.8 -> 11.3  13.9 -> 12.0  22.6 -> 15.1  32.3 -> 19.0  35 -> 36
+//   4096 x 14336 38.5 -> 26.2  39.8 -> 27.6  75.9 -> 33.3   103 -> 40   108 -> 95
+//   2048 x 8192  13.2 -> 10.5  20.9 -> 11.5  20.2 -> 15.1  25.4 -> 18.8  44 -> 37
+//   12576 x 2048 17.1 -> 14.6  16.5 -> 14.9  19.4 -> 18.6  26.1 -> 21.0  45 -> 48
+// with the activation (there a pass of its own):
+//   28672 x 4096 54.5 -> 44.7  53.9 -> 43.3  57.6 -> 51.0  67.7 -> 58.9 176 -> 176
+//   16384 x 2048 22.0 -> 15.0  20.9 -> 15.5  24.1 -> 19.1  30.9 -> 23.2  57 -> 53
+// and 820 -> 735 at 13,800 rows.  What limits 256 x 256 at 1.3 PFLOP/s (28672 x
+// 4096 x 8192, the library 1.5): matrix cores 72 % busy at 1.6 GHz (82 %), LDS as
+// many cycles as they; four waves of 128 x 128, stages of 32, products of 32 x 32
+// and other orders of reads and loads were within 3 % or slower.
 #include "lm_common.h"
 
+using rsrc_t = __amdgpu_buffer_rsrc_t;
+
 struct RowsArgs {
-  const bf16_t* A;
-  const bf16_t* W;
-  float* part;                         // [S][M][N]
-  int M, N, K;
+  const bf16_t* A;                     // [M, K], row stride lda
+  const bf16_t* W;                     // [N, K]
+  bf16_t* C;                           // [M, N], or [M, N/2] with an activation
+  float* part;                         // [S][M][N] where S > 1
+  int M, N, K, S;
+  int MB, NB;                          // blocks along rows and columns
   unsigned int lda;                    // elements
 };
 
-// 64 of K a step; two steps of A and W are under way in registers
-template <int MT>                      // row tiles of 16
-__global__ void __launch_bounds__(256)
+enum { ACT_NONE = 0, ACT_SILU = 1, ACT_GELU = 2 };
+
+__device__ __forceinline__ float as_bf16(float v) {
+  return bf16_to_f32(cvt_bf16(v));
+}
+
+// all of a wave's LDS reads are in, and at most N of its loads under way
+template <int N> __device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "the counter's range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 7 << 4);
+}
+
+// A barrier that neither waits for loads nor lets memory accesses pass: what
+// the waves have read and received is settled by wait_loads before it.
+__device__ __forceinline__ void stage_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
+// BM x BN of C in a block of WM x WN waves, K in stages of 64 through a ring of
+// ST places in LDS; with ACT, W's rows are [gate; up] and a wave's column tiles
+// are alternately of either.
+template <int BM, int BN, int WM, int WN, int ST, int ACT>
+__global__ void __launch_bounds__(WM * WN * 64)
 qsa_rows_gemm(RowsArgs p) {
-  constexpr int CT = 2, D = 2;         // column tiles of a wave, steps ahead
-  constexpr int AF = MT * 2;           // fragments of A a step
-  constexpr int AL = (AF + 3) / 4;     // and of them per wave
-  __shared__ __attribute__((aligned(16))) bf16_t at[2][AF * 512];
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr int NW = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16;
+  constexpr int STAGE = (BM + BN) * 64;           // elements
+  constexpr int L = (BM + BN) / 8 / NW;           // loads of a wave and stage
+  constexpr int AL = BM / 8 / NW;                 // of them A's
+  constexpr int RD = MT + NT, MM = MT * NT;       // reads, MFMAs of half a stage
+  constexpr int OP = (ACT ? 8 : 16) * NT + 8;     // pitch of a wave's results
+  constexpr int OUT = NW * MT * 16 * OP;
+  static_assert(BM / 8 % NW == 0 && BN / 8 % NW == 0, "whole loads");
+  static_assert(!ACT || NT % 2 == 0, "pairs of column tiles");
+  __shared__ __attribute__((aligned(16)))
+      bf16_t lds[ST * STAGE > OUT ? ST * STAGE : OUT];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
-  const int n0 = (blockIdx.x * 4 + wave) * 16 * CT;
-  const int steps = p.K >> 6, S = gridDim.y;      // K % 64 == 0, S <= steps
-  const int s0 = (int)((long long)steps * blockIdx.y / S);
-  const int s1 = (int)((long long)steps * (blockIdx.y + 1) / S);
 
-  // rows and columns beyond the end shadow the last one and are not stored
-  unsigned int aoff[AL];
-#pragma unroll
-  for (int j = 0; j < AL; ++j) {
-    const int f = min(wave + j * 4, AF - 1);      // row tile * 2 + half
-    aoff[j] = (unsigned int)min((f >> 1) * 16 + col, p.M - 1) * p.lda +
-              (f & 1) * 32 + hi * 8;
-  }
-  const bf16_t* wrow[CT];
-#pragma unroll
-  for (int t = 0; t < CT; ++t)
-    wrow[t] = p.W + (long long)min(n0 + t * 16 + col, p.N - 1) * p.K + hi * 8;
+  // A die takes neighbouring work: one share of K, then groups of four block
+  // rows, whose weights it reads together.
+  const int per = gridDim.x >> 3, tiles = p.MB * p.NB;
+  const int at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (at >= tiles * p.S) return;                  // uniform over the block
+  const int share = at / tiles, t = at - share * tiles;
+  const int g = t / (4 * p.NB), gm = min(4, p.MB - 4 * g);
+  const int mb = 4 * g + (t - 4 * g * p.NB) % gm;
+  const int nb = (t - 4 * g * p.NB) / gm;
+  const int m0 = mb * BM, n0 = nb * BN;
+  const int all = p.K >> 6;
+  const int s0 = (int)((long long)all * share / p.S);
+  const int steps = (int)((long long)all * (share + 1) / p.S) - s0;
+  // Where a block starts in its share: rows of W lie a multiple of the memory
+  // channels' period apart, so blocks in step would meet in the same channels
+  // (28672 x 4096 at 64 rows: 56 us in step, 46 in turn).  Many block rows share
+  // the columns through L2 instead.
+  const int turn = p.MB > 2 ? 0 : (int)((long long)nb * steps / p.NB);
 
-  u32x4_v ar[D][AL];
-  bf16x8_v wr[D][CT][2];
-  auto load_a = [&](int d, int s) {
-    const bf16_t* a = p.A + (long long)min(s, s1 - 1) * 64;
+  const rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.A + (long long)m0 * p.lda + s0 * 64), 0, 0xffffffffu,
+      0x00027000);
+  const rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.W + (long long)(ACT ? n0 / 2 : n0) * p.K + s0 * 64), 0,
+      0xffffffffu, 0x00027000);
+  // A load brings 8 rows of 128 bytes, a row's eight segments exchanged by its
+  // number so that the reads below spread over the banks.  Rows and columns
+  // beyond the end shadow the last one and are not stored.
+  unsigned int off[L];
 #pragma unroll
-    for (int j = 0; j < AL; ++j)
-      ar[d][j] = *reinterpret_cast<const u32x4_v*>(a + aoff[j]);
-  };
-  auto load_w = [&](int d, int s) {
-    const int k = min(s, s1 - 1) * 64;
-#pragma unroll
-    for (int t = 0; t < CT; ++t)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        wr[d][t][h] = *reinterpret_cast<const bf16x8_v*>(wrow[t] + k + h * 32);
-  };
-  auto store_a = [&](int d, int buf) {
-#pragma unroll
-    for (int j = 0; j < AL; ++j)
-      if (AF % 4 == 0 || wave + j * 4 < AF)
-        *reinterpret_cast<u32x4_v*>(
-            &at[buf][(wave + j * 4) * 512 + lane * 8]) = ar[d][j];
-  };
-  f32x4_v acc[MT][CT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int t = 0; t < CT; ++t) acc[m][t] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
-
-  // step s sits in place (s - s0) % D of the registers and half (s - s0) & 1
-  // of LDS, which the step before last has left
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    load_a(d, s0 + d);
-    load_w(d, s0 + d);
-  }
-  store_a(0, 0);
-  load_a(0, s0 + D);
-  lds_barrier();
-  for (int sb = s0; sb < s1; sb += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int s = sb + d;
-      store_a((d + 1) % D, (d + 1) & 1);
-      load_a((d + 1) % D, s + 1 + D);
-      // uniform; the loads take no branch, or their waits would meet there
-      if (s < s1)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            const bf16x8_v a = *reinterpret_cast<const bf16x8_v*>(
-                &at[d & 1][(m * 2 + h) * 512 + lane * 8]);
-#pragma unroll
-            for (int t = 0; t < CT; ++t)
-              acc[m][t] = mfma_bf16(wr[d][t][h], a, acc[m][t]);
-          }
-      load_w(d, s + D);
-      lds_barrier();
+  for (int j = 0; j < L; ++j) {
+    const int r = (wave + j * NW) * 8 + (lane >> 3);
+    const int seg = (lane & 7) ^ (r & 7);
+    if (j < AL) {
+      off[j] = ((unsigned)min(r, p.M - 1 - m0) * p.lda + seg * 8) * 2;
+    } else {
+      const int q = r - BM;
+      const int n = ACT ? min((q >> 5) * 16 + (q & 15),
+                              (p.N - n0) / 2 - 1) + (q >> 4 & 1) * (p.N >> 1)
+                        : min(q, p.N - 1 - n0);
+      off[j] = ((unsigned)n * (unsigned)p.K + seg * 8) * 2;
     }
   }
+  auto load = [&](int s, int place) {
+    const int k = s + turn < steps ? s + turn : s + turn - steps;
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int row = m * 16 + col;
-    if (row >= p.M) continue;
+    for (int j = 0; j < L; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          j < AL ? ra : rw,
+          (__attribute__((address_space(3))) void*)(
+              lds + place * STAGE + (wave + j * NW) * 512),
+          16, off[j], k * 128, 0, 0);
+  };
+  const int wm = wave / WN * MT, wn = wave % WN * NT;
+  bf16x8_v fa[2][MT], fb[2][NT];
+  auto read = [&](int h, int place) {
+    const bf16_t* b = lds + place * STAGE + col * 64 +
+                      ((h * 4 + hi) ^ (col & 7)) * 8;
 #pragma unroll
-    for (int t = 0; t < CT; ++t) {
-      const int c = n0 + t * 16 + hi * 4;         // N % 16 == 0
-      if (c < p.N)
-        *reinterpret_cast<f32x4_v*>(
-            p.part + ((long long)blockIdx.y * p.M + row) * p.N + c) =
-            acc[m][t];
+    for (int j = 0; j < NT; ++j)
+      fb[h][j] = *reinterpret_cast<const bf16x8_v*>(b + BM * 64 +
+                                                    (wn + j) * 1024);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      fa[h][i] = *reinterpret_cast<const bf16x8_v*>(b + (wm + i) * 1024);
+  };
+  f32x4_v acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int h) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[i][j] = mfma_bf16(fb[h][j], fa[h][i], acc[i][j]);
+  };
+
+  // Half a stage is multiplied while the next half is read.  Once both of a
+  // stage are in registers its place takes the stage ST further on.
+#pragma unroll
+  for (int s = 0; s < ST; ++s)
+    if (s < steps) load(s, s);
+  if (steps >= ST) wait_loads<(ST - 1) * L>();
+  else wait_loads<0>();
+  stage_barrier();
+  read(0, 0);
+  int place = 0, s = 0;
+  for (; s < steps - ST; ++s) {
+    read(1, place);
+    multiply(0);
+#pragma unroll
+    for (int i = 0; i < RD; ++i) {     // a read every few MFMAs
+      __builtin_amdgcn_sched_group_barrier(0x8, MM / RD ? MM / RD : 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
+    wait_loads<(ST - 2) * L>();        // stage s + 1 is there
+    stage_barrier();
+    load(s + ST, place);
+    place = place + 1 == ST ? 0 : place + 1;
+    read(0, place);
+    multiply(1);
+    constexpr int PM = MM / (RD + L) ? MM / (RD + L) : 1;
+#pragma unroll
+    for (int i = 0; i < (RD > L ? RD : L); ++i) {
+      if (i < L) {
+        __builtin_amdgcn_sched_group_barrier(0x8, PM, 0);
+        __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
+      }
+      if (i < RD) {
+        __builtin_amdgcn_sched_group_barrier(0x8, PM, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
+  for (; s < steps; ++s) {             // no more loads: those under way
+    read(1, place);
+    multiply(0);
+    const int ahead = steps - 2 - s;   // stages that may still be under way
+    if (ahead >= ST - 2) wait_loads<(ST - 2) * L>();
+    else if (ST > 3 && ahead == ST - 3) wait_loads<(ST > 3 ? ST - 3 : 0) * L>();
+    else if (ST > 4 && ahead == ST - 4) wait_loads<(ST > 4 ? ST - 4 : 0) * L>();
+    else if (ST > 5 && ahead == ST - 5) wait_loads<(ST > 5 ? ST - 5 : 0) * L>();
+    else wait_loads<0>();
+    stage_barrier();
+    place = place + 1 == ST ? 0 : place + 1;
+    read(0, place);                    // after the last stage: not used
+    multiply(1);
+  }
+
+  // a lane has columns hi * 4 .. + 3 of row `col` of each tile
+  if (p.S > 1) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int row = m0 + (wm + i) * 16 + col;
+      if (row >= p.M) continue;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int c = n0 + (wn + j) * 16 + hi * 4;          // N % 16 == 0
+        if (c < p.N)
+          *reinterpret_cast<f32x4_v*>(
+              p.part + ((long long)share * p.M + row) * p.N + c) = acc[i][j];
+      }
+    }
+    return;
+  }
+  // results through LDS to whole lines; the last reads above are in a wave's
+  // own registers, so its barrier suffices
+  wait_loads<0>();
+  stage_barrier();
+  bf16_t* o = lds + wave * (MT * 16 * OP);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; j += ACT ? 2 : 1) {
+      f32x4_v v = acc[i][j];
+      if constexpr (ACT != ACT_NONE)   // of the products as they are stored
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[r] = act_f<false, ACT - 1>(as_bf16(v[r])) *
+                 as_bf16(acc[i][j + 1][r]);
+      *reinterpret_cast<uint2*>(o + (i * 16 + col) * OP +
+                                (ACT ? j / 2 : j) * 16 + hi * 4) =
+          make_uint2(cvt_bf16x2(v[0], v[1]), cvt_bf16x2(v[2], v[3]));
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+  constexpr int G = ACT ? NT : 2 * NT;            // 16 B groups of a row
+  const int N = ACT ? p.N >> 1 : p.N;
+  const int c0 = (ACT ? n0 / 2 : n0) + wave % WN * G * 8;
+#pragma unroll
+  for (int x = 0; x < MT * G / 4; ++x) {
+    const int i = x * 64 + lane, row = i / G, c = i % G * 8;
+    const int m = m0 + wm * 16 + row;
+    if (m < p.M && c0 + c < N)                    // N % 8 == 0
+      *reinterpret_cast<u32x4_v*>(p.C + (long long)m * N + c0 + c) =
+          *reinterpret_cast<const u32x4_v*>(o + row * OP + c);
+  }
+#endif
 }
 
 __global__ void __launch_bounds__(256)
@@ -149,30 +280,92 @@ qsa_rows_sum(const float* __restrict__ part, bf16_t* __restrict__ C,
       make_uint2(cvt_bf16x2(v[0], v[1]), cvt_bf16x2(v[2], v[3]));
 }
 
-// Shares of K: a block for each of the 256 CUs and none left over, which would
-// have some CUs do the work of two (2560 x 10240 with 13 shares, 260 blocks:
-// 28.8 us at 40 rows, 56.8 at 192; with 12: 19.5 and 34.7).
-extern "C" int qsa_rows_gemm_shares(int N, int K) {
-  const int blocks = (N + 127) / 128, steps = K >> 6;
-  const int want = blocks < 256 ? 256 / blocks : 1;
-  return want < steps ? want : steps;
+template <int BM, int BN, int WM, int WN, int ST>
+static void rows_go(RowsArgs p, int act, hipStream_t st) {
+  p.MB = (p.M + BM - 1) / BM;
+  p.NB = (p.N + BN - 1) / BN;
+  const dim3 grid((unsigned)((long long)p.MB * p.NB * p.S + 7) / 8 * 8);
+#define QSA_RG(ACT) \
+  hipLaunchKernelGGL((qsa_rows_gemm<BM, BN, WM, WN, ST, ACT>), grid, \
+                     dim3(WM * WN * 64), 0, st, p)
+  if constexpr (BN / WN / 16 % 2 == 0) {
+    if (act == ACT_SILU) { QSA_RG(ACT_SILU); return; }
+    if (act == ACT_GELU) { QSA_RG(ACT_GELU); return; }
+  }
+  QSA_RG(ACT_NONE);
+#undef QSA_RG
 }
 
+// BM, BN, waves, places of the ring; a block's own time and that of a stage, us
+#define QSA_TILES(X) \
+  X(64, 32, 2, 2, 6, 0.67f, 0.141f)   X(64, 64, 2, 2, 4, 0.71f, 0.208f) \
+  X(64, 128, 2, 4, 6, 1.86f, 0.353f)  X(128, 64, 4, 2, 6, 1.92f, 0.334f) \
+  X(128, 128, 2, 4, 4, 2.38f, 0.497f) X(192, 64, 4, 2, 4, 1.94f, 0.431f) \
+  X(192, 128, 4, 2, 4, 2.98f, 0.644f) X(256, 128, 4, 2, 3, 3.41f, 0.822f) \
+  X(128, 256, 2, 4, 3, 3.32f, 0.843f) X(192, 192, 2, 4, 3, 4.03f, 0.800f) \
+  X(256, 192, 4, 2, 2, 3.57f, 1.189f) X(192, 256, 2, 4, 2, 3.19f, 1.227f) \
+  X(256, 256, 2, 4, 2, 4.06f, 1.482f)
+
+struct RowsTile { int bm, bn, wn; float own, stage; };
+static const RowsTile rows_tiles[] = {
+#define X(BM, BN, WM, WN, ST, OWN, STAGE) {BM, BN, WN, OWN, STAGE},
+    QSA_TILES(X)
+#undef X
+};
+
+// The tile and the shares of K that should be over first.  Blocks take turns on
+// the 256 CUs, a turn as long as its stages or the whole product's way from
+// memory, whichever binds; shares cost the writing and adding of their sums.
+// The figures above and here are fitted to 382 shapes at up to 20 tiles and
+// shares each (M 33 to 20000, N 128 to 32000, K 128 to 14336; off by 9 % each,
+// and the choice by 1 % from the best of them).  Two blocks of the smallest
+// tiles share a CU, so alone on it they take longer.  `cheap`: the reader of the
+// product adds the shares.
+extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
+                                  int* shares) {
+  const int all = K >> 6;
+  const float mem = 2e-6f / 5.14f * ((float)N * K + (float)M * K +
+                                     (float)M * N);
+  const float sum = (cheap ? 0.5f : 3.25f), each = 1.28e-6f * (float)M * N;
+  float best = 1e30f;
+  int tile = 0;
+  *shares = 1;
+  for (int i = 0; i < (int)(sizeof(rows_tiles) / sizeof(*rows_tiles)); ++i) {
+    const RowsTile& t = rows_tiles[i];
+    if (act && t.bn / t.wn / 16 % 2) continue;    // no pairs of column tiles
+    const long long blocks =
+        (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const int fill = blocks < 256 ? (int)(256 / blocks) : 1;
+    for (int S = act || all < 8 ? 1 : fill; S >= 1; S = S > 1 ? S / 2 : 0) {
+      if (S > all / 4 && S > 1) continue;
+      const long long turns = (blocks * S + 255) / 256;
+      float stage = t.stage;
+      if (turns == 1 && t.bn * t.bm <= 4096) stage *= i ? 1.48f : 1.32f;
+      const float run = (float)turns * (t.own + stage * ((all + S - 1) / S));
+      const float r2 = run * run, m2 = mem * mem;
+      const float us = sqrtf(sqrtf(r2 * r2 + m2 * m2)) +
+                       (S > 1 ? sum + each * S : 0.f);
+      if (us < best) { best = us; tile = i; *shares = S; }
+    }
+  }
+  return tile;
+}
+
+// act: 0, or 1 silu / 2 gelu of the first half of W's rows times the second (one
+// share only).  With part and S > 1 and no C the shares are left to the caller.
 extern "C" void qsa_rows_gemm_launch(const bf16_t* A, const bf16_t* W,
                                      bf16_t* C, float* part, int M, int N,
-                                     int K, long long lda, int S,
-                                     hipStream_t st) {
-  const RowsArgs p{A, W, part, M, N, K, (unsigned int)lda};
-  const dim3 grid((N + 127) / 128, S);
-#define QSA_RG(MT) \
-  hipLaunchKernelGGL((qsa_rows_gemm<MT>), grid, dim3(256), 0, st, p)
-  if (M <= 48) QSA_RG(3);
-  else if (M <= 64) QSA_RG(4);
-  else if (M <= 96) QSA_RG(6);
-  else if (M <= 128) QSA_RG(8);
-  else QSA_RG(12);
-#undef QSA_RG
-  const long long n = (long long)M * N;
-  hipLaunchKernelGGL(qsa_rows_sum, dim3((unsigned)((n / 4 + 255) / 256)),
-                     dim3(256), 0, st, part, C, n, S);
+                                     int K, long long lda, int tile, int S,
+                                     int act, hipStream_t st) {
+  const RowsArgs p{A, W, C, part, M, N, K, S, 0, 0, (unsigned int)lda};
+  int i = 0;
+#define X(BM, BN, WM, WN, ST, OWN, STAGE) \
+  if (tile == i++) rows_go<BM, BN, WM, WN, ST>(p, act, st);
+  QSA_TILES(X)
+#undef X
+  if (S > 1 && C) {
+    const long long n = (long long)M * N;
+    hipLaunchKernelGGL(qsa_rows_sum, dim3((unsigned)((n / 4 + 255) / 256)),
+                       dim3(256), 0, st, part, C, n, S);
+  }
 }

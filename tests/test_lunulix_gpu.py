@@ -577,6 +577,52 @@ def test_rows_gemm_uneven_shares(M, N, K):
     test_rows_gemm(M, N, K)
 
 
+# sizes that the rule gives to every tile, with ends inside tiles and shares
+ROWS_SIZES = [(65, 32, 128), (33, 10768, 128), (40, 2048, 1024),
+              (64, 28688, 512), (257, 6160, 1088), (100, 4112, 4096),
+              (330, 10096, 128), (1000, 3104, 1088), (130, 2032, 8256),
+              (191, 4112, 4032), (330, 12304, 192), (700, 9696, 832),
+              (300, 16416, 576), (700, 8256, 64), (2100, 4112, 576),
+              (385, 16400, 704), (1500, 6176, 1024), (1000, 8880, 576),
+              (1700, 8208, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", ROWS_SIZES)
+def test_rows_gemm_tiles(M, N, K):
+    test_rows_gemm(M, N, K)
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("M,N,K", ROWS_SIZES)
+def test_rows_glu(M, N, K, act):
+    """Gate and up are rounded to bf16 after the product's f32 error, e in all,
+    and both activations have a slope of at most 1.13; __expf and the division
+    are good to some 2^-20, the result is rounded to bf16."""
+    N = N // 32 * 32
+    g = gen(M + N)
+    x = rnd(g, M, K + 24, dtype=BF)[:, 8:K + 8].to(DEV)
+    w = rnd(g, N, K, dtype=BF, scale=K ** -0.5).to(DEV)
+    got = D.glu_linear(x, w, act).double()
+    a, b = x.double(), w.double()
+    e = K * 2.0 ** -24 * (a.abs() @ b.abs().T) + 2.0 ** -20 \
+        + 2.0 ** -8 * (a @ b.T).abs()
+    (p, q), (ep, eq) = (a @ b.T).chunk(2, 1), e.chunk(2, 1)
+    f = torch.nn.functional.silu(p) if act == "silu" else \
+        torch.nn.functional.gelu(p, approximate="tanh")
+    bound = (2.0 ** -8 + 2.0 ** -18) * (f * q).abs() + 1.13 * ep * q.abs() \
+        + (f.abs() + ep) * eq
+    assert ((got - f * q).abs() <= bound).all()
+
+
+def test_rows_gemm_sizes_reach_every_tile():
+    from quickstart_streaming_agents_amd.ops import lm_ext
+    plain = {lm_ext().rows_gemm_plan(*s, False)[0] for s in ROWS_SIZES}
+    assert plain == set(range(13))
+    gated = {lm_ext().rows_gemm_plan(m, n // 32 * 32, k, True)[0]
+             for m, n, k in ROWS_SIZES}
+    assert len(gated) >= 9
+
+
 def test_linear_of_rows_far_apart():
     """The kernel's offsets of a row have 32 bits; rows too far apart for them
     are the library's."""
