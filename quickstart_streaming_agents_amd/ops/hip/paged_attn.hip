@@ -12,20 +12,23 @@
 //     via A = P [16 heads x 32 pos] (packed bf16, redistributed with 8
 //     cross-lane shuffles) and B = V^T [32 pos x 16 dims].  Every KV byte is
 //     read exactly once.
-//   - K cache layout [page, kvh, D/8, 64, 8] (d-major x8) and V cache layout
-//     [page, kvh, D, 64] (transposed, pos minor): both fragment reads are
-//     coalesced 1 KiB wave loads.  The values of a page and the keys of the
-//     next one are under way while its scores are computed: 32 KiB a wave.
+//   - K cache layout [page, kvh, D/8, 64, 8] (d-major x8): a page's fragments
+//     are loads of four 256-byte pieces, and the next page's are under way while
+//     one is multiplied.  V cache layout [page, kvh, D, 64] (transposed, pos
+//     minor): its fragments would be pieces of 16 bytes, four times the address
+//     cycles, so a page goes into the wave's LDS in whole lines and is read from
+//     there (8 rows of 500-900 keys 16.7 -> 14.6 us).
 //   - The waves of a block merge in LDS.  One block per (row, kv head) stores
 //     the result; several leave (o, m, l) for qsa_attn_reduce.
 //   - FUSE is a decoding step's attention: q is rotated in registers, and the
 //     wave with the last page writes the rotated new key and the new value to
-//     the cache, so that no launch has to come before.  It reads the page
-//     beside that and fills their place in from LDS: waiting for its own
-//     stores cost a round trip to memory.
-// 192 rows of 400-1000 keys, 32/8 heads of 128: rotation 11, attention 172,
-// merge 7 us as separate kernels with a wave per share, 130 us here (4.2 TB/s); 16
-// rows of 1536-2048: 5 + 35 + 9, 29 + 5.
+//     the cache, so that no launch has to come before.  It puts both in their
+//     place among what it has read: waiting for its own stores cost a round
+//     trip to memory.
+// 192 rows of 400-1000 keys, 32/8 heads of 128: 131 -> 124 us, of which 105 are
+// the reads (5.6 TB/s) and the rest the 128 lines per row and head that a
+// transposed value touches, whatever the width of the stores or their cache
+// policy (64-byte pieces, whole lines and write-through were the same).
 //
 // The online softmax runs per head-column in registers: column max/sum
 // reduce with two shfl_xor hops (the 4 hi-lane groups of a column).
@@ -98,14 +101,22 @@ __device__ __forceinline__ void rotate_pair(bf16x8_a& a, bf16x8_a& b,
   }
 }
 
+// Up to 63 of a wave's loads under way, whatever it stored or read from LDS.
+template <int N> __device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 7 << 4 | 15 << 8);
+  asm volatile("" ::: "memory");
+}
+
 template <int D, int NW, bool FUSE>
 __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
 qsa_paged_attn_mfma(DecodeArgs p) {
   constexpr int KSTEPS = D / 32;      // QK^T k-steps (4 for D=128)
   constexpr int DTILES = D / 16;      // PV d-tiles (8 for D=128)
-  extern __shared__ float smem[];     // [NW][R][D] o, [NW][16] m, [NW][16] l
-  // the new key and value: one wave of a block has the last page
-  __shared__ __attribute__((aligned(16))) unsigned short fresh[FUSE ? 2 * D : 8];
+  constexpr int VT = D * QSA_PAGE;    // elements of a value page
+  constexpr int KL = 4 * KSTEPS;      // loads of a wave for a page's keys
+  // a wave's values, afterwards its part of the output [R][D]
+  __shared__ __attribute__((aligned(16))) unsigned short vlds[NW * VT];
+  __shared__ float ml[2 * NW * 16];   // and its maxima and sums
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (FUSE && (int)blockIdx.x >= p.blocks) {
@@ -119,6 +130,8 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   const int b = bk / p.KVH;
   const int kvh = bk % p.KVH;
   const int R = p.QH / p.KVH;
+  const int first = split * NW + wave, step = NW * p.NS;
+  const int* btab = p.block_table + (long long)b * p.max_pages;
   const int seqlen = p.seq_lens[b];
   const int npages = (seqlen + QSA_PAGE - 1) / QSA_PAGE;
   const int col = lane & 15;          // head col (scores) / dim col (PV)
@@ -130,7 +143,6 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   for (int dt = 0; dt < DTILES; ++dt)
     o_acc[dt] = (f32x4_a){0.f, 0.f, 0.f, 0.f};
 
-  const int first = split * NW + wave, step = NW * p.NS;
   if (first < npages) {               // uniform over the wave
     // ---- Q B-fragments: lane holds Q[head=col][k = ks*32 + hi*8 + e] ----
     const int qh_l = kvh * R + min(col, R - 1);   // clamp: pad heads compute
@@ -140,7 +152,22 @@ qsa_paged_attn_mfma(DecodeArgs p) {
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
       qf[ks] = *reinterpret_cast<const bf16x8_a*>(qrow + ks * 32 + hi * 8);
-    const int* btab = p.block_table + (long long)b * p.max_pages;
+    // the new key, in the same order: every lane's column is a copy
+    bf16x8_a kn[FUSE ? KSTEPS : 1];
+    float cs[FUSE ? KSTEPS / 2 : 1][8], sn[FUSE ? KSTEPS / 2 : 1][8];
+    if constexpr (FUSE) {
+      const unsigned short* krow =
+          p.k + (long long)b * p.kvstride + (long long)kvh * D;
+      const long long at = (long long)(seqlen - 1) * (D / 2) + hi * 8;
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks)
+        kn[ks] = *reinterpret_cast<const bf16x8_a*>(krow + ks * 32 + hi * 8);
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS / 2; ++ks) {
+        ldv<float, 8>(p.cos_t + at + ks * 32, cs[ks]);
+        ldv<float, 8>(p.sin_t + at + ks * 32, sn[ks]);
+      }
+    }
     auto load_k = [&](int page, bf16x8_a (&kf)[4][KSTEPS]) {
       const unsigned short* kbase =
           p.kc + ((((long long)page * p.KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
@@ -151,77 +178,44 @@ qsa_paged_attn_mfma(DecodeArgs p) {
           kf[pt][ks] = *reinterpret_cast<const bf16x8_a*>(
               kbase + ((ks * 4 + hi) * QSA_PAGE + pt * 16 + col) * 8);
     };
+    // Values go straight to the wave's LDS, 8 rows of 128 bytes at a time, a
+    // row's segments exchanged by its number (the reads below then spread over
+    // the banks).
+    unsigned short* vl = vlds + wave * VT;
+    auto load_v = [&](int page) {
+      const unsigned short* vbase =
+          p.vc + ((long long)page * p.KVH + kvh) * VT + (lane >> 3) * QSA_PAGE +
+          ((lane & 7) ^ (lane >> 3)) * 8;
+#pragma unroll
+      for (int i = 0; i < D / 8; ++i)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(vbase + i * 512),
+            (__attribute__((address_space(3))) void*)(vl + i * 512), 16, 0, 0);
+    };
     bf16x8_a kf[4][KSTEPS];
     int page = btab[first];
-    load_k(page, kf);                 // under way before anything else
+    load_k(page, kf);
+    load_v(page);
     if constexpr (FUSE) {
-      const long long at = (long long)(seqlen - 1) * (D / 2) + hi * 8;
 #pragma unroll
       for (int ks = 0; ks < KSTEPS / 2; ++ks) {
-        float c[8], s[8];
-        ldv<float, 8>(p.cos_t + at + ks * 32, c);
-        ldv<float, 8>(p.sin_t + at + ks * 32, s);
-        rotate_pair(qf[ks], qf[ks + KSTEPS / 2], c, s);
-      }
-      if ((npages - 1 - first) % step == 0) {     // the last page is this wave's
-        const int pin = (seqlen - 1) % QSA_PAGE;  // the new token's slot
-        const long long tile =
-            ((long long)btab[npages - 1] * p.KVH + kvh) * D * QSA_PAGE;
-        const long long row = (long long)b * p.kvstride + (long long)kvh * D;
-        const int d = lane * 8;
-        if (d < D / 2) {              // lane: keys d.. and d + D/2..
-          bf16x8_a x = *reinterpret_cast<const bf16x8_a*>(p.k + row + d);
-          bf16x8_a y =
-              *reinterpret_cast<const bf16x8_a*>(p.k + row + d + D / 2);
-          const long long t = (long long)(seqlen - 1) * (D / 2) + d;
-          float c[8], s[8];
-          ldv<float, 8>(p.cos_t + t, c);
-          ldv<float, 8>(p.sin_t + t, s);
-          rotate_pair(x, y, c, s);
-          unsigned short* kp = p.kw + tile + (lane * QSA_PAGE + pin) * 8;
-          *reinterpret_cast<bf16x8_a*>(kp) = x;
-          *reinterpret_cast<bf16x8_a*>(kp + D / 2 * QSA_PAGE) = y;
-          *reinterpret_cast<bf16x8_a*>(fresh + d) = x;
-          *reinterpret_cast<bf16x8_a*>(fresh + d + D / 2) = y;
-        }
-#pragma unroll
-        for (int i = 0; i < D; i += 64) {
-          const unsigned short x = p.v[row + i + lane];
-          p.vw[tile + (long long)(i + lane) * QSA_PAGE + pin] = x;
-          fresh[D + i + lane] = x;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        rotate_pair(qf[ks], qf[ks + KSTEPS / 2], cs[ks], sn[ks]);
+        rotate_pair(kn[ks], kn[ks + KSTEPS / 2], cs[ks], sn[ks]);
       }
     }
 
-    // patch: the row's last page, which came from memory with or without the
-    // new token, gets its place filled in from LDS
+    // patch: the row's last page, where the new token has its place
     auto walk = [&](int pi, auto patch) {
-      const bool more = pi + step < npages;
+      const bool more = !patch.value && pi + step < npages;
       const int next = more ? btab[pi + step] : 0;
-      const long long head = (long long)page * p.KVH + kvh;
-      const unsigned short* vbase = p.vc + head * D * QSA_PAGE;
       const int nvalid = min(seqlen - pi * QSA_PAGE, QSA_PAGE);
-      bf16x8_a vf[2][DTILES];
-      // B-frag: lane holds V^T[pos = half*32 + hi*8 + e][d = dt*16+col]
-      auto load_v = [&](int half) {
-#pragma unroll
-        for (int dt = 0; dt < DTILES; ++dt)
-          vf[half][dt] = *reinterpret_cast<const bf16x8_a*>(
-              vbase + (dt * 16 + col) * QSA_PAGE + half * 32 + hi * 8);
-      };
-      load_v(0);
+      const int pin = nvalid - 1;
       if constexpr (patch.value) {
 #pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-          const bf16x8_a x = *reinterpret_cast<const bf16x8_a*>(
-              fresh + ks * 32 + hi * 8);
+        for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
           for (int pt = 0; pt < 4; ++pt)
-            if (pt * 16 + col == nvalid - 1) kf[pt][ks] = x;
-        }
+            if (pt * 16 + col == pin) kf[pt][ks] = kn[ks];
       }
       // ---- scores: 4 pos-tiles x KSTEPS MFMAs ---------------------------
       // A-frag: lane holds K[pos = pt*16 + col][k = ks*32 + hi*8 + e]
@@ -235,7 +229,6 @@ qsa_paged_attn_mfma(DecodeArgs p) {
                                                         acc, 0, 0, 0);
         sc[pt] = acc;
       }
-      load_v(1);
       if (more) load_k(next, kf);
       // scale + mask invalid positions; C layout: row pos = hi*4 + r,
       // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
@@ -284,22 +277,22 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       psum += __shfl_xor(psum, 32, QSA_WAVE);
       lsum = lsum * alpha + psum;
 
+      // the values are there; the next page's keys, behind them, need not be
+      if (more) wait_vm<KL>();
+      else wait_vm<0>();
       if constexpr (patch.value) {
+        const unsigned short* vrow =
+            p.v + (long long)b * p.kvstride + (long long)kvh * D;
 #pragma unroll
-        for (int dt = 0; dt < DTILES; ++dt) {
-          const unsigned int x = fresh[D + dt * 16 + col];
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            const int e = nvalid - 1 - half * 32 - hi * 8;
-            u32x4_v u = __builtin_bit_cast(u32x4_v, vf[half][dt]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              if (e == 2 * i) u[i] = (u[i] & 0xffff0000u) | x;
-              if (e == 2 * i + 1) u[i] = (u[i] & 0xffffu) | x << 16;
-            }
-            vf[half][dt] = __builtin_bit_cast(bf16x8_a, u);
-          }
+        for (int i = 0; i < D; i += 64) {
+          const int d = i + lane;
+          const unsigned short x = vrow[d];
+          vl[d * 64 + ((pin >> 3) ^ (d & 7)) * 8 + (pin & 7)] = x;
+          p.vw[((long long)page * p.KVH + kvh) * VT + d * 64 + pin] = x;
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
       }
       // ---- PV: two 32-pos halves ---------------------------------------
       // A-frag needs lane (head=col, hi) to hold P[head][pos = hi*8 + e]:
@@ -307,6 +300,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       // and (2*hi+1)&3, tile = half*2 + (hi>>1).  __shfl evaluates its value
       // in EACH lane and a register index has to be a constant: shuffle both
       // candidate tiles' registers and select by hi.
+      // B-frag: lane holds V^T[pos = half*32 + hi*8 + e][d = dt*16+col]
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         const int src_a = col + (((2 * hi) & 3) << 4);
@@ -325,10 +319,34 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         const u32x4_v pu = {lo ? a0A : a0B, lo ? a1A : a1B, lo ? b0A : b0B,
                             lo ? b1A : b1B};
         const bf16x8_a pa = __builtin_bit_cast(bf16x8_a, pu);
+        const unsigned short* vr =
+            vl + col * 64 + ((half * 4 + hi) ^ (col & 7)) * 8;
+        bf16x8_a vf[DTILES];
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt)
+          vf[dt] = *reinterpret_cast<const bf16x8_a*>(vr + dt * 1024);
 #pragma unroll
         for (int dt = 0; dt < DTILES; ++dt)
           o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              pa, vf[half][dt], o_acc[dt], 0, 0, 0);
+              pa, vf[dt], o_acc[dt], 0, 0, 0);
+      }
+      if constexpr (patch.value) {     // the key's lines: 8 positions each
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt)
+          if (pt * 16 + col == pin) {
+            unsigned short* kw =
+                p.kw + ((long long)page * p.KVH + kvh) * VT;
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks)
+              *reinterpret_cast<bf16x8_a*>(
+                  kw + ((ks * 4 + hi) * QSA_PAGE + pt * 16 + col) * 8) =
+                  kf[pt][ks];
+          }
+      }
+      if (more) {                      // all of the values have been read
+        __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        load_v(next);
       }
       page = next;
     };
@@ -339,14 +357,15 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   }
 
   // ---- the waves of the block meet: O C-layout row = head = hi*4 + r -----
-  float* ml = smem + NW * R * D;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  float* os = reinterpret_cast<float*>(vlds);     // [NW][VT / 2]
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int head = hi * 4 + r;
     if (head < R)
 #pragma unroll
       for (int dt = 0; dt < DTILES; ++dt)
-        smem[(wave * R + head) * D + dt * 16 + col] = o_acc[dt][r];
+        os[wave * (VT / 2) + head * D + dt * 16 + col] = o_acc[dt][r];
   }
   if (lane < 16) {
     ml[wave * 16 + lane] = m;
@@ -365,7 +384,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       // a wave without keys: no weight, whatever M is
       const float f = ls > 0.f ? __expf(ml[w * 16 + head] - M) : 0.f;
       L += f * ls;
-      acc += f * smem[(w * R + head) * D + d];
+      acc += f * os[w * (VT / 2) + i];
     }
     const int qh = kvh * R + head;
     if (p.NS == 1) {
@@ -412,31 +431,33 @@ qsa_attn_reduce(const float* __restrict__ part_o,   // [rows, NS, D]
     out[row * D + d] = v;
 }
 
-// Waves of a block and blocks per (row, kv head): one block of four waves where
-// the rows alone give every CU two, one of eight for few pages (a second launch
-// would cost more than it spreads: 32/8 heads of 64, 1 row of 700 keys 9.2 us
-// against 11.1; 32/8 of 128, 16 rows of 20-100 8.8 against 13.5; even at 1 row
-// of 700 of those, 13.3 / 13.2); otherwise blocks of four until there are 2048
-// waves.
-// max_pages is the table's width, since the rows' lengths are on the device: a
-// table of 64 columns has short rows split, with the merge and without the
-// read-ahead below (a 16-layer step of 2048 width, 1 row of 700 keys: 602 us
-// with a table of 11 columns, 634 of 64, 677 of 128; 4 rows of 500-900 668, 682,
-// 683; 4096 width, 8 layers, 1 row 549, 520, 542, 16 rows 658, 648, 649).
+// Waves of a block and blocks per (row, kv head), of which several cost a second
+// launch (3 to 4 us).  Up to 16 pages a block of eight waves is over before one
+// of several and the merge (32/8 heads of 128, 1 row of 700 keys 11.5 us against
+// 13.1, 16 rows 16.5 / 19.1); four once they share CUs (48 rows 38.1 / 41.6).
+// Longer rows: from 129 pairs eight waves alone (24 rows of 1000-2000 keys 35.8
+// us, three blocks of four 43; 28 of 2500-4000 77 / 84), from 257 four alone (48 of
+// 1000-2000 69.8, two blocks 70.4; 63: 84.4 / 89.4), but three of four while the
+// chip's second round is nearly empty and rows are long (33 of 3000-4096 102 / 111);
+// below, what fills the chip (8 of 1000-2000 19.1, eight blocks of four 21.5; 12
+// 23.0 / 27.9).
+// max_pages is the table's width, since the rows' lengths are on the device: in
+// a table for longer rows short ones of up to 128 pairs are split, with the merge
+// and without the read-ahead below.
 extern "C" void qsa_paged_attn_split(int B, int QH, int KVH, int max_pages,
                                      int D, int* waves, int* splits) {
   const long long heads = (long long)B * KVH;
-  const int lds = QH / KVH * D * 4;    // bytes per wave
-  *waves = 4;
+  const bool few = max_pages <= 16;
+  *waves = heads > 256 || max_pages <= 4 || (heads <= 48 && !few) ? 4 : 8;
   *splits = 1;
-  if (heads >= 512) return;
-  if (max_pages <= 16 && 8 * lds <= 60 * 1024) {
-    *waves = max_pages <= 4 ? 4 : 8;
-    return;
+  if (heads > 256) {
+    if (heads < 384 && max_pages > 32) *splits = 3;
+  } else if (!few && heads <= 128) {
+    const long long fill = (2048 + 4 * heads - 1) / (4 * heads);
+    *splits = heads > 64   ? 2
+              : heads > 48 ? 4
+                           : (int)std::min<long long>(fill, (max_pages + 7) / 8);
   }
-  const long long want = (2048 + 4 * heads - 1) / (4 * heads);
-  *splits = (int)std::max<long long>(
-      1, std::min<long long>(want, (max_pages + 3) / 4));
 }
 
 extern "C" void qsa_paged_attn_mfma_launch(
@@ -467,15 +488,14 @@ extern "C" void qsa_paged_attn_mfma_launch(
     }
     grid.x = 256;
   }
-  const size_t lds = sizeof(float) * waves * ((size_t)QH / KVH * D + 32);
 #define QSA_DECODE(DD, NW)                                                  \
   if (D == DD && waves == NW) {                                             \
     if (k)                                                                  \
       hipLaunchKernelGGL((qsa_paged_attn_mfma<DD, NW, true>), grid, block,  \
-                         lds, stream, p);                                   \
+                         0, stream, p);                                     \
     else                                                                    \
       hipLaunchKernelGGL((qsa_paged_attn_mfma<DD, NW, false>), grid, block, \
-                         lds, stream, p);                                   \
+                         0, stream, p);                                     \
   }
   QSA_DECODE(128, 4) QSA_DECODE(128, 8) QSA_DECODE(64, 4) QSA_DECODE(64, 8)
 #undef QSA_DECODE
