@@ -257,10 +257,10 @@ qsa_rows_gemm(RowsArgs p) {
   const int N = ACT ? p.N >> 1 : p.N;
   const int c0 = (ACT ? n0 / 2 : n0) + wave % WN * G * 8;
 #pragma unroll
-  for (int x = 0; x < MT * G / 4; ++x) {
+  for (int x = 0; x < (MT * G + 3) / 4; ++x) {
     const int i = x * 64 + lane, row = i / G, c = i % G * 8;
     const int m = m0 + wm * 16 + row;
-    if (m < p.M && c0 + c < N)                    // N % 8 == 0
+    if (row < MT * 16 && m < p.M && c0 + c < N)   // N % 8 == 0
       *reinterpret_cast<u32x4_v*>(p.C + (long long)m * N + c0 + c) =
           *reinterpret_cast<const u32x4_v*>(o + row * OP + c);
   }
