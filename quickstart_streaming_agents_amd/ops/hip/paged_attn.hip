@@ -132,6 +132,8 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   const int R = p.QH / p.KVH;
   const int first = split * NW + wave, step = NW * p.NS;
   const int* btab = p.block_table + (long long)b * p.max_pages;
+  // side by side: the first page's number waits for no length
+  int page = btab[min(first, p.max_pages - 1)];
   const int seqlen = p.seq_lens[b];
   const int npages = (seqlen + QSA_PAGE - 1) / QSA_PAGE;
   const int col = lane & 15;          // head col (scores) / dim col (PV)
@@ -152,22 +154,6 @@ qsa_paged_attn_mfma(DecodeArgs p) {
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
       qf[ks] = *reinterpret_cast<const bf16x8_a*>(qrow + ks * 32 + hi * 8);
-    // the new key, in the same order: every lane's column is a copy
-    bf16x8_a kn[FUSE ? KSTEPS : 1];
-    float cs[FUSE ? KSTEPS / 2 : 1][8], sn[FUSE ? KSTEPS / 2 : 1][8];
-    if constexpr (FUSE) {
-      const unsigned short* krow =
-          p.k + (long long)b * p.kvstride + (long long)kvh * D;
-      const long long at = (long long)(seqlen - 1) * (D / 2) + hi * 8;
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks)
-        kn[ks] = *reinterpret_cast<const bf16x8_a*>(krow + ks * 32 + hi * 8);
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS / 2; ++ks) {
-        ldv<float, 8>(p.cos_t + at + ks * 32, cs[ks]);
-        ldv<float, 8>(p.sin_t + at + ks * 32, sn[ks]);
-      }
-    }
     auto load_k = [&](int page, bf16x8_a (&kf)[4][KSTEPS]) {
       const unsigned short* kbase =
           p.kc + ((((long long)page * p.KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
@@ -193,9 +179,26 @@ qsa_paged_attn_mfma(DecodeArgs p) {
             (__attribute__((address_space(3))) void*)(vl + i * 512), 16, 0, 0);
     };
     bf16x8_a kf[4][KSTEPS];
-    int page = btab[first];
     load_k(page, kf);
-    load_v(page);
+    // the new key, in the same order: every lane's column is a copy; and value
+    bf16x8_a kn[FUSE ? KSTEPS : 1];
+    unsigned short vn[FUSE ? D / 64 : 1];
+    float cs[FUSE ? KSTEPS / 2 : 1][8], sn[FUSE ? KSTEPS / 2 : 1][8];
+    if constexpr (FUSE) {
+      const long long row = (long long)b * p.kvstride + (long long)kvh * D;
+      const unsigned short* krow = p.k + row;
+#pragma unroll
+      for (int i = 0; i < D / 64; ++i) vn[i] = p.v[row + i * 64 + lane];
+      const long long at = (long long)(seqlen - 1) * (D / 2) + hi * 8;
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks)
+        kn[ks] = *reinterpret_cast<const bf16x8_a*>(krow + ks * 32 + hi * 8);
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS / 2; ++ks) {
+        ldv<float, 8>(p.cos_t + at + ks * 32, cs[ks]);
+        ldv<float, 8>(p.sin_t + at + ks * 32, sn[ks]);
+      }
+    }
     if constexpr (FUSE) {
 #pragma unroll
       for (int ks = 0; ks < KSTEPS / 2; ++ks) {
@@ -229,6 +232,8 @@ qsa_paged_attn_mfma(DecodeArgs p) {
                                                         acc, 0, 0, 0);
         sc[pt] = acc;
       }
+      // values only now: before the keys they would delay them
+      load_v(page);
       if (more) load_k(next, kf);
       // scale + mask invalid positions; C layout: row pos = hi*4 + r,
       // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
@@ -281,14 +286,11 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       if (more) wait_vm<KL>();
       else wait_vm<0>();
       if constexpr (patch.value) {
-        const unsigned short* vrow =
-            p.v + (long long)b * p.kvstride + (long long)kvh * D;
 #pragma unroll
         for (int i = 0; i < D; i += 64) {
           const int d = i + lane;
-          const unsigned short x = vrow[d];
-          vl[d * 64 + ((pin >> 3) ^ (d & 7)) * 8 + (pin & 7)] = x;
-          p.vw[((long long)page * p.KVH + kvh) * VT + d * 64 + pin] = x;
+          vl[d * 64 + ((pin >> 3) ^ (d & 7)) * 8 + (pin & 7)] = vn[i / 64];
+          p.vw[((long long)page * p.KVH + kvh) * VT + d * 64 + pin] = vn[i / 64];
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
@@ -343,11 +345,9 @@ qsa_paged_attn_mfma(DecodeArgs p) {
                   kf[pt][ks];
           }
       }
-      if (more) {                      // all of the values have been read
-        __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0)
-        asm volatile("" ::: "memory");
-        load_v(next);
-      }
+      // all of the values have been read when the next page's come
+      __builtin_amdgcn_s_waitcnt(0xc07f);         // lgkmcnt(0)
+      asm volatile("" ::: "memory");
       page = next;
     };
     int pi = first;
