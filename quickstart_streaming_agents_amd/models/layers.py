@@ -33,6 +33,12 @@ class Linear:
             return D.skinny_linear(x, self.packed, *self.w.shape)
         return D.linear(x, self.w)
 
+    def parts(self, x: torch.Tensor) -> torch.Tensor:
+        """y for a reader that adds shares of K (D.linear_parts)."""
+        if self._skinny(x):
+            return D.skinny_linear(x, self.packed, *self.w.shape)
+        return D.linear_parts(x, self.w)
+
     def _skinny(self, x: torch.Tensor) -> bool:
         return self.packed is not None and \
             1 <= x.shape[0] <= self.SKINNY_ROWS and x.stride(0) % 8 == 0
@@ -88,13 +94,16 @@ class RopeTable:
 
 
 class DenseGLU:
-    """W_down(act(W_gate h) * (W_up h)); gate and up share one GEMM."""
+    """W_down(act(W_gate h) * (W_up h)); gate and up share one GEMM.  `whole`:
+    this is the entire sum, not a rank's part, so shares of it may be left to
+    the residual's norm."""
 
     def __init__(self, gate: torch.Tensor, up: torch.Tensor,
-                 down: torch.Tensor, act: str = "silu"):
+                 down: torch.Tensor, act: str = "silu", whole: bool = False):
         self.act = act
         self.gate_up = Linear(torch.cat([gate, up]).contiguous())
-        self.down = Linear(down)
+        down = Linear(down)
+        self.down = down.parts if whole else down
 
     def __call__(self, h: torch.Tensor) -> torch.Tensor:
         return self.down(self.gate_up.glu(h, self.act))
@@ -111,8 +120,8 @@ class TokenSide:
         self.gate, self.proj = Linear(gate), Linear(proj)
 
     def __call__(self, x: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
-        return self.proj(D.glu_table(self.gate(x), self.table, ids,
-                                     self.col0, self.act))
+        return self.proj.parts(D.glu_table(
+            self.gate.parts(x), self.table, ids, self.col0, self.act))
 
 
 def upload(a: np.ndarray, device) -> torch.Tensor:

@@ -213,11 +213,13 @@ class LlamaModel:
 
     def _linear(self, x: torch.Tensor, w: torch.Tensor,
                 wf: torch.Tensor | None = None,
-                wf8: tuple | None = None) -> torch.Tensor:
+                wf8: tuple | None = None,
+                parts: bool = False) -> torch.Tensor:
         """Projection: decode-sized cuda batches go through the
         weight-streaming skinny GEMM — fp8 (W8A16, half the weight
         stream) when packed, else bf16; what does not fill a library's tiles
-        through rows_gemm; everything else rocBLAS."""
+        through rows_gemm; everything else rocBLAS.  `parts`: the reader is the
+        residual's norm, which adds shares of K."""
         n, k = w.shape
         M = x.shape[0]
         if x.is_cuda and wf8 is not None:
@@ -242,7 +244,7 @@ class LlamaModel:
             # bf16 skinny wins only the small decode shapes (qkv/wo);
             # rocBLAS is at the bandwidth floor for the big-N ones
             return D.skinny_linear(x, wf, n, k)
-        return D.linear(x, w)
+        return D.linear_parts(x, w) if parts else D.linear(x, w)
 
     def _tp_all_reduce(self, t: torch.Tensor) -> torch.Tensor:
         if self.tp_size > 1:
@@ -286,7 +288,8 @@ class LlamaModel:
             attn = self._decode_attention(qkv, L, li, kv, block_table,
                                           seq_lens).view(B, -1)
             o = self._tp_all_reduce(
-                self._linear(attn, L["wo"], L.get("wo_f"), L.get("wo_f8")))
+                self._linear(attn, L["wo"], L.get("wo_f"), L.get("wo_f8"),
+                             self.tp_size == 1))
             h = D.rmsnorm_residual(o, res, L["mlp_norm"], c.norm_eps)
             mlp_out = self._ffn(L, h)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)
@@ -357,7 +360,7 @@ class LlamaModel:
             act = D.swiglu(gu[:, :self.ffn_local], gu[:, self.ffn_local:])
         return self._tp_all_reduce(
             self._linear(act, L["wdown"], L.get("wdown_f"),
-                         L.get("wdown_f8")))
+                         L.get("wdown_f8"), self.tp_size == 1))
 
     def _gather_kv(self, kc_l: torch.Tensor, vc_l: torch.Tensor,
                    pages: list[int], n: int):
@@ -529,7 +532,9 @@ class LlamaModel:
                     .permute(0, 3, 1, 2, 4) \
                     .reshape(nb * nmax, self.n_q * c.d_head) \
                     .index_select(0, dst_idx)
-            o = self._tp_all_reduce(D.linear(attn, L["wo"]))
+            o = self._tp_all_reduce(
+                D.linear_parts(attn, L["wo"]) if self.tp_size == 1
+                else D.linear(attn, L["wo"]))
             h = D.rmsnorm_residual(o, res, L["mlp_norm"], c.norm_eps)
             mlp_out = self._ffn(L, h)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)

@@ -190,7 +190,8 @@ class LunulixModel(MixerDecoder):
                 layer.norm2 = get(p + "norm2")
                 layer.ff = DenseGLU(shard.rows(get(p + "mlp.gate")),
                                     shard.rows(get(p + "mlp.up")),
-                                    shard.cols(get(p + "mlp.down")), "gelu")
+                                    shard.cols(get(p + "mlp.down")), "gelu",
+                                    shard.size == 1)
                 layer.norm2b = get(p + "norm2b")
             self.layers.append(layer)
 
@@ -217,10 +218,10 @@ class LunulixModel(MixerDecoder):
             x = D.residual_norm(res, y, None, None, eps, post=post)
             y, post = L.side(x, ids), L.side_norm
             if trail is not None:
-                e = y.float()
+                e = D.add_shares(y).float()
                 trail.append(res + e * torch.rsqrt(
                     e.pow(2).mean(-1, keepdim=True) + eps) * post.float())
         if rows is not None:
-            res, y = res.index_select(0, rows), y.index_select(0, rows)
+            res, y = res.index_select(0, rows), y.index_select(-2, rows)
         return self.head(D.residual_norm(res, y, self.final, None, eps,
                                          layer=False, post=post))

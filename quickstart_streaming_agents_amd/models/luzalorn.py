@@ -188,7 +188,8 @@ class LuzalornModel(MixerDecoder):
                 layer.norm2 = (get(p + "norm2"), get(p + "norm2.b"))
                 layer.ff = DenseGLU(shard.rows(get(p + "mlp.gate")),
                                     shard.rows(get(p + "mlp.up")),
-                                    shard.cols(get(p + "mlp.down")))
+                                    shard.cols(get(p + "mlp.down")),
+                                    whole=shard.size == 1)
             self.layers.append(layer)
 
     # ---- forward -----------------------------------------------------------
@@ -213,7 +214,7 @@ class LuzalornModel(MixerDecoder):
                 h = D.residual_norm(res, y, *L.norm2, eps)
                 y = self._reduce(L.ff(h))
             if trail is not None:
-                trail.append(res + y.float())
+                trail.append(res + D.add_shares(y).float())
         if rows is not None:
-            res, y = res.index_select(0, rows), y.index_select(0, rows)
+            res, y = res.index_select(0, rows), y.index_select(-2, rows)
         return self.head(D.residual_norm(res, y, *self.final, eps))

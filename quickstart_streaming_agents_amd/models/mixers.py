@@ -42,6 +42,12 @@ class Shard:
         n = t.shape[1] // self.size
         return t[:, self.rank * n:(self.rank + 1) * n].contiguous()
 
+    def out(self, w: torch.Tensor):
+        """A mixer's output projection.  Alone, its shares of K may be left to
+        the residual's norm; ranks have to add theirs first."""
+        lin = Linear(w)
+        return lin.parts if self.size == 1 else lin
+
 
 class Retention:
     """Linear attention with one fixed decay per head, rotated q and k, and
@@ -61,7 +67,7 @@ class Retention:
         self.kscale = self.D ** -0.5
         self.proj = Linear(torch.cat([shard.rows(get(n))
                                       for n in ("q", "k", "v", "g")]))
-        self.out = Linear(shard.cols(get("o")))
+        self.out = shard.out(shard.cols(get("o")))
         dev = self.proj.w.device
         decay = shard.rows(torch.tensor(m["decay"], dtype=torch.float64))
         self.decay = decay.float().to(dev)
@@ -140,7 +146,7 @@ class LatentAttention:
         self.uk_t = uk.view(H, self.D, self.R).transpose(1, 2).contiguous()
         self.uv = uv.view(H, self.E, self.R).contiguous()
         self.sink = shard.rows(get("sink"))
-        self.out = Linear(shard.cols(get("o")))
+        self.out = shard.out(shard.cols(get("o")))
         self.longest = None
         # sizes of the flash kernel, and a gate slice it can read in words
         if uk.is_cuda and dtype == torch.bfloat16 and \
@@ -367,7 +373,7 @@ class Parallel:
                                     w.shape[1])]
         self.at = at[1]
         self.proj = Linear(torch.cat(rows))
-        self.out = Linear(torch.cat([self.left.out, self.right.out], 1))
+        self.out = shard.out(torch.cat([self.left.out, self.right.out], 1))
         del self.left.out, self.right.out
 
     @staticmethod

@@ -31,8 +31,13 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 
 def rmsnorm_residual(x: torch.Tensor, res: torch.Tensor, w: torch.Tensor,
                      eps: float) -> torch.Tensor:
-    """res <- res + x (in place); returns rmsnorm(res) * w."""
+    """res <- res + x (in place); returns rmsnorm(res) * w.  x may be
+    linear_parts' shares."""
     if _cuda(x):
+        if x.dim() == res.dim() + 1:
+            if res.shape[-1] <= 8192:
+                return lm_ext().rmsnorm_shares(x, res, w, eps)
+            x = add_shares(x)
         return ext().rmsnorm_residual(x, res, w, eps)
     res.add_(x)
     rf = res.float()
@@ -216,6 +221,24 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear() for a reader that adds shares (residual_norm, rmsnorm_residual,
+    glu_table): where K is split, [S, rows, columns] in f32."""
+    if rows_linear_ok(x, w):
+        return lm_ext().rows_parts(x, w)
+    return torch.nn.functional.linear(x, w)
+
+
+def add_shares(y: torch.Tensor) -> torch.Tensor:
+    """linear_parts' result as linear's, for any other reader."""
+    if y.dim() == 2:
+        return y
+    out = y[0]
+    for part in y[1:]:
+        out = out + part
+    return out.to(torch.bfloat16)
+
+
 def glu_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the activation is glu_linear's to apply: W's rows are [gate; up]
     and both fit its kernel (the rules are beside rows_linear's)."""
@@ -323,7 +346,7 @@ def residual_norm(res: torch.Tensor, y: torch.Tensor | None,
     """res (f32) <- (0 if init else res) + y + tscale * table[ids] + vec, in
     place; returns the layer norm (layer=True) or rms norm of it, times w,
     plus b, or without w the residual itself.  With `post`, y enters as its
-    own rms norm times post."""
+    own rms norm times post.  On the GPU y may be linear_parts' shares."""
     if _cuda(res):
         return lm_ext().residual_norm(res, y, table, ids, vec, w, b, eps,
                                       init, layer, post, tscale)
@@ -344,7 +367,8 @@ def glu(gate: torch.Tensor, up: torch.Tensor,
 
 def glu_table(gate: torch.Tensor, table: torch.Tensor, ids: torch.Tensor,
               col0: int, act: str = "gelu") -> torch.Tensor:
-    """act(gate [T, n]) * table[ids, col0 : col0 + n]."""
+    """act(gate [T, n]) * table[ids, col0 : col0 + n]; on the GPU gate may be
+    linear_parts' shares."""
     if _cuda(gate):
         return lm_ext().glu_table(gate, table, ids, col0, act == "gelu")
     from .cpu_ref import gated_act_ref

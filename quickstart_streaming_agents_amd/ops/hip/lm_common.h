@@ -82,6 +82,34 @@ __device__ __forceinline__ float sigmoid_f(float z) {
   return 1.f / (1.f + expf(-z));
 }
 
+// VEC values of a product whose shares of K were left to its reader: S f32 sums,
+// `step` elements apart, added in order and rounded as the product is stored
+template <int VEC>
+__device__ __forceinline__ void ld_shares(const float* p, long long step,
+                                          int S, float* v) {
+  static_assert(VEC % 4 == 0, "16-byte groups");
+  constexpr int U = 4;                 // shares under way at a time
+  f32x4_v sum[VEC / 4];
+#pragma unroll
+  for (int i = 0; i < VEC / 4; ++i) sum[i] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < S; s += U) {
+    f32x4_v x[U][VEC / 4];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < VEC / 4; ++i)
+        x[u][i] = *reinterpret_cast<const f32x4_v*>(
+            p + min(s + u, S - 1) * step + i * 4);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s + u < S)
+#pragma unroll
+        for (int i = 0; i < VEC / 4; ++i) sum[i] += x[u][i];
+  }
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) v[i] = bf16_to_f32(cvt_bf16(sum[i / 4][i % 4]));
+}
+
 // silu, or the tanh form of gelu
 #define QSA_ACT_SILU 0
 #define QSA_ACT_GELU 1

@@ -13,11 +13,14 @@
 //                              + eps).  b optional; without w, out = r.
 // The row stays in registers between the passes up to CACHED groups per
 // thread; wider rows re-read the residual this thread wrote itself.
+// SHARES: y is a product whose shares of K have not been added; doing it here
+// saves the launch that would (64 x 2048, four shares: 4.6 us).
 // ---------------------------------------------------------------------------
-template <typename T, int VEC, bool LAYER, bool POST>
+template <typename T, int VEC, bool LAYER, bool POST, bool SHARES>
 __global__ void __launch_bounds__(1024)
 qsa_residual_norm(float* __restrict__ res, const T* __restrict__ y,
-                  long long ystride, const T* __restrict__ post,
+                  long long ystride, const float* __restrict__ parts,
+                  long long pstep, int S, const T* __restrict__ post,
                   const T* __restrict__ table,
                   const long long* __restrict__ ids, float tscale,
                   const T* __restrict__ vec, const T* __restrict__ w,
@@ -34,6 +37,10 @@ qsa_residual_norm(float* __restrict__ res, const T* __restrict__ y,
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
     er = table + id * W;
   }
+  auto load_y = [&](int i, float* v) {
+    if constexpr (SHARES) ld_shares<VEC>(parts + row * W + i, pstep, S, v);
+    else ldv<T, VEC>(yr + i, v);
+  };
   const int step = blockDim.x * VEC;
   const int i0 = threadIdx.x * VEC;
   float cache[CACHED][VEC];
@@ -44,14 +51,14 @@ qsa_residual_norm(float* __restrict__ res, const T* __restrict__ y,
     for (int c = 0; c < CACHED; ++c) {
       const int i = i0 + c * step;
       if (i < W) {
-        ldv<T, VEC>(yr + i, cache[c]);
+        load_y(i, cache[c]);
 #pragma unroll
         for (int j = 0; j < VEC; ++j) ss = fmaf(cache[c][j], cache[c][j], ss);
       }
     }
     for (int i = i0 + CACHED * step; i < W; i += step) {
       float v[VEC];
-      ldv<T, VEC>(yr + i, v);
+      load_y(i, v);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) ss = fmaf(v[j], v[j], ss);
     }
@@ -77,8 +84,8 @@ qsa_residual_norm(float* __restrict__ res, const T* __restrict__ y,
       } else {
         ldv<float, VEC>(rr + i, v);
       }
-      if (yr) {
-        ldv<T, VEC>(yr + i, t);
+      if (SHARES || yr) {
+        load_y(i, t);
 #pragma unroll
         for (int j = 0; j < VEC; ++j) v[j] += t[j];
       }
@@ -107,7 +114,7 @@ qsa_residual_norm(float* __restrict__ res, const T* __restrict__ y,
   }
   for (int i = i0 + CACHED * step; i < W; i += step) {
     float v[VEC];
-    if (POST) ldv<T, VEC>(yr + i, v);
+    if (POST) load_y(i, v);
     load_row(i, v);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) sum += LAYER ? v[j] : v[j] * v[j];
@@ -172,8 +179,9 @@ qsa_residual_norm(float* __restrict__ res, const T* __restrict__ y,
   }
 }
 
-template <typename T, int VEC, bool LAYER, bool POST>
+template <typename T, int VEC, bool LAYER, bool POST, bool SHARES>
 static void residual_norm_go(float* res, const void* y, long long ystride,
+                             const float* parts, int S,
                              const void* post, const void* table,
                              const long long* ids, float tscale,
                              const void* vec, const void* w, const void* b,
@@ -183,33 +191,84 @@ static void residual_norm_go(float* res, const void* y, long long ystride,
   // few rows: wide blocks, one round of loads; many rows: narrow ones
   const int most = rows <= 256 ? 1024 : 256;
   threads = threads > most ? most : threads;
-  hipLaunchKernelGGL((qsa_residual_norm<T, VEC, LAYER, POST>),
+  hipLaunchKernelGGL((qsa_residual_norm<T, VEC, LAYER, POST, SHARES>),
                      dim3((unsigned)rows), dim3(threads), 0, st, res,
-                     (const T*)y, ystride, (const T*)post, (const T*)table,
+                     (const T*)y, ystride, parts, rows * W, S,
+                     (const T*)post, (const T*)table,
                      ids, tscale, (const T*)vec, (const T*)w, (const T*)b,
                      (T*)out, W, vocab, eps, init);
 }
 
+// parts and S: y as S shares [S][rows][W], bf16 storage and vec4 only
 extern "C" void qsa_residual_norm_launch(
-    float* res, const void* y, long long ystride, const void* post,
+    float* res, const void* y, long long ystride, const float* parts, int S,
+    const void* post,
     const void* table, const long long* ids, float tscale, const void* vec,
     const void* w, const void* b, void* out, long long rows, int W, int vocab,
     float eps, int init, int layer, int f32, int vec4, hipStream_t st) {
-#define QSA_RN(T, V, L, P)                                                    \
-  residual_norm_go<T, V, L, P>(res, y, ystride, post, table, ids, tscale,     \
-                               vec, w, b, out, rows, W, vocab, eps, init, st)
-#define QSA_RN_L(T, V)                                                        \
-  if (layer) { if (post) QSA_RN(T, V, true, true);                            \
-               else QSA_RN(T, V, true, false); }                              \
-  else { if (post) QSA_RN(T, V, false, true);                                 \
-         else QSA_RN(T, V, false, false); }
-  if (f32) {
-    if (vec4) { QSA_RN_L(float, 4) } else { QSA_RN_L(float, 1) }
+#define QSA_RN(T, V, L, P, H)                                                 \
+  residual_norm_go<T, V, L, P, H>(res, y, ystride, parts, S, post, table,     \
+                                  ids, tscale, vec, w, b, out, rows, W,       \
+                                  vocab, eps, init, st)
+#define QSA_RN_L(T, V, H)                                                     \
+  if (layer) { if (post) QSA_RN(T, V, true, true, H);                         \
+               else QSA_RN(T, V, true, false, H); }                           \
+  else { if (post) QSA_RN(T, V, false, true, H);                              \
+         else QSA_RN(T, V, false, false, H); }
+  if (parts) {
+    QSA_RN_L(bf16_t, 4, true)
+  } else if (f32) {
+    if (vec4) { QSA_RN_L(float, 4, false) } else { QSA_RN_L(float, 1, false) }
   } else {
-    if (vec4) { QSA_RN_L(bf16_t, 4) } else { QSA_RN_L(bf16_t, 1) }
+    if (vec4) { QSA_RN_L(bf16_t, 4, false) } else { QSA_RN_L(bf16_t, 1, false) }
   }
 #undef QSA_RN_L
 #undef QSA_RN
+}
+
+// ---------------------------------------------------------------------------
+// The Llama decoder's norm behind such a product: res <- res + sum of shares in
+// bf16, out = rms norm of it times w, with the roundings of a stored product and
+// of qsa_rmsnorm_kernel (elementwise.hip).  A row is one round of loads of its
+// block (W <= 8192), S of them per thread.  192 x 4096, four shares: sum and norm
+// as launches of their own 8.8 us, 5.2 here.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(1024)
+qsa_rmsnorm_shares(const float* __restrict__ parts, long long step, int S,
+                   bf16_t* __restrict__ res, const bf16_t* __restrict__ w,
+                   bf16_t* __restrict__ out, int W, float eps) {
+  __shared__ float scratch[16];
+  const long long row = (long long)blockIdx.x * W;
+  const int i = threadIdx.x * 8;
+  float r[8], g[8], ss = 0.f;
+  if (i < W) {
+    float x[8];
+    ldv<bf16_t, 8>(res + row + i, r);
+    ldv<bf16_t, 8>(w + i, g);
+    ld_shares<8>(parts + row + i, step, S, x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      r[j] += x[j];
+      ss = fmaf(r[j], r[j], ss);
+      r[j] = bf16_to_f32(cvt_bf16(r[j]));
+    }
+    stv<bf16_t, 8>(res + row + i, r);
+  }
+  const float inv = rsqrtf(block_reduce_sum(ss, scratch) / (float)W + eps);
+  if (i < W) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = r[j] * inv * g[j];
+    stv<bf16_t, 8>(out + row + i, r);
+  }
+}
+
+extern "C" void qsa_rmsnorm_shares_launch(const float* parts, int S,
+                                          bf16_t* res, const bf16_t* w,
+                                          bf16_t* out, long long rows, int W,
+                                          float eps, hipStream_t st) {
+  hipLaunchKernelGGL(qsa_rmsnorm_shares, dim3((unsigned)rows),
+                     dim3((W / 8 + 63) / 64 * 64), 0, st, parts, rows * W, S,
+                     res, w, out, W, eps);
 }
 
 // ---------------------------------------------------------------------------
@@ -220,9 +279,11 @@ extern "C" void qsa_residual_norm_launch(
 // act: silu, or the tanh form of gelu, z / (1 + exp(-2 sqrt(2/pi)
 // (z + 0.044715 z^3))).
 // ---------------------------------------------------------------------------
-template <typename T, int VEC, int ACT>
+// S > 0 with a table: the gate is a product whose S shares have not been added.
+template <typename T, int VEC, int ACT, bool SHARES>
 __global__ void __launch_bounds__(256)
-qsa_glu(const T* __restrict__ gate, const T* __restrict__ up,
+qsa_glu(const T* __restrict__ gate, const float* __restrict__ parts, int S,
+        const T* __restrict__ up,
         const long long* __restrict__ ids, T* __restrict__ out,
         long long rows, long long cols, long long stride, long long ustride,
         long long vocab) {
@@ -237,7 +298,8 @@ qsa_glu(const T* __restrict__ gate, const T* __restrict__ up,
       ur = ur < 0 ? 0 : (ur >= vocab ? vocab - 1 : ur);
     }
     float g[VEC], u[VEC];
-    ldv<T, VEC>(gate + r * stride + c, g);
+    if constexpr (SHARES) ld_shares<VEC>(parts + i * VEC, rows * cols, S, g);
+    else ldv<T, VEC>(gate + r * stride + c, g);
     ldv<T, VEC>(up + ur * ustride + c, u);
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
@@ -246,7 +308,8 @@ qsa_glu(const T* __restrict__ gate, const T* __restrict__ up,
   }
 }
 
-extern "C" void qsa_glu_launch(const void* gate, const void* up,
+extern "C" void qsa_glu_launch(const void* gate, const float* parts, int S,
+                               const void* up,
                                const long long* ids, void* out,
                                long long rows, long long cols,
                                long long stride, long long ustride,
@@ -255,14 +318,21 @@ extern "C" void qsa_glu_launch(const void* gate, const void* up,
   const long long n = rows * (cols / (vec ? 8 : 1));
   const long long want = (n + 255) / 256;
   dim3 grid((unsigned)(want < 1 ? 1 : (want > 16384 ? 16384 : want)));
-#define QSA_GLU(T, V, A)                                                   \
-  hipLaunchKernelGGL((qsa_glu<T, V, A>), grid, dim3(256), 0, st,           \
-                     (const T*)gate, (const T*)up, ids, (T*)out, rows,     \
-                     cols, stride, ustride, vocab)
-#define QSA_GLU_A(T, V)                                                    \
-  if (gelu) QSA_GLU(T, V, QSA_ACT_GELU); else QSA_GLU(T, V, QSA_ACT_SILU)
-  if (f32) { if (vec) { QSA_GLU_A(float, 8); } else { QSA_GLU_A(float, 1); } }
-  else     { if (vec) { QSA_GLU_A(bf16_t, 8); } else { QSA_GLU_A(bf16_t, 1); } }
+#define QSA_GLU(T, V, A, H)                                                \
+  hipLaunchKernelGGL((qsa_glu<T, V, A, H>), grid, dim3(256), 0, st,        \
+                     (const T*)gate, parts, S, (const T*)up, ids, (T*)out, \
+                     rows, cols, stride, ustride, vocab)
+#define QSA_GLU_A(T, V, H)                                                 \
+  if (gelu) QSA_GLU(T, V, QSA_ACT_GELU, H);                                \
+  else QSA_GLU(T, V, QSA_ACT_SILU, H)
+  if (parts) { QSA_GLU_A(bf16_t, 8, true); }
+  else if (f32) {
+    if (vec) { QSA_GLU_A(float, 8, false); }
+    else { QSA_GLU_A(float, 1, false); }
+  } else {
+    if (vec) { QSA_GLU_A(bf16_t, 8, false); }
+    else { QSA_GLU_A(bf16_t, 1, false); }
+  }
 #undef QSA_GLU_A
 #undef QSA_GLU
 }

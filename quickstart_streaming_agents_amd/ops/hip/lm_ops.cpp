@@ -47,10 +47,13 @@ struct ConvStep {
 };
 
 extern "C" void qsa_residual_norm_launch(float*, const void*, long long,
-    const void*, const void*, const long long*, float, const void*,
+    const float*, int, const void*, const void*, const long long*, float, const void*,
     const void*, const void*, void*, long long, int, int, float, int, int,
     int, int, hipStream_t);
-extern "C" void qsa_glu_launch(const void*, const void*, const long long*,
+extern "C" void qsa_rmsnorm_shares_launch(const float*, int, bf16_t*,
+    const bf16_t*, bf16_t*, long long, int, float, hipStream_t);
+extern "C" void qsa_glu_launch(const void*, const float*, int, const void*,
+    const long long*,
     void*, long long, long long, long long, long long, long long, int, int,
     int, hipStream_t);
 extern "C" void qsa_conv_qkv_launch(const void*, long long, const float*, int,
@@ -133,6 +136,25 @@ extern "C" int qsa_rows_gemm_plan(int, int, int, int, int, int*);
 extern "C" void qsa_rows_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     float*, int, int, int, long long, int, int, int, hipStream_t);
 
+// Whether t [S, rows, cols] is a product of bf16 rows whose shares of K have not
+// been added (rows_parts)
+static bool is_shares(const Tensor& t, const Tensor& like, int64_t rows,
+                      int64_t cols) {
+  if (t.dim() != 3) return false;
+  TORCH_CHECK(t.scalar_type() == at::kFloat && t.is_contiguous() &&
+                  t.device() == like.device() && t.size(0) >= 1 &&
+                  t.size(1) == rows && t.size(2) == cols && cols % 8 == 0 &&
+                  like.scalar_type() == at::kBFloat16 && aligned(t, 16),
+              "shares [S, rows, cols], f32, of bf16 rows");
+  return true;
+}
+
+static Tensor add_shares(const Tensor& parts) {
+  Tensor sum = parts[0];
+  for (int64_t s = 1; s < parts.size(0); ++s) sum = sum + parts[s];
+  return sum.to(at::kBFloat16);
+}
+
 // res [T, W] f32 updated in place; returns norm(res) * w (+ b), or res itself
 // in y's storage type when w is not given
 Tensor residual_norm(Tensor res, OptTensor y, OptTensor table, OptTensor ids,
@@ -143,9 +165,13 @@ Tensor residual_norm(Tensor res, OptTensor y, OptTensor table, OptTensor ids,
   TORCH_CHECK(w || y, "norm weight or y");
   const long long T = res.size(0);
   const int W = (int)res.size(1);
-  const Tensor& like = w ? *w : *y;
+  const bool shares = y && y->dim() == 3;
+  const auto opts = w ? w->options()
+                      : y->options().dtype(shares ? at::kBFloat16
+                                                  : y->scalar_type());
+  auto out = torch::empty({T, (long long)W}, opts);
+  const Tensor& like = out;
   const int f32 = is_f32(like);
-  auto out = torch::empty({T, (long long)W}, like.options());
   if (T == 0) return out;
   bool v4 = W % 4 == 0;
   const int word = f32 ? 16 : 8;
@@ -166,7 +192,9 @@ Tensor residual_norm(Tensor res, OptTensor y, OptTensor table, OptTensor ids,
   long long ys = 0;
   int vocab = 0;
   const long long* ip = nullptr;
-  if (y) {
+  if (shares) {
+    is_shares(*y, like, T, W);
+  } else if (y) {
     CHK_SAME(*y, like); chk_rows(*y, "y");
     TORCH_CHECK(y->size(0) == T && y->size(1) == W, "y shape");
     yp = y->data_ptr(); ys = y->stride(0);
@@ -181,7 +209,12 @@ Tensor residual_norm(Tensor res, OptTensor y, OptTensor table, OptTensor ids,
     ip = reinterpret_cast<const long long*>(ids->data_ptr<int64_t>());
     v4 = v4 && aligned(*table, word);
   }
-  qsa_residual_norm_launch(res.data_ptr<float>(), yp, ys, pp, tp, ip,
+  if (shares && !v4)                   // rows that the kernel reads one by one
+    return residual_norm(res, add_shares(*y), table, ids, vec, w, b, eps, init,
+                         layer, post, tscale);
+  qsa_residual_norm_launch(res.data_ptr<float>(), yp, ys,
+                           shares ? y->data_ptr<float>() : nullptr,
+                           shares ? (int)y->size(0) : 0, pp, tp, ip,
                            (float)tscale, vp, wp, bp, out.data_ptr(), T, W,
                            vocab, (float)eps, init, layer, f32, v4,
                            cur_stream());
@@ -197,7 +230,8 @@ Tensor glu(Tensor gate, Tensor up, bool gelu) {
   if (rows == 0 || cols == 0) return out;
   const int v = cols % 8 == 0 && gate.stride(0) % 8 == 0 &&
                 up.stride(0) % 8 == 0 && aligned(gate, 16) && aligned(up, 16);
-  qsa_glu_launch(gate.data_ptr(), up.data_ptr(), nullptr, out.data_ptr(),
+  qsa_glu_launch(gate.data_ptr(), nullptr, 0, up.data_ptr(), nullptr,
+                 out.data_ptr(),
                  rows, cols, gate.stride(0), up.stride(0), 0, gelu,
                  is_f32(gate), v, cur_stream());
   return out;
@@ -206,23 +240,34 @@ Tensor glu(Tensor gate, Tensor up, bool gelu) {
 // act(gate [T, n]) * table[ids, col0 : col0 + n]
 Tensor glu_table(Tensor gate, Tensor table, Tensor ids, long col0,
                  bool gelu) {
-  CHK_DEV(gate); chk_rows(gate, "gate"); CHK_CONT(table); CHK_CONT(ids);
-  CHK_SAME(gate, table);
-  const long long rows = gate.size(0), cols = gate.size(1);
+  CHK_DEV(gate); CHK_CONT(table); CHK_CONT(ids);
+  const bool shares = gate.dim() == 3;
+  const long long rows = gate.size(shares ? 1 : 0);
+  const long long cols = gate.size(shares ? 2 : 1);
+  if (shares) {
+    is_shares(gate, table, rows, cols);
+  } else {
+    chk_rows(gate, "gate"); CHK_SAME(gate, table);
+  }
   TORCH_CHECK(ids.scalar_type() == at::kLong && ids.numel() == rows, "ids");
   TORCH_CHECK(table.dim() == 2 && col0 >= 0 && table.size(0) > 0 &&
                   col0 + cols <= table.size(1), "columns of the table");
-  auto out = torch::empty({rows, cols}, gate.options());
+  auto out = torch::empty({rows, cols}, table.options());
   if (rows == 0 || cols == 0) return out;
-  const int v = cols % 8 == 0 && gate.stride(0) % 8 == 0 && col0 % 8 == 0 &&
-                table.size(1) % 8 == 0 && aligned(gate, 16) &&
+  const int v = cols % 8 == 0 && (shares || gate.stride(0) % 8 == 0) &&
+                col0 % 8 == 0 && table.size(1) % 8 == 0 && aligned(gate, 16) &&
                 aligned(table, 16);
+  if (shares && !v)
+    return glu_table(add_shares(gate), table, ids, col0, gelu);
   const char* base = reinterpret_cast<const char*>(table.data_ptr()) +
                      col0 * table.element_size();
-  qsa_glu_launch(gate.data_ptr(), base,
+  qsa_glu_launch(shares ? nullptr : gate.data_ptr(),
+                 shares ? gate.data_ptr<float>() : nullptr,
+                 shares ? (int)gate.size(0) : 0, base,
                  reinterpret_cast<const long long*>(ids.data_ptr<int64_t>()),
-                 out.data_ptr(), rows, cols, gate.stride(0), table.size(1),
-                 table.size(0), gelu, is_f32(gate), v, cur_stream());
+                 out.data_ptr(), rows, cols, shares ? 0 : gate.stride(0),
+                 table.size(1), table.size(0), gelu, is_f32(table), v,
+                 cur_stream());
   return out;
 }
 
@@ -969,20 +1014,22 @@ bool rows_glu_ok(const Tensor& a, const Tensor& w) {
   return rows_gemm_rule(a, w, true);
 }
 
-static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act) {
+// parts: a product whose K is split may stay in its shares, [S, M, N] f32
+static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
+                            bool parts = false) {
   CHK_DEV(a); CHK_SAME(a, w);
   TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
               "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
   const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
   int S;
-  const int tile = qsa_rows_gemm_plan(M, N, K, act, 0, &S);
-  auto out = torch::empty({M, act ? N / 2 : N}, a.options());
-  Tensor part;
+  const int tile = qsa_rows_gemm_plan(M, N, K, act, parts, &S);
+  Tensor out, part;
   if (S > 1) part = torch::empty({S, M, N}, a.options().dtype(at::kFloat));
-  qsa_rows_gemm_launch(u16(a), u16(w), u16m(out),
+  if (S == 1 || !parts) out = torch::empty({M, act ? N / 2 : N}, a.options());
+  qsa_rows_gemm_launch(u16(a), u16(w), out.defined() ? u16m(out) : nullptr,
                        S > 1 ? part.data_ptr<float>() : nullptr, M, N, K,
                        a.stride(0), tile, S, act, cur_stream());
-  return out;
+  return out.defined() ? out : part;
 }
 
 // (tile, shares of K) that the rule in rows_gemm.hip takes
@@ -995,6 +1042,24 @@ std::tuple<int, int> rows_gemm_plan(int64_t M, int64_t N, int64_t K,
 
 // a @ w^T on W as it is stored
 Tensor rows_gemm(Tensor a, Tensor w) { return rows_gemm_run(a, w, 0); }
+
+// the same for a reader that adds shares: [M, N], or [S, M, N] in f32
+Tensor rows_parts(Tensor a, Tensor w) { return rows_gemm_run(a, w, 0, true); }
+
+// res [rows, W] bf16 <- res + the sum of shares [S, rows, W], in place; returns
+// rms norm of it times w
+Tensor rmsnorm_shares(Tensor parts, Tensor res, Tensor w, double eps) {
+  CHK_DEV(res); CHK_CONT(res); CHK_CONT(w); CHK_SAME(res, w);
+  const int64_t W = res.size(-1), rows = W ? res.numel() / W : 0;
+  TORCH_CHECK(is_shares(parts, res, rows, W) && w.numel() == W && W <= 8192 &&
+                  aligned(res, 16) && aligned(w, 16), "shares, W <= 8192");
+  auto out = torch::empty_like(res);
+  if (rows)
+    qsa_rmsnorm_shares_launch(parts.data_ptr<float>(), (int)parts.size(0),
+                              u16m(res), u16(w), u16m(out), rows, (int)W,
+                              (float)eps, cur_stream());
+  return out;
+}
 
 // act of the first half of a @ w^T's columns times the second
 Tensor rows_glu(Tensor a, Tensor w, bool gelu) {
@@ -1035,6 +1100,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "packed-weight decode GEMM (M <= 32)");
   m.def("rows_gemm", &rows_gemm, "GEMM of decode batches and short prompts");
   m.def("rows_gemm_ok", &rows_gemm_ok, "whether a product is rows_gemm's");
+  m.def("rows_parts", &rows_parts, "the same, shares of K left to the reader");
+  m.def("rmsnorm_shares", &rmsnorm_shares,
+        "residual add of such shares + RMSNorm (bf16)");
   m.def("rows_gemm_plan", &rows_gemm_plan, "tile and shares of a product");
   m.def("rows_glu", &rows_glu, "the same with the gated activation inside");
   m.def("rows_glu_ok", &rows_glu_ok, "whether a gated product is rows_glu's");

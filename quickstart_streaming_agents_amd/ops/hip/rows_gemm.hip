@@ -272,10 +272,8 @@ qsa_rows_sum(const float* __restrict__ part, bf16_t* __restrict__ C,
              long long n, int S) {
   const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= n) return;                  // n % 4 == 0
-  f32x4_v v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-  for (int s = 0; s < S; ++s)
-    v += *reinterpret_cast<const f32x4_v*>(part + s * n + i);
+  float v[4];
+  ld_shares<4>(part + i, n, S, v);
   *reinterpret_cast<uint2*>(C + i) =
       make_uint2(cvt_bf16x2(v[0], v[1]), cvt_bf16x2(v[2], v[3]));
 }

@@ -631,7 +631,53 @@ def test_rows_gemm_sizes_reach_every_tile():
     assert plain == set(range(13))
     gated = {lm_ext().rows_gemm_plan(m, n // 32 * 32, k, True)[0]
              for m, n, k in ROWS_SIZES}
-    assert len(gated) >= 9
+    assert gated == set(range(13)) - {0, 9}       # no pairs of column tiles
+
+
+@pytest.mark.parametrize("S", [2, 7, 16])
+@pytest.mark.parametrize("W", [8, 1032, 4096, 8200])
+def test_shares_meet_their_reader(S, W):
+    """Shares of a product give what the stored product gives, bit for bit."""
+    from quickstart_streaming_agents_amd.ops import ext
+    g, T = gen(S + W), 5
+    parts = rnd(g, S, T, W).to(DEV)
+    y = D.add_shares(parts)
+    w, post, table = (rnd(g, n, W, dtype=BF).to(DEV) for n in (1, 1, 9))
+    ids = torch.tensor([0, 8, 3, 3, 1], device=DEV)
+    res = rnd(g, T, W).to(DEV)
+    for kw in ({}, {"post": post[0]}, {"layer": False, "post": post[0]},
+               {"layer": False, "table": table, "ids": ids}, {"init": True}):
+        for weight in (w[0], None):
+            a, b = res.clone(), res.clone()
+            got = D.residual_norm(a, parts, weight, None, 1e-5, **kw)
+            want = D.residual_norm(b, y, weight, None, 1e-5, **kw)
+            assert torch.equal(a, b) and torch.equal(got, want)
+    for act in ("silu", "gelu"):
+        assert torch.equal(D.glu_table(parts, table, ids, 0, act),
+                           D.glu_table(y, table, ids, 0, act))
+    a, b = (res.to(BF) for _ in range(2))
+    got = D.rmsnorm_residual(parts, a, w[0], 1e-5)
+    want = ext().rmsnorm_residual(y, b, w[0], 1e-5)
+    assert torch.equal(a, b)
+    # sums of squares in another order: one place of bf16
+    close(got, want.cpu(), BF)
+    odd = torch.empty(W + 1, dtype=BF, device=DEV)[1:].copy_(w[0])
+    a, b = res.clone(), res.clone()
+    assert torch.equal(D.residual_norm(a, parts, odd, None, 1e-5),
+                       D.residual_norm(b, y, odd, None, 1e-5))
+
+
+def test_product_in_shares():
+    """What is left in shares adds up to the product."""
+    g = gen(3)
+    x, w = rnd(g, 100, 8192, dtype=BF).to(DEV), rnd(g, 512, 8192, dtype=BF)
+    w = w.to(DEV)
+    parts = D.linear_parts(x, w)
+    assert parts.dim() == 3 and parts.shape[0] > 1
+    a, b = x.double(), w.double()
+    bound = 2.0 ** -8 * (a @ b.T).abs() + \
+        8192 * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    assert ((D.add_shares(parts).double() - a @ b.T).abs() <= bound).all()
 
 
 def test_linear_of_rows_far_apart():
