@@ -10,7 +10,7 @@ well-distributed; the retrieval CONTRACT (dims, cosine, top-k) is what the
 pipelines rely on.
 
 On the GPU the tokens of a batch are rows without padding: the projections are
-ops/hip/short_gemm.hip's, the activation inside, and attention runs on the
+kernels of our own with the activation inside, and attention runs on the
 projection's rows as they are (ops/hip/encoder_attn.hip) — no padded bmm, no
 materialized score matrix.  The CPU path keeps a padded bmm + masked-softmax
 reference of the same semantics (GPU-vs-CPU parity test in
@@ -21,11 +21,13 @@ from __future__ import annotations
 
 from dataclasses import dataclass
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
 from ..ops import dispatch as D
 from ..vector.index import EMBED_DIM
+from .layers import ints_to_device
 from .tokenizer import BpeTokenizer
 
 
@@ -85,43 +87,40 @@ class EmbeddingEncoder:
         self._use_hip = str(device).startswith("cuda")
 
     def _linear(self, x: torch.Tensor, w: torch.Tensor,
-                glu: bool = False) -> torch.Tensor:
-        """x W^T, with glu silu(gate) * up of it, w = [gate; up] (GPU).  Short
-        K goes to a kernel of our own at any number of rows: at some it is
-        behind the library's as a kernel (1536 x 384, 8800 rows: 19.7 us, 17.4),
-        but a call with those products from the library above 3500 rows is
-        never faster (12 layers, 3848 rows 870 us here, 1130 with; 6396 1186,
-        1241; 7744 1263, 1403; 10,325 1579, 1577; 12,868 1801, 2032; 20,870
-        2709, 2722), as its kernels are uneven and its host path is 16 us a
-        product.  That also bounds few rows of longer K (384 x 1536: 10.9 us
-        of kernel at 400 rows, 7.6 in the library; at 8800, where kernels
-        count, 22.6 and 16.9)."""
+                glu: bool = False, parts: bool = False) -> torch.Tensor:
+        """x W^T (`parts`: for the residual's norm), with glu silu(gate) * up of it, w = [gate; up] (GPU).  Few
+        tiles are short_gemm's (ops/hip/short_gemm.hip: 384 x 512 at 400 rows
+        4.3 us, 4.5 in rows_gemm, 5.5 in the library), the others rows_gemm's:
+        at 8800 rows 1536 x 384 takes 17.0 us (short_gemm 20.7, the library
+        18.3), 3072 x 384 with the activation 32 (36, 72 with a pass of its
+        own), 384 x 512 8.0 (10.5, 10.7), 384 x 1536 14.6 (23.4, 17.2)."""
         n, k = w.shape
-        if w.dtype == torch.bfloat16 and k % 64 == 0 and n % 32 == 0 and \
-                (k <= 512 or x.shape[0] <= 2048):
+        if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
+                n % 32 == 0 and (k <= 512 or x.shape[0] <= 32) and \
+                -(-x.shape[0] // 32) * -(-n // 64) <= 192:
             return D.ext().short_gemm(x, w, glu)
+        if not glu:
+            return D.linear_parts(x, w) if parts else D.linear(x, w)
+        if D.glu_linear_ok(x, w):
+            return D.glu_linear(x, w, "silu", rounded=False)
         y = F.linear(x, w)
-        return D.swiglu(y[:, :n // 2], y[:, n // 2:]) if glu else y
+        return D.swiglu(y[:, :n // 2], y[:, n // 2:])
 
     # -- varlen attention plumbing (GPU path) ------------------------------
     QROWS = 64      # query tokens per attention block: one 16-row tile a wave
 
-    def _embed_rows(self, enc: list[list[int]]) -> torch.Tensor:
-        """Mean-pooled final states [n, hidden] f32 of the token lists, all
-        rows in one concatenation without padding."""
-        import numpy as np
-
-        from .layers import ints_to_device
+    def _embed_rows(self, ids: np.ndarray, lens: np.ndarray) -> torch.Tensor:
+        """Mean-pooled final states [n, hidden] f32 of texts whose tokens follow
+        each other in ids, all rows in one concatenation without padding."""
         c, dev = self.cfg, self.device
-        lens = np.array([len(x) for x in enc])
-        n = len(enc)
+        n = len(lens)
         off = np.cumsum(lens) - lens
         nqb = -(-lens // self.QROWS)
         qb_item = np.repeat(np.arange(n), nqb)
         qb_pos0 = (np.arange(int(nqb.sum()))
                    - (np.cumsum(nqb) - nqb)[qb_item]) * self.QROWS
         toks, qb_item, qb_pos0, off, lens_t = ints_to_device(
-            dev, np.concatenate(enc), qb_item, qb_pos0, off, lens)
+            dev, ids, qb_item, qb_pos0, off, lens)
         res = self.tok_embed.index_select(0, toks)
         mlp_out = None
         for Ly in self.layers:
@@ -133,10 +132,10 @@ class EmbeddingEncoder:
             attn = D.ext().encoder_attn(
                 self._linear(h, Ly["wqkv"]), self.rope_cos, self.rope_sin,
                 qb_item, qb_pos0, off, lens_t, c.n_heads, self.scale)
-            o = self._linear(attn, Ly["wo"])
+            o = self._linear(attn, Ly["wo"], parts=True)
             h = D.rmsnorm_residual(o, res, Ly["mlp_norm"], c.norm_eps)
             act = self._linear(h, Ly["wgu"], glu=True)
-            mlp_out = self._linear(act, Ly["wdown"])
+            mlp_out = self._linear(act, Ly["wdown"], parts=True)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm,
                                      c.norm_eps)
         return D.ext().mean_rows(final_h, off, lens_t)
@@ -202,17 +201,17 @@ class EmbeddingEncoder:
 
     @torch.no_grad()
     def embed_batch(self, texts: list[str]):
-        import numpy as np
         if not texts:
             return np.zeros((0, self.cfg.out_dim), dtype=np.float32)
         c = self.cfg
-        enc = [self.tokenizer.encode(t)[: c.max_pos] or [BpeTokenizer.BOS]
-               for t in texts]
+        ids, lens = self.tokenizer.encode_batch(list(texts), c.max_pos)
         # mean over the tokens, project, L2-normalize
         from ..ops import have_ext
         if self._use_hip and have_ext():
-            out = self._linear(self._embed_rows(enc).to(self.dtype), self.proj)
+            out = self._linear(self._embed_rows(ids, lens).to(self.dtype),
+                               self.proj)
         else:
+            enc = [x.tolist() for x in np.split(ids, np.cumsum(lens)[:-1])]
             out = F.linear(self._embed_padded(enc).to(self.dtype), self.proj)
         out = out.float()
         out = out / out.norm(dim=-1, keepdim=True).clamp(min=1e-9)

@@ -21,6 +21,10 @@ import os
 import re
 from functools import lru_cache
 
+import numpy as np
+
+from ..ops import ext, have_ext
+
 _SPLIT = re.compile(r"[A-Za-z0-9_$]+|[^\sA-Za-z0-9_]")
 
 
@@ -99,6 +103,11 @@ class BpeTokenizer:
             self._sym_bytes.append(self._sym_bytes[a] + self._sym_bytes[b])
         self._special_re = re.compile(
             "(" + "|".join(re.escape(s) for s in self.specials) + ")")
+        # the same in native code, where it is built (ops/hip/bpe.cpp)
+        self._native = None
+        if have_ext() and all(self.specials):
+            self._native = ext().Bpe(merges, list(self.specials.items()),
+                                     self._BYTE0)
 
     @lru_cache(maxsize=65536)
     def _bpe_word(self, word: str) -> tuple[int, ...]:
@@ -116,6 +125,21 @@ class BpeTokenizer:
         return tuple(s + self._BYTE0 for s in syms)
 
     def encode(self, text: str, bos: bool = True) -> list[int]:
+        if self._native is not None:
+            return self._native.encode(text or "", self.BOS if bos else -1)
+        return self._encode(text, bos)
+
+    def encode_batch(self, texts: list[str], longest: int):
+        """At most `longest` tokens of every text behind BOS: all of them in one
+        array, and how many each text has."""
+        if self._native is not None:
+            return self._native.encode_batch([t or "" for t in texts],
+                                             self.BOS, longest)
+        enc = [self._encode(t, True)[:longest] for t in texts]
+        return (np.array([i for x in enc for i in x], dtype=np.int32),
+                np.array([len(x) for x in enc], dtype=np.int64))
+
+    def _encode(self, text: str, bos: bool) -> list[int]:
         ids = [self.BOS] if bos else []
         for part in self._special_re.split(text or ""):
             if not part:

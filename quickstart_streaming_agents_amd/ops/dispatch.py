@@ -247,9 +247,11 @@ def glu_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def glu_linear(x: torch.Tensor, w: torch.Tensor,
-               act: str = "silu") -> torch.Tensor:
-    """act(x @ W_gate^T) * (x @ W_up^T) of W = [gate; up], in one kernel."""
-    return lm_ext().rows_glu(x, w, act == "gelu")
+               act: str = "silu", rounded: bool = True) -> torch.Tensor:
+    """act(x @ W_gate^T) * (x @ W_up^T) of W = [gate; up], in one kernel; with
+    `rounded` of the products as linear() would store them, without (silu only)
+    of their f32 sums."""
+    return lm_ext().rows_glu(x, w, act == "gelu", rounded)
 
 
 def skinny_linear(x: torch.Tensor, wf: torch.Tensor, n: int,

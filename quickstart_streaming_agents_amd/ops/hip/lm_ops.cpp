@@ -1061,9 +1061,11 @@ Tensor rmsnorm_shares(Tensor parts, Tensor res, Tensor w, double eps) {
   return out;
 }
 
-// act of the first half of a @ w^T's columns times the second
-Tensor rows_glu(Tensor a, Tensor w, bool gelu) {
-  return rows_gemm_run(a, w, gelu ? 2 : 1);
+// act of the first half of a @ w^T's columns times the second, of the products
+// as they would be stored or (silu) of their sums
+Tensor rows_glu(Tensor a, Tensor w, bool gelu, bool rounded) {
+  TORCH_CHECK(rounded || !gelu, "gelu of the stored products only");
+  return rows_gemm_run(a, w, gelu ? 2 : rounded ? 1 : 3);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {

@@ -129,6 +129,7 @@ extern "C" void qsa_window_agg_launch(const long long*, const int*,
 extern "C" long long qsa_window_workspace(long long, long long, long long,
                                           long long);
 void register_avro(pybind11::module_&);  // avro_codec.cpp
+void register_bpe(pybind11::module_&);   // bpe.cpp
 extern "C" void qsa_anomaly_batch_launch(const float*, const int*, float*,
                                          float*, int*, int, int, int,
                                          hipStream_t);
@@ -885,4 +886,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("window_agg", &window_agg, "segmented (key, window) count/sum");
   m.def("anomaly_batch", &anomaly_batch, "batched AR+ridge anomaly scorer");
   register_avro(m);
+  register_bpe(m);
 }

@@ -10,7 +10,7 @@
 // shares of K are chosen by what they should take (qsa_rows_gemm_plan); a tile's
 // LDS traffic per product falls with its sides, which is why the large ones are
 // the fast ones where the chip is full.  The activation
-// is that of the rounded products, so either way gives the same.
+// is applied to the sums, rounded first where a stored product was read before.
 // us, library -> here (sums of shares included, weights from memory):
 //   rows            33            64           128           192           768
 //   6144 x 4096  17.4 -> 15.6  17.9 -> 16.9  25.6 -> 21.0  34.1 -> 25.3  49 -> 47
@@ -39,7 +39,8 @@ struct RowsArgs {
   unsigned int lda;                    // elements
 };
 
-enum { ACT_NONE = 0, ACT_SILU = 1, ACT_GELU = 2 };
+// of the products as they are stored, or of their sums
+enum { ACT_NONE = 0, ACT_SILU = 1, ACT_GELU = 2, ACT_SILU_SUM = 3 };
 
 __device__ __forceinline__ float as_bf16(float v) {
   return bf16_to_f32(cvt_bf16(v));
@@ -241,11 +242,16 @@ qsa_rows_gemm(RowsArgs p) {
 #pragma unroll
     for (int j = 0; j < NT; j += ACT ? 2 : 1) {
       f32x4_v v = acc[i][j];
-      if constexpr (ACT != ACT_NONE)   // of the products as they are stored
+      if constexpr (ACT == ACT_SILU_SUM) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[r] = act_f<false, QSA_ACT_SILU>(v[r]) * acc[i][j + 1][r];
+      } else if constexpr (ACT != ACT_NONE) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           v[r] = act_f<false, ACT - 1>(as_bf16(v[r])) *
                  as_bf16(acc[i][j + 1][r]);
+      }
       *reinterpret_cast<uint2*>(o + (i * 16 + col) * OP +
                                 (ACT ? j / 2 : j) * 16 + hi * 4) =
           make_uint2(cvt_bf16x2(v[0], v[1]), cvt_bf16x2(v[2], v[3]));
@@ -289,6 +295,7 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
   if constexpr (BN / WN / 16 % 2 == 0) {
     if (act == ACT_SILU) { QSA_RG(ACT_SILU); return; }
     if (act == ACT_GELU) { QSA_RG(ACT_GELU); return; }
+    if (act == ACT_SILU_SUM) { QSA_RG(ACT_SILU_SUM); return; }
   }
   QSA_RG(ACT_NONE);
 #undef QSA_RG
@@ -349,8 +356,8 @@ extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
   return tile;
 }
 
-// act: 0, or 1 silu / 2 gelu of the first half of W's rows times the second (one
-// share only).  With part and S > 1 and no C the shares are left to the caller.
+// act: 0, or an ACT_ of the first half of W's rows times the second (one share
+// only).  With part and S > 1 and no C the shares are left to the caller.
 extern "C" void qsa_rows_gemm_launch(const bf16_t* A, const bf16_t* W,
                                      bf16_t* C, float* part, int M, int N,
                                      int K, long long lda, int tile, int S,

@@ -1,22 +1,16 @@
 // GEMM of a short K for CDNA4 (gfx950): C[M,N] = A[M,K] @ W[N,K]^T, bf16 with f32
 // sums, and with GLU silu(gate) * up of it, W's rows being [gate; up]: the
-// encoder's projections (K 384 and 512, and 1536 for few rows).
+// encoder's projections of few rows.
 //
-// With a few steps of K a product is over before a deep pipeline is full; its
-// reads and writes and, for few rows, the host's way to a library's kernel (20
-// us a call, 4 here) count as much as the matrix cores.  So: tiles by the number
-// of blocks they leave, K in steps of 64 through two halves of LDS with the next
-// one in registers, whole 128-byte lines of every operand, a block row's columns
-// on one die, results through LDS to whole lines, and the gate's columns beside
-// the up's in a wave, so that the activation costs no pass over memory.
-// us as kernels, library -> here, at 400 / 1600 / 4000 / 8800 / 16000 rows:
-//   1536 x 384  6.6 / 9.3 / 12.2 / 17.4 / 34.0 -> 5.3 / 7.2 / 12.3 / 19.7 / 29.1
-//   384 x 512   6.7 / 7.6 /  9.6 / 10.8 / 14.6 -> 5.3 / 5.7 /  6.7 / 10.3 / 15.3
-//   384 x 1536  7.6 / 9.6 / 13.1 / 16.9 / 23.4 -> 10.9 / 11.7 / 13.6 / 22.6 / 34
-//   3072 x 384 with the activation, there a pass of its own
-//               11.3 / 18.4 / 31.9 / 71 / 72.6 -> 6.3 / 11.3 / 17.9 / 34.1 / 56.9
-// The library is uneven in the rows (1536 x 384: 14.3 at 5470, 22.1 at 5817, 16.5
-// at 8246, 29 to 42 from 11000 to 12500).
+// With a few steps of K a product is over before a deep pipeline is full, and few
+// tiles leave nothing to overlap with, so: tiles of 32 x 64, K in steps of 64
+// through two halves of LDS with the next one in registers, whole 128-byte lines
+// of every operand, a block row's columns on one die, results through LDS to
+// whole lines, and the gate's columns beside the up's in a wave, so that the
+// activation costs no pass over memory.  Larger products are rows_gemm.hip's.
+// us, library / rows_gemm -> here:
+//   384 x 512  at 100 / 400 / 1000 rows 5.4 / 5.5 / 6.2, 4.5 -> 4.2 / 4.3 / 4.4
+//   1536 x 384 at 40 rows 5.0, 4.1 -> 3.8;  512 x 256 at 700 5.1, 4.0 -> 3.6
 #include "lm_common.h"
 
 struct ShortArgs {
@@ -175,19 +169,10 @@ static void short_go(ShortArgs p, int glu, hipStream_t st) {
                        p);
 }
 
-// Tiles of 128 x 128 once two rounds of blocks are left, 64 x 64 while they
-// make half a round, 32 x 64 below (384 x 512 at 400 rows: 8.2 / 4.5 / 3.7 us;
-// 1536 x 384 at 1600: 7.9 / 6.8 / 8.0, at 8800: 20.9 / 23.0 / 28.4).
 extern "C" void qsa_short_gemm_launch(const bf16_t* A, const bf16_t* W,
                                       bf16_t* C, int M, int N, int K,
                                       long long lda, int glu,
                                       hipStream_t st) {
   if (M == 0) return;
-  const ShortArgs p{A, W, C, M, N, K, 0, lda};
-  auto blocks = [&](int b) {
-    return (long long)((M + b - 1) / b) * ((N + b - 1) / b);
-  };
-  if (blocks(128) >= 512) short_go<4, 4>(p, glu, st);
-  else if (blocks(64) >= 128) short_go<2, 2>(p, glu, st);
-  else short_go<1, 2>(p, glu, st);
+  short_go<1, 2>({A, W, C, M, N, K, 0, lda}, glu, st);
 }

@@ -33,7 +33,7 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
 # Mixtral / encoder kernels.  qsa_lm_hip: the mixer decoders' kernels; it
 # builds alone in about a minute when that is all a program needs.
 MODULES = {
-    "qsa_hip": ["ops.cpp", "avro_codec.cpp", "elementwise.hip",
+    "qsa_hip": ["ops.cpp", "avro_codec.cpp", "bpe.cpp", "elementwise.hip",
                 "paged_attn.hip", "skinny_gemm.hip", "skinny_gemm_fp8.hip",
                 "hash_join.hip", "gemm_fp8_batch.hip", "topk_cosine.hip",
                 "streaming.hip", "encoder_attn.hip", "short_gemm.hip"],

@@ -602,21 +602,23 @@ def test_rows_gemm_tiles(M, N, K):
     assert ((got - a @ b.T).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("act", ["silu", "gelu", "silu of sums"])
 @pytest.mark.parametrize("M,N,K", ROWS_SIZES)
 def test_rows_glu(M, N, K, act):
-    """Gate and up are rounded to bf16 after the product's f32 error, e in all,
-    and both activations have a slope of at most 1.13; __expf and the division
+    """Gate and up are rounded to bf16 (but for sums) after the product's f32
+    error, e in all, and both activations have a slope of at most 1.13; __expf and the division
     are good to some 2^-20, the result is rounded to bf16."""
     N = N // 32 * 32
     g = gen(M + N)
     x = rnd(g, M, K + 24, dtype=BF)[:, 8:K + 8].to(DEV)
     w = rnd(g, N, K, dtype=BF, scale=K ** -0.5).to(DEV)
     stale(M, N // 2)
-    got = D.glu_linear(x, w, act).double()
+    sums = act == "silu of sums"
+    act = act.split()[0]
+    got = D.glu_linear(x, w, act, not sums).double()
     a, b = x.double(), w.double()
     e = K * 2.0 ** -24 * (a.abs() @ b.abs().T) + 2.0 ** -20 \
-        + 2.0 ** -8 * (a @ b.T).abs()
+        + (0.0 if sums else 2.0 ** -8) * (a @ b.T).abs()
     (p, q), (ep, eq) = (a @ b.T).chunk(2, 1), e.chunk(2, 1)
     f = torch.nn.functional.silu(p) if act == "silu" else \
         torch.nn.functional.gelu(p, approximate="tanh")
