@@ -623,6 +623,14 @@ def topk_cosine(queries: torch.Tensor, docs: torch.Tensor, k: int):
     return topk_cosine_ref(queries, docs, k)
 
 
+def topk_cosine_packed(queries: torch.Tensor, docs: torch.Tensor, k: int):
+    """topk_cosine as one tensor [2, Q, k]: the scores' bits, the documents."""
+    if _cuda(queries):
+        return ext().topk_cosine_packed(queries, docs, k)
+    scores, ids = topk_cosine(queries, docs, k)
+    return torch.stack([scores.contiguous().view(torch.int32), ids])
+
+
 def window_agg(ts: torch.Tensor, key: torch.Tensor,
                value: torch.Tensor | None, t0: int, win_ms: int, nwin: int,
                nkeys: int):

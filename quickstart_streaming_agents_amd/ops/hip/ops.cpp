@@ -745,8 +745,10 @@ torch::Tensor encoder_attn(torch::Tensor qkv, torch::Tensor cos_t,
   return out;
 }
 
-std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
-                                       torch::Tensor docs, long k) {
+// [2, Q, k]: scores, as the bits of floats, and documents; one buffer, so that a
+// caller on the host waits for one copy.
+torch::Tensor topk_cosine_packed(torch::Tensor queries, torch::Tensor docs,
+                                 long k) {
   CHK_DEV(queries); CHK_CONT(queries); CHK_F32(queries); CHK_F32(docs);
   CHK_CONT(docs);
   const int Q = queries.size(0), D = queries.size(1), N = docs.size(0);
@@ -754,30 +756,34 @@ std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
   TORCH_CHECK(k >= 1 && k <= 16, "k in [1,16]");
   const int per = qsa_topk_block_docs(Q, N);
   int lists = (N + per - 1) / per;
-  auto opts_f = queries.options();
-  auto opts_i = queries.options().dtype(at::kInt);
-  if (Q == 0)
-    return {torch::empty({Q, k}, opts_f), torch::empty({Q, k}, opts_i)};
-  auto s = torch::empty({Q, lists, k}, opts_f);
-  auto i = torch::empty({Q, lists, k}, opts_i);
+  auto lists_of = [&](long n) {
+    return torch::empty({2, Q, n * k}, queries.options().dtype(at::kInt));
+  };
+  auto from = lists_of(lists);
+  if (Q == 0) return torch::empty({2, 0, k}, from.options());
+  auto scores = [&](torch::Tensor& t) {
+    return reinterpret_cast<float*>(t.data_ptr<int>());
+  };
+  auto ids = [](torch::Tensor& t) { return t.data_ptr<int>() + t.stride(0); };
   qsa_topk_scan_launch(queries.data_ptr<float>(), docs.data_ptr<float>(),
-                       s.data_ptr<float>(), i.data_ptr<int>(), Q, N, D, (int)k,
-                       lists, cur_stream());
+                       scores(from), ids(from), Q, N, D, (int)k, lists,
+                       cur_stream());
   // a single list is the result (5 rows, k = 5: 17.5 us with the merge)
-  if (lists == 1) return {s.view({Q, k}), i.view({Q, k})};
-  do {
+  while (lists != 1) {
     const int groups = qsa_topk_groups(lists);
-    auto to_s = groups > 1 ? torch::empty({Q, groups, k}, opts_f)
-                           : torch::empty({Q, k}, opts_f);
-    auto to_i = torch::empty(to_s.sizes(), opts_i);
-    qsa_topk_merge_launch(s.data_ptr<float>(), i.data_ptr<int>(),
-                          to_s.data_ptr<float>(), to_i.data_ptr<int>(), Q,
+    auto to = lists_of(groups);
+    qsa_topk_merge_launch(scores(from), ids(from), scores(to), ids(to), Q,
                           lists, (int)k, cur_stream());
-    s = to_s;
-    i = to_i;
+    from = to;
     lists = groups;
-  } while (lists > 1);
-  return {s, i};
+  }
+  return from;
+}
+
+std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
+                                       torch::Tensor docs, long k) {
+  auto both = topk_cosine_packed(queries, docs, k);
+  return {both[0].view(at::kFloat), both[1]};
 }
 
 std::vector<torch::Tensor> window_agg(torch::Tensor ts, torch::Tensor key,
@@ -878,6 +884,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fp8-weight decode GEMM added to the residual stream");
   m.def("embed_rows", &embed_rows,
         "a step's first rows and their sums of squares");
+  m.def("topk_cosine_packed", &topk_cosine_packed,
+        "the same, scores and documents in one buffer");
   m.def("topk_cosine", &topk_cosine, "exact cosine top-k over the HBM index");
   m.def("hash_build", &hash_build,
         "build latest-per-key hash table from (keys, event ts)");

@@ -4,15 +4,15 @@
 // 1536-dim cosine, k=3, numCandidates=500) with an exact scan of the
 // normalized index matrix in HBM.
 //
-// Bound by one read of the index.  A block scores 16*T documents against 16
+// Bound by one read of the index.  A block scores 16*T documents against 16*QT
 // queries at once on the f32 matrix cores (16x16x4, f32 products and sums), so
-// up to 16 queries (32 with QT = 2) cost one read of the matrix; its four waves
-// split the vector dimension and meet in LDS, so a block needs no query staging
-// and small indexes still spread over the chip.  T = 4 keeps 8 KiB of documents
-// per wave in flight while the previous step multiplies; T = 1 serves indexes
-// whose 64-document blocks would leave CUs idle.
-// 100,000 x 1536, 8 queries, k = 3: 4490 us with one dot product per wave and
-// a pass per query, before; 145 us here (4.2 TB/s), and 7 us of merge.
+// up to 16 queries cost one read of the matrix; its four waves split the vector
+// dimension and meet in LDS, so small indexes still spread over the chip.  T = 4
+// keeps 8 KiB of documents per wave on their way while the previous step
+// multiplies; T = 1 serves indexes whose 64-document blocks would leave CUs idle.
+// 100,000 x 1536, k = 3: 8 queries 146 us with rows loaded straight into the
+// matrix cores' layout, 115 through LDS (5.3 TB/s), and 7 of merge; 32 queries
+// 200 and 136; 10,000 documents, 8 queries 19.5 and 14.7.
 //
 // Results: scores > -2 in descending order, equal scores by ascending
 // document; what k asks for beyond them is (-2, -1).  NaN scores never enter.
@@ -25,105 +25,15 @@ __device__ __forceinline__ bool qsa_better(float s, int i, float t, int j) {
   return s > t || (s == t && i < j);
 }
 
-// floats k..k+7 of a row; what lies beyond D is zero
-template <bool VEC>
-__device__ __forceinline__ void qsa_row8(const float* __restrict__ row, int k,
-                                         int D, float* v) {
-  if constexpr (VEC) {                 // D % 4 == 0, rows 16-byte aligned
-    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4_t a = *reinterpret_cast<const f32x4_t*>(row + (k < D ? k : 0));
-    f32x4_t b = *reinterpret_cast<const f32x4_t*>(row +
-                                                  (k + 4 < D ? k + 4 : 0));
-    if (k >= D) a = zero;
-    if (k + 4 >= D) b = zero;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[e] = a[e];
-      v[4 + e] = b[e];
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = row[k + e < D ? k + e : 0];
-      v[e] = k + e < D ? x : 0.f;
-    }
-  }
-}
-
-template <int T, int QT, bool VEC>     // 16*T documents, 16*QT queries
-__global__ void __launch_bounds__(256, 2)
-qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
-              const float* __restrict__ docs,     // [N, D] L2-normalized
-              float* __restrict__ cand_scores,    // [Q, nblk, k]
-              int* __restrict__ cand_ids,         // [Q, nblk, k]
-              int Qn, int N, int D, int k) {
-  __shared__ float part[4][16 * T][17];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+// The best k of a block's 16*T documents for each of its queries, from its four
+// waves' sums; `part` is [4][16*T][17].
+template <int T, int QT>
+__device__ __forceinline__ void qsa_topk_candidates(
+    float (*part)[16 * T][17], const double (&total)[T][QT][4], int doc0,
+    int q0, float* __restrict__ cand_scores, int* __restrict__ cand_ids, int Qn,
+    int N, int k) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, hi = lane >> 4;
-  const int doc0 = blockIdx.x * 16 * T, q0 = blockIdx.y * 16 * QT;
-
-  // rows beyond the end shadow the last one; nothing of theirs is kept
-  const float* qrow[QT];
-#pragma unroll
-  for (int u = 0; u < QT; ++u)
-    qrow[u] = queries + (long long)min(q0 + u * 16 + col, Qn - 1) * D;
-  const float* drow[T];
-#pragma unroll
-  for (int t = 0; t < T; ++t)
-    drow[t] = docs + (long long)min(doc0 + t * 16 + col, N - 1) * D;
-
-  double total[T][QT][4];
-#pragma unroll
-  for (int t = 0; t < T; ++t)
-#pragma unroll
-    for (int u = 0; u < QT; ++u)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) total[t][u][r] = 0.0;
-
-  const int steps = (D + 31) / 32;     // 32 floats of every row, 8 per lane
-  float qn[QT][8], dn[T][8];
-  auto fetch = [&](int s) {
-    const int kk = s * 32 + hi * 8;
-#pragma unroll
-    for (int u = 0; u < QT; ++u) qsa_row8<VEC>(qrow[u], kk, D, qn[u]);
-#pragma unroll
-    for (int t = 0; t < T; ++t) qsa_row8<VEC>(drow[t], kk, D, dn[t]);
-  };
-  if (wave < steps) fetch(wave);
-  for (int s = wave; s < steps; s += 4) {
-    float qc[QT][8], dc[T][8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-#pragma unroll
-      for (int u = 0; u < QT; ++u) qc[u][e] = qn[u][e];
-#pragma unroll
-      for (int t = 0; t < T; ++t) dc[t][e] = dn[t][e];
-    }
-    if (s + 4 < steps) fetch(s + 4);
-    // sums of 32 products, added up in f64: one f32 chain over the row would
-    // double the rounding of a score
-    f32x4_t acc[T][QT];
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-      for (int u = 0; u < QT; ++u) acc[t][u] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-#pragma unroll
-      for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int u = 0; u < QT; ++u)
-          acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              dc[t][e], qc[u][e], acc[t][u], 0, 0, 0);
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-      for (int u = 0; u < QT; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) total[t][u][r] += (double)acc[t][u][r];
-  }
-
 #pragma unroll
   for (int u = 0; u < QT; ++u) {       // 16 queries at a time
     if (u) __syncthreads();
@@ -176,11 +86,209 @@ qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
   }
 }
 
+// sums of 32 products, added up in f64: one f32 chain over the row would double
+// the rounding of a score
+template <int T, int QT>
+__device__ __forceinline__ void qsa_topk_step(const float (&dc)[T][8],
+                                              const float (&qc)[QT][8],
+                                              double (&total)[T][QT][4]) {
+  f32x4_t acc[T][QT];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int u = 0; u < QT; ++u) acc[t][u] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+        acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            dc[t][e], qc[u][e], acc[t][u], 0, 0, 0);
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int u = 0; u < QT; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) total[t][u][r] += (double)acc[t][u][r];
+}
+
+// numbers k..k+7 of a row; what lies beyond D is zero
+__device__ __forceinline__ void qsa_row8(const float* __restrict__ row, int k,
+                                         int D, float* v) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x = row[k + e < D ? k + e : 0];
+    v[e] = k + e < D ? x : 0.f;
+  }
+}
+
+// waits until at most N loads of the wave are on their way
+template <int N>
+__device__ __forceinline__ void qsa_topk_wait() {
+  static_assert(N < 64, "the counter's range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | N >> 4 << 14 | 7 << 4 | 15 << 8);
+  asm volatile("" ::: "memory");
+}
+
+// Rows of whole 16-byte pieces (D % 4 == 0, aligned).  32 numbers of every row,
+// queries and documents, go straight to the wave's LDS, 8 rows of 128 bytes per
+// load: read into registers in the matrix cores' layout, the lanes of one load
+// touch 16 rows, which the address unit takes four times as long for.  The next
+// 32 are on their way while these multiply; no wave waits for another.
+template <int T, int QT>               // 16*T documents, 16*QT queries
+__global__ void __launch_bounds__(256, T + QT <= 2 ? 4 : T + QT <= 3 ? 3 : 1)
+qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
+              const float* __restrict__ docs,     // [N, D] L2-normalized
+              float* __restrict__ cand_scores,    // [Q, nblk, k]
+              int* __restrict__ cand_ids,         // [Q, nblk, k]
+              int Qn, int N, int D, int k) {
+  constexpr int ROWS = 16 * (T + QT), LOADS = ROWS / 8, STAGE = ROWS * 32;
+  constexpr int RING = 4 * 2 * STAGE, PART = 4 * 16 * T * 17;
+  __shared__ __attribute__((aligned(16))) float lds[RING > PART ? RING : PART];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, hi = lane >> 4;
+  const int doc0 = blockIdx.x * 16 * T, q0 = blockIdx.y * 16 * QT;
+
+  // Rows beyond the end shadow the last one; nothing of theirs is kept.  A
+  // row's eight 16-byte pieces are exchanged by its number, which spreads the
+  // reads below over the banks.
+  const float* row[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = i * 8 + (lane >> 3);
+    row[i] = (i < 2 * T
+                  ? docs + (long long)min(doc0 + r, N - 1) * D
+                  : queries + (long long)min(q0 + r - 16 * T, Qn - 1) * D) +
+             ((lane & 7) ^ (r >> 1 & 7)) * 4;
+  }
+
+  double total[T][QT][4];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int u = 0; u < QT; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) total[t][u][r] = 0.0;
+
+  const int steps = D / 32;            // whole ones
+  float* ring = lds + wave * 2 * STAGE;
+  auto fetch = [&](int s, int at) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(row[i] + s * 32),
+          (__attribute__((address_space(3))) void*)(ring + at * STAGE +
+                                                    i * 256),
+          16, 0, 0);
+  };
+  float dc[T][8], qc[QT][8];
+  int at = 0;
+  if (wave < steps) fetch(wave, 0);
+  for (int s = wave; s < steps; s += 4, at ^= 1) {
+    if (s + 4 < steps) {
+      fetch(s + 4, at ^ 1);
+      qsa_topk_wait<LOADS>();
+    } else {
+      qsa_topk_wait<0>();
+    }
+    const float* tile = ring + at * STAGE + col * 32;
+    auto take = [&](int i, float* v) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(
+            tile + i * 512 + ((hi * 2 + h) ^ (col >> 1)) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[h * 4 + e] = x[e];
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < T; ++t) take(t, dc[t]);
+#pragma unroll
+    for (int u = 0; u < QT; ++u) take(T + u, qc[u]);
+    qsa_topk_step<T, QT>(dc, qc, total);
+    // the reads are done before the stage is written again
+    __builtin_amdgcn_s_waitcnt(0xc07f);            // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+  }
+  if (steps * 32 < D && (steps & 3) == wave) {     // the last, part of a step
+    const int kk = steps * 32 + hi * 8;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      qsa_row8(docs + (long long)min(doc0 + t * 16 + col, N - 1) * D, kk, D,
+               dc[t]);
+#pragma unroll
+    for (int u = 0; u < QT; ++u)
+      qsa_row8(queries + (long long)min(q0 + u * 16 + col, Qn - 1) * D, kk, D,
+               qc[u]);
+    qsa_topk_step<T, QT>(dc, qc, total);
+  }
+  __syncthreads();                     // every wave has read its last stage
+  qsa_topk_candidates<T, QT>(reinterpret_cast<float (*)[16 * T][17]>(lds),
+                             total, doc0, q0, cand_scores, cand_ids, Qn, N, k);
+}
+
+// The same for any other D and alignment, number by number.
+template <int T, int QT>
+__global__ void __launch_bounds__(256, 2)
+qsa_topk_scan_any(const float* __restrict__ queries,
+                  const float* __restrict__ docs,
+                  float* __restrict__ cand_scores, int* __restrict__ cand_ids,
+                  int Qn, int N, int D, int k) {
+  __shared__ float part[4][16 * T][17];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, hi = lane >> 4;
+  const int doc0 = blockIdx.x * 16 * T, q0 = blockIdx.y * 16 * QT;
+
+  const float* qrow[QT];
+#pragma unroll
+  for (int u = 0; u < QT; ++u)
+    qrow[u] = queries + (long long)min(q0 + u * 16 + col, Qn - 1) * D;
+  const float* drow[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    drow[t] = docs + (long long)min(doc0 + t * 16 + col, N - 1) * D;
+
+  double total[T][QT][4];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int u = 0; u < QT; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) total[t][u][r] = 0.0;
+
+  const int steps = (D + 31) / 32;     // 32 floats of every row, 8 per lane
+  float qn[QT][8], dn[T][8];
+  auto fetch = [&](int s) {
+#pragma unroll
+    for (int u = 0; u < QT; ++u) qsa_row8(qrow[u], s * 32 + hi * 8, D, qn[u]);
+#pragma unroll
+    for (int t = 0; t < T; ++t) qsa_row8(drow[t], s * 32 + hi * 8, D, dn[t]);
+  };
+  if (wave < steps) fetch(wave);
+  for (int s = wave; s < steps; s += 4) {
+    float qc[QT][8], dc[T][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+      for (int u = 0; u < QT; ++u) qc[u][e] = qn[u][e];
+#pragma unroll
+      for (int t = 0; t < T; ++t) dc[t][e] = dn[t][e];
+    }
+    if (s + 4 < steps) fetch(s + 4);
+    qsa_topk_step<T, QT>(dc, qc, total);
+  }
+  qsa_topk_candidates<T, QT>(part, total, doc0, q0, cand_scores, cand_ids, Qn,
+                             N, k);
+}
+
 // A block per query and group of lists: k rounds, each the best candidate behind
 // the last one.  Lists are sorted, so a thread keeps the heads of HEADS of them
 // and a round compares heads only.  A block has room for 4096 heads; what more
-// lists there are (indexes beyond 262,144 documents, 131,072 with 17 and more
-// queries) form groups, whose results are merged in turn.  Going through the
+// lists there are (indexes beyond 262,144 documents, 196,608 or 131,072 with 17
+// and more queries) form groups, whose results are merged in turn.  Going through the
 // lists beyond 4096 in every round instead cost 2.6 of 4.1 ms for a million
 // documents, 16 queries and k = 16.
 #define QSA_MERGE_THREADS 512
@@ -260,11 +368,22 @@ qsa_topk_merge(const float* __restrict__ cand_scores,  // [Q, all, k]
   }
 }
 
-// Documents per block: 16 for small indexes; 64 as soon as that gives every CU
-// two blocks, or 32 beside twice the queries (17 and more of them: 32 queries
-// in one read of the index, 222 us where two reads took 296).
+// A block: 16 documents times the first digit, 16 queries times the second.  Up
+// to 16 queries: 16 documents for small indexes, 64 as soon as that gives every
+// CU two blocks.  More share a read of the index, 32 queries beside 48 documents
+// or 48 beside 32, once that fills the CUs (us at 1536, blocks of 16 documents
+// and queries / these: 24 queries of 6000 documents 15.7 / 19.3, 10,000 22.4 /
+// 20.6, 100,000 248 / 136; 64 of 3000 14.7 / 20.1, 6000 25.5 / 21.0).  33 to 48
+// queries are one read where 32 at a time take two (100,000: 195 and 269).
+static int qsa_topk_tile(long long Q, long long N) {
+  if (Q <= 16) return N < 64 * 512 ? 11 : 41;
+  if ((Q + 31) / 32 * N < 8192) return 11;
+  return Q > 32 && Q <= 48 ? 23 : 32;
+}
+
+// Documents per block.
 extern "C" int qsa_topk_block_docs(long long Q, long long N) {
-  return N < 64 * 512 ? 16 : Q > 16 ? 32 : 64;
+  return qsa_topk_tile(Q, N) / 10 * 16;
 }
 
 extern "C" void qsa_topk_scan_launch(const float* queries, const float* docs,
@@ -279,18 +398,19 @@ extern "C" void qsa_topk_scan_launch(const float* queries, const float* docs,
   {                                                                          \
     const dim3 grid(nblk, (Q + 16 * QT - 1) / (16 * QT));                    \
     if (vec)                                                                 \
-      hipLaunchKernelGGL((qsa_topk_scan<T, QT, true>), grid, dim3(256), 0,   \
-                         stream, queries, docs, cand_scores, cand_ids, Q, N, \
-                         D, k);                                              \
+      hipLaunchKernelGGL((qsa_topk_scan<T, QT>), grid, dim3(256), 0, stream, \
+                         queries, docs, cand_scores, cand_ids, Q, N, D, k);  \
     else                                                                     \
-      hipLaunchKernelGGL((qsa_topk_scan<T, QT, false>), grid, dim3(256), 0,  \
+      hipLaunchKernelGGL((qsa_topk_scan_any<T, QT>), grid, dim3(256), 0,     \
                          stream, queries, docs, cand_scores, cand_ids, Q, N, \
                          D, k);                                              \
   }
-  const int per = qsa_topk_block_docs(Q, N);
-  if (per == 64) QSA_SCAN(4, 1)
-  else if (per == 32) QSA_SCAN(2, 2)
-  else QSA_SCAN(1, 1)
+  switch (qsa_topk_tile(Q, N)) {
+    case 11: QSA_SCAN(1, 1) break;
+    case 41: QSA_SCAN(4, 1) break;
+    case 32: QSA_SCAN(3, 2) break;
+    default: QSA_SCAN(2, 3)
+  }
 #undef QSA_SCAN
 }
 

@@ -66,11 +66,11 @@ class HashingEmbedder:
 def _scan_wins(queries: int, rows: int, k: int) -> bool:
     """Whether a search is the kernel's (ops/hip/topk_cosine.hip) or a matmul's
     with a sort.  Measured at 1536 numbers a row (us, kernel / matmul): up to
-    16 queries are one read of the matrix (16, k = 16: 100k rows 194 / 312, 1M
-    1517 / 1536), up to 32 one and more work per row (32, k = 3: 100k 219 /
-    311, 200k 418 / 571, 300k 609 / 659, 500k 1001 / 924, 1M 1973 / 1556).
-    More are GEMM-shaped (48, k = 8: 26k 138 / 170, 45k 189 / 189, 100k 384 /
-    289)."""
+    16 queries are one read of the matrix (16, k = 16: 100k rows 156 / 314, 1M
+    1231 / 1579), up to 32 one and more work per row (32, k = 16: 100k 220 /
+    313, 300k 599 / 663, 1M 1725 / 1593).  More are GEMM-shaped, and a block's
+    choice of its best k costs per query and k (64, k = 16: 10k 68 / 101, 30k
+    132 / 143; 256, k = 16: 1k 50 / 50, 10k 166 / 176, 30k 392 / 382)."""
     if k > 16:                       # what the kernel keeps
         return False
     return queries <= 16 or \
@@ -185,12 +185,14 @@ class VectorIndex:
             # kernel has no answer for a query that is not a number
             scores_all = qt @ docs.T
             scores, idx = torch.topk(scores_all, k_eff, dim=1)
-            idx = idx.int()
+            scores = scores.cpu().numpy().tolist()
+            idx = idx.cpu().numpy().tolist()
         else:
-            # the tiled cosine/top-k HIP kernel
-            scores, idx = D.topk_cosine(qt.contiguous(), docs, k_eff)
-        scores = scores.cpu().numpy().tolist()
-        idx = idx.cpu().numpy().tolist()
+            # the tiled cosine/top-k HIP kernel, and one copy of its results
+            both = D.topk_cosine_packed(qt.contiguous(), docs,
+                                        k_eff).cpu().numpy()
+            scores = both[0].view(np.float32).tolist()
+            idx = both[1].tolist()
         # -1: fewer documents than k have a score
         return [[SearchHit(self.ids[i], self.chunks[i], s, self.metadata[i])
                  for i, s in zip(ids, row) if i >= 0]

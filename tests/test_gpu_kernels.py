@@ -205,6 +205,40 @@ def test_topk_cosine_edges(ext, Q, N, D, k):
     assert torch.equal(i.cpu(), want_i)
 
 
+@pytest.mark.parametrize("Q,N,D,k", [
+    (16, 32_767, 96, 3), (16, 32_768, 100, 3), (1, 32_785, 132, 16),  # 16 | 64
+    (17, 8191, 160, 5), (17, 8192, 4, 5), (32, 8209, 124, 3),  # 16 | 48 x 32
+    (33, 4095, 64, 3), (33, 4097, 28, 3), (48, 4128, 260, 16),  # 16 | 32 x 48
+    (49, 4096, 128, 3), (64, 4143, 36, 2),
+    (17, 196_608, 4, 5), (33, 131_104, 4, 5),     # 4096 lists, and one more
+    (33, 5000, 27, 3), (17, 9000, 31, 3), (16, 33_000, 1, 3)])  # odd rows
+def test_topk_cosine_blocks(ext, Q, N, D, k):
+    """Either side of each choice of a block; rows that end at, before and behind
+    a step of 32 numbers.  Small whole numbers: scores are exact.  Memory that
+    the search takes is poisoned first: nothing of it may be left."""
+    g = torch.Generator().manual_seed(Q * 1000 + N + D)
+    docs = torch.randint(-2, 3, (N, D), generator=g).float()
+    qs = torch.randint(-2, 3, (Q, D), generator=g).float()
+    docs[2] = float("nan")
+    docs[N - 1] = qs[Q - 1] * 3
+    a, b = qs.to(dev()), docs.to(dev())
+    stale = [torch.full((n,), float("nan"), device=dev())
+             for n in (Q * N // 8, Q * N // 4, 1 << 12)]
+    del stale
+    s, i = ext.topk_cosine(a, b, k)
+    full = (qs @ docs.T).nan_to_num(-9e9)
+    full[full <= -2] = -float("inf")
+    top, order = torch.sort(full, dim=1, descending=True, stable=True)
+    some = top[:, :k] > -2
+    assert torch.equal(s.cpu(), top[:, :k].where(some, torch.tensor(-2.0)))
+    assert torch.equal(i.cpu(), order[:, :k].int().where(
+        some, torch.tensor(-1, dtype=torch.int32)))
+    both = ext.topk_cosine_packed(a, b, k)
+    assert both.shape == (2, Q, k)
+    assert torch.equal(both[0].view(torch.float32), s)
+    assert torch.equal(both[1], i)
+
+
 def test_window_agg(ext):
     torch.manual_seed(6)
     n, nkeys, nwin = 50000, 7, 288
