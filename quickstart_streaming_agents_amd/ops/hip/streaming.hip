@@ -17,7 +17,7 @@
 // a chunk reach the output is chosen by qsa_window_workspace:
 //   merged   chunks of 4096 leave (windows spanned) * nkeys cells in a
 //            workspace, qsa_window_merge adds them up, without atomics and in
-//            a fixed order (35 us)
+//            a fixed order (26 us, clearing the output and both launches)
 //   direct   chunks of 256 or 1024 add their cells to the output with atomics
 // More keys than fit in LDS have neither: an event at a time.
 // ---------------------------------------------------------------------------
@@ -65,9 +65,42 @@ qsa_window_events(const long long* __restrict__ ts,
   }
 }
 
-// PER events of a thread, chunk == 256 * PER; PER 0: any.  win_ms > 0.
-template <int PER, int CELLS>
-__global__ void __launch_bounds__(256)
+// A value as a whole number of units of 2^unit; exact where its lowest bit is no
+// less than one (see the kernel).
+struct QsaBits {
+  unsigned mant;                       // 24 bits, 0: the value is zero
+  int exp;                             // of the mantissa's lowest bit
+};
+
+__device__ __forceinline__ QsaBits qsa_bits(float v) {
+  const unsigned u = __float_as_uint(v), e = u >> 23 & 255, f = u & 0x7fffff;
+  return {e ? f | 0x800000 : f, (int)max(e, 1u) - 150};
+}
+
+__device__ __forceinline__ long long qsa_units(float v, int unit) {
+  const QsaBits b = qsa_bits(v);
+  const int s = b.exp - unit;          // below 0: zeros are shifted out
+  const long long x = b.mant == 0 ? 0
+                      : s >= 0    ? (long long)b.mant << s
+                                  : (long long)(b.mant >> -s);
+  return v < 0.f ? -x : x;
+}
+
+// A float added to LDS occupies the unit some 3 cycles a lane, a 64-bit integer
+// under a third of that: of 20 us for 2M events of 1000 keys 10 were these sums
+// (7 so, with 512 threads a chunk, 256 before).  So where
+// the values of a chunk allow it their sums are whole numbers of the lowest bit
+// that is set in any of them, in one word with the count: exact, in any order,
+// rounded once at the end.  They do if the highest is below 2^38 of these units
+// (as 24-bit numbers do within 2^14 of each other), for 4096 of them then stay
+// below the 2^50 that the word has room for.  Others, and chunks of more, are
+// float sums.
+#define QSA_AGG_SUM_BITS 51
+#define QSA_AGG_UNIT_BITS 38
+
+// PER events of a thread, chunk == NT * PER; PER 0: any.  win_ms > 0.
+template <int PER, int CELLS, int NT>
+__global__ void __launch_bounds__(NT)
 qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
                const float* __restrict__ value,  // nullptr -> count only
                int* __restrict__ counts, float* __restrict__ sums,
@@ -75,18 +108,27 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
                long long n, long long chunk,
                int2* __restrict__ span,          // [blocks] {first, windows}
                int* __restrict__ ws) {           // [blocks, 2, QSA_AGG_CELLS]
-  __shared__ int cnt[CELLS];
-  __shared__ float sum[CELLS];
-  __shared__ int lo_s, hi_s;
+  constexpr bool FIT = PER > 4;        // smaller chunks gain nothing by it
+  static_assert(!FIT || (long long)PER * NT <= 1 << (QSA_AGG_SUM_BITS - 1 -
+                                             QSA_AGG_UNIT_BITS) &&
+                            (long long)PER * NT <
+                                1 << (64 - QSA_AGG_SUM_BITS),
+                "the sum and the count of a chunk fit");
+  __shared__ unsigned long long cell[CELLS];     // or counts, then float sums
+  __shared__ int lo_s, hi_s, bit_s, top_s;
+  int* cnt = reinterpret_cast<int*>(cell);
+  float* sum = reinterpret_cast<float*>(cell) + CELLS;
   const int tid = threadIdx.x;
   const long long first = (long long)blockIdx.x * chunk;
   const long long end = min(first + chunk, n);
   if (tid == 0) {
-    lo_s = 0x7fffffff;
+    lo_s = bit_s = 0x7fffffff;
     hi_s = -1;
+    top_s = -0x7fffffff;
   }
   __syncthreads();
   int lo = 0x7fffffff, hi = -1;
+  int bit = 0x7fffffff, top = -0x7fffffff;       // lowest bit, highest 24 bits
   // PER: every load of the chunk is under way before the first is used, and
   // an event's window is found once
   int win[PER ? PER : 1], ek[PER ? PER : 1];
@@ -98,23 +140,30 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
     const double inv = 1.0 / (double)win_ms;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const long long i = min(first + tid + j * 256, n - 1);
+      const long long i = min(first + tid + j * NT, n - 1);
       et[j] = ts[i];
       ek[j] = key[i];
       ev[j] = value ? value[i] : 0.f;
     }
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      win[j] = first + tid + j * 256 < end
+      win[j] = first + tid + j * NT < end
                    ? qsa_window_by(et[j], t0, win_ms, limit, inv) : -1;
       if (win[j] >= 0) {
         lo = min(lo, win[j]);
         hi = max(hi, win[j]);
+        if (FIT && value) {
+          const QsaBits b = qsa_bits(ev[j]);
+          if (b.mant && ek[j] >= 0 && ek[j] < nkeys) {
+            bit = min(bit, b.exp + __ffs(b.mant) - 1);
+            top = max(top, b.exp);     // 255 - 150: not a number, infinite
+          }
+        }
       }
     }
   } else {
 #pragma unroll 4
-    for (long long i = first + tid; i < end; i += 256) {
+    for (long long i = first + tid; i < end; i += NT) {
       const int w = qsa_window_of(ts[i], t0, win_ms, nwin);
       if (w >= 0) {
         lo = min(lo, w);
@@ -126,23 +175,44 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
   for (int o = 1; o < 64; o <<= 1) {
     lo = min(lo, __shfl_xor(lo, o, QSA_WAVE));
     hi = max(hi, __shfl_xor(hi, o, QSA_WAVE));
+    if constexpr (FIT) {
+      bit = min(bit, __shfl_xor(bit, o, QSA_WAVE));
+      top = max(top, __shfl_xor(top, o, QSA_WAVE));
+    }
   }
   if ((tid & 63) == 0) {
     atomicMin(&lo_s, lo);
     atomicMax(&hi_s, hi);
+    if constexpr (FIT) {
+      atomicMin(&bit_s, bit);
+      atomicMax(&top_s, top);
+    }
   }
   __syncthreads();
   lo = lo_s;
   hi = hi_s;
   const long long cells = hi < 0 ? 0 : (long long)(hi - lo + 1) * nkeys;
-  const bool local = cells <= CELLS;     // uniform over the block
+  const bool local = cells <= CELLS;     // uniform over the block, as is whole
   if (ws && tid == 0)
     span[blockIdx.x] = make_int2(lo, local && hi >= 0 ? hi - lo + 1 : 0);
   if (cells == 0) return;              // no event of the chunk counts
+  int unit = 0;                        // no value but zeros: any
+  bool whole = false;
+  if constexpr (FIT) {
+    const bool some = bit_s != 0x7fffffff;
+    if (some) unit = bit_s;
+    whole = local && value &&
+            (!some || (top_s < 255 - 150 &&
+                       top_s + 24 - bit_s <= QSA_AGG_UNIT_BITS));
+  }
   if (local) {
-    for (int c = tid; c < (int)cells; c += 256) {
-      cnt[c] = 0;
-      sum[c] = 0.f;
+    for (int c = tid; c < (int)cells; c += NT) {
+      if (whole) {
+        cell[c] = 0;
+      } else {
+        cnt[c] = 0;
+        sum[c] = 0.f;
+      }
     }
     __syncthreads();
   }
@@ -150,6 +220,11 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
     if (w < 0 || kk < 0 || kk >= nkeys) return;
     if (local) {
       const int c = (w - lo) * nkeys + kk;
+      if (whole) {
+        atomicAdd(cell + c, (1ull << QSA_AGG_SUM_BITS) +
+                                (unsigned long long)qsa_units(v, unit));
+        return;
+      }
       atomicAdd(cnt + c, 1);
       if (value) unsafeAtomicAdd(sum + c, v);
     } else {
@@ -163,34 +238,43 @@ qsa_window_agg(const long long* __restrict__ ts, const int* __restrict__ key,
     for (int j = 0; j < PER; ++j) count(win[j], ek[j], ev[j]);
   } else {
 #pragma unroll 4
-    for (long long i = first + tid; i < end; i += 256)
+    for (long long i = first + tid; i < end; i += NT)
       count(qsa_window_of(ts[i], t0, win_ms, nwin), key[i],
             value ? value[i] : 0.f);
   }
   if (!local) return;
   __syncthreads();
-  if (ws) {
-    int* wc = ws + (long long)blockIdx.x * 2 * QSA_AGG_CELLS;
-    float* wf = reinterpret_cast<float*>(wc + QSA_AGG_CELLS);
-    for (int c = tid; c < (int)cells; c += 256) {
-      wc[c] = cnt[c];
-      if (value) wf[c] = sum[c];
+  const double one = __longlong_as_double((long long)(unit + 1023) << 52);
+  for (int c = tid; c < (int)cells; c += NT) {
+    int many;
+    float v;
+    if (whole) {
+      constexpr int UP = 64 - QSA_AGG_SUM_BITS;
+      const long long word = (long long)cell[c], x = word << UP >> UP;
+      many = (int)((unsigned long long)(word - x) >> QSA_AGG_SUM_BITS);
+      v = (float)((double)x * one);
+    } else {
+      many = cnt[c];
+      v = sum[c];
     }
-    return;
-  }
-  for (int c = tid; c < (int)cells; c += 256) {
-    if (cnt[c] == 0) continue;
-    const long long slot = (long long)(c % nkeys) * nwin + lo + c / nkeys;
-    atomicAdd(counts + slot, cnt[c]);
-    if (value) unsafeAtomicAdd(sums + slot, sum[c]);
+    if (ws) {
+      int* wc = ws + (long long)blockIdx.x * 2 * QSA_AGG_CELLS + c;
+      wc[0] = many;
+      if (value) wc[QSA_AGG_CELLS] = __float_as_int(v);
+    } else if (many) {
+      const long long slot = (long long)(c % nkeys) * nwin + lo + c / nkeys;
+      atomicAdd(counts + slot, many);
+      if (value) unsafeAtomicAdd(sums + slot, v);
+    }
   }
 }
 
 // Block = 8 windows x 64 keys, a wave per window: the chunks that reach it, in
 // order, added to what other chunks left in the output.  Bound by a chain of
 // latencies (spans, cells, output), so the output is fetched first and four
-// chunks' cells at a time: 288 x 1000 cells of 489 chunks 12.5 us with two
-// windows a wave, 10.6 here.
+// chunks' cells at a time; the output is read and written with 8 windows of a
+// key in neighbouring lanes, where a wave's 64 keys were 64 lines, four times:
+// 288 x 1000 cells of 489 chunks 12 us before, 9 so.
 __global__ void __launch_bounds__(512)
 qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
                  int blocks, int* __restrict__ counts,
@@ -199,13 +283,19 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
   __shared__ int list[QSA_AGG_BLOCKS];
   __shared__ int2 range[QSA_AGG_BLOCKS];
   __shared__ int wave_n[8];
+  __shared__ int out_c[8][65];
+  __shared__ float out_v[8][65];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int w0 = blockIdx.x * 8, w = w0 + wave, k = blockIdx.y * 64 + lane;
+  const int w0 = blockIdx.x * 8, w = w0 + wave, k0 = blockIdx.y * 64;
+  const int k = k0 + lane;
   const bool live = k < nkeys && w < nwin;
-  const long long slot = live ? (long long)k * nwin + w : 0;
-  int c = counts[slot];
-  float v = has_value ? sums[slot] : 0.f;
+  // a thread's cell of the output: 8 windows of a key are 8 lanes, one line
+  const int ow = tid & 7, ok = tid >> 3;
+  const bool mine = k0 + ok < nkeys && w0 + ow < nwin;
+  const long long slot = mine ? (long long)(k0 + ok) * nwin + w0 + ow : 0;
+  const int c = counts[slot];
+  const float v = has_value ? sums[slot] : 0.f;
   int total = 0;
   for (int base = 0; base < blocks; base += 512) {
     const int b = base + tid;
@@ -261,9 +351,13 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
       pv += gv[j];
     }
   }
-  if (live && reached) {
-    counts[slot] = c + pc;
-    if (has_value) sums[slot] = v + pv;
+  out_c[wave][lane] = pc;
+  out_v[wave][lane] = pv;
+  if (lane == 0) wave_n[wave] = reached;
+  __syncthreads();
+  if (mine && wave_n[ow]) {
+    counts[slot] = c + out_c[ow][ok];
+    if (has_value) sums[slot] = v + out_v[ow][ok];
   }
 }
 
@@ -273,21 +367,38 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
 // lambda = 0.3 * tr(G)/p, prediction se with leverage.  p <= 4.
 // series: [K, Tmax] f32 (ragged via lengths[]); outputs per key.
 //
-// Bound by latency: three passes over a series that L1 holds after the first.
-// All lanes share every pass and solve the padded 4x4 system in registers
-// (rows beyond p are the identity).  1000 series of 288: 171 us with the
-// solve and the residuals on one lane, 11 us here.
+// Bound by latency: three passes over a series.  All lanes share every pass and
+// solve the padded 4x4 system in registers (rows beyond p are the identity).
+// A series of up to 512 goes to LDS at once, beside its length: passes that
+// waited for memory 64 numbers at a time made 10.5 us of 1000 series of 288,
+// 8.9 so (171 us with the solve and the residuals on one lane).
 // ---------------------------------------------------------------------------
 #define QSA_AR_MAXP 4
 
+template <int STAGE>                   // Tmax <= STAGE, or 0: any
 __global__ void __launch_bounds__(64)
 qsa_anomaly_batch(const float* __restrict__ series, const int* __restrict__ lengths,
                   float* __restrict__ forecast, float* __restrict__ pred_se,
                   int* __restrict__ dof_out, int Tmax, int order) {
   const int kidx = blockIdx.x;
   const int lane = threadIdx.x;
-  const float* h = series + (long long)kidx * Tmax;
+  const float* row = series + (long long)kidx * Tmax;
   const int n = lengths[kidx];
+  __shared__ float staged[STAGE ? STAGE : 1];
+  const float* h;
+  if constexpr (STAGE > 0) {           // without waiting for the length
+    float x[STAGE / QSA_WAVE];
+#pragma unroll
+    for (int j = 0; j < STAGE / QSA_WAVE; ++j)
+      if (j * QSA_WAVE < Tmax) x[j] = row[min(lane + j * QSA_WAVE, Tmax - 1)];
+#pragma unroll
+    for (int j = 0; j < STAGE / QSA_WAVE; ++j)
+      if (j * QSA_WAVE < Tmax) staged[lane + j * QSA_WAVE] = x[j];
+    __syncthreads();
+    h = staged;
+  } else {
+    h = row;
+  }
 
   if (n < 6) {  // mean/std fallback (matches CPU path)
     float sum = 0.f, sq = 0.f;
@@ -478,14 +589,14 @@ extern "C" void qsa_window_agg_launch(const long long* ts, const int* key,
   const int blocks = (int)((n + chunk - 1) / chunk);
   int2* span = reinterpret_cast<int2*>(ws);
   int* cells = ws ? ws + 2 * blocks : nullptr;
-#define QSA_AGG(PER, CELLS)                                                  \
-  hipLaunchKernelGGL((qsa_window_agg<PER, CELLS>), dim3(blocks), dim3(256),  \
-                     0, stream, ts, key, value, counts, sums, t0, win_ms,    \
-                     nwin, nkeys, n, chunk, span, cells)
-  if (chunk > QSA_AGG_CHUNK) QSA_AGG(0, QSA_AGG_CELLS);
-  else if (ws) QSA_AGG(QSA_AGG_CHUNK / 256, QSA_AGG_CELLS);
-  else if (chunk == 1024) QSA_AGG(4, QSA_AGG_CELLS);
-  else QSA_AGG(1, QSA_AGG_FEW);
+#define QSA_AGG(PER, CELLS, NT)                                              \
+  hipLaunchKernelGGL((qsa_window_agg<PER, CELLS, NT>), dim3(blocks),         \
+                     dim3(NT), 0, stream, ts, key, value, counts, sums, t0,  \
+                     win_ms, nwin, nkeys, n, chunk, span, cells)
+  if (chunk > QSA_AGG_CHUNK) QSA_AGG(0, QSA_AGG_CELLS, 256);
+  else if (ws) QSA_AGG(QSA_AGG_CHUNK / 512, QSA_AGG_CELLS, 512);
+  else if (chunk == 1024) QSA_AGG(4, QSA_AGG_CELLS, 256);
+  else QSA_AGG(1, QSA_AGG_FEW, 256);
 #undef QSA_AGG
   if (ws)
     hipLaunchKernelGGL(qsa_window_merge,
@@ -499,6 +610,12 @@ extern "C" void qsa_anomaly_batch_launch(const float* series,
                                          float* pred_se, int* dof_out, int K,
                                          int Tmax, int order,
                                          hipStream_t stream) {
-  hipLaunchKernelGGL(qsa_anomaly_batch, dim3(K), dim3(64), 0, stream, series,
-                     lengths, forecast, pred_se, dof_out, Tmax, order);
+  if (Tmax <= 512)
+    hipLaunchKernelGGL(qsa_anomaly_batch<512>, dim3(K), dim3(64), 0, stream,
+                       series, lengths, forecast, pred_se, dof_out, Tmax,
+                       order);
+  else
+    hipLaunchKernelGGL(qsa_anomaly_batch<0>, dim3(K), dim3(64), 0, stream,
+                       series, lengths, forecast, pred_se, dof_out, Tmax,
+                       order);
 }

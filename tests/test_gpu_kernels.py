@@ -275,6 +275,81 @@ def test_topk_cosine_many_lists(ext, Q, N, k):
     assert torch.equal(i.cpu(), order[:, :k].int())
 
 
+def _agg_values(kind, n, g):
+    v = torch.rand(n, generator=g) * 90 + 5
+    if kind == "signed":
+        v = torch.randn(n, generator=g) * 50
+        v[::7], v[1::7] = 0.0, -0.0
+    elif kind == "edge":                  # 38 bits from the lowest to the highest
+        v = torch.full((n,), 1.0 - 2.0 ** -24)
+        v[1::2] = -(2.0 ** -38)
+    elif kind == "beyond":                # 39
+        v = torch.full((n,), 2.0 - 2.0 ** -23)
+        v[1::2] = -(2.0 ** -38)
+    elif kind == "denormal":
+        v = torch.randint(-99, 99, (n,), generator=g).float() * 2.0 ** -149
+    elif kind == "huge":
+        v = v * 2.0 ** 100
+    elif kind == "zero":
+        v = v * 0
+    return v
+
+
+@pytest.mark.parametrize("n,nkeys,nwin", [
+    (69_633, 20, 300),                   # the last chunk is one event
+    (400_000, 300, 150), (262_145, 1000, 30)])
+@pytest.mark.parametrize("kind", ["plain", "signed", "edge", "beyond",
+                                  "denormal", "huge", "zero", "none"])
+def test_window_agg_values(ext, n, nkeys, nwin, kind):
+    """Chunks whose values are whole numbers of a common unit are summed as such,
+    the others as floats.  A chunk's sum is rounded once, the chunks of a cell
+    (some share of n / 4096 / nwin, and two more) are added in f32; float sums
+    round for every event."""
+    g = torch.Generator().manual_seed(n)
+    win = 60_000
+    ts = (torch.arange(n) * (nwin * win / n)).long()
+    key = (torch.rand(n, generator=g) ** 2 * nkeys).int().clamp(max=nkeys - 1)
+    key[5::1000], key[6::1000] = -1, nkeys        # of no key: not counted
+    val = _agg_values(kind, n, g)
+    ok = (key >= 0) & (key < nkeys)
+    bad = val.clone()
+    if kind == "plain":                  # nor do their values matter
+        bad[~ok] = float("nan")
+    c, s = ext.window_agg(ts.to(dev()), key.to(dev()),
+                          None if kind == "none" else bad.to(dev()), 0, win,
+                          nwin, nkeys)
+    slot = (key.long() * nwin + ts // win)[ok]
+    want = torch.zeros(nkeys * nwin, dtype=torch.int32).scatter_add_(
+        0, slot, torch.ones_like(slot, dtype=torch.int32))
+    assert torch.equal(c.cpu().view(-1), want)
+    if kind == "none":
+        assert not s.any()
+        return
+    total, size = (torch.zeros(nkeys * nwin, dtype=torch.float64).scatter_add_(
+        0, slot, x[ok].double()) for x in (val, val.abs()))
+    roundings = n / 4096 / nwin + 3
+    if kind == "beyond":
+        roundings = want
+    err = (s.cpu().view(-1).double() - total).abs()
+    assert (err <= size * roundings * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_window_agg_not_finite(ext, bad):
+    n, nkeys, nwin, win = 80_000, 20, 300, 1000
+    ts = (torch.arange(n) * (nwin * win / n)).long()
+    key = (torch.arange(n) % nkeys).int()
+    val = torch.ones(n)
+    val[40_003] = bad
+    c, s = ext.window_agg(ts.to(dev()), key.to(dev()), val.to(dev()), 0, win,
+                          nwin, nkeys)
+    s = s.cpu()
+    k, w = int(key[40_003]), int(ts[40_003]) // win
+    assert not torch.isfinite(s[k, w])
+    s[k, w] = c.cpu()[k, w]
+    assert torch.equal(s, c.cpu().float())
+
+
 @pytest.mark.parametrize("n,nkeys,nwin,shuffle", [
     (1, 1, 1, False), (255, 3, 2, True), (257, 6144, 1, False),
     (5000, 6145, 2, False),              # one key more than a block's cells
@@ -365,6 +440,11 @@ def test_hash_table_as_two_arrays(ext):
                            torch.arange(1000, device=dev()), -1).flip(0)
         assert torch.equal(rows[:1000].long(), want)
         assert (rows[1000:] == -1).all()
+
+
+@pytest.mark.parametrize("n", [61, 62, 509, 510])     # rows of 64, 512 and more
+def test_anomaly_batch_staged(ext, n):
+    test_anomaly_batch_lengths(ext, n)
 
 
 def test_anomaly_batch_matches_cpu(ext):
