@@ -92,6 +92,7 @@ class BpeTokenizer:
         assert vocab_size >= self.N_SPECIAL + 256, "vocab too small for BPE"
         merges = [tuple(p) for p in v["merges"]]
         merges = merges[: vocab_size - self.N_SPECIAL - 256]
+        self._merges = merges
         self._ranks: dict[tuple[int, int], int] = {
             p: i for i, p in enumerate(merges)}
         self._merge_sym = {p: 256 + i for i, p in enumerate(merges)}
@@ -103,11 +104,21 @@ class BpeTokenizer:
             self._sym_bytes.append(self._sym_bytes[a] + self._sym_bytes[b])
         self._special_re = re.compile(
             "(" + "|".join(re.escape(s) for s in self.specials) + ")")
-        # the same in native code, where it is built (ops/hip/bpe.cpp)
+        self._load_native()
+
+    def _load_native(self):
+        """The same in native code, where it is built (ops/hip/bpe.cpp)."""
         self._native = None
         if have_ext() and all(self.specials):
-            self._native = ext().Bpe(merges, list(self.specials.items()),
-                                     self._BYTE0)
+            self._native = ext().Bpe(self._merges,
+                                     list(self.specials.items()), self._BYTE0)
+
+    def __getstate__(self):
+        return dict(self.__dict__, _native=None)
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._load_native()
 
     @lru_cache(maxsize=65536)
     def _bpe_word(self, word: str) -> tuple[int, ...]:

@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import copy
+import pickle
 import random
 
 import pytest
@@ -61,3 +63,13 @@ def test_more_words_than_are_kept():
     tok.encode_batch(words, 99)
     for w in words[::997] + words[-3:]:
         assert tok.encode(w) == tok._encode(w, True)
+
+
+def test_copies_and_pickles():
+    """A tokenizer goes to other processes and is copied like any object."""
+    tok = BpeTokenizer(1024)
+    for other in (copy.deepcopy(tok), copy.copy(tok),
+                  pickle.loads(pickle.dumps(tok))):
+        assert other._native is not None
+        assert other.encode("a window<|finish|> of 12") == \
+            tok.encode("a window<|finish|> of 12")
