@@ -14,16 +14,10 @@ using bf16x4_v = __attribute__((ext_vector_type(4))) short;
 using u32x4_v = __attribute__((ext_vector_type(4))) unsigned int;
 using f32x4_v = __attribute__((ext_vector_type(4))) float;
 
-// round-to-nearest-even with the hardware's packed conversion
 __device__ __forceinline__ unsigned int cvt_bf16x2(float a, float b) {
-  typedef __attribute__((ext_vector_type(2))) float f2;
-  typedef __attribute__((ext_vector_type(2))) __bf16 b2;
-  return __builtin_bit_cast(unsigned int,
-                            __builtin_convertvector((f2){a, b}, b2));
+  return f32x2_to_bf16x2(a, b);
 }
-__device__ __forceinline__ bf16_t cvt_bf16(float a) {
-  return __builtin_bit_cast(bf16_t, (__bf16)a);
-}
+__device__ __forceinline__ bf16_t cvt_bf16(float a) { return f32_to_bf16(a); }
 
 template <typename T> __device__ __forceinline__ float ldf(const T* p);
 template <> __device__ __forceinline__ float ldf<bf16_t>(const bf16_t* p) {

@@ -92,13 +92,17 @@ __device__ __forceinline__ void qsa_warm(const u32x4_v* at, long long n,
 // rotate elements k0.. and k0 + D/2.. of a row held in two fragments
 __device__ __forceinline__ void rotate_pair(bf16x8_a& a, bf16x8_a& b,
                                             const float* c, const float* s) {
+  u32x4_v u = __builtin_bit_cast(u32x4_v, a), v = __builtin_bit_cast(u32x4_v, b);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float x = bf16_to_f32((unsigned short)a[e]);
-    const float y = bf16_to_f32((unsigned short)b[e]);
-    a[e] = (short)f32_to_bf16(x * c[e] - y * s[e]);
-    b[e] = (short)f32_to_bf16(x * s[e] + y * c[e]);
+  for (int e = 0; e < 4; ++e) {
+    const float2 x = bf16x2_to_f32x2(u[e]), y = bf16x2_to_f32x2(v[e]);
+    const float c0 = c[2 * e], c1 = c[2 * e + 1];
+    const float s0 = s[2 * e], s1 = s[2 * e + 1];
+    u[e] = cvt_bf16x2(x.x * c0 - y.x * s0, x.y * c1 - y.y * s1);
+    v[e] = cvt_bf16x2(x.x * s0 + y.x * c0, x.y * s1 + y.y * c1);
   }
+  a = __builtin_bit_cast(bf16x8_a, u);
+  b = __builtin_bit_cast(bf16x8_a, v);
 }
 
 // Up to 63 of a wave's loads under way, whatever it stored or read from LDS.
