@@ -118,6 +118,10 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   constexpr int DTILES = D / 16;      // PV d-tiles (8 for D=128)
   constexpr int VT = D * QSA_PAGE;    // elements of a value page
   constexpr int KL = 4 * KSTEPS;      // loads of a wave for a page's keys
+  // Values are asked for a page ahead where few rows leave latencies to hide, and
+  // where many share the memory once the page's keys are there: with four waves
+  // a page ahead made 33 rows of 3000-4000 keys 103 -> 104 us, so 100.
+  constexpr bool EARLY = NW == 8;
   // a wave's values, afterwards its part of the output [R][D]
   __shared__ __attribute__((aligned(16))) unsigned short vlds[NW * VT];
   __shared__ float ml[2 * NW * 16];   // and its maxima and sums
@@ -135,9 +139,13 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   const int kvh = bk % p.KVH;
   const int R = p.QH / p.KVH;
   const int first = split * NW + wave, step = NW * p.NS;
-  const int* btab = p.block_table + (long long)b * p.max_pages;
-  // side by side: the first page's number waits for no length
+  // scalar loads: as a vector load a page's number, newer than the loads under
+  // way, would have waited for all of them
+  const auto btab = (const __attribute__((address_space(4))) int*)(
+      p.block_table + (long long)b * p.max_pages);
+  // side by side: the first pages' numbers wait for no length
   int page = btab[min(first, p.max_pages - 1)];
+  int next = btab[min(first + step, p.max_pages - 1)];
   const int seqlen = p.seq_lens[b];
   const int npages = (seqlen + QSA_PAGE - 1) / QSA_PAGE;
   const int col = lane & 15;          // head col (scores) / dim col (PV)
@@ -170,17 +178,20 @@ qsa_paged_attn_mfma(DecodeArgs p) {
     };
     // Values go straight to the wave's LDS, 8 rows of 128 bytes at a time, a
     // row's segments exchanged by its number (the reads below then spread over
-    // the banks).
+    // the banks).  By buffer loads: behind a global one to LDS the compiler waits
+    // for everything that is under way wherever it has to wait for anything.
     unsigned short* vl = vlds + wave * VT;
+    const unsigned int voff =
+        ((lane >> 3) * QSA_PAGE + ((lane & 7) ^ (lane >> 3)) * 8) * 2;
     auto load_v = [&](int page) {
-      const unsigned short* vbase =
-          p.vc + ((long long)page * p.KVH + kvh) * VT + (lane >> 3) * QSA_PAGE +
-          ((lane & 7) ^ (lane >> 3)) * 8;
+      const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(p.vc + ((long long)page * p.KVH + kvh) * VT), 0, VT * 2,
+          0x00027000);
 #pragma unroll
       for (int i = 0; i < D / 8; ++i)
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)(vbase + i * 512),
-            (__attribute__((address_space(3))) void*)(vl + i * 512), 16, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rv, (__attribute__((address_space(3))) void*)(vl + i * 512), 16,
+            voff, i * 1024, 0, 0);
     };
     bf16x8_a kf[4][KSTEPS];
     load_k(page, kf);
@@ -203,6 +214,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         ldv<float, 8>(p.sin_t + at + ks * 32, sn[ks]);
       }
     }
+    if constexpr (EARLY) load_v(page);  // behind all that the scores wait for
     if constexpr (FUSE) {
 #pragma unroll
       for (int ks = 0; ks < KSTEPS / 2; ++ks) {
@@ -211,13 +223,16 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       }
     }
 
-    // patch: the row's last page, where the new token has its place
-    auto walk = [&](int pi, auto patch) {
-      const bool more = !patch.value && pi + step < npages;
-      const int next = more ? btab[pi + step] : 0;
+    // Page pi; the keys of the wave's next one are asked for once these have been
+    // multiplied.  The last page is code of its own, or the waits of both would be
+    // for all that is under way.  patch: the row's last page, where the new token
+    // has its place.
+    auto walk = [&](int pi, auto last) {
+      const int after = btab[min(pi + 2 * step, p.max_pages - 1)];
       const int nvalid = min(seqlen - pi * QSA_PAGE, QSA_PAGE);
       const int pin = nvalid - 1;
-      if constexpr (patch.value) {
+      const bool patch = FUSE && last.value && pi == npages - 1;
+      if (patch) {
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
@@ -236,9 +251,8 @@ qsa_paged_attn_mfma(DecodeArgs p) {
                                                         acc, 0, 0, 0);
         sc[pt] = acc;
       }
-      // values only now: before the keys they would delay them
-      load_v(page);
-      if (more) load_k(next, kf);
+      if constexpr (!EARLY) load_v(page);
+      if constexpr (!last.value) load_k(next, kf);
       // scale + mask invalid positions; C layout: row pos = hi*4 + r,
       // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
       float pagemax = -3.0e38f;
@@ -287,9 +301,8 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       lsum = lsum * alpha + psum;
 
       // the values are there; the next page's keys, behind them, need not be
-      if (more) wait_vm<KL>();
-      else wait_vm<0>();
-      if constexpr (patch.value) {
+      wait_vm<last.value ? 0 : KL>();
+      if (patch) {
 #pragma unroll
         for (int i = 0; i < D; i += 64) {
           const int d = i + lane;
@@ -336,7 +349,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
           o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               pa, vf[dt], o_acc[dt], 0, 0, 0);
       }
-      if constexpr (patch.value) {     // the key's lines: 8 positions each
+      if (patch) {                     // the key's lines: 8 positions each
 #pragma unroll
         for (int pt = 0; pt < 4; ++pt)
           if (pt * 16 + col == pin) {
@@ -349,15 +362,18 @@ qsa_paged_attn_mfma(DecodeArgs p) {
                   kf[pt][ks];
           }
       }
-      // all of the values have been read when the next page's come
-      __builtin_amdgcn_s_waitcnt(0xc07f);         // lgkmcnt(0)
-      asm volatile("" ::: "memory");
-      page = next;
+      if constexpr (!last.value) {
+        // all of the values have been read when the next page's come
+        __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        if constexpr (EARLY) load_v(next);
+        page = next;
+        next = after;
+      }
     };
     int pi = first;
-    for (; pi < npages - (FUSE ? 1 : 0); pi += step)
-      walk(pi, std::false_type{});
-    if (FUSE && pi == npages - 1) walk(pi, std::true_type{});
+    for (; pi + step < npages; pi += step) walk(pi, std::false_type{});
+    walk(pi, std::true_type{});
   }
 
   // ---- the waves of the block meet: O C-layout row = head = hi*4 + r -----
