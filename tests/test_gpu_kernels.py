@@ -442,6 +442,19 @@ def test_hash_table_as_two_arrays(ext):
         assert (rows[1000:] == -1).all()
 
 
+# half full where n is a power of two; steps of one beyond 131072 rows
+@pytest.mark.parametrize("n", [1, 32, 33, 1024, 131_072, 131_073])
+def test_hash_table_fill(ext, n):
+    g = torch.Generator(device=dev()).manual_seed(n)
+    keys = torch.randperm(4 * n, generator=g, device=dev()) * 3 - n
+    ts = torch.randint(0, 1000, (n,), generator=g, device=dev())
+    k, p = ext.hash_build(keys[:n], ts)
+    rows = ext.hash_probe(k, p, keys, 500)
+    want = torch.where(ts >= 500, torch.arange(n, device=dev()), -1)
+    assert torch.equal(rows[:n].long(), want)
+    assert (rows[n:] == -1).all()
+
+
 @pytest.mark.parametrize("n", [61, 62, 509, 510])     # rows of 64, 512 and more
 def test_anomaly_batch_staged(ext, n):
     test_anomaly_batch_lengths(ext, n)
