@@ -66,7 +66,9 @@ __device__ __forceinline__ void stage_barrier() {
 // ST places in LDS; with ACT, W's rows are [gate; up] and a wave's column tiles
 // are alternately of either.
 template <int BM, int BN, int WM, int WN, int ST, int ACT>
-__global__ void __launch_bounds__(WM * WN * 64)
+__global__ void __launch_bounds__(WM * WN * 64,
+                                  (ST * (BM + BN) * 128 <= 80 * 1024 ? 2 : 1) *
+                                      WM * WN / 4)
 qsa_rows_gemm(RowsArgs p) {
 #ifdef __HIP_DEVICE_COMPILE__
   constexpr int NW = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16;
@@ -301,7 +303,12 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
 #undef QSA_RG
 }
 
-// BM, BN, waves, places of the ring; a block's own time and that of a stage, us
+// BM, BN, waves, places of the ring; a block's own time and that of a stage, us.
+// Of the last tile two blocks share a CU: one's start and end lie beside the
+// other's products, which short K gains by (us, the best of the others and so:
+// 16,000 x 3072 x 384 with the activation 52.7, 49.3; 24,000 79.2, 71.7; 8263 x
+// 2048 x 128 15.7, 13.0; 30,000 38.2, 30.7; 4400 x 16384 x 2048 263, 253).  Its
+// figures are those of a pair, set where 42 such shapes part.
 #define QSA_TILES(X) \
   X(64, 32, 2, 2, 6, 0.67f, 0.141f)   X(64, 64, 2, 2, 4, 0.71f, 0.208f) \
   X(64, 128, 2, 4, 6, 1.86f, 0.353f)  X(128, 64, 4, 2, 6, 1.92f, 0.334f) \
@@ -309,11 +316,16 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
   X(192, 128, 4, 2, 4, 2.98f, 0.644f) X(256, 128, 4, 2, 3, 3.41f, 0.822f) \
   X(128, 256, 2, 4, 3, 3.32f, 0.843f) X(192, 192, 2, 4, 3, 4.03f, 0.800f) \
   X(256, 192, 4, 2, 2, 3.57f, 1.189f) X(192, 256, 2, 4, 2, 3.19f, 1.227f) \
-  X(256, 256, 2, 4, 2, 4.06f, 1.482f)
+  X(256, 256, 2, 4, 2, 4.06f, 1.482f) X(192, 128, 4, 2, 2, 0.77f, 1.27f)
 
-struct RowsTile { int bm, bn, wn; float own, stage; };
+struct RowsTile {
+  int bm, bn, wn;
+  bool pair;                           // of large blocks on a CU
+  float own, stage;
+};
 static const RowsTile rows_tiles[] = {
-#define X(BM, BN, WM, WN, ST, OWN, STAGE) {BM, BN, WN, OWN, STAGE},
+#define X(BM, BN, WM, WN, ST, OWN, STAGE)                              \
+  {BM, BN, WN, WM * WN == 8 && ST * (BM + BN) <= 640, OWN, STAGE},
     QSA_TILES(X)
 #undef X
 };
@@ -340,13 +352,16 @@ extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
     if (act && t.bn / t.wn / 16 % 2) continue;    // no pairs of column tiles
     const long long blocks =
         (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    if (t.pair && blocks <= 256) continue;        // alone on their CUs
     const int fill = blocks < 256 ? (int)(256 / blocks) : 1;
     for (int S = act || all < 8 ? 1 : fill; S >= 1; S = S > 1 ? S / 2 : 0) {
       if (S > all / 4 && S > 1) continue;
-      const long long turns = (blocks * S + 255) / 256;
+      const int slots = t.pair ? 512 : 256;
+      const long long turns = (blocks * S + slots - 1) / slots;
       float stage = t.stage;
       if (turns == 1 && t.bn * t.bm <= 4096) stage *= i ? 1.48f : 1.32f;
-      const float run = (float)turns * (t.own + stage * ((all + S - 1) / S));
+      float run = (float)turns * (t.own + stage * ((all + S - 1) / S));
+      if (t.pair && turns == 1) run += 1.5f;      // neither end beside another
       const float r2 = run * run, m2 = mem * mem;
       const float us = sqrtf(sqrtf(r2 * r2 + m2 * m2)) +
                        (S > 1 ? sum + each * S : 0.f);

@@ -584,7 +584,8 @@ ROWS_SIZES = [(65, 32, 128), (33, 10768, 128), (40, 2048, 1024),
               (191, 4112, 4032), (330, 12304, 192), (700, 9696, 832),
               (300, 16416, 576), (700, 8256, 64), (2100, 4112, 576),
               (385, 16400, 704), (1500, 6176, 1024), (1000, 8880, 576),
-              (1700, 8208, 256), (167, 16384, 2048), (70, 10240, 512)]
+              (1700, 8208, 256), (167, 16384, 2048), (70, 10240, 512),
+              (1159, 9376, 128), (1283, 8128, 1600)]
 
 
 def stale(*shape):
@@ -630,10 +631,10 @@ def test_rows_glu(M, N, K, act):
 def test_rows_gemm_sizes_reach_every_tile():
     from quickstart_streaming_agents_amd.ops import lm_ext
     plain = {lm_ext().rows_gemm_plan(*s, False)[0] for s in ROWS_SIZES}
-    assert plain == set(range(13))
+    assert plain == set(range(14))
     gated = {lm_ext().rows_gemm_plan(m, n // 32 * 32, k, True)[0]
              for m, n, k in ROWS_SIZES}
-    assert gated == set(range(13)) - {0, 9}       # no pairs of column tiles
+    assert gated == set(range(14)) - {0, 9}       # no pairs of column tiles
 
 
 @pytest.mark.parametrize("S", [2, 7, 16])
