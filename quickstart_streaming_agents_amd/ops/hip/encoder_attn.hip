@@ -11,7 +11,9 @@
 // blocks fit a CU (128 rows and keys a block rotate each key fewer times, but
 // one block fits: 30 us).
 // 64 items of 137 tokens, 8 heads of 64: rotation into pages and attention over
-// them 13.4 + 17.6 us as two kernels, 23.3 us here.
+// them 13.4 + 17.6 us as two kernels, 19.2 us here (20.2 with the last tile's
+// 16s of keys without a key computed as well).  A block per item that has all keys
+// in LDS once, and heads of an item on one die, were no faster.
 #include <type_traits>
 
 #include "lm_common.h"
@@ -127,12 +129,13 @@ qsa_encoder_attn(const bf16_t* __restrict__ qkv,      // [T, 3, H, D]
     const int left = n - tile * ENC_KEYS;
     float alpha, top, psum;
     uint2 pk[4];
-    // edge: some keys are hidden; guard: a NaN score counts as no key
+    // edge: some keys are hidden, 16 without one are left out; guard: a NaN score counts as no key
     auto weigh = [&](auto edge, auto guard) {
       f32x4_v sc[4];
       float mx = -INFINITY;
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt) {
+        if (edge.value && pt * 16 >= left) break;
         sc[pt] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < KS; ++k)
@@ -155,6 +158,10 @@ qsa_encoder_attn(const bf16_t* __restrict__ qkv,      // [T, 3, H, D]
       psum = 0.f;
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt) {
+        if (edge.value && pt * 16 >= left) {
+          pk[pt] = make_uint2(0, 0);
+          continue;
+        }
         float p[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -174,6 +181,7 @@ qsa_encoder_attn(const bf16_t* __restrict__ qkv,      // [T, 3, H, D]
     for (int t = 0; t < ET; ++t) acc[t] *= alpha;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
+      if (k * 32 >= left) break;
       const bf16x8_v pf = __builtin_bit_cast(
           bf16x8_v, make_uint4(pk[2 * k].x, pk[2 * k].y, pk[2 * k + 1].x,
                                pk[2 * k + 1].y));
