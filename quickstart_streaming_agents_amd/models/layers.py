@@ -12,10 +12,18 @@ from ..ops import dispatch as D
 
 
 class Linear:
-    """y = x W^T.  On the GPU in bf16, decode-sized batches of the small
-    shapes stream a packed copy of W (ops/hip/skinny_gemm.hip, the measured
-    winner there), all that do not fill a library's tiles are
-    ops/hip/rows_gemm.hip's, and the rest is a vendor GEMM."""
+    """y = x W^T.  On the GPU in bf16, the fewest rows of the small shapes stream
+    a packed copy of W (ops/hip/skinny_gemm.hip), all that do not fill a library's
+    tiles are ops/hip/rows_gemm.hip's, and the rest is a vendor GEMM.
+
+    The stream's time grows with the rows, rows_gemm's does not, but splitting K
+    for few columns costs it a launch where no reader adds the shares.  With the
+    norm that adds them, us stream / rows_gemm: 2048 x 8192 at 1 row 13.8 / 13.7,
+    4 15.2 / 13.9, 16 18.6 / 14.5, 32 25.1 / 13.8; 2048 x 6144 8 13.4 / 12.9, 32
+    20.3 / 12.0; 1024 x 2048 8 7.7 / 7.6; 2048 x 2048 4 8.1 / 8.0, 17 9.7 / 8.1;
+    4096 x 4096 17 14.8 / 15.0, 32 17.1 / 13.4; 6144 x 4096 24 18.8 / 19.0.
+    Alone: 6144 x 2048 16 8.9 / 8.9, 32 12.3 / 9.1; 2048 x 4096 16 8.6 / 8.7, 32
+    11.9 / 8.6; 4096 x 2048 32 7.8 / 8.5; 8192 x 3072 24 12.6 / 12.7."""
 
     SKINNY_ROWS = 32
     SKINNY_MAX = 6144 * 4096
@@ -27,25 +35,33 @@ class Linear:
         if w.is_cuda and w.dtype == torch.bfloat16 and \
                 D.can_pack_weight(n, k) and n * k <= self.SKINNY_MAX:
             self.packed = D.pack_weight_frag(w)
+        # rows from which the stream is behind, alone and with shares
+        middling = n * k <= 20 << 20
+        self.rows = 17 if n >= 5632 and middling or \
+            k >= max(2 * n, 4096) else self.SKINNY_ROWS + 1
+        self.rows_parts = 4 if k >= 3 * n else 8 if k >= 2 * n else \
+            17 if middling else self.SKINNY_ROWS + 1
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
-        if self._skinny(x):
+        if self._skinny(x, self.rows):
             return D.skinny_linear(x, self.packed, *self.w.shape)
         return D.linear(x, self.w)
 
     def parts(self, x: torch.Tensor) -> torch.Tensor:
         """y for a reader that adds shares of K (D.linear_parts)."""
-        if self._skinny(x):
+        if self._skinny(x, self.rows_parts):
             return D.skinny_linear(x, self.packed, *self.w.shape)
         return D.linear_parts(x, self.w)
 
-    def _skinny(self, x: torch.Tensor) -> bool:
+    def _skinny(self, x: torch.Tensor, below: int) -> bool:
         return self.packed is not None and \
-            1 <= x.shape[0] <= self.SKINNY_ROWS and x.stride(0) % 8 == 0
+            1 <= x.shape[0] <= self.SKINNY_ROWS and x.stride(0) % 8 == 0 and \
+            (x.shape[0] < below or not D.rows_linear_ok(x, self.w))
 
     def glu(self, x: torch.Tensor, act: str) -> torch.Tensor:
         """act(gate) * up of y = [gate, up]."""
-        if not self._skinny(x) and D.glu_linear_ok(x, self.w):
+        if not self._skinny(x, self.SKINNY_ROWS + 1) and \
+                D.glu_linear_ok(x, self.w):
             return D.glu_linear(x, self.w, act)
         y, half = self(x), self.w.shape[0] // 2
         return D.glu(y[:, :half], y[:, half:], act)

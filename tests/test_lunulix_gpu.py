@@ -637,6 +637,20 @@ def test_rows_gemm_sizes_reach_every_tile():
     assert gated == set(range(14)) - {0, 9}       # no pairs of column tiles
 
 
+@pytest.mark.parametrize("M", [1, 3, 4, 7, 8, 16, 17, 32, 33])
+@pytest.mark.parametrize("N,K", [(512, 1536), (512, 1024), (512, 512),
+                                 (5632, 512), (512, 4096)])
+def test_linear_by_rows(M, N, K):
+    """Either side of the rows at which a product leaves the packed stream."""
+    from quickstart_streaming_agents_amd.models.layers import Linear
+    lin = Linear(rnd(gen(N + K), N, K, dtype=BF).to(DEV))
+    x = rnd(gen(M), M, K, dtype=BF).to(DEV)
+    a, b = x.double(), lin.w.double()
+    bound = 2.0 ** -8 * (a @ b.T).abs() + K * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    for got in (lin(x), D.add_shares(lin.parts(x))):
+        assert ((got.double() - a @ b.T).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("S", [2, 7, 16])
 @pytest.mark.parametrize("W", [8, 1032, 4096, 8200])
 def test_shares_meet_their_reader(S, W):
