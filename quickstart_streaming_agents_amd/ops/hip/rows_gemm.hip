@@ -62,13 +62,17 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Whether two blocks of eight waves share a CU's 160 KB (128 bytes a row and stage)
+constexpr bool rows_pair(int bm, int bn, int waves, int st) {
+  return waves == 8 && st * (bm + bn) * 128 <= 80 * 1024;
+}
+
 // BM x BN of C in a block of WM x WN waves, K in stages of 64 through a ring of
 // ST places in LDS; with ACT, W's rows are [gate; up] and a wave's column tiles
 // are alternately of either.
 template <int BM, int BN, int WM, int WN, int ST, int ACT>
 __global__ void __launch_bounds__(WM * WN * 64,
-                                  (ST * (BM + BN) * 128 <= 80 * 1024 ? 2 : 1) *
-                                      WM * WN / 4)
+                                  rows_pair(BM, BN, WM * WN, ST) ? 4 : 1)
 qsa_rows_gemm(RowsArgs p) {
 #ifdef __HIP_DEVICE_COMPILE__
   constexpr int NW = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16;
@@ -325,7 +329,7 @@ struct RowsTile {
 };
 static const RowsTile rows_tiles[] = {
 #define X(BM, BN, WM, WN, ST, OWN, STAGE)                              \
-  {BM, BN, WN, WM * WN == 8 && ST * (BM + BN) <= 640, OWN, STAGE},
+  {BM, BN, WN, rows_pair(BM, BN, WM * WN, ST), OWN, STAGE},
     QSA_TILES(X)
 #undef X
 };
