@@ -700,10 +700,17 @@ static bool gqa_aligned(const Tensor& q, const OptTensor& gate,
 
 // q [R, H*D] rows -> rows of out; row_item: which block_table row a query row
 // uses (none: its own index); row_len: position + 1 (0: row not in use)
-// Rows that fill the chip with four shares each may be finished by the block,
-// which saves the partial results and a launch; where rows are so many or so
-// short that a wave each is enough, three of its four waves are in the way.  us,
-// shares and a merge kernel / in the block, heads of 128, keys 8:
+// A row may be finished by the block, as four shares, which saves the partial
+// results and a launch: where rows fill the chip so, or are over before the merge
+// would start; where they are so many or so short that a wave each is enough,
+// three of its four waves are in the way.  us, shares and a merge kernel / in the
+// block, 16 heads of 128 on 8:
+//   1 row (8 tiles), 20-60 keys 9.1 / 5.7, 300-500 11.2 / 9.3, 500-1000 11.1 / 13.9
+//   15 rows (120)               9.8 / 5.8,         13.7 / 10.2,         19.6 / 20.6
+//   17 rows (136)              10.0 / 5.9,         16.6 / 11.0,         23.5 / 20.5
+//   24 rows (192), 500-1000 27.6 / 21.6, 1000-2000 40.2 / 35.2, 3000-4096 77 / 69
+//   17 rows (136)           23.5 / 20.5,           34.3 / 33.6,           58 / 62
+// and of many:
 //    64 rows (512 tiles), 10-60 keys 10.5 /  7.4, 400-1000 37.5 / 34.1
 //   256 rows (2048)            14.0 / 20.9,                79.9 / 71.7
 //   1024 rows (8192)           39.6 / 71.6,                 264 / 250
@@ -714,8 +721,10 @@ static bool gqa_aligned(const Tensor& q, const OptTensor& gate,
 // 50-300 (512) 26.7 / 21.6, 192 of 400-1000 (768) 90 / 76, 512 (2048) 136 / 141.
 // mp: the table's columns, as the rows' lengths are on the device.
 static bool gqa_merge_in_block(long long tiles, int mp, int D, int E) {
-  if (tiles < 512) return false;
   const int wide = std::max(D, E);
+  if (tiles < 512)
+    return wide <= 128 &&
+           (mp <= 8 || tiles >= 192 || (mp <= 16 && tiles >= 129));
   if (wide > 128)
     return tiles == 512 || (mp >= 8 && tiles <= (E <= 128 ? 1600 : 800));
   if (tiles <= 1024 || mp >= 8) return true;

@@ -552,6 +552,15 @@ def test_grouped_attention_forms(R, H, G, Dm, E, pages):
     close(out, want.reshape(R, -1), BF)
 
 
+# fewer than 512 tiles: up to 8 pages, 129 tiles to 16, 192 tiles
+@pytest.mark.parametrize("R,H,G,Dm,E,pages", [
+    (4, 16, 8, 128, 128, 8), (4, 16, 8, 128, 128, 9), (16, 8, 8, 64, 64, 16),
+    (43, 3, 3, 40, 72, 16), (43, 3, 3, 40, 72, 17), (24, 8, 8, 128, 128, 17),
+    (5, 2, 1, 136, 128, 3)])
+def test_grouped_attention_few_rows(R, H, G, Dm, E, pages):
+    test_grouped_attention_forms(R, H, G, Dm, E, pages)
+
+
 # ---- projections of larger decode batches -----------------------------------
 
 @pytest.mark.parametrize("M", [1, 33, 48, 49, 65, 97, 128, 129, 192])
