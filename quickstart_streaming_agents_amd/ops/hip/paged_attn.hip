@@ -664,7 +664,9 @@ extern "C" void qsa_kv_scatter_launch(const unsigned short* knew,
 // once for all heads, and every access is 16 bytes wide; the page's K groups
 // and V columns of neighbouring tokens lie together.  Bound by memory:
 // 45k tokens, 32/8 heads of 128: 468 (rotation) + 292 us (scatter by elements)
-// before, 234 us here (4.7 TB/s, what a copy reaches).
+// before, 224 us here (4.9 TB/s, what a copy reaches); few tokens are bound by
+// round trips, so all reads of a pass come before its writes (5 tokens 6.8 -> 4.3
+// us, 200 11.5 -> 6.1, 764 14.7 -> 7.8, the conversion's part among it).
 // ---------------------------------------------------------------------------
 template <int D>
 __global__ void __launch_bounds__(256)
@@ -696,31 +698,41 @@ qsa_rope_kv_scatter(unsigned short* __restrict__ q,        // [T, QH, D] strided
     float c[8], s[8];
     ldv<float, 8>(cos_t + at, c);
     ldv<float, 8>(sin_t + at, s);
-    unsigned short* qp = q + t * qstride + (long long)g * R * D + d;
-    for (int h = 0; h < R; ++h, qp += D) {
-      bf16x8_a x = *reinterpret_cast<bf16x8_a*>(qp);
-      bf16x8_a y = *reinterpret_cast<bf16x8_a*>(qp + D / 2);
-      rotate_pair(x, y, c, s);
-      *reinterpret_cast<bf16x8_a*>(qp) = x;
-      *reinterpret_cast<bf16x8_a*>(qp + D / 2) = y;
-    }
-    const long long row = t * kvstride + (long long)g * D + d;
-    bf16x8_a x = *reinterpret_cast<const bf16x8_a*>(k + row);
-    bf16x8_a y = *reinterpret_cast<const bf16x8_a*>(k + row + D / 2);
-    rotate_pair(x, y, c, s);
+    // all reads before the first write: few tokens are a chain of latencies
     const int slot = slots[t];
+    const long long row = t * kvstride + (long long)g * D + d;
+    bf16x8_a kx = *reinterpret_cast<const bf16x8_a*>(k + row);
+    bf16x8_a ky = *reinterpret_cast<const bf16x8_a*>(k + row + D / 2);
+    const bf16x8_a vx = *reinterpret_cast<const bf16x8_a*>(v + row);
+    const bf16x8_a vy = *reinterpret_cast<const bf16x8_a*>(v + row + D / 2);
+    unsigned short* qp = q + t * qstride + (long long)g * R * D + d;
+    for (int h = 0; h < R; h += 4, qp += 4 * D) {
+      bf16x8_a x[4], y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (h + j < R) {
+          x[j] = *reinterpret_cast<bf16x8_a*>(qp + j * D);
+          y[j] = *reinterpret_cast<bf16x8_a*>(qp + j * D + D / 2);
+        }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (h + j < R) {
+          rotate_pair(x[j], y[j], c, s);
+          *reinterpret_cast<bf16x8_a*>(qp + j * D) = x[j];
+          *reinterpret_cast<bf16x8_a*>(qp + j * D + D / 2) = y[j];
+        }
+    }
+    rotate_pair(kx, ky, c, s);
     if (slot >= 0) {
       const long long tile =
           ((long long)(slot / QSA_PAGE) * KVH + g) * D * QSA_PAGE;
       unsigned short* kp =
           kc + tile + ((d / 8) * QSA_PAGE + slot % QSA_PAGE) * 8;
-      *reinterpret_cast<bf16x8_a*>(kp) = x;
-      *reinterpret_cast<bf16x8_a*>(kp + D / 2 * QSA_PAGE) = y;
+      *reinterpret_cast<bf16x8_a*>(kp) = kx;
+      *reinterpret_cast<bf16x8_a*>(kp + D / 2 * QSA_PAGE) = ky;
     }
-    *reinterpret_cast<bf16x8_a*>(vt + i * VP + d) =
-        *reinterpret_cast<const bf16x8_a*>(v + row);
-    *reinterpret_cast<bf16x8_a*>(vt + i * VP + d + D / 2) =
-        *reinterpret_cast<const bf16x8_a*>(v + row + D / 2);
+    *reinterpret_cast<bf16x8_a*>(vt + i * VP + d) = vx;
+    *reinterpret_cast<bf16x8_a*>(vt + i * VP + d + D / 2) = vy;
   }
   __syncthreads();
   // lane = token: a wave's store is one column of the page's value tile
