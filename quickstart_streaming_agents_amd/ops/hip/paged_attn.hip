@@ -118,10 +118,6 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   constexpr int DTILES = D / 16;      // PV d-tiles (8 for D=128)
   constexpr int VT = D * QSA_PAGE;    // elements of a value page
   constexpr int KL = 4 * KSTEPS;      // loads of a wave for a page's keys
-  // Values are asked for a page ahead where few rows leave latencies to hide, and
-  // where many share the memory once the page's keys are there: with four waves
-  // a page ahead made 33 rows of 3000-4000 keys 103 -> 104 us, so 100.
-  constexpr bool EARLY = NW == 8;
   // a wave's values, afterwards its part of the output [R][D]
   __shared__ __attribute__((aligned(16))) unsigned short vlds[NW * VT];
   __shared__ float ml[2 * NW * 16];   // and its maxima and sums
@@ -214,7 +210,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         ldv<float, 8>(p.sin_t + at + ks * 32, sn[ks]);
       }
     }
-    if constexpr (EARLY) load_v(page);  // behind all that the scores wait for
+    load_v(page);                     // behind all that the scores wait for
     if constexpr (FUSE) {
 #pragma unroll
       for (int ks = 0; ks < KSTEPS / 2; ++ks) {
@@ -224,9 +220,10 @@ qsa_paged_attn_mfma(DecodeArgs p) {
     }
 
     // Page pi; the keys of the wave's next one are asked for once these have been
-    // multiplied.  The last page is code of its own, or the waits of both would be
-    // for all that is under way.  patch: the row's last page, where the new token
-    // has its place.
+    // multiplied, its values once these have (values only behind the page's own
+    // keys: 100 rows of 400-1000 keys +1 %, 33 of 3000-4000 -3 %).  The last page is
+    // code of its own, or the waits of both would be for all that is under way.
+    // patch: the row's last page, where the new token has its place.
     auto walk = [&](int pi, auto last) {
       const int after = btab[min(pi + 2 * step, p.max_pages - 1)];
       const int nvalid = min(seqlen - pi * QSA_PAGE, QSA_PAGE);
@@ -251,7 +248,6 @@ qsa_paged_attn_mfma(DecodeArgs p) {
                                                         acc, 0, 0, 0);
         sc[pt] = acc;
       }
-      if constexpr (!EARLY) load_v(page);
       if constexpr (!last.value) load_k(next, kf);
       // scale + mask invalid positions; C layout: row pos = hi*4 + r,
       // col head = lane&15 -> lane's r-th value is position pt*16 + hi*4 + r
@@ -366,7 +362,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         // all of the values have been read when the next page's come
         __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0)
         asm volatile("" ::: "memory");
-        if constexpr (EARLY) load_v(next);
+        load_v(next);
         page = next;
         next = after;
       }
