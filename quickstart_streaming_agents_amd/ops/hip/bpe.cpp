@@ -11,7 +11,6 @@
 #include <cstring>
 #include <string>
 #include <string_view>
-#include <unordered_map>
 #include <vector>
 
 namespace py = pybind11;
@@ -76,13 +75,24 @@ class Bpe {
   // merges: pairs of symbols, 0..255 bytes and 256 + i what merge i makes;
   // specials: texts that are a token of their own, in order of preference;
   // base: token of byte 0
-  Bpe(const std::vector<std::pair<uint32_t, uint32_t>>& merges,
+  Bpe(const py::list& merges,
       std::vector<std::pair<std::string, int>> specials, int base)
       : specials_(std::move(specials)), base_(base) {
     for (const auto& sp : specials_) starts_[(unsigned char)sp.first[0]] = true;
     clear();
-    for (size_t i = 0; i < merges.size(); ++i)
-      merged_[key(merges[i].first, merges[i].second)] = 256 + (uint32_t)i;
+    size_t places = 16;
+    while (places < 2 * merges.size()) places *= 2;
+    merged_.assign(places, {0, 0});
+    for (size_t i = 0; i < merges.size(); ++i) {
+      PyObject* pair = PyList_GET_ITEM(merges.ptr(), (Py_ssize_t)i);
+      if (!PyTuple_Check(pair) || PyTuple_GET_SIZE(pair) != 2)
+        throw py::type_error("a merge is a pair of symbols");
+      const unsigned long a = PyLong_AsUnsignedLong(PyTuple_GET_ITEM(pair, 0));
+      const unsigned long b = PyLong_AsUnsignedLong(PyTuple_GET_ITEM(pair, 1));
+      if (PyErr_Occurred()) throw py::error_already_set();
+      *find(key((uint32_t)a, (uint32_t)b)) = {
+          key((uint32_t)a, (uint32_t)b), 256 + (uint32_t)i};
+    }
   }
 
   py::list encode(const py::str& text, int first) {
@@ -112,8 +122,21 @@ class Bpe {
   }
 
  private:
-  static constexpr size_t kKeep = 65536, kWord = 64;
-  static uint64_t key(uint32_t a, uint32_t b) { return (uint64_t)a << 32 | b; }
+  static constexpr size_t kKeep = 65536, kWord = 64, kStart = 2048;
+  struct Merge {
+    uint64_t key;                                 // 0: a free place
+    uint32_t symbol;
+  };
+  static uint64_t key(uint32_t a, uint32_t b) {
+    return ((uint64_t)a << 32 | b) + 1;
+  }
+
+  Merge* find(uint64_t k) {            // its place, or the free one for it
+    size_t at = (k * 0x9e3779b97f4a7c15ull >> 32) & (merged_.size() - 1);
+    while (merged_[at].key && merged_[at].key != k)
+      at = (at + 1) & (merged_.size() - 1);
+    return &merged_[at];
+  }
 
   void run(const py::str& text, int first, std::vector<int32_t>& ids) {
     Py_ssize_t n = 0;
@@ -149,7 +172,8 @@ class Bpe {
     }
   }
 
-  // A word's tokens, once found, stay in an open table of twice kKeep places.
+  // A word's tokens, once found, stay in an open table of at least twice as many
+  // places, which grows up to kKeep words.
   void word(std::string_view w, std::vector<int32_t>& ids) {
     if (w.size() > kWord) {
       merge(w);
@@ -157,8 +181,8 @@ class Bpe {
       return;
     }
     const uint64_t h = hash(w);
-    size_t at = h % (2 * kKeep);
-    for (; table_[at]; at = (at + 1) % (2 * kKeep)) {
+    size_t at = h & (table_.size() - 1);
+    for (; table_[at]; at = (at + 1) & (table_.size() - 1)) {
       const Known& k = known_[table_[at] - 1];
       if (k.hash == h && k.size == w.size() &&
           std::memcmp(bytes_.data() + k.word, w.data(), w.size()) == 0) {
@@ -169,9 +193,11 @@ class Bpe {
     }
     merge(w);
     ids.insert(ids.end(), syms_.begin(), syms_.end());
-    if (known_.size() >= kKeep) {
-      clear();
-      at = h % (2 * kKeep);
+    if (2 * known_.size() >= table_.size()) {
+      if (known_.size() >= kKeep) clear();
+      else grow();
+      for (at = h & (table_.size() - 1); table_[at];)
+        at = (at + 1) & (table_.size() - 1);
     }
     known_.push_back({h, (uint32_t)bytes_.size(), (uint32_t)w.size(),
                       (uint32_t)tokens_.size(), (uint32_t)syms_.size()});
@@ -191,8 +217,17 @@ class Bpe {
     return h;
   }
 
+  void grow() {
+    table_.assign(2 * table_.size(), 0);
+    for (size_t i = 0; i < known_.size(); ++i) {
+      size_t at = known_[i].hash & (table_.size() - 1);
+      while (table_[at]) at = (at + 1) & (table_.size() - 1);
+      table_[at] = 1 + (uint32_t)i;
+    }
+  }
+
   void clear() {
-    table_.assign(2 * kKeep, 0);
+    table_.assign(kStart, 0);
     known_.clear();
     bytes_.clear();
     tokens_.clear();
@@ -207,9 +242,9 @@ class Bpe {
       uint32_t best = UINT32_MAX;
       size_t at = 0;
       for (size_t i = 0; i + 1 < syms_.size(); ++i) {
-        const auto m = merged_.find(key(syms_[i], syms_[i + 1]));
-        if (m != merged_.end() && m->second < best) {
-          best = m->second;
+        const Merge* m = find(key(syms_[i], syms_[i + 1]));
+        if (m->key && m->symbol < best) {
+          best = m->symbol;
           at = i;
         }
       }
@@ -220,7 +255,7 @@ class Bpe {
     for (auto& x : syms_) x += base_;
   }
 
-  std::unordered_map<uint64_t, uint32_t> merged_;
+  std::vector<Merge> merged_;                     // open, half full at most
   struct Known {
     uint64_t hash;
     uint32_t word, size, first, count;            // in bytes_ and tokens_
@@ -239,7 +274,7 @@ class Bpe {
 
 void register_bpe(py::module_& m) {
   py::class_<Bpe>(m, "Bpe")
-      .def(py::init<const std::vector<std::pair<uint32_t, uint32_t>>&,
+      .def(py::init<const py::list&,
                     std::vector<std::pair<std::string, int>>, int>())
       .def("encode", &Bpe::encode)
       .def("encode_batch", &Bpe::encode_batch);
