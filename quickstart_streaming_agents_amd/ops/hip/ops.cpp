@@ -254,10 +254,20 @@ static torch::Tensor decode_attention(
   TORCH_CHECK(vc.size(2) == D && vc.size(3) == 64,
               "V cache layout [P, KVH, D, 64] (transposed)");
   TORCH_CHECK(!step || (B >= 1 && B <= 32), "step rows: B in [1,32]");
+  TORCH_CHECK(block_table.dim() == 2 && seq_lens.numel() >= B,
+              "block_table [B, pages], a length per row");
   const int max_pages = block_table.size(1);
   const int mt = step ? step_tiles(B) : 0;
   auto out = mt ? step_rows(B, (long)QH * D, q.options())
                 : torch::empty({B, QH, D}, q.options());
+  // Every row's first page is read beside its length, so a table without pages
+  // (all rows empty) and one without the last rows (these empty) have no launch
+  // or get the rows.
+  if (B == 0 || max_pages == 0) return out.zero_();
+  const torch::Tensor table =
+      block_table.size(0) >= B
+          ? block_table
+          : at::constant_pad_nd(block_table, {0, 0, 0, B - block_table.size(0)});
   int waves, ns;
   qsa_paged_attn_split(B, QH, KVH, max_pages, D, &waves, &ns);
   torch::Tensor part_o, part_ml;
@@ -277,12 +287,21 @@ static torch::Tensor decode_attention(
   }
   qsa_paged_attn_mfma_launch(
       u16(q), k ? u16(*k) : nullptr, v ? u16(*v) : nullptr, u16m(kc), u16m(vc),
-      cos_t, sin_t, block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
+      cos_t, sin_t, table.data_ptr<int>(), seq_lens.data_ptr<int>(),
       ns > 1 ? part_o.data_ptr<float>() : nullptr,
       ns > 1 ? part_ml.data_ptr<float>() : nullptr, u16m(out), (float)scale, B,
       QH, KVH, max_pages, D, q.stride(0), k ? k->stride(0) : 0, waves, ns, mt,
       at, bytes, cur_stream());
   return out;
+}
+
+// (waves of a block, blocks per row and key head) that decode_attention takes
+std::tuple<int, int> paged_attn_split(long B, long QH, long KVH,
+                                      long max_pages, long D) {
+  int waves, ns;
+  qsa_paged_attn_split((int)B, (int)QH, (int)KVH, (int)max_pages, (int)D,
+                       &waves, &ns);
+  return {waves, ns};
 }
 
 torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor kc,
@@ -850,6 +869,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("causal"), py::arg("rows") = 16);
   m.def("paged_attn_decode", &paged_attn_decode,
         "paged-attention decode (bf16, GQA, page=64)");
+  m.def("paged_attn_split", &paged_attn_split,
+        "waves and blocks of a decoding step's attention");
   m.def("paged_attn_step", &paged_attn_step,
         "a decoding step's rotation, cache append and attention",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("kc"),

@@ -466,6 +466,7 @@ extern "C" void qsa_paged_attn_split(int B, int QH, int KVH, int max_pages,
   const bool few = max_pages <= 16;
   *waves = heads > 256 || max_pages <= 4 || (heads <= 48 && !few) ? 4 : 8;
   *splits = 1;
+  if (heads == 0) return;
   if (heads > 256) {
     if (heads < 384 && max_pages > 32) *splits = 3;
   } else if (!few && heads <= 128) {

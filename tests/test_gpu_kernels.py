@@ -1179,3 +1179,31 @@ def test_llama_batched_decode_routes_fp8():
     rel = (out.float() - ref).abs().max().item() / \
         (ref.abs().std().item() + 1e-6)
     assert rel < 0.5
+
+
+@pytest.mark.parametrize("fuse", [False, True])
+def test_paged_attn_without_pages(ext, fuse):
+    """No rows, a table without columns, one without the last, empty rows."""
+    B, QH, KVH, D = 5, 8, 4, 64
+    kc, vc, bt = _make_paged_kv(B, KVH, D, [70, 3, 1, 0, 0], 5)
+    kept = kc.clone(), vc.clone()
+    qkv = torch.randn(B, (QH + 2 * KVH) * D, device=dev()).bfloat16()
+    rot = torch.rand(128, D // 2, device=dev())
+
+    def run(rows, table, lens):
+        q, k, v = (t.view(B, -1, D)[:rows] for t in
+                   qkv.split([QH * D, KVH * D, KVH * D], 1))
+        sl = torch.tensor(lens, dtype=torch.int32, device=dev())
+        if not fuse:
+            return ext.paged_attn_decode(q, kc, vc, table, sl, 0.125)
+        return ext.paged_attn_step(q, k, v, kc, vc, rot, rot, table, sl,
+                                   0.125, False)
+
+    assert run(0, bt[:0], []).shape == (0, QH, D)
+    assert run(0, bt[:0, :1].expand(0, 40).contiguous(), []).numel() == 0
+    none = run(B, bt[:, :0].contiguous(), [0] * B)
+    assert none.shape == (B, QH, D) and not none.any()
+    assert torch.equal(kc, kept[0]) and torch.equal(vc, kept[1])
+    want = run(B, bt, [70, 3, 1, 0, 0])
+    assert torch.equal(run(B, bt[:3].contiguous(), [70, 3, 1, 0, 0]), want)
+    assert want[:3].any() and not want[3:].any()
