@@ -105,8 +105,11 @@ __device__ __forceinline__ void rotate_pair(bf16x8_a& a, bf16x8_a& b,
   b = __builtin_bit_cast(bf16x8_a, v);
 }
 
-// Up to 63 of a wave's loads under way, whatever it stored or read from LDS.
+// Up to 63 of a wave's loads under way, whatever it stored or read from LDS.  It
+// counts, so no load may pass it either way (tests/test_isa_audit.py looks at what
+// stands before it).
 template <int N> __device__ __forceinline__ void wait_vm() {
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 7 << 4 | 15 << 8);
   asm volatile("" ::: "memory");
 }
@@ -363,6 +366,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
         __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0)
         asm volatile("" ::: "memory");
         load_v(next);
+        asm volatile("" ::: "memory");            // and no key's load before
         page = next;
         next = after;
       }

@@ -4,7 +4,9 @@ register spills or scratch (CDNA4 guide rule: runtime-indexed register
 arrays spill silently)."""
 
 import os
+import re
 import sys
+import tempfile
 
 import pytest
 
@@ -69,6 +71,48 @@ def test_matrix_kernels_use_mfma(stats):
     for frag in ("encoder_attn", "short_gemm", "topk_scan"):
         for name, st in _named(stats, frag).items():
             assert st["mfma"] >= 4, f"{name}: only {st['mfma']} v_mfma"
+
+
+def counted_waits(code, loads):
+    """Waits for all but `loads` of a wave's loads that have exactly so many,
+    16 bytes a lane into registers, before them since the last branch, with
+    no read of LDS by 16 bytes between."""
+    found, run, vm = 0, [], re.compile(r"(global|buffer|flat|scratch)_")
+    for text in code:
+        if not text or text.startswith(("s_cbranch", "s_branch")):
+            run = []
+        elif vm.match(text) or text.startswith("ds_read_b128"):
+            run.append(text)
+        elif re.match(rf"s_waitcnt vmcnt\({loads}\)", text):
+            found += len(run) == loads and all(
+                t.startswith("global_load_dwordx4") for t in run)
+    return found
+
+
+def test_counted_waits_of_decode_attention():
+    """A page's values are there when the next page's keys, loaded behind them,
+    need not be: right only with these keys and nothing else in between."""
+    import isa_check
+    so = isa_check.find_so()
+    if so is None or not os.path.exists(isa_check.BUNDLER):
+        pytest.skip("built extension or ROCm LLVM tools unavailable")
+    with tempfile.TemporaryDirectory() as wd:
+        kernels = isa_check.instructions(
+            isa_check.extract_hsacos(so, wd), "qsa_paged_attn_mfma")
+    assert len(kernels) == 8
+    for name, code in kernels.items():
+        keys = 16 if "ILi128E" in name else 8
+        assert counted_waits(code, keys) == 1, name
+
+
+def test_the_audit_sees_a_moved_load():
+    keys = ["global_load_dwordx4 v[0:3], v[4:5], off"] * 2
+    wait = ["s_waitcnt vmcnt(2)"]
+    assert counted_waits(keys + wait, 2) == 1
+    assert counted_waits(keys[:1] + wait + keys[1:], 2) == 0
+    assert counted_waits(keys + ["global_load_dword v1, v2, off"] + wait, 2) == 0
+    assert counted_waits(keys[:1] + [""] + keys[1:] + wait, 2) == 0
+    assert counted_waits(keys + ["ds_read_b128 v[0:3], v9"] + wait, 2) == 0
 
 
 def test_no_spills_or_scratch_on_hot_kernels(stats):

@@ -101,6 +101,26 @@ def kernel_stats(hsacos: list[str]) -> dict[str, dict]:
     return stats
 
 
+def instructions(hsacos: list[str], fragment: str) -> dict[str, list[str]]:
+    """Kernels whose name has the fragment -> their instructions; a branch's
+    target is an empty line before."""
+    out: dict[str, list[str]] = {}
+    for h in hsacos:
+        dis = subprocess.run(
+            [os.path.join(LLVM, "llvm-objdump"), "-d", "--mcpu=gfx950",
+             "--symbolize-operands", h], capture_output=True, text=True).stdout
+        cur = None
+        for line in dis.splitlines():
+            m = re.match(r"^(?:[0-9a-f]+ )?<(.+)>:", line)
+            if m and not re.fullmatch(r"L\d+", m.group(1)):
+                cur = m.group(1)
+            elif cur and fragment in cur:
+                text = "" if m else line.split("//")[0].strip()
+                if m or text:
+                    out.setdefault(cur, []).append(text)
+    return out
+
+
 def main() -> int:
     found = [so for so in map(find_so, ("qsa_hip", "qsa_lm_hip")) if so]
     if not found:
