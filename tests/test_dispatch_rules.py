@@ -4,6 +4,8 @@ from __future__ import annotations
 
 import pytest
 
+import torch
+
 from quickstart_streaming_agents_amd.ops import ext, have_ext
 
 pytestmark = pytest.mark.skipif(not have_ext(), reason="extension not built")
@@ -13,3 +15,90 @@ pytestmark = pytest.mark.skipif(not have_ext(), reason="extension not built")
 def test_decode_attention_of_no_rows(pages):
     """A batch without rows has no blocks to share its pages."""
     assert ext().paged_attn_split(0, 32, 8, pages, 128)[1] == 1
+
+
+# rows, key heads, pages: either side of every line of the rule, tables that a
+# block of eight waves walks once, twice and often
+SPLITS = [(12, 4, 4), (12, 4, 5), (12, 4, 16), (12, 4, 17), (7, 7, 16),
+          (7, 7, 17), (8, 8, 33), (13, 5, 16), (13, 5, 17), (13, 5, 40),
+          (16, 8, 17), (16, 8, 33), (43, 3, 16), (43, 3, 17), (43, 3, 33),
+          (32, 8, 4), (32, 8, 17), (32, 8, 40), (257, 1, 32), (257, 1, 33),
+          (257, 1, 50), (383, 1, 33), (48, 8, 33), (1, 1, 70), (1, 8, 130),
+          (5, 1, 17), (3, 2, 64)]
+
+
+def _kind(pairs, pages, heads=1):
+    """Waves and blocks; of few rows any number of blocks, as 2."""
+    waves, blocks = ext().paged_attn_split(pairs // heads, 2 * heads, heads,
+                                           pages, 128)
+    return waves, min(blocks, 2) if pairs <= 48 else blocks
+
+
+def test_sizes_reach_every_split():
+    want = {_kind(pairs, pages) for pairs in range(1, 520)
+            for pages in range(1, 200)}
+    assert len(want) == 6
+    assert {_kind(b * g, n, g) for b, g, n in SPLITS} == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("rows,heads,pages", SPLITS)
+def test_decode_attention_splits(rows, heads, pages, D):
+    """Lengths of no key, one, ends of pages, fewer pages than a row has waves
+    and the whole table, whose other columns point anywhere."""
+    g = torch.Generator().manual_seed(rows + pages)
+    R, top = 3, pages * 64
+    lens = torch.randint(1, top + 1, (rows,), generator=g)
+    some = [top, 0, 1, 64, 65, top - 63, 5 * 64, 9 * 64 + 1, top - 64]
+    lens[:len(some)] = torch.tensor(some)[:rows].clamp(0, top)
+    used = [-(-int(n) // 64) for n in lens]
+    total = sum(used) + 1
+    table = torch.randint(0, total, (rows, pages), generator=g,
+                          dtype=torch.int32)
+    order, at = torch.randperm(total, generator=g).int(), 0
+    for i, n in enumerate(used):
+        table[i, :n] = order[at:at + n]
+        at += n
+    dev, bf = "cuda:0", torch.bfloat16
+
+    def rnd(*s):
+        return torch.randn(*s, device=dev, dtype=bf)
+
+    torch.manual_seed(pages)
+    kc, vc = rnd(total, heads, D // 8, 64, 8), rnd(total, heads, D, 64)
+    qkv = rnd(rows, (R + 2) * heads * D)
+    q, k, v = (t.view(rows, -1, D) for t in qkv.split(
+        [R * heads * D, heads * D, heads * D], 1))
+    rot = torch.rand(top, D // 2, device=dev) * 6.28
+    cos, sin = rot.cos(), rot.sin()
+    bt, sl = table.to(dev), lens.int().to(dev)
+
+    def check(out, q):
+        for i, n in enumerate(lens.tolist()):
+            if n == 0:
+                assert not out[i].any()
+                continue
+            p = bt[i, :used[i]].long()
+            ks = kc[p].permute(1, 0, 3, 2, 4).reshape(heads, -1, D)[:, :n]
+            vs = vc[p].permute(1, 0, 3, 2).reshape(heads, -1, D)[:, :n]
+            qs = q[i].view(heads, R, D).float()
+            s = torch.matmul(qs, ks.float().transpose(1, 2).contiguous())
+            ref = torch.matmul((s * D ** -0.5).softmax(-1), vs.float())
+            err = out[i].view(heads, R, D).float() - ref
+            # probabilities and the result are rounded to bf16, 2^-9 each
+            assert err.norm() <= 5e-3 * ref.norm(), (i, n)
+            assert err.abs().max() <= 2 ** -7 * vs.abs().max(), (i, n)
+
+    # the step first: it writes the new keys and values that both attend to
+    out = ext().paged_attn_step(q, k, v, kc, vc, cos, sin, bt, sl, D ** -0.5,
+                                False)
+    live = sl > 0
+    pos = (sl - 1).clamp(min=0)
+    turned = q.clone()
+    ext().rope_inplace(turned, k.clone(), cos, sin, pos)
+    check(out, turned)
+    i = live.nonzero()[:, 0]
+    slot = bt[i, (pos[i] // 64).long()].long(), (pos[i] % 64).long()
+    assert torch.equal(vc[slot[0], :, :, slot[1]], v[i])
+    check(ext().paged_attn_decode(turned, kc, vc, bt, sl, D ** -0.5), turned)
