@@ -5,6 +5,7 @@ from __future__ import annotations
 import copy
 import pickle
 import random
+import time
 
 import pytest
 
@@ -73,3 +74,43 @@ def test_copies_and_pickles():
         assert other._native is not None
         assert other.encode("a window<|finish|> of 12") == \
             tok.encode("a window<|finish|> of 12")
+
+
+@pytest.mark.parametrize("n", [47, 48, 49, 64, 65, 200, 900])
+def test_long_words(n):
+    """Above some 48 bytes pairs are merged from a heap, in the same order."""
+    for vocab in (300, 1024, 30_522):
+        tok, r = BpeTokenizer(vocab), random.Random(n)
+        for letters in ("ab", "aeinorst", "abcdefghijklmnopqrstuvwxyz"):
+            for size in (n, n + r.randint(1, 40)):
+                word = "".join(r.choices(letters, k=size))
+                want = tok._encode(word, True)
+                assert tok.encode(word) == want
+                assert tok.encode(word) == want           # and as it is kept
+        word = "streaming" * (n // 9 + 1)
+        assert tok.encode(word + " " + word) == tok._encode(
+            word + " " + word, True)
+
+
+def test_long_words_take_no_square_of_their_length():
+    """20,000 letters were 1.2 s each time; now once some 10 ms."""
+    tok, r = BpeTokenizer(30_522), random.Random(1)
+    word = "".join(r.choices("abcdefghijklmnopqrstuvwxyz", k=20_000))
+    t = time.perf_counter()
+    for _ in range(50):
+        ids = tok.encode(word)
+    assert time.perf_counter() - t < 5
+    assert tok.decode(ids) == word
+
+
+def test_a_batch_reads_no_further_than_it_keeps():
+    tok = BpeTokenizer(30_522)
+    text = "one window " * 50_000 + "<|finish|>"
+    t = time.perf_counter()
+    for _ in range(200):
+        ids, lens = tok.encode_batch([text, "a<|finish|>b"], 3)
+    assert time.perf_counter() - t < 5
+    assert ids.tolist() == tok._encode(text[:100], True)[:3] + \
+        tok._encode("a<|finish|>b", True)[:3] and lens.tolist() == [3, 3]
+    with pytest.raises(UnicodeEncodeError):
+        tok.encode_batch([text + "\ud800"], 3)
