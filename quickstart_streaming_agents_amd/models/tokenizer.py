@@ -107,9 +107,11 @@ class BpeTokenizer:
         self._load_native()
 
     def _load_native(self):
-        """The same in native code, where it is built (ops/hip/bpe.cpp)."""
+        """The same in native code, where it is built (ops/hip/bpe.cpp).  Not for
+        an empty special or none at all, at which the pattern splits a text
+        between any two characters."""
         self._native = None
-        if have_ext() and all(self.specials):
+        if have_ext() and self.specials and all(self.specials):
             self._native = ext().Bpe(self._merges,
                                      list(self.specials.items()), self._BYTE0)
 

@@ -3,12 +3,14 @@
 from __future__ import annotations
 
 import copy
+import json
 import pickle
 import random
 import time
 
 import pytest
 
+from quickstart_streaming_agents_amd.models import tokenizer
 from quickstart_streaming_agents_amd.models.tokenizer import BpeTokenizer
 from quickstart_streaming_agents_amd.ops import have_ext
 
@@ -114,3 +116,16 @@ def test_a_batch_reads_no_further_than_it_keeps():
         tok._encode("a<|finish|>b", True)[:3] and lens.tolist() == [3, 3]
     with pytest.raises(UnicodeEncodeError):
         tok.encode_batch([text + "\ud800"], 3)
+
+
+@pytest.mark.parametrize("specials", [{}, {"": 3}, {"<|eot|>": 2}])
+def test_vocabularies_of_other_specials(specials, tmp_path):
+    with open(tokenizer._VOCAB_PATH) as f:
+        vocab = dict(json.load(f), specials=specials)
+    path = tmp_path / "vocab.json"
+    path.write_text(json.dumps(vocab))
+    tok = BpeTokenizer(1024, str(path))
+    for text in ("one window<|eot|> of 12", "", "a"):
+        assert tok.encode(text) == tok._encode(text, True)
+        ids, _ = tok.encode_batch([text], 99)
+        assert ids.tolist() == tok._encode(text, True)
