@@ -1,16 +1,20 @@
 // GEMM of a short K for CDNA4 (gfx950): C[M,N] = A[M,K] @ W[N,K]^T, bf16 with f32
 // sums, and with GLU silu(gate) * up of it, W's rows being [gate; up]: the
-// encoder's projections of few rows.
+// encoder's projections, of few rows beside rows_gemm.hip and of any where that
+// module is not built.
 //
-// With a few steps of K a product is over before a deep pipeline is full, and few
-// tiles leave nothing to overlap with, so: tiles of 32 x 64, K in steps of 64
-// through two halves of LDS with the next one in registers, whole 128-byte lines
-// of every operand, a block row's columns on one die, results through LDS to
-// whole lines, and the gate's columns beside the up's in a wave, so that the
-// activation costs no pass over memory.  Larger products are rows_gemm.hip's.
+// With a few steps of K a product is over before a deep pipeline is full; its
+// reads and writes and, for few rows, the host's way to a library's kernel count
+// as much as the matrix cores.  So: tiles by the number of blocks they leave, K in
+// steps of 64 through two halves of LDS with the next one in registers, whole
+// 128-byte lines of every operand, a block row's columns on one die, results
+// through LDS to whole lines, and the gate's columns beside the up's in a wave, so
+// that the activation costs no pass over memory.
 // us, library / rows_gemm -> here:
 //   384 x 512  at 100 / 400 / 1000 rows 5.4 / 5.5 / 6.2, 4.5 -> 4.2 / 4.3 / 4.4
 //   1536 x 384 at 40 rows 5.0, 4.1 -> 3.8;  512 x 256 at 700 5.1, 4.0 -> 3.6
+//   at 8800 rows 1536 x 384 18.3, 17.0 -> 20.7, 384 x 512 10.7, 8.0 -> 11.7, 3072
+//   x 384 with the activation 72, 32 -> 34.8
 #include "lm_common.h"
 
 struct ShortArgs {
@@ -169,10 +173,20 @@ static void short_go(ShortArgs p, int glu, hipStream_t st) {
                        p);
 }
 
+// Tiles of 128 x 128 once two rounds of blocks are left, 64 x 64 while they
+// make half a round, 32 x 64 below (384 x 512 at 400 rows: 8.2 / 4.5 / 3.7 us;
+// 1536 x 384 at 1600: 7.9 / 6.8 / 8.0, at 8800: 20.9 / 23.0 / 28.4; 3072 x 384
+// with the activation at 16,000: 58 with 128 x 128, 94 with 32 x 64).
 extern "C" void qsa_short_gemm_launch(const bf16_t* A, const bf16_t* W,
                                       bf16_t* C, int M, int N, int K,
                                       long long lda, int glu,
                                       hipStream_t st) {
   if (M == 0) return;
-  short_go<1, 2>({A, W, C, M, N, K, 0, lda}, glu, st);
+  const ShortArgs p{A, W, C, M, N, K, 0, lda};
+  auto blocks = [&](int b) {
+    return (long long)((M + b - 1) / b) * ((N + b - 1) / b);
+  };
+  if (blocks(128) >= 512) short_go<4, 4>(p, glu, st);
+  else if (blocks(64) >= 128) short_go<2, 2>(p, glu, st);
+  else short_go<1, 2>(p, glu, st);
 }
