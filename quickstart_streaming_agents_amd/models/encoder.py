@@ -26,6 +26,7 @@ import torch
 import torch.nn.functional as F
 
 from ..ops import dispatch as D
+from ..ops import have_ext, have_lm_ext
 from ..vector.index import EMBED_DIM
 from .layers import ints_to_device
 from .tokenizer import BpeTokenizer
@@ -94,18 +95,25 @@ class EmbeddingEncoder:
         5.5 in the library), the others rows_gemm's: at 8800 rows 1536 x 384
         takes 17.0 us (short_gemm 20.7, the library 18.3), 3072 x 384 with the
         activation 32 (36, 72 with a pass of its own), 384 x 512 8.0 (10.5,
-        10.7), 384 x 1536 14.6 (23.4, 17.2)."""
+        10.7), 384 x 1536 14.6 (23.4, 17.2).  With qsa_hip alone they are
+        short_gemm's and, of long K and many rows, the library's."""
         n, k = w.shape
-        if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
-                n % 32 == 0 and (k <= 512 or x.shape[0] <= 32) and \
-                -(-x.shape[0] // 32) * -(-n // 64) <= 192:
-            return D.ext().short_gemm(x, w, glu)
-        if not glu:
-            return D.linear_parts(x, w) if parts else D.linear(x, w)
-        if D.glu_linear_ok(x, w):
-            return D.glu_linear(x, w, "silu", rounded=False)
+        rows = x.shape[0]
+        fits = x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
+            n % 32 == 0
+        if not have_lm_ext():            # rows_gemm is that module's
+            if fits and (k <= 512 or rows <= 2048):
+                return D.ext().short_gemm(x, w, glu)
+        else:
+            if fits and (k <= 512 or rows <= 32) and \
+                    -(-rows // 32) * -(-n // 64) <= 192:
+                return D.ext().short_gemm(x, w, glu)
+            if not glu:
+                return D.linear_parts(x, w) if parts else D.linear(x, w)
+            if D.glu_linear_ok(x, w):
+                return D.glu_linear(x, w, "silu", rounded=False)
         y = F.linear(x, w)
-        return D.swiglu(y[:, :n // 2], y[:, n // 2:])
+        return D.swiglu(y[:, :n // 2], y[:, n // 2:]) if glu else y
 
     # -- varlen attention plumbing (GPU path) ------------------------------
     QROWS = 64      # query tokens per attention block: one 16-row tile a wave
@@ -207,7 +215,6 @@ class EmbeddingEncoder:
         c = self.cfg
         ids, lens = self.tokenizer.encode_batch(list(texts), c.max_pos)
         # mean over the tokens, project, L2-normalize
-        from ..ops import have_ext
         if self._use_hip and have_ext():
             out = self._linear(self._embed_rows(ids, lens).to(self.dtype),
                                self.proj)

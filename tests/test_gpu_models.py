@@ -634,3 +634,18 @@ def test_generic_sql_lab1_model_driven_on_engine():
     assert all(r["agent_status"] in ("SUCCESS", "FAILED") for r in rows)
     ids = [r["order_id"] for r in rows]
     assert len(ids) == len(set(ids))
+
+
+def test_encoder_needs_one_module(monkeypatch):
+    """qsa_hip alone serves the encoder; products in other tiles differ in the
+    order of their f32 sums and in whether the gate is rounded before it acts."""
+    from quickstart_streaming_agents_amd import ops
+    from quickstart_streaming_agents_amd.models.encoder import EmbeddingEncoder
+    enc = EmbeddingEncoder(device="cuda:0")
+    for n in (1, 40):                    # a few rows, and beyond 2048
+        texts = [f"ticket {i} about the harbor route " * 20 for i in range(n)]
+        want = enc.embed_batch(texts)
+        with monkeypatch.context() as m:
+            m.setattr(ops, "_lm_ext", None)
+            got = enc.embed_batch(texts)
+        assert np.abs(got - want).max() <= 0.02 * np.abs(want).max()
