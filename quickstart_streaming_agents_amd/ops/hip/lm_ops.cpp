@@ -132,7 +132,7 @@ extern "C" void qsa_window_attn_prefill_launch(const bf16_t*, long long,
     const int*, bf16_t*, int, int, int, int, int, float, hipStream_t);
 extern "C" void qsa_skinny_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     int, int, long long, long long, hipStream_t);
-extern "C" int qsa_rows_gemm_plan(int, int, int, int, int, int*);
+extern "C" int qsa_rows_gemm_plan(int, int, int, int, int, int*, float*);
 extern "C" void qsa_rows_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     float*, int, int, int, long long, int, int, int, hipStream_t);
 
@@ -1031,7 +1031,7 @@ static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
               "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
   const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
   int S;
-  const int tile = qsa_rows_gemm_plan(M, N, K, act, parts, &S);
+  const int tile = qsa_rows_gemm_plan(M, N, K, act, parts, &S, nullptr);
   Tensor out, part;
   if (S > 1) part = torch::empty({S, M, N}, a.options().dtype(at::kFloat));
   if (S == 1 || !parts) out = torch::empty({M, act ? N / 2 : N}, a.options());
@@ -1045,7 +1045,8 @@ static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
 std::tuple<int, int> rows_gemm_plan(int64_t M, int64_t N, int64_t K,
                                     bool glu) {
   int S;
-  const int tile = qsa_rows_gemm_plan((int)M, (int)N, (int)K, glu, 0, &S);
+  const int tile = qsa_rows_gemm_plan((int)M, (int)N, (int)K, glu, 0, &S,
+                                      nullptr);
   return {tile, S};
 }
 

@@ -314,7 +314,7 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
 // 2048 x 128 15.7, 13.0; 30,000 38.2, 30.7; 4400 x 16384 x 2048 263, 253).  Its
 // figures are those of a pair, set where 42 such shapes part.
 #define QSA_TILES(X) \
-  X(64, 32, 2, 2, 6, 0.67f, 0.141f)   X(64, 64, 2, 2, 4, 0.71f, 0.208f) \
+  X(64, 32, 2, 2, 6, 0.67f, 0.200f)   X(64, 64, 2, 2, 4, 0.71f, 0.208f) \
   X(64, 128, 2, 4, 6, 1.86f, 0.353f)  X(128, 64, 4, 2, 6, 1.92f, 0.334f) \
   X(128, 128, 2, 4, 4, 2.38f, 0.497f) X(192, 64, 4, 2, 4, 1.94f, 0.431f) \
   X(192, 128, 4, 2, 4, 2.98f, 0.644f) X(256, 128, 4, 2, 3, 3.41f, 0.822f) \
@@ -340,10 +340,17 @@ static const RowsTile rows_tiles[] = {
 // The figures above and here are fitted to 382 shapes at up to 20 tiles and
 // shares each (M 33 to 20000, N 128 to 32000, K 128 to 14336; off by 9 % each,
 // and the choice by 1 % from the best of them).  Two blocks of the smallest
-// tiles share a CU, so alone on it they take longer.  `cheap`: the reader of the
-// product adds the shares.
+// tiles share a CU, so a stage takes another time alone on it.  The one of 64 x 32,
+// which fetches two rows of A with every row of W, follows 368 more shapes (M 1 to
+// 20,000, N 96 to 57,000): at 0.141 a stage beside another block it was the choice
+// for 64 x 12288 x 8192 (60 us for 45, the library 46) and 64 x 16384 x 2048 (21
+// for 15).  Over these the choice is 2.5 % from the best, 5.1 before, and 18 of
+// them, 37 before, are more than 5 % behind the library, the larger by up to 14 %
+// (450 to 512 x 12288, 64 x 40960 x 12288).
+// cheap: the reader of the product adds the shares; us_out: what the choice should
+// take, or null.
 extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
-                                  int* shares) {
+                                  int* shares, float* us_out) {
   const int all = K >> 6;
   const float mem = 2e-6f / 5.14f * ((float)N * K + (float)M * K +
                                      (float)M * N);
@@ -363,7 +370,7 @@ extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
       const int slots = t.pair ? 512 : 256;
       const long long turns = (blocks * S + slots - 1) / slots;
       float stage = t.stage;
-      if (turns == 1 && t.bn * t.bm <= 4096) stage *= i ? 1.48f : 1.32f;
+      if (turns == 1 && t.bn * t.bm <= 4096) stage *= i ? 1.48f : 0.93f;
       float run = (float)turns * (t.own + stage * ((all + S - 1) / S));
       if (t.pair && turns == 1) run += 1.5f;      // neither end beside another
       const float r2 = run * run, m2 = mem * mem;
@@ -372,6 +379,7 @@ extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
       if (us < best) { best = us; tile = i; *shares = S; }
     }
   }
+  if (us_out) *us_out = best;
   return tile;
 }
 

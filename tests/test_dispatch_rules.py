@@ -3,12 +3,13 @@
 from __future__ import annotations
 
 import pytest
-
 import torch
 
-from quickstart_streaming_agents_amd.ops import ext, have_ext
+from quickstart_streaming_agents_amd.ops import (
+    ext, have_ext, have_lm_ext, lm_ext)
 
-pytestmark = pytest.mark.skipif(not have_ext(), reason="extension not built")
+pytestmark = pytest.mark.skipif(not (have_ext() and have_lm_ext()),
+                                reason="extensions not built")
 
 
 @pytest.mark.parametrize("pages", [0, 1, 16, 17, 40])
@@ -102,3 +103,17 @@ def test_decode_attention_splits(rows, heads, pages, D):
     slot = bt[i, (pos[i] // 64).long()].long(), (pos[i] % 64).long()
     assert torch.equal(vc[slot[0], :, :, slot[1]], v[i])
     check(ext().paged_attn_decode(turned, kc, vc, bt, sl, D ** -0.5), turned)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (64, 12288, 8192), (64, 12288, 4096), (64, 16384, 2048), (33, 16384, 12288),
+    (48, 14336, 4096), (64, 9216, 4096), (128, 8192, 4096)])
+def test_few_rows_of_many_columns_take_wider_tiles(M, N, K):
+    """Tiles of 64 x 32 cost up to half as much again here."""
+    assert lm_ext().rows_gemm_plan(M, N, K, False)[0] != 0
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 2048), (64, 2048, 4096),
+                                   (192, 1024, 512)])
+def test_smallest_tiles_where_they_are_few(M, N, K):
+    assert lm_ext().rows_gemm_plan(M, N, K, False)[0] == 0
