@@ -996,23 +996,44 @@ static bool rows_gemm_fits(const Tensor& a, const Tensor& w, bool glu) {
          aligned(w, 16);
 }
 
-// Whether a @ w^T, with `glu` the gated activation of it, is rows_gemm's.  As
-// plain products of 26 pairs of N and K with M of 33 to 14000 it is 18 % faster
-// than the library's on average while M N is at most 9 million; beyond, the
-// library's 256 x 256 tiles fill the chip and reach 1.5 PFLOP/s, ours 1.3
-// (figures in rows_gemm.hip).  With K up to 768 they are not yet in their
-// stride: 8800 x 4096 x 512 takes 46 us for 75.  With the activation inside, a
-// pass over M N is saved, which is more than the library is ahead by up to K =
-// 3072 (13800 x 16384 x 2048: 735 us for 820) and at 4096 while the tiles are few
-// (1024 x 28672: 212 us for 211, 8192: 1450 for 1440, 44800: 1.6 % behind).  And
-// a call that is not captured is spared 15 us of the library's host path.  The
-// whole rule is here: in Python the last part alone took 2 us a call.
+// Whether a @ w^T, with `glu` the gated activation of it, is rows_gemm's by its
+// sizes.  As plain products of 26 pairs of N and K with M of 33 to 14000 it is 18 %
+// faster than the library's on average while M N is at most 9 million, and as 15
+// pairs with M of 1 to 32 13 % (6144 x 4096 alone, which the packed stream has, is
+// up to 8 % behind); beyond, the library's 256 x 256 tiles mostly fill the chip and
+// reach 1.5 PFLOP/s, ours 1.3 (figures in rows_gemm.hip).  The line is one for all
+// K, while the library is uneven: 10,650 x 4096 x 4096 takes it 388 us, 0.92
+// PFLOP/s, which these tiles should do in 276.  With K up to 768 the library's are
+// not yet in their stride: 8800 x 4096 x 512 takes 46 us for 75.
+// With the activation inside, a pass over M N is saved, which is more than the
+// library is ahead by up to K = 3072 (13800 x 16384 x 2048: 735 us for 820) and at
+// 4096 while the tiles are few (1024 x 28672: 212 us for 211, 8192: 1450 for 1440,
+// 44800: 1.6 % behind).  But it leaves K whole: where a plain product is this
+// kernel's too and few blocks would split it, that and a launch for the activation
+// is sooner (33 x 2048 x 16384 22 us, inside 69, the library 27; 64 x 4096 x 8192
+// 21, 41, 27; 100 x 4096 x 2048 11.8, 10.9, 12.2).  Of 881 gated shapes that left
+// 4 slower than inside, by up to 10 %, and takes 0.84 of the library's time on
+// average, 0.93 with all inside; 300 to 2000 rows of K from 6144 on remain between
+// 0.63 and 1.20 of it.
+static bool rows_gemm_sizes(int64_t M, int64_t N, int64_t K, bool glu) {
+  const int64_t MN = M * N;
+  const bool plain = MN <= 9000000 || K <= 768;
+  if (!glu) return plain;
+  if (MN > 48000000 && K > 3072) return false;
+  if (!plain) return true;
+  int S;
+  float in, apart;
+  qsa_rows_gemm_plan((int)M, (int)N, (int)K, 1, 0, &S, &in);
+  qsa_rows_gemm_plan((int)M, (int)N, (int)K, 0, 0, &S, &apart);
+  return in <= apart + 4.f + 6.4e-7f * (float)MN;
+}
+
+// Such a call as a whole; one that is not captured is spared 15 us of the library's
+// host path.  All of it is here: in Python the last part alone took 2 us a call.
 static bool rows_gemm_rule(const Tensor& a, const Tensor& w, bool glu) {
-  if (a.dim() != 2 || w.dim() != 2) return false;
-  const int64_t MN = a.size(0) * w.size(0), K = w.size(1);
-  return (MN <= (glu ? 48000000 : 9000000) || K <= (glu ? 3072 : 768)) && a.is_cuda() &&
-         a.device() == w.device() && no_observer() && unobserved(a) &&
-         unobserved(w) && rows_gemm_fits(a, w, glu);
+  return a.is_cuda() && a.device() == w.device() && no_observer() &&
+         unobserved(a) && unobserved(w) && rows_gemm_fits(a, w, glu) &&
+         rows_gemm_sizes(a.size(0), w.size(0), w.size(1), glu);
 }
 
 bool rows_gemm_ok(const Tensor& a, const Tensor& w) {
@@ -1115,6 +1136,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_parts", &rows_parts, "the same, shares of K left to the reader");
   m.def("rmsnorm_shares", &rmsnorm_shares,
         "residual add of such shares + RMSNorm (bf16)");
+  m.def("rows_gemm_sizes", &rows_gemm_sizes,
+        "whether sizes are rows_gemm's, or with the activation inside");
   m.def("rows_gemm_plan", &rows_gemm_plan, "tile and shares of a product");
   m.def("rows_glu", &rows_glu, "the same with the gated activation inside");
   m.def("rows_glu_ok", &rows_glu_ok, "whether a gated product is rows_glu's");

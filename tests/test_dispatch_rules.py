@@ -117,3 +117,44 @@ def test_few_rows_of_many_columns_take_wider_tiles(M, N, K):
                                    (192, 1024, 512)])
 def test_smallest_tiles_where_they_are_few(M, N, K):
     assert lm_ext().rows_gemm_plan(M, N, K, False)[0] == 0
+
+
+@pytest.mark.parametrize("M,N,K,inside", [
+    (33, 2048, 16384, False), (64, 4096, 8192, False), (100, 1024, 4096, False),
+    (64, 16384, 2048, True), (192, 28672, 4096, True), (100, 4096, 2048, True),
+    (1024, 28672, 4096, True), (13_800, 16384, 2048, True),
+    (8800, 3072, 384, True), (9000, 28672, 4096, False)])
+def test_gated_products_that_would_split_k(M, N, K, inside):
+    """The activation inside a product leaves K whole."""
+    assert lm_ext().rows_gemm_sizes(M, N, K, True) == inside
+    _, shares = lm_ext().rows_gemm_plan(M, N, K, False)
+    assert inside or shares > 1 or not lm_ext().rows_gemm_sizes(M, N, K, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 4096), (100, 1024, 4096),
+                                   (100, 4096, 2048)])
+def test_gated_layers_on_either_side(M, N, K):
+    """Inside or apart, gate and up are rounded before the activation."""
+    from quickstart_streaming_agents_amd.models.layers import DenseGLU
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    torch.manual_seed(M + K)
+    dev, bf = "cuda:0", torch.bfloat16
+    gate, up = (torch.randn(N // 2, K, device=dev, dtype=bf) * K ** -0.5
+                for _ in range(2))
+    x = torch.randn(M, K, device=dev, dtype=bf)
+    ff = DenseGLU(gate, up, torch.eye(N // 2, device=dev, dtype=bf))
+    assert D.glu_linear_ok(x, ff.gate_up.w) == \
+        lm_ext().rows_gemm_sizes(M, N, K, True)
+    a, b = x.double(), ff.gate_up.w.double()
+    g, u = (a @ b.T).chunk(2, 1)
+    # gate and up: f32 sums of K products, __expf and a rounding to bf16 each;
+    # the activation's slope is 1.13 at most, the result is rounded
+    e = K * 2.0 ** -24 * (a.abs() @ b.abs().T) + 2.0 ** -20 \
+        + 2.0 ** -8 * (a @ b.T).abs()
+    (eg, eu), f = e.chunk(2, 1), torch.nn.functional.silu(g)
+    want = f * u
+    bound = (2.0 ** -8 + 2.0 ** -18) * want.abs() + 1.13 * eg * u.abs() \
+        + (f.abs() + eg) * eu
+    got = ff.gate_up.glu(x, "silu").double()
+    assert ((got - want).abs() <= bound).all()
