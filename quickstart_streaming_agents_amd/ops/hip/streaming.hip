@@ -387,7 +387,10 @@ qsa_window_merge(const int2* __restrict__ span, const int* __restrict__ ws,
 // solve the padded 4x4 system in registers (rows beyond p are the identity).
 // A series of up to 512 goes to LDS at once, beside its length: passes that
 // waited for memory 64 numbers at a time made 10.5 us of 1000 series of 288,
-// 8.9 so (171 us with the solve and the residuals on one lane).
+// 8.9 so (171 us with the solve and the residuals on one lane).  Many short ones
+// keep LDS busy as it is, with the sums over lanes: 30,000 of 128 43.3 us read
+// from memory, 45.8 from LDS, 8000 16.3 both, 4000 11.2 and 11.0; 30,000 of 150
+// 50.4 and 48.1.
 // ---------------------------------------------------------------------------
 #define QSA_AR_MAXP 4
 
@@ -626,7 +629,7 @@ extern "C" void qsa_anomaly_batch_launch(const float* series,
                                          float* pred_se, int* dof_out, int K,
                                          int Tmax, int order,
                                          hipStream_t stream) {
-  if (Tmax <= 512)
+  if (Tmax <= 512 && (Tmax > 2 * QSA_WAVE || K <= 8192))
     hipLaunchKernelGGL(qsa_anomaly_batch<512>, dim3(K), dim3(64), 0, stream,
                        series, lengths, forecast, pred_se, dof_out, Tmax,
                        order);

@@ -460,6 +460,20 @@ def test_anomaly_batch_staged(ext, n):
     test_anomaly_batch_lengths(ext, n)
 
 
+@pytest.mark.parametrize("T", [7, 128, 129])
+def test_anomaly_batch_of_many_series(ext, T):
+    """Series read from memory or from LDS, either side of that rule: the same
+    sums in the same order."""
+    g = torch.Generator().manual_seed(T)
+    x = torch.rand(8193, T, generator=g).to(dev())
+    n = torch.randint(0, T + 1, (8193,), generator=g).int().to(dev())
+    n[:2] = T
+    many = ext.anomaly_batch(x, n, 4)
+    few = ext.anomaly_batch(x[:8192], n[:8192], 4)
+    for a, b in zip(many, few):
+        assert torch.equal(a[:8192], b)
+
+
 def test_anomaly_batch_matches_cpu(ext):
     from quickstart_streaming_agents_amd.runtime.anomaly import ar_forecast
     rng = np.random.default_rng(0)
