@@ -22,8 +22,13 @@ class Linear:
     4 15.2 / 13.9, 16 18.6 / 14.5, 32 25.1 / 13.8; 2048 x 6144 8 13.4 / 12.9, 32
     20.3 / 12.0; 1024 x 2048 8 7.7 / 7.6; 2048 x 2048 4 8.1 / 8.0, 17 9.7 / 8.1;
     4096 x 4096 17 14.8 / 15.0, 32 17.1 / 13.4; 6144 x 4096 24 18.8 / 19.0.
-    Alone: 6144 x 2048 16 8.9 / 8.9, 32 12.3 / 9.1; 2048 x 4096 16 8.6 / 8.7, 32
-    11.9 / 8.6; 4096 x 2048 32 7.8 / 8.5; 8192 x 3072 24 12.6 / 12.7."""
+    Alone: 6144 x 2048 16 8.8 / 9.3, 17 9.6 / 9.3, 32 12.2 / 9.3; 2048 x 4096 16
+    7.7 / 8.3, 17 8.8 / 8.3, 32 11.5 / 8.6; 4096 x 2048 32 7.5 / 8.9.  From 6144
+    columns of K beyond 2048 on the stream has two tiles a block, which keeps it
+    ahead: 6144 x 3072 17 10.2 / 12.5, 32 11.9 / 12.6; 8192 x 3072 32 12.7 / 12.9.
+    The lines are coarse: 4608 to 5631 columns of 2048 would gain from 17 rows on
+    too (9.4 / 9.1, 32 12.0 / 9.1), and 4096 x 4096 with the norm only from 24
+    (17 14.0 / 15.1, 24 15.2 / 12.9)."""
 
     SKINNY_ROWS = 32
     SKINNY_MAX = 6144 * 4096
@@ -37,7 +42,8 @@ class Linear:
             self.packed = D.pack_weight_frag(w)
         # rows from which the stream is behind, alone and with shares
         middling = n * k <= 20 << 20
-        self.rows = 17 if n >= 5632 and middling or \
+        pairs = n >= 6144 and k > 2048
+        self.rows = 17 if n >= 5632 and middling and not pairs or \
             k >= max(2 * n, 4096) else self.SKINNY_ROWS + 1
         self.rows_parts = 4 if k >= 3 * n else 8 if k >= 2 * n else \
             17 if middling else self.SKINNY_ROWS + 1
