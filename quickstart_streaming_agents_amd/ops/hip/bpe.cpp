@@ -153,7 +153,7 @@ class Bpe {
     const std::string_view s(p, (size_t)n);
     if (first >= 0) ids.push_back(first);
     size_t from = 0;
-    for (size_t i = 0; i < s.size() && ids.size() < most;) {
+    for (size_t i = 0; i < s.size();) {
       const std::pair<std::string, int>* hit = nullptr;
       if (starts_[(unsigned char)s[i]])
         for (const auto& sp : specials_)
@@ -166,6 +166,7 @@ class Bpe {
         continue;
       }
       words(s.substr(from, i - from), most, ids);
+      if (ids.size() >= most) return;
       ids.push_back(hit->second);
       from = i += hit->first.size();
     }
@@ -241,7 +242,7 @@ class Bpe {
 
   // leaves the word's tokens in syms_: the pair of lowest rank, the first of
   // equals, until none is left
-  void merge(std::string_view w) {
+  __attribute__((noinline)) void merge(std::string_view w) {
     syms_.assign(w.size(), 0);
     for (size_t i = 0; i < w.size(); ++i) syms_[i] = (unsigned char)w[i];
     if (w.size() > kShort) merge_long();
