@@ -218,7 +218,7 @@ class LlamaModel:
         """Projection: decode-sized cuda batches go through the
         weight-streaming skinny GEMM — fp8 (W8A16, half the weight
         stream) when packed, else bf16; what does not fill a library's tiles
-        through rows_gemm; everything else rocBLAS.  `parts`: the reader is the
+        through rows_gemm; everything else the library.  `parts`: the reader is the
         residual's norm, which adds shares of K."""
         n, k = w.shape
         M = x.shape[0]
@@ -227,10 +227,10 @@ class LlamaModel:
                 return D.skinny_linear_fp8(x, wf8[0], wf8[1], n, k)
             # 32 < M <= 256 (continuous-batching decode): the batched fp8
             # kernel (ops/hip/gemm_fp8_batch.hip) is measured SLOWER than
-            # rocBLAS bf16 at these M on MI355X — the problem is L2-/
+            # bf16 products at these M on MI355X — the problem is L2-/
             # compute-bound, not weight-stream-bound, so halved weight
             # bytes don't pay (profiles/fp8_decode_gemm.md).  Keep it
-            # opt-in for further tuning; rocBLAS is the measured winner.
+            # opt-in for further tuning.
             import os as _os
             if _os.environ.get("QSA_FP8_BATCH") == "1" and M <= 256 \
                     and n % 64 == 0 and n <= 32768:
@@ -241,8 +241,9 @@ class LlamaModel:
                                             splitk)
         if x.is_cuda and M <= 32 and wf is not None and \
                 n * k <= 6144 * 4096:
-            # bf16 skinny wins only the small decode shapes (qkv/wo);
-            # rocBLAS is at the bandwidth floor for the big-N ones
+            # the packed stream wins only the small decode shapes (qkv/wo);
+            # large ones are rows_gemm's (one row, us: 28672 x 4096 45, the
+            # library 56; 128256 x 2048 95 and 108)
             return D.skinny_linear(x, wf, n, k)
         return D.linear_parts(x, w) if parts else D.linear(x, w)
 

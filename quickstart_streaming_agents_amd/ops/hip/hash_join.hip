@@ -18,11 +18,12 @@
 // Both words of a slot lie in one cache line, so a probe is one 16-byte load
 // where separate key and payload arrays take two dependent ones; the probes of
 // a wave hit 64 different lines and that access rate is what bounds them.
-// 2M probes of a 50,000-row table: 27 us with separate arrays, 17 us here.
+// 2M probes of a 50,000-row table: 27 us with separate arrays, 18 us here.
 // (The bindings hand the two words out as strided views; STRIDE 1 serves
 // tables held as two arrays.)
-// Insert: atomicCAS on the key slots in turn, then atomicMax on the payload.  No locks, no host round trips; eviction is at probe time
-// (ts >= cutoff), full compaction = rebuild from the surviving rows.
+// Insert: atomicCAS on the key slots in turn, then atomicMax on the payload.  No
+// locks, no host round trips; eviction is at probe time (ts >= cutoff), full
+// compaction = rebuild from the surviving rows.
 #include "common.h"
 
 #define QSA_HJ_EMPTY 0xFFFFFFFFFFFFFFFFull
@@ -38,8 +39,8 @@ __device__ __forceinline__ unsigned long long qsa_hj_mix(
 
 // Where a key is looked for.  Neighbours in the table would form runs, whose
 // longest is what a build waits for, an atomic access to memory per slot: 50,000
-// rows 13.1 us with steps of one, 10.1 so, 2M probes of them 19.8 and 17.0, 500k
-// 8.7 and 6.5.  A table beyond a die's L2 (4 MiB) has steps of one, whose next
+// rows 13.1 us with steps of one, 10 to 12 so, 2M probes of them 19.8 and 17 to 18,
+// 500k 8.7 and 7.  A table beyond a die's L2 (4 MiB) has steps of one, whose next
 // slot mostly lies in the line that has come (2M probes of 1M rows 43.5 us, 50.3
 // with others).
 #define QSA_HJ_NEAR (1u << 18)         // slots

@@ -26,9 +26,10 @@
 //     place among what it has read: waiting for its own stores cost a round
 //     trip to memory.
 // 192 rows of 400-1000 keys, 32/8 heads of 128: 131 -> 124 us, of which 105 are
-// the reads (5.6 TB/s) and the rest the 128 lines per row and head that a
-// transposed value touches, whatever the width of the stores or their cache
-// policy (64-byte pieces, whole lines and write-through were the same).
+// the reads (5.2 TB/s of keys and values, 5.5 with the rest of last pages) and the
+// rest the 128 lines per row and head that a transposed value touches, whatever the
+// width of the stores or their cache policy (64-byte pieces, whole lines and
+// write-through were the same).
 //
 // The online softmax runs per head-column in registers: column max/sum
 // reduce with two shfl_xor hops (the 4 hi-lane groups of a column).
@@ -462,8 +463,13 @@ qsa_attn_reduce(const float* __restrict__ part_o,   // [rows, NS, D]
 // below, what fills the chip (8 of 1000-2000 19.1, eight blocks of four 21.5; 12
 // 23.0 / 27.9).
 // max_pages is the table's width, since the rows' lengths are on the device: in
-// a table for longer rows short ones of up to 128 pairs are split, with the merge
-// and without the read-ahead below.
+// a table for longer rows, as a captured step's is, short ones of up to 128 pairs
+// are split, with the merge and without the read-ahead below.  us, a table as wide
+// as the longest row / of 33 / 128 / 256 pages: 1 row of 700 keys 8.6 / 9.2 / 11.1 /
+// 13.8; 4 of 500-900 11.6 / 10.8 / 14.2 / 14.5; 8 11.8 / 14.4 / 14.2 / 14.3; 16
+// 17.1 / 17.8 / 17.5 / 17.5; of 60-100 keys 1 row 6.5 / 8.7 / 10.1 / 12.9, 16 6.8 /
+// 9.7 / 9.6 / 9.7; from 24 rows on and beyond 1000 keys the width is nothing.  Rows
+// of 12,000 to 16,000 keys follow the same rule: 8 93 us, 24 252, 64 652 (5.6 TB/s).
 extern "C" void qsa_paged_attn_split(int B, int QH, int KVH, int max_pages,
                                      int D, int* waves, int* splits) {
   const long long heads = (long long)B * KVH;

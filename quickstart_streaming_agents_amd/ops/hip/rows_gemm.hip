@@ -4,8 +4,8 @@
 //
 // Up to some 200 rows it is bound by the read of W, then by the matrix cores.
 // Both operands go from memory straight into LDS (16 bytes a lane, whole lines),
-// two to five stages of K ahead, so the bytes under way do not cost registers;
-// the ring is as deep as the 160 KB of a CU allow.  A wave multiplies half a
+// through a ring of two to six stages of K, as deep as the 160 KB of a CU allow, so
+// the bytes under way do not cost registers.  A wave multiplies half a
 // stage while it reads the next half.  Tiles from 64 x 32 to 256 x 256 and
 // shares of K are chosen by what they should take (qsa_rows_gemm_plan); a tile's
 // LDS traffic per product falls with its sides, which is why the large ones are
@@ -13,14 +13,14 @@
 // is applied to the sums, rounded first where a stored product was read before.
 // us, library -> here (sums of shares included, weights from memory):
 //   rows            33            64           128           192           768
-//   6144 x 4096  17.4 -> 15.6  17.9 -> 16.9  25.6 -> 21.0  34.1 -> 25.3  49 -> 47
-//   4096 x 4096  12.8 -> 11.3  13.9 -> 12.0  22.6 -> 15.1  32.3 -> 19.0  35 -> 36
-//   4096 x 14336 38.5 -> 26.2  39.8 -> 27.6  75.9 -> 33.3   103 -> 40   108 -> 95
-//   2048 x 8192  13.2 -> 10.5  20.9 -> 11.5  20.2 -> 15.1  25.4 -> 18.8  44 -> 37
-//   12576 x 2048 17.1 -> 14.6  16.5 -> 14.9  19.4 -> 18.6  26.1 -> 21.0  45 -> 48
+//   6144 x 4096  17.2 -> 15.7  18.0 -> 17.3  25.7 -> 22.6  33.5 -> 27.3  48 -> 46
+//   4096 x 4096  13.9 -> 11.4  15.4 -> 12.9  24.8 -> 16.5  32.9 -> 19.3  34 -> 35
+//   4096 x 14336 34.6 -> 26.4  39.2 -> 27.5  75.7 -> 36.4   103 -> 45   107 -> 95
+//   2048 x 8192  14.1 -> 12.3  22.6 -> 13.4  21.1 -> 16.0  26.5 -> 19.7  43 -> 36
+//   12576 x 2048 16.6 -> 12.9  16.5 -> 14.3  19.3 -> 18.3  26.0 -> 22.4  42 -> 47
 // with the activation (there a pass of its own):
-//   28672 x 4096 54.5 -> 44.7  53.9 -> 43.3  57.6 -> 51.0  67.7 -> 58.9 176 -> 176
-//   16384 x 2048 22.0 -> 15.0  20.9 -> 15.5  24.1 -> 19.1  30.9 -> 23.2  57 -> 53
+//   28672 x 4096 53.3 -> 43.0  53.5 -> 43.0  57.1 -> 51.2  66.4 -> 59.3 167 -> 180
+//   16384 x 2048 21.9 -> 14.3  20.9 -> 15.3  24.0 -> 19.2  30.6 -> 23.6  53 -> 52
 // and 820 -> 735 at 13,800 rows.  What limits 256 x 256 at 1.3 PFLOP/s (28672 x
 // 4096 x 8192, the library 1.5): matrix cores 72 % busy at 1.6 GHz (82 %), LDS as
 // many cycles as they; four waves of 128 x 128, stages of 32, products of 32 x 32

@@ -67,10 +67,15 @@ def _scan_wins(queries: int, rows: int, k: int) -> bool:
     """Whether a search is the kernel's (ops/hip/topk_cosine.hip) or a matmul's
     with a sort.  Measured at 1536 numbers a row (us, kernel / matmul): up to
     16 queries are one read of the matrix (16, k = 16: 100k rows 156 / 314, 1M
-    1231 / 1579), up to 32 one and more work per row (32, k = 16: 100k 220 /
-    313, 300k 599 / 663, 1M 1725 / 1593).  More are GEMM-shaped, and a block's
-    choice of its best k costs per query and k (64, k = 16: 10k 68 / 101, 30k
-    132 / 143; 256, k = 16: 1k 50 / 50, 10k 166 / 176, 30k 392 / 382)."""
+    1231 / 1579), up to 32 one and more work per row (32: 100k k = 3 158 / 307,
+    16 210 / 309).  More are GEMM-shaped, and a block's choice of its best k costs
+    per query and k (128: 10k k = 3 69 / 127, 16 104 / 127).
+    Within these lines the kernel is the faster at every size and k measured.
+    They are an earlier, slower scan's, though, and most of what lies just outside
+    would be the kernel's by now, above all for small k: 32 of 300k k = 3 416 /
+    646, 16 545 / 641; 48 of 45k 100 / 174, 158 / 177; 64 of 100k 292 / 378, 362 /
+    382; 256 of 10k 110 / 169, 162 / 170; but 33 of 100k 211 / 308, 310 / 307, and
+    256 of 30k 284 / 379, 387 / 379."""
     if k > 16:                       # what the kernel keeps
         return False
     return queries <= 16 or \
