@@ -761,9 +761,10 @@ void gqa_rows(Tensor q, Tensor kc, Tensor vc, Tensor block_table,
     long long ns = 4;
     if (!merge) {
       ns = (2048 + tiles - 1) / tiles;
-      ns = std::max<long long>(1, std::min<long long>(ns, mp));
-      const long long per = (mp + ns - 1) / ns;
-      ns = (mp + per - 1) / per;
+      const long long pages = std::max(mp, 1);       // none: rows not in use
+      ns = std::min(ns, pages);
+      const long long per = (pages + ns - 1) / ns;
+      ns = (pages + per - 1) / per;
     }
     TORCH_CHECK(tiles * ns < (1LL << 31), "rows per call");
     auto of = q.options().dtype(at::kFloat);

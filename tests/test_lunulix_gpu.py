@@ -317,6 +317,19 @@ def test_grouped_attention_many_rows(R, H, G, Dm, E):
         assert not out[:, H * E:].any()
 
 
+@pytest.mark.parametrize("R", [3, 2100])
+def test_grouped_attention_without_pages(R):
+    """A table without columns: no row is in use."""
+    H, Dm = 4, 32
+    kc = torch.ones(1, 1, 64, Dm, dtype=BF, device=DEV)
+    out = torch.ones(R, H * Dm, dtype=BF, device=DEV)
+    D.gqa_rows(out.clone(), kc, kc, torch.zeros(R, 0, dtype=torch.int32,
+                                                device=DEV), None,
+               torch.zeros(R, dtype=torch.int32, device=DEV), None, None, out,
+               H, 1.0)
+    assert not out.any()
+
+
 def test_portions_of_several_sequences():
     """One launch over portions of two sequences, rows behind each other."""
     g = gen(9)
