@@ -95,23 +95,30 @@ class EmbeddingEncoder:
         5.5 in the library), the others rows_gemm's: at 8800 rows 1536 x 384
         takes 17.0 us (short_gemm 20.7, the library 18.3), 3072 x 384 with the
         activation 32 (36, 72 with a pass of its own), 384 x 512 8.0 (10.5,
-        10.7), 384 x 1536 14.6 (23.4, 17.2).  With qsa_hip alone they are
-        short_gemm's and, of long K and many rows, the library's."""
+        10.7), 384 x 1536 14.6 (23.4, 17.2)."""
         n, k = w.shape
-        rows = x.shape[0]
-        fits = x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
-            n % 32 == 0
-        if not have_lm_ext():            # rows_gemm is that module's
-            if fits and (k <= 512 or rows <= 2048):
-                return D.ext().short_gemm(x, w, glu)
-        else:
-            if fits and (k <= 512 or rows <= 32) and \
-                    -(-rows // 32) * -(-n // 64) <= 192:
-                return D.ext().short_gemm(x, w, glu)
-            if not glu:
-                return D.linear_parts(x, w) if parts else D.linear(x, w)
-            if D.glu_linear_ok(x, w):
-                return D.glu_linear(x, w, "silu", rounded=False)
+        if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
+                n % 32 == 0 and (k <= 512 or x.shape[0] <= 32) and \
+                -(-x.shape[0] // 32) * -(-n // 64) <= 192:
+            return D.ext().short_gemm(x, w, glu)
+        if not glu:
+            return D.linear_parts(x, w) if parts else D.linear(x, w)
+        if D.glu_linear_ok(x, w):
+            return D.glu_linear(x, w, "silu", rounded=False)
+        y = F.linear(x, w)
+        return D.swiglu(y[:, :n // 2], y[:, n // 2:])
+
+    @property
+    def _project(self):
+        return self._linear if have_lm_ext() else self._linear_alone
+
+    def _linear_alone(self, x: torch.Tensor, w: torch.Tensor,
+                      glu: bool = False, parts: bool = False) -> torch.Tensor:
+        """The same with qsa_hip alone: rows_gemm is qsa_lm_hip's."""
+        n, k = w.shape
+        if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
+                n % 32 == 0 and (k <= 512 or x.shape[0] <= 2048):
+            return D.ext().short_gemm(x, w, glu)
         y = F.linear(x, w)
         return D.swiglu(y[:, :n // 2], y[:, n // 2:]) if glu else y
 
@@ -121,7 +128,7 @@ class EmbeddingEncoder:
     def _embed_rows(self, ids: np.ndarray, lens: np.ndarray) -> torch.Tensor:
         """Mean-pooled final states [n, hidden] f32 of texts whose tokens follow
         each other in ids, all rows in one concatenation without padding."""
-        c, dev = self.cfg, self.device
+        c, dev, project = self.cfg, self.device, self._project
         n = len(lens)
         off = np.cumsum(lens) - lens
         nqb = -(-lens // self.QROWS)
@@ -139,12 +146,12 @@ class EmbeddingEncoder:
                 h = D.rmsnorm_residual(mlp_out, res, Ly["attn_norm"],
                                        c.norm_eps)
             attn = D.ext().encoder_attn(
-                self._linear(h, Ly["wqkv"]), self.rope_cos, self.rope_sin,
+                project(h, Ly["wqkv"]), self.rope_cos, self.rope_sin,
                 qb_item, qb_pos0, off, lens_t, c.n_heads, self.scale)
-            o = self._linear(attn, Ly["wo"], parts=True)
+            o = project(attn, Ly["wo"], parts=True)
             h = D.rmsnorm_residual(o, res, Ly["mlp_norm"], c.norm_eps)
-            act = self._linear(h, Ly["wgu"], glu=True)
-            mlp_out = self._linear(act, Ly["wdown"], parts=True)
+            act = project(h, Ly["wgu"], glu=True)
+            mlp_out = project(act, Ly["wdown"], parts=True)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm,
                                      c.norm_eps)
         return D.ext().mean_rows(final_h, off, lens_t)
@@ -216,8 +223,8 @@ class EmbeddingEncoder:
         ids, lens = self.tokenizer.encode_batch(list(texts), c.max_pos)
         # mean over the tokens, project, L2-normalize
         if self._use_hip and have_ext():
-            out = self._linear(self._embed_rows(ids, lens).to(self.dtype),
-                               self.proj)
+            out = self._project(self._embed_rows(ids, lens).to(self.dtype),
+                                self.proj)
         else:
             enc = [x.tolist() for x in np.split(ids, np.cumsum(lens)[:-1])]
             out = F.linear(self._embed_padded(enc).to(self.dtype), self.proj)

@@ -1021,7 +1021,7 @@ static bool rows_gemm_sizes(int64_t M, int64_t N, int64_t K, bool glu) {
   const bool plain = MN <= 9000000 || K <= 768;
   if (!glu) return plain;
   if (MN > 48000000 && K > 3072) return false;
-  if (!plain) return true;
+  if (!plain || K < 512) return true;  // beside the library's; not split
   int S;
   float in, apart;
   qsa_rows_gemm_plan((int)M, (int)N, (int)K, 1, 0, &S, &in);
