@@ -217,8 +217,8 @@ class LlamaModel:
                 parts: bool = False) -> torch.Tensor:
         """Projection: decode-sized cuda batches go through the
         weight-streaming skinny GEMM — fp8 (W8A16, half the weight
-        stream) when packed, else bf16; what does not fill a library's tiles
-        through rows_gemm; everything else the library.  `parts`: the reader is the
+        stream) when packed, else bf16; everything else rows_gemm or
+        wide_gemm, and what these refuse the library.  `parts`: the reader is the
         residual's norm, which adds shares of K."""
         n, k = w.shape
         M = x.shape[0]

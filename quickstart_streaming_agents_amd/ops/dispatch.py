@@ -214,18 +214,25 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return lm_ext().rows_gemm(x, w)
 
 
+def _gemm_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x[M,K] @ W^T is one of this framework's kernels': rows_linear's,
+    or of many rows (ops/hip/wide_gemm.hip)."""
+    return x.is_cuda and type(x) is torch.Tensor and \
+        lm_ext().gemm_ok(x, w) and not torch.compiler.is_compiling()
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ W^T for a weight as it is stored."""
-    if rows_linear_ok(x, w):
-        return rows_linear(x, w)
+    if _gemm_ok(x, w):
+        return lm_ext().gemm(x, w)
     return torch.nn.functional.linear(x, w)
 
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear() for a reader that adds shares (residual_norm, rmsnorm_residual,
     glu_table): where K is split, [S, rows, columns] in f32."""
-    if rows_linear_ok(x, w):
-        return lm_ext().rows_parts(x, w)
+    if _gemm_ok(x, w):
+        return lm_ext().gemm_parts(x, w)
     return torch.nn.functional.linear(x, w)
 
 
@@ -243,7 +250,7 @@ def glu_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the activation is glu_linear's to apply: W's rows are [gate; up]
     and both fit its kernel (the rules are beside rows_linear's)."""
     return x.is_cuda and type(x) is torch.Tensor and \
-        lm_ext().rows_glu_ok(x, w) and not torch.compiler.is_compiling()
+        lm_ext().glu_gemm_ok(x, w) and not torch.compiler.is_compiling()
 
 
 def glu_linear(x: torch.Tensor, w: torch.Tensor,
@@ -251,7 +258,7 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor,
     """act(x @ W_gate^T) * (x @ W_up^T) of W = [gate; up], in one kernel; with
     `rounded` of the products as linear() would store them, without (silu only)
     of their f32 sums."""
-    return lm_ext().rows_glu(x, w, act == "gelu", rounded)
+    return lm_ext().glu_gemm(x, w, act == "gelu", rounded)
 
 
 def skinny_linear(x: torch.Tensor, wf: torch.Tensor, n: int,

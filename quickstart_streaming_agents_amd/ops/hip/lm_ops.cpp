@@ -133,6 +133,10 @@ extern "C" void qsa_window_attn_prefill_launch(const bf16_t*, long long,
 extern "C" void qsa_skinny_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     int, int, long long, long long, hipStream_t);
 extern "C" int qsa_rows_gemm_plan(int, int, int, int, int, int*, float*);
+extern "C" bool qsa_wide_gemm_fits(int, int, int);
+extern "C" float qsa_wide_gemm_plan(int, int, int, int, int*, int*, int*);
+extern "C" void qsa_wide_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*, int,
+                                     int, int, long long, int, int, hipStream_t);
 extern "C" void qsa_rows_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     float*, int, int, int, long long, int, int, int, hipStream_t);
 
@@ -998,24 +1002,17 @@ static bool rows_gemm_fits(const Tensor& a, const Tensor& w, bool glu) {
 }
 
 // Whether a @ w^T, with `glu` the gated activation of it, is rows_gemm's by its
-// sizes.  As plain products of 26 pairs of N and K with M of 33 to 14000 it is 18 %
-// faster than the library's on average while M N is at most 9 million, and as 15
-// pairs with M of 1 to 32 13 % (6144 x 4096 alone, which the packed stream has, is
-// up to 8 % behind); beyond, the library's 256 x 256 tiles mostly fill the chip and
-// reach 1.5 PFLOP/s, ours 1.3 (figures in rows_gemm.hip).  The line is one for all
-// K, while the library is uneven: 10,650 x 4096 x 4096 takes it 388 us, 0.92
-// PFLOP/s, which these tiles should do in 276.  With K up to 768 the library's are
-// not yet in their stride: 8800 x 4096 x 512 takes 46 us for 75.
-// With the activation inside, a pass over M N is saved, which is more than the
-// library is ahead by up to K = 3072 (13800 x 16384 x 2048: 735 us for 820) and at
-// 4096 while the tiles are few (1024 x 28672: 212 us for 211, 8192: 1450 for 1440,
-// 44800: 1.6 % behind).  But it leaves K whole: where a plain product is this
-// kernel's too and few blocks would split it, that and a launch for the activation
+// sizes, before wide_gemm is looked at.  As plain products of 26 pairs of N and K with M
+// of 33 to 14000 it is 18 % faster than the library's on average while M N is at most
+// 9 million, and as 15 pairs with M of 1 to 32 13 % (6144 x 4096 alone, which the packed
+// stream has, is up to 8 % behind).  With K up to 768 the library's are not yet in
+// their stride: 8800 x 4096 x 512 takes 46 us for 75.
+// The activation inside leaves K whole: where a plain product is this kernel's too and
+// few blocks would split it, that and a launch for the activation
 // is sooner (33 x 2048 x 16384 22 us, inside 69, the library 27; 64 x 4096 x 8192
 // 21, 41, 27; 100 x 4096 x 2048 11.8, 10.9, 12.2).  Of 881 gated shapes that left
 // 4 slower than inside, by up to 10 %, and takes 0.84 of the library's time on
-// average, 0.93 with all inside; 300 to 2000 rows of K from 6144 on remain between
-// 0.63 and 1.20 of it.
+// average, 0.93 with all inside.
 static bool rows_gemm_sizes(int64_t M, int64_t N, int64_t K, bool glu) {
   const int64_t MN = M * N;
   const bool plain = MN <= 9000000 || K <= 768;
@@ -1031,18 +1028,50 @@ static bool rows_gemm_sizes(int64_t M, int64_t N, int64_t K, bool glu) {
 
 // Such a call as a whole; one that is not captured is spared 15 us of the library's
 // host path.  All of it is here: in Python the last part alone took 2 us a call.
-static bool rows_gemm_rule(const Tensor& a, const Tensor& w, bool glu) {
+static bool gemm_takes(const Tensor& a, const Tensor& w, bool glu) {
   return a.is_cuda() && a.device() == w.device() && no_observer() &&
-         unobserved(a) && unobserved(w) && rows_gemm_fits(a, w, glu) &&
-         rows_gemm_sizes(a.size(0), w.size(0), w.size(1), glu);
+         unobserved(a) && unobserved(w) && rows_gemm_fits(a, w, glu);
 }
 
 bool rows_gemm_ok(const Tensor& a, const Tensor& w) {
-  return rows_gemm_rule(a, w, false);
+  return gemm_takes(a, w, false) &&
+         rows_gemm_sizes(a.size(0), w.size(0), w.size(1), false);
 }
 
-bool rows_glu_ok(const Tensor& a, const Tensor& w) {
-  return rows_gemm_rule(a, w, true);
+// What wide_gemm.hip would do with a product; its offsets are of whole tiles.  Decode
+// batches, bound by the read of W, are not looked at.
+struct WidePlan {
+  int tile = 0, rows = 0, rest = 0;
+  float us = 1e30f;
+};
+static WidePlan wide_plan(const Tensor& a, const Tensor& w, int act) {
+  WidePlan p;
+  const int64_t M = a.size(0), N = w.size(0), K = w.size(1);
+  if (M < 256 || (256 * a.stride(0) + K) * 2 >= (4ll << 30) ||
+      256 * N * 2 >= (4ll << 30))
+    return p;
+  p.us = qsa_wide_gemm_plan((int)M, (int)N, (int)K, act, &p.tile, &p.rows, &p.rest);
+  return p;
+}
+
+// Whether a product is wide_gemm.hip's where it is not rows_gemm.hip's by its size: in
+// 150 shapes from 30 us on the two take 0.86 of the library's time on average (the
+// activation a pass of its own there), and at most 1.10 of it, where its division of K
+// over all CUs evens out a last turn of few tiles (4620 x 5568 x 5888).
+static bool wide_sizes(const Tensor& a, const Tensor& w, bool glu) {
+  return a.size(0) * w.size(0) > 9000000 && wide_plan(a, w, glu).us < 1e30f;
+}
+
+bool gemm_ok(const Tensor& a, const Tensor& w) {
+  return gemm_takes(a, w, false) &&
+         (rows_gemm_sizes(a.size(0), w.size(0), w.size(1), false) ||
+          wide_sizes(a, w, false));
+}
+
+bool glu_gemm_ok(const Tensor& a, const Tensor& w) {
+  return gemm_takes(a, w, true) &&
+         (rows_gemm_sizes(a.size(0), w.size(0), w.size(1), true) ||
+          wide_sizes(a, w, true));
 }
 
 // parts: a product whose K is split may stay in its shares, [S, M, N] f32
@@ -1061,6 +1090,56 @@ static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
                        S > 1 ? part.data_ptr<float>() : nullptr, M, N, K,
                        a.stride(0), tile, S, act, cur_stream());
   return out.defined() ? out : part;
+}
+
+// The same by whichever of the two should be over first.  rows_gemm's estimate is of
+// CUs that keep their clock: where it comes within 14 % of the other's, the other is
+// sooner (of 200 shapes, M 200 to 45,000, the choice is then 0.5 % from the best).
+static Tensor gemm_run(const Tensor& a, const Tensor& w, int act,
+                       bool parts = false) {
+  CHK_DEV(a); CHK_SAME(a, w);
+  TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
+              "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
+  const WidePlan p = wide_plan(a, w, act);
+  if (p.us == 1e30f) return rows_gemm_run(a, w, act, parts);
+  const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
+  int S;
+  float us;
+  qsa_rows_gemm_plan(M, N, K, act, parts, &S, &us);
+  if (us * 1.14f < p.us) return rows_gemm_run(a, w, act, parts);
+  const int64_t cols = act ? N / 2 : N;
+  Tensor out = torch::empty({M, cols}, a.options());
+  qsa_wide_gemm_launch(u16(a), u16(w), u16m(out), p.rows, N, K, a.stride(0), p.tile,
+                       act, cur_stream());
+  if (p.rows < M)
+    qsa_wide_gemm_launch(u16(a) + p.rows * a.stride(0), u16(w),
+                         u16m(out) + p.rows * cols, M - p.rows, N, K, a.stride(0),
+                         p.rest, act, cur_stream());
+  return out;
+}
+
+// (tile, its rows, the tile of the rest) that the rule in wide_gemm.hip takes
+std::tuple<int, int, int> wide_gemm_plan(int64_t M, int64_t N, int64_t K,
+                                         bool glu) {
+  int tile = -1, rows, rest;
+  if (qsa_wide_gemm_plan((int)M, (int)N, (int)K, glu, &tile, &rows, &rest) == 1e30f)
+    tile = -1;
+  return {tile, rows, rest};
+}
+
+// a @ w^T by a tile of wide_gemm.hip, with act as in glu_gemm's kernels
+Tensor wide_gemm(Tensor a, Tensor w, int64_t tile, int64_t act) {
+  CHK_DEV(a); CHK_SAME(a, w);
+  TORCH_CHECK(rows_gemm_fits(a, w, act != 0) && act >= 0 && act <= 3,
+              "bf16 a [M, K], w [N, K] with K % 64 and N % 16 (gated: 32)");
+  const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
+  TORCH_CHECK(qsa_wide_gemm_fits((int)tile, K, (int)act) &&
+                  (256 * a.stride(0) + K) * 2 < (4ll << 30) &&
+                  256ll * N * 2 < (4ll << 30), "tile, K and strides");
+  Tensor out = torch::empty({M, act ? N / 2 : N}, a.options());
+  qsa_wide_gemm_launch(u16(a), u16(w), u16m(out), M, N, K, a.stride(0), (int)tile,
+                       (int)act, cur_stream());
+  return out;
 }
 
 // (tile, shares of K) that the rule in rows_gemm.hip takes
@@ -1098,6 +1177,15 @@ Tensor rmsnorm_shares(Tensor parts, Tensor res, Tensor w, double eps) {
 Tensor rows_glu(Tensor a, Tensor w, bool gelu, bool rounded) {
   TORCH_CHECK(rounded || !gelu, "gelu of the stored products only");
   return rows_gemm_run(a, w, gelu ? 2 : rounded ? 1 : 3);
+}
+
+// a @ w^T, for a reader that adds shares perhaps in them, and the gated activation of
+// it, by whichever kernel the rules give
+Tensor gemm(Tensor a, Tensor w) { return gemm_run(a, w, 0); }
+Tensor gemm_parts(Tensor a, Tensor w) { return gemm_run(a, w, 0, true); }
+Tensor glu_gemm(Tensor a, Tensor w, bool gelu, bool rounded) {
+  TORCH_CHECK(rounded || !gelu, "gelu of the stored products only");
+  return gemm_run(a, w, gelu ? 2 : rounded ? 1 : 3);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1141,5 +1229,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "whether sizes are rows_gemm's, or with the activation inside");
   m.def("rows_gemm_plan", &rows_gemm_plan, "tile and shares of a product");
   m.def("rows_glu", &rows_glu, "the same with the gated activation inside");
-  m.def("rows_glu_ok", &rows_glu_ok, "whether a gated product is rows_glu's");
+  m.def("gemm", &gemm, "rows_gemm or wide_gemm by size");
+  m.def("gemm_ok", &gemm_ok, "whether a product is one of theirs");
+  m.def("gemm_parts", &gemm_parts, "the same, shares of K left to the reader");
+  m.def("glu_gemm", &glu_gemm, "the same with the gated activation inside");
+  m.def("glu_gemm_ok", &glu_gemm_ok, "whether a gated product is one of theirs");
+  m.def("wide_gemm", &wide_gemm, "GEMM of many rows by a given tile");
+  m.def("wide_gemm_plan", &wide_gemm_plan, "tiles and rows of a product");
 }

@@ -21,13 +21,9 @@
 // with the activation (there a pass of its own):
 //   28672 x 4096 53.3 -> 43.0  53.5 -> 43.0  57.1 -> 51.2  66.4 -> 59.3 167 -> 180
 //   16384 x 2048 21.9 -> 14.3  20.9 -> 15.3  24.0 -> 19.2  30.6 -> 23.6  53 -> 52
-// and 820 -> 735 at 13,800 rows.  What limits 256 x 256 at 1.3 PFLOP/s (28672 x
-// 4096 x 8192, the library 1.5): matrix cores 72 % busy at 1.6 GHz (82 %), LDS as
-// many cycles as they; four waves of 128 x 128, stages of 32, products of 32 x 32
-// and other orders of reads and loads were within 3 % or slower.
-#include "lm_common.h"
-
-using rsrc_t = __amdgpu_buffer_rsrc_t;
+// What limits 256 x 256 at 1.3 PFLOP/s is the loads' latency with two stages in LDS;
+// products that fill the chip are wide_gemm.hip's.
+#include "tile_gemm.h"
 
 struct RowsArgs {
   const bf16_t* A;                     // [M, K], row stride lda
@@ -38,29 +34,6 @@ struct RowsArgs {
   int MB, NB;                          // blocks along rows and columns
   unsigned int lda;                    // elements
 };
-
-// of the products as they are stored, or of their sums
-enum { ACT_NONE = 0, ACT_SILU = 1, ACT_GELU = 2, ACT_SILU_SUM = 3 };
-
-__device__ __forceinline__ float as_bf16(float v) {
-  return bf16_to_f32(cvt_bf16(v));
-}
-
-// all of a wave's LDS reads are in, and at most N of its loads under way
-template <int N> __device__ __forceinline__ void wait_loads() {
-  static_assert(N < 64, "the counter's range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 7 << 4);
-}
-
-// A barrier that neither waits for loads nor lets memory accesses pass: what
-// the waves have read and received is settled by wait_loads before it.
-__device__ __forceinline__ void stage_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-}
 
 // Whether two blocks of eight waves share a CU's 160 KB (128 bytes a row and stage)
 constexpr bool rows_pair(int bm, int bn, int waves, int st) {

@@ -1,0 +1,113 @@
+"""Products of many rows (ops/hip/wide_gemm.hip): every tile at the ends of rows,
+columns and K, blocks that take several tiles, and the split of a product's rows."""
+
+import pytest
+import torch
+
+from quickstart_streaming_agents_amd.ops import dispatch as D
+from quickstart_streaming_agents_amd.ops import lm_ext
+
+BF, DEV = torch.bfloat16, "cuda:0"
+TILES = [(256, 256, 2), (192, 256, 2), (256, 192, 2), (192, 192, 2),
+         (256, 128, 3), (128, 256, 2), (192, 128, 3), (128, 192, 3),
+         (128, 128, 4)]            # rows, columns, stages ahead
+
+
+def operands(M, N, K, scale=1.0):
+    """Rows of a slice, 16 bytes aligned."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + 24, generator=g).to(BF).to(DEV)[:, 8:K + 8]
+    w = (torch.randn(N, K, generator=g) * scale).to(BF).to(DEV)
+    torch.full((M, N), float("nan"), dtype=BF, device=DEV)      # stale memory
+    return x, w
+
+
+def check(got, x, w, act):
+    """f32 sums of K products; gate and up are rounded to bf16 (but for act 3)
+    before an activation whose slope is at most 1.13 and whose __expf and division
+    are good to 2^-20; the result is rounded to bf16."""
+    a, b, K = x.double(), w.double(), x.shape[1]
+    y, e = a @ b.T, K * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    if act == 0:
+        assert ((got.double() - y).abs() <= 2.0 ** -8 * y.abs() + e).all()
+        return
+    e = e + 2.0 ** -20 + (0.0 if act == 3 else 2.0 ** -8) * y.abs()
+    (p, q), (ep, eq) = y.chunk(2, 1), e.chunk(2, 1)
+    f = torch.nn.functional.gelu(p, approximate="tanh") if act == 2 else \
+        torch.nn.functional.silu(p)
+    bound = (2.0 ** -8 + 2.0 ** -18) * (f * q).abs() + 1.13 * ep * q.abs() \
+        + (f.abs() + ep) * eq
+    assert ((got.double() - f * q).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [0, 1, 2, 3])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_tiles(tile, act):
+    """One row and one column tile, ends inside a tile, the shortest K, and so many
+    tiles that blocks take three of them, the last turn a part."""
+    bm, bn, ahead = TILES[tile]
+    if act and bn % 128:
+        with pytest.raises(RuntimeError):
+            lm_ext().wide_gemm(*operands(64, 64, 1024), tile, act)
+        return
+    short = 64 * (2 * ahead - 1)
+    for M, N, K in [(1, 32, short), (bm - 1, bn - 32, short + 64),
+                    (bm + 1, bn + 32, short), (17 * bm + 5, 33 * bn, short)]:
+        x, w = operands(M, N, K, K ** -0.5 if act else 1.0)
+        check(lm_ext().wide_gemm(x, w, tile, act), x, w, act)
+    with pytest.raises(RuntimeError):
+        lm_ext().wide_gemm(*operands(64, 64, short - 64), tile, act)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,tail", [(16, 0), (48, 16), (272, 16)])
+def test_columns_in_sixteens(N, tail):
+    for tile in range(len(TILES)):
+        x, w = operands(300, N, 448)
+        check(lm_ext().wide_gemm(x, w, tile, 0), x, w, 0)
+
+
+SPLIT = [(2213, 9216, 448), (3677, 6784, 1536), (5595, 4864, 512)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SPLIT)
+def test_by_the_rules(M, N, K):
+    """As models call them: gated or not, and with rows apart."""
+    x, w = operands(M, N, K, K ** -0.5)
+    assert lm_ext().gemm_ok(x, w) and D.glu_linear_ok(x, w)
+    assert lm_ext().wide_gemm_plan(M, N, K, False)[1] < M
+    check(D.linear(x, w), x, w, 0)
+    check(D.glu_linear(x, w), x, w, 1)
+
+
+@pytest.mark.gpu
+def test_replayed():
+    x, w = operands(1024, 10_240, 512)
+    want = D.linear(x, w)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        got = D.linear(x, w)
+    for _ in range(3):
+        got.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("glu", [False, True])
+def test_plans(glu):
+    """Whole tiles apart, tiles that the activation and K allow."""
+    apart = 0
+    for M in (256, 1000, 2700, 4700, 10_816, 13_800, 44_800):
+        for N, K in ((512, 192), (2048, 448), (4096, 4096), (5568, 5888),
+                     (28_672, 4096), (32_736, 256)):
+            tile, rows, rest = lm_ext().wide_gemm_plan(M, N, K, glu)
+            for t in [tile] + [rest] * (rows < M):
+                bm, bn, ahead = TILES[t]
+                assert K >= 64 * (2 * ahead - 1) and not (glu and bn % 128)
+            assert rows == M or (0 < rows < M and rows % TILES[tile][0] == 0)
+            apart += rows < M
+    assert apart > 3
+    assert lm_ext().wide_gemm_plan(1000, 1024, 128, glu)[0] == -1
