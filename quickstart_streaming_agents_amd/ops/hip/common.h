@@ -6,6 +6,12 @@
 
 #define QSA_WAVE 64
 
+// The last-level cache, and the cache policy of loads through buffers or to LDS that
+// leave no trace in it (__builtin_nontemporal_load otherwise).  What is read once
+// in a step whose reads do not fit there together only drives out the rest.
+#define QSA_LLC (256ll << 20)
+#define QSA_NT 2
+
 // ---- bf16 <-> f32 ----------------------------------------------------------
 __device__ __forceinline__ float bf16_to_f32(unsigned short h) {
   union { unsigned int u; float f; } v;

@@ -11,8 +11,8 @@
 // keeps 8 KiB of documents per wave on their way while the previous step
 // multiplies; T = 1 serves indexes whose 64-document blocks would leave CUs idle.
 // 100,000 x 1536, k = 3: 8 queries 146 us with rows loaded straight into the
-// matrix cores' layout, 115 through LDS (5.3 TB/s), and 7 of merge; 32 queries
-// 200 and 136; 10,000 documents, 8 queries 19.5 and 14.7.
+// matrix cores' layout, 112 through LDS, 98 past the last-level cache (6.3 TB/s),
+// and 7 of merge; 32 queries 200 and 136; 10,000 documents, 8 queries 19.5 and 14.7.
 //
 // Results: scores > -2 in descending order, equal scores by ascending
 // document; what k asks for beyond them is (-2, -1).  NaN scores never enter.
@@ -136,13 +136,17 @@ __device__ __forceinline__ void qsa_topk_wait() {
 // load: read into registers in the matrix cores' layout, the lanes of one load
 // touch 16 rows, which the address unit takes four times as long for.  The next
 // 32 are on their way while these multiply; no wave waits for another.
-template <int T, int QT>               // 16*T documents, 16*QT queries
+// FAR: the index is larger than the last-level cache of 256 MB, where it only drives
+// itself out before the next search: loads that do not stay there (100,000 documents, 8
+// queries 111.5 -> 97.6 us, 6.3 TB/s; 30,000, which stay, 35.4 -> 44.4).
+template <int T, int QT, bool FAR>     // 16*T documents, 16*QT queries
 __global__ void __launch_bounds__(256, T + QT <= 2 ? 4 : T + QT <= 3 ? 3 : 1)
 qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
               const float* __restrict__ docs,     // [N, D] L2-normalized
               float* __restrict__ cand_scores,    // [Q, nblk, k]
               int* __restrict__ cand_ids,         // [Q, nblk, k]
               int Qn, int N, int D, int k) {
+#ifdef __HIP_DEVICE_COMPILE__
   constexpr int ROWS = 16 * (T + QT), LOADS = ROWS / 8, STAGE = ROWS * 32;
   constexpr int RING = 4 * 2 * STAGE, PART = 4 * 16 * T * 17;
   __shared__ __attribute__((aligned(16))) float lds[RING > PART ? RING : PART];
@@ -175,13 +179,18 @@ qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
   const int steps = D / 32;            // whole ones
   float* ring = lds + wave * 2 * STAGE;
   auto fetch = [&](int s, int at) {
+    auto to = [&](int i) {
+      return (__attribute__((address_space(3))) void*)(ring + at * STAGE + i * 256);
+    };
+    auto of = [&](int i) {
+      return (const __attribute__((address_space(1))) void*)(row[i] + s * 32);
+    };
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(row[i] + s * 32),
-          (__attribute__((address_space(3))) void*)(ring + at * STAGE +
-                                                    i * 256),
-          16, 0, 0);
+    for (int i = 0; i < 2 * T; ++i)
+      __builtin_amdgcn_global_load_lds(of(i), to(i), 16, 0, FAR ? QSA_NT : 0);
+#pragma unroll
+    for (int i = 2 * T; i < LOADS; ++i)
+      __builtin_amdgcn_global_load_lds(of(i), to(i), 16, 0, 0);
   };
   float dc[T][8], qc[QT][8];
   int at = 0;
@@ -227,6 +236,7 @@ qsa_topk_scan(const float* __restrict__ queries,  // [Q, D] L2-normalized
   __syncthreads();                     // every wave has read its last stage
   qsa_topk_candidates<T, QT>(reinterpret_cast<float (*)[16 * T][17]>(lds),
                              total, doc0, q0, cand_scores, cand_ids, Qn, N, k);
+#endif
 }
 
 // The same for any other D and alignment, number by number.
@@ -397,9 +407,14 @@ extern "C" void qsa_topk_scan_launch(const float* queries, const float* docs,
 #define QSA_SCAN(T, QT)                                                      \
   {                                                                          \
     const dim3 grid(nblk, (Q + 16 * QT - 1) / (16 * QT));                    \
-    if (vec)                                                                 \
-      hipLaunchKernelGGL((qsa_topk_scan<T, QT>), grid, dim3(256), 0, stream, \
-                         queries, docs, cand_scores, cand_ids, Q, N, D, k);  \
+    if (vec && (long long)N * D * 4 > QSA_LLC)                               \
+      hipLaunchKernelGGL((qsa_topk_scan<T, QT, true>), grid, dim3(256), 0,   \
+                         stream, queries, docs, cand_scores, cand_ids, Q, N, \
+                         D, k);                                              \
+    else if (vec)                                                            \
+      hipLaunchKernelGGL((qsa_topk_scan<T, QT, false>), grid, dim3(256), 0,  \
+                         stream, queries, docs, cand_scores, cand_ids, Q, N, \
+                         D, k);                                              \
     else                                                                     \
       hipLaunchKernelGGL((qsa_topk_scan_any<T, QT>), grid, dim3(256), 0,     \
                          stream, queries, docs, cand_scores, cand_ids, Q, N, \
