@@ -178,6 +178,12 @@ class LlamaModel:
                             L[key + "_f8"] = D.pack_weight_fp8(wt)
                 if D.can_pack_weight(*self.lm_head.shape):
                     self.lm_head_f8 = D.pack_weight_fp8(self.lm_head)
+                # whether a step's weights are more than the last-level cache of
+                # 256 MB keeps beside keys and values (skinny_stream.h, FAR)
+                packs = [p for L in self.layers for k, p in L.items()
+                         if k.endswith("_f8")] + [self.lm_head_f8]
+                self.weights_far = sum(p[0].numel() for p in packs
+                                       if p is not None) > 192 << 20
             else:
                 def want(shape):
                     # only shapes where bf16 skinny beats rocBLAS
@@ -326,28 +332,28 @@ class LlamaModel:
         """A step of at most 32 rows on the fp8 weight streams: the
         projections norm their input, gate and add to the residual, so a
         layer is four of them and the attention."""
-        B, eps = tokens.shape[0], self.cfg.norm_eps
+        B, eps, far = tokens.shape[0], self.cfg.norm_eps, self.weights_far
         parts = self.cfg.hidden // 16        # of a row's sum of squares
         norms = [L["attn_norm"] for L in self.layers] + [self.final_norm]
         res, x, ss = D.embed_rows(self.embed, tokens, norms[0])
         n = 1
         for li, L in enumerate(self.layers):
             qkv = D.norm_linear_fp8(x, ss, n, B, eps, L["wqkv_f8"],
-                                    *L["wqkv"].shape)
+                                    *L["wqkv"].shape, far=far)
             attn = self._decode_attention(qkv, L, li, kv, block_table,
                                           seq_lens, True,
                                           (L["wdown_f8"][0], L["wo_f8"][0]))
             x, ss = D.linear_residual_fp8(
                 attn if attn.dim() == 4 else attn.view(B, -1), L["wo_f8"],
-                *L["wo"].shape, res, L["mlp_norm"])
+                *L["wo"].shape, res, L["mlp_norm"], far)
             n = parts
             act = D.norm_linear_fp8(x, ss, n, B, eps, L["wgu_f8"],
-                                    *L["wgu"].shape, glu=True)
+                                    *L["wgu"].shape, glu=True, far=far)
             x, ss = D.linear_residual_fp8(act, L["wdown_f8"],
                                           *L["wdown"].shape, res,
-                                          norms[li + 1])
+                                          norms[li + 1], far)
         return D.norm_linear_fp8(x, ss, n, B, eps, self.lm_head_f8,
-                                 *self.lm_head.shape)
+                                 *self.lm_head.shape, far=far)
 
     def _ffn(self, L: dict, h: torch.Tensor) -> torch.Tensor:
         """Dense SwiGLU FFN (TP row/col-parallel). Mixtral overrides with

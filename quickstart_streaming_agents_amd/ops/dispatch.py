@@ -326,19 +326,21 @@ def embed_rows(embed: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor):
 
 def norm_linear_fp8(x: torch.Tensor, ss: torch.Tensor, parts: int, rows: int,
                     eps: float, packed: tuple, n: int, k: int,
-                    glu: bool = False) -> torch.Tensor:
+                    glu: bool = False, far: bool = True) -> torch.Tensor:
     """Normed step rows through a packed fp8 weight: [rows, n].  With `glu`
-    its rows are [gate; up] and the result is silu(gate) * up, step rows."""
+    its rows are [gate; up] and the result is silu(gate) * up, step rows.
+    `far`: the step's weights exceed the last-level cache, so they are read past
+    it (ops/hip/skinny_stream.h)."""
     return ext().skinny_gemm_fp8_norm(x, ss, parts, rows, eps, packed[0],
-                                      packed[1], n, k, glu)
+                                      packed[1], n, k, glu, far)
 
 
 def linear_residual_fp8(x: torch.Tensor, packed: tuple, n: int, k: int,
-                        res: torch.Tensor, w: torch.Tensor):
+                        res: torch.Tensor, w: torch.Tensor, far: bool = True):
     """res <- res + step rows x through a packed fp8 weight, in place; returns
     the step rows of the norm with weight w that follows, and ss."""
     return ext().skinny_gemm_fp8_residual(x, packed[0], packed[1], n, k, res,
-                                          w)
+                                          w, far)
 
 
 # ---- mixer decoders (qsa_lm_hip) ------------------------------------------

@@ -126,7 +126,8 @@ struct GqaFinish {
   float out_scale;
 };
 
-template <int KS, int ET, bool MERGE>  // D <= 32*KS, E <= 16*ET
+// FAR: past the last-level cache.
+template <int KS, int ET, bool MERGE, bool FAR>  // D <= 32*KS, E <= 16*ET
 __global__ void __launch_bounds__(256, KS <= 4 && ET <= 8 ? 2 : 1)
 qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                   const bf16_t* __restrict__ vc,
@@ -183,8 +184,9 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
           const int d = s * 32 + hi * 8;          // past D: times zero
-          kf[pt][s] = *reinterpret_cast<const bf16x8_v*>(
+          const bf16x8_v* at = reinterpret_cast<const bf16x8_v*>(
               kb + (unsigned)((pt * 16 + col) * D + (d < D ? d : 0)));
+          kf[pt][s] = FAR ? __builtin_nontemporal_load(at) : *at;
         }
     };
     auto fetch_v = [&](int i) {
@@ -195,8 +197,9 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
         const int k = lane + u * 64;
         const int r = k / VG, c = (k % VG) * 8;
         const bool ok = c < E && i * 32 + r < n;
-        const u32x4_v v = *reinterpret_cast<const u32x4_v*>(
+        const u32x4_v* at = reinterpret_cast<const u32x4_v*>(
             vb + (unsigned)(ok ? r * E + c : 0));
+        const u32x4_v v = FAR ? __builtin_nontemporal_load(at) : *at;
         vr[u] = ok ? v : (u32x4_v){0, 0, 0, 0};
       }
     };
@@ -419,17 +422,22 @@ extern "C" void qsa_gqa_rows_mfma_launch(
   dim3 grid((unsigned)((units + 3) / 4));
   const float scale2 = scale * LOG2E;
   const GqaFinish fin{sink, gate, out, gstride, ostride, out_scale};
+  // pages of many rows, read once a step beside those of other layers, would drive
+  // each other out of the last-level cache (16 heads on 8 of 128, 64 rows of 600-1400
+  // keys, 4 layers of 268 MB: 68.9 us with loads that stay there, 52.7 with others);
+  // rows that share pages (portions' few tokens) read them from L2
+  const bool far = (long long)R * max_pages * G * (D + E) * 2 * PG > 32 << 20 &&
+                   !row_item;
 #define QSA_GM(K, V)                                                          \
-  if (part_o)                                                                 \
-    hipLaunchKernelGGL((qsa_gqa_rows_mfma<K, V, false>), grid, dim3(256), 0,  \
-                       st, q, kc, vc, block_table, max_pages, row_item,       \
-                       row_len, part_o, part_ml, H, G, D, E, scale2, NS,      \
-                       units, fin);                                           \
-  else                                                                        \
-    hipLaunchKernelGGL((qsa_gqa_rows_mfma<K, V, true>), grid, dim3(256), 0,   \
-                       st, q, kc, vc, block_table, max_pages, row_item,       \
-                       row_len, part_o, part_ml, H, G, D, E, scale2, NS,      \
-                       units, fin)
+  if (part_o && far) QSA_GM_AS(K, V, false, true);                            \
+  else if (part_o) QSA_GM_AS(K, V, false, false);                             \
+  else if (far) QSA_GM_AS(K, V, true, true);                                  \
+  else QSA_GM_AS(K, V, true, false)
+#define QSA_GM_AS(K, V, MERGE, FAR)                                           \
+  hipLaunchKernelGGL((qsa_gqa_rows_mfma<K, V, MERGE, FAR>), grid, dim3(256),  \
+                     0, st, q, kc, vc, block_table, max_pages, row_item,      \
+                     row_len, part_o, part_ml, H, G, D, E, scale2, NS,        \
+                     units, fin)
 #define QSA_GM_E(K)                                                           \
   if (E <= 32) { QSA_GM(K, 2); }                                              \
   else if (E <= 64) { QSA_GM(K, 4); }                                         \
@@ -441,6 +449,7 @@ extern "C" void qsa_gqa_rows_mfma_launch(
   else { QSA_GM_E(8); }
 #undef QSA_GM_E
 #undef QSA_GM
+#undef QSA_GM_AS
   if (!part_o) return;
   const long long total = (long long)R * H;
   if (NS > 8)

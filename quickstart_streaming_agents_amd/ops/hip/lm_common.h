@@ -71,6 +71,37 @@ __device__ __forceinline__ void stv(T* p, const float* v) {
   }
 }
 
+// VEC numbers of a recurrent state; FAR: they leave no trace in the last-level cache,
+// where the states of many rows and layers would drive each other out between steps
+template <bool FAR, int VEC>
+__device__ __forceinline__ void ld_state(const float* p, float* v) {
+  if constexpr (VEC == 4) {
+    typedef __attribute__((ext_vector_type(4))) float f4;
+    const f4* at = reinterpret_cast<const f4*>(p);
+    const f4 x = FAR ? __builtin_nontemporal_load(at) : *at;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = x[j];
+  } else {
+    static_assert(VEC == 1, "one or four");
+    v[0] = FAR ? __builtin_nontemporal_load(p) : *p;
+  }
+}
+template <bool FAR, int VEC>
+__device__ __forceinline__ void st_state(float* p, const float* v) {
+  if constexpr (VEC == 4) {
+    typedef __attribute__((ext_vector_type(4))) float f4;
+    const f4 x = {v[0], v[1], v[2], v[3]};
+    if constexpr (FAR) __builtin_nontemporal_store(x, reinterpret_cast<f4*>(p));
+    else *reinterpret_cast<f4*>(p) = x;
+  } else if constexpr (FAR) {
+    __builtin_nontemporal_store(v[0], p);
+  } else {
+    *p = v[0];
+  }
+}
+// states of one layer beyond this
+#define QSA_FAR_STATE (32ll << 20)
+
 __device__ __forceinline__ float silu_f(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float sigmoid_f(float z) {
   return 1.f / (1.f + expf(-z));

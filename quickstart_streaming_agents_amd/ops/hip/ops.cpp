@@ -86,7 +86,8 @@ extern "C" int qsa_skinny_gemm_probe_launch(const unsigned short*,
 extern "C" void qsa_skinny_gemm_fp8_launch(
     const unsigned short*, const unsigned char*, const float*,
     unsigned short*, unsigned short*, int, int, long long, long long, int,
-    const unsigned short*, const float*, int, float, int, float*, hipStream_t);
+    const unsigned short*, const float*, int, float, int, float*, int,
+    hipStream_t);
 extern "C" int qsa_skinny_gemm_fp8_probe_launch(
     const unsigned short*, const unsigned char*, const float*,
     unsigned short*, int, int, long long, long long, int, int, int,
@@ -606,7 +607,7 @@ static int chk_skinny_fp8(const torch::Tensor& a, const torch::Tensor& qf,
 }
 
 torch::Tensor skinny_gemm_fp8(torch::Tensor a, torch::Tensor qf,
-                              torch::Tensor scale, long N, long K) {
+                              torch::Tensor scale, long N, long K, bool far) {
   // C[M,N] = a @ (scale[N] * dequant(Q))^T; Q pre-packed fp8 e4m3 in the
   // fragment-pair-major stream layout (skinny_gemm_fp8.hip header).
   const int M = chk_skinny_fp8(a, qf, scale, N, K);
@@ -614,7 +615,7 @@ torch::Tensor skinny_gemm_fp8(torch::Tensor a, torch::Tensor qf,
   qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
                              scale.data_ptr<float>(), u16m(out), nullptr, M,
                              (int)N, K, a.stride(0), 0, nullptr, nullptr, 0,
-                             0.f, 0, nullptr, cur_stream());
+                             0.f, 0, nullptr, far, cur_stream());
   return out;
 }
 
@@ -632,7 +633,7 @@ static void chk_step_rows(const torch::Tensor& a, long M, long K) {
 torch::Tensor skinny_gemm_fp8_norm(torch::Tensor a, torch::Tensor ss,
                                    long parts, long M, double eps,
                                    torch::Tensor qf, torch::Tensor scale,
-                                   long N, long K, bool glu) {
+                                   long N, long K, bool glu, bool far) {
   // a: rows x * w of an rms norm; 1/rms from the rows' sums of squares.
   // glu: Q's rows are [gate; up], returns silu(gate) * up as step rows.
   chk_step_rows(a, M, K);
@@ -647,13 +648,13 @@ torch::Tensor skinny_gemm_fp8_norm(torch::Tensor a, torch::Tensor ss,
                              scale.data_ptr<float>(), u16m(out), nullptr,
                              (int)M, (int)N, K, K, step_tiles(M) > 0, nullptr,
                              ss.data_ptr<float>(), (int)parts, (float)eps,
-                             glu ? 1 : 0, nullptr, cur_stream());
+                             glu ? 1 : 0, nullptr, far, cur_stream());
   return out;
 }
 
 std::vector<torch::Tensor> skinny_gemm_fp8_residual(
     torch::Tensor a, torch::Tensor qf, torch::Tensor scale, long N, long K,
-    torch::Tensor res, torch::Tensor w) {
+    torch::Tensor res, torch::Tensor w, bool far) {
   // res [M, N] <- res + the product; returns the rows of the norm with weight
   // w that follows (before 1/rms) and the sums of squares in N/16 parts
   CHK_DEV(res); CHK_BF16(res); CHK_CONT(res);
@@ -669,7 +670,7 @@ std::vector<torch::Tensor> skinny_gemm_fp8_residual(
   qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
                              scale.data_ptr<float>(), u16m(res), u16m(next),
                              (int)M, (int)N, K, K, step_tiles(M) > 0, u16(w),
-                             nullptr, 0, 0.f, 0, ss.data_ptr<float>(),
+                             nullptr, 0, 0.f, 0, ss.data_ptr<float>(), far,
                              cur_stream());
   return {next, ss};
 }
@@ -894,15 +895,22 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm_probe", &skinny_gemm_probe,
         "tuning probe: waves, tiles");
   m.def("skinny_gemm_fp8", &skinny_gemm_fp8,
-        "fp8-weight decode GEMM (M<=32): half the weight stream");
+        "fp8-weight decode GEMM (M<=32): half the weight stream",
+        py::arg("a"), py::arg("qf"), py::arg("scale"), py::arg("N"),
+        py::arg("K"), py::arg("far") = true);
   m.def("gemm_fp8_batch", &gemm_fp8_batch,
         "batched-M (<=256) fp8 weight-stream GEMM with optional split-K");
   m.def("skinny_gemm_fp8_probe", &skinny_gemm_fp8_probe,
         "fp8 tuning probe: waves, tiles");
   m.def("skinny_gemm_fp8_norm", &skinny_gemm_fp8_norm,
-        "fp8-weight decode GEMM of rms-normed rows, optionally gated");
+        "fp8-weight decode GEMM of rms-normed rows, optionally gated",
+        py::arg("a"), py::arg("ss"), py::arg("parts"), py::arg("M"),
+        py::arg("eps"), py::arg("qf"), py::arg("scale"), py::arg("N"),
+        py::arg("K"), py::arg("glu"), py::arg("far") = true);
   m.def("skinny_gemm_fp8_residual", &skinny_gemm_fp8_residual,
-        "fp8-weight decode GEMM added to the residual stream");
+        "fp8-weight decode GEMM added to the residual stream",
+        py::arg("a"), py::arg("qf"), py::arg("scale"), py::arg("N"),
+        py::arg("K"), py::arg("res"), py::arg("w"), py::arg("far") = true);
   m.def("embed_rows", &embed_rows,
         "a step's first rows and their sums of squares");
   m.def("topk_cosine_packed", &topk_cosine_packed,

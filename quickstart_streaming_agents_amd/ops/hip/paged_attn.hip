@@ -115,9 +115,9 @@ template <int N> __device__ __forceinline__ void wait_vm() {
   asm volatile("" ::: "memory");
 }
 
-template <int D, int NW, bool FUSE>
-__global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
-qsa_paged_attn_mfma(DecodeArgs p) {
+// FAR: loads of pages that leave no trace in the last-level cache (see the launch).
+template <int D, int NW, bool FUSE, bool FAR>
+__device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p) {
   constexpr int KSTEPS = D / 32;      // QK^T k-steps (4 for D=128)
   constexpr int DTILES = D / 16;      // PV d-tiles (8 for D=128)
   constexpr int VT = D * QSA_PAGE;    // elements of a value page
@@ -172,9 +172,11 @@ qsa_paged_attn_mfma(DecodeArgs p) {
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks)
-          kf[pt][ks] = *reinterpret_cast<const bf16x8_a*>(
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          const bf16x8_a* at = reinterpret_cast<const bf16x8_a*>(
               kbase + ((ks * 4 + hi) * QSA_PAGE + pt * 16 + col) * 8);
+          kf[pt][ks] = FAR ? __builtin_nontemporal_load(at) : *at;
+        }
     };
     // Values go straight to the wave's LDS, 8 rows of 128 bytes at a time, a
     // row's segments exchanged by its number (the reads below then spread over
@@ -191,7 +193,7 @@ qsa_paged_attn_mfma(DecodeArgs p) {
       for (int i = 0; i < D / 8; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             rv, (__attribute__((address_space(3))) void*)(vl + i * 512), 16,
-            voff, i * 1024, 0, 0);
+            voff, i * 1024, 0, FAR ? QSA_NT : 0);
     };
     bf16x8_a kf[4][KSTEPS];
     load_k(page, kf);
@@ -423,6 +425,17 @@ qsa_paged_attn_mfma(DecodeArgs p) {
   }
 }
 
+template <int D, int NW, bool FUSE>
+__global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
+qsa_paged_attn_mfma(DecodeArgs p) {
+  qsa_paged_attn<D, NW, FUSE, false>(p);
+}
+template <int D, int NW, bool FUSE>
+__global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
+qsa_paged_attn_far(DecodeArgs p) {
+  qsa_paged_attn<D, NW, FUSE, true>(p);
+}
+
 template <int D>
 __global__ void __launch_bounds__(128)
 qsa_attn_reduce(const float* __restrict__ part_o,   // [rows, NS, D]
@@ -515,17 +528,26 @@ extern "C" void qsa_paged_attn_mfma_launch(
     }
     grid.x = 256;
   }
+  // A step reads the pages of all layers and all weights, once.  Pages of small
+  // batches may stay in the last-level cache for the next step (the weights are read
+  // past it, skinny_stream.h); large ones would drive each other out.  us a step, with
+  // loads that stay / that do not: 2048-wide, 8 layers, 4 rows of 600-1000 keys (13 MB a
+  // layer) 321 / 350; 16 layers of 64-dim heads, 8 rows of 300-600 (8 MB) 585 / 609, 24
+  // of 800-2000 (80 MB) 987 / 971; 4096-wide, 8 layers, 1 row of 900 (4 MB) 504 / 522,
+  // 16 of 1536-2048 (134 MB) 722 / 702, 192 of 400-1000 (600 MB) 2295 / 2180.
+  const bool far = (long long)B * max_pages * KVH * D * QSA_PAGE * 4 > 32 << 20;
 #define QSA_DECODE(DD, NW)                                                  \
   if (D == DD && waves == NW) {                                             \
-    if (k)                                                                  \
-      hipLaunchKernelGGL((qsa_paged_attn_mfma<DD, NW, true>), grid, block,  \
-                         0, stream, p);                                     \
-    else                                                                    \
-      hipLaunchKernelGGL((qsa_paged_attn_mfma<DD, NW, false>), grid, block, \
-                         0, stream, p);                                     \
+    if (k && far) QSA_DECODE_AS(qsa_paged_attn_far, DD, NW, true);          \
+    else if (k) QSA_DECODE_AS(qsa_paged_attn_mfma, DD, NW, true);           \
+    else if (far) QSA_DECODE_AS(qsa_paged_attn_far, DD, NW, false);         \
+    else QSA_DECODE_AS(qsa_paged_attn_mfma, DD, NW, false);                 \
   }
+#define QSA_DECODE_AS(NAME, DD, NW, FUSE)                                   \
+  hipLaunchKernelGGL((NAME<DD, NW, FUSE>), grid, block, 0, stream, p)
   QSA_DECODE(128, 4) QSA_DECODE(128, 8) QSA_DECODE(64, 4) QSA_DECODE(64, 8)
 #undef QSA_DECODE
+#undef QSA_DECODE_AS
   if (NS == 1) return;
   if (D == 128)
     hipLaunchKernelGGL((qsa_attn_reduce<128>), dim3(B * QH), dim3(128), 0,

@@ -46,7 +46,7 @@ __device__ __forceinline__ float rot_elem(const T* x, int d, int rot,
 // ---------------------------------------------------------------------------
 // Decode: one block per (row, head).
 // ---------------------------------------------------------------------------
-template <typename T, int VEC>
+template <typename T, int VEC, bool FAR>
 __global__ void __launch_bounds__(1024)
 qsa_retention_decode(const T* __restrict__ x, long long xstride,
                      const float* __restrict__ cos_t,
@@ -105,7 +105,7 @@ qsa_retention_decode(const T* __restrict__ x, long long xstride,
 #pragma unroll
           for (int j = 0; j < VEC; ++j) s[j] = 0.f;
         } else {
-          ldv<float, VEC>(sp + (long long)d * E, s);
+          ld_state<FAR, VEC>(sp + (long long)d * E, s);
         }
         const float kd = ks[d], qd = qs[d];
 #pragma unroll
@@ -113,7 +113,7 @@ qsa_retention_decode(const T* __restrict__ x, long long xstride,
           s[j] = fmaf(dec, s[j], kd * vv[j]);
           acc[j] = fmaf(qd, s[j], acc[j]);
         }
-        stv<float, VEC>(sp + (long long)d * E, s);
+        st_state<FAR, VEC>(sp + (long long)d * E, s);
       }
     }
 #pragma unroll
@@ -150,13 +150,16 @@ extern "C" void qsa_retention_decode_launch(
       (long long)B * H <= 512 && (long long)D * E >= 16384 ? 1024 : 256;
   const size_t lds = sizeof(float) *
       (2 * (size_t)D + (E + 3) / 4 * 4 + threads * (vec4 ? 4 : 1));
-#define QSA_RD(T, V)                                                         \
-  hipLaunchKernelGGL((qsa_retention_decode<T, V>), dim3((unsigned)(B * H)),  \
+#define QSA_RD(T, V, FAR)                                                    \
+  hipLaunchKernelGGL((qsa_retention_decode<T, V, FAR>), dim3((unsigned)(B * H)),  \
                      dim3(threads), lds, st, (const T*)x, xstride, cos_t,    \
                      sin_t, decay, state, slots, seq_lens, (T*)out, H, D, E, \
                      rot, cw, kscale, eps, table_len)
-  if (f32) { if (vec4) QSA_RD(float, 4); else QSA_RD(float, 1); }
-  else     { if (vec4) QSA_RD(bf16_t, 4); else QSA_RD(bf16_t, 1); }
+  const bool far = (long long)B * H * D * E * 4 > QSA_FAR_STATE;
+  if (f32) { if (vec4) QSA_RD(float, 4, false); else QSA_RD(float, 1, false); }
+  else if (!vec4) QSA_RD(bf16_t, 1, false);
+  else if (far) QSA_RD(bf16_t, 4, true);
+  else QSA_RD(bf16_t, 4, false);
 #undef QSA_RD
 }
 

@@ -43,7 +43,8 @@ constexpr bool rows_pair(int bm, int bn, int waves, int st) {
 // BM x BN of C in a block of WM x WN waves, K in stages of 64 through a ring of
 // ST places in LDS; with ACT, W's rows are [gate; up] and a wave's column tiles
 // are alternately of either.
-template <int BM, int BN, int WM, int WN, int ST, int ACT>
+// ONCE: W's loads leave no trace in the last-level cache (see the launch).
+template <int BM, int BN, int WM, int WN, int ST, int ACT, bool ONCE>
 __global__ void __launch_bounds__(WM * WN * 64,
                                   rows_pair(BM, BN, WM * WN, ST) ? 4 : 1)
 qsa_rows_gemm(RowsArgs p) {
@@ -110,11 +111,14 @@ qsa_rows_gemm(RowsArgs p) {
     const int k = s + turn < steps ? s + turn : s + turn - steps;
 #pragma unroll
     for (int j = 0; j < L; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          j < AL ? ra : rw,
-          (__attribute__((address_space(3))) void*)(
-              lds + place * STAGE + (wave + j * NW) * 512),
-          16, off[j], k * 128, 0, 0);
+      if (j < AL)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            ra, (lds_void_t*)(lds + place * STAGE + (wave + j * NW) * 512), 16,
+            off[j], k * 128, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rw, (lds_void_t*)(lds + place * STAGE + (wave + j * NW) * 512), 16,
+            off[j], k * 128, 0, ONCE ? QSA_NT : 0);
   };
   const int wm = wave / WN * MT, wn = wave % WN * NT;
   bf16x8_v fa[2][MT], fb[2][NT];
@@ -268,15 +272,28 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
   p.MB = (p.M + BM - 1) / BM;
   p.NB = (p.N + BN - 1) / BN;
   const dim3 grid((unsigned)((long long)p.MB * p.NB * p.S + 7) / 8 * 8);
-#define QSA_RG(ACT) \
-  hipLaunchKernelGGL((qsa_rows_gemm<BM, BN, WM, WN, ST, ACT>), grid, \
+  // One block row reads every weight once, and the weights of a step's other layers
+  // drive it out of the last-level cache before the next step; past it they come faster
+  // and leave it to what fits (decoder of width 4096, 8 layers, 192 rows of 400-1000
+  // keys 2295 -> 2180 us a step with keys and values likewise, 28672 x 4096 57 -> 54;
+  // of width 2048, 64 rows 813 -> 746).  Small ones may be of a model that fits.
+  const bool once = BM <= 192 && p.MB == 1 && (long long)p.N * p.K >= 2 << 20;
+#define QSA_RG_AS(ACT, ONCE) \
+  hipLaunchKernelGGL((qsa_rows_gemm<BM, BN, WM, WN, ST, ACT, ONCE>), grid, \
                      dim3(WM * WN * 64), 0, st, p)
-  if constexpr (BN / WN / 16 % 2 == 0) {
-    if (act == ACT_SILU) { QSA_RG(ACT_SILU); return; }
-    if (act == ACT_GELU) { QSA_RG(ACT_GELU); return; }
-    if (act == ACT_SILU_SUM) { QSA_RG(ACT_SILU_SUM); return; }
+#define QSA_RG(ACT) \
+  if constexpr (BM <= 192) { \
+    if (once) QSA_RG_AS(ACT, true); else QSA_RG_AS(ACT, false); \
+  } else { \
+    QSA_RG_AS(ACT, false); \
   }
-  QSA_RG(ACT_NONE);
+  if constexpr (BN / WN / 16 % 2 == 0) {
+    if (act == ACT_SILU) { QSA_RG(ACT_SILU) return; }
+    if (act == ACT_GELU) { QSA_RG(ACT_GELU) return; }
+    if (act == ACT_SILU_SUM) { QSA_RG(ACT_SILU_SUM) return; }
+  }
+  QSA_RG(ACT_NONE)
+#undef QSA_RG_AS
 #undef QSA_RG
 }
 

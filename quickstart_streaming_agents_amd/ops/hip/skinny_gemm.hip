@@ -10,25 +10,30 @@
 // W is packed once at model init into [N/16, K/32, 16, 32]: one wave
 // instruction reads one 1 KiB 16x32 fragment block.
 //
+// Weights of 4 MB on are taken to be of a model whose weights exceed the last-level
+// cache (skinny_stream.h, FAR).
 // Block shapes follow the fp8 form's measurements: one tile of 16 columns per
 // block, two from 6144 columns on; 4 waves for K up to 2048, 8 above.
 #include "skinny_stream.h"
 
-template <int WAVES, int TILES, int MT>
+template <int WAVES, int TILES, int MT, bool FAR>
 __global__ void __launch_bounds__(WAVES * 64)
 qsa_skinny_gemm(SkinnyArgs p) {
-  skinny_stream<WAVES, TILES, MT, false, false, false, false, false>(p);
+  skinny_stream<WAVES, TILES, MT, false, false, false, false, false, FAR>(p);
 }
 
 template <int WAVES, int TILES>
 static void bf16_go(const SkinnyArgs& p, hipStream_t st) {
   const dim3 grid(p.N / (16 * TILES)), block(WAVES * 64);
-  if (p.M <= 16)
-    hipLaunchKernelGGL((qsa_skinny_gemm<WAVES, TILES, 1>), grid, block, 0, st,
-                       p);
-  else
-    hipLaunchKernelGGL((qsa_skinny_gemm<WAVES, TILES, 2>), grid, block, 0, st,
-                       p);
+#define QSA_GO(MT, FAR)                                                      \
+  hipLaunchKernelGGL((qsa_skinny_gemm<WAVES, TILES, MT, FAR>), grid, block,  \
+                     0, st, p)
+  if (p.M <= 16) {
+    if (p.far) QSA_GO(1, true); else QSA_GO(1, false);
+  } else {
+    if (p.far) QSA_GO(2, true); else QSA_GO(2, false);
+  }
+#undef QSA_GO
 }
 
 static SkinnyArgs bf16_args(const unsigned short* A, const unsigned short* Wf,
@@ -36,7 +41,7 @@ static SkinnyArgs bf16_args(const unsigned short* A, const unsigned short* Wf,
                             long long lda) {
   return SkinnyArgs{A, reinterpret_cast<const u32x4_v*>(Wf), nullptr, C,
                     nullptr, nullptr, nullptr, nullptr, M, N, 0, K, lda,
-                    0.f};
+                    0.f, (long long)N * K >= 2 << 20};
 }
 
 extern "C" void qsa_skinny_gemm_launch(const unsigned short* A,

@@ -28,25 +28,28 @@
 #include "skinny_stream.h"
 
 template <int WAVES, int TILES, int MT, bool PACK, bool NORM, bool GLU,
-          bool RES>
+          bool RES, bool FAR>
 __global__ void __launch_bounds__(WAVES * 64)
 qsa_skinny_gemm_fp8(SkinnyArgs p) {
-  skinny_stream<WAVES, TILES, MT, true, PACK, NORM, GLU, RES>(p);
+  skinny_stream<WAVES, TILES, MT, true, PACK, NORM, GLU, RES, FAR>(p);
 }
 
 template <int WAVES, int TILES, bool NORM, bool GLU, bool RES>
 static void fp8_go(const SkinnyArgs& p, int pack, hipStream_t st) {
   const dim3 grid(p.N / (16 * TILES)), block(WAVES * 64);
-#define QSA_GO(MT, PACK)                                                      \
+#define QSA_GO_AS(MT, PACK, FAR)                                              \
   hipLaunchKernelGGL(                                                         \
-      (qsa_skinny_gemm_fp8<WAVES, TILES, MT, PACK, NORM, GLU, RES>), grid,    \
-      block, 0, st, p)
+      (qsa_skinny_gemm_fp8<WAVES, TILES, MT, PACK, NORM, GLU, RES, FAR>),     \
+      grid, block, 0, st, p)
+#define QSA_GO(MT, PACK)                                                      \
+  if (p.far) QSA_GO_AS(MT, PACK, true); else QSA_GO_AS(MT, PACK, false)
   if (p.M <= 16) {
-    if (pack) QSA_GO(1, true); else QSA_GO(1, false);
+    if (pack) { QSA_GO(1, true); } else { QSA_GO(1, false); }
   } else {
-    if (pack) QSA_GO(2, true); else QSA_GO(2, false);
+    if (pack) { QSA_GO(2, true); } else { QSA_GO(2, false); }
   }
 #undef QSA_GO
+#undef QSA_GO_AS
 }
 
 // Blocks, measured on the projections of 2048- and 4096-wide decoders: waves
@@ -84,9 +87,10 @@ extern "C" void qsa_skinny_gemm_fp8_launch(
     const unsigned short* A, const unsigned char* Qf, const float* scale,
     unsigned short* C, unsigned short* next, int M, int N, long long K,
     long long lda, int pack, const unsigned short* norm_w, const float* ss_in,
-    int parts, float eps, int glu, float* ss_out, hipStream_t stream) {
+    int parts, float eps, int glu, float* ss_out, int far, hipStream_t stream) {
   const SkinnyArgs p{A, reinterpret_cast<const u32x4_v*>(Qf), scale, C, next,
-                     norm_w, ss_in, ss_out, M, N, parts, K, lda, eps};
+                     norm_w, ss_in, ss_out, M, N, parts, K, lda, eps,
+                     far != 0};
   if (ss_out) fp8_any<false, false, true>(p, pack, stream);
   else if (ss_in && glu) fp8_any<true, true, false>(p, pack, stream);
   else if (ss_in) fp8_any<true, false, false>(p, pack, stream);
@@ -100,7 +104,7 @@ extern "C" int qsa_skinny_gemm_fp8_probe_launch(
     int waves, int tiles, hipStream_t stream) {
   const SkinnyArgs p{A, reinterpret_cast<const u32x4_v*>(Qf), scale, C,
                      nullptr, nullptr, nullptr, nullptr, M, N, 0, K, lda,
-                     0.f};
+                     0.f, true};
 #define QSA_CASE(W, T)                                      \
   if (waves == W && tiles == T) {                           \
     fp8_go<W, T, false, false, false>(p, pack, stream);     \

@@ -16,6 +16,13 @@
 //     so.  MT row tiles of 16: one for up to 16 rows, two above.
 //   * Row-major rows beyond M shadow row M-1, packed ones are whatever the
 //     buffer holds; they meet no other row and are never stored.
+//   * FAR: where the weights of a step exceed the last-level cache, each of them
+//     is driven out before the next step, and with it what would stay: keys and
+//     values of small batches, activations, weights read ahead.  Their loads leave
+//     no trace then (16 layers of width 2048, 1 row of 700 keys 577 -> 537 us a
+//     step; 8 layers, 4 rows 357 -> 320; of width 4096, 1 row 547 -> 504).  Weights
+//     that fit are to stay (8 layers of width 1024, 119 MB, 1 row: 187 us, 195 past
+//     the cache).
 // What surrounds a projection in the decoder is done on the way, since every
 // launch costs a few microseconds of a step that is made of hundreds:
 //   NORM  A is x * w of an rms norm; the row factor 1/rms meets the sums at the
@@ -44,6 +51,7 @@ struct SkinnyArgs {
   int M, N, parts;
   long long K, lda;
   float eps;
+  bool far;                            // W is read past the last-level cache
 };
 
 // 8 fp8 bytes (as 2 dwords) -> bf16x8 fragment, exact: every e4m3 value is a
@@ -70,7 +78,7 @@ __device__ __forceinline__ long long packed_at(int row, int k, int mt) {
 }
 
 template <int WAVES, int TILES, int MT, bool FP8, bool PACK, bool NORM,
-          bool GLU, bool RES>
+          bool GLU, bool RES, bool FAR>
 __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   constexpr int WL = FP8 ? 1 : 2;      // 16 B loads of a tile per step
   constexpr int PER = TILES * WL * 4 + MT * 8;
@@ -152,7 +160,9 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
       for (int t = 0; t < TILES; ++t)
 #pragma unroll
         for (int i = 0; i < WL; ++i)
-          g.w[u][t][i] = wp[t][s * (64 * WL) + i * 64];
+          g.w[u][t][i] =
+              FAR ? __builtin_nontemporal_load(wp[t] + s * (64 * WL) + i * 64)
+                  : wp[t][s * (64 * WL) + i * 64];
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll

@@ -38,7 +38,7 @@ __device__ __forceinline__ float softplus_f(float v) {
 // ---------------------------------------------------------------------------
 // Decode: one block per (row, head).
 // ---------------------------------------------------------------------------
-template <typename T, int VEC>
+template <typename T, int VEC, bool FAR>
 __global__ void __launch_bounds__(1024)
 qsa_ssd_decode(const T* __restrict__ u, long long ustride, int zoff,
                int dtoff, const T* __restrict__ xbc,
@@ -95,7 +95,7 @@ qsa_ssd_decode(const T* __restrict__ u, long long ustride, int zoff,
 #pragma unroll
           for (int j = 0; j < VEC; ++j) s[j] = 0.f;
         } else {
-          ldv<float, VEC>(sp + (long long)d * P, s);
+          ld_state<FAR, VEC>(sp + (long long)d * P, s);
         }
         const float kd = bs[d], qd = cs[d];
 #pragma unroll
@@ -103,7 +103,7 @@ qsa_ssd_decode(const T* __restrict__ u, long long ustride, int zoff,
           s[j] = fmaf(dec, s[j], kd * xv[j]);
           acc[j] = fmaf(qd, s[j], acc[j]);
         }
-        stv<float, VEC>(sp + (long long)d * P, s);
+        st_state<FAR, VEC>(sp + (long long)d * P, s);
       }
     }
 #pragma unroll
@@ -137,13 +137,16 @@ extern "C" void qsa_ssd_decode_launch(
       (long long)B * H <= 512 && (long long)N * P >= 16384 ? 1024 : 256;
   const size_t lds = sizeof(float) *
       ((2 * (size_t)N + 3) / 4 * 4 + threads * (vec4 ? 4 : 1));
-#define QSA_SD(T, V)                                                         \
-  hipLaunchKernelGGL((qsa_ssd_decode<T, V>), dim3((unsigned)(B * H)),        \
+#define QSA_SD(T, V, FAR)                                                    \
+  hipLaunchKernelGGL((qsa_ssd_decode<T, V, FAR>), dim3((unsigned)(B * H)),        \
                      dim3(threads), lds, st, (const T*)u, ustride, zoff,     \
                      dtoff, (const T*)xbc, A, dt_bias, Dskip, state, slots,  \
                      seq_lens, (T*)out, H, N, P, G, cw)
-  if (f32) { if (vec4) QSA_SD(float, 4); else QSA_SD(float, 1); }
-  else     { if (vec4) QSA_SD(bf16_t, 4); else QSA_SD(bf16_t, 1); }
+  const bool far = (long long)B * H * N * P * 4 > QSA_FAR_STATE;
+  if (f32) { if (vec4) QSA_SD(float, 4, false); else QSA_SD(float, 1, false); }
+  else if (!vec4) QSA_SD(bf16_t, 1, false);
+  else if (far) QSA_SD(bf16_t, 4, true);
+  else QSA_SD(bf16_t, 4, false);
 #undef QSA_SD
 }
 

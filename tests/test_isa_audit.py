@@ -105,6 +105,22 @@ def test_counted_waits_of_decode_attention():
         assert counted_waits(code, keys) == 1, name
 
 
+def test_counted_waits_past_the_cache():
+    """The same of the forms whose pages are read past the last-level cache."""
+    import isa_check
+    so = isa_check.find_so()
+    if so is None or not os.path.exists(isa_check.BUNDLER):
+        pytest.skip("built extension or ROCm LLVM tools unavailable")
+    with tempfile.TemporaryDirectory() as wd:
+        kernels = isa_check.instructions(
+            isa_check.extract_hsacos(so, wd), "qsa_paged_attn_far")
+    assert len(kernels) == 8
+    for name, code in kernels.items():
+        keys = 16 if "ILi128E" in name else 8
+        assert counted_waits(code, keys) == 1, name
+        assert sum(t.endswith(" nt") for t in code) >= keys, name
+
+
 def test_the_audit_sees_a_moved_load():
     keys = ["global_load_dwordx4 v[0:3], v[4:5], off"] * 2
     wait = ["s_waitcnt vmcnt(2)"]
