@@ -807,18 +807,30 @@ extern "C" void qsa_rope_kv_scatter_launch(
 // of 16-row tiles, QT per wave, four waves.  Short portions thus fill tiles
 // with heads, and K and V are read once per kv head.  Key heads run fastest
 // over the blocks: with 8 of them a die's L2 keeps one.
-// Each K and V page goes through LDS once per block; the next page is fetched
-// into registers meanwhile.  Scores come out transposed (row = key, column =
-// query row): softmax state and rescale are lane-local, and the keys are dealt
-// to the score tiles so that a lane ends up with 8 consecutive ones, which is
-// the operand layout of the second product and of 16-byte V reads.  V's 16-byte
-// groups are swizzled by row, so that 8 rows of a tile read all banks once.
-// The bound is LDS reads (each K/V fragment serves QT tiles; at QT = 2 they
-// take as long as the matrix cores) beside exp2, so rescaling is left out when
+// Scores come out transposed (row = key, column = query row): softmax state and
+// rescale are lane-local, and the keys are dealt to the score tiles so that a
+// lane ends up with 8 consecutive ones, which is the operand layout of the
+// second product and of 16-byte V reads.  V's 16-byte groups are swizzled by
+// row, so that 8 rows of a tile read all banks once.
+//
+// Each K and V page goes into LDS once per block, by loads that write it there
+// in that order (the lanes' addresses are permuted, not the places), and both
+// stand twice, so that a turn has one barrier: turn pg loads K of page pg + 2
+// and V of page pg, and multiplies what came a turn before.  A page's products
+// and its softmax depend on each other, and two blocks of a CU that stand at
+// the same barriers do not fill each other's gaps, so a turn's softmax of page
+// pg runs beside the products of page pg - 1 with its values, a few exponents
+// and one fragment of V to each QT products, and the scores of page pg + 1
+// follow with each fragment of K read PD - 1 ahead.  Maxima cross the groups of
+// a column by lane swaps instead of the LDS crossbar.  The matrix cores are busy
+// half of the time, the exponents a quarter; LDS reads (each K/V fragment
+// serves QT tiles) take as long as the matrix cores.  Rescaling is left out when
 // no maximum of the wave moved.
-// 1 x 8192 tokens, 32/8 heads of 128: 3128 us with one wave per 16 rows and
-// head reading K and V through L1, 787 us here (700 TFLOP/s); 64 x 700: 1757 ->
-// 523 us.
+// us, 32/8 heads of 128, with pages by way of registers and one after the other
+// / here: 1 x 8192 tokens 613 / 519 (897 / 1060 TFLOP/s), 64 x 500-900 488 / 457,
+// 96 x 20-200 behind 500-1200 292 / 259, 300 + 200 10.4 / 9.7; 16/8 heads, 8 x
+// 1500-3000 198 / 170; 32/8 heads of 64, 32 x 500-900 127 / 121.  PD 2 / 3 / 4: 536 /
+// 519 / 526 us for the first, 125 / 144 / 121 for the last.
 // ---------------------------------------------------------------------------
 #define QSA_NEG (-3.0e38f)
 
@@ -836,11 +848,14 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
                        unsigned short* __restrict__ out,       // [T, QH*D]
                        float scale2, int QH, int KVH, int npmax,
                        long long qstride, int rows, int subs) {
+#ifdef __HIP_DEVICE_COMPILE__          // loads into LDS: not for the host
   constexpr int KS = D / 32;           // k-steps of a score tile
   constexpr int ET = D / 16;           // tiles of value columns
-  constexpr int L = D / 32;            // 16 B loads per thread, K and V each
-  __shared__ __attribute__((aligned(16))) unsigned short kt[64 * D];
-  __shared__ __attribute__((aligned(16))) unsigned short vt[64 * D];
+  constexpr int L = D / 32;            // 1 KB loads per wave, K and V each
+  constexpr int PD = D == 64 ? 4 : 3;  // fragments of K or V in registers
+  constexpr int TILE = QSA_PAGE * D;
+  __shared__ __attribute__((aligned(16))) unsigned short kt[2 * TILE];
+  __shared__ __attribute__((aligned(16))) unsigned short vt[2 * TILE];
   const int tid = threadIdx.x, lane = tid & 63;
   // a scalar: branches on it skip MFMAs, which ignore disabled lanes
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -848,18 +863,63 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
   const int R = QH / KVH;
   const int g = blockIdx.x % KVH;
   const int qb = blockIdx.x / KVH / subs, sub = blockIdx.x / KVH % subs;
-  const int item = qb_item[qb], pos0 = qb_pos0[qb];
-  const int n = item_len[item], start = item_start[item];
+  const int item = __builtin_amdgcn_readfirstlane(qb_item[qb]);
+  const int pos0 = __builtin_amdgcn_readfirstlane(qb_pos0[qb]);
+  const int n = __builtin_amdgcn_readfirstlane(item_len[item]);
+  const int start = __builtin_amdgcn_readfirstlane(item_start[item]);
   const int v0 = pos0 * R + sub * 64 * QT;
   const int vend = min(pos0 + rows, n) * R;
   if (v0 >= vend) return;              // uniform over the block
   const long long off = item_off[item];
   // last key that any row of the block / of this wave sees
-  const int last = start + (CAUSAL ? (min(v0 + 64 * QT, vend) - 1) / R : n - 1);
+  const int last = __builtin_amdgcn_readfirstlane(
+      start + (CAUSAL ? (min(v0 + 64 * QT, vend) - 1) / R : n - 1));
   const int w0 = v0 + wave * 16 * QT;
   const int wfirst = start + min(w0, vend - 1) / R;
   const int wlast = w0 >= vend ? -1
       : CAUSAL ? start + (min(w0 + 16 * QT, vend) - 1) / R : last;
+  // pages of the block, those with keys for this wave, and those whose keys
+  // all its rows see
+  const int pages = last / QSA_PAGE + 1;
+  const int mine =
+      __builtin_amdgcn_readfirstlane(wlast < 0 ? 0 : wlast / QSA_PAGE + 1);
+  const int whole = __builtin_amdgcn_readfirstlane(
+      ((CAUSAL ? wfirst : last) + 1) / QSA_PAGE);
+
+  // LDS places, in pieces of 16 bytes.  K [D/8][64 keys]: place p of a row holds
+  // the key that row p % 16 of score tile p / 16 stands for, 32s + 8h + 4t + r in
+  // row 4h + r of tile 2s + t.  V [D][8]: group j of 8 keys of column e stands
+  // at j ^ sw(e), sw = e&3 | (e>>3 & 1) << 2.  A load fills 1 KB in the order of
+  // the lanes: one row of K, 8 columns of V.
+  const unsigned kfrom = ((lane >> 5) * 32 + (lane >> 2 & 3) * 8 +
+                          (lane >> 4 & 1) * 4 + (lane & 3)) * 16;
+  const unsigned vfrom = (lane >> 3) * 128 +
+      ((lane & 7) ^ ((lane >> 3 & 3) | (wave & 1) << 2)) * 16;
+  const auto table = (const __attribute__((address_space(4))) int*)(
+      block_table + (long long)item * npmax);
+  auto load = [&](const unsigned short* cache, unsigned short* to, int pg,
+                  unsigned from) __attribute__((always_inline)) {
+    const long long tile = ((long long)table[pg] * KVH + g) * TILE;
+    const __amdgpu_buffer_rsrc_t page = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(cache + tile), 0, TILE * 2, 0x00027000);
+#pragma unroll
+    for (int i = 0; i < L; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          page, (__attribute__((address_space(3))) void*)(
+                    to + (pg & 1) * TILE + (wave + 4 * i) * 512),
+          16, from, (wave + 4 * i) * 1024, 0, 0);
+  };
+  // all that the waves loaded has arrived, and they have read what they wanted
+  auto arrived = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(7 << 4);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  };
+  load(kc, kt, 0, kfrom);
+  if (pages > 1) load(kc, kt, 1, kfrom);
 
   // maxima are taken before the scale, which therefore has to be positive
   const bool negative = scale2 < 0.f;
@@ -879,142 +939,149 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
       if (negative) qf[u][s] ^= (short)0x8000;
     }
   }
-  f32x4_v acc[QT][ET];
-  float m[QT], l[QT];
+  f32x4_v acc[QT][ET], sc[QT][4];
+  bf16x8_v pf[QT][2];
+  float m[QT], l[QT], alpha[QT], psum[QT], top[QT];
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
     m[u] = QSA_NEG;
     l[u] = 0.f;
+    alpha[u] = 1.f;
 #pragma unroll
     for (int t = 0; t < ET; ++t) acc[u][t] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
   }
+  bool moved = false;                  // a maximum, by the last softmax
 
-  // LDS places.  K [D/8][64 keys][8]: key 32s + 8h + 4p + r of a page stands
-  // where row h*4 + r of score tile 2s + p reads it.  V [D][64 keys]: group j
-  // of 8 keys of column e stands at j ^ sw(e), sw = e&3 | (e>>3 & 1) << 2.
-  int kdst[L], vdst[L];
-#pragma unroll
-  for (int u = 0; u < L; ++u) {
-    const int i = tid + u * 256, key = i & 63;
-    kdst[u] = ((i & ~63) + (key >> 5) * 32 + ((key >> 2) & 1) * 16 +
-               ((key >> 3) & 3) * 4 + (key & 3)) * 8;
-    const int e = i >> 3;
-    vdst[u] = (e * 8 + ((i & 7) ^ ((e & 3) | ((e >> 1) & 4)))) * 8;
-  }
-  const int* bt = block_table + (long long)item * npmax;
-  u32x4_v kr[L], vr[L];
-  auto fetch = [&](int page) {
-    const long long tile = ((long long)page * KVH + g) * (D * QSA_PAGE);
-    const u32x4_v* kp = reinterpret_cast<const u32x4_v*>(kc + tile) + tid;
-    const u32x4_v* vp = reinterpret_cast<const u32x4_v*>(vc + tile) + tid;
-#pragma unroll
-    for (int u = 0; u < L; ++u) {
-      kr[u] = kp[u * 256];
-      vr[u] = vp[u * 256];
-    }
+  // fragment c of a page: keys of tile c % 4, k-step c / 4; row i of tile t of
+  // the values is column 32(t/2) + 8(i/4) + 4(t%2) + i%4, so that a lane
+  // collects 8 consecutive columns over two tiles
+  auto keys = [&](const unsigned short* k, int c) __attribute__((always_inline)) {
+    return *reinterpret_cast<const bf16x8_v*>(
+        k + (((c >> 2) * 4 + hi) * 64 + (c & 3) * 16 + col) * 8);
   };
-  const int pages = last / QSA_PAGE + 1;
-  fetch(bt[0]);
-  int next = pages > 1 ? bt[1] : 0;
-  for (int pg = 0; pg < pages; ++pg) {
-    const int have = last - pg * QSA_PAGE;        // keys 0..have count
-    lds_barrier();
-    if (have < QSA_PAGE - 1) {
-      // slots nobody has written yet may hold anything, NaN too
-      const int k0 = (tid & 7) * 8;
+  const int vrow = (col >> 2) * 8 + (col & 3);
+  auto vals = [&](const unsigned short* v, int c) __attribute__((always_inline)) {
+    const int s = c / ET, t = c % ET;
+    const int e = (t >> 1) * 32 + (t & 1) * 4 + vrow;
+    return *reinterpret_cast<const bf16x8_v*>(
+        v + (e * 8 + ((s * 4 + hi) ^ (col & 7))) * 8);
+  };
+  auto scores = [&](const unsigned short* k) __attribute__((always_inline)) {
+    bf16x8_v f[PD];
 #pragma unroll
-      for (int u = 0; u < L; ++u)
+    for (int c = 0; c < PD - 1; ++c) f[c] = keys(k, c);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int k = k0 + 2 * e;
-          const unsigned int w = vr[u][e];
-          vr[u][e] = k > have ? 0u : k + 1 > have ? w & 0xffffu : w;
-        }
+    for (int c = 0; c < 4 * KS; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (c + PD - 1 < 4 * KS) f[(c + PD - 1) % PD] = keys(k, c + PD - 1);
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+        sc[u][c & 3] = mfma_bf16(
+            f[c % PD], qf[u][c >> 2],
+            c < 4 ? (f32x4_v){0.f, 0.f, 0.f, 0.f} : sc[u][c & 3]);
     }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // maximum over a column's four groups of lanes
+  auto over = [&](float x) __attribute__((always_inline)) {
+    const auto a = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  };
+  auto maximum = [&](int u) __attribute__((always_inline)) {
+    float mx = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < L; ++u) {
-      *reinterpret_cast<u32x4_v*>(kt + kdst[u]) = kr[u];
-      *reinterpret_cast<u32x4_v*>(vt + vdst[u]) = vr[u];
-    }
-    lds_barrier();
-    if (pg + 1 < pages) {
-      fetch(next);
-      next = pg + 2 < pages ? bt[pg + 2] : 0;
-    }
-    if (pg * QSA_PAGE > wlast) continue;          // nothing for this wave
-
-    f32x4_v sc[QT][4];
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[u][i >> 2][i & 3]);
+    top[u] = fmaxf(m[u], over(mx) * scale2);
+    moved |= top[u] > m[u];
+    alpha[u] = __builtin_amdgcn_exp2f(m[u] - top[u]);
+    psum[u] = 0.f;
+  };
+  unsigned int pk[QT][8];
+  auto weights = [&](int u, int j) __attribute__((always_inline)) {
+    const float a = __builtin_amdgcn_exp2f(
+        fmaf(sc[u][j >> 1][(j & 1) * 2], scale2, -top[u]));
+    const float b = __builtin_amdgcn_exp2f(
+        fmaf(sc[u][j >> 1][(j & 1) * 2 + 1], scale2, -top[u]));
+    psum[u] += a;
+    psum[u] += b;
+    pk[u][j] = cvt_bf16x2(a, b);
+  };
+  auto packed = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int pt = 0; pt < 4; ++pt) {
+    for (int u = 0; u < QT; ++u)
 #pragma unroll
-      for (int u = 0; u < QT; ++u) sc[u][pt] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const bf16x8_v a = *reinterpret_cast<const bf16x8_v*>(
-            kt + ((s * 4 + hi) * 64 + pt * 16 + col) * 8);
-#pragma unroll
-        for (int u = 0; u < QT; ++u)
-          sc[u][pt] = mfma_bf16(a, qf[u][s], sc[u][pt]);
-      }
-    }
-    bf16x8_v pf[QT][2];
-    float alpha[QT], psum[QT], top[QT];
-    bool moved = false;
-    auto softmax = [&](auto edge, auto guard) {
-#pragma unroll
-      for (int u = 0; u < QT; ++u) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            if constexpr (edge.value) {
-              const int p = pg * QSA_PAGE + (pt >> 1) * 32 + hi * 8 +
-                            (pt & 1) * 4 + r;
-              if (p > qpos[u]) sc[u][pt][r] = -INFINITY;
-            }
-            if constexpr (guard.value)
-              sc[u][pt][r] = fmaxf(sc[u][pt][r], -INFINITY);
-            mx = fmaxf(mx, sc[u][pt][r]);
-          }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
-        const float mn = fmaxf(m[u], mx * scale2);
-        moved |= mn > m[u];
-        alpha[u] = __builtin_amdgcn_exp2f(m[u] - mn);
-        psum[u] = 0.f;
-        uint2 pk[4];
-#pragma unroll
-        for (int pt = 0; pt < 4; ++pt) {
-          float p[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            p[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][pt][r], scale2, -mn));
-            psum[u] += p[r];
-          }
-          pk[pt] = make_uint2(cvt_bf16x2(p[0], p[1]), cvt_bf16x2(p[2], p[3]));
-        }
-        top[u] = mn;
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-          pf[u][s] = __builtin_bit_cast(
-              bf16x8_v, make_uint4(pk[2 * s].x, pk[2 * s].y, pk[2 * s + 1].x,
-                                   pk[2 * s + 1].y));
-      }
-    };
-    if (pg * QSA_PAGE + QSA_PAGE - 1 > (CAUSAL ? wfirst : last))
-      softmax(std::true_type{}, std::false_type{});
-    else
-      softmax(std::false_type{}, std::false_type{});
-    bool bad = false;
-#pragma unroll
-    for (int u = 0; u < QT; ++u) bad |= !(psum[u] <= 64.f);
-    // a NaN score counts as no key: masked ones are -inf by now
-    if (__any(bad)) softmax(std::false_type{}, std::true_type{});
+      for (int s = 0; s < 2; ++s)
+        pf[u][s] = __builtin_bit_cast(
+            bf16x8_v, make_uint4(pk[u][4 * s], pk[u][4 * s + 1],
+                                 pk[u][4 * s + 2], pk[u][4 * s + 3]));
+  };
+  // softmax of sc by itself; a NaN score counts as no key
+  auto guarded = [&]() __attribute__((always_inline)) {
+    moved = false;
 #pragma unroll
     for (int u = 0; u < QT; ++u) {
-      m[u] = top[u];
-      l[u] = l[u] * alpha[u] + psum[u];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        sc[u][i >> 2][i & 3] = fmaxf(sc[u][i >> 2][i & 3], -INFINITY);
+      maximum(u);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) weights(u, j);
+    }
+    packed();
+  };
+  // softmax of sc beside the products of the weights before it with v; the
+  // first QT chunks take the maxima, the rest share the exponents
+  auto beside = [&](const unsigned short* v) __attribute__((always_inline)) {
+    constexpr int NC = ET * 2, PAIRS = QT * 8, SPAN = NC - 2;
+    bf16x8_v f[PD];
+    moved = false;
+#pragma unroll
+    for (int c = 0; c < PD - 1; ++c) f[c] = vals(v, c);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (c + PD - 1 < NC) f[(c + PD - 1) % PD] = vals(v, c + PD - 1);
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+        acc[u][c % ET] = mfma_bf16(f[c % PD], pf[u][c / ET], acc[u][c % ET]);
+      if (c < QT) maximum(c);
+#pragma unroll
+      for (int i = 0; i < PAIRS; ++i)
+        if (c == 2 + i * SPAN / PAIRS) weights(i >> 3, i & 7);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    packed();
+  };
+
+  arrived();
+  if (mine > 0) scores(kt);
+#pragma clang loop unroll(disable)
+  for (int pg = 0; pg <= pages; ++pg) {
+    arrived();                         // K of page pg + 1, V of pg - 1
+    if (pg + 2 < pages) load(kc, kt, pg + 2, kfrom);
+    if (pg < pages) load(vc, vt, pg, vfrom);
+    const int other = ((pg + 1) & 1) * TILE;
+    unsigned short* v = vt + other;
+    const int have = last - (pg - 1) * QSA_PAGE;  // keys 0..have of pg - 1 count
+    if (have < QSA_PAGE - 1) {
+      // slots nobody has written yet may hold anything, NaN too
+#pragma unroll
+      for (int i = 0; i < L; ++i) {
+        const int at = tid + i * 256, e = at >> 3;
+        const int k0 = ((at & 7) ^ ((e & 3) | (e >> 1 & 4))) * 8;
+        u32x4_v x = *reinterpret_cast<u32x4_v*>(v + at * 8);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int k = k0 + 2 * c;
+          x[c] = k > have ? 0u : k + 1 > have ? x[c] & 0xffffu : x[c];
+        }
+        *reinterpret_cast<u32x4_v*>(v + at * 8) = x;
+      }
+      lds_barrier();
     }
     if (__any(moved)) {
 #pragma unroll
@@ -1022,19 +1089,43 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
 #pragma unroll
         for (int t = 0; t < ET; ++t) acc[u][t] *= alpha[u];
     }
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int t = 0; t < ET; ++t) {
-        // row i of tile t is column 32(t/2) + 8(i/4) + 4(t%2) + i%4: a lane
-        // collects 8 consecutive columns over two tiles
-        const int e = (t >> 1) * 32 + (col >> 2) * 8 + (t & 1) * 4 + (col & 3);
-        const bf16x8_v a = *reinterpret_cast<const bf16x8_v*>(
-            vt + (e * 8 + ((s * 4 + hi) ^ ((col & 3) | (col & 4)))) * 8);
+    moved = false;
+    if (pg < mine) {
+      if (pg >= whole) {
 #pragma unroll
         for (int u = 0; u < QT; ++u)
-          acc[u][t] = mfma_bf16(a, pf[u][s], acc[u][t]);
+#pragma unroll
+          for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int p = pg * QSA_PAGE + (pt >> 1) * 32 + hi * 8 +
+                            (pt & 1) * 4 + r;
+              if (p > qpos[u]) sc[u][pt][r] = -INFINITY;
+            }
       }
+      bool bad = pg == 0;
+      if (pg > 0) {
+        beside(v);
+#pragma unroll
+        for (int u = 0; u < QT; ++u) bad |= !(psum[u] <= 64.f);
+      }
+      if (__any(bad)) guarded();       // masked scores are -inf by now
+#pragma unroll
+      for (int u = 0; u < QT; ++u) {
+        m[u] = top[u];
+        l[u] = l[u] * alpha[u] + psum[u];
+      }
+      if (pg + 1 < mine) scores(kt + other);
+    } else if (pg == mine && pg > 0) {
+#pragma unroll
+      for (int c = 0; c < 2 * ET; ++c) {
+        const bf16x8_v a = vals(v, c);
+#pragma unroll
+        for (int u = 0; u < QT; ++u)
+          acc[u][c % ET] = mfma_bf16(a, pf[u][c / ET], acc[u][c % ET]);
+        if (c & 1) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
   }
 
 #pragma unroll
@@ -1055,6 +1146,7 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
                      cvt_bf16x2(b[0], b[1]), cvt_bf16x2(b[2], b[3]));
     }
   }
+#endif
 }
 
 extern "C" void qsa_paged_attn_prefill_launch(

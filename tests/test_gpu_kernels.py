@@ -982,6 +982,59 @@ def test_paged_attn_prefill_blocks(ext, D, QH, KVH, rows, causal):
         assert (got - ref).abs().max() <= 2 ** -7 * v.abs().max(), i
 
 
+@pytest.mark.parametrize("D,QH,KVH,rows,scale", [
+    (128, 8, 2, 32, 1.0), (64, 8, 2, 32, 1.0), (128, 8, 2, 16, -1.0),
+    (64, 4, 4, 64, 1.0)])
+def test_paged_attn_prefill_turns(ext, D, QH, KVH, rows, scale):
+    """Every number of pages up to five, waves of a block that end a page
+    apart, larger scores on later pages, and keys of NaN on any page but the
+    first one, which count as none."""
+    from quickstart_streaming_agents_amd.ops import dispatch as disp
+    g = torch.Generator().manual_seed(D + rows)
+    R = QH // KVH
+    items = [(a + d, n) for a in (0, 64, 128, 192) for d, n in
+             ((0, 1), (0, 64), (33, 32), (50, 31), (63, 2), (47, 80))]
+    lens = [n for _, n in items]
+    np_ = [-(-(a + n) // 64) for a, n in items]
+    kc = torch.full((sum(np_), KVH, D // 8, 64, 8), float("nan"))
+    kc = kc.bfloat16().to(dev())
+    vc = torch.full((sum(np_), KVH, D, 64), float("nan")).bfloat16().to(dev())
+    bt = torch.zeros(len(items), max(np_), dtype=torch.int32)
+    offs = [sum(lens[:i]) for i in range(len(items))]
+    q = torch.randn(sum(lens), QH, D, generator=g).bfloat16().to(dev())
+    kv, at = [], 0
+    for i, (a, n) in enumerate(items):
+        bt[i, :np_[i]] = torch.arange(at, at + np_[i])
+        at += np_[i]
+        k = torch.randn(a + n, KVH, D, generator=g)
+        k = k * (1 + torch.arange(a + n) / 64).floor()[:, None, None]
+        for j in (70, 129, 200):
+            k[j:j + 1] = float("nan")
+        k, v = (t.bfloat16().to(dev()) for t in (
+            k, torch.randn(a + n, KVH, D, generator=g)))
+        pos = torch.arange(a + n)
+        disp.kv_scatter(k, v, kc, vc,
+                        (bt[i][pos // 64] * 64 + pos % 64).int().to(dev()))
+        kv.append((k.double(), v.double()))
+    blocks = [(i, p) for i, n in enumerate(lens) for p in range(0, n, rows)]
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=dev())
+    out = ext.paged_attn_prefill(
+        q, kc, vc, bt.to(dev()), mk([b[0] for b in blocks]),
+        mk([b[1] for b in blocks]), mk(offs), mk([a for a, _ in items]),
+        mk(lens), scale * D ** -0.5, True, rows)
+    for i, (a, n) in enumerate(items):
+        k, v = (t.repeat_interleave(R, 1).transpose(0, 1) for t in kv[i])
+        qi = q[offs[i]:offs[i] + n].double().transpose(0, 1)
+        s = qi @ k.transpose(1, 2).contiguous() * (scale * D ** -0.5)
+        j = torch.arange(a + n, device=dev())
+        s = s.masked_fill(s.isnan() | (j[None] > j[a:, None]), float("-inf"))
+        ref = (s.softmax(-1) @ v).transpose(0, 1).reshape(n, QH * D)
+        got = out[offs[i]:offs[i] + n].double()
+        # as above: weights and results rounded to bf16
+        assert (got - ref).norm() <= 5e-3 * ref.norm(), (i, a, n)
+        assert (got - ref).abs().max() <= 2 ** -7 * v.abs().max(), (i, a, n)
+
+
 @pytest.mark.parametrize("T,QH,KVH,D", [
     (1, 8, 8, 64), (63, 4, 2, 128), (65, 32, 8, 128), (200, 28, 4, 128),
     (130, 16, 1, 64)])
