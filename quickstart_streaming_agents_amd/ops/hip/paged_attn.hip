@@ -821,16 +821,17 @@ extern "C" void qsa_rope_kv_scatter_launch(
 // the same barriers do not fill each other's gaps, so a turn's softmax of page
 // pg runs beside the products of page pg - 1 with its values, a few exponents
 // and one fragment of V to each QT products, and the scores of page pg + 1
-// follow with each fragment of K read PD - 1 ahead.  Maxima cross the groups of
+// follow, each fragment of K read PD - 1 ahead.  Maxima cross the groups of
 // a column by lane swaps instead of the LDS crossbar.  The matrix cores are busy
 // half of the time, the exponents a quarter; LDS reads (each K/V fragment
 // serves QT tiles) take as long as the matrix cores.  Rescaling is left out when
 // no maximum of the wave moved.
+// A wave's first and last page stand outside of the loop over the others: paths that
+// meet behind the products took 30 registers more (D = 64: 149 us for 122).
 // us, 32/8 heads of 128, with pages by way of registers and one after the other
-// / here: 1 x 8192 tokens 613 / 519 (897 / 1060 TFLOP/s), 64 x 500-900 488 / 457,
-// 96 x 20-200 behind 500-1200 292 / 259, 300 + 200 10.4 / 9.7; 16/8 heads, 8 x
-// 1500-3000 198 / 170; 32/8 heads of 64, 32 x 500-900 127 / 121.  PD 2 / 3 / 4: 536 /
-// 519 / 526 us for the first, 125 / 144 / 121 for the last.
+// / here: 1 x 8192 tokens 643 / 533 (856 / 1032 TFLOP/s), 64 x 500-900 501 / 463,
+// 96 x 20-200 behind 500-1200 293 / 256, 300 + 200 10.6 / 9.1; 16/8 heads, 8 x
+// 1500-3000 206 / 175; 32/8 heads of 64, 32 x 500-900 130 / 124.
 // ---------------------------------------------------------------------------
 #define QSA_NEG (-3.0e38f)
 
@@ -852,7 +853,7 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
   constexpr int KS = D / 32;           // k-steps of a score tile
   constexpr int ET = D / 16;           // tiles of value columns
   constexpr int L = D / 32;            // 1 KB loads per wave, K and V each
-  constexpr int PD = D == 64 ? 4 : 3;  // fragments of K or V in registers
+  constexpr int PD = D == 64 ? 4 : 5;  // fragments of K or V in registers
   constexpr int TILE = QSA_PAGE * D;
   __shared__ __attribute__((aligned(16))) unsigned short kt[2 * TILE];
   __shared__ __attribute__((aligned(16))) unsigned short vt[2 * TILE];
@@ -891,9 +892,9 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
   // row 4h + r of tile 2s + t.  V [D][8]: group j of 8 keys of column e stands
   // at j ^ sw(e), sw = e&3 | (e>>3 & 1) << 2.  A load fills 1 KB in the order of
   // the lanes: one row of K, 8 columns of V.
-  const unsigned kfrom = ((lane >> 5) * 32 + (lane >> 2 & 3) * 8 +
-                          (lane >> 4 & 1) * 4 + (lane & 3)) * 16;
-  const unsigned vfrom = (lane >> 3) * 128 +
+  const unsigned kfrom = wave * 1024 + ((lane >> 5) * 32 + (lane >> 2 & 3) * 8 +
+                                        (lane >> 4 & 1) * 4 + (lane & 3)) * 16;
+  const unsigned vfrom = wave * 1024 + (lane >> 3) * 128 +
       ((lane & 7) ^ ((lane >> 3 & 3) | (wave & 1) << 2)) * 16;
   const auto table = (const __attribute__((address_space(4))) int*)(
       block_table + (long long)item * npmax);
@@ -907,7 +908,7 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           page, (__attribute__((address_space(3))) void*)(
                     to + (pg & 1) * TILE + (wave + 4 * i) * 512),
-          16, from, (wave + 4 * i) * 1024, 0, 0);
+          16, from, i * 4096, 0, 0);
   };
   // all that the waves loaded has arrived, and they have read what they wanted
   auto arrived = [&]() __attribute__((always_inline)) {
@@ -1057,76 +1058,101 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
     packed();
   };
 
+  // a turn's barrier and loads: K of page pg + 1 and V of pg - 1 are there
+  auto stage = [&](int pg) __attribute__((always_inline)) {
+    arrived();
+    if (pg + 2 < pages) load(kc, kt, pg + 2, kfrom);
+    if (pg < pages) {
+      load(vc, vt, pg, vfrom);
+      return;
+    }
+    const int have = last - (pg - 1) * QSA_PAGE;  // keys 0..have count
+    if (have == QSA_PAGE - 1) return;
+    // slots nobody has written yet may hold anything, NaN too
+    unsigned short* v = vt + ((pg + 1) & 1) * TILE;
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      const int at = tid + i * 256, e = at >> 3;
+      const int k0 = ((at & 7) ^ ((e & 3) | (e >> 1 & 4))) * 8;
+      u32x4_v x = *reinterpret_cast<u32x4_v*>(v + at * 8);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int k = k0 + 2 * c;
+        x[c] = k > have ? 0u : k + 1 > have ? x[c] & 0xffffu : x[c];
+      }
+      *reinterpret_cast<u32x4_v*>(v + at * 8) = x;
+    }
+    lds_barrier();
+  };
+  // keys of page pg that a row does not see
+  auto hide = [&](int pg) __attribute__((always_inline)) {
+    if (pg < whole) return;
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      const int see = qpos[u] - pg * QSA_PAGE - hi * 8;
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if ((pt >> 1) * 32 + (pt & 1) * 4 + r > see) sc[u][pt][r] = -INFINITY;
+        __builtin_amdgcn_sched_barrier(0);  // few masks at a time
+      }
+    }
+  };
+  auto advance = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      m[u] = top[u];
+      l[u] = l[u] * alpha[u] + psum[u];
+    }
+  };
+  auto rescale = [&]() __attribute__((always_inline)) {
+    if (!__any(moved)) return;         // every factor is 1
+#pragma unroll
+    for (int u = 0; u < QT; ++u)
+#pragma unroll
+      for (int t = 0; t < ET; ++t) acc[u][t] *= alpha[u];
+  };
+
   arrived();
   if (mine > 0) scores(kt);
+  stage(0);
+  int pg = 1;
+  if (mine > 0) {
+    hide(0);
+    guarded();
+    advance();
+    moved = false;                     // there is nothing to rescale yet
+    if (mine > 1) scores(kt + TILE);
 #pragma clang loop unroll(disable)
-  for (int pg = 0; pg <= pages; ++pg) {
-    arrived();                         // K of page pg + 1, V of pg - 1
-    if (pg + 2 < pages) load(kc, kt, pg + 2, kfrom);
-    if (pg < pages) load(vc, vt, pg, vfrom);
-    const int other = ((pg + 1) & 1) * TILE;
-    unsigned short* v = vt + other;
-    const int have = last - (pg - 1) * QSA_PAGE;  // keys 0..have of pg - 1 count
-    if (have < QSA_PAGE - 1) {
-      // slots nobody has written yet may hold anything, NaN too
+    for (; pg < mine; ++pg) {
+      stage(pg);
+      const int other = ((pg + 1) & 1) * TILE;
+      rescale();
+      hide(pg);
+      beside(vt + other);
+      bool bad = false;
 #pragma unroll
-      for (int i = 0; i < L; ++i) {
-        const int at = tid + i * 256, e = at >> 3;
-        const int k0 = ((at & 7) ^ ((e & 3) | (e >> 1 & 4))) * 8;
-        u32x4_v x = *reinterpret_cast<u32x4_v*>(v + at * 8);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int k = k0 + 2 * c;
-          x[c] = k > have ? 0u : k + 1 > have ? x[c] & 0xffffu : x[c];
-        }
-        *reinterpret_cast<u32x4_v*>(v + at * 8) = x;
-      }
-      lds_barrier();
+      for (int u = 0; u < QT; ++u) bad |= !(psum[u] <= 64.f);
+      if (__any(bad)) guarded();       // masked scores are -inf by now
+      advance();
+      if (pg + 1 < mine) scores(kt + other);
     }
-    if (__any(moved)) {
+    stage(pg);
+    rescale();
+    const unsigned short* v = vt + ((pg + 1) & 1) * TILE;
+#pragma unroll
+    for (int c = 0; c < 2 * ET; ++c) {
+      const bf16x8_v a = vals(v, c);
 #pragma unroll
       for (int u = 0; u < QT; ++u)
-#pragma unroll
-        for (int t = 0; t < ET; ++t) acc[u][t] *= alpha[u];
+        acc[u][c % ET] = mfma_bf16(a, pf[u][c / ET], acc[u][c % ET]);
+      if (c & 1) __builtin_amdgcn_sched_barrier(0);
     }
-    moved = false;
-    if (pg < mine) {
-      if (pg >= whole) {
-#pragma unroll
-        for (int u = 0; u < QT; ++u)
-#pragma unroll
-          for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int p = pg * QSA_PAGE + (pt >> 1) * 32 + hi * 8 +
-                            (pt & 1) * 4 + r;
-              if (p > qpos[u]) sc[u][pt][r] = -INFINITY;
-            }
-      }
-      bool bad = pg == 0;
-      if (pg > 0) {
-        beside(v);
-#pragma unroll
-        for (int u = 0; u < QT; ++u) bad |= !(psum[u] <= 64.f);
-      }
-      if (__any(bad)) guarded();       // masked scores are -inf by now
-#pragma unroll
-      for (int u = 0; u < QT; ++u) {
-        m[u] = top[u];
-        l[u] = l[u] * alpha[u] + psum[u];
-      }
-      if (pg + 1 < mine) scores(kt + other);
-    } else if (pg == mine && pg > 0) {
-#pragma unroll
-      for (int c = 0; c < 2 * ET; ++c) {
-        const bf16x8_v a = vals(v, c);
-#pragma unroll
-        for (int u = 0; u < QT; ++u)
-          acc[u][c % ET] = mfma_bf16(a, pf[u][c / ET], acc[u][c % ET]);
-        if (c & 1) __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+    ++pg;
   }
+#pragma clang loop unroll(disable)
+  for (; pg <= pages; ++pg) stage(pg);
 
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
