@@ -685,6 +685,357 @@ qsa_gqa_portions(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same for heads beyond 64.  Pages go straight into LDS, both K and V stand
+// twice, and a turn has one barrier: turn pg loads K of page pg + 2 and V of
+// page pg, and multiplies what came a turn before.  The softmax of page pg runs
+// beside the products of page pg - 1 with its values, a few exponents to each
+// fragment of V; the scores of page pg + 1 follow.  Maxima cross the groups of a
+// column by lane swaps.  A wave's first and last page stand outside of its loop:
+// paths that meet behind the products keep the accumulators twice.
+// us, one page after the other with two barriers / here (16 heads on 8, 4 x 2000
+// tokens unless said; keys x values): 128 x 128 4 x 1700-2048 115 / 104, 1 x
+// 8192 356 / 330, 16 x 1024 134 / 125, 100 + 200 27.6 / 24.9; 64 x 128 94.4 / 91.2;
+// 16 heads on 4: 256 x 64 183 / 128, 256 x 128 205 / 151, 128 x 256 350 / 288,
+// 256 x 256 407 / 344.  Heads of 64 and 32 have little to multiply and are bound
+// by the exponents, with three blocks a CU above (63.5 us for 4 x 2000; 69 here).
+// ---------------------------------------------------------------------------
+template <int KS, int ET, int QT>  // D <= 32*KS, E <= 16*ET
+__global__ void __launch_bounds__(256, ET <= 8 ? 2 : 1)
+qsa_gqa_portions_beside(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
+                 const bf16_t* __restrict__ vc,
+                 const int* __restrict__ block_table, int max_pages,
+                 const float* __restrict__ sink,
+                 const bf16_t* __restrict__ gate, long long gstride,
+                 const int* __restrict__ qb_item,
+                 const int* __restrict__ qb_t0, const int* __restrict__ off,
+                 const int* __restrict__ start, const int* __restrict__ len,
+                 bf16_t* __restrict__ out, long long ostride, int H, int G,
+                 int D, int E, float scale2, float out_scale) {
+#ifdef __HIP_DEVICE_COMPILE__          // loads into LDS: not for the host
+  constexpr int KP = 32 * KS, VP = 16 * ET;       // elements of an LDS row
+  constexpr int KG = KP / 8, VG = VP / 8;         // its pieces of 16 bytes
+  constexpr int PD = 4;                // fragments of K or V in registers
+  constexpr int VN = KS == 8 && ET == 8 ? 1 : 2;  // pages of V in LDS: two
+                                                  // blocks fit a CU
+  __shared__ __attribute__((aligned(16))) bf16_t kt[2 * PG * KP];
+  __shared__ __attribute__((aligned(16))) bf16_t vt[VN * PG * VP];
+  const int RG = H / G;
+  const int g = blockIdx.x % G;
+  const int h = g * RG + blockIdx.x / G % RG;
+  const int qb = blockIdx.x / H;
+  const int it = __builtin_amdgcn_readfirstlane(qb_item[qb]);
+  const int t0 = __builtin_amdgcn_readfirstlane(qb_t0[qb]);
+  const int n = __builtin_amdgcn_readfirstlane(len[it]);
+  const int p0 = __builtin_amdgcn_readfirstlane(start[it]);
+  const int r0 = off[it];
+  const auto table = (const __attribute__((address_space(4))) int*)(
+      block_table + (long long)it * max_pages);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, hi = lane >> 4;
+  const int w0 = t0 + wave * 16 * QT;             // first row of this wave
+  const int last = p0 + min(t0 + 64 * QT, n) - 1; // last visible position
+  // pages of the block, those with keys for this wave, and those whose keys
+  // all its rows see
+  const int pages = (last + PG) / PG;
+  const int mine = w0 >= n ? 0 : min(p0 + w0 + 16 * QT - 1, last) / PG + 1;
+  const int whole = (p0 + w0 + 1) / PG;
+
+  // A load fills 1 KB of LDS in the order of the lanes, so their addresses are
+  // permuted: place j of row r has the row's piece j ^ sw(r), with which a read
+  // of a fragment meets every bank once (two rows twice at KS = 8).  Columns from
+  // D on and rows without a key are outside of the descriptor, which reads as
+  // zero, and so do slots that nobody has written yet.
+  auto ksw = [](int r) {
+    return KS == 1 ? r >> 2 & 3 : KS == 2 ? r >> 1 & 7 : KS == 4 ? r & 15
+                                                                 : r & 7;
+  };
+  auto vsw = [](int r) {
+    return (ET == 2 ? r >> 2 & 1 : ET == 4 ? r >> 1 & 3 : r & 7) * 2;
+  };
+  const int kj = (lane % KG) ^ ksw((wave * 64 + lane) / KG);
+  const int vj = (lane % VG) ^ vsw((wave * 64 + lane) / VG);
+  const unsigned kfrom =
+      kj * 8 < D ? (lane / KG) * D * 2 + kj * 16 : 0x7fffffffu;
+  const unsigned vfrom =
+      vj * 8 < E ? (lane / VG) * E * 2 + vj * 16 : 0x7fffffffu;
+  auto load = [&](const bf16_t* cache, bf16_t* to, int pg, int place,
+                  int width, unsigned from,
+                  auto pieces) __attribute__((always_inline)) {
+    constexpr int PR = decltype(pieces)::value;   // of a row
+    const bf16_t* tile = cache + ((long long)table[pg] * G + g) * PG * width;
+    const int bytes = min(last - pg * PG + 1, PG) * width * 2;
+#pragma unroll
+    for (int i = 0; i < PR / 4; ++i) {
+      const int at = (wave + 4 * i) * (64 / PR) * width * 2;  // bytes before
+      const __amdgpu_buffer_rsrc_t part = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(tile + at / 2), 0, max(bytes - at, 0), 0x00027000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          part, (__attribute__((address_space(3))) void*)(
+                    to + place * PG * PR * 8 + (wave + 4 * i) * 512),
+          16, from, 0, 0, 0);
+    }
+  };
+  using KGt = std::integral_constant<int, KG>;
+  using VGt = std::integral_constant<int, VG>;
+  // all that the waves loaded has arrived, and they have read what they wanted
+  auto arrived = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(7 << 4);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  };
+  load(kc, kt, 0, 0, D, kfrom, KGt{});
+  if (pages > 1) load(kc, kt, 1, 1, D, kfrom, KGt{});
+
+  // maxima are taken before the scale, which therefore has to be positive
+  const bool negative = scale2 < 0.f;
+  scale2 = fmaxf(fabsf(scale2), 1e-30f);
+  const bf16x8_v zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  bf16x8_v qf[QT][KS];
+#pragma unroll
+  for (int u = 0; u < QT; ++u) {
+    const long long qrow = r0 + min(w0 + u * 16 + col, n - 1);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int d = s * 32 + hi * 8;              // D % 8 == 0
+      bf16x8_v v = *reinterpret_cast<const bf16x8_v*>(
+          q + (qrow * H + h) * D + (d < D ? d : 0));
+      if (negative) v ^= (short)0x8000;
+      qf[u][s] = d < D ? v : zero;
+    }
+  }
+  f32x4_v acc[QT][ET], sc[QT][4];
+  bf16x8_v pf[QT][2];
+  float m[QT], l[QT], alpha[QT], psum[QT], top[QT];
+#pragma unroll
+  for (int u = 0; u < QT; ++u) {
+    m[u] = NEG_BIG;
+    l[u] = 0.f;
+    alpha[u] = 1.f;
+#pragma unroll
+    for (int t = 0; t < ET; ++t) acc[u][t] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  }
+  bool moved = false;                  // a maximum, by the last softmax
+
+  // fragment c of a page: keys of tile c % 4, k-step c / 4; values of rows
+  // 32(c / ET).., columns 16(c % ET)..
+  auto keys = [&](const bf16_t* k, int c) __attribute__((always_inline)) {
+    const int r = (c & 3) * 16 + col;
+    return *reinterpret_cast<const bf16x8_v*>(
+        k + r * KP + (((c >> 2) * 4 + hi) ^ ksw(col)) * 8);
+  };
+  const int vr = hi * 4 + (col >> 2);
+  auto vals = [&](const bf16_t* v, int c) __attribute__((always_inline)) {
+    const int s = c / ET, t = c % ET;
+    const bf16_t* at = v + (s * 32 + vr) * VP + ((t * 2) ^ vsw(vr)) * 8 +
+                       (lane & 3) * 4;
+    return __builtin_shufflevector(lds_read_tr(at), lds_read_tr(at + 16 * VP),
+                                   0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  auto scores = [&](const bf16_t* k) __attribute__((always_inline)) {
+    bf16x8_v f[PD];
+#pragma unroll
+    for (int c = 0; c < PD - 1; ++c) f[c] = keys(k, c);
+#pragma unroll
+    for (int c = 0; c < 4 * KS; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (c + PD - 1 < 4 * KS) f[(c + PD - 1) % PD] = keys(k, c + PD - 1);
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+        sc[u][c & 3] = mfma_bf16(
+            f[c % PD], qf[u][c >> 2],
+            c < 4 ? (f32x4_v){0.f, 0.f, 0.f, 0.f} : sc[u][c & 3]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // maximum over a column's four groups of lanes
+  auto over = [&](float x) __attribute__((always_inline)) {
+    const auto a = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  };
+  auto maximum = [&](int u) __attribute__((always_inline)) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[u][i >> 2][i & 3]);
+    top[u] = fmaxf(m[u], over(mx) * scale2);      // page 0 shows every row a
+    moved |= top[u] > m[u];                       // key: it is finite
+    alpha[u] = exp2_hw(m[u] - top[u]);
+    psum[u] = 0.f;
+  };
+  unsigned int pk[QT][8];
+  auto weights = [&](int u, int j) __attribute__((always_inline)) {
+    const float a = exp2_hw(fmaf(sc[u][j >> 1][(j & 1) * 2], scale2, -top[u]));
+    const float b =
+        exp2_hw(fmaf(sc[u][j >> 1][(j & 1) * 2 + 1], scale2, -top[u]));
+    psum[u] += a;
+    psum[u] += b;
+    pk[u][j] = cvt_bf16x2(a, b);
+  };
+  auto packed = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        pf[u][s] = __builtin_bit_cast(
+            bf16x8_v, make_uint4(pk[u][4 * s], pk[u][4 * s + 1],
+                                 pk[u][4 * s + 2], pk[u][4 * s + 3]));
+      m[u] = top[u];
+      l[u] = l[u] * alpha[u] + psum[u];
+    }
+  };
+  // softmax of sc by itself
+  auto first = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      maximum(u);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) weights(u, j);
+    }
+    packed();
+  };
+  auto products = [&](const bf16_t* v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2 * ET; ++c) {
+      const bf16x8_v a = vals(v, c);
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+        acc[u][c % ET] = mfma_bf16(a, pf[u][c / ET], acc[u][c % ET]);
+      if (c & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // softmax of sc beside the products of the weights before it with v
+  auto beside = [&](const bf16_t* v) __attribute__((always_inline)) {
+    constexpr int NC = ET * 2, PAIRS = QT * 8, SPAN = NC - 2;
+    bf16x8_v f[PD];
+#pragma unroll
+    for (int c = 0; c < PD - 1; ++c) f[c] = vals(v, c);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (c + PD - 1 < NC) f[(c + PD - 1) % PD] = vals(v, c + PD - 1);
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+        acc[u][c % ET] = mfma_bf16(f[c % PD], pf[u][c / ET], acc[u][c % ET]);
+      if (c < QT) maximum(c);
+#pragma unroll
+      for (int i = 0; i < PAIRS; ++i)
+        if (c == 2 + i * SPAN / PAIRS) weights(i >> 3, i & 7);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    packed();
+  };
+
+  arrived();
+  if (mine > 0) scores(kt);
+  // a turn's barrier and loads: K of page pg + 1 and V of pg - 1 are there
+  auto stage = [&](int pg) __attribute__((always_inline)) {
+    arrived();
+    if (pg + 2 < pages) load(kc, kt, pg + 2, pg & 1, D, kfrom, KGt{});
+    if (VN == 2 && pg < pages) load(vc, vt, pg, pg & 1, E, vfrom, VGt{});
+  };
+  // after a turn's products with values
+  auto after = [&](int pg) __attribute__((always_inline)) {
+    if constexpr (VN == 1) {
+      lds_barrier();
+      if (pg < pages) load(vc, vt, pg, 0, E, vfrom, VGt{});
+    }
+  };
+  // keys of page pg that a row does not see
+  auto hide = [&](int pg) __attribute__((always_inline)) {
+    if (pg < whole) return;
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      const int see =
+          min(p0 + w0 + u * 16 + col, last) - pg * PG - hi * 4;
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (pt * 16 + r > see) sc[u][pt][r] = -INFINITY;
+        __builtin_amdgcn_sched_barrier(0);  // few masks at a time
+      }
+    }
+  };
+  auto rescale = [&]() __attribute__((always_inline)) {
+    if (__any(moved)) {                // else every factor is 1
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+#pragma unroll
+        for (int t = 0; t < ET; ++t) acc[u][t] *= alpha[u];
+    }
+    moved = false;
+  };
+  stage(0);
+  after(0);
+  int pg = 1;
+  if (mine > 0) {
+    hide(0);
+    first();
+    moved = false;                     // nothing to rescale
+    if (mine > 1) scores(kt + PG * KP);
+#pragma clang loop unroll(disable)
+    for (; pg < mine; ++pg) {
+      stage(pg);
+      rescale();
+      hide(pg);
+      beside(vt + (VN == 2 ? (pg + 1) & 1 : 0) * PG * VP);
+      after(pg);
+      if (pg + 1 < mine) scores(kt + ((pg + 1) & 1) * PG * KP);
+    }
+    stage(pg);
+    rescale();
+    products(vt + (VN == 2 ? (pg + 1) & 1 : 0) * PG * VP);
+    after(pg);
+    ++pg;
+  }
+#pragma clang loop unroll(disable)
+  for (; pg <= pages; ++pg) {
+    stage(pg);
+    after(pg);
+  }
+  const float sk = sink ? sink[h] * LOG2E : NEG_BIG;
+#pragma unroll
+  for (int u = 0; u < QT; ++u) {
+    l[u] += __shfl_xor(l[u], 16, QSA_WAVE);
+    l[u] += __shfl_xor(l[u], 32, QSA_WAVE);
+    const float top = fmaxf(m[u], sk);
+    const float f = m[u] > NEG_BIG ? exp2f(m[u] - top) : 0.f;
+    const float den = l[u] * f + (sink ? exp2f(sk - top) : 0.f);
+    const float inv = den > 0.f ? f / den * out_scale : 0.f;
+    const int i = w0 + u * 16 + col;
+    if (i < n) {
+      const bf16_t* gr = gate + (long long)(r0 + i) * gstride +
+                         (long long)h * E;
+      bf16_t* orow = out + (long long)(r0 + i) * ostride + (long long)h * E;
+#pragma unroll
+      for (int t = 0; t < ET; ++t) {
+        const int e = t * 16 + hi * 4;
+        if (e < E) {                              // E % 8 == 0
+          float o[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = acc[u][t][r] * inv;
+          if (gate) {
+            float gv[4];
+            ldv<bf16_t, 4>(gr + e, gv);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] /= 1.f + __expf(-gv[r]);
+          }
+          stv<bf16_t, 4>(orow + e, o);
+        }
+      }
+    }
+  }
+#endif
+}
+
 extern "C" void qsa_gqa_portions_launch(
     const bf16_t* q, const bf16_t* kc, const bf16_t* vc,
     const int* block_table, int max_pages, const float* sink,
@@ -695,7 +1046,10 @@ extern "C" void qsa_gqa_portions_launch(
   dim3 grid((unsigned)((long long)QB * H));
   const float scale2 = scale * LOG2E;
 #define QSA_GP(K, V, Q)                                                      \
-  hipLaunchKernelGGL((qsa_gqa_portions<K, V, Q>), grid, dim3(256), 0, st, q, \
+  if constexpr (K <= 2 && V <= 4) QSA_GP_AS(qsa_gqa_portions, K, V, Q);      \
+  else QSA_GP_AS(qsa_gqa_portions_beside, K, V, Q)
+#define QSA_GP_AS(NAME, K, V, Q)                                             \
+  hipLaunchKernelGGL((NAME<K, V, Q>), grid, dim3(256), 0, st, q,             \
                      kc, vc, block_table, max_pages, sink, gate, gstride,    \
                      qb_item, qb_t0, off, start, len, out, ostride, H, G, D, \
                      E, scale2, out_scale)
@@ -713,4 +1067,5 @@ extern "C" void qsa_gqa_portions_launch(
   else { QSA_GP(8, 16, 1); }
 #undef QSA_GP_E
 #undef QSA_GP
+#undef QSA_GP_AS
 }

@@ -361,6 +361,46 @@ def test_portions_of_several_sequences():
     close(out, torch.cat(want), BF)
 
 
+@pytest.mark.parametrize("Dm,E", [(k, e) for k in (32, 64, 128, 248)
+                                  for e in (24, 64, 128, 256)])
+def test_portions_that_end_anywhere(Dm, E):
+    """Every width of keys and values, portions of one to five pages whose
+    waves end a page apart; slots that nobody has written hold NaN."""
+    g = gen(Dm + E)
+    H, G, scale = 4, 2, Dm ** -0.5
+    items = [(a + d, n) for a in (0, 64, 128) for d, n in
+             ((0, 1), (0, 64), (33, 32), (50, 31), (63, 2), (0, 129))]
+    lens = [n for _, n in items]
+    pages = [-(-(a + n) // 64) for a, n in items]
+    bt = torch.zeros(len(items), max(pages), dtype=torch.int32)
+    kc = torch.full((sum(pages), G, 64, Dm), float("nan"), dtype=BF)
+    vc = torch.full((sum(pages), G, 64, E), float("nan"), dtype=BF)
+    q, want, at = [], [], 0
+    for i, (a, n) in enumerate(items):
+        bt[i, :pages[i]] = torch.arange(at, at + pages[i])
+        qq, k, v = (rnd(g, a + n, m, d, dtype=BF)
+                    for m, d in ((H, Dm), (G, Dm), (G, E)))
+        for p in range(pages[i]):
+            rows = slice(p * 64, min(p * 64 + 64, a + n))
+            kc[at + p, :, :rows.stop - rows.start] = k[rows].transpose(0, 1)
+            vc[at + p, :, :rows.stop - rows.start] = v[rows].transpose(0, 1)
+        at += pages[i]
+        want.append(O.sink_attention(qq.double(), k.double(), v.double(),
+                                     scale, torch.zeros(H).double())
+                    [a:].reshape(n, -1))
+        q.append(qq[a:].reshape(n, -1))
+    block = D.gqa_portion_rows(Dm, E)
+    item = [i for i, n in enumerate(lens) for _ in range(0, n, block)]
+    t0 = [t for n in lens for t in range(0, n, block)]
+    off = [sum(lens[:i]) for i in range(len(lens))]
+    out = torch.empty(sum(lens), H * E, dtype=BF, device=DEV)
+    D.gqa_portions(torch.cat(q).to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+                   torch.zeros(H, device=DEV), None, i32(*item), i32(*t0),
+                   i32(*off), i32(*[a for a, _ in items]), i32(*lens), out, H,
+                   scale)
+    close(out, torch.cat(want), BF)
+
+
 # ---- state space ------------------------------------------------------------
 
 SSD_SHAPES = [(3, 7, 13, 1), (4, 16, 8, 2), (2, 40, 48, 1), (6, 24, 32, 3),
