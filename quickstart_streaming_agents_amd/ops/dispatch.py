@@ -640,6 +640,12 @@ def topk_cosine_packed(queries: torch.Tensor, docs: torch.Tensor, k: int):
     return torch.stack([scores.contiguous().view(torch.int32), ids])
 
 
+def topk_cosine_host(queries, docs: torch.Tensor, k: int):
+    """topk_cosine_packed of queries in numpy, normalized on the way, as an
+    array; None if one holds a NaN or an infinity (docs on the GPU)."""
+    return ext().topk_cosine_host(queries, docs, k)
+
+
 def window_agg(ts: torch.Tensor, key: torch.Tensor,
                value: torch.Tensor | None, t0: int, win_ms: int, nwin: int,
                nkeys: int):

@@ -6,6 +6,10 @@
 #include <hip/hip_runtime.h>
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+#include <pybind11/numpy.h>
+
+#include <algorithm>
+#include <cmath>
 
 #define CHK(x) TORCH_CHECK(x, #x)
 #define CHK_DEV(t) TORCH_CHECK((t).is_cuda(), #t " must be on the GPU")
@@ -120,6 +124,8 @@ extern "C" void qsa_encoder_attn_launch(
 extern "C" int qsa_topk_block_docs(long long, long long);
 extern "C" void qsa_topk_scan_launch(const float*, const float*, float*, int*,
                                      int, int, int, int, int, hipStream_t);
+extern "C" void qsa_topk_fetch_launch(const float*, float*, long long,
+                                      hipStream_t);
 extern "C" int qsa_topk_groups(int);
 extern "C" void qsa_topk_merge_launch(const float*, const int*, float*, int*,
                                       int, int, int, hipStream_t);
@@ -765,39 +771,100 @@ torch::Tensor encoder_attn(torch::Tensor qkv, torch::Tensor cos_t,
   return out;
 }
 
-// [2, Q, k]: scores, as the bits of floats, and documents; one buffer, so that a
-// caller on the host waits for one copy.
-torch::Tensor topk_cosine_packed(torch::Tensor queries, torch::Tensor docs,
-                                 long k) {
-  CHK_DEV(queries); CHK_CONT(queries); CHK_F32(queries); CHK_F32(docs);
-  CHK_CONT(docs);
+// Scans and merges on the current stream.  The result is [2, Q, k]: scores, as the
+// bits of floats, and documents, in `out` or, without it, in a tensor of its own.
+static torch::Tensor topk_run(const torch::Tensor& queries,
+                              const torch::Tensor& docs, long k, int* out) {
   const int Q = queries.size(0), D = queries.size(1), N = docs.size(0);
   TORCH_CHECK(docs.size(1) == D, "dim mismatch");
   TORCH_CHECK(k >= 1 && k <= 16, "k in [1,16]");
   const int per = qsa_topk_block_docs(Q, N);
   int lists = (N + per - 1) / per;
+  const auto opt = queries.options().dtype(at::kInt);
+  if (Q == 0) return torch::empty({2, 0, k}, opt);
+  torch::Tensor kept, from;            // the candidates, and what they merge into
   auto lists_of = [&](long n) {
-    return torch::empty({2, Q, n * k}, queries.options().dtype(at::kInt));
+    if (n == 1 && out) return out;
+    kept = torch::empty({2, Q, n * k}, opt);
+    return kept.data_ptr<int>();
   };
-  auto from = lists_of(lists);
-  if (Q == 0) return torch::empty({2, 0, k}, from.options());
-  auto scores = [&](torch::Tensor& t) {
-    return reinterpret_cast<float*>(t.data_ptr<int>());
-  };
-  auto ids = [](torch::Tensor& t) { return t.data_ptr<int>() + t.stride(0); };
+  auto scores = [](int* at) { return reinterpret_cast<float*>(at); };
+  auto ids = [&](int* at, long n) { return at + Q * n * k; };
+  int* now = lists_of(lists);
   qsa_topk_scan_launch(queries.data_ptr<float>(), docs.data_ptr<float>(),
-                       scores(from), ids(from), Q, N, D, (int)k, lists,
+                       scores(now), ids(now, lists), Q, N, D, (int)k, lists,
                        cur_stream());
   // a single list is the result (5 rows, k = 5: 17.5 us with the merge)
   while (lists != 1) {
     const int groups = qsa_topk_groups(lists);
-    auto to = lists_of(groups);
-    qsa_topk_merge_launch(scores(from), ids(from), scores(to), ids(to), Q,
-                          lists, (int)k, cur_stream());
-    from = to;
+    from = kept;
+    int* to = lists_of(groups);
+    qsa_topk_merge_launch(scores(now), ids(now, lists), scores(to),
+                          ids(to, groups), Q, lists, (int)k, cur_stream());
+    now = to;
     lists = groups;
   }
-  return from;
+  return kept;
+}
+
+torch::Tensor topk_cosine_packed(torch::Tensor queries, torch::Tensor docs,
+                                 long k) {
+  CHK_DEV(queries); CHK_CONT(queries); CHK_F32(queries); CHK_F32(docs);
+  CHK_CONT(docs);
+  return topk_run(queries, docs, k, nullptr);
+}
+
+// The same of queries on the host, normalized on the way, with the result on the
+// host: array [2, Q, k], or none if a query holds what is not a number or infinite.
+// Queries and result pass through pinned memory that a kernel reads and the last
+// one writes, so that neither waits for a copy (see the caller for times).
+py::object topk_cosine_host(
+    py::array_t<float, py::array::c_style | py::array::forcecast> queries,
+    torch::Tensor docs, long k) {
+  CHK_DEV(docs); CHK_F32(docs); CHK_CONT(docs);
+  TORCH_CHECK(queries.ndim() == 2, "queries must be rows");
+  const long Q = queries.shape(0), D = queries.shape(1), n = Q * D;
+  TORCH_CHECK(docs.dim() == 2 && docs.size(1) == D, "dim mismatch");
+  TORCH_CHECK(k >= 1 && k <= 16, "k in [1,16]");
+  py::array_t<int> result({2L, Q, k});
+  if (Q == 0) return result;
+  const float* q = queries.data();
+  int* res = result.mutable_data();
+  bool numbers = true;
+  {
+    py::gil_scoped_release release;
+    const c10::DeviceGuard guard(docs.device());
+    const long rows = (n + 3) / 4 * 4;
+    auto pinned = torch::empty(
+        {rows + 2 * Q * k},
+        torch::TensorOptions().dtype(at::kFloat).pinned_memory(true));
+    float* host = pinned.data_ptr<float>();
+    for (long i = 0; i < Q && numbers; ++i) {
+      double s[4] = {0, 0, 0, 0};      // four sums: vector operations
+      const float* x = q + i * D;
+      long j = 0;
+      for (; j + 4 <= D; j += 4)
+        for (int e = 0; e < 4; ++e) s[e] += (double)x[j + e] * x[j + e];
+      for (; j < D; ++j) s[0] += (double)x[j] * x[j];
+      const double sum = s[0] + s[1] + s[2] + s[3];
+      numbers = std::isfinite(sum);    // squares of floats stay in range
+      // the norm is a float, infinite beyond what floats hold
+      const float norm = std::max(std::sqrt((float)sum), 1e-12f);
+      for (j = 0; j < D; ++j) host[i * D + j] = x[j] / norm;
+    }
+    if (numbers) {
+      auto rows_on = torch::empty({Q, D}, docs.options());
+      qsa_topk_fetch_launch(host, rows_on.data_ptr<float>(), n, cur_stream());
+      int* out = reinterpret_cast<int*>(host + rows);
+      topk_run(rows_on, docs, k, out);
+      // waits, and reports what the launches left
+      const hipError_t err = hipStreamSynchronize(cur_stream());
+      TORCH_CHECK(err == hipSuccess, "top-k search: ", hipGetErrorString(err));
+      std::copy(out, out + 2 * Q * k, res);
+    }
+  }
+  if (!numbers) return py::none();
+  return result;
 }
 
 std::vector<torch::Tensor> topk_cosine(torch::Tensor queries,
@@ -913,6 +980,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("K"), py::arg("res"), py::arg("w"), py::arg("far") = true);
   m.def("embed_rows", &embed_rows,
         "a step's first rows and their sums of squares");
+  m.def("topk_cosine_host", &topk_cosine_host,
+        "exact cosine top-k of host queries, normalized; result on the host");
   m.def("topk_cosine_packed", &topk_cosine_packed,
         "the same, scores and documents in one buffer");
   m.def("topk_cosine", &topk_cosine, "exact cosine top-k over the HBM index");

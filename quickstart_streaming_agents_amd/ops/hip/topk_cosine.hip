@@ -378,6 +378,26 @@ qsa_topk_merge(const float* __restrict__ cand_scores,  // [Q, all, k]
   }
 }
 
+// Queries from the host's pinned memory, a read of some 10 to 100 KB over the bus
+// that the scan's blocks would each repeat.
+__global__ void __launch_bounds__(256)
+qsa_topk_fetch(const float* __restrict__ host, float* __restrict__ queries,
+               long long n) {
+  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i + 4 <= n) {
+    *reinterpret_cast<float4*>(queries + i) =
+        *reinterpret_cast<const float4*>(host + i);
+  } else {
+    for (long long j = i; j < n; ++j) queries[j] = host[j];
+  }
+}
+
+extern "C" void qsa_topk_fetch_launch(const float* host, float* queries,
+                                      long long n, hipStream_t stream) {
+  hipLaunchKernelGGL(qsa_topk_fetch, dim3((unsigned)((n + 1023) / 1024)),
+                     dim3(256), 0, stream, host, queries, n);
+}
+
 // A block: 16 documents times the first digit, 16 queries times the second.  Up
 // to 16 queries: 16 documents for small indexes, 64 as soon as that gives every
 // CU two blocks.  More share a read of the index, 32 queries beside 48 documents

@@ -82,6 +82,14 @@ def _scan_wins(queries: int, rows: int, k: int) -> bool:
         queries * rows <= 1_500_000 or queries <= 32 and rows <= 262_144
 
 
+# Queries that pass through pinned memory (topk_cosine_host, ops/hip/ops.cpp), in
+# numbers: 1 MB.  us of a search with queries normalized in numpy and copied, and
+# the result copied back / so: 8 of 1536 against 100k rows 164 / 131, 1000 rows 65 /
+# 39, one against 5 rows 40 / 24.  More are copied at the bus's rate anyway, and
+# pinned memory is kept for later calls.
+_HOST_QUERIES = 1 << 18
+
+
 class VectorIndex:
     """Exact cosine top-k over L2-normalized rows.
 
@@ -179,25 +187,33 @@ class VectorIndex:
         if not len(self):
             return [[] for _ in range(len(queries))]
         q = np.asarray(queries, dtype=np.float32)
-        norms = np.linalg.norm(q, axis=1, keepdims=True)
-        q = q / np.maximum(norms, 1e-12)
         docs = self.to_torch(device)
-        qt = torch.from_numpy(q).to(device=device, dtype=torch.float32)
         k_eff = min(k, len(self))
-        if not _scan_wins(len(q), len(self), k_eff) or not (
-                np.isfinite(norms).all() or np.isfinite(q).all()):
+        scan = _scan_wins(len(q), len(self), k_eff)
+        both = None
+        if scan and docs.is_cuda and q.size <= _HOST_QUERIES:
+            # none if a query is not a number, or infinite
+            both = D.topk_cosine_host(q, docs, k_eff)
+        if both is None:
+            norms = np.linalg.norm(q, axis=1, keepdims=True)
+            q = q / np.maximum(norms, 1e-12)
+            qt = torch.from_numpy(q).to(device=device, dtype=torch.float32)
+            scan = scan and (np.isfinite(norms).all() or
+                             np.isfinite(q).all())
+            if scan:
+                # the tiled cosine/top-k HIP kernel, one copy of its results
+                both = D.topk_cosine_packed(qt.contiguous(), docs,
+                                            k_eff).cpu().numpy()
+        if both is not None:
+            scores = both[0].view(np.float32).tolist()
+            idx = both[1].tolist()
+        else:
             # a matmul over the HBM matrix and a sort of the scores; the
             # kernel has no answer for a query that is not a number
             scores_all = qt @ docs.T
             scores, idx = torch.topk(scores_all, k_eff, dim=1)
             scores = scores.cpu().numpy().tolist()
             idx = idx.cpu().numpy().tolist()
-        else:
-            # the tiled cosine/top-k HIP kernel, and one copy of its results
-            both = D.topk_cosine_packed(qt.contiguous(), docs,
-                                        k_eff).cpu().numpy()
-            scores = both[0].view(np.float32).tolist()
-            idx = both[1].tolist()
         # -1: fewer documents than k have a score
         return [[SearchHit(self.ids[i], self.chunks[i], s, self.metadata[i])
                  for i, s in zip(ids, row) if i >= 0]

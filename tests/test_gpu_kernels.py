@@ -239,6 +239,46 @@ def test_topk_cosine_blocks(ext, Q, N, D, k):
     assert torch.equal(both[1], i)
 
 
+@pytest.mark.parametrize("N,Q,D,k", [
+    (1, 1, 1536, 1), (5, 3, 7, 5), (64, 1, 1536, 3), (65, 17, 129, 16),
+    (3000, 2, 1534, 3), (40_000, 8, 64, 4), (0, 2, 8, 1), (9, 0, 8, 2)])
+def test_topk_of_host_queries(ext, N, Q, D, k):
+    """Queries in numpy of any order and length, among them zero, one whose
+    norm floats do not hold and, where it does not fit, a NaN or infinity."""
+    g = torch.Generator().manual_seed(N + Q)
+    docs = torch.nn.functional.normalize(
+        torch.randn(N, D, generator=g), dim=1).to(dev())
+    q = torch.randn(Q, D, generator=g).numpy() * 3
+    if Q > 1:
+        q[1] = 0
+    if Q > 2:
+        q[2] = 3e38
+    with np.errstate(over="ignore"):
+        norm = np.linalg.norm(q, axis=1, keepdims=True)
+    unit = (q / np.maximum(norm, 1e-12)).astype(np.float32)
+    want = ext.topk_cosine_packed(torch.from_numpy(unit).to(dev()), docs,
+                                  k).cpu().numpy()
+    for x in (q, np.asfortranarray(q), np.repeat(q, 2, 0)[::2], q.tolist()
+              if Q else q):
+        got = ext.topk_cosine_host(x, docs, k)
+        assert got.shape == (2, Q, k)
+        # the norm's last bit, which numpy rounds on the way
+        np.testing.assert_allclose(got[0].view(np.float32),
+                                   want[0].view(np.float32), rtol=0,
+                                   atol=4e-7)
+        if N <= 64:
+            assert (got[1] == want[1]).all()
+    for bad in (np.nan, np.inf, -np.inf):
+        if Q:
+            x = q.copy()
+            x[-1, D // 2] = bad
+            assert ext.topk_cosine_host(x, docs, k) is None
+    with pytest.raises(RuntimeError):
+        ext.topk_cosine_host(np.zeros((1, D + 1)), docs, k)
+    with pytest.raises(RuntimeError):
+        ext.topk_cosine_host(q, docs, 17)
+
+
 def test_window_agg(ext):
     torch.manual_seed(6)
     n, nkeys, nwin = 50000, 7, 288
