@@ -42,16 +42,116 @@ __device__ __forceinline__ float2 bf16x2_to_f32x2(unsigned int p) {
 }
 
 // ---- wave reductions (64-lane) --------------------------------------------
-__device__ __forceinline__ float wave_reduce_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, QSA_WAVE);
-  return v;
+// Reductions over lanes by exchanges between registers: __shfl_xor goes through
+// LDS, some 100 cycles a step that a chain of six waits for.  Every lane ends up
+// with the value, in the order of a butterfly of steps 32, 16, 8, 4, 2, 1: behind
+// a step the lanes that the later ones tell apart are all that differ, so turning
+// a row of 16 is as good as crossing lanes (sums of two do not mind their order).
+template <int CTRL>
+__device__ __forceinline__ float qsa_dpp(float v) {
+  const int x = __float_as_int(v);
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, false));
+}
+#define QSA_ROW_TURN 0x120             // + lanes
+#define QSA_ROW_MIRROR 0x140           // lane i of a row from 15 - i
+#define QSA_HALF_MIRROR 0x141          // ... of half a row from 7 - i
+#define QSA_QUAD_1 0xb1                // lane i from i ^ 1
+#define QSA_QUAD_2 0x4e                // ... i ^ 2
+
+// f(v of lane i, v of lane i ^ 16), and 32
+template <class F>
+__device__ __forceinline__ float qsa_cross16(float v, F f) {
+  const auto r = __builtin_amdgcn_permlane16_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <class F>
+__device__ __forceinline__ float qsa_cross32(float v, F f) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+struct QsaAdd {
+  __device__ float operator()(float a, float b) const { return a + b; }
+};
+struct QsaMax {
+  __device__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+
+// over the four lanes that share a lane's place in its row of 16
+template <class F>
+__device__ __forceinline__ float qsa_over_rows(float v, F f) {
+  return qsa_cross32(qsa_cross16(v, f), f);
+}
+__device__ __forceinline__ float rows_sum(float v) {
+  return qsa_over_rows(v, QsaAdd());
+}
+__device__ __forceinline__ float rows_max(float v) {
+  return qsa_over_rows(v, QsaMax());
+}
+
+// over a row of 16, in steps 1, 2, 4, 8
+__device__ __forceinline__ float row16_sum(float v) {
+  v += qsa_dpp<QSA_QUAD_1>(v);
+  v += qsa_dpp<QSA_QUAD_2>(v);
+  v += qsa_dpp<QSA_HALF_MIRROR>(v);
+  return v + qsa_dpp<QSA_ROW_MIRROR>(v);
+}
+
+template <class F>
+__device__ __forceinline__ float qsa_over_wave(float v, F f) {
+  v = qsa_cross16(qsa_cross32(v, f), f);
+  v = f(v, qsa_dpp<QSA_ROW_TURN + 8>(v));
+  v = f(v, qsa_dpp<QSA_ROW_TURN + 4>(v));
+  v = f(v, qsa_dpp<QSA_ROW_TURN + 2>(v));
+  return f(v, qsa_dpp<QSA_ROW_TURN + 1>(v));
+}
+__device__ __forceinline__ float wave_reduce_sum(float v) {
+  return qsa_over_wave(v, QsaAdd());
+}
 __device__ __forceinline__ float wave_reduce_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, QSA_WAVE));
-  return v;
+  return qsa_over_wave(v, QsaMax());
+}
+
+// Exchanges of two words at once, for the better of two (value, place) pairs:
+// better(other value, other place, value, place).
+template <int CTRL, class B>
+__device__ __forceinline__ void qsa_dpp_best(float& v, int& i, B better) {
+  const float ov = qsa_dpp<CTRL>(v);
+  const int oi = __builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false);
+  if (better(ov, oi, v, i)) {
+    v = ov;
+    i = oi;
+  }
+}
+// the best of a row of 16, in all its lanes
+template <class B>
+__device__ __forceinline__ void row16_best(float& v, int& i, B better) {
+  qsa_dpp_best<QSA_QUAD_1>(v, i, better);
+  qsa_dpp_best<QSA_QUAD_2>(v, i, better);
+  qsa_dpp_best<QSA_HALF_MIRROR>(v, i, better);
+  qsa_dpp_best<QSA_ROW_MIRROR>(v, i, better);
+}
+template <class B>
+__device__ __forceinline__ void wave_best(float& v, int& i, B better) {
+  row16_best(v, i, better);
+  auto pick = [&](auto a, auto b) {
+    const float x = __uint_as_float(a[0]), y = __uint_as_float(a[1]);
+    const int p = (int)b[0], q = (int)b[1];
+    const bool second = better(y, q, x, p);
+    v = second ? y : x;
+    i = second ? q : p;
+  };
+  pick(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v),
+                                        false, false),
+       __builtin_amdgcn_permlane16_swap((unsigned)i, (unsigned)i, false,
+                                        false));
+  pick(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v),
+                                        false, false),
+       __builtin_amdgcn_permlane32_swap((unsigned)i, (unsigned)i, false,
+                                        false));
 }
 
 // Block reduction via LDS (callers pass scratch of >= nwaves floats).

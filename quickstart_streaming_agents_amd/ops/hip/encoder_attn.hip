@@ -151,8 +151,7 @@ qsa_encoder_attn(const bf16_t* __restrict__ qkv,      // [T, 3, H, D]
           mx = fmaxf(mx, sc[pt][r]);
         }
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
+      mx = rows_max(mx);
       top = fmaxf(m, mx * scale2);
       alpha = __builtin_amdgcn_exp2f(m - top);
       psum = 0.f;
@@ -192,8 +191,7 @@ qsa_encoder_attn(const bf16_t* __restrict__ qkv,      // [T, 3, H, D]
                            pf, acc[t]);
     }
   }
-  l += __shfl_xor(l, 16, QSA_WAVE);
-  l += __shfl_xor(l, 32, QSA_WAVE);
+  l = rows_sum(l);
   const int t = w0 + col;
   if (t >= n) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;

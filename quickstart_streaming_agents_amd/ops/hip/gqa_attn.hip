@@ -239,8 +239,7 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
           s4[pt][r] = p < n ? s4[pt][r] * scale2 : NEG_BIG;
           mx = fmaxf(mx, s4[pt][r]);
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
+      mx = rows_max(mx);
       const float mn = fmaxf(m, mx);
       const float alpha = exp2_hw(m - mn);        // a step sees a key: mn is
                                                   // finite, masked terms 0
@@ -267,8 +266,7 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
         acc[t] = mfma_bf16(lds_frag_tr(vt, VP, 0, 16, t * 16, lane), pf,
                            acc[t]);
     }
-    l += __shfl_xor(l, 16, QSA_WAVE);
-    l += __shfl_xor(l, 32, QSA_WAVE);
+    l = rows_sum(l);
   }
   if constexpr (MERGE) {
     // [16 heads][E] of every wave where its values were
@@ -605,8 +603,7 @@ qsa_gqa_portions(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                 s4[u][pt][r] = -INFINITY;
             mx = fmaxf(mx, s4[u][pt][r]);
           }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
+        mx = rows_max(mx);
         const float mn = fmaxf(m[u], mx * scale2);
         moved |= mn > m[u];
         alpha[u] = exp2_hw(m[u] - mn);            // page 0 shows every row a
@@ -654,8 +651,7 @@ qsa_gqa_portions(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
   const float sk = sink ? sink[h] * LOG2E : NEG_BIG;
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
-    l[u] += __shfl_xor(l[u], 16, QSA_WAVE);
-    l[u] += __shfl_xor(l[u], 32, QSA_WAVE);
+    l[u] = rows_sum(l[u]);
     const float top = fmaxf(m[u], sk);
     const float f = m[u] > NEG_BIG ? exp2f(m[u] - top) : 0.f;
     const float den = l[u] * f + (sink ? exp2f(sk - top) : 0.f);
@@ -852,20 +848,11 @@ qsa_gqa_portions_beside(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  // maximum over a column's four groups of lanes
-  auto over = [&](float x) __attribute__((always_inline)) {
-    const auto a = __builtin_amdgcn_permlane16_swap(
-        __float_as_uint(x), __float_as_uint(x), false, false);
-    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-  };
   auto maximum = [&](int u) __attribute__((always_inline)) {
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[u][i >> 2][i & 3]);
-    top[u] = fmaxf(m[u], over(mx) * scale2);      // page 0 shows every row a
+    top[u] = fmaxf(m[u], rows_max(mx) * scale2);      // page 0 shows every row a
     moved |= top[u] > m[u];                       // key: it is finite
     alpha[u] = exp2_hw(m[u] - top[u]);
     psum[u] = 0.f;
@@ -1004,8 +991,7 @@ qsa_gqa_portions_beside(const bf16_t* __restrict__ q, const bf16_t* __restrict__
   const float sk = sink ? sink[h] * LOG2E : NEG_BIG;
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
-    l[u] += __shfl_xor(l[u], 16, QSA_WAVE);
-    l[u] += __shfl_xor(l[u], 32, QSA_WAVE);
+    l[u] = rows_sum(l[u]);
     const float top = fmaxf(m[u], sk);
     const float f = m[u] > NEG_BIG ? exp2f(m[u] - top) : 0.f;
     const float den = l[u] * f + (sink ? exp2f(sk - top) : 0.f);

@@ -340,8 +340,7 @@ qsa_latent_rows_mfma(const bf16_t* __restrict__ qa,
         s4[r] = (p >= lo && p < n) ? s4[r] * scale2 : NEG_BIG;
         mx = fmaxf(mx, s4[r]);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
+      mx = rows_max(mx);
       if (hi == 0) smax[wave][col] = mx;
       lds_barrier();
       float mn = m;
@@ -374,8 +373,7 @@ qsa_latent_rows_mfma(const bf16_t* __restrict__ qa,
     }
   }
   // l: sum over the hi groups of each wave, then over the waves
-  l += __shfl_xor(l, 16, QSA_WAVE);
-  l += __shfl_xor(l, 32, QSA_WAVE);
+  l = rows_sum(l);
   lds_barrier();
   if (hi == 0) smax[wave][col] = l;
   lds_barrier();
@@ -595,8 +593,7 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
           if constexpr (guard.value) s4[pt][r] = fmaxf(s4[pt][r], -INFINITY);
           mx = fmaxf(mx, s4[pt][r]);
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, QSA_WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, QSA_WAVE));
+      mx = rows_max(mx);
       top = fmaxf(m, mx * scale2);                // NEG_BIG: no key so far
       alpha = __builtin_amdgcn_exp2f(m - top);
       psum = 0.f;
@@ -640,8 +637,7 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
         acc[t] = mfma_bf16(a, pf[s], acc[t]);
       }
   }
-  l += __shfl_xor(l, 16, QSA_WAVE);
-  l += __shfl_xor(l, 32, QSA_WAVE);
+  l = rows_sum(l);
   const float sk = bf16_to_f32(sink[h]) * LOG2E;
   const float top = fmaxf(m, sk);
   const float f = m > NEG_BIG ? exp2f(m - top) : 0.f;

@@ -269,8 +269,7 @@ __device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p) {
         }
       }
       // column (per-head) max across the 4 hi groups
-      pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 16, QSA_WAVE));
-      pagemax = fmaxf(pagemax, __shfl_xor(pagemax, 32, QSA_WAVE));
+      pagemax = rows_max(pagemax);
       const float m_new = fmaxf(m, pagemax);
       float alpha = __expf(m - m_new);
       if (m <= -3.0e38f) alpha = 0.f;
@@ -298,8 +297,7 @@ __device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p) {
         ppk[pt * 2] = cvt_bf16x2(pr[0], pr[1]);
         ppk[pt * 2 + 1] = cvt_bf16x2(pr[2], pr[3]);
       }
-      psum += __shfl_xor(psum, 16, QSA_WAVE);
-      psum += __shfl_xor(psum, 32, QSA_WAVE);
+      psum = rows_sum(psum);
       lsum = lsum * alpha + psum;
 
       // the values are there; the next page's keys, behind them, need not be
@@ -983,20 +981,11 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  // maximum over a column's four groups of lanes
-  auto over = [&](float x) __attribute__((always_inline)) {
-    const auto a = __builtin_amdgcn_permlane16_swap(
-        __float_as_uint(x), __float_as_uint(x), false, false);
-    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-  };
   auto maximum = [&](int u) __attribute__((always_inline)) {
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[u][i >> 2][i & 3]);
-    top[u] = fmaxf(m[u], over(mx) * scale2);
+    top[u] = fmaxf(m[u], rows_max(mx) * scale2);
     moved |= top[u] > m[u];
     alpha[u] = __builtin_amdgcn_exp2f(m[u] - top[u]);
     psum[u] = 0.f;
@@ -1156,8 +1145,7 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
 
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
-    l[u] += __shfl_xor(l[u], 16, QSA_WAVE);
-    l[u] += __shfl_xor(l[u], 32, QSA_WAVE);
+    l[u] = rows_sum(l[u]);
     const float inv = l[u] > 0.f ? 1.f / l[u] : 0.f;
     const int v = w0 + u * 16 + col;
     if (v >= vend) continue;

@@ -703,8 +703,7 @@ qsa_retention_out(const bf16_t* __restrict__ x, long long xstride,
         for (int r = 0; r < 4; ++r)
           ss = fmaf(acc[u][rt][r], acc[u][rt][r], ss);
       }
-    ss += __shfl_xor(ss, 16, QSA_WAVE);
-    ss += __shfl_xor(ss, 32, QSA_WAVE);
+    ss = rows_sum(ss);
     if (hi == 0) red[wave][rt * 16 + col] = ss;
   }
   lds_barrier();

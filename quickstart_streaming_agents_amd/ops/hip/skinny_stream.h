@@ -255,9 +255,7 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
         p.next[place(p.N)] = cvt_bf16(bf16_to_f32(b) *
                                       bf16_to_f32(nw[i]));
       }
-      float q = v * v;
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) q += __shfl_xor(q, o, 16);
+      const float q = row16_sum(v * v);
       const int parts = p.N >> 4;
       if (live && col == 0)
         p.ss_out[row * ((parts + 3) & ~3) + (ncol >> 4)] = q;

@@ -65,15 +65,7 @@ __device__ __forceinline__ void qsa_topk_candidates(
           bs = sc[t];
           bi = doc0 + t * 16 + sub;
         }
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) {
-        const float os = __shfl_xor(bs, o, 16);
-        const int oi = __shfl_xor(bi, o, 16);
-        if (qsa_better(os, oi, bs, bi)) {
-          bs = os;
-          bi = oi;
-        }
-      }
+      row16_best(bs, bi, qsa_better);
 #pragma unroll
       for (int t = 0; t < T; ++t)
         if (doc0 + t * 16 + sub == bi) sc[t] = -INFINITY;
@@ -337,15 +329,7 @@ qsa_topk_merge(const float* __restrict__ cand_scores,  // [Q, all, k]
         bs = hs[j];
         bi = hd[j];
       }
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const float os = __shfl_xor(bs, o, QSA_WAVE);
-      const int oi = __shfl_xor(bi, o, QSA_WAVE);
-      if (qsa_better(os, oi, bs, bi)) {
-        bs = os;
-        bi = oi;
-      }
-    }
+    wave_best(bs, bi, qsa_better);
     __syncthreads();                   // the round before has been read
     if ((tid & 63) == 0) {
       ws[wave] = bs;
