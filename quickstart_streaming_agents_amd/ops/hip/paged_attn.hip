@@ -9,8 +9,8 @@
 //   - All R GQA query heads of a kv head compute TOGETHER on the matrix
 //     cores: scores via mfma_f32_16x16x32_bf16 with A = K-tile
 //     [16 pos x 32 k] and B = Q [32 k x 16 heads] (heads pad to 16), PV
-//     via A = P [16 heads x 32 pos] (packed bf16, redistributed with 8
-//     cross-lane shuffles) and B = V^T [32 pos x 16 dims].  Every KV byte is
+//     via A = P [16 heads x 32 pos] (packed bf16, redistributed by lane
+//     swaps) and B = V^T [32 pos x 16 dims].  Every KV byte is
 //     read exactly once.
 //   - K cache layout [page, kvh, D/8, 64, 8] (d-major x8): a page's fragments
 //     are loads of four 256-byte pieces, and the next page's are under way while
@@ -32,7 +32,7 @@
 // write-through were the same).
 //
 // The online softmax runs per head-column in registers: column max/sum
-// reduce with two shfl_xor hops (the 4 hi-lane groups of a column).
+// reduce by two lane swaps (the 4 hi-lane groups of a column).
 #include <algorithm>
 #include <type_traits>
 
@@ -314,29 +314,25 @@ __device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
       }
       // ---- PV: two 32-pos halves ---------------------------------------
-      // A-frag needs lane (head=col, hi) to hold P[head][pos = hi*8 + e]:
-      // packed pairs come from source lanes (same col) with hi' = (2*hi)&3
-      // and (2*hi+1)&3, tile = half*2 + (hi>>1).  __shfl evaluates its value
-      // in EACH lane and a register index has to be a constant: shuffle both
-      // candidate tiles' registers and select by hi.
+      // A-frag needs lane (head=col, hi) to hold P[head][pos = hi*8 + e]: packed
+      // pairs of the groups 2hi & 3 and the next of tile half*2 + (hi>>1).  Of
+      // two tiles' groups (0 1 2 3) and (4 5 6 7) a swap of halves makes (0 1 4
+      // 5) and (2 3 6 7), and one of rows (0 2 4 6) and (1 3 5 7), which is that
+      // (16 exchanges through LDS: a step of one row 524 us, 521 so; of 24 rows of
+      // 800-2000 keys 937 and 931).
       // B-frag: lane holds V^T[pos = half*32 + hi*8 + e][d = dt*16+col]
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        const int src_a = col + (((2 * hi) & 3) << 4);
-        const int src_b = col + (((2 * hi + 1) & 3) << 4);
-        const int tA = half * 2;           // tile for hi 0,1
-        const int tB = half * 2 + 1;       // tile for hi 2,3
-        const unsigned int a0A = __shfl(ppk[tA * 2], src_a, QSA_WAVE);
-        const unsigned int a1A = __shfl(ppk[tA * 2 + 1], src_a, QSA_WAVE);
-        const unsigned int b0A = __shfl(ppk[tA * 2], src_b, QSA_WAVE);
-        const unsigned int b1A = __shfl(ppk[tA * 2 + 1], src_b, QSA_WAVE);
-        const unsigned int a0B = __shfl(ppk[tB * 2], src_a, QSA_WAVE);
-        const unsigned int a1B = __shfl(ppk[tB * 2 + 1], src_a, QSA_WAVE);
-        const unsigned int b0B = __shfl(ppk[tB * 2], src_b, QSA_WAVE);
-        const unsigned int b1B = __shfl(ppk[tB * 2 + 1], src_b, QSA_WAVE);
-        const bool lo = hi < 2;
-        const u32x4_v pu = {lo ? a0A : a0B, lo ? a1A : a1B, lo ? b0A : b0B,
-                            lo ? b1A : b1B};
+        u32x4_v pu;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          const auto x = __builtin_amdgcn_permlane32_swap(
+              ppk[half * 4 + w], ppk[half * 4 + 2 + w], false, false);
+          const auto y =
+              __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+          pu[w] = y[0];
+          pu[2 + w] = y[1];
+        }
         const bf16x8_a pa = __builtin_bit_cast(bf16x8_a, pu);
         const unsigned short* vr =
             vl + col * 64 + ((half * 4 + hi) ^ (col & 7)) * 8;
