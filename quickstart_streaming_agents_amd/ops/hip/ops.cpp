@@ -133,6 +133,7 @@ extern "C" void qsa_window_agg_launch(const long long*, const int*,
                                       const float*, int*, float*, long long,
                                       long long, int, int, long long, int*,
                                       hipStream_t);
+extern "C" void qsa_window_clear_launch(int*, long long, hipStream_t);
 extern "C" long long qsa_window_workspace(long long, long long, long long,
                                           long long);
 void register_avro(pybind11::module_&);  // avro_codec.cpp
@@ -880,8 +881,9 @@ std::vector<torch::Tensor> window_agg(torch::Tensor ts, torch::Tensor key,
   CHK_DEV(ts); CHK_CONT(ts); CHK_I32(key);
   TORCH_CHECK(ts.scalar_type() == at::kLong, "ts must be i64");
   const long long n = ts.numel();
-  // one buffer: the two tables are cleared by one fill
-  auto cells = torch::zeros({2, nkeys, nwin}, key.options());
+  // one buffer: the two tables are cleared by one launch
+  auto cells = torch::empty({2, nkeys, nwin}, key.options());
+  qsa_window_clear_launch(cells.data_ptr<int>(), cells.numel(), cur_stream());
   auto counts = cells[0];
   auto sums = cells[1].view(at::kFloat);
   const float* vptr = nullptr;
