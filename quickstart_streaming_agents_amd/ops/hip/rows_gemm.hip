@@ -297,29 +297,37 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
 #undef QSA_RG
 }
 
-// BM, BN, waves, places of the ring; a block's own time and that of a stage, us.
+// BM, BN, waves, places of the ring; a block's own time and that of a stage, us, and
+// the same where few rows meet weights from memory (qsa_rows_gemm_plan).
 // Of the last tile two blocks share a CU: one's start and end lie beside the
 // other's products, which short K gains by (us, the best of the others and so:
 // 16,000 x 3072 x 384 with the activation 52.7, 49.3; 24,000 79.2, 71.7; 8263 x
 // 2048 x 128 15.7, 13.0; 30,000 38.2, 30.7; 4400 x 16384 x 2048 263, 253).  Its
 // figures are those of a pair, set where 42 such shapes part.
 #define QSA_TILES(X) \
-  X(64, 32, 2, 2, 6, 0.67f, 0.200f)   X(64, 64, 2, 2, 4, 0.71f, 0.208f) \
-  X(64, 128, 2, 4, 6, 1.86f, 0.353f)  X(128, 64, 4, 2, 6, 1.92f, 0.334f) \
-  X(128, 128, 2, 4, 4, 2.38f, 0.497f) X(192, 64, 4, 2, 4, 1.94f, 0.431f) \
-  X(192, 128, 4, 2, 4, 2.98f, 0.644f) X(256, 128, 4, 2, 3, 3.41f, 0.822f) \
-  X(128, 256, 2, 4, 3, 3.32f, 0.843f) X(192, 192, 2, 4, 3, 4.03f, 0.800f) \
-  X(256, 192, 4, 2, 2, 3.57f, 1.189f) X(192, 256, 2, 4, 2, 3.19f, 1.227f) \
-  X(256, 256, 2, 4, 2, 4.06f, 1.482f) X(192, 128, 4, 2, 2, 0.77f, 1.27f)
+  X(64, 32, 2, 2, 6, 0.67f, 0.200f, 1.04f, 0.178f) \
+  X(64, 64, 2, 2, 4, 0.71f, 0.208f, 1.40f, 0.235f) \
+  X(64, 128, 2, 4, 6, 1.86f, 0.353f, 3.17f, 0.377f) \
+  X(128, 64, 4, 2, 6, 1.92f, 0.334f, 3.39f, 0.309f) \
+  X(128, 128, 2, 4, 4, 2.38f, 0.497f, 4.44f, 0.438f) \
+  X(192, 64, 4, 2, 4, 1.94f, 0.431f, 3.05f, 0.456f) \
+  X(192, 128, 4, 2, 4, 2.98f, 0.644f, 5.12f, 0.592f) \
+  X(256, 128, 4, 2, 3, 3.41f, 0.822f, 4.68f, 0.688f) \
+  X(128, 256, 2, 4, 3, 3.32f, 0.843f, 6.16f, 0.712f) \
+  X(192, 192, 2, 4, 3, 4.03f, 0.800f, 6.82f, 0.674f) \
+  X(256, 192, 4, 2, 2, 3.57f, 1.189f, 3.45f, 1.160f) \
+  X(192, 256, 2, 4, 2, 3.19f, 1.227f, 5.16f, 1.223f) \
+  X(256, 256, 2, 4, 2, 4.06f, 1.482f, 3.51f, 1.350f) \
+  X(192, 128, 4, 2, 2, 0.77f, 1.27f, 2.31f, 0.956f)
 
 struct RowsTile {
   int bm, bn, wn;
   bool pair;                           // of large blocks on a CU
-  float own, stage;
+  float own, stage, own_few, stage_few;
 };
 static const RowsTile rows_tiles[] = {
-#define X(BM, BN, WM, WN, ST, OWN, STAGE)                              \
-  {BM, BN, WN, rows_pair(BM, BN, WM * WN, ST), OWN, STAGE},
+#define X(BM, BN, WM, WN, ST, OWN, STAGE, OWN2, STAGE2)                \
+  {BM, BN, WN, rows_pair(BM, BN, WM * WN, ST), OWN, STAGE, OWN2, STAGE2},
     QSA_TILES(X)
 #undef X
 };
@@ -337,14 +345,25 @@ static const RowsTile rows_tiles[] = {
 // for 15).  Over these the choice is 2.5 % from the best, 5.1 before, and 18 of
 // them, 37 before, are more than 5 % behind the library, the larger by up to 14 %
 // (450 to 512 x 12288, 64 x 40960 x 12288).
+// Few rows are another matter: their weights come from memory, each block's rows of A
+// once more from L2, and what a CU gets through it binds (192 x 6144 x 4096, us: 192 x
+// 64 in two shares 28.2, for which the figures above say 22.7, 128 x 64 whole 24.2;
+// 192 x 4096 x 14336: 192 x 64 in four 42.9, 192 x 128 in eight 37.0).  For 81 to
+// 192 rows and from 2M weights on the tiles' second figures are fitted to 1722 times of
+// 84 shapes (weights in turn from 700 MB): off by 6 %, and the choice 1.0 % from the
+// best, 3.3 % with the figures above; a decoder's step of
+// width 4096, 8 layers, 192 rows 2166 -> 2081 us, of 150 1644 -> 1614, of 100 1354 -> 1339,
+// but of 66 1146 -> 1152.
 // cheap: the reader of the product adds the shares; us_out: what the choice should
 // take, or null.
 extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
                                   int* shares, float* us_out) {
   const int all = K >> 6;
-  const float mem = 2e-6f / 5.14f * ((float)N * K + (float)M * K +
-                                     (float)M * N);
-  const float sum = (cheap ? 0.5f : 3.25f), each = 1.28e-6f * (float)M * N;
+  const bool few = M > 80 && M <= 192 && (long long)N * K >= 2 << 20;
+  const float mem = 2e-6f / (few ? 7.06f : 5.14f) *
+                    ((float)N * K + (float)M * K + (float)M * N);
+  const float sum = few ? (cheap ? 1.22f : 3.79f) : (cheap ? 0.5f : 3.25f);
+  const float each = (few ? 1.40e-6f : 1.28e-6f) * (float)M * N;
   float best = 1e30f;
   int tile = 0;
   *shares = 1;
@@ -355,16 +374,21 @@ extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
         (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     if (t.pair && blocks <= 256) continue;        // alone on their CUs
     const int fill = blocks < 256 ? (int)(256 / blocks) : 1;
-    for (int S = act || all < 8 ? 1 : fill; S >= 1; S = S > 1 ? S / 2 : 0) {
+    int most = act || all < 8 ? 1 : fill;
+    if (few)                           // 1, 2, 4 or 8
+      for (most = std::min(most, 8); most & (most - 1); --most) {}
+    for (int S = most; S >= 1; S = S > 1 ? S / 2 : 0) {
       if (S > all / 4 && S > 1) continue;
       const int slots = t.pair ? 512 : 256;
       const long long turns = (blocks * S + slots - 1) / slots;
-      float stage = t.stage;
-      if (turns == 1 && t.bn * t.bm <= 4096) stage *= i ? 1.48f : 0.93f;
-      float run = (float)turns * (t.own + stage * ((all + S - 1) / S));
+      float stage = few ? t.stage_few : t.stage;
+      if (turns == 1 && t.bn * t.bm <= 4096)
+        stage *= few ? (i ? 1.26f : 1.39f) : (i ? 1.48f : 0.93f);
+      float run = (float)turns * ((few ? t.own_few : t.own) +
+                                  stage * ((all + S - 1) / S));
       if (t.pair && turns == 1) run += 1.5f;      // neither end beside another
       const float r2 = run * run, m2 = mem * mem;
-      const float us = sqrtf(sqrtf(r2 * r2 + m2 * m2)) +
+      const float us = (few ? sqrtf(r2 + m2) : sqrtf(sqrtf(r2 * r2 + m2 * m2))) +
                        (S > 1 ? sum + each * S : 0.f);
       if (us < best) { best = us; tile = i; *shares = S; }
     }
@@ -381,7 +405,7 @@ extern "C" void qsa_rows_gemm_launch(const bf16_t* A, const bf16_t* W,
                                      int act, hipStream_t st) {
   const RowsArgs p{A, W, C, part, M, N, K, S, 0, 0, (unsigned int)lda};
   int i = 0;
-#define X(BM, BN, WM, WN, ST, OWN, STAGE) \
+#define X(BM, BN, WM, WN, ST, OWN, STAGE, OWN2, STAGE2) \
   if (tile == i++) rows_go<BM, BN, WM, WN, ST>(p, act, st);
   QSA_TILES(X)
 #undef X
