@@ -333,10 +333,9 @@ class LlamaModel:
         projections norm their input, gate and add to the residual, so a
         layer is four of them and the attention."""
         B, eps, far = tokens.shape[0], self.cfg.norm_eps, self.weights_far
-        parts = self.cfg.hidden // 16        # of a row's sum of squares
         norms = [L["attn_norm"] for L in self.layers] + [self.final_norm]
         res, x, ss = D.embed_rows(self.embed, tokens, norms[0])
-        n = 1
+        n = 1                                # parts of a row's sum of squares
         for li, L in enumerate(self.layers):
             qkv = D.norm_linear_fp8(x, ss, n, B, eps, L["wqkv_f8"],
                                     *L["wqkv"].shape, far=far)
@@ -346,12 +345,13 @@ class LlamaModel:
             x, ss = D.linear_residual_fp8(
                 attn if attn.dim() == 4 else attn.view(B, -1), L["wo_f8"],
                 *L["wo"].shape, res, L["mlp_norm"], far)
-            n = parts
+            n = D.residual_parts_fp8(B, *L["wo"].shape)
             act = D.norm_linear_fp8(x, ss, n, B, eps, L["wgu_f8"],
                                     *L["wgu"].shape, glu=True, far=far)
             x, ss = D.linear_residual_fp8(act, L["wdown_f8"],
                                           *L["wdown"].shape, res,
                                           norms[li + 1], far)
+            n = D.residual_parts_fp8(B, *L["wdown"].shape)
         return D.norm_linear_fp8(x, ss, n, B, eps, self.lm_head_f8,
                                  *self.lm_head.shape, far=far)
 

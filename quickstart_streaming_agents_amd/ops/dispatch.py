@@ -338,9 +338,15 @@ def norm_linear_fp8(x: torch.Tensor, ss: torch.Tensor, parts: int, rows: int,
 def linear_residual_fp8(x: torch.Tensor, packed: tuple, n: int, k: int,
                         res: torch.Tensor, w: torch.Tensor, far: bool = True):
     """res <- res + step rows x through a packed fp8 weight, in place; returns
-    the step rows of the norm with weight w that follows, and ss."""
+    the step rows of the norm with weight w that follows, and ss, in
+    residual_parts_fp8 parts."""
     return ext().skinny_gemm_fp8_residual(x, packed[0], packed[1], n, k, res,
                                           w, far)
+
+
+def residual_parts_fp8(rows: int, n: int, k: int) -> int:
+    """The parts of ss that linear_residual_fp8 returns for these sizes."""
+    return ext().skinny_gemm_fp8_parts(rows, n, k)
 
 
 # ---- mixer decoders (qsa_lm_hip) ------------------------------------------

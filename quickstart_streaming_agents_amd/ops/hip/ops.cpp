@@ -92,6 +92,7 @@ extern "C" void qsa_skinny_gemm_fp8_launch(
     unsigned short*, unsigned short*, int, int, long long, long long, int,
     const unsigned short*, const float*, int, float, int, float*, int,
     hipStream_t);
+extern "C" int qsa_skinny_fp8_half(int, int, long long);
 extern "C" int qsa_skinny_gemm_fp8_probe_launch(
     const unsigned short*, const unsigned char*, const float*,
     unsigned short*, int, int, long long, long long, int, int, int,
@@ -659,11 +660,16 @@ torch::Tensor skinny_gemm_fp8_norm(torch::Tensor a, torch::Tensor ss,
   return out;
 }
 
+// parts that skinny_gemm_fp8_residual leaves of a row's sum of squares
+long skinny_gemm_fp8_parts(long M, long N, long K) {
+  return N / (qsa_skinny_fp8_half((int)M, (int)N, K) ? 8 : 16);
+}
+
 std::vector<torch::Tensor> skinny_gemm_fp8_residual(
     torch::Tensor a, torch::Tensor qf, torch::Tensor scale, long N, long K,
     torch::Tensor res, torch::Tensor w, bool far) {
   // res [M, N] <- res + the product; returns the rows of the norm with weight
-  // w that follows (before 1/rms) and the sums of squares in N/16 parts
+  // w that follows (before 1/rms) and the sums of squares in their parts
   CHK_DEV(res); CHK_BF16(res); CHK_CONT(res);
   TORCH_CHECK(res.dim() == 2 && res.size(1) == N, "residual [M, N]");
   const long M = res.size(0);
@@ -672,7 +678,7 @@ std::vector<torch::Tensor> skinny_gemm_fp8_residual(
   CHK_DEV(w); CHK_BF16(w); CHK_CONT(w);
   TORCH_CHECK(w.numel() == N && N % 32 == 0, "norm weight [N], N % 32 == 0");
   auto next = step_rows(M, N, a.options());
-  auto ss = torch::empty({32, (N / 16 + 3) & ~3L},
+  auto ss = torch::empty({32, (skinny_gemm_fp8_parts(M, N, K) + 3) & ~3L},
                          a.options().dtype(at::kFloat));
   qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
                              scale.data_ptr<float>(), u16m(res), u16m(next),
@@ -976,6 +982,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("a"), py::arg("ss"), py::arg("parts"), py::arg("M"),
         py::arg("eps"), py::arg("qf"), py::arg("scale"), py::arg("N"),
         py::arg("K"), py::arg("glu"), py::arg("far") = true);
+  m.def("skinny_gemm_fp8_parts", &skinny_gemm_fp8_parts,
+        "parts of a row's sum of squares behind a residual");
   m.def("skinny_gemm_fp8_residual", &skinny_gemm_fp8_residual,
         "fp8-weight decode GEMM added to the residual stream",
         py::arg("a"), py::arg("qf"), py::arg("scale"), py::arg("N"),

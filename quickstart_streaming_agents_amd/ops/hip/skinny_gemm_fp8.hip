@@ -34,6 +34,12 @@ qsa_skinny_gemm_fp8(SkinnyArgs p) {
   skinny_stream<WAVES, TILES, MT, true, PACK, NORM, GLU, RES, FAR>(p);
 }
 
+template <int WAVES, bool PACK, bool FAR>
+__global__ void __launch_bounds__(WAVES * 64)
+qsa_skinny_gemm_fp8_half(SkinnyArgs p) {
+  skinny_stream<WAVES, 1, 1, true, PACK, false, false, true, FAR, true>(p);
+}
+
 template <int WAVES, int TILES, bool NORM, bool GLU, bool RES>
 static void fp8_go(const SkinnyArgs& p, int pack, hipStream_t st) {
   const dim3 grid(p.N / (16 * TILES)), block(WAVES * 64);
@@ -83,6 +89,35 @@ static void fp8_any(const SkinnyArgs& p, int pack, hipStream_t st) {
   }
 }
 
+// Whether a product with a residual is done in half tiles: up to 2048 columns are
+// 128 tiles or fewer, and from 3072 numbers of K on a block's part of the stream is
+// more than it has in flight at once (us at 1 / 4 / 8 rows, weights from memory, whole
+// tiles -> half ones: 2048 x 8192 8.0 / 8.6 / 9.7 -> 5.6 / 6.3 / 6.2; 2048 x 4096 5.1 /
+// 5.3 / 6.0 -> 4.2 / 4.6 / 4.6; 1024 x 3072 4.6 / 5.0 / 5.3 -> 3.7 / 4.2 / 4.1; 512 x
+// 14336 10.7 / 12.0 / 14.0 -> 7.5 / 9.4 / 8.6; but 2048 x 2048 3.8 / 4.1 / 4.3 -> 3.7 /
+// 4.2 / 4.1, 2560 x 8192 9.1 / 8.9 / 10.0 -> 8.2 / 9.8 / 9.6).  16 layers of width 2048,
+// a step of one row 517 -> 495 us, of eight 570 -> 536; 8 layers, 4 rows 308 -> 293.
+extern "C" int qsa_skinny_fp8_half(int M, int N, long long K) {
+  return M <= 8 && N <= 2048 && K >= 3072 && K % 128 == 0;
+}
+
+static void fp8_half(const SkinnyArgs& p, int pack, hipStream_t st) {
+  const dim3 grid(p.N / 8);
+#define QSA_HALF_AS(WAVES, PACK, FAR)                                         \
+  hipLaunchKernelGGL((qsa_skinny_gemm_fp8_half<WAVES, PACK, FAR>), grid,      \
+                     dim3(WAVES * 64), 0, st, p)
+#define QSA_HALF(WAVES, PACK)                                                 \
+  if (p.far) QSA_HALF_AS(WAVES, PACK, true);                                  \
+  else QSA_HALF_AS(WAVES, PACK, false)
+  if (p.K < 6144) {                    // a wave has 6 or more steps
+    if (pack) { QSA_HALF(4, true); } else { QSA_HALF(4, false); }
+  } else {
+    if (pack) { QSA_HALF(8, true); } else { QSA_HALF(8, false); }
+  }
+#undef QSA_HALF
+#undef QSA_HALF_AS
+}
+
 extern "C" void qsa_skinny_gemm_fp8_launch(
     const unsigned short* A, const unsigned char* Qf, const float* scale,
     unsigned short* C, unsigned short* next, int M, int N, long long K,
@@ -91,7 +126,8 @@ extern "C" void qsa_skinny_gemm_fp8_launch(
   const SkinnyArgs p{A, reinterpret_cast<const u32x4_v*>(Qf), scale, C, next,
                      norm_w, ss_in, ss_out, M, N, parts, K, lda, eps,
                      far != 0};
-  if (ss_out) fp8_any<false, false, true>(p, pack, stream);
+  if (ss_out && qsa_skinny_fp8_half(M, N, K)) fp8_half(p, pack, stream);
+  else if (ss_out) fp8_any<false, false, true>(p, pack, stream);
   else if (ss_in && glu) fp8_any<true, true, false>(p, pack, stream);
   else if (ss_in) fp8_any<true, false, false>(p, pack, stream);
   else fp8_any<false, false, false>(p, pack, stream);

@@ -33,6 +33,11 @@
 //   RES   the result is added to the residual stream in place; the next norm's
 //         operand (new row * norm_w, packed if A is) goes to `next`, the
 //         sums of squares of the new rows to ss_out, one part per tile.
+//   HALF  a block has half a tile, for few columns, whose tiles would leave CUs idle
+//         and the others a stream each that one memory latency does not cover.  Lanes
+//         of columns 8 to 15 take the same eight columns further on in K, and rows 8
+//         to 15 of A are its rows 0 to 7 there; the result is the sum of the two
+//         diagonal quarters, so up to 8 rows.  One part of a sum per half.
 // (Multiplying by w on the way in instead cost 20 us of 25 at 28672 x 4096:
 // every block redoes it, and its loads take the place of the stream's.)
 #pragma once
@@ -78,8 +83,9 @@ __device__ __forceinline__ long long packed_at(int row, int k, int mt) {
 }
 
 template <int WAVES, int TILES, int MT, bool FP8, bool PACK, bool NORM,
-          bool GLU, bool RES, bool FAR>
+          bool GLU, bool RES, bool FAR, bool HALF = false>
 __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
+  static_assert(!HALF || (FP8 && RES && TILES == 1 && MT == 1), "half a tile");
   constexpr int WL = FP8 ? 1 : 2;      // 16 B loads of a tile per step
   constexpr int PER = TILES * WL * 4 + MT * 8;
   constexpr int U = PER <= 12 ? 4 : PER <= 24 ? 2 : 1;
@@ -90,7 +96,10 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   // would otherwise run with no lane enabled and still add up
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
-  const int steps = (int)(p.K >> 6);   // K % 64 == 0
+  // K % 64 == 0, HALF: % 128 and steps of either half of K
+  const int steps = (int)(p.K >> (HALF ? 7 : 6));
+  // a lane's column of its tile, as results are stored
+  const int tcol = HALF ? ((int)blockIdx.x & 1) * 8 + (col & 7) : col;
 
   // row factors: the parts' loads go ahead of the stream, a row per wave
   constexpr int NR = NORM ? MT * 16 / WAVES : 1;
@@ -108,7 +117,7 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   auto tile_of = [&](int t) {
     return GLU ? (int)blockIdx.x * (TILES / 2) + t / 2 +
                      (t & 1) * (p.N >> 5)
-               : (int)blockIdx.x * TILES + t;
+               : HALF ? (int)blockIdx.x >> 1 : (int)blockIdx.x * TILES + t;
   };
   // what the results need besides the sums is fetched ahead of the stream: at
   // the end each of these would be a memory latency of its own (2048 x 2048
@@ -124,9 +133,9 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
     if constexpr (FP8)
 #pragma unroll
       for (int e = 0; e < (GLU ? 2 : 1); ++e)
-        sc[i][e] = p.scale[tile_of(GLU ? 2 * j + e : j) * 16 + col];
+        sc[i][e] = p.scale[tile_of(GLU ? 2 * j + e : j) * 16 + tcol];
     if constexpr (RES) {
-      const int row = m * 16 + hi * 4 + r, c = tile_of(j) * 16 + col;
+      const int row = m * 16 + hi * 4 + r, c = tile_of(j) * 16 + tcol;
       old[i] = p.C[(long long)(row < p.M ? row : 0) * p.N + c];
       nw[i] = p.norm_w[c];
     }
@@ -134,13 +143,20 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   const u32x4_v* wp[TILES];
 #pragma unroll
   for (int t = 0; t < TILES; ++t)
-    wp[t] = p.W + (long long)tile_of(t) * steps * (64 * WL) + col * 4 + hi;
+    wp[t] = p.W + (HALF ? ((long long)tile_of(t) * 2 + (col >> 3)) * steps * 64
+                        : (long long)tile_of(t) * steps * (64 * WL)) +
+            tcol * 4 + hi;
   const bf16_t* ap[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m)
-    ap[m] = PACK ? p.A + m * 512 + lane * 8
-                 : p.A + (long long)min(m * 16 + col, p.M - 1) * p.lda +
-                       hi * 8;
+    if constexpr (HALF)
+      ap[m] = p.A + (long long)(col >> 3) * steps * (PACK ? 1024 : 64) +
+              (PACK ? ((col & 7) + hi * 16) * 8
+                    : min(col & 7, p.M - 1) * p.lda + hi * 8);
+    else
+      ap[m] = PACK ? p.A + m * 512 + lane * 8
+                   : p.A + (long long)min(m * 16 + col, p.M - 1) * p.lda +
+                         hi * 8;
 
   struct Group {
     u32x4_v w[U][TILES][WL];
@@ -234,12 +250,15 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
       float v = 0.f;
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) v += red[w][(t * MT + m) * 4 + r][lane];
+      if constexpr (HALF)              // row + 8, column + 8
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) v += red[w][r][(lane + 40) & 63];
       if constexpr (FP8) v *= sc[i][e];
       return v;
     };
     const float inv = NORM ? inv_s[row] : 1.f;
-    const int ncol = tile_of(GLU ? 2 * j : j) * 16 + col;
-    const bool live = row < p.M;
+    const int ncol = tile_of(GLU ? 2 * j : j) * 16 + tcol;
+    const bool live = row < p.M && (!HALF || (row < 8 && col < 8));
     auto place = [&](int width) {
       return PACK ? packed_at(row, ncol, MT) : (long long)row * width + ncol;
     };
@@ -255,10 +274,11 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
         p.next[place(p.N)] = cvt_bf16(bf16_to_f32(b) *
                                       bf16_to_f32(nw[i]));
       }
-      const float q = row16_sum(v * v);
-      const int parts = p.N >> 4;
+      const float q = row16_sum(HALF && col >= 8 ? 0.f : v * v);
+      constexpr int PART = HALF ? 3 : 4;           // log2 of its columns
+      const int parts = p.N >> PART;
       if (live && col == 0)
-        p.ss_out[row * ((parts + 3) & ~3) + (ncol >> 4)] = q;
+        p.ss_out[row * ((parts + 3) & ~3) + (ncol >> PART)] = q;
     } else {
       const float v = total(j, 0) * inv;
       if (live) p.C[(long long)row * p.N + ncol] = cvt_bf16(v);

@@ -770,6 +770,44 @@ def test_skinny_fp8_forms(M, N, K):
             < tol * want.square().sum(1)).all()
 
 
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("N,K", [(32, 3072), (2048, 3328), (224, 5888),
+                                 (992, 6144), (2048, 8192), (2080, 8192)])
+def test_skinny_fp8_half_tiles(M, N, K):
+    """The residual form of few columns in half tiles, and on either side of
+    where they are taken; rows that do not exist hold NaN, and the norm that
+    follows reads the parts."""
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    torch.manual_seed(M + N + K)
+    w = torch.randn(N, K, device=dev(), dtype=torch.bfloat16) * K ** -0.5
+    packed = D.pack_weight_fp8(w)
+    W = D.unpack_weight_fp8(*packed, N, K).double()
+    x = torch.randn(M, K, device=dev(), dtype=torch.bfloat16)
+    res = torch.randn(M, N, device=dev(), dtype=torch.bfloat16)
+    nw = (1 + 0.2 * torch.randn(N, device=dev())).bfloat16()
+    want = res.double() + x.double() @ W.T
+    nxt, ss = D.linear_residual_fp8(_step_rows(x), packed, N, K, res, nw)
+    # operands are exact, sums f32 (K 2^-24), the result rounded (2^-9)
+    assert ((res.double() - want).abs() <= 2 ** -8 * want.abs()
+            + K * 2 ** -24 * (x.double().abs() @ W.abs().T)).all()
+    assert torch.equal(_from_step_rows(nxt, M),
+                       (res.float() * nw.float()).bfloat16())
+    parts = D.residual_parts_fp8(M, N, K)
+    assert parts == N // (8 if M <= 8 and N <= 2048 else 16)
+    assert ss.shape == (32, -(-parts // 4) * 4)
+    sums = ss[:M, :parts].double().sum(1)
+    assert ((sums - want.square().sum(1)).abs()
+            < 2 ** -8 * want.square().sum(1)).all()
+    if N % 256 == 0:
+        v = torch.randn(64, N, device=dev(), dtype=torch.bfloat16) * N ** -0.5
+        p2 = D.pack_weight_fp8(v)
+        got = D.norm_linear_fp8(nxt, ss, parts, M, 1e-5, p2, 64, N).double()
+        r = res.double()
+        h = (r * nw.double()) @ D.unpack_weight_fp8(*p2, 64, N).double().T \
+            * torch.rsqrt(r.square().mean(1, keepdim=True) + 1e-5)
+        assert (got - h).norm() < 2 ** -7 * h.norm()
+
+
 @pytest.mark.parametrize("B,QH,KVH,D,longest", [
     (1, 32, 8, 64, 700), (1, 32, 8, 128, 60), (4, 32, 8, 128, 1100),
     (5, 32, 8, 128, 900), (17, 16, 1, 64, 2000), (32, 28, 4, 128, 300),
