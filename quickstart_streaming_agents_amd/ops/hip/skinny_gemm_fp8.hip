@@ -63,7 +63,13 @@ static void fp8_go(const SkinnyArgs& p, int pack, hipStream_t st) {
 // two tiles of columns as soon as 192 blocks are left (half the A reads per
 // weight).  Four tiles for a vocabulary, and from 16384 columns on where A is
 // two row tiles and costs more than the weights (28672 x 4096, 32 rows: 37 us
-// with two tiles, 29 with four).
+// with two tiles, 29 with four).  With 9 to 16 rows, of which A
+// still is twice the weights, from 28672 on and K beyond 2048 (16 rows 24.5 us with two
+// tiles, 23.2 with four; 32768 x 3072 20.1 / 19.2, but 22016 x 4096 19.5 / 21.4, 32768 x
+// 2048 13.8 / 14.2).  12288 to 16384 columns are one block of four tiles for a CU, and
+// with eight waves (us at 16 / 24 rows, before -> so: 12288 x 2048 7.9 / 9.9 -> 7.3 / 7.8;
+// 16384 x 2048 8.6 / 9.9 -> 8.2 / 8.7; 16384 x 3072 11.5 / 12.8 -> 11.0 / 11.5; of 24 rows
+// 12288 x 1024 6.1 -> 5.4, 16384 x 4096 16.1 -> 15.6; but of 16 14.1 -> 16.8).
 // us at 1 / 16 rows, one tile per block and row-major A before -> here (packed
 // from 5 rows on, norm or residual included): 6144 x 4096 13.1 / 14.2 -> 7.5 /
 // 8.6; 4096 x 4096 8.1 / 9.4 -> 6.2 / 7.2; 28672 x 4096 32 / 36 -> 24.6 / 27.9
@@ -71,15 +77,24 @@ static void fp8_go(const SkinnyArgs& p, int pack, hipStream_t st) {
 // -> 48.6 / 52.2 (5.4 TB/s).
 template <bool NORM, bool GLU, bool RES>
 static void fp8_any(const SkinnyArgs& p, int pack, hipStream_t st) {
+  // four tiles, of one block a CU or of more than three for two
+  const bool once = p.M > 8 && p.N >= 12288 && p.N <= 16384 &&
+                    (p.M > 16 ? p.K >= 1024 : p.K >= 2048 && p.K <= 3072);
+  const int four = p.M > 16 ? 16384 : p.M > 8 && p.K > 2048 ? 28672 : 65536;
   if constexpr (GLU) {
-    if (p.M > 16 && p.N >= 16384 && p.N % 128 == 0)
+    if (once && p.N % 128 == 0)
+      fp8_go<8, 4, NORM, GLU, RES>(p, pack, st);
+    else if (p.M > 8 && p.N >= four && p.N % 128 == 0)
       fp8_go<4, 4, NORM, GLU, RES>(p, pack, st);
     else if (p.K <= 2048) fp8_go<4, 2, NORM, GLU, RES>(p, pack, st);
     else fp8_go<8, 2, NORM, GLU, RES>(p, pack, st);
   } else {
-    if constexpr (!RES)
-      if (p.N >= (p.M > 16 ? 16384 : 65536) && p.N % 64 == 0)
+    if constexpr (!RES) {
+      if (once && p.N % 64 == 0)
+        return fp8_go<8, 4, NORM, GLU, RES>(p, pack, st);
+      if (p.N >= four && p.N % 64 == 0)
         return fp8_go<4, 4, NORM, GLU, RES>(p, pack, st);
+    }
     if (p.N >= 6144 && p.N % 32 == 0)
       fp8_go<8, 2, NORM, GLU, RES>(p, pack, st);
     else if (p.K <= 2048)

@@ -770,6 +770,30 @@ def test_skinny_fp8_forms(M, N, K):
             < tol * want.square().sum(1)).all()
 
 
+@pytest.mark.parametrize("M", [8, 9, 16, 17])
+@pytest.mark.parametrize("N,K", [(12288, 1024), (12352, 2048), (16384, 2304),
+                                 (28672, 2304), (28736, 2304)])
+def test_skinny_fp8_wide_blocks(M, N, K):
+    """Plain and gated forms about where a block takes four tiles of columns."""
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    torch.manual_seed(M + N + K)
+    w = torch.randn(N, K, device=dev(), dtype=torch.bfloat16) * K ** -0.5
+    packed = D.pack_weight_fp8(w)
+    x = torch.randn(M, K, device=dev(), dtype=torch.bfloat16)
+    ss = torch.full((32, 4), float("nan"), device=dev())
+    ss[:M, 0] = x.float().square().sum(1)
+    h = x.double() @ D.unpack_weight_fp8(*packed, N, K).double().T \
+        * torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-5)
+    got = D.norm_linear_fp8(_step_rows(x), ss, 1, M, 1e-5, packed, N, K)
+    assert (got.double() - h).norm() < 2 ** -8 * h.norm()   # rounded to bf16
+    act = D.norm_linear_fp8(_step_rows(x), ss, 1, M, 1e-5, packed, N, K,
+                            glu=True)
+    g, u = h.chunk(2, 1)
+    want = torch.nn.functional.silu(g) * u
+    assert (_from_step_rows(act, M).double() - want).norm() \
+        < 2 ** -8 * want.norm()
+
+
 @pytest.mark.parametrize("M", [1, 3, 4, 5, 8, 9])
 @pytest.mark.parametrize("N,K", [(32, 3072), (2048, 3328), (224, 5888),
                                  (992, 6144), (2048, 8192), (2080, 8192)])
