@@ -48,14 +48,18 @@ __device__ __forceinline__ int qsa_window_by(long long ts, long long t0,
 }
 
 // A launch of its own: up to 100k events are bound by the host, for whom a tensor's
-// fill is dearer (an aggregation 10.2 us with it, 9.2 so; 2M events 23.1 both).
+// fill is dearer (an aggregation 10.2 us with it, 9.2 so; 2M events 23.1 both). The
+// grid is bounded, since a launch holds fewer than 2^32 threads: tables of more than
+// 268 MB take several turns of it.
+#define QSA_CLEAR_BLOCKS 65536
 __global__ void __launch_bounds__(256)
 qsa_window_clear(int* __restrict__ cells, long long n) {
-  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i + 4 <= n)
-    *reinterpret_cast<int4*>(cells + i) = make_int4(0, 0, 0, 0);
-  else
-    for (long long j = i; j < n; ++j) cells[j] = 0;
+  const long long step = (long long)gridDim.x * 1024;
+  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += step)
+    if (i + 4 <= n)
+      *reinterpret_cast<int4*>(cells + i) = make_int4(0, 0, 0, 0);
+    else
+      for (long long j = i; j < n; ++j) cells[j] = 0;
 }
 
 // An event at a time, straight to the output.
@@ -598,9 +602,13 @@ extern "C" long long qsa_window_workspace(long long n, long long nkeys,
 
 extern "C" void qsa_window_clear_launch(int* cells, long long n,
                                         hipStream_t stream) {
-  if (n > 0)
-    hipLaunchKernelGGL(qsa_window_clear, dim3((unsigned)((n + 1023) / 1024)),
+  if (n > 0) {
+    const long long blocks = (n + 1023) / 1024;
+    hipLaunchKernelGGL(qsa_window_clear,
+                       dim3((unsigned)(blocks < QSA_CLEAR_BLOCKS ? blocks
+                                                                 : QSA_CLEAR_BLOCKS)),
                        dim3(256), 0, stream, cells, n);
+  }
 }
 
 extern "C" void qsa_window_agg_launch(const long long* ts, const int* key,

@@ -419,6 +419,24 @@ def test_window_agg_edges(ext, n, nkeys, nwin, shuffle):
     assert torch.equal(c.cpu(), counts) and not s.any()
 
 
+@pytest.mark.parametrize("nkeys,nwin", [(1, 1), (511, 1), (1, 513),
+                                        ((1 << 21) + 1, 16),
+                                        ((1 << 21) + 1, 17)])
+def test_window_agg_clears_its_tables(ext, nkeys, nwin):
+    """Around the 1024 cells of a block and the 67,108,864 of a full grid: nothing of
+    what the memory held before is left, to the last cell."""
+    dirty = torch.ones(2, nkeys, nwin, dtype=torch.int32, device=dev())
+    del dirty                                   # its block is the next one given
+    ts = torch.tensor([0, 10 * nwin - 1], device=dev())
+    key = torch.tensor([0, nkeys - 1], dtype=torch.int32, device=dev())
+    val = torch.tensor([2., 3.], device=dev())
+    counts, sums = ext.window_agg(ts, key, val, 0, 10, nwin, nkeys)
+    assert int(counts.sum()) == 2 and float(sums.double().sum()) == 5
+    assert int(torch.count_nonzero(counts)) <= 2
+    assert int(torch.count_nonzero(sums)) <= 2
+    assert int(counts[-1, -1]) >= 1 and float(sums[-1, -1]) >= 3
+
+
 @pytest.mark.parametrize("n,nkeys,nwin", [
     (131_072, 40, 200), (131_073, 40, 200),    # chunks of 256, of 1024
     (140_000, 2049, 3), (262_144, 40, 154),
