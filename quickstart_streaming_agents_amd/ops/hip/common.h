@@ -11,6 +11,8 @@
 // in a step whose reads do not fit there together only drives out the rest.
 #define QSA_LLC (256ll << 20)
 #define QSA_NT 2
+// keys and values of one layer, in bytes, beyond which a step reads them so
+#define QSA_FAR_PAGES (32ll << 20)
 
 // ---- bf16 <-> f32 ----------------------------------------------------------
 __device__ __forceinline__ float bf16_to_f32(unsigned short h) {
@@ -113,6 +115,25 @@ __device__ __forceinline__ float wave_reduce_sum(float v) {
 }
 __device__ __forceinline__ float wave_reduce_max(float v) {
   return qsa_over_wave(v, QsaMax());
+}
+
+// Sum over n numbers of what `of` makes of them, in every lane (all lanes on): what a
+// launch has before it, where only the device knows.  Up to 256 numbers are loads
+// side by side, beside those that a kernel begins with.
+template <class F>
+__device__ __forceinline__ float wave_total(const int* at, int n, F of) {
+  constexpr int U = 4;
+  float v = 0.f;
+  for (int i = threadIdx.x & 63; i < n; i += U * QSA_WAVE) {
+    int x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = at[min(i + u * QSA_WAVE, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u * QSA_WAVE < n) v += of(x[u]);
+  }
+  return __int_as_float(
+      __builtin_amdgcn_readfirstlane(__float_as_int(wave_reduce_sum(v))));
 }
 
 // Exchanges of two words at once, for the better of two (value, place) pairs:

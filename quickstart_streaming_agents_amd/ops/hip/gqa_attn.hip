@@ -128,18 +128,16 @@ struct GqaFinish {
 
 // FAR: past the last-level cache.
 template <int KS, int ET, bool MERGE, bool FAR>  // D <= 32*KS, E <= 16*ET
-__global__ void __launch_bounds__(256, KS <= 4 && ET <= 8 ? 2 : 1)
-qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
-                  const bf16_t* __restrict__ vc,
-                  const int* __restrict__ block_table, int max_pages,
-                  const int* __restrict__ row_item,
-                  const int* __restrict__ row_len,
-                  float* __restrict__ part_o, float* __restrict__ part_ml,
-                  int H, int G, int D, int E, float scale2, int NS,
-                  int units, GqaFinish fin) {
+__device__ __forceinline__ void
+gqa_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
+         const bf16_t* __restrict__ vc, const int* __restrict__ block_table,
+         int max_pages, const int* __restrict__ row_item,
+         const int* __restrict__ row_len, float* __restrict__ part_o,
+         float* __restrict__ part_ml, int H, int G, int D, int E, float scale2,
+         int NS, int units, const GqaFinish& fin,
+         bf16_t (*vt_all)[32 * (16 * ET + 16)], float (*ml)[16][2]) {
   constexpr int VP = 16 * ET + 16;
   constexpr int VG = 2 * ET;                      // 16 B groups per V row
-  __shared__ __attribute__((aligned(16))) bf16_t vt_all[4][32 * VP];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int unit = blockIdx.x * 4 + wave;
   if (unit >= units) return;                      // MERGE: never
@@ -270,7 +268,6 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
   }
   if constexpr (MERGE) {
     // [16 heads][E] of every wave where its values were
-    __shared__ float ml[4][16][2];
     float* mine = reinterpret_cast<float*>(vt);
     __builtin_amdgcn_wave_barrier();
     if (hi == 0) {
@@ -332,6 +329,31 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
         *reinterpret_cast<f32x4_v*>(part_o + o * E + e) = acc[t];
     }
   }
+}
+
+// BOTH: past the cache if all rows together have more than far_keys.
+template <int KS, int ET, bool MERGE, bool BOTH>
+__global__ void __launch_bounds__(256, KS <= 4 && ET <= 8 ? 2 : 1)
+qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
+                  const bf16_t* __restrict__ vc,
+                  const int* __restrict__ block_table, int max_pages,
+                  const int* __restrict__ row_item,
+                  const int* __restrict__ row_len,
+                  float* __restrict__ part_o, float* __restrict__ part_ml,
+                  int H, int G, int D, int E, float scale2, int NS,
+                  int units, GqaFinish fin, int rows, float far_keys) {
+  __shared__ __attribute__((aligned(16))) bf16_t vt[4][32 * (16 * ET + 16)];
+  __shared__ float ml[4][16][2];                  // MERGE
+  if (BOTH && wave_total(row_len, rows, [=](int n) {
+                return (float)min(max(n, 0), max_pages * PG);
+              }) > far_keys)
+    gqa_rows<KS, ET, MERGE, true>(q, kc, vc, block_table, max_pages, row_item,
+                                  row_len, part_o, part_ml, H, G, D, E, scale2,
+                                  NS, units, fin, vt, ml);
+  else
+    gqa_rows<KS, ET, MERGE, false>(q, kc, vc, block_table, max_pages, row_item,
+                                   row_len, part_o, part_ml, H, G, D, E, scale2,
+                                   NS, units, fin, vt, ml);
 }
 
 // Splits -> normalized, gated output; the sink joins the denominator here.
@@ -423,9 +445,11 @@ extern "C" void qsa_gqa_rows_mfma_launch(
   // pages of many rows, read once a step beside those of other layers, would drive
   // each other out of the last-level cache (16 heads on 8 of 128, 64 rows of 600-1400
   // keys, 4 layers of 268 MB: 68.9 us with loads that stay there, 52.7 with others);
-  // rows that share pages (portions' few tokens) read them from L2
-  const bool far = (long long)R * max_pages * G * (D + E) * 2 * PG > 32 << 20 &&
-                   !row_item;
+  // rows that share pages (portions' few tokens) read them from L2.  As in
+  // paged_attn.hip the kernel sums up the keys where the table has room for so many.
+  const bool far =
+      (long long)R * max_pages * G * (D + E) * 2 * PG > QSA_FAR_PAGES && !row_item;
+  const float far_keys = (float)(QSA_FAR_PAGES / (G * (D + E) * 2));
 #define QSA_GM(K, V)                                                          \
   if (part_o && far) QSA_GM_AS(K, V, false, true);                            \
   else if (part_o) QSA_GM_AS(K, V, false, false);                             \
@@ -435,7 +459,7 @@ extern "C" void qsa_gqa_rows_mfma_launch(
   hipLaunchKernelGGL((qsa_gqa_rows_mfma<K, V, MERGE, FAR>), grid, dim3(256),  \
                      0, st, q, kc, vc, block_table, max_pages, row_item,      \
                      row_len, part_o, part_ml, H, G, D, E, scale2, NS,        \
-                     units, fin)
+                     units, fin, R, far_keys)
 #define QSA_GM_E(K)                                                           \
   if (E <= 32) { QSA_GM(K, 2); }                                              \
   else if (E <= 64) { QSA_GM(K, 4); }                                         \

@@ -72,6 +72,9 @@ struct DecodeArgs {
   int blocks;
   const u32x4_v* warm[2];
   long long warm_n[2];
+  // keys of all `rows` beyond which pages are read past the last-level cache
+  int rows;
+  float far_keys;
 };
 
 // Reads memory for the launches that follow, towards the last-level cache.
@@ -115,24 +118,21 @@ template <int N> __device__ __forceinline__ void wait_vm() {
   asm volatile("" ::: "memory");
 }
 
-// FAR: loads of pages that leave no trace in the last-level cache (see the launch).
-template <int D, int NW, bool FUSE, bool FAR>
-__device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p) {
+// How pages are read: STAY, to be found in the last-level cache by the next step, or
+// PAST it (see the launch).  STAY_BUFFER is STAY in a kernel that has both, with keys
+// by buffer loads, so that an audit of its counted waits tells the two apart.
+enum { STAY, PAST, STAY_BUFFER };
+
+template <int D, int NW, bool FUSE, int PAGES>
+__device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p,
+                                               unsigned short* vlds, float* ml) {
+  constexpr bool FAR = PAGES == PAST;
   constexpr int KSTEPS = D / 32;      // QK^T k-steps (4 for D=128)
   constexpr int DTILES = D / 16;      // PV d-tiles (8 for D=128)
   constexpr int VT = D * QSA_PAGE;    // elements of a value page
   constexpr int KL = 4 * KSTEPS;      // loads of a wave for a page's keys
-  // a wave's values, afterwards its part of the output [R][D]
-  __shared__ __attribute__((aligned(16))) unsigned short vlds[NW * VT];
-  __shared__ float ml[2 * NW * 16];   // and its maxima and sums
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (FUSE && (int)blockIdx.x >= p.blocks) {
-    for (int i = 0; i < 2; ++i)
-      qsa_warm<NW * 64>(p.warm[i], p.warm_n[i], blockIdx.x - p.blocks,
-                        gridDim.x - p.blocks);
-    return;
-  }
   const int split = blockIdx.x % p.NS;
   const int bk = blockIdx.x / p.NS;
   const int b = bk / p.KVH;
@@ -169,6 +169,18 @@ __device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p) {
     auto load_k = [&](int page, bf16x8_a (&kf)[4][KSTEPS]) {
       const unsigned short* kbase =
           p.kc + ((((long long)page * p.KVH + kvh) * (D / 8)) * QSA_PAGE) * 8;
+      if constexpr (PAGES == STAY_BUFFER) {
+        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)kbase, 0, VT * 2, 0x00027000);
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+          for (int ks = 0; ks < KSTEPS; ++ks)
+            kf[pt][ks] = __builtin_bit_cast(
+                bf16x8_a, __builtin_amdgcn_raw_buffer_load_b128(
+                              rk, hi * 1024 + col * 16 + pt * 256, ks * 4096, 0));
+        return;
+      }
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
@@ -419,16 +431,42 @@ __device__ __forceinline__ void qsa_paged_attn(const DecodeArgs& p) {
   }
 }
 
+// the blocks beyond the attention's
+template <int NW>
+__device__ __forceinline__ bool qsa_warmed(const DecodeArgs& p) {
+  if ((int)blockIdx.x < p.blocks) return false;
+  for (int i = 0; i < 2; ++i)
+    qsa_warm<NW * 64>(p.warm[i], p.warm_n[i], blockIdx.x - p.blocks,
+                      gridDim.x - p.blocks);
+  return true;
+}
+
+// LDS: a wave's values, afterwards its part of the output [R][D], and its maxima and
+// sums
+#define QSA_DECODE_LDS                                                      \
+  __shared__ __attribute__((aligned(16)))                                   \
+      unsigned short vlds[NW * D * QSA_PAGE];                               \
+  __shared__ float ml[2 * NW * 16];                                         \
+  if (FUSE && qsa_warmed<NW>(p)) return
+
 template <int D, int NW, bool FUSE>
 __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
 qsa_paged_attn_mfma(DecodeArgs p) {
-  qsa_paged_attn<D, NW, FUSE, false>(p);
+  QSA_DECODE_LDS;
+  qsa_paged_attn<D, NW, FUSE, STAY>(p, vlds, ml);
 }
+// of a table that has room for far more than is live, perhaps
 template <int D, int NW, bool FUSE>
 __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
 qsa_paged_attn_far(DecodeArgs p) {
-  qsa_paged_attn<D, NW, FUSE, true>(p);
+  QSA_DECODE_LDS;
+  if (wave_total(p.seq_lens, p.rows, [](int n) { return (float)max(n, 0); }) >
+      p.far_keys)
+    qsa_paged_attn<D, NW, FUSE, PAST>(p, vlds, ml);
+  else
+    qsa_paged_attn<D, NW, FUSE, STAY_BUFFER>(p, vlds, ml);
 }
+#undef QSA_DECODE_LDS
 
 template <int D>
 __global__ void __launch_bounds__(128)
@@ -504,7 +542,8 @@ extern "C" void qsa_paged_attn_mfma_launch(
     const long long* warm_bytes, hipStream_t stream) {
   DecodeArgs p{q, kc, vc, block_table, seq_lens, part_o, part_ml, out,
                k, v, kc, vc, cos_t, sin_t, scale, QH, KVH, max_pages,
-               NS, mt, qstride, kvstride, 0, {nullptr, nullptr}, {0, 0}};
+               NS, mt, qstride, kvstride, 0, {nullptr, nullptr}, {0, 0},
+               B, (float)(QSA_FAR_PAGES / (KVH * D * 4))};
   dim3 grid((unsigned)((long long)B * KVH * NS)), block(waves * 64);
   if (grid.x == 0) return;
   p.blocks = (int)grid.x;
@@ -529,7 +568,13 @@ extern "C" void qsa_paged_attn_mfma_launch(
   // layer) 321 / 350; 16 layers of 64-dim heads, 8 rows of 300-600 (8 MB) 585 / 609, 24
   // of 800-2000 (80 MB) 987 / 971; 4096-wide, 8 layers, 1 row of 900 (4 MB) 504 / 522,
   // 16 of 1536-2048 (134 MB) 722 / 702, 192 of 400-1000 (600 MB) 2295 / 2180.
-  const bool far = (long long)B * max_pages * KVH * D * QSA_PAGE * 4 > 32 << 20;
+  // What counts are the keys that are there, which only the device knows: a captured
+  // step's table has room for `max_batch` rows of `max_seq_len`, so where that exceeds
+  // the line the kernel sums them up (us a step by room / by keys: 4096-wide, 4 rows of
+  // 600-1000 in a table of 256 pages 528 / 515, 4 live ones of 32 656 / 633; 1 row of
+  // 700 in 512 pages of the 16 layers 690 / 676; the sum itself: 192 rows 2111 / 2115).
+  const bool far =
+      (long long)B * max_pages * KVH * D * QSA_PAGE * 4 > QSA_FAR_PAGES;
 #define QSA_DECODE(DD, NW)                                                  \
   if (D == DD && waves == NW) {                                             \
     if (k && far) QSA_DECODE_AS(qsa_paged_attn_far, DD, NW, true);          \

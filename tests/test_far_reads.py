@@ -34,6 +34,68 @@ def test_pages(dim):
     assert torch.equal(run(slice(0, 66)), both)
 
 
+@pytest.mark.parametrize("fuse", [False, True])
+@pytest.mark.parametrize("over", [-1, 0, 1, 2000])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_keys_that_are_there(dim, over, fuse):
+    """A table with room for more: on either side of the keys beyond which pages are
+    read past the cache, some rows empty, bit for bit as in tables without such room."""
+    rows, heads, pages, R = 66, 8, 384 // dim, 4
+    line = (32 << 20) // (heads * dim * 4)
+    g = torch.Generator().manual_seed(dim + over)
+    sl = torch.randint(1, line // rows, (rows,), generator=g, dtype=torch.int32)
+    sl[::9] = 0
+    for i in range(1, rows):                      # up to the sum that is wanted
+        if i % 9:
+            sl[i] += min(pages * 64 - int(sl[i]), line + over - int(sl.sum()))
+    assert int(sl.sum()) == line + over
+    bt = torch.randperm(rows * pages, generator=g).int().view(rows, pages)
+    bt, sl = bt.to(DEV), sl.to(DEV)
+    kc = rnd(rows * pages, heads, dim // 8, 64, 8)
+    vc = rnd(rows * pages, heads, dim, 64)
+    q, k, v = rnd(rows, R * heads, dim), rnd(rows, heads, dim), rnd(rows, heads, dim)
+    ang = torch.rand(pages * 64, dim // 2, device=DEV)
+
+    def run(i, kc, vc):
+        if not fuse:
+            return ext().paged_attn_decode(q[i], kc, vc, bt[i], sl[i], dim ** -0.5)
+        return ext().paged_attn_step(q[i], k[i], v[i], kc, vc, ang.cos(), ang.sin(),
+                                     bt[i], sl[i], dim ** -0.5, False, [])
+
+    halves = kc.clone(), vc.clone()
+    whole = run(slice(0, rows), kc, vc)
+    both = torch.cat([run(slice(0, 33), *halves), run(slice(33, 66), *halves)])
+    assert torch.equal(whole, both)
+    assert torch.equal(kc, halves[0]) and torch.equal(vc, halves[1])
+
+
+@pytest.mark.parametrize("over", [-1, 0, 1])
+def test_keys_of_grouped_rows_that_are_there(over):
+    """The same of grouped rows; lengths beyond the table count as its width."""
+    rows, heads, G, dim, pages = 132, 16, 8, 128, 8
+    line = (32 << 20) // (G * 2 * dim * 2)
+    g = torch.Generator().manual_seed(over + 7)
+    n = torch.full((rows,), line // rows - 6, dtype=torch.int32)
+    n[1] = 0
+    n[2] = pages * 64 + 9
+    n[0] = line + over - int(n[3:].sum()) - pages * 64
+    assert 0 < n[0] < pages * 64
+    bt = torch.randint(0, 40, (rows, pages), generator=g, dtype=torch.int32)
+    bt, n = bt.to(DEV), n.to(DEV)
+    kc, vc = rnd(40, G, 64, dim), rnd(40, G, 64, dim)
+    q, gate = rnd(rows, heads * dim), rnd(rows, heads * dim)
+
+    def run(i):
+        out = torch.empty(len(range(*i.indices(rows))), heads * dim, dtype=BF,
+                          device=DEV)
+        D.gqa_rows(q[i], kc, vc, bt[i], None, n[i], None, gate[i], out, heads,
+                   dim ** -0.5)
+        return out
+
+    assert torch.equal(run(slice(0, rows)),
+                       torch.cat([run(slice(0, 66)), run(slice(66, rows))]))
+
+
 def test_pages_of_grouped_rows():
     torch.manual_seed(1)
     rows, heads, G, dim, pages = 132, 16, 8, 128, 8

@@ -121,6 +121,28 @@ def test_counted_waits_past_the_cache():
         assert sum(t.endswith(" nt") for t in code) >= keys, name
 
 
+def test_counted_waits_of_few_keys_in_a_large_table():
+    """The same kernels' form for pages that stay in the cache, whose keys are buffer
+    loads: its counted wait stands behind exactly one page's."""
+    import isa_check
+    so = isa_check.find_so()
+    if so is None or not os.path.exists(isa_check.BUNDLER):
+        pytest.skip("built extension or ROCm LLVM tools unavailable")
+    with tempfile.TemporaryDirectory() as wd:
+        kernels = isa_check.instructions(
+            isa_check.extract_hsacos(so, wd), "qsa_paged_attn_far")
+    assert len(kernels) == 8
+    for name, code in kernels.items():
+        keys = 16 if "ILi128E" in name else 8
+        stay = [t.replace("buffer_load_dwordx4", "global_load_dwordx4")
+                if t.startswith("buffer_load_dwordx4") and " lds" not in t
+                else t.replace("global_load_dwordx4", "global_load_past")
+                for t in code]
+        assert counted_waits(stay, keys) == 1, name
+        assert not any(t.startswith("buffer_load_dwordx4") and " lds" not in t
+                       and t.endswith(" nt") for t in code), name
+
+
 def test_the_audit_sees_a_moved_load():
     keys = ["global_load_dwordx4 v[0:3], v[4:5], off"] * 2
     wait = ["s_waitcnt vmcnt(2)"]
