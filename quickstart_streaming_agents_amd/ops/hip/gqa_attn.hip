@@ -344,9 +344,19 @@ qsa_gqa_rows_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                   int units, GqaFinish fin, int rows, float far_keys) {
   __shared__ __attribute__((aligned(16))) bf16_t vt[4][32 * (16 * ET + 16)];
   __shared__ float ml[4][16][2];                  // MERGE
-  if (BOTH && wave_total(row_len, rows, [=](int n) {
-                return (float)min(max(n, 0), max_pages * PG);
-              }) > far_keys)
+  bool past = false;
+  if constexpr (BOTH) {
+    // the row's length and first page are on their way meanwhile
+    const int unit = __builtin_amdgcn_readfirstlane(
+        min(blockIdx.x * 4 + (threadIdx.x >> 6), (unsigned)units - 1));
+    const int row = unit / (NS * ((H / G + 15) / 16) * G);
+    const int n = row_len[row], page = block_table[(long long)row * max_pages];
+    past = wave_total(row_len, rows, [=](int k) {
+             return (float)min(max(k, 0), max_pages * PG);
+           }) > far_keys;
+    asm volatile("" ::"s"(n), "s"(page));
+  }
+  if (past)
     gqa_rows<KS, ET, MERGE, true>(q, kc, vc, block_table, max_pages, row_item,
                                   row_len, part_o, part_ml, H, G, D, E, scale2,
                                   NS, units, fin, vt, ml);
