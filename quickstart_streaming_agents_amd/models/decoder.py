@@ -14,8 +14,9 @@ from dataclasses import dataclass
 
 import torch
 
+from ..ops import dispatch as D
 from .kv_cache import HybridCache
-from .layers import RopeTable, StepPlan
+from .layers import RopeTable, StepPlan, projections
 from .mixers import MIXERS, Shard, cache_args
 from .weights import SafetensorsFile
 
@@ -78,6 +79,10 @@ class MixerDecoder:
             return t.to(device=device, dtype=dtype).contiguous()
 
         self.build(get)
+        found = projections(self)
+        far = D.far_weights(sum(p.w.nbytes for p in found))
+        for p in found:
+            p.far = far
         self.ensure_positions(256)
 
     @classmethod

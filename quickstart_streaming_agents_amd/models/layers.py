@@ -4,6 +4,7 @@ tables, feed-forwards and the device-side description of a step."""
 from __future__ import annotations
 
 import math
+from types import MethodType
 
 import numpy as np
 import torch
@@ -35,6 +36,7 @@ class Linear:
 
     def __init__(self, w: torch.Tensor):
         self.w = w
+        self.far = False           # of a model whose weights exceed the cache
         n, k = w.shape
         self.packed = None
         if w.is_cuda and w.dtype == torch.bfloat16 and \
@@ -50,14 +52,14 @@ class Linear:
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         if self._skinny(x, self.rows):
-            return D.skinny_linear(x, self.packed, *self.w.shape)
-        return D.linear(x, self.w)
+            return D.skinny_linear(x, self.packed, *self.w.shape, self.far)
+        return D.linear(x, self.w, self.far)
 
     def parts(self, x: torch.Tensor) -> torch.Tensor:
         """y for a reader that adds shares of K (D.linear_parts)."""
         if self._skinny(x, self.rows_parts):
-            return D.skinny_linear(x, self.packed, *self.w.shape)
-        return D.linear_parts(x, self.w)
+            return D.skinny_linear(x, self.packed, *self.w.shape, self.far)
+        return D.linear_parts(x, self.w, self.far)
 
     def _skinny(self, x: torch.Tensor, below: int) -> bool:
         return self.packed is not None and \
@@ -68,9 +70,30 @@ class Linear:
         """act(gate) * up of y = [gate, up]."""
         if not self._skinny(x, self.SKINNY_ROWS + 1) and \
                 D.glu_linear_ok(x, self.w):
-            return D.glu_linear(x, self.w, act)
+            return D.glu_linear(x, self.w, act, far=self.far)
         y, half = self(x), self.w.shape[0] // 2
         return D.glu(y[:, :half], y[:, half:], act)
+
+
+def projections(part) -> list[Linear]:
+    """The Linears in a model's parts: attributes, lists, bound calls of one."""
+    found, seen, todo = [], set(), [part]
+    while todo:
+        p = todo.pop()
+        if isinstance(p, MethodType):
+            p = p.__self__
+        if id(p) in seen:
+            continue
+        seen.add(id(p))
+        if isinstance(p, Linear):
+            found.append(p)
+        elif isinstance(p, (list, tuple)):
+            todo += p
+        elif isinstance(p, dict):
+            todo += p.values()
+        elif type(p).__module__.startswith(__package__ + "."):
+            todo += vars(p).values()
+    return found
 
 
 def rope_frequencies(dims: int, base: float,

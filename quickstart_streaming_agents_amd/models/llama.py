@@ -178,12 +178,6 @@ class LlamaModel:
                             L[key + "_f8"] = D.pack_weight_fp8(wt)
                 if D.can_pack_weight(*self.lm_head.shape):
                     self.lm_head_f8 = D.pack_weight_fp8(self.lm_head)
-                # whether a step's weights are more than the last-level cache of
-                # 256 MB keeps beside keys and values (skinny_stream.h, FAR)
-                packs = [p for L in self.layers for k, p in L.items()
-                         if k.endswith("_f8")] + [self.lm_head_f8]
-                self.weights_far = sum(p[0].numel() for p in packs
-                                       if p is not None) > 192 << 20
             else:
                 def want(shape):
                     # only shapes where bf16 skinny beats rocBLAS
@@ -197,6 +191,19 @@ class LlamaModel:
                             L[key + "_f"] = D.pack_weight_frag(wt)
                 if want(self.lm_head.shape):
                     self.lm_head_f = D.pack_weight_frag(self.lm_head)
+        # of a step of up to 32 rows, and of more: weights in fp8 where packed, and
+        # as they are stored
+        self.weights_far = D.far_weights(sum(self._weight_bytes(True)))
+        self.stored_far = D.far_weights(sum(self._weight_bytes(False)))
+
+    def _weight_bytes(self, packed: bool):
+        for L in self.layers:
+            for key in ("wqkv", "wo", "wgu", "wdown"):
+                if key in L:
+                    yield (L[key + "_f8"][0] if packed and key + "_f8" in L
+                           else L[key]).nbytes
+        yield (self.lm_head_f8[0] if packed and self.lm_head_f8 is not None
+               else self.lm_head).nbytes
 
     def _ffn_weights(self, w, rows, cols) -> dict:
         """Per-layer FFN weights; the generator order is part of the
@@ -230,7 +237,8 @@ class LlamaModel:
         M = x.shape[0]
         if x.is_cuda and wf8 is not None:
             if M <= 32:
-                return D.skinny_linear_fp8(x, wf8[0], wf8[1], n, k)
+                return D.skinny_linear_fp8(x, wf8[0], wf8[1], n, k,
+                                           self.weights_far)
             # 32 < M <= 256 (continuous-batching decode): the batched fp8
             # kernel (ops/hip/gemm_fp8_batch.hip) is measured SLOWER than
             # bf16 products at these M on MI355X — the problem is L2-/
@@ -250,8 +258,9 @@ class LlamaModel:
             # the packed stream wins only the small decode shapes (qkv/wo);
             # large ones are rows_gemm's (one row, us: 28672 x 4096 45, the
             # library 56; 128256 x 2048 95 and 108)
-            return D.skinny_linear(x, wf, n, k)
-        return D.linear_parts(x, w) if parts else D.linear(x, w)
+            return D.skinny_linear(x, wf, n, k, self.weights_far)
+        far = self.weights_far if M <= 32 else self.stored_far
+        return D.linear_parts(x, w, far) if parts else D.linear(x, w, far)
 
     def _tp_all_reduce(self, t: torch.Tensor) -> torch.Tensor:
         if self.tp_size > 1:
@@ -361,7 +370,7 @@ class LlamaModel:
         import os as _os
         if h.shape[0] > 32 and _os.environ.get("QSA_FP8_BATCH") != "1" and \
                 D.glu_linear_ok(h, L["wgu"]):
-            act = D.glu_linear(h, L["wgu"])
+            act = D.glu_linear(h, L["wgu"], far=self.stored_far)
         else:
             gu = self._linear(h, L["wgu"], L.get("wgu_f"), L.get("wgu_f8"))
             act = D.swiglu(gu[:, :self.ffn_local], gu[:, self.ffn_local:])
@@ -497,7 +506,7 @@ class LlamaModel:
                 h = D.rmsnorm_residual(mlp_out, res, L["attn_norm"],
                                        c.norm_eps)
             qkv = F.linear(h, L["wqkv"], L["bqkv"]) if "bqkv" in L \
-                else D.linear(h, L["wqkv"])
+                else D.linear(h, L["wqkv"], self.stored_far)
             q, k, v = self._split_qkv(qkv, T_pad)
             if use_hip_prefill:
                 D.rope_kv_scatter(q[:T], k[:T], v[:T], kv.k[li], kv.v[li],
@@ -540,8 +549,9 @@ class LlamaModel:
                     .reshape(nb * nmax, self.n_q * c.d_head) \
                     .index_select(0, dst_idx)
             o = self._tp_all_reduce(
-                D.linear_parts(attn, L["wo"]) if self.tp_size == 1
-                else D.linear(attn, L["wo"]))
+                D.linear_parts(attn, L["wo"], self.stored_far)
+                if self.tp_size == 1
+                else D.linear(attn, L["wo"], self.stored_far))
             h = D.rmsnorm_residual(o, res, L["mlp_norm"], c.norm_eps)
             mlp_out = self._ffn(L, h)
         final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)

@@ -102,6 +102,13 @@ class MixtralModel(LlamaModel):
         return {"router": router, "experts": experts,
                 "experts_f": packed}
 
+    def _weight_bytes(self, packed: bool):
+        """Steps choose other experts, so all of them count."""
+        yield from super()._weight_bytes(packed)
+        for L in self.layers:
+            for pair in L["experts"].values():
+                yield sum(w.nbytes for w in pair)
+
     def _ffn(self, L: dict, h: torch.Tensor) -> torch.Tensor:
         c = self._moe_cfg
         logits = F.linear(h, L["router"]).float()
@@ -113,9 +120,10 @@ class MixtralModel(LlamaModel):
             wgu, wdown = L["experts"][e]
             pk = L.get("experts_f", {}).get(e)
             if pk is not None and rows.is_cuda and rows.shape[0] <= 32:
-                gu = D.skinny_linear(rows, pk[0], *wgu.shape)
+                far = self.weights_far
+                gu = D.skinny_linear(rows, pk[0], *wgu.shape, far)
                 act = D.swiglu(gu[:, :c.ffn], gu[:, c.ffn:])
-                return D.skinny_linear(act, pk[1], *wdown.shape)
+                return D.skinny_linear(act, pk[1], *wdown.shape, far)
             gu = F.linear(rows, wgu)
             act = D.swiglu(gu[:, :c.ffn], gu[:, c.ffn:])
             return F.linear(act, wdown)

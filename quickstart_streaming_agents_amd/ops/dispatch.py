@@ -221,18 +221,32 @@ def _gemm_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
         lm_ext().gemm_ok(x, w) and not torch.compiler.is_compiling()
 
 
-def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+# `far` of the projections: a step's weights exceed the last-level cache, so each is
+# read past it (ops/hip/skinny_stream.h); only the model knows.  us a step of 40 rows,
+# weights that stay / past the cache, decoders of width 1024 with 122 MB of weights
+# 91 / 97, 182 MB 163 / 169, 242 MB 246 / 240, 302 MB 338 / 313, 422 MB 492 / 458.
+FAR_WEIGHTS = 192 << 20
+
+
+def far_weights(nbytes: int) -> bool:
+    """Whether a decoding step's weights are more than the last-level cache of 256 MB
+    keeps beside keys and values."""
+    return nbytes > FAR_WEIGHTS
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, far: bool = False) -> torch.Tensor:
     """x @ W^T for a weight as it is stored."""
     if _gemm_ok(x, w):
-        return lm_ext().gemm(x, w)
+        return lm_ext().gemm(x, w, far)
     return torch.nn.functional.linear(x, w)
 
 
-def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def linear_parts(x: torch.Tensor, w: torch.Tensor,
+                 far: bool = False) -> torch.Tensor:
     """linear() for a reader that adds shares (residual_norm, rmsnorm_residual,
     glu_table): where K is split, [S, rows, columns] in f32."""
     if _gemm_ok(x, w):
-        return lm_ext().gemm_parts(x, w)
+        return lm_ext().gemm_parts(x, w, far)
     return torch.nn.functional.linear(x, w)
 
 
@@ -253,19 +267,19 @@ def glu_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
         lm_ext().glu_gemm_ok(x, w) and not torch.compiler.is_compiling()
 
 
-def glu_linear(x: torch.Tensor, w: torch.Tensor,
-               act: str = "silu", rounded: bool = True) -> torch.Tensor:
+def glu_linear(x: torch.Tensor, w: torch.Tensor, act: str = "silu",
+               rounded: bool = True, far: bool = False) -> torch.Tensor:
     """act(x @ W_gate^T) * (x @ W_up^T) of W = [gate; up], in one kernel; with
     `rounded` of the products as linear() would store them, without (silu only)
     of their f32 sums."""
-    return lm_ext().glu_gemm(x, w, act == "gelu", rounded)
+    return lm_ext().glu_gemm(x, w, act == "gelu", rounded, far)
 
 
-def skinny_linear(x: torch.Tensor, wf: torch.Tensor, n: int,
-                  k: int) -> torch.Tensor:
+def skinny_linear(x: torch.Tensor, wf: torch.Tensor, n: int, k: int,
+                  far: bool = False) -> torch.Tensor:
     """x[M,K] @ W^T via the weight-streaming decode kernel (M <= 32)."""
     if x.is_cuda:
-        return lm_ext().skinny_gemm(x, wf, n, k)
+        return lm_ext().skinny_gemm(x, wf, n, k, far)
     w = wf.reshape(n // 16, k // 32, 16, 32).permute(0, 2, 1, 3) \
         .reshape(n, k)
     return (x.float() @ w.float().T).to(x.dtype)
@@ -306,10 +320,11 @@ def gemm_fp8_batch(x: torch.Tensor, qf: torch.Tensor,
 
 
 def skinny_linear_fp8(x: torch.Tensor, qf: torch.Tensor,
-                      scale: torch.Tensor, n: int, k: int) -> torch.Tensor:
+                      scale: torch.Tensor, n: int, k: int,
+                      far: bool = False) -> torch.Tensor:
     """x[M,K] bf16 @ dequant(Q)^T via the fp8 weight-streaming kernel."""
     if x.is_cuda:
-        return ext().skinny_gemm_fp8(x, qf, scale, n, k)
+        return ext().skinny_gemm_fp8(x, qf, scale, n, k, far)
     w = unpack_weight_fp8(qf, scale, n, k)
     return (x.float() @ w.T).to(x.dtype)
 
@@ -326,17 +341,15 @@ def embed_rows(embed: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor):
 
 def norm_linear_fp8(x: torch.Tensor, ss: torch.Tensor, parts: int, rows: int,
                     eps: float, packed: tuple, n: int, k: int,
-                    glu: bool = False, far: bool = True) -> torch.Tensor:
+                    glu: bool = False, far: bool = False) -> torch.Tensor:
     """Normed step rows through a packed fp8 weight: [rows, n].  With `glu`
-    its rows are [gate; up] and the result is silu(gate) * up, step rows.
-    `far`: the step's weights exceed the last-level cache, so they are read past
-    it (ops/hip/skinny_stream.h)."""
+    its rows are [gate; up] and the result is silu(gate) * up, step rows."""
     return ext().skinny_gemm_fp8_norm(x, ss, parts, rows, eps, packed[0],
                                       packed[1], n, k, glu, far)
 
 
 def linear_residual_fp8(x: torch.Tensor, packed: tuple, n: int, k: int,
-                        res: torch.Tensor, w: torch.Tensor, far: bool = True):
+                        res: torch.Tensor, w: torch.Tensor, far: bool = False):
     """res <- res + step rows x through a packed fp8 weight, in place; returns
     the step rows of the norm with weight w that follows, and ss, in
     residual_parts_fp8 parts."""

@@ -131,14 +131,14 @@ extern "C" void qsa_window_attn_prefill_launch(const bf16_t*, long long,
     const int*, const int*, const int*, const int*, const int*, const int*,
     const int*, bf16_t*, int, int, int, int, int, float, hipStream_t);
 extern "C" void qsa_skinny_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
-    int, int, long long, long long, hipStream_t);
+    int, int, long long, long long, bool, hipStream_t);
 extern "C" int qsa_rows_gemm_plan(int, int, int, int, int, int*, float*);
 extern "C" bool qsa_wide_gemm_fits(int, int, int);
 extern "C" float qsa_wide_gemm_plan(int, int, int, int, int*, int*, int*);
 extern "C" void qsa_wide_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*, int,
                                      int, int, long long, int, int, hipStream_t);
 extern "C" void qsa_rows_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
-    float*, int, int, int, long long, int, int, int, hipStream_t);
+    float*, int, int, int, long long, int, int, int, bool, hipStream_t);
 
 // Whether t [S, rows, cols] is a product of bf16 rows whose shares of K have not
 // been added (rows_parts)
@@ -951,7 +951,7 @@ void part_norm(Tensor x, Tensor w, Tensor out, long parts, double eps) {
 }
 
 // weight-streaming decode product, W packed as [N/16, K/32, 16, 32]
-Tensor skinny_gemm(Tensor a, Tensor wf, long N, long K) {
+Tensor skinny_gemm(Tensor a, Tensor wf, long N, long K, bool far) {
   CHK_DEV(a); chk_rows(a, "a"); CHK_CONT(wf); CHK_SAME(a, wf);
   TORCH_CHECK(a.scalar_type() == at::kBFloat16, "bf16");
   const int M = (int)a.size(0);
@@ -960,7 +960,7 @@ Tensor skinny_gemm(Tensor a, Tensor wf, long N, long K) {
   TORCH_CHECK(a.stride(0) % 8 == 0 && aligned(a, 16), "a alignment");
   auto out = torch::empty({M, (long long)N}, a.options());
   qsa_skinny_gemm_launch(u16(a), u16(wf), u16m(out), M, (int)N, K,
-                         a.stride(0), cur_stream());
+                         a.stride(0), far, cur_stream());
   return out;
 }
 
@@ -1074,9 +1074,10 @@ bool glu_gemm_ok(const Tensor& a, const Tensor& w) {
           wide_sizes(a, w, true));
 }
 
-// parts: a product whose K is split may stay in its shares, [S, M, N] f32
+// parts: a product whose K is split may stay in its shares, [S, M, N] f32; far: w is
+// read past the last-level cache, where each of its numbers is read once
 static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
-                            bool parts = false) {
+                            bool parts = false, bool far = false) {
   CHK_DEV(a); CHK_SAME(a, w);
   TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
               "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
@@ -1088,25 +1089,25 @@ static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
   if (S == 1 || !parts) out = torch::empty({M, act ? N / 2 : N}, a.options());
   qsa_rows_gemm_launch(u16(a), u16(w), out.defined() ? u16m(out) : nullptr,
                        S > 1 ? part.data_ptr<float>() : nullptr, M, N, K,
-                       a.stride(0), tile, S, act, cur_stream());
+                       a.stride(0), tile, S, act, far, cur_stream());
   return out.defined() ? out : part;
 }
 
 // The same by whichever of the two should be over first.  rows_gemm's estimate is of
 // CUs that keep their clock: where it comes within 14 % of the other's, the other is
 // sooner (of 200 shapes, M 200 to 45,000, the choice is then 0.5 % from the best).
-static Tensor gemm_run(const Tensor& a, const Tensor& w, int act,
-                       bool parts = false) {
+static Tensor gemm_run(const Tensor& a, const Tensor& w, int act, bool parts,
+                       bool far) {
   CHK_DEV(a); CHK_SAME(a, w);
   TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
               "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
   const WidePlan p = wide_plan(a, w, act);
-  if (p.us == 1e30f) return rows_gemm_run(a, w, act, parts);
+  if (p.us == 1e30f) return rows_gemm_run(a, w, act, parts, far);
   const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
   int S;
   float us;
   qsa_rows_gemm_plan(M, N, K, act, parts, &S, &us);
-  if (us * 1.14f < p.us) return rows_gemm_run(a, w, act, parts);
+  if (us * 1.14f < p.us) return rows_gemm_run(a, w, act, parts, far);
   const int64_t cols = act ? N / 2 : N;
   Tensor out = torch::empty({M, cols}, a.options());
   qsa_wide_gemm_launch(u16(a), u16(w), u16m(out), p.rows, N, K, a.stride(0), p.tile,
@@ -1152,7 +1153,9 @@ std::tuple<int, int> rows_gemm_plan(int64_t M, int64_t N, int64_t K,
 }
 
 // a @ w^T on W as it is stored
-Tensor rows_gemm(Tensor a, Tensor w) { return rows_gemm_run(a, w, 0); }
+Tensor rows_gemm(Tensor a, Tensor w, bool far) {
+  return rows_gemm_run(a, w, 0, false, far);
+}
 
 // the same for a reader that adds shares: [M, N], or [S, M, N] in f32
 Tensor rows_parts(Tensor a, Tensor w) { return rows_gemm_run(a, w, 0, true); }
@@ -1181,11 +1184,15 @@ Tensor rows_glu(Tensor a, Tensor w, bool gelu, bool rounded) {
 
 // a @ w^T, for a reader that adds shares perhaps in them, and the gated activation of
 // it, by whichever kernel the rules give
-Tensor gemm(Tensor a, Tensor w) { return gemm_run(a, w, 0); }
-Tensor gemm_parts(Tensor a, Tensor w) { return gemm_run(a, w, 0, true); }
-Tensor glu_gemm(Tensor a, Tensor w, bool gelu, bool rounded) {
+Tensor gemm(Tensor a, Tensor w, bool far) {
+  return gemm_run(a, w, 0, false, far);
+}
+Tensor gemm_parts(Tensor a, Tensor w, bool far) {
+  return gemm_run(a, w, 0, true, far);
+}
+Tensor glu_gemm(Tensor a, Tensor w, bool gelu, bool rounded, bool far) {
   TORCH_CHECK(rounded || !gelu, "gelu of the stored products only");
-  return gemm_run(a, w, gelu ? 2 : rounded ? 1 : 3);
+  return gemm_run(a, w, gelu ? 2 : rounded ? 1 : 3, false, far);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1219,8 +1226,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("window_attn_prefill", &window_attn_prefill,
         "windowed flash attention with sink and gate (MFMA)");
   m.def("window_attn_ok", &window_attn_ok, "size support");
-  m.def("skinny_gemm", &skinny_gemm, "packed-weight decode GEMM (M <= 32)");
-  m.def("rows_gemm", &rows_gemm, "GEMM of decode batches and short prompts");
+  m.def("skinny_gemm", &skinny_gemm, "packed-weight decode GEMM (M <= 32)",
+        py::arg("a"), py::arg("wf"), py::arg("N"), py::arg("K"),
+        py::arg("far") = false);
+  m.def("rows_gemm", &rows_gemm, "GEMM of decode batches and short prompts",
+        py::arg("a"), py::arg("w"), py::arg("far") = false);
   m.def("rows_gemm_ok", &rows_gemm_ok, "whether a product is rows_gemm's");
   m.def("rows_parts", &rows_parts, "the same, shares of K left to the reader");
   m.def("rmsnorm_shares", &rmsnorm_shares,
@@ -1229,10 +1239,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "whether sizes are rows_gemm's, or with the activation inside");
   m.def("rows_gemm_plan", &rows_gemm_plan, "tile and shares of a product");
   m.def("rows_glu", &rows_glu, "the same with the gated activation inside");
-  m.def("gemm", &gemm, "rows_gemm or wide_gemm by size");
+  m.def("gemm", &gemm, "rows_gemm or wide_gemm by size", py::arg("a"), py::arg("w"),
+        py::arg("far") = false);
   m.def("gemm_ok", &gemm_ok, "whether a product is one of theirs");
-  m.def("gemm_parts", &gemm_parts, "the same, shares of K left to the reader");
-  m.def("glu_gemm", &glu_gemm, "the same with the gated activation inside");
+  m.def("gemm_parts", &gemm_parts, "the same, shares of K left to the reader",
+        py::arg("a"), py::arg("w"), py::arg("far") = false);
+  m.def("glu_gemm", &glu_gemm, "the same with the gated activation inside",
+        py::arg("a"), py::arg("w"), py::arg("gelu"), py::arg("rounded"),
+        py::arg("far") = false);
   m.def("glu_gemm_ok", &glu_gemm_ok, "whether a gated product is one of theirs");
   m.def("wide_gemm", &wide_gemm, "GEMM of many rows by a given tile");
   m.def("wide_gemm_plan", &wide_gemm_plan, "tiles and rows of a product");

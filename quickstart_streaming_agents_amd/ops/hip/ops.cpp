@@ -80,7 +80,7 @@ extern "C" void qsa_kv_scatter_launch(const unsigned short*,
                                       int, long long, hipStream_t);
 extern "C" void qsa_skinny_gemm_launch(const unsigned short*,
                                        const unsigned short*, unsigned short*,
-                                       int, int, long long, long long,
+                                       int, int, long long, long long, bool,
                                        hipStream_t);
 extern "C" int qsa_skinny_gemm_probe_launch(const unsigned short*,
                                             const unsigned short*,
@@ -495,7 +495,7 @@ torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor wf, long N, long K) {
   TORCH_CHECK(wf.numel() == (long long)N * K, "wf size");
   auto out = torch::empty({M, (long long)N}, a.options());
   qsa_skinny_gemm_launch(u16(a), u16(wf), u16m(out), M, (int)N, K,
-                         a.stride(0), cur_stream());
+                         a.stride(0), false, cur_stream());
   return out;
 }
 
@@ -972,7 +972,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm_fp8", &skinny_gemm_fp8,
         "fp8-weight decode GEMM (M<=32): half the weight stream",
         py::arg("a"), py::arg("qf"), py::arg("scale"), py::arg("N"),
-        py::arg("K"), py::arg("far") = true);
+        py::arg("K"), py::arg("far") = false);
   m.def("gemm_fp8_batch", &gemm_fp8_batch,
         "batched-M (<=256) fp8 weight-stream GEMM with optional split-K");
   m.def("skinny_gemm_fp8_probe", &skinny_gemm_fp8_probe,
@@ -981,13 +981,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fp8-weight decode GEMM of rms-normed rows, optionally gated",
         py::arg("a"), py::arg("ss"), py::arg("parts"), py::arg("M"),
         py::arg("eps"), py::arg("qf"), py::arg("scale"), py::arg("N"),
-        py::arg("K"), py::arg("glu"), py::arg("far") = true);
+        py::arg("K"), py::arg("glu"), py::arg("far") = false);
   m.def("skinny_gemm_fp8_parts", &skinny_gemm_fp8_parts,
         "parts of a row's sum of squares behind a residual");
   m.def("skinny_gemm_fp8_residual", &skinny_gemm_fp8_residual,
         "fp8-weight decode GEMM added to the residual stream",
         py::arg("a"), py::arg("qf"), py::arg("scale"), py::arg("N"),
-        py::arg("K"), py::arg("res"), py::arg("w"), py::arg("far") = true);
+        py::arg("K"), py::arg("res"), py::arg("w"), py::arg("far") = false);
   m.def("embed_rows", &embed_rows,
         "a step's first rows and their sums of squares");
   m.def("topk_cosine_host", &topk_cosine_host,

@@ -33,6 +33,8 @@ struct RowsArgs {
   int M, N, K, S;
   int MB, NB;                          // blocks along rows and columns
   unsigned int lda;                    // elements
+  bool far;                            // W is larger than the last-level cache,
+                                       // together with what a step reads beside it
 };
 
 // Whether two blocks of eight waves share a CU's 160 KB (128 bytes a row and stage)
@@ -276,8 +278,9 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
   // drive it out of the last-level cache before the next step; past it they come faster
   // and leave it to what fits (decoder of width 4096, 8 layers, 192 rows of 400-1000
   // keys 2295 -> 2180 us a step with keys and values likewise, 28672 x 4096 57 -> 54;
-  // of width 2048, 64 rows 813 -> 746).  Small ones may be of a model that fits.
-  const bool once = BM <= 192 && p.MB == 1 && (long long)p.N * p.K >= 2 << 20;
+  // of width 2048, 64 rows 813 -> 746).
+  const bool once =
+      p.far && BM <= 192 && p.MB == 1 && (long long)p.N * p.K >= 2 << 20;
 #define QSA_RG_AS(ACT, ONCE) \
   hipLaunchKernelGGL((qsa_rows_gemm<BM, BN, WM, WN, ST, ACT, ONCE>), grid, \
                      dim3(WM * WN * 64), 0, st, p)
@@ -402,8 +405,8 @@ extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
 extern "C" void qsa_rows_gemm_launch(const bf16_t* A, const bf16_t* W,
                                      bf16_t* C, float* part, int M, int N,
                                      int K, long long lda, int tile, int S,
-                                     int act, hipStream_t st) {
-  const RowsArgs p{A, W, C, part, M, N, K, S, 0, 0, (unsigned int)lda};
+                                     int act, bool far, hipStream_t st) {
+  const RowsArgs p{A, W, C, part, M, N, K, S, 0, 0, (unsigned int)lda, far};
   int i = 0;
 #define X(BM, BN, WM, WN, ST, OWN, STAGE, OWN2, STAGE2) \
   if (tile == i++) rows_go<BM, BN, WM, WN, ST>(p, act, st);

@@ -10,8 +10,8 @@
 // W is packed once at model init into [N/16, K/32, 16, 32]: one wave
 // instruction reads one 1 KiB 16x32 fragment block.
 //
-// Weights of 4 MB on are taken to be of a model whose weights exceed the last-level
-// cache (skinny_stream.h, FAR).
+// Whether W is read past the last-level cache (skinny_stream.h, FAR) is the caller's
+// to say, who knows what else a step reads; matrices below 4 MB stay there.
 // Block shapes follow the fp8 form's measurements: one tile of 16 columns per
 // block, two from 6144 columns on; 4 waves for K up to 2048, 8 above.
 #include "skinny_stream.h"
@@ -38,18 +38,18 @@ static void bf16_go(const SkinnyArgs& p, hipStream_t st) {
 
 static SkinnyArgs bf16_args(const unsigned short* A, const unsigned short* Wf,
                             unsigned short* C, int M, int N, long long K,
-                            long long lda) {
+                            long long lda, bool far) {
   return SkinnyArgs{A, reinterpret_cast<const u32x4_v*>(Wf), nullptr, C,
                     nullptr, nullptr, nullptr, nullptr, M, N, 0, K, lda,
-                    0.f, (long long)N * K >= 2 << 20};
+                    0.f, far && (long long)N * K >= 2 << 20};
 }
 
 extern "C" void qsa_skinny_gemm_launch(const unsigned short* A,
                                        const unsigned short* Wf,
                                        unsigned short* Cbf, int M, int N,
-                                       long long K, long long lda,
+                                       long long K, long long lda, bool far,
                                        hipStream_t stream) {
-  const SkinnyArgs p = bf16_args(A, Wf, Cbf, M, N, K, lda);
+  const SkinnyArgs p = bf16_args(A, Wf, Cbf, M, N, K, lda, far);
   if (K <= 2048) bf16_go<4, 1>(p, stream);
   else if (N >= 6144 && N % 32 == 0) bf16_go<8, 2>(p, stream);
   else bf16_go<8, 1>(p, stream);
@@ -60,7 +60,7 @@ extern "C" int qsa_skinny_gemm_probe_launch(
     const unsigned short* A, const unsigned short* Wf, unsigned short* Cbf,
     int M, int N, long long K, long long lda, int waves, int tiles,
     hipStream_t stream) {
-  const SkinnyArgs p = bf16_args(A, Wf, Cbf, M, N, K, lda);
+  const SkinnyArgs p = bf16_args(A, Wf, Cbf, M, N, K, lda, true);
 #define QSA_CASE(W, T)               \
   if (waves == W && tiles == T) {    \
     bf16_go<W, T>(p, stream);        \
