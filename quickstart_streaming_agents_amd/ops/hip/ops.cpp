@@ -855,9 +855,10 @@ py::object topk_cosine_host(
       for (; j < D; ++j) s[0] += (double)x[j] * x[j];
       const double sum = s[0] + s[1] + s[2] + s[3];
       numbers = std::isfinite(sum);    // squares of floats stay in range
-      // the norm is a float, infinite beyond what floats hold
-      const float norm = std::max(std::sqrt((float)sum), 1e-12f);
-      for (j = 0; j < D; ++j) host[i * D + j] = x[j] / norm;
+      // rounded once, at the end; a norm beyond what floats hold is infinite
+      const double inv = std::isinf((float)sum)
+          ? 0.0 : 1.0 / std::max(std::sqrt(sum), 1e-12);
+      for (j = 0; j < D; ++j) host[i * D + j] = (float)(x[j] * inv);
     }
     if (numbers) {
       auto rows_on = torch::empty({Q, D}, docs.options());
