@@ -189,9 +189,9 @@ class VectorIndex:
         q = np.asarray(queries, dtype=np.float32)
         docs = self.to_torch(device)
         k_eff = min(k, len(self))
-        scan = _scan_wins(len(q), len(self), k_eff)
+        scan = q.ndim > 0 and _scan_wins(len(q), len(self), k_eff)
         both = None
-        if scan and docs.is_cuda and q.size <= _HOST_QUERIES:
+        if scan and docs.is_cuda and q.ndim == 2 and q.size <= _HOST_QUERIES:
             # none if a query is not a number, or infinite
             both = D.topk_cosine_host(q, docs, k_eff)
         if both is None:

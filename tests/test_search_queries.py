@@ -26,3 +26,14 @@ def test_norms_are_rounded_once(dim, scale):
     want = np.take_along_axis(x / np.maximum(norm, 1e-12), at, 1)
     assert (np.abs(score - want) <= 2.0 ** -24 * (1 + 1e-6) * np.abs(want)
             + 2.0 ** -150).all()
+
+
+@pytest.mark.parametrize("queries", [np.zeros(8, np.float32), np.float32(1.0),
+                                     [0.5] * 8])
+def test_queries_that_are_not_rows(queries):
+    """The error that numpy raises for their norms, on either device."""
+    index = VectorIndex()
+    index.add("a", "", np.ones(8, np.float32))
+    for device in ("cpu", "cuda:0"):
+        with pytest.raises(np.exceptions.AxisError):
+            index.search_batch_gpu(queries, 1, device=device)
