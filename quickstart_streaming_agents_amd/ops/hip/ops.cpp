@@ -93,6 +93,7 @@ extern "C" void qsa_skinny_gemm_fp8_launch(
     const unsigned short*, const float*, int, float, int, float*, int,
     hipStream_t);
 extern "C" int qsa_skinny_fp8_half(int, int, long long);
+extern "C" void qsa_skinny_fp8_block(int, int, long long, int, int, int*, int*);
 extern "C" int qsa_skinny_gemm_fp8_probe_launch(
     const unsigned short*, const unsigned char*, const float*,
     unsigned short*, int, int, long long, long long, int, int, int,
@@ -665,6 +666,14 @@ long skinny_gemm_fp8_parts(long M, long N, long K) {
   return N / (qsa_skinny_fp8_half((int)M, (int)N, K) ? 8 : 16);
 }
 
+// (waves, tiles of 16 columns) of a block
+std::tuple<int, int> skinny_gemm_fp8_block(long M, long N, long K, bool glu,
+                                           bool res) {
+  int waves, tiles;
+  qsa_skinny_fp8_block((int)M, (int)N, K, glu, res, &waves, &tiles);
+  return {waves, tiles};
+}
+
 std::vector<torch::Tensor> skinny_gemm_fp8_residual(
     torch::Tensor a, torch::Tensor qf, torch::Tensor scale, long N, long K,
     torch::Tensor res, torch::Tensor w, bool far) {
@@ -983,6 +992,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("a"), py::arg("ss"), py::arg("parts"), py::arg("M"),
         py::arg("eps"), py::arg("qf"), py::arg("scale"), py::arg("N"),
         py::arg("K"), py::arg("glu"), py::arg("far") = false);
+  m.def("skinny_gemm_fp8_block", &skinny_gemm_fp8_block,
+        "waves and tiles of a block of the fp8 stream");
   m.def("skinny_gemm_fp8_parts", &skinny_gemm_fp8_parts,
         "parts of a row's sum of squares behind a residual");
   m.def("skinny_gemm_fp8_residual", &skinny_gemm_fp8_residual,

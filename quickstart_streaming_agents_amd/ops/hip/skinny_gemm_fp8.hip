@@ -63,44 +63,60 @@ static void fp8_go(const SkinnyArgs& p, int pack, hipStream_t st) {
 // two tiles of columns as soon as 192 blocks are left (half the A reads per
 // weight).  Four tiles for a vocabulary, and from 16384 columns on where A is
 // two row tiles and costs more than the weights (28672 x 4096, 32 rows: 37 us
-// with two tiles, 29 with four).  With 9 to 16 rows, of which A
-// still is twice the weights, from 28672 on and K beyond 2048 (16 rows 24.5 us with two
-// tiles, 23.2 with four; 32768 x 3072 20.1 / 19.2, but 22016 x 4096 19.5 / 21.4, 32768 x
-// 2048 13.8 / 14.2).  12288 to 16384 columns are one block of four tiles for a CU, and
-// with eight waves (us at 16 / 24 rows, before -> so: 12288 x 2048 7.9 / 9.9 -> 7.3 / 7.8;
-// 16384 x 2048 8.6 / 9.9 -> 8.2 / 8.7; 16384 x 3072 11.5 / 12.8 -> 11.0 / 11.5; of 24 rows
-// 12288 x 1024 6.1 -> 5.4, 16384 x 4096 16.1 -> 15.6; but of 16 14.1 -> 16.8).
+// with two tiles, 29 with four).
+// With 9 to 16 rows A still is twice the weights, and four tiles of K beyond 2048 are
+// ahead from 24577 columns on where the CU with most blocks has no more tiles so than in
+// blocks of two: up to 32768, from 40961 to 49152 and 57345 to 65536 (us with two / four:
+// 25600 x 3072 18.7 / 16.8, 32768 21.1 / 19.2, but 24576 16.6 / 16.9, 36864 24.0 / 24.3
+// and of K 4096 29.5 / 32.2; 49152 x 5120 47.0 / 42.6; 61440 x 4096 45.4 / 43.3; of 160
+// shapes of K 2304 to 8192 the choice is 0.2 % from the best, at most 5 %).
+// 12288 to 16384 columns are one block of four tiles for a CU, and with eight waves (us
+// at 16 / 24 rows, eight waves of two tiles -> so: 12288 x 2048 7.9 / 9.9 -> 7.4 / 7.8;
+// 16384 x 3072 11.3 / 14.3 -> 10.6 / 11.3; of 24 rows 12288 x 1024 8.7 -> 5.6, 15360 x
+// 4096 17.4 -> 14.4; but of 16 13.9 -> 15.0, and 16384 x 4096 with 24 rows 16.2 in four
+// waves of four, 16.8 so).
 // us at 1 / 16 rows, one tile per block and row-major A before -> here (packed
 // from 5 rows on, norm or residual included): 6144 x 4096 13.1 / 14.2 -> 7.5 /
 // 8.6; 4096 x 4096 8.1 / 9.4 -> 6.2 / 7.2; 28672 x 4096 32 / 36 -> 24.6 / 27.9
 // with the gating; 4096 x 14336 22 / 25 -> 14.7 / 17.9; 128256 x 2048 57 / 62
 // -> 48.6 / 52.2 (5.4 TB/s).
+extern "C" void qsa_skinny_fp8_block(int M, int N, long long K, int glu, int res,
+                                     int* waves, int* tiles) {
+  const bool whole = N % (glu ? 128 : 64) == 0 && M > (glu ? 8 : 0) && !res;
+  const bool once = M > 8 && N >= 12288 && N <= 16384 &&
+                    (M > 16 ? K >= 1024 && (K != 4096 || N < 16384)
+                            : K >= 2048 && K <= 3072);
+  // tiles of the CU with most blocks, in blocks of four and of two
+  const bool even = (N + 16383) / 16384 * 4 == (N + 8191) / 8192 * 2;
+  const bool four = N >= 65536 || (M > 16 && N >= 16384) ||
+                    (M > 8 && K > 2048 && N > 24576 && even);
+  if (whole && (once || four)) {
+    *waves = once ? 8 : 4;
+    *tiles = 4;
+  } else if (glu) {
+    *waves = K <= 2048 ? 4 : 8;
+    *tiles = 2;
+  } else {
+    *tiles = N >= 6144 && N % 32 == 0 ? 2 : 1;
+    *waves = *tiles == 1 && K <= 2048 ? 4 : 8;
+  }
+}
+
 template <bool NORM, bool GLU, bool RES>
 static void fp8_any(const SkinnyArgs& p, int pack, hipStream_t st) {
-  // four tiles, of one block a CU or of more than three for two
-  const bool once = p.M > 8 && p.N >= 12288 && p.N <= 16384 &&
-                    (p.M > 16 ? p.K >= 1024 : p.K >= 2048 && p.K <= 3072);
-  const int four = p.M > 16 ? 16384 : p.M > 8 && p.K > 2048 ? 28672 : 65536;
+  int waves, tiles;
+  qsa_skinny_fp8_block(p.M, p.N, p.K, GLU, RES, &waves, &tiles);
+  if constexpr (!RES)
+    if (tiles == 4)
+      return waves == 8 ? fp8_go<8, 4, NORM, GLU, RES>(p, pack, st)
+                        : fp8_go<4, 4, NORM, GLU, RES>(p, pack, st);
   if constexpr (GLU) {
-    if (once && p.N % 128 == 0)
-      fp8_go<8, 4, NORM, GLU, RES>(p, pack, st);
-    else if (p.M > 8 && p.N >= four && p.N % 128 == 0)
-      fp8_go<4, 4, NORM, GLU, RES>(p, pack, st);
-    else if (p.K <= 2048) fp8_go<4, 2, NORM, GLU, RES>(p, pack, st);
+    if (waves == 4) fp8_go<4, 2, NORM, GLU, RES>(p, pack, st);
     else fp8_go<8, 2, NORM, GLU, RES>(p, pack, st);
   } else {
-    if constexpr (!RES) {
-      if (once && p.N % 64 == 0)
-        return fp8_go<8, 4, NORM, GLU, RES>(p, pack, st);
-      if (p.N >= four && p.N % 64 == 0)
-        return fp8_go<4, 4, NORM, GLU, RES>(p, pack, st);
-    }
-    if (p.N >= 6144 && p.N % 32 == 0)
-      fp8_go<8, 2, NORM, GLU, RES>(p, pack, st);
-    else if (p.K <= 2048)
-      fp8_go<4, 1, NORM, GLU, RES>(p, pack, st);
-    else
-      fp8_go<8, 1, NORM, GLU, RES>(p, pack, st);
+    if (tiles == 2) fp8_go<8, 2, NORM, GLU, RES>(p, pack, st);
+    else if (waves == 4) fp8_go<4, 1, NORM, GLU, RES>(p, pack, st);
+    else fp8_go<8, 1, NORM, GLU, RES>(p, pack, st);
   }
 }
 

@@ -105,6 +105,37 @@ def test_decode_attention_splits(rows, heads, pages, D):
     check(ext().paged_attn_decode(turned, kc, vc, bt, sl, D ** -0.5), turned)
 
 
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("K", [2304, 3072, 4096, 8192])
+def test_tiles_of_the_fp8_stream(K, glu):
+    """9 to 16 rows: four tiles a block where no CU gets more of them than in blocks
+    of two, and from 24577 columns on."""
+    def tiles(M, N, k=K):
+        return ext().skinny_gemm_fp8_block(M, N, k, glu, False)[1]
+
+    for M in (9, 16):
+        for N in (24_704, 28_672, 32_768, 41_088, 45_056, 49_152, 57_472, 65_536,
+                  131_072):
+            assert tiles(M, N) == 4, N
+        for N in (18_432, 24_576, 32_896, 36_864, 40_960, 49_280, 57_344):
+            assert tiles(M, N) == 2, N
+            assert tiles(M, N + 4096, 2048) == 2
+    for N in range(16_512, 131_072, 1664):
+        assert tiles(17, N) == tiles(32, N) == 4
+        assert tiles(8, N) == (2 if glu or N < 65_536 else 4)
+
+
+@pytest.mark.parametrize("M,N,K,block", [
+    (9, 12_288, 2048, (8, 4)), (16, 16_384, 3072, (8, 4)), (16, 14_336, 3328, (8, 2)),
+    (24, 12_288, 1024, (8, 4)), (24, 15_360, 4096, (8, 4)), (24, 16_384, 4096, (4, 4)),
+    (24, 16_384, 8192, (8, 4)), (8, 14_336, 2048, (8, 2)), (24, 12_160, 2048, (8, 2)),
+    (16, 16_400, 4096, (8, 1)), (3, 4096, 2048, (4, 1)), (3, 4096, 2304, (8, 1))])
+def test_blocks_of_the_fp8_stream(M, N, K, block):
+    assert ext().skinny_gemm_fp8_block(M, N, K, False, False) == block
+    if N >= 12_288 and N % 32 == 0:
+        assert ext().skinny_gemm_fp8_block(M, N, K, False, True) == (8, 2)
+
+
 @pytest.mark.parametrize("M,N,K", [
     (64, 12288, 8192), (64, 12288, 4096), (64, 16384, 2048), (33, 16384, 12288),
     (48, 14336, 4096), (64, 9216, 4096), (128, 8192, 4096)])
