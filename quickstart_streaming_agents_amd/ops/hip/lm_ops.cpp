@@ -1044,11 +1044,9 @@ struct WidePlan {
   int tile = 0, rows = 0, rest = 0;
   float us = 1e30f;
 };
-static WidePlan wide_plan(const Tensor& a, const Tensor& w, int act) {
+static WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int act) {
   WidePlan p;
-  const int64_t M = a.size(0), N = w.size(0), K = w.size(1);
-  if (M < 256 || (256 * a.stride(0) + K) * 2 >= (4ll << 30) ||
-      256 * N * 2 >= (4ll << 30))
+  if (M < 256 || (256 * lda + K) * 2 >= (4ll << 30) || 256 * N * 2 >= (4ll << 30))
     return p;
   p.us = qsa_wide_gemm_plan((int)M, (int)N, (int)K, act, &p.tile, &p.rows, &p.rest);
   return p;
@@ -1059,7 +1057,8 @@ static WidePlan wide_plan(const Tensor& a, const Tensor& w, int act) {
 // activation a pass of its own there), and at most 1.10 of it, where its division of K
 // over all CUs evens out a last turn of few tiles (4620 x 5568 x 5888).
 static bool wide_sizes(const Tensor& a, const Tensor& w, bool glu) {
-  return a.size(0) * w.size(0) > 9000000 && wide_plan(a, w, glu).us < 1e30f;
+  return a.size(0) * w.size(0) > 9000000 &&
+         wide_plan(a.size(0), w.size(0), w.size(1), a.stride(0), glu).us < 1e30f;
 }
 
 bool gemm_ok(const Tensor& a, const Tensor& w) {
@@ -1093,21 +1092,29 @@ static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
   return out.defined() ? out : part;
 }
 
-// The same by whichever of the two should be over first.  rows_gemm's estimate is of
+// Whichever of the two should be over first.  rows_gemm's estimate is of
 // CUs that keep their clock: where it comes within 14 % of the other's, the other is
 // sooner (of 200 shapes, M 200 to 45,000, the choice is then 0.5 % from the best).
+static WidePlan gemm_wide(int64_t M, int64_t N, int64_t K, int64_t lda, int act,
+                          bool parts) {
+  WidePlan p = wide_plan(M, N, K, lda, act);
+  if (p.us < 1e30f) {
+    int S;
+    float us;
+    qsa_rows_gemm_plan((int)M, (int)N, (int)K, act, parts, &S, &us);
+    if (us * 1.14f < p.us) p.us = 1e30f;
+  }
+  return p;
+}
+
 static Tensor gemm_run(const Tensor& a, const Tensor& w, int act, bool parts,
                        bool far) {
   CHK_DEV(a); CHK_SAME(a, w);
   TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
               "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
-  const WidePlan p = wide_plan(a, w, act);
-  if (p.us == 1e30f) return rows_gemm_run(a, w, act, parts, far);
   const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
-  int S;
-  float us;
-  qsa_rows_gemm_plan(M, N, K, act, parts, &S, &us);
-  if (us * 1.14f < p.us) return rows_gemm_run(a, w, act, parts, far);
+  const WidePlan p = gemm_wide(M, N, K, a.stride(0), act, parts);
+  if (p.us == 1e30f) return rows_gemm_run(a, w, act, parts, far);
   const int64_t cols = act ? N / 2 : N;
   Tensor out = torch::empty({M, cols}, a.options());
   qsa_wide_gemm_launch(u16(a), u16(w), u16m(out), p.rows, N, K, a.stride(0), p.tile,
@@ -1126,6 +1133,12 @@ std::tuple<int, int, int> wide_gemm_plan(int64_t M, int64_t N, int64_t K,
   if (qsa_wide_gemm_plan((int)M, (int)N, (int)K, glu, &tile, &rows, &rest) == 1e30f)
     tile = -1;
   return {tile, rows, rest};
+}
+
+// the same of a product as gemm() and glu_gemm() run it; -1: rows_gemm's
+std::tuple<int, int, int> gemm_plan(int64_t M, int64_t N, int64_t K, bool glu) {
+  const WidePlan p = gemm_wide(M, N, K, K, glu, false);
+  return {p.us < 1e30f ? p.tile : -1, p.rows, p.rest};
 }
 
 // a @ w^T by a tile of wide_gemm.hip, with act as in glu_gemm's kernels
@@ -1248,6 +1261,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("a"), py::arg("w"), py::arg("gelu"), py::arg("rounded"),
         py::arg("far") = false);
   m.def("glu_gemm_ok", &glu_gemm_ok, "whether a gated product is one of theirs");
+  m.def("gemm_plan", &gemm_plan, "the same where gemm() takes wide_gemm, else -1");
   m.def("wide_gemm", &wide_gemm, "GEMM of many rows by a given tile");
   m.def("wide_gemm_plan", &wide_gemm_plan, "tiles and rows of a product");
 }

@@ -61,14 +61,14 @@ def test_tiles(tile, act):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,tail", [(16, 0), (48, 16), (272, 16)])
-def test_columns_in_sixteens(N, tail):
+@pytest.mark.parametrize("N", [16, 48, 272])
+def test_columns_in_sixteens(N):
     for tile in range(len(TILES)):
         x, w = operands(300, N, 448)
         check(lm_ext().wide_gemm(x, w, tile, 0), x, w, 0)
 
 
-SPLIT = [(2213, 9216, 448), (3677, 6784, 1536), (5595, 4864, 512)]
+SPLIT = [(785, 21_248, 1536), (3666, 9888, 768), (8221, 4512, 768)]
 
 
 @pytest.mark.gpu
@@ -77,7 +77,9 @@ def test_by_the_rules(M, N, K):
     """As models call them: gated or not, and with rows apart."""
     x, w = operands(M, N, K, K ** -0.5)
     assert lm_ext().gemm_ok(x, w) and D.glu_linear_ok(x, w)
-    assert lm_ext().wide_gemm_plan(M, N, K, False)[1] < M
+    for glu in (False, True):
+        tile, rows, rest = lm_ext().gemm_plan(M, N, K, glu)
+        assert tile >= 0 and rows < M
     check(D.linear(x, w), x, w, 0)
     check(D.glu_linear(x, w), x, w, 1)
 
@@ -85,6 +87,7 @@ def test_by_the_rules(M, N, K):
 @pytest.mark.gpu
 def test_replayed():
     x, w = operands(1024, 10_240, 512)
+    assert lm_ext().gemm_plan(1024, 10_240, 512, False)[0] >= 0
     want = D.linear(x, w)
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
@@ -111,3 +114,11 @@ def test_plans(glu):
             apart += rows < M
     assert apart > 3
     assert lm_ext().wide_gemm_plan(1000, 1024, 128, glu)[0] == -1
+
+
+@pytest.mark.parametrize("M,N,K,glu", [
+    (18_556, 1536, 384, False), (2213, 9216, 448, False), (5034, 8192, 512, False),
+    (10_626, 2560, 640, False), (14_758, 3072, 384, True), (5595, 4864, 512, True)])
+def test_short_products_stay_whole(M, N, K, glu):
+    """A launch of its own for the last rows costs more than it saves."""
+    assert lm_ext().wide_gemm_plan(M, N, K, glu)[1] == M
