@@ -1052,25 +1052,36 @@ static WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int act)
   return p;
 }
 
-// Whether a product is wide_gemm.hip's where it is not rows_gemm.hip's by its size: in
-// 150 shapes from 30 us on the two take 0.86 of the library's time on average (the
-// activation a pass of its own there), and at most 1.10 of it, where its division of K
-// over all CUs evens out a last turn of few tiles (4620 x 5568 x 5888).
-static bool wide_sizes(const Tensor& a, const Tensor& w, bool glu) {
-  return a.size(0) * w.size(0) > 9000000 &&
-         wide_plan(a.size(0), w.size(0), w.size(1), a.stride(0), glu).us < 1e30f;
+// Whether a product is wide_gemm.hip's where it is not rows_gemm.hip's by its size.
+// With the activation, a pass of its own beside the library's product, it takes 0.91
+// of that time (157 products of M 300 to 30,000), at most 1.02.  Plain ones take 0.93
+// (260 of M 256 to 46,000), but which way depends on the library, that is uneven:
+// 0.50 (3000 x 3584 x 18944) to 1.13.  It is ahead where tiles of 256 x 256 come in whole
+// turns of the 256 CUs: there 77 products took 1.04 of its time (8192 x 4096 x 4096
+// 178 / 186 us, 20,480 x 8192 x 8192 1753 / 1849; of K up to 1024 0.99), and these stay
+// with it.  Left are 1.05 to 1.13 in 30 of 260, full but for part of one turn (2048 x
+// 28672 x 4096 328 / 363, 13,800 x 2048 x 8192 318 / 340), beside products as full that
+// the library takes 1.1 to 1.7 times as long for (10,816 x 4096 x 4096, 7500 x 4096 x
+// 14336, 20,000 x 4096 x 4096).
+static bool wide_sizes(int64_t M, int64_t N, int64_t K, int64_t lda, bool glu) {
+  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+  return M * N > 9000000 && (glu || K <= 1024 || tiles % 256) &&
+         wide_plan(M, N, K, lda, glu).us < 1e30f;
+}
+
+// Whether a product of these sizes is one of the two's.
+static bool gemm_sizes(int64_t M, int64_t N, int64_t K, int64_t lda, bool glu) {
+  return rows_gemm_sizes(M, N, K, glu) || wide_sizes(M, N, K, lda, glu);
 }
 
 bool gemm_ok(const Tensor& a, const Tensor& w) {
   return gemm_takes(a, w, false) &&
-         (rows_gemm_sizes(a.size(0), w.size(0), w.size(1), false) ||
-          wide_sizes(a, w, false));
+         gemm_sizes(a.size(0), w.size(0), w.size(1), a.stride(0), false);
 }
 
 bool glu_gemm_ok(const Tensor& a, const Tensor& w) {
   return gemm_takes(a, w, true) &&
-         (rows_gemm_sizes(a.size(0), w.size(0), w.size(1), true) ||
-          wide_sizes(a, w, true));
+         gemm_sizes(a.size(0), w.size(0), w.size(1), a.stride(0), true);
 }
 
 // parts: a product whose K is split may stay in its shares, [S, M, N] f32; far: w is
@@ -1255,6 +1266,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm", &gemm, "rows_gemm or wide_gemm by size", py::arg("a"), py::arg("w"),
         py::arg("far") = false);
   m.def("gemm_ok", &gemm_ok, "whether a product is one of theirs");
+  m.def("gemm_sizes", &gemm_sizes, "the same by its sizes and the rows' distance",
+        py::arg("M"), py::arg("N"), py::arg("K"), py::arg("lda"), py::arg("glu"));
   m.def("gemm_parts", &gemm_parts, "the same, shares of K left to the reader",
         py::arg("a"), py::arg("w"), py::arg("far") = false);
   m.def("glu_gemm", &glu_gemm, "the same with the gated activation inside",

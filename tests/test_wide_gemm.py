@@ -122,3 +122,15 @@ def test_plans(glu):
 def test_short_products_stay_whole(M, N, K, glu):
     """A launch of its own for the last rows costs more than it saves."""
     assert lm_ext().wide_gemm_plan(M, N, K, glu)[1] == M
+
+
+@pytest.mark.parametrize("M,N,K", [(8192, 4096, 4096), (8189, 4096, 4096),
+                                   (20_480, 8192, 8192), (2048, 16_384, 2048)])
+def test_whole_turns_are_the_library_s(M, N, K):
+    """Plain products whose tiles of 256 x 256 fill the chip so many times; not those
+    of one row more, of short K, or with the activation inside."""
+    def ours(m, k=K, glu=False):
+        return lm_ext().gemm_sizes(m, N, k, k, glu)
+
+    assert not ours(M) and ours(M, glu=True)
+    assert ours(M // 256 * 256 + 257) and ours(M, 1024)
