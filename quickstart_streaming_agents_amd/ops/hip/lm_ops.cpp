@@ -1038,18 +1038,12 @@ bool rows_gemm_ok(const Tensor& a, const Tensor& w) {
          rows_gemm_sizes(a.size(0), w.size(0), w.size(1), false);
 }
 
-// What wide_gemm.hip would do with a product; its offsets are of whole tiles.  Decode
-// batches, bound by the read of W, are not looked at.
-struct WidePlan {
-  int tile = 0, rows = 0, rest = 0;
-  float us = 1e30f;
-};
-static WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int act) {
-  WidePlan p;
-  if (M < 256 || (256 * lda + K) * 2 >= (4ll << 30) || 256 * N * 2 >= (4ll << 30))
-    return p;
-  p.us = qsa_wide_gemm_plan((int)M, (int)N, (int)K, act, &p.tile, &p.rows, &p.rest);
-  return p;
+// Whether wide_gemm.hip can do a product, whose first tile takes the shortest K; its
+// offsets are of whole tiles.  Decode batches, bound by the read of W, are not looked
+// at.
+static bool wide_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int act) {
+  return M >= 256 && (256 * lda + K) * 2 < (4ll << 30) &&
+         256 * N * 2 < (4ll << 30) && qsa_wide_gemm_fits(0, (int)K, act);
 }
 
 // Whether a product is wide_gemm.hip's where it is not rows_gemm.hip's by its size.
@@ -1066,7 +1060,7 @@ static WidePlan wide_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int act)
 static bool wide_sizes(int64_t M, int64_t N, int64_t K, int64_t lda, bool glu) {
   const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
   return M * N > 9000000 && (glu || K <= 1024 || tiles % 256) &&
-         wide_plan(M, N, K, lda, glu).us < 1e30f;
+         wide_takes(M, N, K, lda, glu);
 }
 
 // Whether a product of these sizes is one of the two's.
@@ -1084,16 +1078,40 @@ bool glu_gemm_ok(const Tensor& a, const Tensor& w) {
          gemm_sizes(a.size(0), w.size(0), w.size(1), a.stride(0), true);
 }
 
-// parts: a product whose K is split may stay in its shares, [S, M, N] f32; far: w is
-// read past the last-level cache, where each of its numbers is read once
-static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
-                            bool parts = false, bool far = false) {
+// How a product is run.  wide: wide_gemm's tile, the rows that it takes and the tile of
+// the rest; else rows_gemm's tile and shares of K.
+struct GemmPlan {
+  bool wide = false;
+  int tile = 0, rows = 0, rest = 0, shares = 1;
+};
+
+// Whichever of the two should be over first, each asked once.  rows_gemm's estimate is
+// of CUs that keep their clock: where it comes within 14 % of the other's, the other is
+// sooner (of 200 shapes, M 200 to 45,000, the choice is then 0.5 % from the best).
+static GemmPlan gemm_choice(int64_t M, int64_t N, int64_t K, int64_t lda, int act,
+                            bool parts) {
+  GemmPlan p;
+  float rows_us, wide_us = 1e30f;
+  p.tile = qsa_rows_gemm_plan((int)M, (int)N, (int)K, act, parts, &p.shares, &rows_us);
+  if (!wide_takes(M, N, K, lda, act)) return p;
+  int tile;
+  wide_us = qsa_wide_gemm_plan((int)M, (int)N, (int)K, act, &tile, &p.rows, &p.rest);
+  p.wide = wide_us < 1e30f && rows_us * 1.14f >= wide_us;
+  if (p.wide) p.tile = tile;
+  return p;
+}
+
+static void chk_product(const Tensor& a, const Tensor& w, int act) {
   CHK_DEV(a); CHK_SAME(a, w);
   TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
               "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
+}
+
+// parts: a product whose K is split may stay in its shares, [S, M, N] f32; far: w is
+// read past the last-level cache, where each of its numbers is read once
+static Tensor rows_gemm_by(const Tensor& a, const Tensor& w, int act, bool parts,
+                           bool far, int tile, int S) {
   const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
-  int S;
-  const int tile = qsa_rows_gemm_plan(M, N, K, act, parts, &S, nullptr);
   Tensor out, part;
   if (S > 1) part = torch::empty({S, M, N}, a.options().dtype(at::kFloat));
   if (S == 1 || !parts) out = torch::empty({M, act ? N / 2 : N}, a.options());
@@ -1103,29 +1121,21 @@ static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
   return out.defined() ? out : part;
 }
 
-// Whichever of the two should be over first.  rows_gemm's estimate is of
-// CUs that keep their clock: where it comes within 14 % of the other's, the other is
-// sooner (of 200 shapes, M 200 to 45,000, the choice is then 0.5 % from the best).
-static WidePlan gemm_wide(int64_t M, int64_t N, int64_t K, int64_t lda, int act,
-                          bool parts) {
-  WidePlan p = wide_plan(M, N, K, lda, act);
-  if (p.us < 1e30f) {
-    int S;
-    float us;
-    qsa_rows_gemm_plan((int)M, (int)N, (int)K, act, parts, &S, &us);
-    if (us * 1.14f < p.us) p.us = 1e30f;
-  }
-  return p;
+static Tensor rows_gemm_run(const Tensor& a, const Tensor& w, int act,
+                            bool parts = false, bool far = false) {
+  chk_product(a, w, act);
+  int S;
+  const int tile = qsa_rows_gemm_plan((int)a.size(0), (int)w.size(0),
+                                      (int)w.size(1), act, parts, &S, nullptr);
+  return rows_gemm_by(a, w, act, parts, far, tile, S);
 }
 
 static Tensor gemm_run(const Tensor& a, const Tensor& w, int act, bool parts,
                        bool far) {
-  CHK_DEV(a); CHK_SAME(a, w);
-  TORCH_CHECK(rows_gemm_fits(a, w, act != 0), "bf16 a [M, K], w [N, K] with K % "
-              "64 and N % 16 (gated: 32), aligned rows less than 2^24 apart");
+  chk_product(a, w, act);
   const int M = (int)a.size(0), N = (int)w.size(0), K = (int)w.size(1);
-  const WidePlan p = gemm_wide(M, N, K, a.stride(0), act, parts);
-  if (p.us == 1e30f) return rows_gemm_run(a, w, act, parts, far);
+  const GemmPlan p = gemm_choice(M, N, K, a.stride(0), act, parts);
+  if (!p.wide) return rows_gemm_by(a, w, act, parts, far, p.tile, p.shares);
   const int64_t cols = act ? N / 2 : N;
   Tensor out = torch::empty({M, cols}, a.options());
   qsa_wide_gemm_launch(u16(a), u16(w), u16m(out), p.rows, N, K, a.stride(0), p.tile,
@@ -1148,8 +1158,8 @@ std::tuple<int, int, int> wide_gemm_plan(int64_t M, int64_t N, int64_t K,
 
 // the same of a product as gemm() and glu_gemm() run it; -1: rows_gemm's
 std::tuple<int, int, int> gemm_plan(int64_t M, int64_t N, int64_t K, bool glu) {
-  const WidePlan p = gemm_wide(M, N, K, K, glu, false);
-  return {p.us < 1e30f ? p.tile : -1, p.rows, p.rest};
+  const GemmPlan p = gemm_choice(M, N, K, K, glu, false);
+  return {p.wide ? p.tile : -1, p.rows, p.rest};
 }
 
 // a @ w^T by a tile of wide_gemm.hip, with act as in glu_gemm's kernels

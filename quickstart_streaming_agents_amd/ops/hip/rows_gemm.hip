@@ -390,9 +390,11 @@ extern "C" int qsa_rows_gemm_plan(int M, int N, int K, int act, int cheap,
       float run = (float)turns * ((few ? t.own_few : t.own) +
                                   stage * ((all + S - 1) / S));
       if (t.pair && turns == 1) run += 1.5f;      // neither end beside another
+      const float after = S > 1 ? sum + each * S : 0.f;
+      if (run + after >= best) continue;          // no root makes it less
       const float r2 = run * run, m2 = mem * mem;
-      const float us = (few ? sqrtf(r2 + m2) : sqrtf(sqrtf(r2 * r2 + m2 * m2))) +
-                       (S > 1 ? sum + each * S : 0.f);
+      const float us =
+          (few ? sqrtf(r2 + m2) : sqrtf(sqrtf(r2 * r2 + m2 * m2))) + after;
       if (us < best) { best = us; tile = i; *shares = S; }
     }
   }

@@ -303,11 +303,16 @@ constexpr int WIDE_TILES = sizeof(wide_tiles) / sizeof(*wide_tiles);
 
 static float pow6(float x) { return x * x * x * x * x * x; }
 
-// What a tile should take for a product, us: the turns that the blocks of a die
-// take, the energy of all stages, or the way from memory, whichever binds.
-static float wide_us(const WideTile& t, int M, int N, int K, bool act) {
+// Whether a tile can do a product.
+static bool wide_fits(const WideTile& t, int K, bool act) {
+  return K >> 6 >= 2 * t.pa - 1 && !(act && t.nt % 4);
+}
+
+// What a tile should take for a product, us without some 2, to the power of 6: the
+// turns that the blocks of a die take, the energy of all stages, or the way from memory,
+// whichever binds.  Roots cost more than all the rest: only the best has one.
+static float wide_pow(const WideTile& t, int M, int N, int K, bool act) {
   const int stages = K >> 6;
-  if (stages < 2 * t.pa - 1 || (act && t.nt % 4)) return 1e30f;
   const long long tiles = (long long)((M + 32 * t.mt - 1) / (32 * t.mt)) *
                           ((N + 32 * t.nt - 1) / (32 * t.nt));
   const long long turns = ((tiles + 7) / 8 + 31) / 32;
@@ -316,16 +321,18 @@ static float wide_us(const WideTile& t, int M, int N, int K, bool act) {
   const float all = t.full * (float)stages * (float)tiles * (1.f / 256);
   const float mem = 2e-6f / 5.14f * ((float)N * K + (float)M * K +
                                      (float)M * N * (act ? 0.5f : 1.f));
-  return 2.f + powf(pow6(run) + pow6(all) + pow6(mem), 1.f / 6);
+  return pow6(run) + pow6(all) + pow6(mem);
 }
+static float wide_us(float pow) { return 2.f + cbrtf(sqrtf(pow)); }
 
 static float wide_best(int M, int N, int K, bool act, int* tile) {
-  float best = 1e30f;
+  float best = INFINITY;
   for (int i = 0; i < WIDE_TILES; ++i) {
-    const float us = wide_us(wide_tiles[i], M, N, K, act);
-    if (us < best) { best = us; *tile = i; }
+    if (!wide_fits(wide_tiles[i], K, act)) continue;
+    const float pow = wide_pow(wide_tiles[i], M, N, K, act);
+    if (pow < best) { best = pow; *tile = i; }
   }
-  return best;
+  return best < INFINITY ? wide_us(best) : 1e30f;
 }
 
 // The tile that should be over first, the rows that it takes and the tile of the
@@ -343,10 +350,13 @@ extern "C" float qsa_wide_gemm_plan(int M, int N, int K, int act, int* tile,
     const int bm = 32 * wide_tiles[i].mt, bn = 32 * wide_tiles[i].nt;
     const long long nb = (N + bn - 1) / bn, tiles = (M + bm - 1) / bm * nb;
     const int part = (int)(tiles / 256 * 256 / nb) * bm;
-    if (tiles <= 256 || part == 0 || part >= M) continue;
+    if (tiles <= 256 || part == 0 || part >= M ||
+        !wide_fits(wide_tiles[i], K, act))
+      continue;
+    const float first = wide_us(wide_pow(wide_tiles[i], part, N, K, act)) + 2.f;
+    if (first >= best) continue;
     int t;
-    const float us = wide_us(wide_tiles[i], part, N, K, act) +
-                     wide_best(M - part, N, K, act, &t) + 2.f;
+    const float us = first + wide_best(M - part, N, K, act, &t);
     if (us < best) { best = us; *tile = i; *rows = part; *rest = t; }
   }
   return best;
@@ -354,7 +364,7 @@ extern "C" float qsa_wide_gemm_plan(int M, int N, int K, int act, int* tile,
 
 extern "C" bool qsa_wide_gemm_fits(int tile, int K, int act) {
   return tile >= 0 && tile < WIDE_TILES &&
-         wide_us(wide_tiles[tile], 1, 16, K, act != 0) < 1e30f;
+         wide_fits(wide_tiles[tile], K, act != 0);
 }
 
 // act: 0, or an ACT_ of the first half of W's rows times the second
