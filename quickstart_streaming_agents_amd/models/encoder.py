@@ -92,10 +92,10 @@ class EmbeddingEncoder:
         """x W^T (`parts`: for the residual's norm), with glu silu(gate) * up of
         it, w = [gate; up] (GPU).  Few tiles are short_gemm's
         (ops/hip/short_gemm.hip: 384 x 512 at 400 rows 4.3 us, 4.5 in rows_gemm,
-        5.5 in the library), the others rows_gemm's: at 8800 rows 1536 x 384
-        takes 17.0 us (short_gemm 20.7, the library 18.3), 3072 x 384 with the
-        activation 32 (36, 72 with a pass of its own), 384 x 512 8.0 (10.5,
-        10.7), 384 x 1536 14.6 (23.4, 17.2)."""
+        5.5 in the library), the others rows_gemm's or wide_gemm's: at 8800 rows
+        1536 x 384 takes 16.5 us (short_gemm 20.7, the library 18.3), 3072 x 384
+        with the activation 32 (36, 72 with a pass of its own), 384 x 512 7.4
+        (10.5, 10.7), 384 x 1536 14.1 (23.4, 17.2)."""
         n, k = w.shape
         if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
                 n % 32 == 0 and (k <= 512 or x.shape[0] <= 32) and \
@@ -114,7 +114,7 @@ class EmbeddingEncoder:
 
     def _linear_alone(self, x: torch.Tensor, w: torch.Tensor,
                       glu: bool = False, parts: bool = False) -> torch.Tensor:
-        """The same with qsa_hip alone: rows_gemm is qsa_lm_hip's."""
+        """The same with qsa_hip alone: the others are qsa_lm_hip's."""
         n, k = w.shape
         if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
                 n % 32 == 0 and (k <= 512 or x.shape[0] <= 2048):

@@ -203,20 +203,20 @@ def pack_weight_frag(w: torch.Tensor) -> torch.Tensor:
 
 
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether x[M,K] @ W^T is rows_linear's: a product short of the sizes that
-    a library's tiles need, where nobody looks at the operation itself (the
-    rules are in ops/hip/lm_ops.cpp)."""
+    """Whether x[M,K] @ W^T is rows_linear's by its sizes, where nobody looks at the
+    operation itself (the rules are in ops/hip/lm_ops.cpp)."""
     return x.is_cuda and type(x) is torch.Tensor and \
         lm_ext().rows_gemm_ok(x, w) and not torch.compiler.is_compiling()
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """The product by ops/hip/rows_gemm.hip, whatever its size; linear() chooses."""
     return lm_ext().rows_gemm(x, w)
 
 
 def _gemm_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether x[M,K] @ W^T is one of this framework's kernels': rows_linear's,
-    or of many rows (ops/hip/wide_gemm.hip)."""
+    """Whether x[M,K] @ W^T is one of this framework's kernels': rows_linear's or,
+    of many rows, mostly ops/hip/wide_gemm.hip's."""
     return x.is_cuda and type(x) is torch.Tensor and \
         lm_ext().gemm_ok(x, w) and not torch.compiler.is_compiling()
 

@@ -141,7 +141,7 @@ extern "C" void qsa_rows_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*,
     float*, int, int, int, long long, int, int, int, bool, hipStream_t);
 
 // Whether t [S, rows, cols] is a product of bf16 rows whose shares of K have not
-// been added (rows_parts)
+// been added (gemm_parts)
 static bool is_shares(const Tensor& t, const Tensor& like, int64_t rows,
                       int64_t cols) {
   if (t.dim() != 3) return false;
@@ -1006,7 +1006,9 @@ static bool rows_gemm_fits(const Tensor& a, const Tensor& w, bool glu) {
 // of 33 to 14000 it is 18 % faster than the library's on average while M N is at most
 // 9 million, and as 15 pairs with M of 1 to 32 13 % (6144 x 4096 alone, which the packed
 // stream has, is up to 8 % behind).  With K up to 768 the library's are not yet in
-// their stride: 8800 x 4096 x 512 takes 46 us for 75.
+// their stride: 8800 x 4096 x 512 takes 46 us for 75.  Beyond these lines, and gated
+// beyond 48 million of longer K, wide_gemm is asked (wide_sizes) and, where it cannot,
+// with fewer than 256 rows or rows too far apart, the library.
 // The activation inside leaves K whole: where a plain product is this kernel's too and
 // few blocks would split it, that and a launch for the activation
 // is sooner (33 x 2048 x 16384 22 us, inside 69, the library 27; 64 x 4096 x 8192
@@ -1036,6 +1038,11 @@ static bool gemm_takes(const Tensor& a, const Tensor& w, bool glu) {
 bool rows_gemm_ok(const Tensor& a, const Tensor& w) {
   return gemm_takes(a, w, false) &&
          rows_gemm_sizes(a.size(0), w.size(0), w.size(1), false);
+}
+
+bool rows_glu_ok(const Tensor& a, const Tensor& w) {
+  return gemm_takes(a, w, true) &&
+         rows_gemm_sizes(a.size(0), w.size(0), w.size(1), true);
 }
 
 // Whether wide_gemm.hip can do a product, whose first tile takes the shortest K; its
@@ -1186,7 +1193,8 @@ std::tuple<int, int> rows_gemm_plan(int64_t M, int64_t N, int64_t K,
   return {tile, S};
 }
 
-// a @ w^T on W as it is stored
+// a @ w^T on W as it is stored.  These run rows_gemm.hip whatever the size, for its
+// tests and for comparisons; models go through gemm() and its like below.
 Tensor rows_gemm(Tensor a, Tensor w, bool far) {
   return rows_gemm_run(a, w, 0, false, far);
 }
@@ -1273,6 +1281,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "whether sizes are rows_gemm's, or with the activation inside");
   m.def("rows_gemm_plan", &rows_gemm_plan, "tile and shares of a product");
   m.def("rows_glu", &rows_glu, "the same with the gated activation inside");
+  m.def("rows_glu_ok", &rows_glu_ok, "whether a gated product is rows_glu's");
   m.def("gemm", &gemm, "rows_gemm or wide_gemm by size", py::arg("a"), py::arg("w"),
         py::arg("far") = false);
   m.def("gemm_ok", &gemm_ok, "whether a product is one of theirs");

@@ -134,3 +134,25 @@ def test_whole_turns_are_the_library_s(M, N, K):
 
     assert not ours(M) and ours(M, glu=True)
     assert ours(M // 256 * 256 + 257) and ours(M, 1024)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(40, 2048, 1024), (9000, 28_672, 3136)])
+def test_rows_gemm_s_own_rules(M, N, K):
+    """What is rows_gemm's by its sizes, whatever wide_gemm takes."""
+    x, w = (torch.empty(n, K, dtype=BF, device=DEV) for n in (M, N))
+    for ok, glu in ((lm_ext().rows_gemm_ok, False), (lm_ext().rows_glu_ok, True)):
+        assert ok(x, w) == lm_ext().rows_gemm_sizes(M, N, K, glu) == (M == 40)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [1, 2, 3])
+@pytest.mark.parametrize("M,N,K", [
+    (257, 6144, 1088), (330, 10_080, 128), (330, 12_288, 192), (300, 16_416, 576),
+    (700, 9696, 832), (385, 16_384, 704), (1000, 8864, 576), (1159, 9376, 128),
+    (1283, 8128, 1600), (1500, 6176, 1024), (1700, 8192, 256), (2100, 4096, 576)])
+def test_rows_gemm_s_gated_tiles(M, N, K, act):
+    """Gated products of many rows by rows_gemm.hip, where the rules may take
+    wide_gemm.hip."""
+    x, w = operands(M, N, K, K ** -0.5)
+    check(lm_ext().rows_glu(x, w, act == 2, act != 3), x, w, act)
