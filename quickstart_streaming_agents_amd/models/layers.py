@@ -15,7 +15,7 @@ from ..ops import dispatch as D
 class Linear:
     """y = x W^T.  On the GPU in bf16, the fewest rows of the small shapes stream
     a packed copy of W (ops/hip/skinny_gemm.hip), the others are ops/hip/rows_gemm.hip's
-    or, of many rows, ops/hip/wide_gemm.hip's; what these refuse is a vendor GEMM.
+    or, of many rows, mostly ops/hip/wide_gemm.hip's; the rest is a vendor GEMM.
 
     The stream's time grows with the rows, rows_gemm's does not, but splitting K
     for few columns costs it a launch where no reader adds the shares.  With the
