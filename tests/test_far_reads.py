@@ -69,6 +69,31 @@ def test_keys_that_are_there(dim, over, fuse):
     assert torch.equal(kc, halves[0]) and torch.equal(vc, halves[1])
 
 
+def test_replays_on_either_side():
+    """A captured call reads as many keys as there are at each replay."""
+    torch.manual_seed(9)
+    rows, heads, pages, dim = 66, 8, 3, 128
+    line = (32 << 20) // (heads * dim * 4)
+    bt = torch.randint(0, 40, (rows, pages), device=DEV, dtype=torch.int32)
+    sl = torch.ones(rows, device=DEV, dtype=torch.int32)
+    kc, vc = rnd(40, heads, dim // 8, 64, 8), rnd(40, heads, dim, 64)
+    q = rnd(rows, 4 * heads, dim)
+
+    def run(i):
+        return ext().paged_attn_decode(q[i], kc, vc, bt[i], sl[i], dim ** -0.5)
+
+    run(slice(0, rows))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        got = run(slice(0, rows))
+    for n in (1, pages * 64, 100, line // rows, line // rows + 1, 150):
+        sl.fill_(n)
+        got.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, torch.cat([run(slice(0, 33)), run(slice(33, 66))]))
+
+
 @pytest.mark.parametrize("over", [-1, 0, 1])
 def test_keys_of_grouped_rows_that_are_there(over):
     """The same of grouped rows; lengths beyond the table count as its width."""
