@@ -251,14 +251,22 @@ class ConvAttention:
         c = (shard.heads(m["heads"]) + g) * m["dim"] + g * m["vdim"]
         return {"kv": (g, m["dim"], m["vdim"]), "tail": (m["conv"] - 1, c)}
 
+    def conv_args(self, x: torch.Tensor, plan: StepPlan, kv, run: int,
+                  tails: torch.Tensor) -> tuple:
+        return (x[:, :self.channels], self.filters, tails, self.rope.cos,
+                self.rope.sin, self.rot, plan.cache_slots, kv.keys[run],
+                kv.values[run], self.H)
+
     def __call__(self, x: torch.Tensor, plan: StepPlan, kv, run: int,
                  tails: torch.Tensor, y: torch.Tensor) -> None:
+        q = D.conv_qkv(*self.conv_args(x, plan, kv, run, tails), *plan.conv)
+        self.attend(q, x, plan, kv, run, y)
+
+    def attend(self, q: torch.Tensor, x: torch.Tensor, plan: StepPlan, kv,
+               run: int, y: torch.Tensor) -> None:
         c = self.channels
         k, v = kv.keys[run], kv.values[run]
         gate = x[:, c:c + self.width]
-        q = D.conv_qkv(x[:, :c], self.filters, tails, self.rope.cos,
-                       self.rope.sin, self.rot, plan.cache_slots, k, v,
-                       self.H, *plan.conv)
         rows = plan.attn_rows(self.longest)
         n = rows.n
         if n:
@@ -304,8 +312,11 @@ class StateSpace:
         self.norm = shard.rows(get("norm")).float() * float(out_scale)
         self.out = shard.cols(get("o"))
         self.channels = self.filters.shape[1]
-        self.chunked = self.rows.is_cuda and dtype == torch.bfloat16 and \
-            D.ssd_chunked_ok(self.H, self.N, self.P, self.G)
+        fast = self.rows.is_cuda and dtype == torch.bfloat16
+        self.chunked = fast and D.ssd_chunked_ok(self.H, self.N, self.P,
+                                                 self.G)
+        self.whole = fast and D.ssd_step_ok(self.H, self.N, self.P, self.G,
+                                            self.parts, self.filters.shape[0])
 
     @staticmethod
     def shapes(m: dict, width: int) -> dict[str, tuple[int, ...]]:
@@ -321,6 +332,15 @@ class StateSpace:
         c = h * m["vdim"] + 2 * shard.heads(m["groups"]) * m["state"]
         return {"state": (h, m["state"], m["vdim"]),
                 "tail": (m["conv"] - 1, c)}
+
+    def step(self, u: torch.Tensor, plan: StepPlan, kv, run: int,
+             tails: torch.Tensor, y: torch.Tensor, beside: tuple
+             ) -> torch.Tensor:
+        """Single tokens, and the attention's convolutions beside them."""
+        return D.ssd_step(*beside, u, self.filters, self.bias, tails, self.A,
+                          self.dt_bias, self.skip, kv.states[run], self.G,
+                          self.norm, self.eps, y, plan.one_slots,
+                          plan.one_lens)
 
     def __call__(self, u: torch.Tensor, plan: StepPlan, kv, run: int,
                  tails: torch.Tensor, y: torch.Tensor) -> None:
@@ -374,6 +394,10 @@ class Parallel:
         self.at = at[1]
         self.proj = Linear(torch.cat(rows))
         self.out = shard.out(torch.cat([self.left.out, self.right.out], 1))
+        a = self.left
+        # steps of single tokens in one launch beside the attention
+        self.whole = self.right.whole and a.filters.shape[0] <= 4 and \
+            a.D % 4 == a.E % 4 == a.rot % 8 == 0
         del self.left.out, self.right.out
 
     @staticmethod
@@ -395,6 +419,13 @@ class Parallel:
         wl, wr = self.left.width, self.right.width
         y = torch.empty(plan.n_rows, wl + wr, dtype=h.dtype, device=h.device)
         tails = kv.tails[run]
+        if plan.items is None and self.whole:
+            u = x[:, :self.at]
+            q = self.right.step(
+                x[:, self.at:], plan, kv, run, tails[1], y[:, wl:],
+                self.left.conv_args(u, plan, kv, run, tails[0]))
+            self.left.attend(q, u, plan, kv, run, y[:, :wl])
+            return self.out(y)
         self.left(x[:, :self.at], plan, kv, run, tails[0], y[:, :wl])
         self.right(x[:, self.at:], plan, kv, run, tails[1], y[:, wl:])
         return self.out(y)

@@ -605,6 +605,24 @@ def ssd_decode(u, zoff: int, dtoff: int, xbc, A, dt_bias, D, state,
     return out
 
 
+def ssd_step_ok(h: int, n: int, p: int, groups: int, parts: int,
+                taps: int) -> bool:
+    return lm_ext().ssd_step_ok(h, n, p, groups, parts, taps)
+
+
+def ssd_step(x, qfilters, qtails, cos_t, sin_t, rot: int, cache_slots, kc, vc,
+             heads: int, u, filters, bias, tails, A, dt_bias, D, state,
+             groups: int, norm, eps: float, out, slots,
+             seq_lens) -> torch.Tensor:
+    """Single tokens of a parallel layer in one launch (GPU, bf16): conv_qkv of
+    x, and conv_silu, ssd_decode and part_norm of u's columns
+    [z | x | B | C | dt] to rows of out.  Returns q."""
+    return lm_ext().ssd_step(x, qfilters, qtails, cos_t, sin_t, rot,
+                             cache_slots, kc, vc, heads, u, filters, bias,
+                             tails, A, dt_bias, D, state, groups, norm, eps,
+                             out, slots, seq_lens)
+
+
 def ssd_seq(u, zoff: int, dtoff: int, xbc, A, dt_bias, D, state, groups: int,
             slots, off, start, len_, out) -> None:
     """Portions of several tokens, token by token (any size and type)."""

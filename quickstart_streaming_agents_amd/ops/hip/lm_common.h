@@ -39,6 +39,11 @@ template <typename T, int VEC>
 __device__ __forceinline__ void ldv(const T* p, float* v) {
   if constexpr (VEC == 1) {
     v[0] = ldf<T>(p);
+  } else if constexpr (VEC == 2) {
+    float2 f;
+    if constexpr (sizeof(T) == 4) f = *reinterpret_cast<const float2*>(p);
+    else f = bf16x2_to_f32x2(*reinterpret_cast<const unsigned int*>(p));
+    v[0] = f.x; v[1] = f.y;
   } else if constexpr (sizeof(T) == 4) {
 #pragma unroll
     for (int i = 0; i < VEC; i += 4) {
@@ -58,6 +63,11 @@ template <typename T, int VEC>
 __device__ __forceinline__ void stv(T* p, const float* v) {
   if constexpr (VEC == 1) {
     stf<T>(p, v[0]);
+  } else if constexpr (VEC == 2) {
+    if constexpr (sizeof(T) == 4)
+      *reinterpret_cast<float2*>(p) = make_float2(v[0], v[1]);
+    else
+      *reinterpret_cast<unsigned int*>(p) = cvt_bf16x2(v[0], v[1]);
   } else if constexpr (sizeof(T) == 4) {
 #pragma unroll
     for (int i = 0; i < VEC; i += 4)

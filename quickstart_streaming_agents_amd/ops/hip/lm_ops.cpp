@@ -8,7 +8,7 @@
 #include <ATen/hip/HIPContext.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 
-typedef unsigned short bf16_t;
+#include "step_args.h"
 
 #define CHK_DEV(t) TORCH_CHECK((t).is_cuda(), #t " must be on the GPU")
 #define CHK_CONT(t) TORCH_CHECK((t).is_contiguous(), #t " must be contiguous")
@@ -41,11 +41,6 @@ static inline bf16_t* u16m(const Tensor& t) {
   return reinterpret_cast<bf16_t*>(t.data_ptr());
 }
 
-// a step's rows for the short convolutions (ops/hip/short_conv.hip)
-struct ConvStep {
-  const int *item, *t0, *off, *start, *len, *slots;
-};
-
 extern "C" void qsa_residual_norm_launch(float*, const void*, long long,
     const float*, int, const void*, const void*, const long long*, float, const void*,
     const void*, const void*, void*, long long, int, int, float, int, int,
@@ -56,9 +51,7 @@ extern "C" void qsa_glu_launch(const void*, const float*, int, const void*,
     const long long*,
     void*, long long, long long, long long, long long, long long, int, int,
     int, hipStream_t);
-extern "C" void qsa_conv_qkv_launch(const void*, long long, const float*, int,
-    void*, ConvStep, int, const float*, const float*, int, int, const int*,
-    void*, void*, void*, int, int, int, int, int, int, hipStream_t);
+extern "C" void qsa_conv_qkv_launch(ConvQkv, int, int, int, hipStream_t);
 extern "C" void qsa_conv_silu_launch(const void*, long long, const float*,
     const float*, int, void*, ConvStep, int, void*, int, int, int,
     hipStream_t);
@@ -77,6 +70,8 @@ extern "C" void qsa_gqa_portions_launch(const bf16_t*, const bf16_t*,
 extern "C" void qsa_ssd_decode_launch(const void*, long long, int, int,
     const void*, const float*, const float*, const float*, float*, const int*,
     const int*, void*, int, int, int, int, int, int, int, hipStream_t);
+extern "C" int qsa_ssd_step_rows(int, int, int, int, int, int);
+extern "C" void qsa_ssd_step_launch(SsdStep, hipStream_t);
 extern "C" void qsa_ssd_seq_launch(const void*, long long, int, int,
     const void*, const float*, const float*, const float*, float*, const int*,
     const int*, const int*, const int*, void*, int, int, int, int, int, int,
@@ -602,11 +597,13 @@ static void chk_conv(const Tensor& x, const Tensor& w, const Tensor& tails,
   TORCH_CHECK(x.size(1) >= C, "columns");
 }
 
-// x columns [q | k | v]; returns rotated q [T, H*D], k and v to their pages
-Tensor conv_qkv(Tensor x, Tensor w, Tensor tails, Tensor cos_t, Tensor sin_t,
-                long rot, Tensor cache_slots, Tensor kc, Tensor vc, long H,
-                OptTensor item, OptTensor t0, OptTensor off, Tensor start,
-                OptTensor len, Tensor slots) {
+// x columns [q | k | v] to rotated q [T, H*D], k and v to their pages: what the
+// kernels take, without the step
+static ConvQkv conv_qkv_args(const Tensor& x, const Tensor& w,
+                             const Tensor& tails, const Tensor& cos_t,
+                             const Tensor& sin_t, long rot,
+                             const Tensor& cache_slots, const Tensor& kc,
+                             const Tensor& vc, long H, Tensor& q, int* v4) {
   CHK_CONT(kc); CHK_CONT(vc); CHK_SAME(x, kc); CHK_SAME(x, vc);
   CHK_I32(cache_slots);
   TORCH_CHECK(kc.dim() == 4 && kc.size(2) == 64 && vc.dim() == 4 &&
@@ -626,19 +623,29 @@ Tensor conv_qkv(Tensor x, Tensor w, Tensor tails, Tensor cos_t, Tensor sin_t,
   }
   const long T = x.size(0);
   TORCH_CHECK(cache_slots.numel() == T, "one cache slot per row");
-  auto q = torch::empty({T, H * (long)D}, x.options());
-  if (T == 0) return q;
-  ConvStep st;
-  const int chunks = conv_step(st, item, t0, off, start, len, slots, T);
-  const int v4 = D % 4 == 0 && E % 4 == 0 && rot % 8 == 0 &&
-                 x.stride(0) % 4 == 0 && aligned(x, is_f32(x) ? 16 : 8);
-  qsa_conv_qkv_launch(x.data_ptr(), x.stride(0), w.data_ptr<float>(),
-                      (int)w.size(0), tails.data_ptr(), st, chunks,
-                      rot ? cos_t.data_ptr<float>() : nullptr,
-                      rot ? sin_t.data_ptr<float>() : nullptr, (int)rot,
-                      table_len, cache_slots.data_ptr<int>(), q.data_ptr(),
-                      kc.data_ptr(), vc.data_ptr(), (int)H, G, D, E,
-                      is_f32(x), v4, cur_stream());
+  q = torch::empty({T, H * (long)D}, x.options());
+  *v4 = D % 4 == 0 && E % 4 == 0 && rot % 8 == 0 && x.stride(0) % 4 == 0 &&
+        aligned(x, is_f32(x) ? 16 : 8);
+  return ConvQkv{x.data_ptr(), x.stride(0), w.data_ptr<float>(),
+                 (int)w.size(0), tails.data_ptr(), ConvStep{},
+                 rot ? cos_t.data_ptr<float>() : nullptr,
+                 rot ? sin_t.data_ptr<float>() : nullptr, (int)rot, table_len,
+                 cache_slots.data_ptr<int>(), q.data_ptr(), kc.data_ptr(),
+                 vc.data_ptr(), (int)H, G, D, E};
+}
+
+Tensor conv_qkv(Tensor x, Tensor w, Tensor tails, Tensor cos_t, Tensor sin_t,
+                long rot, Tensor cache_slots, Tensor kc, Tensor vc, long H,
+                OptTensor item, OptTensor t0, OptTensor off, Tensor start,
+                OptTensor len, Tensor slots) {
+  Tensor q;
+  int v4;
+  ConvQkv p = conv_qkv_args(x, w, tails, cos_t, sin_t, rot, cache_slots, kc,
+                            vc, H, q, &v4);
+  if (x.size(0) == 0) return q;
+  const int chunks = conv_step(p.step, item, t0, off, start, len, slots,
+                               x.size(0));
+  qsa_conv_qkv_launch(p, chunks, is_f32(x), v4, cur_stream());
   return q;
 }
 
@@ -873,6 +880,57 @@ Tensor ssd_decode(Tensor u, long zoff, long dtoff, Tensor xbc, Tensor A,
       seq_lens.data_ptr<int>(), out.data_ptr(), B, s.H, s.N, s.P, s.G,
       is_f32(u), v4, cur_stream());
   return out;
+}
+
+bool ssd_step_ok(long H, long N, long P, long G, long parts, long taps) {
+  return qsa_ssd_step_rows((int)H, (int)N, (int)P, (int)G, (int)parts,
+                           (int)taps) > 0;
+}
+
+// Single tokens of a parallel layer: x | u are columns of its projection's rows.  The
+// attention's convolutions (returns q, writes k and v to their pages), and the whole
+// state-space branch, its normed read-out to rows of out.
+Tensor ssd_step(Tensor x, Tensor qw, Tensor qtails, Tensor cos_t, Tensor sin_t,
+                long rot, Tensor cache_slots, Tensor kc, Tensor vc, long H,
+                Tensor u, Tensor w, Tensor bias, Tensor tails, Tensor A,
+                Tensor dt_bias, Tensor D, Tensor state, long G, Tensor norm,
+                double eps, Tensor out, Tensor slots, Tensor seq_lens) {
+  Tensor q;
+  int v4;
+  ConvQkv conv = conv_qkv_args(x, qw, qtails, cos_t, sin_t, rot,
+                                     cache_slots, kc, vc, H, q, &v4);
+  CHK_F32(state); CHK_F32(bias); CHK_F32(A); CHK_F32(dt_bias); CHK_F32(D);
+  CHK_F32(norm); CHK_SAME(u, x); CHK_SAME(u, out);
+  CHK_DEV(u); chk_rows(u, "u"); chk_rows(out, "out");
+  TORCH_CHECK(u.scalar_type() == at::kBFloat16, "bf16 storage");
+  TORCH_CHECK(state.dim() == 4, "state [slots, H, N, P]");
+  const int SH = (int)state.size(1), N = (int)state.size(2),
+            P = (int)state.size(3), B = (int)u.size(0);
+  const long inner = (long)SH * P, C = inner + 2 * G * N;
+  const Tensor xbc = u.narrow(1, inner, C);
+  chk_conv(xbc, w, tails, C);
+  TORCH_CHECK(ssd_step_ok(SH, N, P, G, G, w.size(0)) && conv.taps <= 4,
+              "sizes of the step");
+  TORCH_CHECK(bias.numel() == C && A.numel() == SH && dt_bias.numel() == SH &&
+                  D.numel() == SH && norm.numel() == inner, "constants");
+  TORCH_CHECK(x.size(0) == B && out.size(0) == B && out.size(1) == inner &&
+                  u.size(1) >= inner + C + SH, "rows and columns");
+  conv_step(conv.step, c10::nullopt, c10::nullopt,
+            c10::nullopt, seq_lens, c10::nullopt, slots, B);
+  TORCH_CHECK(v4 && u.stride(0) % 4 == 0 && aligned(u, 8) &&
+                  out.stride(0) % 4 == 0 && aligned(out, 8) &&
+                  aligned(norm, 16) && aligned(state, 16), "alignment");
+  if (B == 0) return q;
+  qsa_ssd_step_launch(
+      SsdStep{u16(u), u.stride(0), 0, (int)inner, (int)(inner + C),
+              w.data_ptr<float>(), bias.data_ptr<float>(), (int)w.size(0),
+              u16m(tails), A.data_ptr<float>(), dt_bias.data_ptr<float>(),
+              D.data_ptr<float>(), norm.data_ptr<float>(),
+              state.data_ptr<float>(), slots.data_ptr<int>(),
+              seq_lens.data_ptr<int>(), u16m(out), out.stride(0), B, SH, N, P,
+              (int)G, (float)eps, 0, conv},
+      cur_stream());
+  return q;
 }
 
 void ssd_seq(Tensor u, long zoff, long dtoff, Tensor xbc, Tensor A,
@@ -1251,6 +1309,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gqa_mfma_ok", &gqa_mfma_ok, "size support");
   m.def("gqa_portion_rows", &gqa_portion_rows, "query rows per block");
   m.def("ssd_decode", &ssd_decode, "one token per row");
+  m.def("ssd_step", &ssd_step,
+        "single tokens of a parallel layer: convolutions, state and norm");
+  m.def("ssd_step_ok", &ssd_step_ok, "size support");
   m.def("ssd_seq", &ssd_seq, "token loop over portions");
   m.def("ssd_chunked", &ssd_chunked, "chunked prefill (MFMA)");
   m.def("ssd_chunked_ok", &ssd_chunked_ok, "size support");

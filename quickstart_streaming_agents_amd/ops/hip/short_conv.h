@@ -1,0 +1,248 @@
+// Device code of the short convolutions (short_conv.hip) that other kernels of a
+// decoding step share.
+#pragma once
+
+#include "lm_common.h"
+#include "step_args.h"
+
+#define CONV_ROWS 16  // tokens per thread; taps - 1 must not exceed it
+
+struct ConvSpan { int r0, t0, t1, n, p0, slot; };
+
+__device__ __forceinline__ ConvSpan conv_span(const ConvStep& st, int c) {
+  ConvSpan s;
+  if (st.item) {
+    const int it = st.item[c];
+    s.r0 = st.off[it];
+    s.t0 = st.t0[c];
+    s.n = st.len[it];
+    s.p0 = st.start[it];
+    s.slot = st.slots[it];
+    s.t1 = min(s.t0 + CONV_ROWS, s.n);
+  } else {
+    s.r0 = c;
+    s.t0 = 0;
+    s.n = s.t1 = 1;
+    s.p0 = st.start[c] - 1;
+    s.slot = st.slots[c];
+  }
+  return s;
+}
+
+// NP (1 or 2) groups of VEC channels, c0.. and c1..; TAPS 0: `taps` of them,
+// through memory.  pre(t) loads what emit(t, values, .) wants besides.
+template <typename T, int TAPS, int VEC, int NP, typename Pre, typename Emit>
+__device__ __forceinline__ void conv_rows(
+    const T* x, long long xstride, T* tail, int C, int c0, int c1,
+    const float* w, const float* bias, int taps, const ConvSpan& s, Pre pre,
+    Emit emit) {
+  const int NT = (TAPS ? TAPS : taps) - 1;
+  auto ch = [&](int p) { return p == 0 ? c0 : c1; };
+  auto load = [&](int t, int p, float* v) {
+    if (t >= 0) {
+      ldv<T, VEC>(x + (long long)(s.r0 + t) * xstride + ch(p), v);
+    } else if (s.p0 + t >= 0) {
+      ldv<T, VEC>(tail + (long long)(NT + t) * C + ch(p), v);
+    } else {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) v[i] = 0.f;
+    }
+  };
+  float b[NP][VEC];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    if (bias) {
+      ldv<float, VEC>(bias + ch(p), b[p]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) b[p][i] = 0.f;
+    }
+  }
+  if constexpr (TAPS > 0) {
+    constexpr int K = TAPS > 1 ? TAPS - 1 : 1;
+    float wt[NP][TAPS][VEC], win[NP][K][VEC];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j)
+        ldv<float, VEC>(w + (long long)j * C + ch(p), wt[p][j]);
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j)
+        load(s.t0 - (TAPS - 1) + j, p, win[p][j]);
+    }
+#pragma unroll 4
+    for (int t = s.t0; t < s.t1; ++t) {
+      const auto aux = pre(t);
+      float a[NP][VEC];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        float u[VEC];
+        ldv<T, VEC>(x + (long long)(s.r0 + t) * xstride + ch(p), u);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+          a[p][i] = b[p][i];
+#pragma unroll
+          for (int j = 0; j < TAPS - 1; ++j)
+            a[p][i] = fmaf(wt[p][j][i], win[p][j][i], a[p][i]);
+          a[p][i] = fmaf(wt[p][TAPS - 1][i], u[i], a[p][i]);
+#pragma unroll
+          for (int j = 0; j + 2 < TAPS; ++j) win[p][j][i] = win[p][j + 1][i];
+          win[p][K - 1][i] = u[i];
+        }
+      }
+      emit(t, a, aux);
+    }
+    if (s.t0 == 0 && s.t1 == s.n) {
+      // The whole portion, as of a single token: the window is the new tail.
+      // Moving entries in memory takes a round trip each (64 single tokens, four
+      // taps, 4096 channels to pages 8.7 us, 7.5 so, dense 5.8, 5.1).
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j)
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+          stv<T, VEC>(tail + (long long)j * C + ch(p), win[p][j]);
+      return;
+    }
+  } else {
+    for (int t = s.t0; t < s.t1; ++t) {
+      const auto aux = pre(t);
+      float a[NP][VEC];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) a[p][i] = b[p][i];
+        for (int j = 0; j <= NT; ++j) {
+          float u[VEC], wj[VEC];
+          load(t - NT + j, p, u);
+          ldv<float, VEC>(w + (long long)j * C + ch(p), wj);
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) a[p][i] = fmaf(wj[i], u[i], a[p][i]);
+        }
+      }
+      emit(t, a, aux);
+    }
+  }
+  if (s.t0 == 0) {
+    // entry j moves from n + j, never from a place already overwritten
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        float v[VEC];
+        load(s.n - NT + j, p, v);
+        stv<T, VEC>(tail + (long long)j * C + ch(p), v);
+      }
+  }
+}
+
+#define CONV_CASE(T, TAPS, VEC, NP)                                          \
+  conv_rows<T, TAPS, VEC, NP>(x, xstride, tail, C, c0, c1, w, bias, taps, s, \
+                              pre, emit)
+#define CONV_DISPATCH(T, VEC, NP)              \
+  switch (taps) {                              \
+    case 1: CONV_CASE(T, 1, VEC, NP); break;   \
+    case 2: CONV_CASE(T, 2, VEC, NP); break;   \
+    case 3: CONV_CASE(T, 3, VEC, NP); break;   \
+    case 4: CONV_CASE(T, 4, VEC, NP); break;   \
+    default: CONV_CASE(T, 0, VEC, NP);         \
+  }
+
+template <int VEC>
+struct Turn {
+  int slot;                    // where k or v goes
+  float c[VEC], s[VEC];
+};
+
+// A thread owns a pair of channel groups: of q and k a rotated pair (i,
+// i + rot/2) or two groups behind the rotated ones, of v two groups.
+// Pages: k [pages, G, 64, D], v [pages, G, 64, E].
+// units of a row
+__host__ __device__ inline int conv_qkv_units(const ConvQkv& p, int vec) {
+  return (p.H + p.G) * (p.rot / 2 / vec +
+                        (p.D - p.rot + 2 * vec - 1) / (2 * vec)) +
+         p.G * ((p.E + 2 * vec - 1) / (2 * vec));
+}
+
+// ONE: the step has one token per row and filters of up to CONV_ONE_TAPS taps
+#define CONV_ONE_TAPS 4
+template <typename T, int VEC, bool ONE = false>
+__device__ __forceinline__ void conv_qkv_unit(const ConvQkv& p, int chunk,
+                                              int u) {
+  const T* x = (const T*)p.x;
+  const long long xstride = p.xstride;
+  const float* __restrict__ w = p.w;
+  const int taps = p.taps, rot = p.rot, H = p.H, G = p.G, D = p.D, E = p.E;
+  const float* __restrict__ cos_t = p.cos_t;
+  const float* __restrict__ sin_t = p.sin_t;
+  const int table_len = p.table_len;
+  const int* __restrict__ cache_slots = p.cache_slots;
+  T *q = (T*)p.q, *kc = (T*)p.kc, *vc = (T*)p.vc;
+  const int half = rot >> 1;
+  const int ur = half / VEC, up = (D - rot + 2 * VEC - 1) / (2 * VEC);
+  const int ud = ur + up, ue = (E + 2 * VEC - 1) / (2 * VEC);
+  if (u >= (H + G) * ud + G * ue) return;
+  ConvSpan s;
+  if constexpr (ONE)
+    s = {chunk, 0, 1, 1, p.step.start[chunk] - 1, p.step.slots[chunk]};
+  else
+    s = conv_span(p.step, chunk);
+  if (s.slot < 0 || s.p0 < 0) return;
+  const int C = (H + G) * D + G * E;
+  T* tail = (T*)p.tails + (long long)s.slot * (taps - 1) * C;
+  const float* bias = nullptr;
+  const bool val = u >= (H + G) * ud;
+  const int un = val ? ue : ud;
+  const int r = (val ? u - (H + G) * ud : u) % un;
+  const int head = (val ? u - (H + G) * ud : u) / un;
+  const bool turn = !val && r < ur;
+  const int d0 = val || turn ? r * VEC : rot + (r - ur) * VEC;
+  const int far = d0 + (val ? ue * VEC : turn ? half : up * VEC);
+  const bool two = far < (val ? E : D);
+  const int d1 = two ? far : d0;
+  const int base = val ? (H + G) * D + head * E : head * D;
+  const int c0 = base + d0, c1 = base + d1;
+  const bool query = !val && head < H;
+  auto pre = [=](int t) {
+    Turn<VEC> r;
+    r.slot = query ? 0 : cache_slots[s.r0 + t];
+    if (turn) {
+      const long long at =
+          (long long)min(s.p0 + t, table_len - 1) * half + d0;
+      ldv<float, VEC>(cos_t + at, r.c);
+      ldv<float, VEC>(sin_t + at, r.s);
+    }
+    return r;
+  };
+  auto emit = [=](int t, float (&a)[2][VEC], const Turn<VEC>& r) {
+    const long long row = s.r0 + t;
+    if (turn) {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        const float u0 = a[0][i], v0 = a[1][i];
+        a[0][i] = u0 * r.c[i] - v0 * r.s[i];
+        a[1][i] = v0 * r.c[i] + u0 * r.s[i];
+      }
+    }
+    T* dst;
+    if (query) {
+      dst = q + (row * H + head) * D;
+    } else {
+      if (r.slot < 0) return;
+      const long long at = (long long)(r.slot >> 6) * G +
+                           (val ? head : head - H);
+      dst = val ? vc + (at * 64 + (r.slot & 63)) * E
+                : kc + (at * 64 + (r.slot & 63)) * D;
+    }
+    stv<T, VEC>(dst + d0, a[0]);
+    if (two) stv<T, VEC>(dst + d1, a[1]);
+  };
+  if constexpr (ONE) {
+    switch (taps) {
+      case 1: CONV_CASE(T, 1, VEC, 2); break;
+      case 2: CONV_CASE(T, 2, VEC, 2); break;
+      case 3: CONV_CASE(T, 3, VEC, 2); break;
+      case 4: CONV_CASE(T, 4, VEC, 2); break;
+    }
+  } else {
+    CONV_DISPATCH(T, VEC, 2)
+  }
+}

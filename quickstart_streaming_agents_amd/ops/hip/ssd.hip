@@ -12,6 +12,9 @@
 // Kernels
 //   qsa_ssd_decode   one token per row: step size, decay, update, read-out and
 //                    gate in one pass over the state (HBM-bound).
+//   qsa_ssd_step     the same for the heads of a group, with the convolution before
+//                    it, the norm behind it and the convolutions of the attention
+//                    beside it, where a step has single tokens only
 //   qsa_ssd_seq      token loop per (portion, head), any size and storage
 //                    type; the f32 path.
 //   chunked prefill (bf16 storage, matrix cores), chunks of 64 tokens; with
@@ -26,7 +29,7 @@
 //   cores (decayed x, state, intra-chunk weights) is a bf16 hi/lo pair, so the
 //   chunked result agrees with the token loop to about 2^-16.
 //   qsa_part_norm    rms norm in equal parts of a row, with a weight
-#include "lm_common.h"
+#include "short_conv.h"
 
 #define RC 64  // tokens per chunk
 #define LOG2E 1.4426950408889634f
@@ -148,6 +151,204 @@ extern "C" void qsa_ssd_decode_launch(
   else if (far) QSA_SD(bf16_t, 4, true);
   else QSA_SD(bf16_t, 4, false);
 #undef QSA_SD
+}
+
+// ---------------------------------------------------------------------------
+// One token per row, all of a state-space layer's columns of a group of heads, whose
+// norm part it is: the convolution and silu of its x, B and C, step sizes, decay,
+// update, read-out, gate and norm.  Blocks behind those do the attention's
+// convolutions (conv_qkv_unit), which depend on the projection alone as well: three
+// launches less, each some 5 us of latencies that the state's way from memory covers.
+// A thread has R rows of four columns of the state, which it asks for before anything
+// is waited for: 1024 threads hold a group's state of up to 256 KB, and two blocks
+// fit a CU up to R = 8.  us, 8 groups of 4 heads, states of 64 x 128, 64 rows: 4.9
+// (convolution) + 27.8 + 4.7 (norm) + 5.8 (the attention's convolutions) -> 30.6, 4.4
+// TB/s of state; 4 layers of width 2048, a step of 64 rows 707 -> 662, of 32 580 ->
+// 525, of 8 482 -> 414, of one 387 -> 339.
+// ---------------------------------------------------------------------------
+#define STEP_THREADS 1024
+#define STEP_COLS 512                  // most columns of a group
+#define STEP_TAPS 4
+#define STEP_VEC 2                     // channels of the attention's: few registers
+
+template <int R, bool FAR>
+__global__ void __launch_bounds__(STEP_THREADS, R <= 8 ? 8 : 4)
+qsa_ssd_step(SsdStep p) {
+  __shared__ f32x4_v red[STEP_THREADS];
+  __shared__ __attribute__((aligned(16))) float xs[STEP_COLS];
+  __shared__ float bc[STEP_THREADS];   // B and C of the group
+  __shared__ float dts[STEP_COLS / 4], decs[STEP_COLS / 4];
+  const int tid = threadIdx.x;
+  // the attention's first: they are short
+  const int convs = p.B * p.conv_blocks;
+  if ((int)blockIdx.x < convs) {
+    conv_qkv_unit<bf16_t, STEP_VEC, true>(p.conv, blockIdx.x / p.conv_blocks,
+                             blockIdx.x % p.conv_blocks * STEP_THREADS + tid);
+    return;
+  }
+  const int b = (blockIdx.x - convs) / p.G, g = (blockIdx.x - convs) % p.G;
+  const int N = p.N, P = p.P, HG = p.H / p.G, CG = HG * P, h0 = g * HG;
+  const int pos = p.seq_lens[b] - 1, slot = p.slots[b];
+  bf16_t* orow = p.out + b * p.ostride + (long long)g * CG;
+  if (pos < 0 || slot < 0) {                       // uniform over the block
+    if (tid < CG) orow[tid] = 0;
+    return;
+  }
+  const int C = p.H * P + 2 * p.G * N, NT = p.taps - 1;
+  const bf16_t* ur = p.u + b * p.ustride;
+
+  // what the convolution, the step sizes and the results want, then the state
+  const bool mine = tid < CG + 2 * N;
+  const int ch = tid < CG       ? h0 * P + tid
+                 : tid < CG + N ? p.H * P + g * N + tid - CG
+                                : p.H * P + (p.G + g) * N + tid - CG - N;
+  bf16_t* tail = p.tails + (long long)slot * NT * C + ch;
+  float cx = 0.f, cb = 0.f, cw[STEP_TAPS];
+  unsigned raw = 0, old[STEP_TAPS - 1] = {};
+  if (mine) {
+    raw = ur[p.xoff + ch];
+    cb = p.bias[ch];
+#pragma unroll
+    for (int j = 0; j < STEP_TAPS; ++j)            // beyond the filter: again
+      cw[j] = p.w[(unsigned)(min(j, NT) * C + ch)];
+    if (NT > 0) {
+#pragma unroll
+      for (int j = 0; j < STEP_TAPS - 1; ++j)
+        old[j] = tail[(unsigned)(min(j, NT - 1) * C)];
+    }
+  }
+  const int ht = tid - (STEP_THREADS - 64) * (HG <= 64);   // the last wave's
+  const bool head = ht >= 0 && ht < HG;
+  unsigned hraw = 0;
+  float hb = 0.f, ha = 0.f;
+  if (head) {
+    hraw = ur[p.dtoff + h0 + ht];
+    hb = p.dt_bias[h0 + ht];
+    ha = p.A[h0 + ht];
+  }
+  const int cols = CG / 4, GR = STEP_THREADS / cols;       // powers of two
+  const int c4 = tid & (cols - 1), g0 = tid / cols;
+  const int hh = c4 * 4 / P;
+  float* S = p.state + ((long long)slot * p.H + h0) * N * P;
+  const unsigned at = (unsigned)((hh * N + g0) * P + c4 * 4 - hh * P);
+  float s[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    ld_state<FAR, 4>(S + (at + (unsigned)(r * GR * P)), s[r]);
+
+  // nothing of the above is worked on, and waited for, before the state's loads
+#pragma unroll
+  for (int j = 0; j < STEP_TAPS - 1; ++j) asm volatile("" : "+v"(old[j]));
+  asm volatile("" : "+v"(raw), "+v"(hraw));
+  if (mine) {
+    cx = cb;
+    const float in = bf16_to_f32(raw);
+#pragma unroll
+    for (int j = 0; j < STEP_TAPS - 1; ++j) {
+      if (pos - NT + j < 0) old[j] = 0;            // before the first token
+      if (j < NT) cx = fmaf(cw[j], bf16_to_f32(old[j]), cx);
+    }
+    cx = fmaf(cw[STEP_TAPS - 1], in, cx);
+#pragma unroll
+    for (int j = 0; j < STEP_TAPS - 1; ++j)
+      if (j < NT)
+        tail[(unsigned)(j * C)] =
+            (bf16_t)(j + 1 < NT ? old[j + 1 < STEP_TAPS - 1 ? j + 1 : j] : raw);
+    cx = bf16_to_f32(cvt_bf16(cx / (1.f + __expf(-cx))));
+    if (tid < CG) xs[tid] = cx;
+    else bc[tid - CG] = cx;
+  }
+  if (head) {
+    const float dt = softplus_f(bf16_to_f32(hraw) + hb);
+    dts[ht] = dt;
+    decs[ht] = expf(-ha * dt);
+  }
+  // on their way while the state is
+  float nw[4], dk = 0.f;
+  uint2 zr = {};
+  if (tid < cols) {
+    zr = *reinterpret_cast<const uint2*>(ur + p.zoff + (long long)h0 * P +
+                                         tid * 4);
+    ldv<float, 4>(p.norm + (long long)h0 * P + tid * 4, nw);
+    dk = p.Dskip[h0 + tid * 4 / P];
+  }
+  lds_barrier();
+  f32x4_v acc = {0.f, 0.f, 0.f, 0.f};
+  {
+    const float dt = dts[hh], dec = decs[hh];
+    const f32x4_v x = *reinterpret_cast<const f32x4_v*>(&xs[c4 * 4]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int d = g0 + r * GR;
+      const float kd = bc[d] * dt, qd = bc[N + d];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        // slots are not cleared: what lies there before the first token is no state
+        s[r][j] = fmaf(dec, pos == 0 ? 0.f : s[r][j], kd * x[j]);
+        acc[j] = fmaf(qd, s[r][j], acc[j]);
+      }
+      st_state<FAR, 4>(S + (at + (unsigned)(r * GR * P)), s[r]);
+      // all rows' B and C at once would take the registers of a second block
+      if (r % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  red[tid] = acc;
+  lds_barrier();
+  float ss = 0.f, y[4];
+  if (tid < cols) {
+    f32x4_v sum = {0.f, 0.f, 0.f, 0.f};
+    const float2 za = bf16x2_to_f32x2(zr.x), zb = bf16x2_to_f32x2(zr.y);
+    const float zv[4] = {za.x, za.y, zb.x, zb.y};
+#pragma unroll 8
+    for (int i = 0; i < GR; ++i) sum += red[i * cols + tid];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      y[j] = (sum[j] + dk * xs[tid * 4 + j]) * silu_f(zv[j]);
+      ss = fmaf(y[j], y[j], ss);
+    }
+  }
+  ss = wave_reduce_sum(ss);
+  if (cols > 64) {                     // uniform: a group's part of two waves
+    if (tid < cols && (tid & 63) == 0) dts[tid >> 6] = ss;
+    lds_barrier();
+    ss = dts[0] + dts[1];
+  }
+  if (tid >= cols) return;
+  const float inv = 1.f / sqrtf(ss / (float)CG + p.eps);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[j] *= inv * nw[j];
+  stv<bf16_t, 4>(orow + tid * 4, y);
+}
+
+// Rows of the state of a thread, 0 where the sizes are not the kernel's.
+extern "C" int qsa_ssd_step_rows(int H, int N, int P, int G, int parts,
+                                 int taps) {
+  if (G <= 0 || parts != G || H % G || P % 4 || taps < 1 || taps > STEP_TAPS)
+    return 0;
+  const long long cols = (long long)H / G * P;
+  if (cols < 64 || cols > STEP_COLS || (cols & (cols - 1)) ||
+      cols + 2ll * N > STEP_THREADS || cols * N % (4 * STEP_THREADS))
+    return 0;
+  const int rows = (int)(cols * N / (4 * STEP_THREADS));
+  return rows == 2 || rows == 4 || rows == 8 || rows == 16 ? rows : 0;
+}
+
+extern "C" void qsa_ssd_step_launch(SsdStep p, hipStream_t st) {
+  p.conv_blocks = (conv_qkv_units(p.conv, STEP_VEC) + STEP_THREADS - 1) / STEP_THREADS;
+  const dim3 grid((unsigned)(p.B * (p.G + p.conv_blocks)));
+  const bool far = (long long)p.B * p.H * p.N * p.P * 4 > QSA_FAR_STATE;
+#define QSA_ST_AS(R, FAR) \
+  hipLaunchKernelGGL((qsa_ssd_step<R, FAR>), grid, dim3(STEP_THREADS), 0, st, p)
+#define QSA_ST(R) \
+  case R: if (far) QSA_ST_AS(R, true); else QSA_ST_AS(R, false); break
+  switch (qsa_ssd_step_rows(p.H, p.N, p.P, p.G, p.G, p.taps)) {
+    QSA_ST(2);
+    QSA_ST(4);
+    QSA_ST(8);
+    QSA_ST(16);
+  }
+#undef QSA_ST
+#undef QSA_ST_AS
 }
 
 // ---------------------------------------------------------------------------

@@ -468,6 +468,78 @@ def test_ssd_kernels(H, P, N, G, dtype):
     assert torch.equal(before.nan_to_num(9.0), state.nan_to_num(9.0))
 
 
+# heads, vdim, state, groups, taps of either branch: 2, 4, 8 and 16 rows of state
+# a thread, one and two waves of columns
+STEPS = [(4, 64, 128, 4, 4, 4), (2, 64, 128, 1, 1, 3), (8, 64, 128, 2, 4, 4),
+         (8, 64, 128, 1, 2, 1), (3, 128, 256, 3, 3, 2), (1, 256, 128, 1, 4, 4)]
+
+
+@pytest.mark.parametrize("H,P,N,G,taps,qtaps", STEPS)
+def test_ssd_step(H, P, N, G, taps, qtaps):
+    """One launch for single tokens against the kernels it stands for: rows at
+    their first tokens, later ones, and rows not in use."""
+    g = gen(H * P + taps)
+    B, QH, KG, Dm, E = 9, 6, 2, 40, 72
+    inner, C = H * P, H * P + 2 * G * N
+    qc = (QH + KG) * Dm + KG * E
+    lens = [1, 2, 3, 4, 5, 900, 0, 64, 7]
+    slots = [3, 0, 9, 2, 1, 8, 4, -1, 5]
+    assert D.ssd_step_ok(H, N, P, G, G, taps)
+    x = rnd(g, B, qc + 8, dtype=BF).to(DEV)
+    u = rnd(g, B, C + inner + H + (-(C + inner + H)) % 8, dtype=BF).to(DEV)
+    qw, w = (rnd(g, t, c).to(DEV) for t, c in ((qtaps, qc), (taps, C)))
+    bias, skip, norm = (rnd(g, c).to(DEV) for c in (C, H, inner))
+    A = torch.rand(H, generator=g).to(DEV) * 4
+    db = rnd(g, H).to(DEV)
+    rope = RopeTable(16, 1e4, DEV)
+    rope.ensure(1000)
+
+    def fresh():
+        t = gen(7)
+        return [rnd(t, *s, dtype=d).to(DEV) for s, d in (
+            ((10, qtaps - 1, qc), BF), ((10, taps - 1, C), BF),
+            ((10, H, N, P), F32), ((20, KG, 64, Dm), BF),
+            ((20, KG, 64, E), BF))]
+
+    def run(whole):
+        qt, t, S, k, v = fresh()
+        cache = i32(*[64 * i + 7 for i in range(B)])
+        n, s = i32(*lens), i32(*slots)
+        S[3] = float("nan")                      # row 0's, which is not read
+        y = torch.full((B, inner + 8), 5., device=DEV, dtype=BF)
+        a = (x[:, :qc], qw, qt, rope.cos, rope.sin, 16, cache, k, v, QH)
+        if whole:
+            q = D.ssd_step(*a, u, w, bias, t, A, db, skip, S, G, norm, 1e-4,
+                           y[:, 8:], s, n)
+        else:
+            conv = (None, None, None, n, None, s)
+            q = D.conv_qkv(*a, *conv)
+            o = D.ssd_decode(u, 0, inner + C, D.conv_silu(
+                u[:, inner:inner + C], w, bias, t, *conv), A, db, skip, S, G,
+                s, n)
+            D.part_norm(o, norm, y[:, 8:], G, 1e-4)
+        live = torch.tensor([i for i in range(B) if lens[i] and slots[i] >= 0])
+        return [q[live], y, qt, t, S.nan_to_num(9.), k, v]
+
+    got, want = run(True), run(False)
+    for i in (0, 2, 3, 5, 6):                    # copies of one code
+        assert torch.equal(got[i], want[i]), i
+    # f32 in the same order but for the read-out's sums over N
+    assert float((got[4] - want[4]).abs().max()) <= 1e-5 * float(
+        want[4].abs().max())
+    close(got[1][:, 8:], want[1][:, 8:].cpu(), BF)
+    assert not got[1][[6, 7], 8:].any() and (got[1][:, :8] == 5).all()
+
+
+@pytest.mark.parametrize("case", [(3, 13, 7, 1, 1, 4), (8, 128, 64, 2, 4, 4),
+                                  (8, 128, 64, 2, 2, 5), (6, 128, 64, 2, 2, 4),
+                                  (16, 128, 64, 1, 1, 4)])
+def test_ssd_step_refuses(case):
+    """Norm parts that are not the groups, long filters, columns and states
+    that threads do not divide: the general kernels take those."""
+    assert not D.ssd_step_ok(*case)
+
+
 # ---- the model through the framework ----------------------------------------
 
 @pytest.fixture(scope="module")
