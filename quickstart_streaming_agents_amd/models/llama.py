@@ -511,16 +511,16 @@ class LlamaModel:
             if use_hip_prefill:
                 D.rope_kv_scatter(q[:T], k[:T], v[:T], kv.k[li], kv.v[li],
                                   self.rope_cos, self.rope_sin,
-                                  positions[:T], slots)
+                                  positions[:T], slots, turn_q=False)
             else:
                 D.rope_inplace(q, k, self.rope_cos, self.rope_sin, positions)
                 D.kv_scatter(k[:T], v[:T], kv.k[li], kv.v[li], slots)
             if use_hip_prefill:
                 # ONE varlen flash kernel: streams K/V pages directly, no
-                # gather/pad/score materialization
+                # gather/pad/score materialization, and rotates its queries
                 attn = D.ext().paged_attn_prefill(
                     q, kv.k[li], kv.v[li], bt_t, *maps, self.scale, True,
-                    qrows)
+                    qrows, self.rope_cos, self.rope_sin)
             else:
                 # padded q: [nb*nmax, n_q, D] -> [nb*KVH, R*nmax, D]
                 q_pad = torch.zeros(nb * nmax, self.n_q, c.d_head,

@@ -153,13 +153,15 @@ def kv_scatter(knew: torch.Tensor, vnew: torch.Tensor, kc: torch.Tensor,
         vc[page, :, :, off] = vnew[t]
 
 
-def rope_kv_scatter(q, k, v, kc, vc, cos_t, sin_t, pos, slots) -> None:
+def rope_kv_scatter(q, k, v, kc, vc, cos_t, sin_t, pos, slots,
+                    turn_q: bool = True) -> None:
     """rope_inplace of q and k and kv_scatter in one (on the GPU k is rotated
-    on its way to the cache only)."""
+    on its way to the cache only).  Without turn_q q stays as it is."""
     if _cuda(q):
-        ext().rope_kv_scatter(q, k, v, kc, vc, cos_t, sin_t, pos, slots)
+        ext().rope_kv_scatter(q, k, v, kc, vc, cos_t, sin_t, pos, slots,
+                              turn_q)
         return
-    rope_inplace(q, k, cos_t, sin_t, pos)
+    rope_inplace(q if turn_q else q.clone(), k, cos_t, sin_t, pos)
     kv_scatter(k, v, kc, vc, slots)
 
 

@@ -58,6 +58,7 @@ extern "C" void qsa_paged_attn_prefill_launch(
     const unsigned short*, const unsigned short*, const unsigned short*,
     const int*, const int*, const int*, const int*, const int*, const int*,
     unsigned short*, float, int, int, int, int, int, long long, int, int,
+    const float*, const float*, int,
     hipStream_t);
 extern "C" void qsa_rope_kv_scatter_launch(
     unsigned short*, const unsigned short*, const unsigned short*,
@@ -367,8 +368,11 @@ torch::Tensor paged_attn_prefill(torch::Tensor q, torch::Tensor kc,
                                  torch::Tensor item_off,
                                  torch::Tensor item_start,
                                  torch::Tensor item_len, double scale,
-                                 bool causal, long rows) {
-  // rows: query tokens per block of the maps (qb_item, qb_pos0)
+                                 bool causal, long rows,
+                                 c10::optional<torch::Tensor> cos_t,
+                                 c10::optional<torch::Tensor> sin_t) {
+  // rows: query tokens per block of the maps (qb_item, qb_pos0); with cos_t and
+  // sin_t q is rotated here, by a row's position
   CHK_DEV(q); CHK_BF16(q); CHK_BF16(kc); CHK_BF16(vc);
   CHK_CONT(kc); CHK_CONT(vc); CHK_I32(block_table); CHK_CONT(block_table);
   CHK_I32(qb_item); CHK_I32(qb_pos0); CHK_I32(item_off);
@@ -383,13 +387,26 @@ torch::Tensor paged_attn_prefill(torch::Tensor q, torch::Tensor kc,
   TORCH_CHECK(vc.size(2) == D && vc.size(3) == 64, "V layout [P,KVH,D,64]");
   const int QB = qb_item.numel();
   const int npmax = block_table.size(1);
+  TORCH_CHECK(cos_t.has_value() == sin_t.has_value(), "cos and sin");
+  if (cos_t) {
+    CHK_F32(*cos_t); CHK_F32(*sin_t); CHK_CONT(*cos_t); CHK_CONT(*sin_t);
+    TORCH_CHECK(cos_t->dim() == 2 && cos_t->size(1) == D / 2 &&
+                    cos_t->size(0) > 0 && sin_t->sizes() == cos_t->sizes(),
+                "cos/sin [positions, D/2]");
+    TORCH_CHECK(((reinterpret_cast<uintptr_t>(cos_t->data_ptr()) |
+                  reinterpret_cast<uintptr_t>(sin_t->data_ptr())) & 15) == 0,
+                "cos and sin must be 16-byte aligned");
+  }
   auto out = torch::empty({(long long)T, (long long)QH * D}, q.options());
   qsa_paged_attn_prefill_launch(
       u16(q), u16(kc), u16(vc), block_table.data_ptr<int>(),
       qb_item.data_ptr<int>(), qb_pos0.data_ptr<int>(),
       item_off.data_ptr<int>(), item_start.data_ptr<int>(),
       item_len.data_ptr<int>(), u16m(out), (float)scale, QB, QH, KVH, npmax,
-      D, q.stride(0), causal ? 1 : 0, (int)rows, cur_stream());
+      D, q.stride(0), causal ? 1 : 0, (int)rows,
+      cos_t ? cos_t->data_ptr<float>() : nullptr,
+      sin_t ? sin_t->data_ptr<float>() : nullptr,
+      cos_t ? (int)cos_t->size(0) : 0, cur_stream());
   return out;
 }
 
@@ -416,8 +433,9 @@ void rope_kv_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 void rope_kv_scatter(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                      torch::Tensor kc, torch::Tensor vc, torch::Tensor cos_t,
                      torch::Tensor sin_t, torch::Tensor pos,
-                     torch::Tensor slots) {
-  // rope_inplace on q, and k rotated and v written to the pages; k and v stay
+                     torch::Tensor slots, bool turn_q) {
+  // rope_inplace on q (unless its reader turns it), and k rotated and v written to
+  // the pages; k and v stay
   CHK_DEV(q); CHK_BF16(q); CHK_BF16(k); CHK_BF16(v);
   CHK_BF16(kc); CHK_BF16(vc); CHK_CONT(kc); CHK_CONT(vc);
   CHK_F32(cos_t); CHK_F32(sin_t); CHK_CONT(cos_t); CHK_CONT(sin_t);
@@ -445,8 +463,8 @@ void rope_kv_scatter(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   if (T == 0) return;
   qsa_rope_kv_scatter_launch(u16m(q), u16(k), u16(v), u16m(kc), u16m(vc),
                              cos_t.data_ptr<float>(), sin_t.data_ptr<float>(),
-                             pos.data_ptr<int>(), slots.data_ptr<int>(), T, QH,
-                             KVH, D, q.stride(0), k.stride(0), cur_stream());
+                             pos.data_ptr<int>(), slots.data_ptr<int>(), T,
+                             turn_q ? QH : 0, KVH, D, q.stride(0), k.stride(0), cur_stream());
 }
 
 torch::Tensor mean_rows(torch::Tensor x, torch::Tensor off,
@@ -952,7 +970,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("block_table"),
         py::arg("qb_item"), py::arg("qb_pos0"), py::arg("item_off"),
         py::arg("item_start"), py::arg("item_len"), py::arg("scale"),
-        py::arg("causal"), py::arg("rows") = 16);
+        py::arg("causal"), py::arg("rows") = 16, py::arg("cos_t") = py::none(),
+        py::arg("sin_t") = py::none());
   m.def("paged_attn_decode", &paged_attn_decode,
         "paged-attention decode (bf16, GQA, page=64)");
   m.def("paged_attn_split", &paged_attn_split,
@@ -967,7 +986,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_kv_append", &rope_kv_append,
         "fused decode rope + paged-cache append");
   m.def("rope_kv_scatter", &rope_kv_scatter,
-        "prefill rotation and paged-cache write");
+        "prefill rotation and paged-cache write", py::arg("q"), py::arg("k"),
+        py::arg("v"), py::arg("kc"), py::arg("vc"), py::arg("cos_t"),
+        py::arg("sin_t"), py::arg("pos"), py::arg("slots"),
+        py::arg("turn_q") = true);
   m.def("encoder_attn", &encoder_attn,
         "rotation and bidirectional attention of projection rows");
   m.def("short_gemm", &short_gemm, "GEMM of a short K, optionally gated");

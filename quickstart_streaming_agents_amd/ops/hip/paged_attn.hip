@@ -724,8 +724,9 @@ extern "C" void qsa_kv_scatter_launch(const unsigned short* knew,
 }
 
 // ---------------------------------------------------------------------------
-// Prefill rotation and cache write in one pass: q is rotated in place, k on its
-// way to the pages, v transposed into them through LDS.
+// Prefill rotation and cache write in one pass: q is rotated in place, or left for
+// the attention to rotate (QH 0), k rotated on its way to the pages, v transposed into
+// them through LDS.
 //
 // Block = (64 tokens, kv head): its R query heads, its key and its value.  A
 // lane owns 8 dims and their rotation partners of one token, so angles are read
@@ -734,7 +735,10 @@ extern "C" void qsa_kv_scatter_launch(const unsigned short* knew,
 // 45k tokens, 32/8 heads of 128: 468 (rotation) + 292 us (scatter by elements)
 // before, 224 us here (4.9 TB/s, what a copy reaches); few tokens are bound by
 // round trips, so all reads of a pass come before its writes (5 tokens 6.8 -> 4.3
-// us, 200 11.5 -> 6.1, 764 14.7 -> 7.8, the conversion's part among it).
+// us, 200 11.5 -> 6.1, 764 14.7 -> 7.8, the conversion's part among it).  The
+// attention turns its queries in registers, so a prefill leaves q out: 10,528 tokens
+// 51.7 -> 26.2 us, and the attention of 96 x 20-200 behind 500-1200 244 -> 254; 8192
+// 41.6 -> 22.2, and 626 -> 614.
 // ---------------------------------------------------------------------------
 template <int D>
 __global__ void __launch_bounds__(256)
@@ -865,6 +869,8 @@ extern "C" void qsa_rope_kv_scatter_launch(
 // half of the time, the exponents a quarter; LDS reads (each K/V fragment
 // serves QT tiles) take as long as the matrix cores.  Rescaling is left out when
 // no maximum of the wave moved.
+// Queries may be turned here, on their way into registers (what that saves stands at
+// qsa_rope_kv_scatter): a row's dims d and d + D/2 are fragments of one lane.
 // A wave's first and last page stand outside of the loop over the others: paths that
 // meet behind the products took 30 registers more (D = 64: 149 us for 122).
 // us, 32/8 heads of 128, with pages by way of registers and one after the other
@@ -887,7 +893,10 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
                        const int* __restrict__ item_len,       // [nb] new rows
                        unsigned short* __restrict__ out,       // [T, QH*D]
                        float scale2, int QH, int KVH, int npmax,
-                       long long qstride, int rows, int subs) {
+                       long long qstride, int rows, int subs,
+                       const float* __restrict__ cos_t,  // [positions, D/2], or
+                       const float* __restrict__ sin_t,  // null: q is rotated
+                       int positions) {
 #ifdef __HIP_DEVICE_COMPILE__          // loads into LDS: not for the host
   constexpr int KS = D / 32;           // k-steps of a score tile
   constexpr int ET = D / 16;           // tiles of value columns
@@ -974,11 +983,29 @@ qsa_paged_attn_prefill(const unsigned short* __restrict__ q,   // [T, QH, D] str
     const unsigned short* qrow =
         q + (off + tok) * qstride + (long long)(g * R + v - tok * R) * D;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
+    for (int s = 0; s < KS; ++s)
       qf[u][s] = *reinterpret_cast<const bf16x8_v*>(qrow + s * 32 + hi * 8);
-      if (negative) qf[u][s] ^= (short)0x8000;
+  }
+  if (cos_t) {                         // dims d and d + D/2 are a lane's
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      const int tok = min(w0 + u * 16 + col, vend - 1) / R;
+      const long long at =
+          (long long)min(start + tok, positions - 1) * (D / 2) + hi * 8;
+#pragma unroll
+      for (int s = 0; s < KS / 2; ++s) {
+        float c[8], sn[8];
+        ldv<float, 8>(cos_t + at + s * 32, c);
+        ldv<float, 8>(sin_t + at + s * 32, sn);
+        rotate_pair(qf[u][s], qf[u][s + KS / 2], c, sn);
+      }
     }
   }
+#pragma unroll
+  for (int u = 0; u < QT; ++u)
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      if (negative) qf[u][s] ^= (short)0x8000;
   f32x4_v acc[QT][ET], sc[QT][4];
   bf16x8_v pf[QT][2];
   float m[QT], l[QT], alpha[QT], psum[QT], top[QT];
@@ -1210,6 +1237,7 @@ extern "C" void qsa_paged_attn_prefill_launch(
     const int* qb_pos0, const int* item_off, const int* item_start,
     const int* item_len, unsigned short* out, float scale, int QB, int QH,
     int KVH, int npmax, int D, long long qstride, int causal, int rows,
+    const float* cos_t, const float* sin_t, int positions,
     hipStream_t stream) {
   const float scale2 = scale * 1.4426950408889634f;
   // two tiles per wave as soon as a block's rows fill more than one each
@@ -1222,7 +1250,7 @@ extern "C" void qsa_paged_attn_prefill_launch(
     hipLaunchKernelGGL((qsa_paged_attn_prefill<DD, QQ, CC>), grid, dim3(256), \
                        0, stream, q, kc, vc, block_table, qb_item, qb_pos0,   \
                        item_off, item_start, item_len, out, scale2, QH, KVH,  \
-                       npmax, qstride, rows, subs);                           \
+                       npmax, qstride, rows, subs, cos_t, sin_t, positions);  \
     return;                                                                   \
   }
   QSA_PREFILL_CASE(128, 1, true) QSA_PREFILL_CASE(128, 1, false)

@@ -1188,6 +1188,56 @@ def test_rope_kv_scatter(ext, T, QH, KVH, D):
                 <= 2 ** -7 * b.float().abs() + 1e-6).all()
 
 
+@pytest.mark.parametrize("D,QH,KVH,rows,scale", [
+    (128, 32, 8, 32, 1.0), (128, 28, 4, 9, 1.0), (64, 8, 8, 128, -1.0),
+    (64, 16, 1, 4, 1.0)])
+def test_prefill_rotates_queries(ext, D, QH, KVH, rows, scale):
+    """Queries turned on their way into the attention, at the position of each
+    row, against the same turned before."""
+    g = torch.Generator().manual_seed(D + rows)
+    items = [(0, 1), (63, 2), (5, 130), (64, 64), (200, 33)]
+    lens = [n for _, n in items]
+    np_ = [-(-(a + n) // 64) for a, n in items]
+    bt = torch.zeros(len(items), max(np_), dtype=torch.int32)
+    for i, n in enumerate(np_):
+        bt[i, :n] = torch.arange(sum(np_[:i]), sum(np_[:i]) + n)
+    T, P = sum(lens), sum(np_)
+    qkv = torch.randn(T, (QH + 2 * KVH) * D, generator=g).bfloat16().to(dev())
+    twin = qkv.clone()
+    rot = torch.rand(233, D // 2, generator=g) * 6.28    # up to the last position
+    cos, sin = rot.cos().to(dev()), rot.sin().to(dev())
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=dev())
+    pos = mk([a + i for a, n in items for i in range(n)])
+    slots = mk([int(bt[i, p // 64]) * 64 + p % 64
+                for i, (a, n) in enumerate(items) for p in range(a, a + n)])
+    blocks = [(i, p) for i, n in enumerate(lens) for p in range(0, n, rows)]
+    maps = (bt.to(dev()), mk([b[0] for b in blocks]),
+            mk([b[1] for b in blocks]), mk(list(np.cumsum(lens) - lens)),
+            mk([a for a, _ in items]), mk(lens), scale * D ** -0.5, True, rows)
+    kc = torch.randn(P, KVH, D // 8, 64, 8, generator=g).bfloat16().to(dev())
+    vc = torch.randn(P, KVH, D, 64, generator=g).bfloat16().to(dev())
+    kc2, vc2 = kc.clone(), vc.clone()
+
+    def split(t):
+        return [x.view(T, -1, D) for x in
+                t.split([QH * D, KVH * D, KVH * D], 1)]
+
+    q, k, v = split(qkv)
+    ext.rope_kv_scatter(q, k, v, kc, vc, cos, sin, pos, slots, turn_q=False)
+    assert torch.equal(qkv, twin)                        # nothing of it changed
+    got = ext.paged_attn_prefill(q, kc, vc, *maps, cos, sin)
+    q2, k2, v2 = split(twin)
+    ext.rope_kv_scatter(q2, k2, v2, kc2, vc2, cos, sin, pos, slots)
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    want = ext.paged_attn_prefill(q2, kc2, vc2, *maps).double()
+    # the rotation's products may be fused differently: a bf16 step, 2^-8, of some
+    # of a query's numbers, as much as its rounding; probabilities and results are
+    # rounded alike
+    err = got.double() - want
+    assert err.norm() <= 5e-3 * want.norm()
+    assert err.abs().max() <= 2 ** -7 * vc.abs().max()
+
+
 @pytest.mark.parametrize("D,H", [(64, 8), (128, 4)])
 @pytest.mark.parametrize("lens", [[1], [64, 63, 65, 1, 130], [512, 3, 128]])
 def test_encoder_attn(ext, lens, D, H):
