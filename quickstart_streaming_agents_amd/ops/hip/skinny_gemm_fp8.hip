@@ -7,13 +7,10 @@
 // weights HALVE that stream: per-output-channel symmetric quantization
 // (s[n] = max|W[n,:]| / 448, the standard W8A16 weight-only scheme) keeps
 // activations bf16 and applies the scale once in the epilogue — zero
-// inner-loop cost.  Dequant in-kernel:
-//   v_cvt_pk_f32_fp8 (2 fp8 -> 2 f32, exact)
-//   v_perm_b32       (pack the two f32 high halves -> 2 bf16)
-// The f32 -> bf16 TRUNCATION is exact: e4m3 has 3 mantissa bits, bf16
-// has 8, and every e4m3 value (normals and denormals) is exactly
-// representable in bf16 — the dequantized operand is bit-exact, so the
-// MFMA math matches a bf16 kernel running on the dequantized weights.
+// inner-loop cost.  Dequant in-kernel: v_cvt_scalef32_pk_bf16_fp8 with a scale of
+// one (2 fp8 -> 2 bf16).  It is exact: e4m3 has 3 mantissa bits, bf16 has 8, and
+// every e4m3 value (normals and denormals) is a bf16 value, so the MFMA math
+// matches a bf16 kernel running on the dequantized weights.
 //
 // The kernel is skinny_stream.h's, with the norms, activation and residual of a
 // decoding step done on the way.

@@ -702,6 +702,22 @@ def test_skinny_gemm_fp8_matches_dequant_ref():
         assert qerr < 0.5, f"quantization error blew up: {qerr}"
 
 
+def test_skinny_gemm_fp8_every_code():
+    """Each of the 256 codes comes out as the bf16 value it stands for, the
+    subnormal ones and NaN too."""
+    from quickstart_streaming_agents_amd.ops import ext
+    codes = torch.arange(256, dtype=torch.uint8)
+    q = codes[:, None].expand(256, 256).contiguous()     # a row of W per code
+    qf = q.reshape(16, 16, 4, 2, 4, 8).permute(0, 2, 1, 4, 3, 5).contiguous()
+    a = torch.zeros(3, 256, dtype=torch.bfloat16)
+    a[0, 0] = a[1, 77] = a[2, 255] = 1
+    out = ext().skinny_gemm_fp8(a.cuda(), qf.cuda(), torch.ones(256).cuda(),
+                                256, 256).cpu()
+    want = codes.view(torch.float8_e4m3fn).float()
+    assert torch.equal(out.float().nan_to_num(nan=1e3),
+                       want.nan_to_num(nan=1e3).expand(3, 256))
+
+
 def test_skinny_gemm_fp8_gpu_pack_matches_cpu_pack():
     """CPU and GPU packs agree in VALUE (the f32->e4m3 cast may round
     ties differently across backends; one e4m3 quantum of slack)."""
