@@ -638,6 +638,10 @@ torch::Tensor skinny_gemm_fp8(torch::Tensor a, torch::Tensor qf,
   // C[M,N] = a @ (scale[N] * dequant(Q))^T; Q pre-packed fp8 e4m3 in the
   // fragment-pair-major stream layout (skinny_gemm_fp8.hip header).
   const int M = chk_skinny_fp8(a, qf, scale, N, K);
+  // the kernel's offsets are 32 bits of whole 16 bytes
+  if ((reinterpret_cast<uintptr_t>(a.data_ptr()) & 15) || a.stride(0) % 8 ||
+      a.stride(0) < 0 || M * a.stride(0) >= 1ll << 30)
+    a = a.clone(at::MemoryFormat::Contiguous);
   auto out = torch::empty({M, (long long)N}, a.options());
   qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
                              scale.data_ptr<float>(), u16m(out), nullptr, M,

@@ -96,7 +96,7 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   // would otherwise run with no lane enabled and still add up
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
-  // K % 64 == 0, HALF: % 128 and steps of either half of K
+  // K % 64 == 0, HALF: % 128 and steps of either half of K; A's offsets fit 31 bits
   const int steps = (int)(p.K >> (HALF ? 7 : 6));
   // a lane's column of its tile, as results are stored
   const int tcol = HALF ? ((int)blockIdx.x & 1) * 8 + (col & 7) : col;
@@ -140,25 +140,29 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
       nw[i] = p.norm_w[c];
     }
   }
-  const u32x4_v* wp[TILES];
-#pragma unroll
-  for (int t = 0; t < TILES; ++t)
-    wp[t] = p.W + (HALF ? ((long long)tile_of(t) * 2 + (col >> 3)) * steps * 64
-                        : (long long)tile_of(t) * steps * (64 * WL)) +
-            tcol * 4 + hi;
-  const bf16_t* ap[MT];
+  // Where loads are: a tile's stream and A, a lane's place in them, and the step, which
+  // is a scalar: no vector instruction makes an address.  Steps beyond the end are read
+  // as zeros, from nowhere, and multiplied like others, so that a wave's code is short
+  // and without branches; the groups are worked on as they arrive.  (us a step with
+  // 64-bit addresses and a look at every step, and so: 16 layers of width 2048, one row
+  // 485 -> 460, 24 rows 734 -> 705; 8 layers of 4096, one row 478 -> 467, 6 rows 514 ->
+  // 502, 16 rows 680 -> 672.)
+  using rsrc = __amdgpu_buffer_rsrc_t;
+  constexpr int WB = 1024 * WL;                   // bytes of a tile's step
+  const int stream = (HALF ? 2 : 1) * steps * WB;
+  const unsigned wo = (unsigned)(tcol * 4 + hi) * 16 +
+                      (HALF ? (unsigned)(col >> 3) * steps * WB : 0u);
+  unsigned ao[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m)
     if constexpr (HALF)
-      ap[m] = p.A + (long long)(col >> 3) * steps * (PACK ? 1024 : 64) +
-              (PACK ? ((col & 7) + hi * 16) * 8
-                    : min(col & 7, p.M - 1) * p.lda + hi * 8);
+      ao[m] = ((unsigned)(col >> 3) * steps * (PACK ? 1024 : 64) +
+               (PACK ? ((col & 7) + hi * 16) * 8
+                     : min(col & 7, p.M - 1) * (unsigned)p.lda + hi * 8)) * 2;
     else
       // packed rows that do not exist: the line of eight that do
-      ap[m] = PACK ? p.A + m * 512 +
-                         ((p.M - m * 16 <= 8 ? col & 7 : col) + hi * 16) * 8
-                   : p.A + (long long)min(m * 16 + col, p.M - 1) * p.lda +
-                         hi * 8;
+      ao[m] = (PACK ? m * 512 + ((p.M - m * 16 <= 8 ? col & 7 : col) + hi * 16) * 8
+                    : min(m * 16 + col, p.M - 1) * (unsigned)p.lda + hi * 8) * 2;
 
   struct Group {
     u32x4_v w[U][TILES][WL];
@@ -173,26 +177,34 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   auto load = [&](Group& g, int base) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const long long s = min(base + u * WAVES, steps - 1);
+      const int s = base + u * WAVES;
+      const bool in = s < steps;                  // uniform over the wave
+      const int at = in ? s : 0;
 #pragma unroll
-      for (int t = 0; t < TILES; ++t)
+      for (int t = 0; t < TILES; ++t) {
+        const rsrc rw = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(p.W + (long long)tile_of(t) * (stream / 16)), 0,
+            in ? stream : 0, 0x00027000);
 #pragma unroll
         for (int i = 0; i < WL; ++i)
-          g.w[u][t][i] =
-              FAR ? __builtin_nontemporal_load(wp[t] + s * (64 * WL) + i * 64)
-                  : wp[t][s * (64 * WL) + i * 64];
+          g.w[u][t][i] = __builtin_amdgcn_raw_buffer_load_b128(
+              rw, wo + i * 1024, at * WB, FAR ? QSA_NT : 0);
+      }
+      const rsrc ra = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)p.A, 0, in ? 0x7fffffff : 0, 0x00027000);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          g.a[u][m][i] = *reinterpret_cast<const bf16x8_v*>(
-              ap[m] + (PACK ? (s * 2 + i) * (MT * 512) : s * 64 + i * 32));
+          g.a[u][m][i] = __builtin_bit_cast(
+              bf16x8_v, __builtin_amdgcn_raw_buffer_load_b128(
+                            ra, ao[m] + i * (PACK ? MT * 1024 : 64),
+                            at * (PACK ? MT * 2048 : 128), 0));
     }
   };
-  auto compute = [&](Group& g, int base) {
+  auto compute = [&](Group& g) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (base + u * WAVES >= steps) break;       // uniform over the wave
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int t = 0; t < TILES; ++t)
 #pragma unroll
@@ -206,7 +218,6 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
           for (int m = 0; m < MT; ++m)
             acc[t][m] = mfma_bf16(g.a[u][m][i], w, acc[t][m]);
         }
-    }
   };
 
   Group g0, g1;
@@ -230,12 +241,15 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
       if (lane == 0) inv_s[row] = rsqrtf(s / (float)p.K + p.eps);
     }
   }
-  for (int base = wave; base < steps; base += 2 * ROUND) {
-    compute(g0, base);
-    if (base + 2 * ROUND < steps) load(g0, base + 2 * ROUND);
-    compute(g1, base + ROUND);
-    if (base + 3 * ROUND < steps) load(g1, base + 3 * ROUND);
+  // both groups are always loaded again, so that the waits in the loop are for one
+  for (int base = wave; base + 2 * ROUND < steps; base += 2 * ROUND) {
+    compute(g0);
+    load(g0, base + 2 * ROUND);
+    compute(g1);
+    load(g1, base + 3 * ROUND);
   }
+  compute(g0);
+  compute(g1);
 
 #pragma unroll
   for (int t = 0; t < TILES; ++t)

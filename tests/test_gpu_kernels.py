@@ -718,6 +718,47 @@ def test_skinny_gemm_fp8_every_code():
                        want.nan_to_num(nan=1e3).expand(3, 256))
 
 
+@pytest.mark.parametrize("K", [256, 512, 768, 1024, 1280, 3328, 7168])
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 8, 9, 17])
+def test_skinny_fp8_steps(M, K):
+    """Numbers of steps that the groups of a block's waves do not divide: all forms
+    against f64, rows of A in a wider matrix and off its 16 bytes."""
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    from quickstart_streaming_agents_amd.ops import ext
+    g = torch.Generator(device="cuda").manual_seed(K + M)
+    N, eps = 128, 1e-5
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16() * 0.05
+    packed = D.pack_weight_fp8(w)
+    W = D.unpack_weight_fp8(*packed, N, K).double()
+    wide = torch.full((M, K + 24), float("nan"), device="cuda").bfloat16()
+    wide[:, 8:K + 8] = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    x = wide[:, 8:K + 8]
+    want = x.double() @ W.t()
+
+    def close(got, want):
+        # sums of K products in f32, rounded to bf16: 2^-9 of a value
+        err = (got.double() - want).norm()
+        assert err <= 4e-3 * want.norm(), float(err / want.norm())
+
+    close(ext().skinny_gemm_fp8(x, *packed, N, K), want)
+    off = torch.full((M * K + 3,), float("nan"), device="cuda").bfloat16()
+    off[3:] = x.reshape(-1)
+    close(ext().skinny_gemm_fp8(off[3:].view(M, K), *packed, N, K), want)
+    # steps of the decoder: rows with their norm, and with the residual
+    embed = torch.randn(50, K, generator=g, device="cuda").bfloat16()
+    ids = torch.randint(0, 50, (M,), generator=g, device="cuda")
+    ones = torch.ones(K, device="cuda").bfloat16()
+    res, rows, ss = D.embed_rows(embed, ids, ones)
+    h = embed[ids].double()
+    y = h * torch.rsqrt(h.square().mean(-1, keepdim=True) + eps) @ W.t()
+    close(D.norm_linear_fp8(rows, ss, 1, M, eps, packed, N, K), y)
+    old = torch.randn(M, N, generator=g, device="cuda").bfloat16()
+    new = old.clone()
+    D.linear_residual_fp8(rows, packed, N, K, new,
+                          torch.ones(N, device="cuda").bfloat16())
+    close(new, old.double() + h @ W.t())
+
+
 def test_skinny_gemm_fp8_gpu_pack_matches_cpu_pack():
     """CPU and GPU packs agree in VALUE (the f32->e4m3 cast may round
     ties differently across backends; one e4m3 quantum of slack)."""
