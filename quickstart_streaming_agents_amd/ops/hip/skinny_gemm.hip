@@ -19,7 +19,7 @@
 template <int WAVES, int TILES, int MT, bool FAR>
 __global__ void __launch_bounds__(WAVES * 64)
 qsa_skinny_gemm(SkinnyArgs p) {
-  skinny_stream<WAVES, TILES, MT, false, false, false, false, false, FAR>(p);
+  skinny_stream<WAVES, TILES, MT, false, ROWS, false, false, false, FAR>(p);
 }
 
 template <int WAVES, int TILES>

@@ -24,32 +24,34 @@
 // speed with better numerics.
 #include "skinny_stream.h"
 
-template <int WAVES, int TILES, int MT, bool PACK, bool NORM, bool GLU,
+template <int WAVES, int TILES, int MT, int FORM, bool NORM, bool GLU,
           bool RES, bool FAR>
 __global__ void __launch_bounds__(WAVES * 64)
 qsa_skinny_gemm_fp8(SkinnyArgs p) {
-  skinny_stream<WAVES, TILES, MT, true, PACK, NORM, GLU, RES, FAR>(p);
+  skinny_stream<WAVES, TILES, MT, true, FORM, NORM, GLU, RES, FAR>(p);
 }
 
-template <int WAVES, bool PACK, bool FAR>
+template <int WAVES, int FORM, bool FAR>
 __global__ void __launch_bounds__(WAVES * 64)
 qsa_skinny_gemm_fp8_half(SkinnyArgs p) {
-  skinny_stream<WAVES, 1, 1, true, PACK, false, false, true, FAR, true>(p);
+  skinny_stream<WAVES, 1, 1, true, FORM, false, false, true, FAR, true>(p);
 }
 
 template <int WAVES, int TILES, bool NORM, bool GLU, bool RES>
 static void fp8_go(const SkinnyArgs& p, int pack, hipStream_t st) {
   const dim3 grid(p.N / (16 * TILES)), block(WAVES * 64);
-#define QSA_GO_AS(MT, PACK, FAR)                                              \
+#define QSA_GO_AS(MT, FORM, FAR)                                              \
   hipLaunchKernelGGL(                                                         \
-      (qsa_skinny_gemm_fp8<WAVES, TILES, MT, PACK, NORM, GLU, RES, FAR>),     \
+      (qsa_skinny_gemm_fp8<WAVES, TILES, MT, FORM, NORM, GLU, RES, FAR>),     \
       grid, block, 0, st, p)
-#define QSA_GO(MT, PACK)                                                      \
-  if (p.far) QSA_GO_AS(MT, PACK, true); else QSA_GO_AS(MT, PACK, false)
-  if (p.M <= 16) {
-    if (pack) { QSA_GO(1, true); } else { QSA_GO(1, false); }
+#define QSA_GO(MT, FORM)                                                      \
+  if (p.far) QSA_GO_AS(MT, FORM, true); else QSA_GO_AS(MT, FORM, false)
+  if (p.M <= FEW && !pack) {
+    QSA_GO(1, FEW_ROWS);
+  } else if (p.M <= 16) {
+    if (pack) { QSA_GO(1, PACKED); } else { QSA_GO(1, ROWS); }
   } else {
-    if (pack) { QSA_GO(2, true); } else { QSA_GO(2, false); }
+    if (pack) { QSA_GO(2, PACKED); } else { QSA_GO(2, ROWS); }
   }
 #undef QSA_GO
 #undef QSA_GO_AS
@@ -131,17 +133,22 @@ extern "C" int qsa_skinny_fp8_half(int M, int N, long long K) {
 
 static void fp8_half(const SkinnyArgs& p, int pack, hipStream_t st) {
   const dim3 grid(p.N / 8);
-#define QSA_HALF_AS(WAVES, PACK, FAR)                                         \
-  hipLaunchKernelGGL((qsa_skinny_gemm_fp8_half<WAVES, PACK, FAR>), grid,      \
+#define QSA_HALF_AS(WAVES, FORM, FAR)                                         \
+  hipLaunchKernelGGL((qsa_skinny_gemm_fp8_half<WAVES, FORM, FAR>), grid,      \
                      dim3(WAVES * 64), 0, st, p)
-#define QSA_HALF(WAVES, PACK)                                                 \
-  if (p.far) QSA_HALF_AS(WAVES, PACK, true);                                  \
-  else QSA_HALF_AS(WAVES, PACK, false)
+#define QSA_HALF(WAVES, FORM)                                                 \
+  if (p.far) QSA_HALF_AS(WAVES, FORM, true);                                  \
+  else QSA_HALF_AS(WAVES, FORM, false)
+#define QSA_HALF_OF(WAVES)                                                    \
+  if (pack) { QSA_HALF(WAVES, PACKED); }                                      \
+  else if (p.M <= FEW) { QSA_HALF(WAVES, FEW_ROWS); }                         \
+  else { QSA_HALF(WAVES, ROWS); }
   if (p.K < 6144) {                    // a wave has 6 or more steps
-    if (pack) { QSA_HALF(4, true); } else { QSA_HALF(4, false); }
+    QSA_HALF_OF(4)
   } else {
-    if (pack) { QSA_HALF(8, true); } else { QSA_HALF(8, false); }
+    QSA_HALF_OF(8)
   }
+#undef QSA_HALF_OF
 #undef QSA_HALF
 #undef QSA_HALF_AS
 }

@@ -82,13 +82,29 @@ __device__ __forceinline__ long long packed_at(int row, int k, int mt) {
          ((row & 15) + ((k >> 3) & 3) * 16) * 8 + (k & 7);
 }
 
-template <int WAVES, int TILES, int MT, bool FP8, bool PACK, bool NORM,
+// How A is given: rows, fragments, or up to FEW rows.  Fragments of few rows are mostly
+// lanes of rows that do not exist, and a load brings 1 KB into registers all the same,
+// two of them for each of W: a wave loads the rows that are there, 128 bytes of each for
+// a step, and lays them out in LDS (us a step: 8 layers of width 2048, 4 rows 269 -> 258;
+// 16 layers, 3 rows 501 -> 484; one row level).
+enum { ROWS = 0, PACKED = 1, FEW_ROWS = 2 };
+#define FEW 4
+
+template <int WAVES, int TILES, int MT, bool FP8, int FORM, bool NORM,
           bool GLU, bool RES, bool FAR, bool HALF = false>
 __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   static_assert(!HALF || (FP8 && RES && TILES == 1 && MT == 1), "half a tile");
+  static_assert(FORM != FEW_ROWS || MT == 1, "few rows are one tile");
+  constexpr bool PACK = FORM == PACKED, LITTLE = FORM == FEW_ROWS;
   constexpr int WL = FP8 ? 1 : 2;      // 16 B loads of a tile per step
   constexpr int PER = TILES * WL * 4 + MT * 8;
   constexpr int U = PER <= 12 ? 4 : PER <= 24 ? 2 : 1;
+  // LITTLE: a wave's part of A for a group: rows of U steps of 128 bytes, 64 apart
+  // in the banks; of half a tile both parts of K
+  constexpr int LR = U * 64 + 32, LH = FEW * LR;  // elements of a row, of a part
+  constexpr int AREA = LITTLE ? (HALF ? 2 : 1) * LH : 0;
+  constexpr int AL = LITTLE ? (HALF ? 2 : 1) * FEW * U * 8 / 64 : 1;
+  __shared__ __attribute__((aligned(16))) bf16_t few[WAVES * AREA + 8];
   __shared__ float red[WAVES][TILES * MT * 4][64];
   __shared__ float inv_s[32];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -152,9 +168,21 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   const int stream = (HALF ? 2 : 1) * steps * WB;
   const unsigned wo = (unsigned)(tcol * 4 + hi) * 16 +
                       (HALF ? (unsigned)(col >> 3) * steps * WB : 0u);
-  unsigned ao[MT];
+  unsigned ao[LITTLE ? AL : MT];
+  int am[AL], lo[AL];                             // LITTLE: steps ahead; place in LDS
+  if constexpr (LITTLE) {
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+    for (int j = 0; j < AL; ++j) {
+      const int i = j * 64 + lane, seg = i & 7, u = i / 8 % U;
+      const int m = i / (8 * U) % FEW, h = i / (8 * U * FEW);
+      am[j] = m < p.M ? u * WAVES : 0x40000000;
+      ao[j] = ((unsigned)m * (unsigned)p.lda + (unsigned)(u * WAVES * 64 + seg * 8) +
+               (unsigned)h * steps * 64) * 2;
+      lo[j] = wave * AREA + h * LH + m * LR + u * 64 + seg * 8;
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < (LITTLE ? 0 : MT); ++m)
     if constexpr (HALF)
       ao[m] = ((unsigned)(col >> 3) * steps * (PACK ? 1024 : 64) +
                (PACK ? ((col & 7) + hi * 16) * 8
@@ -166,7 +194,8 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
 
   struct Group {
     u32x4_v w[U][TILES][WL];
-    bf16x8_v a[U][MT][2];
+    bf16x8_v a[LITTLE ? 1 : U][MT][2];
+    u32x4_v few[AL];
   };
   f32x4_v acc[TILES][MT];
 #pragma unroll
@@ -174,7 +203,14 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[t][m] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
 
+  const rsrc rf = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, 0x7fffffff,
+                                                    0x00027000);
   auto load = [&](Group& g, int base) {
+    if constexpr (LITTLE)
+#pragma unroll
+      for (int j = 0; j < AL; ++j)
+        g.few[j] = __builtin_amdgcn_raw_buffer_load_b128(
+              rf, base + am[j] < steps ? ao[j] : 0xffffffffu, base * 128, 0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = base + u * WAVES;
@@ -190,6 +226,7 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
           g.w[u][t][i] = __builtin_amdgcn_raw_buffer_load_b128(
               rw, wo + i * 1024, at * WB, FAR ? QSA_NT : 0);
       }
+      if constexpr (LITTLE) continue;
       const rsrc ra = __builtin_amdgcn_make_buffer_rsrc(
           (void*)p.A, 0, in ? 0x7fffffff : 0, 0x00027000);
 #pragma unroll
@@ -202,7 +239,28 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
                             at * (PACK ? MT * 2048 : 128), 0));
     }
   };
+  const bf16_t* const fa =
+      few + wave * AREA +
+      (HALF ? (col >> 3) * LH + min(col & 7, p.M - 1) * LR
+            : min(col, p.M - 1) * LR) + hi * 8;
   auto compute = [&](Group& g) {
+    bf16x8_v f[U][2];
+    if constexpr (LITTLE) {            // a wave's own: its order suffices
+#pragma unroll
+      for (int j = 0; j < AL; ++j)
+        *reinterpret_cast<u32x4_v*>(few + lo[j]) = g.few[j];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          f[u][i] = *reinterpret_cast<const bf16x8_v*>(fa + u * 64 + i * 32);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -216,7 +274,8 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
             w = __builtin_bit_cast(bf16x8_v, g.w[u][t][i]);
 #pragma unroll
           for (int m = 0; m < MT; ++m)
-            acc[t][m] = mfma_bf16(g.a[u][m][i], w, acc[t][m]);
+            acc[t][m] = mfma_bf16(LITTLE ? f[u][i] : g.a[LITTLE ? 0 : u][m][i], w,
+                                  acc[t][m]);
         }
   };
 
