@@ -554,7 +554,8 @@ extern "C" void qsa_paged_attn_mfma_launch(
   // 120 578 -> 552, 8 rows 715 -> 678; cut to 24 MB of a 4096-wide one's 75 it
   // cost 1-2%.
   const long long bytes = warm_bytes[0] + warm_bytes[1];
-  if (k && NS == 1 && grid.x <= 64 && bytes >= 16 && bytes <= 24 << 20) {
+  if (k && NS == 1 && B > 4 && grid.x <= 64 && bytes >= 16 &&
+      bytes <= 24 << 20) {
     for (int i = 0; i < 2; ++i) {
       p.warm[i] = static_cast<const u32x4_v*>(warm[i]);
       p.warm_n[i] = warm_bytes[i] / 16;
