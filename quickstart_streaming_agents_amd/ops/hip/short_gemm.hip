@@ -13,6 +13,7 @@
 // us, library / rows_gemm -> here:
 //   384 x 512  at 100 / 400 / 1000 rows 5.4 / 5.5 / 6.2, 4.5 -> 4.2 / 4.3 / 4.4
 //   1536 x 384 at 40 rows 5.0, 4.1 -> 3.8;  512 x 256 at 700 5.1, 4.0 -> 3.6
+//   of few rows: qsa_few_gemm
 //   at 8800 rows 1536 x 384 18.3, 17.0 -> 20.7, 384 x 512 10.7, 8.0 -> 11.7, 3072
 //   x 384 with the activation 72, 32 -> 34.8
 #include "lm_common.h"
@@ -73,24 +74,28 @@ qsa_short_gemm(ShortArgs p) {
     return (((row >> 4) * 2 + half) * 64 + h * 16 +
             ((row & 15) ^ (h << 1 | half << 3))) * 8;
   };
-  u32x4_v ar[AL], br[BL];
-  auto load = [&](int k) {
+  // PF steps of K are in registers or under way besides the two in LDS
+  constexpr int PF = MT == 1 ? 6 : 1;  // (384 x 1536 of 15 rows 7.2 -> 6.2 us)
+  u32x4_v ar[PF][AL], br[PF][BL];
+  const int steps = p.K >> 6;
+  auto load = [&](int q, int step) {   // beyond the end: the last one again
+    const int k = min(step, steps - 1) * 64;
 #pragma unroll
     for (int j = 0; j < AL; ++j)
-      ar[j] = *reinterpret_cast<const u32x4_v*>(ap[j] + k);
+      ar[q][j] = *reinterpret_cast<const u32x4_v*>(ap[j] + k);
 #pragma unroll
     for (int j = 0; j < BL; ++j)
-      br[j] = *reinterpret_cast<const u32x4_v*>(bp[j] + k);
+      br[q][j] = *reinterpret_cast<const u32x4_v*>(bp[j] + k);
   };
-  auto store = [&](bf16_t* t) {
+  auto store = [&](int q, bf16_t* t) {
 #pragma unroll
     for (int j = 0; j < AL; ++j)
       *reinterpret_cast<u32x4_v*>(
-          t + place(r8 + 32 * j, seg >> 2, seg & 3)) = ar[j];
+          t + place(r8 + 32 * j, seg >> 2, seg & 3)) = ar[q][j];
 #pragma unroll
     for (int j = 0; j < BL; ++j)
       *reinterpret_cast<u32x4_v*>(
-          t + BM * 64 + place(r8 + 32 * j, seg >> 2, seg & 3)) = br[j];
+          t + BM * 64 + place(r8 + 32 * j, seg >> 2, seg & 3)) = br[q][j];
   };
   f32x4_v acc[MT][NT];
 #pragma unroll
@@ -98,11 +103,7 @@ qsa_short_gemm(ShortArgs p) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
   const int wm = (wave >> 1) * MT, wn = (wave & 1) * NT;
-  const int steps = p.K >> 6;
-  load(0);
-  store(lds);
-  load(min(1, steps - 1) * 64);
-  for (int s = 0; s < steps; ++s) {
+  auto step = [&](int s, int q) {      // q: where the next step's registers are
     lds_barrier();
     const bf16_t* t = lds + (s & 1) * TILE;
 #pragma unroll
@@ -122,11 +123,22 @@ qsa_short_gemm(ShortArgs p) {
         for (int j = 0; j < NT; ++j)
           acc[i][j] = mfma_bf16(b[j], a[i], acc[i][j]);
     }
-    if (s + 1 < steps) {
-      store(lds + ((s + 1) & 1) * TILE);
-      load(min(s + 2, steps - 1) * 64);
+    if (PF > 1 || s + 1 < steps) {     // no branch around loads that are counted
+      store(q, lds + ((s + 1) & 1) * TILE);       // behind the last: not read
+      load(q, s + 1 + PF);
     }
-  }
+  };
+#pragma unroll
+  for (int q = 0; q < PF; ++q) load(q, q);
+  store(0, lds);
+  load(0, PF);
+  int s = 0;
+  for (; s + PF <= steps; s += PF)
+#pragma unroll
+    for (int q = 0; q < PF; ++q) step(s + q, (q + 1) % PF);
+#pragma unroll
+  for (int q = 0; q < PF - 1; ++q)
+    if (s + q < steps) step(s + q, (q + 1) % PF); // uniform over the block
   // results through LDS: a lane has 4 columns (hi*4..) of row col of each tile
   lds_barrier();
   bf16_t* o = lds + wave * (16 * MT * OP);
@@ -160,6 +172,91 @@ qsa_short_gemm(ShortArgs p) {
   }
 }
 
+// Few rows: 8 waves of a block share K, for 32 rows x 16 columns (with GLU of gate and
+// up each), and all of a wave's operands are on their way to registers at once, so that
+// a product is one latency of memory and a sum in LDS, where the tiles above wait for a
+// barrier every 64 of K.
+template <int U, bool GLU>
+__global__ void __launch_bounds__(512)
+qsa_few_gemm(ShortArgs p) {
+  constexpr int NW = 8, T = GLU ? 2 : 1, PITCH = 68;     // banks of a row's sums differ
+  __shared__ float red[NW][T * 8 * PITCH];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, hi = lane >> 4;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 32;
+  const int steps = p.K >> 6;
+  const bf16_t *ap[2], *bp[T];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+    ap[m] = p.A + (long long)min(m0 + m * 16 + col, p.M - 1) * p.lda + hi * 8;
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    bp[t] = p.W + (long long)(n0 + col + t * (p.N >> 1)) * p.K + hi * 8;
+  f32x4_v acc[T][2];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int m = 0; m < 2; ++m) acc[t][m] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  for (int s = wave; s < steps; s += NW * U) {
+    bf16x8_v a[U][2][2], b[U][T][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(s + u * NW, steps - 1) * 64;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+          b[u][t][i] = *reinterpret_cast<const bf16x8_v*>(bp[t] + k + i * 32);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          a[u][m][i] = *reinterpret_cast<const bf16x8_v*>(ap[m] + k + i * 32);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s + u * NW >= steps) break;             // uniform over the wave
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+            acc[t][m] = mfma_bf16(b[u][t][i], a[u][m][i], acc[t][m]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave][((t * 2 + m) * 4 + r) * PITCH + lane] = acc[t][m][r];
+  __syncthreads();
+  // a lane had columns hi * 4 .. + 3 of row `col`; a thread takes one number
+  const int row = tid >> 4, c = tid & 15;
+  const int at = ((row >> 4) * 4 + (c & 3)) * PITCH + (c >> 2) * 16 + (row & 15);
+  float v[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    v[t] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) v[t] += red[w][t * 8 * PITCH + at];
+  }
+  if constexpr (GLU) v[0] = v[0] / (1.f + __expf(-v[0])) * v[T - 1];
+  if (m0 + row < p.M)
+    p.C[(long long)(m0 + row) * (GLU ? p.N >> 1 : p.N) + n0 + c] = cvt_bf16(v[0]);
+}
+
+template <int U>
+static void few_go(const ShortArgs& p, int glu, hipStream_t st) {
+  const dim3 grid((unsigned)(p.N / (glu ? 32 : 16)), (unsigned)((p.M + 31) / 32));
+  if (glu)
+    hipLaunchKernelGGL((qsa_few_gemm<U, true>), grid, dim3(512), 0, st, p);
+  else
+    hipLaunchKernelGGL((qsa_few_gemm<U, false>), grid, dim3(512), 0, st, p);
+}
+
 template <int MT, int NT>
 static void short_go(ShortArgs p, int glu, hipStream_t st) {
   p.NB = (p.N + 32 * NT - 1) / (32 * NT);
@@ -171,6 +268,15 @@ static void short_go(ShortArgs p, int glu, hipStream_t st) {
   else
     hipLaunchKernelGGL((qsa_short_gemm<MT, NT, false>), grid, dim3(256), 0, st,
                        p);
+}
+
+// Blocks of 32 rows and 16 columns while each has a CU to itself, with the gate's half
+// of them (us, tiles / so: 1536 x 384 of 15 rows 3.21 / 2.59, of 60, 192 blocks, 3.24 /
+// 2.92, of 130, 480 blocks, 3.30 / 4.06; 384 x 1536 of 15 rows 7.2 / 4.7, of 250, 192
+// blocks, 7.4 / 5.9, of 400, 312 blocks, 7.4 / 9.8; gated 1536 x 384 of 15 rows 3.31 /
+// 3.00, of 60, 96 blocks, 3.34 / 3.36, of 130, 240 blocks, 3.37 / 3.46).
+extern "C" bool qsa_few_gemm_takes(long long M, long long N, bool glu) {
+  return (M + 31) / 32 * (N / (glu ? 32 : 16)) <= (glu ? 128 : 256);
 }
 
 // Tiles of 128 x 128 once two rounds of blocks are left, 64 x 64 while they
@@ -186,6 +292,10 @@ extern "C" void qsa_short_gemm_launch(const bf16_t* A, const bf16_t* W,
   auto blocks = [&](int b) {
     return (long long)((M + b - 1) / b) * ((N + b - 1) / b);
   };
+  if (qsa_few_gemm_takes(M, N, glu)) {
+    if (K <= 512) few_go<1>(p, glu, st); else few_go<3>(p, glu, st);
+    return;
+  }
   if (blocks(128) >= 512) short_go<4, 4>(p, glu, st);
   else if (blocks(64) >= 128) short_go<2, 2>(p, glu, st);
   else short_go<1, 2>(p, glu, st);

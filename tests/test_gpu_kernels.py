@@ -1376,6 +1376,27 @@ def test_short_gemm(ext, M, N, K, glu):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + err + 1e-30).all()
 
 
+@pytest.mark.parametrize("M,N,K,glu", [
+    (1, 32, 64, False), (32, 384, 1536, False), (40, 96, 1088, False),
+    (17, 48, 576, False), (250, 512, 1600, False), (31, 64, 2112, True),
+    (33, 1536, 448, True), (5, 32, 512, True)])
+def test_short_gemm_few_rows(ext, M, N, K, glu):
+    """K in shares of eight waves: fewer steps than waves, remainders of the steps
+    that are under way together, ragged rows.  The bound is that of the tiles."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, generator=g).bfloat16().to(dev())[:, :K]
+    w = torch.randn(N, K, generator=g).mul(K ** -0.5).bfloat16().to(dev())
+    got = ext.short_gemm(x, w, glu).double()
+    a, b = x.double(), w.double()
+    want, err = a @ b.T, K * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    if glu:
+        z, u = want.chunk(2, 1)
+        want = torch.nn.functional.silu(z) * u
+        err = 1.1 * err[:, :N // 2] * u.abs() + z.abs() * err[:, N // 2:] + \
+            2.0 ** -20 * want.abs()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + err + 1e-30).all()
+
+
 def test_mean_rows(ext):
     lens = [1, 3, 4, 5, 700]
     x = torch.randn(sum(lens), 520, device=dev()).bfloat16()
