@@ -26,7 +26,7 @@ import torch
 import torch.nn.functional as F
 
 from ..ops import dispatch as D
-from ..ops import have_ext, have_lm_ext
+from ..ops import have_ext, have_lm_ext, lm_ext
 from ..vector.index import EMBED_DIM
 from .layers import ints_to_device
 from .tokenizer import BpeTokenizer
@@ -132,8 +132,7 @@ class EmbeddingEncoder:
     def _embed_rows(self, ids: np.ndarray, lens: np.ndarray) -> torch.Tensor:
         """Mean-pooled final states [n, hidden] f32 of texts whose tokens follow
         each other in ids, all rows in one concatenation without padding."""
-        c, dev, project = self.cfg, self.device, self._project
-        n = len(lens)
+        dev, n = self.device, len(lens)
         off = np.cumsum(lens) - lens
         nqb = -(-lens // self.QROWS)
         qb_item = np.repeat(np.arange(n), nqb)
@@ -142,6 +141,26 @@ class EmbeddingEncoder:
         toks, qb_item, qb_pos0, off, lens_t = ints_to_device(
             dev, ids, qb_item, qb_pos0, off, lens)
         res = self.tok_embed.index_select(0, toks)
+        final_h = self._native_layers(res, qb_item, qb_pos0, off, lens_t)
+        if final_h is None:
+            final_h = self._layers_by_call(res, qb_item, qb_pos0, off, lens_t)
+        return D.ext().mean_rows(final_h, off, lens_t)
+
+    def _native_layers(self, res, qb_item, qb_pos0, off, lens):
+        """All layers as one call that launches the kernels of _layers_by_call, or
+        None where it does not take them."""
+        if not have_lm_ext() or type(res) is not torch.Tensor or \
+                torch.compiler.is_compiling():
+            return None
+        c = self.cfg
+        weights = [Ly[k] for Ly in self.layers for k in
+                   ("attn_norm", "mlp_norm", "wqkv", "wo", "wgu", "wdown")]
+        return lm_ext().encoder_layers(
+            res, weights, self.final_norm, self.rope_cos, self.rope_sin,
+            qb_item, qb_pos0, off, lens, c.n_heads, self.scale, c.norm_eps)
+
+    def _layers_by_call(self, res, qb_item, qb_pos0, off, lens):
+        c, project = self.cfg, self._project
         mlp_out = None
         for Ly in self.layers:
             if mlp_out is None:
@@ -151,14 +170,12 @@ class EmbeddingEncoder:
                                        c.norm_eps)
             attn = D.ext().encoder_attn(
                 project(h, Ly["wqkv"]), self.rope_cos, self.rope_sin,
-                qb_item, qb_pos0, off, lens_t, c.n_heads, self.scale)
+                qb_item, qb_pos0, off, lens, c.n_heads, self.scale)
             o = project(attn, Ly["wo"], parts=True)
             h = D.rmsnorm_residual(o, res, Ly["mlp_norm"], c.norm_eps)
             act = project(h, Ly["wgu"], glu=True)
             mlp_out = project(act, Ly["wdown"], parts=True)
-        final_h = D.rmsnorm_residual(mlp_out, res, self.final_norm,
-                                     c.norm_eps)
-        return D.ext().mean_rows(final_h, off, lens_t)
+        return D.rmsnorm_residual(mlp_out, res, self.final_norm, c.norm_eps)
 
     def _embed_padded(self, enc: list[list[int]]) -> torch.Tensor:
         """The same by a padded batch and a materialized softmax (CPU)."""

@@ -45,6 +45,14 @@ extern "C" void qsa_residual_norm_launch(float*, const void*, long long,
     const float*, int, const void*, const void*, const long long*, float, const void*,
     const void*, const void*, void*, long long, int, int, float, int, int,
     int, int, hipStream_t);
+extern "C" void qsa_rmsnorm_launch(const bf16_t*, const bf16_t*, bf16_t*, bf16_t*,
+    long long, int, float, hipStream_t);
+extern "C" void qsa_short_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*, int, int,
+    int, long long, int, hipStream_t);
+extern "C" bool qsa_few_gemm_takes(long long, long long, bool);
+extern "C" void qsa_encoder_attn_launch(const bf16_t*, const float*, const float*, int,
+    const int*, const int*, const int*, const int*, bf16_t*, int, int, int, float,
+    hipStream_t);
 extern "C" void qsa_rmsnorm_shares_launch(const float*, int, bf16_t*,
     const bf16_t*, bf16_t*, long long, int, float, hipStream_t);
 extern "C" void qsa_glu_launch(const void*, const float*, int, const void*,
@@ -1297,6 +1305,147 @@ Tensor glu_gemm(Tensor a, Tensor w, bool gelu, bool rounded, bool far) {
   return gemm_run(a, w, gelu ? 2 : rounded ? 1 : 3, false, far);
 }
 
+// ---- encoder ----------------------------------------------------------------
+
+// A product of the encoder, planned once for all layers: short_gemm.hip's, or as gemm()
+// and its like run it.
+struct EncoderProduct {
+  bool brief = false;
+  GemmPlan plan;
+  int M, N, K, act;
+
+  bool set(const Tensor& a, const Tensor& w, bool glu, bool parts) {
+    if (!gemm_takes(a, w, glu)) return false;
+    const int64_t m = a.size(0), n = w.size(0), k = w.size(1);
+    M = (int)m, N = (int)n, K = (int)k, act = glu ? 3 : 0;
+    brief = n % 32 == 0 && n < 1 << 20 &&
+            (k <= 512 || m <= 32 ||
+             (k <= 2048 && !glu && qsa_few_gemm_takes(m, n, false))) &&
+            (m + 31) / 32 * ((n + 63) / 64) <= 192;
+    if (brief) return true;
+    if (!gemm_sizes(m, n, k, a.stride(0), glu)) return false;
+    plan = gemm_choice(m, n, k, a.stride(0), act, parts);
+    return true;
+  }
+  int shares() const { return brief || plan.wide ? 1 : plan.shares; }
+  int64_t part_size() const { return shares() > 1 ? (int64_t)shares() * M * N : 0; }
+  void run(const Tensor& a, const Tensor& w, bf16_t* out, float* part,
+           hipStream_t st) const {
+    const long long lda = a.stride(0);
+    if (brief) {
+      qsa_short_gemm_launch(u16(a), u16(w), out, M, N, K, lda, act != 0, st);
+    } else if (!plan.wide) {
+      qsa_rows_gemm_launch(u16(a), u16(w), out, shares() > 1 ? part : nullptr, M, N, K,
+                           lda, plan.tile, plan.shares, act, false, st);
+    } else {
+      const int64_t cols = act ? N / 2 : N;
+      qsa_wide_gemm_launch(u16(a), u16(w), out, plan.rows, N, K, lda, plan.tile, act,
+                           st);
+      if (plan.rows < M)
+        qsa_wide_gemm_launch(u16(a) + plan.rows * lda, u16(w), out + plan.rows * cols,
+                             M - plan.rows, N, K, lda, plan.rest, act, st);
+    }
+  }
+};
+
+// The layers of the retrieval encoder on rows res [T, H], which they change, and the
+// norm behind them; weights: attention's norm and feed-forward's, q k v, output,
+// [gate; up] and down of every layer.  The kernels and their choice are those of the
+// calls one by one (models/encoder.py), which are for all that this does not take: then
+// there is no result and nothing has changed.  Up to some 2000 rows a call is as long as
+// the host takes for its launches: 84 calls from Python at 5 us each, products planned
+// each time; here they are planned once, and operands lie in the same places in every
+// layer (texts embedded in one call, us: one of 15 tokens 543 -> 400, 8 of some 50 584 ->
+// 503, from some 1000 tokens on level).
+OptTensor encoder_layers(Tensor res, std::vector<Tensor> weights, Tensor final_norm,
+                         Tensor cos_t, Tensor sin_t, Tensor qb_item, Tensor qb_t0,
+                         Tensor off, Tensor len, int64_t heads, double scale,
+                         double eps) {
+  const size_t layers = weights.size() / 6;
+  if (layers == 0 || weights.size() % 6 || !res.is_cuda() || res.dim() != 2 ||
+      res.scalar_type() != at::kBFloat16 || !res.is_contiguous() || res.size(0) == 0 ||
+      !aligned(res, 16) || !no_observer() || !unobserved(res) || heads <= 0 ||
+      heads % 4)
+    return c10::nullopt;
+  const int64_t T = res.size(0), H = res.size(1), A = weights[3].size(-1),
+                F = weights[5].size(-1), D = A / heads;
+  if (H % 8 || H > 8192 || A % heads || (D != 64 && D != 128)) return c10::nullopt;
+  auto norm_ok = [&](const Tensor& w) {
+    return w.dim() == 1 && w.size(0) == H && w.is_contiguous() && aligned(w, 16) &&
+           w.scalar_type() == at::kBFloat16 && w.device() == res.device() &&
+           unobserved(w);
+  };
+  auto weight_ok = [&](const Tensor& w, int64_t n, int64_t k) {
+    return w.dim() == 2 && w.size(0) == n && w.size(1) == k && w.is_contiguous() &&
+           aligned(w, 16) && w.scalar_type() == at::kBFloat16 &&
+           w.device() == res.device() && unobserved(w);
+  };
+  auto layer_ok = [&](size_t i) {
+    const Tensor* w = &weights[i * 6];
+    return norm_ok(w[0]) && norm_ok(w[1]) && weight_ok(w[2], 3 * A, H) &&
+           weight_ok(w[3], H, A) && weight_ok(w[4], 2 * F, H) && weight_ok(w[5], H, F);
+  };
+  if (!norm_ok(final_norm) || !layer_ok(0)) return c10::nullopt;
+  CHK_F32(cos_t); CHK_F32(sin_t);
+  CHK_I32(qb_item); CHK_I32(qb_t0); CHK_I32(off); CHK_I32(len);
+  TORCH_CHECK(cos_t.dim() == 2 && cos_t.size(0) >= 1 && cos_t.size(1) == D / 2 &&
+                  sin_t.sizes() == cos_t.sizes(), "cos/sin [positions, D/2]");
+  TORCH_CHECK(qb_item.numel() == qb_t0.numel() && off.numel() == len.numel(), "maps");
+  const hipStream_t st = cur_stream();
+  Tensor h = torch::empty_like(res);
+  qsa_rmsnorm_launch(u16(res), u16(weights[0]), u16m(h), nullptr, T, (int)H, (float)eps,
+                     st);
+  // Until a product has been added to res nothing has changed: what the first layer
+  // does before that is under way while the rest is looked at and planned.
+  Tensor y = torch::empty_like(res);
+  Tensor attn = torch::empty({T, A}, res.options());
+  Tensor act = torch::empty({T, F}, res.options());
+  Tensor qkv = torch::empty({T, 3 * A}, res.options());
+  EncoderProduct p[4];
+  Tensor part;
+  auto space = [&](int q) {            // for the shares of product q
+    if (p[q].part_size() > (part.defined() ? part.numel() : 0))
+      part = torch::empty({p[q].part_size()}, res.options().dtype(at::kFloat));
+  };
+  auto shares = [&] { return part.defined() ? part.data_ptr<float>() : nullptr; };
+  auto attention = [&](const Tensor* w) {
+    p[0].run(h, w[2], u16m(qkv), shares(), st);
+    qsa_encoder_attn_launch(u16(qkv), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(),
+                            (int)cos_t.size(0), qb_item.data_ptr<int>(),
+                            qb_t0.data_ptr<int>(), off.data_ptr<int>(),
+                            len.data_ptr<int>(), u16m(attn), (int)qb_item.numel(),
+                            (int)heads, (int)D, (float)scale, st);
+  };
+  // a product for the norm behind it, which adds it to res and leaves the norm in h
+  auto added = [&](int q, const Tensor& a, const Tensor& w, const Tensor& norm) {
+    const bool split = p[q].shares() > 1;
+    p[q].run(a, w, split ? nullptr : u16m(y), shares(), st);
+    if (split)
+      qsa_rmsnorm_shares_launch(shares(), p[q].shares(), u16m(res), u16(norm), u16m(h),
+                                T, (int)H, (float)eps, st);
+    else
+      qsa_rmsnorm_launch(u16(y), u16(norm), u16m(h), u16m(res), T, (int)H, (float)eps,
+                         st);
+  };
+  if (!p[0].set(h, weights[2], false, false)) return c10::nullopt;
+  space(0);
+  attention(&weights[0]);
+  if (!p[1].set(attn, weights[3], false, true) || !p[2].set(h, weights[4], true, false) ||
+      !p[3].set(act, weights[5], false, true))
+    return c10::nullopt;
+  for (size_t i = 1; i < layers; ++i)
+    if (!layer_ok(i)) return c10::nullopt;
+  for (int q = 1; q < 4; ++q) space(q);
+  for (size_t i = 0; i < layers; ++i) {
+    const Tensor* w = &weights[i * 6];
+    if (i) attention(w);
+    added(1, attn, w[3], w[1]);
+    p[2].run(h, w[4], u16m(act), shares(), st);
+    added(3, act, w[5], i + 1 < layers ? w[6] : final_norm);
+  }
+  return h;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("residual_norm", &residual_norm,
         "f32 residual update (+ embedding row, + vector) and layer/rms norm");
@@ -1356,6 +1505,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("a"), py::arg("w"), py::arg("gelu"), py::arg("rounded"),
         py::arg("far") = false);
   m.def("glu_gemm_ok", &glu_gemm_ok, "whether a gated product is one of theirs");
+  m.def("encoder_layers", &encoder_layers,
+        "the layers of the retrieval encoder, or None: call by call");
   m.def("gemm_plan", &gemm_plan, "the same where gemm() takes wide_gemm, else -1");
   m.def("wide_gemm", &wide_gemm, "GEMM of many rows by a given tile");
   m.def("wide_gemm_plan", &wide_gemm_plan, "tiles and rows of a product");

@@ -39,7 +39,8 @@ MODULES = {
                 "streaming.hip", "encoder_attn.hip", "short_gemm.hip"],
     "qsa_lm_hip": ["lm_ops.cpp", "lm_elementwise.hip", "retention.hip",
                    "latent_attn.hip", "short_conv.hip", "gqa_attn.hip", "ssd.hip",
-                   "skinny_gemm.hip", "rows_gemm.hip", "wide_gemm.hip"],
+                   "skinny_gemm.hip", "rows_gemm.hip", "wide_gemm.hip",
+                   "elementwise.hip", "encoder_attn.hip", "short_gemm.hip"],
 }
 
 
