@@ -725,7 +725,7 @@ qsa_retention_out(const bf16_t* __restrict__ x, long long xstride,
           ldv<bf16_t, 4>(g + e0, gv);
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            o[r] = acc[u][rt][r] * inv * (gv[r] / (1.f + __expf(-gv[r])));
+            o[r] = acc[u][rt][r] * inv * (gv[r] * gate_f(gv[r]));
           stv<bf16_t, 4>(orow + e0, o);
         }
       }

@@ -150,7 +150,7 @@ qsa_short_gemm(ShortArgs p) {
       if constexpr (GLU) {
         const f32x4_v u = acc[i][j + 1];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = v[r] / (1.f + __expf(-v[r])) * u[r];
+        for (int r = 0; r < 4; ++r) v[r] = v[r] * gate_f(v[r]) * u[r];
       }
       *reinterpret_cast<uint2*>(
           o + (i * 16 + col) * OP + (GLU ? j / 2 : j) * 16 + hi * 4) =
@@ -243,7 +243,7 @@ qsa_few_gemm(ShortArgs p) {
 #pragma unroll
     for (int w = 0; w < NW; ++w) v[t] += red[w][t * 8 * PITCH + at];
   }
-  if constexpr (GLU) v[0] = v[0] / (1.f + __expf(-v[0])) * v[T - 1];
+  if constexpr (GLU) v[0] = v[0] * gate_f(v[0]) * v[T - 1];
   if (m0 + row < p.M)
     p.C[(long long)(m0 + row) * (GLU ? p.N >> 1 : p.N) + n0 + c] = cvt_bf16(v[0]);
 }
