@@ -11,16 +11,20 @@
 
 struct ConvSpan { int r0, t0, t1, n, p0, slot; };
 
-__device__ __forceinline__ ConvSpan conv_span(const ConvStep& st, int c) {
+// The rows of chunk c, or of one of the `parts` that share them: as short as a filter is
+// long, so that still only the first of a portion looks at the tail.
+#define CONV_PARTS 4
+__device__ __forceinline__ ConvSpan conv_span(const ConvStep& st, int c,
+                                              int part = 0, int parts = 1) {
   ConvSpan s;
   if (st.item) {
-    const int it = st.item[c];
+    const int it = st.item[c], rows = CONV_ROWS / parts;
     s.r0 = st.off[it];
-    s.t0 = st.t0[c];
+    s.t0 = st.t0[c] + part * rows;
     s.n = st.len[it];
     s.p0 = st.start[it];
     s.slot = st.slots[it];
-    s.t1 = min(s.t0 + CONV_ROWS, s.n);
+    s.t1 = min(s.t0 + rows, s.n);
   } else {
     s.r0 = c;
     s.t0 = 0;
@@ -111,6 +115,8 @@ __device__ __forceinline__ void conv_rows(
       }
     };
     if (s.t1 - s.t0 == 1) walk(std::integral_constant<int, 1>{});
+    else if (s.t1 - s.t0 <= CONV_ROWS / CONV_PARTS)
+      walk(std::integral_constant<int, CONV_ROWS / CONV_PARTS>{});
     else walk(std::integral_constant<int, NP == 1 && sizeof(T) == 2 ? 16 : 8>{});
     if (s.t0 == 0) {
       // The new tail: of a whole portion, as of a single token, the window, else the
@@ -192,7 +198,8 @@ __host__ __device__ inline int conv_qkv_units(const ConvQkv& p, int vec) {
 #define CONV_ONE_TAPS 4
 template <typename T, int VEC, bool ONE = false>
 __device__ __forceinline__ void conv_qkv_unit(const ConvQkv& p, int chunk,
-                                              int u) {
+                                              int u, int part = 0,
+                                              int parts = 1) {
   const T* x = (const T*)p.x;
   const long long xstride = p.xstride;
   const float* __restrict__ w = p.w;
@@ -209,8 +216,8 @@ __device__ __forceinline__ void conv_qkv_unit(const ConvQkv& p, int chunk,
   if constexpr (ONE)
     s = {chunk, 0, 1, 1, p.step.start[chunk] - 1, p.step.slots[chunk]};
   else
-    s = conv_span(p.step, chunk);
-  if (s.slot < 0 || s.p0 < 0) return;
+    s = conv_span(p.step, chunk, part, parts);
+  if (s.slot < 0 || s.p0 < 0 || s.t0 >= s.n) return;
   const int C = (H + G) * D + G * E;
   T* tail = (T*)p.tails + (long long)s.slot * (taps - 1) * C;
   const float* bias = nullptr;

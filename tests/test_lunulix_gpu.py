@@ -206,6 +206,55 @@ def test_conv_silu(c, taps, dtype):
         at = [a + n for a, n in zip(at, step)]
 
 
+@BOTH
+@pytest.mark.parametrize("taps", [2, 4, 5])
+def test_conv_chunks_shared_or_whole(taps, dtype):
+    """Few chunks are shared by several blocks, many are not: a step's portions
+    together against one by one, which differ in nothing but that."""
+    g = gen(taps)
+    lens, at, c, H, G, Dm = [2200, 37, 1, 5], [0, 3, 64, 0], 96, 2, 1, 24
+    x = rnd(g, sum(lens), c, dtype=dtype).to(DEV)
+    w, b = rnd(g, taps, c).to(DEV), rnd(g, c).to(DEV)
+    rope = RopeTable(8, 500.0, DEV, C.STRETCH)
+    rope.ensure(2300)
+    old = rnd(g, 6, taps - 1, c, dtype=dtype).to(DEV)
+    pages = i32(*[i * 64 + p for i in range(40) for p in range(64)])
+
+    def run(which):
+        tails, tails2 = old.clone(), old.clone()
+        kc = torch.zeros(40, G, 64, Dm, dtype=dtype, device=DEV)
+        vc = torch.zeros(40, G, 64, Dm, dtype=dtype, device=DEV)
+        out = []
+        for ids in which:
+            item, t0, off, start, n, slots = _steps([lens[i] for i in ids],
+                                                    [at[i] for i in ids])
+            slots = i32(*[4 - i for i in ids])
+            rows = torch.cat([torch.arange(lens[i]) + sum(lens[:i])
+                              for i in ids]).to(DEV)
+            steps = item, t0, off, start, n, slots
+            part = x[rows].contiguous()
+            y = D.conv_silu(part, w, b, tails, *steps)
+            q = D.conv_qkv(part, w, tails2, rope.cos, rope.sin, 8,
+                           pages[rows].contiguous(), kc, vc, H, *steps)
+            out.append(torch.cat([y, q], 1))
+        return torch.cat(out), tails, tails2, kc, vc
+
+    assert 2200 // 16 > 128
+    for together, alone in zip(run([[0, 1, 2, 3]]), run([[0], [1], [2], [3]])):
+        assert torch.equal(together, alone)
+    # the long one in portions of few chunks, its tail carried from one to the next
+    got = []
+    tails = old.clone()
+    for p in range(0, 2200, 320):
+        m = min(320, 2200 - p)
+        item, t0, off, _, n, _ = _steps([m], [p])
+        got.append(D.conv_silu(x[p:p + m], w, b, tails, item, t0, off, i32(p),
+                               n, i32(4)))
+    y, t, *_ = run([[0]])
+    assert torch.equal(torch.cat(got), y[:, :c])
+    assert torch.equal(tails[4], t[4])
+
+
 # ---- attention --------------------------------------------------------------
 
 @BOTH
