@@ -527,6 +527,11 @@ extern "C" void qsa_retention_state_launch(
 // tokens against 32 keys; P^T leaves that product in
 // exactly the operand layout of the next one (the order of the summed index
 // is free) and passes through LDS, over the queries that are used up.
+// Two blocks fit a CU, by their LDS, so registers have room for loads in groups:
+// queries, values and the state before the first barrier, the keys of both tiles
+// together, the gates before the second.  One behind another, as the compiler had them
+// to spare registers, they were some 20 latencies (8 heads of 128 x 256, us: 16 x
+// 700-1024 tokens 144.6 -> 128.6, 5000 50.0 -> 43.4, 60 13.7 -> 11.2).
 // ---------------------------------------------------------------------------
 template <int KS, int ET>  // DP = 32*KS, up to 16*ET value columns
 __global__ void __launch_bounds__(512)
@@ -547,37 +552,81 @@ qsa_retention_out(const bf16_t* __restrict__ x, long long xstride,
   __shared__ __attribute__((aligned(16))) bf16_t qt[QSZ > PSZ ? QSZ : PSZ];
   __shared__ __attribute__((aligned(16))) bf16_t vt[RC * VP];
   __shared__ float red[8][RC];
-  const int h = blockIdx.x % H;
-  const int ch = blockIdx.x / H;
+  // a scalar, as what is derived from it: descriptors of loads are made of it
+  const int ch = __builtin_amdgcn_readfirstlane(blockIdx.x / H);
+  const int h = blockIdx.x - ch * H;
   const int it = chunk_item[ch], t0 = chunk_t0[ch];
   const int m = min(RC, len[it] - t0);
   const long long r0 = off[it] + t0;
   const bool has_prefix = t0 > 0 || start[it] > 0;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, hi = lane >> 4;
   const float l2d = log2_decay[h];
   const long long plane = rows * H * DP;
   const int NT = EP / 16;
 
+  // all loads before the first store to LDS
+  u32x4_v qr[KS], vr[ET / 4];
 #pragma unroll
   for (int u = 0; u < KS; ++u) {
     const int g = tid + u * 512;                    // plane, row, group
     const int p = g / (RC * DP / 8);
     const int row = g / (DP / 8) % RC, c = (g % (DP / 8)) * 8;
-    *reinterpret_cast<u32x4_v*>(&qt[(p * RC + row) * QP + c]) =
-        *reinterpret_cast<const u32x4_v*>(
-            planes + p * plane + ((r0 + min(row, m - 1)) * H + h) * DP + c);
+    qr[u] = *reinterpret_cast<const u32x4_v*>(
+        planes + p * plane + ((r0 + min(row, m - 1)) * H + h) * DP + c);
   }
 #pragma unroll
   for (int u = 0; u < ET / 4; ++u) {
     const int g = tid + u * 512;
     const int row = g / (2 * ET), c = (g % (2 * ET)) * 8;
-    const bool ok = row < m && c < E;               // E % 8 == 0
-    const u32x4_v v = *reinterpret_cast<const u32x4_v*>(
+    vr[u] = *reinterpret_cast<const u32x4_v*>(
         x + (r0 + min(row, m - 1)) * xstride + voff + (long long)h * E +
-        (c < E ? c : 0));
+        (c < E ? c : 0));                           // E % 8 == 0
+  }
+  // and the state before the chunk where registers hold it; none is read as zeros from
+  // nowhere, so that no branch hides how many loads are under way
+  const u32x4_v* const ph =
+      prefix + (((long long)ch * H + h) * 2) * NT * KS * 64 + lane;
+  const u32x4_v* const pl = ph + (long long)NT * KS * 64;
+  constexpr bool EARLY = KS * NV <= 8;
+  bf16x8_v eh[EARLY ? KS : 1][NV], el[EARLY ? KS : 1][NV];
+  if constexpr (EARLY) {
+    const unsigned long long from = reinterpret_cast<unsigned long long>(ph - lane);
+    const auto rp = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void*>(
+            (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(
+                (int)(from >> 32)) << 32 |
+            (unsigned)__builtin_amdgcn_readfirstlane((int)from)),
+        0, __builtin_amdgcn_readfirstlane(has_prefix ? 2 * NT * KS * 1024 : 0),
+        0x00027000);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const int v = min(wave + 8 * u, NT - 1);
+        eh[s][u] = __builtin_bit_cast(
+            bf16x8_v, __builtin_amdgcn_raw_buffer_load_b128(
+                          rp, lane * 16, (v * KS + s) * 1024, 0));
+        el[s][u] = __builtin_bit_cast(
+            bf16x8_v, __builtin_amdgcn_raw_buffer_load_b128(
+                          rp, lane * 16, ((NT + v) * KS + s) * 1024, 0));
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < KS; ++u) {
+    const int g = tid + u * 512;
+    const int p = g / (RC * DP / 8);
+    const int row = g / (DP / 8) % RC, c = (g % (DP / 8)) * 8;
+    *reinterpret_cast<u32x4_v*>(&qt[(p * RC + row) * QP + c]) = qr[u];
+  }
+#pragma unroll
+  for (int u = 0; u < ET / 4; ++u) {
+    const int g = tid + u * 512;
+    const int row = g / (2 * ET), c = (g % (2 * ET)) * 8;
     *reinterpret_cast<u32x4_v*>(&vt[row * VP + c]) =
-        ok ? v : (u32x4_v){0, 0, 0, 0};
+        row < m && c < E ? vr[u] : (u32x4_v){0, 0, 0, 0};
   }
   f32x4_v acc[NV][4];
 #pragma unroll
@@ -587,17 +636,19 @@ qsa_retention_out(const bf16_t* __restrict__ x, long long xstride,
   lds_barrier();
 
   if (has_prefix) {                                 // uniform
-    const u32x4_v* ph =
-        prefix + (((long long)ch * H + h) * 2) * NT * KS * 64 + lane;
-    const u32x4_v* pl = ph + (long long)NT * KS * 64;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       bf16x8_v ah[NV], al[NV];
 #pragma unroll
       for (int u = 0; u < NV; ++u) {
         const int v = min(wave + 8 * u, NT - 1);    // spare tiles: not stored
-        ah[u] = __builtin_bit_cast(bf16x8_v, ph[(v * KS + s) * 64]);
-        al[u] = __builtin_bit_cast(bf16x8_v, pl[(v * KS + s) * 64]);
+        if constexpr (EARLY) {
+          ah[u] = eh[s][u];
+          al[u] = el[s][u];
+        } else {
+          ah[u] = __builtin_bit_cast(bf16x8_v, ph[(v * KS + s) * 64]);
+          al[u] = __builtin_bit_cast(bf16x8_v, pl[(v * KS + s) * 64]);
+        }
       }
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
@@ -630,45 +681,68 @@ qsa_retention_out(const bf16_t* __restrict__ x, long long xstride,
   // from the planes
   const int prt = wave & 3, ps = wave >> 2;
   const int i = prt * 16 + col;
+  // Both tiles' keys at once, and the gates, which the end would wait for; of a tile
+  // behind the tokens there are none, read as zeros from nowhere.
+  bf16x8_v kh[2][KS], kl[2][KS];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int pt = ps * 2 + u;
+    const bf16_t* const keys = planes + 2 * plane + (r0 * H + h) * DP;
+    const int bytes = pt <= prt ? 0x7fffffff : 0;
+    const auto rh = __builtin_amdgcn_make_buffer_rsrc((void*)keys, 0, bytes, 0x00027000);
+    const auto rl =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(keys + plane), 0, bytes, 0x00027000);
+    const unsigned to = ((unsigned)min(pt * 16 + col, m - 1) * (unsigned)(H * DP) +
+                         (unsigned)hi * 8) * 2;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      kh[u][s] = __builtin_bit_cast(
+          bf16x8_v, __builtin_amdgcn_raw_buffer_load_b128(rh, to + s * 64, 0, 0));
+      kl[u][s] = __builtin_bit_cast(
+          bf16x8_v, __builtin_amdgcn_raw_buffer_load_b128(rl, to + s * 64, 0, 0));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
   u32x4_v pbh, pbl;
   {
-    bf16x8_v qh[KS], ql[KS];
+    f32x4_v sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const bf16_t* qr = &qt[i * QP + s * 32 + hi * 8];
-      qh[s] = *reinterpret_cast<const bf16x8_v*>(qr);
-      ql[s] = *reinterpret_cast<const bf16x8_v*>(qr + RC * QP);
+      const bf16x8_v qh = *reinterpret_cast<const bf16x8_v*>(qr);
+      const bf16x8_v ql = *reinterpret_cast<const bf16x8_v*>(qr + RC * QP);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (ps * 2 + u <= prt) {                    // uniform over the wave
+          sc[u] = mfma_bf16(kh[u][s], qh, sc[u]);
+          sc[u] = mfma_bf16(kh[u][s], ql, sc[u]);
+          sc[u] = mfma_bf16(kl[u][s], qh, sc[u]);
+        }
     }
     uint2 ph[2], pl[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int pt = ps * 2 + u;
-      f32x4_v sc = {0.f, 0.f, 0.f, 0.f};
-      if (pt <= prt) {                              // uniform over the wave
-        const bf16_t* kr = planes + 2 * plane +
-            ((r0 + min(pt * 16 + col, m - 1)) * H + h) * DP + hi * 8;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          const bf16x8_v ah = *reinterpret_cast<const bf16x8_v*>(kr + s * 32);
-          const bf16x8_v al =
-              *reinterpret_cast<const bf16x8_v*>(kr + plane + s * 32);
-          sc = mfma_bf16(ah, qh[s], sc);
-          sc = mfma_bf16(ah, ql[s], sc);
-          sc = mfma_bf16(al, qh[s], sc);
-        }
-      }
       float w[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int j = pt * 16 + hi * 4 + r;
         const bool ok = j <= i && j < m;
-        w[r] = ok ? sc[r] * exp2f((float)(i - j) * l2d) : 0.f;
+        w[r] = ok ? sc[u][r] * exp2f((float)(i - j) * l2d) : 0.f;
       }
       split4_bf16(w[0], w[1], w[2], w[3], ph[u], pl[u]);
     }
     pbh = (u32x4_v){ph[0].x, ph[0].y, ph[1].x, ph[1].y};
     pbl = (u32x4_v){pl[0].x, pl[0].y, pl[1].x, pl[1].y};
   }
+  uint2 gate[NV][4];
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+      gate[u][rt] = *reinterpret_cast<const uint2*>(
+          x + (r0 + min(rt * 16 + col, m - 1)) * xstride + voff + (long long)H * E +
+          (long long)h * E + min((wave + 8 * u) * 16 + hi * 4, E - 4));
   lds_barrier();                                    // all queries are read
   u32x4_v* pt = reinterpret_cast<u32x4_v*>(qt);     // [plane][s2][rt][lane]
   pt[wave * 64 + lane] = pbh;
@@ -714,15 +788,15 @@ qsa_retention_out(const bf16_t* __restrict__ x, long long xstride,
                      ((red[4][t] + red[5][t]) + (red[6][t] + red[7][t]));
     const float inv = 1.f / sqrtf(ss / (float)E + eps);
     if (t < m) {
-      const bf16_t* g = x + (r0 + t) * xstride + voff + (long long)H * E +
-                        (long long)h * E;
       bf16_t* orow = out + ((r0 + t) * H + h) * E;
 #pragma unroll
       for (int u = 0; u < NV; ++u) {
         const int e0 = (wave + 8 * u) * 16 + hi * 4;
         if (e0 < E) {                               // E % 8 == 0
-          float gv[4], o[4];
-          ldv<bf16_t, 4>(g + e0, gv);
+          const float2 g0 = bf16x2_to_f32x2(gate[u][rt].x),
+                       g1 = bf16x2_to_f32x2(gate[u][rt].y);
+          const float gv[4] = {g0.x, g0.y, g1.x, g1.y};
+          float o[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             o[r] = acc[u][rt][r] * inv * (gv[r] * gate_f(gv[r]));
