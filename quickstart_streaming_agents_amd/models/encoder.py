@@ -91,11 +91,11 @@ class EmbeddingEncoder:
                 glu: bool = False, parts: bool = False) -> torch.Tensor:
         """x W^T (`parts`: for the residual's norm), with glu silu(gate) * up of
         it, w = [gate; up] (GPU).  Few tiles are short_gemm's
-        (ops/hip/short_gemm.hip: 384 x 512 at 400 rows 4.3 us, 4.5 in rows_gemm,
+        (ops/hip/short_gemm.hip: 384 x 512 at 400 rows 3.6 us, 4.5 in rows_gemm,
         5.5 in the library; of long K while its blocks are few: 384 x 1536 at 130
         rows 5.8, 6.8 in rows_gemm), the others rows_gemm's or wide_gemm's: at 8800 rows
         1536 x 384 takes 16.5 us (short_gemm 20.7, the library 18.3), 3072 x 384
-        with the activation 32 (36, 72 with a pass of its own), 384 x 512 7.4
+        with the activation 25 (31, 72 with a pass of its own), 384 x 512 7.4
         (10.5, 10.7), 384 x 1536 14.1 (23.4, 17.2)."""
         n, k = w.shape
         if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \

@@ -550,9 +550,10 @@ extern "C" void qsa_paged_attn_mfma_launch(
   // Few blocks of few pages leave most of the chip idle for some 9 us: as much
   // as memory delivers meanwhile, or nothing, since a projection whose weights
   // are there in part waits for the rest.  2048-wide decoder, 16 layers, output
-  // and down projections of 21 MB: 1 row of 700 keys 618 -> 605 us a step, of
-  // 120 578 -> 552, 8 rows 715 -> 678; cut to 24 MB of a 4096-wide one's 75 it
-  // cost 1-2%.
+  // and down projections of 21 MB: 8 rows 518 -> 500 us a step; cut to 24 MB of a
+  // 4096-wide one's 75 it cost 1-2%.  Up to 4 rows those projections are as fast on
+  // weights from memory, and the attention is over sooner without the other blocks: 1
+  // row of 700 keys 461 us without, 468 with, of 120 425 and 445; 3 and 4 rows level.
   const long long bytes = warm_bytes[0] + warm_bytes[1];
   if (k && NS == 1 && B > 4 && grid.x <= 64 && bytes >= 16 &&
       bytes <= 24 << 20) {

@@ -11,11 +11,11 @@
 // through LDS to whole lines, and the gate's columns beside the up's in a wave, so
 // that the activation costs no pass over memory.
 // us, library / rows_gemm -> here:
-//   384 x 512  at 100 / 400 / 1000 rows 5.4 / 5.5 / 6.2, 4.5 -> 4.2 / 4.3 / 4.4
-//   1536 x 384 at 40 rows 5.0, 4.1 -> 3.8;  512 x 256 at 700 5.1, 4.0 -> 3.6
+//   384 x 512  at 100 / 400 / 1000 rows 5.4 / 5.5 / 6.2, 4.5 -> 3.1 / 3.6 / 3.8
+//   1536 x 384 at 40 rows 5.0, 4.1 -> 2.8;  512 x 256 at 700 5.1, 4.0 -> 3.1
 //   of few rows: qsa_few_gemm
 //   at 8800 rows 1536 x 384 18.3, 17.0 -> 20.7, 384 x 512 10.7, 8.0 -> 11.7, 3072
-//   x 384 with the activation 72, 32 -> 34.8
+//   x 384 with the activation 72, 25 -> 31.5
 #include "lm_common.h"
 
 struct ShortArgs {

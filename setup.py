@@ -30,8 +30,9 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 # module -> sources.  qsa_hip: streaming operators, retrieval, the Llama /
-# Mixtral / encoder kernels.  qsa_lm_hip: the mixer decoders' kernels; it
-# builds alone in about a minute when that is all a program needs.
+# Mixtral / encoder kernels.  qsa_lm_hip: the mixer decoders' kernels, the products of
+# many rows, and what the encoder's layers in one call need; it builds alone in about a
+# minute when that is all a program needs.
 MODULES = {
     "qsa_hip": ["ops.cpp", "avro_codec.cpp", "bpe.cpp", "elementwise.hip",
                 "paged_attn.hip", "skinny_gemm.hip", "skinny_gemm_fp8.hip",
