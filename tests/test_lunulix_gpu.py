@@ -867,6 +867,40 @@ def test_shares_meet_their_reader(S, W):
                        D.residual_norm(b, y, odd, None, 1e-5))
 
 
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("W", [4, 260, 4096])
+def test_residual_norm_few_rows_or_many(W, dtype):
+    """256 rows go as one round of loads each, 257 with a loop: alike, with
+    whatever is given or absent, and what init replaces is not looked at."""
+    g, T, V = gen(W), 257, 9
+    res, y = rnd(g, T, W).to(DEV), rnd(g, T, W, dtype=dtype).to(DEV)
+    w, b, vec, post, table = (rnd(g, n, W, dtype=dtype).to(DEV)
+                              for n in (1, 1, 1, 1, V))
+    ids = torch.arange(T, device=DEV) % V
+    w, b, vec, post = w[0], b[0], vec[0], post[0]
+    for branch, kw in ((y, {}), (y, {"post": post}), (None, {"vec": vec}),
+                       (y, {"init": True}), (y, {"init": True, "post": post}),
+                       (y, {"table": table, "tscale": .5}),
+                       (y, {"table": table, "vec": vec, "post": post}),
+                       (None, {"init": True, "table": table})):
+        for layer, weight, bias in ((True, w, b), (True, w, None),
+                                    (False, w, None), (False, None, None)):
+            if branch is None and weight is None:
+                continue                            # refused
+            many, few = res.clone(), res[:256].clone()
+            if kw.get("init"):
+                many.fill_(float("nan")), few.fill_(float("nan"))
+            def go(r):
+                n = len(r)
+                k = {**kw, "ids": ids[:n]} if "table" in kw else kw
+                return D.residual_norm(
+                    r, None if branch is None else branch[:n], weight, bias,
+                    1e-4, layer=layer, **k)
+            want, got = go(many), go(few)
+            close(few, many[:256].cpu(), F32)
+            close(got, want[:256].cpu(), dtype)
+
+
 def test_product_in_shares():
     """What is left in shares adds up to the product."""
     g = gen(3)
