@@ -30,6 +30,10 @@ def close(got, want, dtype):
     assert float(err) <= (2e-5 if dtype == F32 else 3e-2), float(err)
 
 
+def i32(*v):
+    return torch.tensor(v, dtype=torch.int32, device=DEV)
+
+
 # ---- kernels ----------------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", [F32, BF])
@@ -285,6 +289,26 @@ def test_latent_norm_store_and_slots():
             if s >= 0:
                 close(flat[s], want[r], dtype)
         assert int((flat != 0).any(-1).sum()) == 5
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("qr,kr,lead", [(4, 1024, 0), (1024, 4, 0),
+                                        (1028, 512, 0), (260, 258, 0),
+                                        (768, 512, 1)])
+def test_latent_norm_wave_or_block(qr, kr, lead, dtype):
+    """A wave's smallest and widest latents; beyond them, and where groups of
+    four do not divide or align, a block's."""
+    g, T = gen(qr), 3
+    x = rnd(g, T, lead + qr + kr + 4, dtype=dtype)
+    wq, wk = rnd(g, qr, dtype=dtype), rnd(g, kr, dtype=dtype)
+    cache = torch.zeros(1, 64, kr, dtype=dtype, device=DEV)
+    cq = D.latent_norm_store(x.to(DEV)[:, lead:], wq.to(DEV), wk.to(DEV),
+                             cache, i32(7, -1, 63), 1e-5)
+    x = x[:, lead:].double()
+    close(cq, O.rms(x[:, :qr], 1e-5, wq.double()), dtype)
+    want = O.rms(x[:, qr:qr + kr], 1e-5, wk.double())
+    close(cache[0, [7, 63]], want[[0, 2]], dtype)
+    assert int((cache[0] != 0).any(-1).sum()) == 2
 
 
 # ---- the model through the framework ----------------------------------------
