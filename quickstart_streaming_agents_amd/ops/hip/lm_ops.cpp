@@ -355,6 +355,7 @@ Tensor retention_decode(Tensor x, Tensor cos_t, Tensor sin_t, Tensor decay,
   TORCH_CHECK(2 * r.D + 2 * r.E <= 8000, "head too wide for the decode block");
   auto out = torch::empty({B, (long long)r.H * r.E}, x.options());
   if (B == 0) return out;
+  if (r.D == 0 || r.E == 0) return out.zero_();   // no state to ask for
   const int v4 = r.E % 4 == 0 && (2LL * r.H * r.D) % 4 == 0 &&
                  x.stride(0) % 4 == 0 && aligned(x, 16);
   qsa_retention_decode_launch(

@@ -167,6 +167,49 @@ def test_retention_kernels(H, Dm, E, rot, dtype):
             at += n
 
 
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("B,H,Dm,E,rot", [
+    (3, 2, 4, 8, 4),          # fewer rows of the state than one round asks for
+    (2, 3, 36, 20, 0),        # the last round half empty, nothing rotated
+    (1, 2, 260, 1028, 256),   # more columns and rows than threads
+    (2, 2, 128, 256, 96),     # wide blocks, one round
+    (2, 2, 132, 260, 132),    # wide blocks, the last round of a few
+    (260, 2, 128, 256, 128),  # many blocks, several rounds
+    (2, 1, 33, 35, 30)])      # element by element
+def test_retention_decode_rounds(B, H, Dm, E, rot, dtype):
+    """Rounds of state rows, whole and ragged; a first token takes nothing
+    from its slot, whatever that holds."""
+    g = gen(Dm + E)
+    x = rnd(g, B, 2 * H * (Dm + E), dtype=dtype)
+    decay = torch.rand(H, generator=g) * .5 + .4
+    state = rnd(g, B + 1, H, Dm, E)
+    pos = (torch.arange(B) + 2) % 3
+    state[torch.arange(B)[pos == 0] + 1] = float("nan")
+    ang = torch.arange(3).double()[:, None] * \
+        torch.rand(rot // 2, generator=g).double()
+    got = state.to(DEV)
+    out = D.retention_decode(
+        x.to(DEV), ang.cos().float().to(DEV), ang.sin().float().to(DEV),
+        decay.to(DEV), got, i32(*range(1, B + 1)),
+        (pos + 1).int().to(DEV), rot, Dm ** -0.5, 1e-5)
+    x, S = x.double(), torch.nan_to_num(state[1:].double(), nan=0.)
+    q, k = x[:, :2 * H * Dm].view(B, 2, H, Dm).unbind(1)
+    v, gate = x[:, 2 * H * Dm:].view(B, 2, H, E).unbind(1)
+
+    def turn(a):
+        h = rot // 2
+        c, s = (f(ang[pos])[:, None] for f in (torch.cos, torch.sin))
+        lo, hi = a[..., :h], a[..., h:rot]
+        return torch.cat((lo * c - hi * s, hi * c + lo * s, a[..., rot:]), -1)
+
+    q, k = turn(q), turn(k) * Dm ** -0.5
+    S = decay.double()[:, None, None] * S + k[..., None] * v[:, :, None]
+    o = torch.matmul(q[:, :, None], S)[:, :, 0]
+    close(out, (O.rms(o, 1e-5) * O.silu(gate)).reshape(B, H * E), dtype)
+    close(got[1:].flatten(0, -2), S.flatten(0, -2), F32)
+    assert torch.equal(got[0].cpu(), state[0])
+
+
 def _attention_reference(q, c, uk, uv, scale, window, sink, gate, start):
     """rows of q [n, H, D] at positions start.. over latents c [T, R]"""
     n, H, Dm = q.shape
