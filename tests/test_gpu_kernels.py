@@ -127,6 +127,23 @@ def test_paged_attn_decode(ext):
     torch.testing.assert_close(out.float().cpu(), ref, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("B,KVH,D,pages", [
+    (20, 4, 128, 17),                        # two shares of a row
+    (2, 2, 64, 17), (2, 2, 128, 32),         # three, four: the first round
+    (2, 2, 128, 33), (1, 2, 64, 81)])        # five, eleven: and a loop
+def test_paged_attn_shares_merged(ext, B, KVH, D, pages):
+    """Shares of long rows, and short rows that leave most of theirs empty."""
+    QH = 4 * KVH
+    seq_lens = [pages * 64 - 5] + [1, 300][:B - 1] + [700] * (B - 3)
+    kc, vc, bt = _make_paged_kv(B, KVH, D, seq_lens, 2 * pages)
+    q = torch.randn(B, QH, D, dtype=torch.bfloat16, device=dev())
+    sl = torch.tensor(seq_lens, dtype=torch.int32, device=dev())
+    out = ext.paged_attn_decode(q, kc, vc, bt, sl, D ** -0.5)
+    ref = cpu_ref.paged_attn_ref(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(),
+                                 sl.cpu(), D ** -0.5)
+    torch.testing.assert_close(out.float().cpu(), ref, atol=2e-2, rtol=2e-2)
+
+
 def test_kv_append_then_attend(ext):
     B, QH, KVH, D = 2, 8, 2, 128
     seq_lens = [65, 120]
