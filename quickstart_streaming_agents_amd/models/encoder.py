@@ -95,7 +95,7 @@ class EmbeddingEncoder:
         5.5 in the library; of long K while its blocks are few: 384 x 1536 at 130
         rows 5.8, 6.8 in rows_gemm), the others rows_gemm's or wide_gemm's: at 8800 rows
         1536 x 384 takes 16.5 us (short_gemm 20.7, the library 18.3), 3072 x 384
-        with the activation 25 (31, 72 with a pass of its own), 384 x 512 7.4
+        with the activation 30 (34, 72 with a pass of its own), 384 x 512 7.4
         (10.5, 10.7), 384 x 1536 14.1 (23.4, 17.2)."""
         n, k = w.shape
         if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \

@@ -43,16 +43,6 @@ __device__ __forceinline__ float2 bf16x2_to_f32x2(unsigned int p) {
   return make_float2(lo.f, hi.f);
 }
 
-// 1 / (1 + e^-z) for a number that is rounded to bf16 next, by the hardware's
-// reciprocal, good to a unit of f32's last place as its exponential is.  A division that
-// is right to half of one is ten more instructions, of which a block of a gated product
-// has 128 a lane while its matrix cores wait (gated products, us: 9600 x 3072 x 384 32.0 ->
-// 27.9, 13,800 x 16384 x 2048 736 -> 703, 10,528 x 28672 x 4096 1792 -> 1744; errors
-// against 64 bits are the same to six digits).
-__device__ __forceinline__ float gate_f(float z) {
-  return __builtin_amdgcn_rcpf(1.f + __expf(-z));
-}
-
 // ---- wave reductions (64-lane) --------------------------------------------
 // Reductions over lanes by exchanges between registers: __shfl_xor goes through
 // LDS, some 100 cycles a step that a chain of six waits for.  Every lane ends up

@@ -219,8 +219,8 @@ qsa_swiglu_kernel(const unsigned short* __restrict__ gate,
     for (int j = 0; j < 4; ++j) {
       float2 a = bf16x2_to_f32x2(gp[j]);
       float2 b = bf16x2_to_f32x2(upk[j]);
-      float s0 = a.x * gate_f(a.x);
-      float s1 = a.y * gate_f(a.y);
+      float s0 = a.x / (1.f + __expf(-a.x));
+      float s1 = a.y / (1.f + __expf(-a.y));
       po[j] = f32x2_to_bf16x2(s0 * b.x, s1 * b.y);
     }
     *reinterpret_cast<uint4*>(y + i) = outv;

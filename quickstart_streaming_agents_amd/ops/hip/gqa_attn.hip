@@ -307,8 +307,8 @@ gqa_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
         const float2 gv = bf16x2_to_f32x2(
             *reinterpret_cast<const unsigned int*>(
                 fin.gate + row * fin.gstride + (long long)h * E + e));
-        a0 *= gate_f(gv.x);
-        a1 *= gate_f(gv.y);
+        a0 /= 1.f + __expf(-gv.x);
+        a1 /= 1.f + __expf(-gv.y);
       }
       *reinterpret_cast<unsigned int*>(fin.out + row * fin.ostride +
                                        (long long)h * E + e) =
@@ -432,8 +432,8 @@ qsa_gqa_merge(const float* __restrict__ part_o,
         const float2 gv = bf16x2_to_f32x2(
             *reinterpret_cast<const unsigned int*>(
                 gate + row * gstride + (long long)h * E + e));
-        a0 *= gate_f(gv.x);
-        a1 *= gate_f(gv.y);
+        a0 /= 1.f + __expf(-gv.x);
+        a1 /= 1.f + __expf(-gv.y);
       }
       *reinterpret_cast<unsigned int*>(out + row * ostride + (long long)h * E +
                                        e) = cvt_bf16x2(a0, a1);
@@ -706,7 +706,7 @@ qsa_gqa_portions(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
             float gv[4];
             ldv<bf16_t, 4>(gr + e, gv);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] *= gate_f(gv[r]);
+            for (int r = 0; r < 4; ++r) o[r] /= 1.f + __expf(-gv[r]);
           }
           stv<bf16_t, 4>(orow + e, o);
         }
@@ -1046,7 +1046,7 @@ qsa_gqa_portions_beside(const bf16_t* __restrict__ q, const bf16_t* __restrict__
             float gv[4];
             ldv<bf16_t, 4>(gr + e, gv);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] *= gate_f(gv[r]);
+            for (int r = 0; r < 4; ++r) o[r] /= 1.f + __expf(-gv[r]);
           }
           stv<bf16_t, 4>(orow + e, o);
         }

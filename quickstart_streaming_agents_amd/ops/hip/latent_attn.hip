@@ -109,7 +109,7 @@ qsa_head_matmul_mfma(const bf16_t* __restrict__ x, long long xrow,
       float g[4];
       ldv<bf16_t, 4>(gate + (long long)m * grow + (long long)h * N + n0, g);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] *= gate_f(g[r]);
+      for (int r = 0; r < 4; ++r) v[r] /= 1.f + __expf(-g[r]);
     }
     stv<bf16_t, 4>(out + ((long long)m * H + h) * N + n0, v);
   };
@@ -653,7 +653,7 @@ qsa_window_attn_prefill(const bf16_t* __restrict__ q, long long qstride,
         ldv<bf16_t, 4>(g + e, gv);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          o[r] = acc[t][r] * inv * gate_f(gv[r]);
+          o[r] = acc[t][r] * inv / (1.f + __expf(-gv[r]));
         stv<bf16_t, 4>(orow + e, o);
       }
     }

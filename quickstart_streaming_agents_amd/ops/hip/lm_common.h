@@ -153,7 +153,7 @@ template <bool EXACT, int ACT>
 __device__ __forceinline__ float act_f(float z) {
   const float a = ACT == QSA_ACT_SILU
       ? z : 1.5957691216057308f * fmaf(0.044715f * z * z, z, z);
-  return EXACT ? z / (1.f + expf(-a)) : z * gate_f(a);
+  return z / (1.f + (EXACT ? expf(-a) : __expf(-a)));
 }
 
 // x = hi + lo with both parts bf16: 16 mantissa bits survive, so a product

@@ -830,7 +830,7 @@ qsa_retention_out(const bf16_t* __restrict__ x, long long xstride,
           float o[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            o[r] = acc[u][rt][r] * inv * (gv[r] * gate_f(gv[r]));
+            o[r] = acc[u][rt][r] * inv * (gv[r] / (1.f + __expf(-gv[r])));
           stv<bf16_t, 4>(orow + e0, o);
         }
       }

@@ -304,7 +304,7 @@ static void rows_go(RowsArgs p, int act, hipStream_t st) {
 // the same where few rows meet weights from memory (qsa_rows_gemm_plan).
 // Of the last tile two blocks share a CU: one's start and end lie beside the
 // other's products, which short K gains by (us, the best of the others and so:
-// 16,000 x 3072 x 384 with the activation 43.3, 42.8; 24,000 63.5, 62.0; 8263 x
+// 16,000 x 3072 x 384 with the activation 52.7, 49.3; 24,000 79.2, 71.7; 8263 x
 // 2048 x 128 15.7, 13.0; 30,000 38.2, 30.7; 4400 x 16384 x 2048 263, 253).  Its
 // figures are those of a pair, set where 42 such shapes part.
 #define QSA_TILES(X) \

@@ -61,7 +61,7 @@ qsa_conv_silu(const T* x, long long xstride, const float* __restrict__ w,
 #pragma unroll
     for (int i = 0; i < VEC; ++i)
       a[0][i] = sizeof(T) == 4 ? silu_f(a[0][i])
-                               : a[0][i] * gate_f(a[0][i]);
+                               : a[0][i] / (1.f + __expf(-a[0][i]));
     stv<T, VEC>(out + (long long)(s.r0 + t) * C + c0, a[0]);
   };
   CONV_DISPATCH(T, VEC, 1)

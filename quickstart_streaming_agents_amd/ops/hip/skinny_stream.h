@@ -344,7 +344,7 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
     if constexpr (GLU) {
       const float g = total(2 * j, 0) * inv, u = total(2 * j + 1, GLU) * inv;
       if (live)
-        p.C[place(p.N >> 1)] = cvt_bf16(g * gate_f(g) * u);
+        p.C[place(p.N >> 1)] = cvt_bf16(g / (1.f + __expf(-g)) * u);
     } else if constexpr (RES) {
       const float v = bf16_to_f32(old[i]) + total(j, 0);
       const bf16_t b = cvt_bf16(v);

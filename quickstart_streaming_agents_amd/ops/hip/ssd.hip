@@ -254,7 +254,7 @@ qsa_ssd_step(SsdStep p) {
       if (j < NT)
         tail[(unsigned)(j * C)] =
             (bf16_t)(j + 1 < NT ? old[j + 1 < STEP_TAPS - 1 ? j + 1 : j] : raw);
-    cx = bf16_to_f32(cvt_bf16(cx * gate_f(cx)));
+    cx = bf16_to_f32(cvt_bf16(cx / (1.f + __expf(-cx))));
     if (tid < CG) xs[tid] = cx;
     else bc[tid - CG] = cx;
   }
@@ -855,7 +855,7 @@ qsa_ssd_out(const bf16_t* __restrict__ u, long long ustride, int zoff,
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             o[r] = (acc[v][t][r] + dk * xv[r]) *
-                   (zv[r] * gate_f(zv[r]));
+                   (zv[r] / (1.f + __expf(-zv[r])));
           stv<bf16_t, 4>(orow + e0, o);
         }
       }

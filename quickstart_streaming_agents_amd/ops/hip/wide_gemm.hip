@@ -19,8 +19,8 @@
 //   rows           512          2048         7500          13800         44800
 //   6144 x 4096    30.8 -> 27.5  78.3 -> 72.0  252 -> 256    549 -> 480    1581 -> 1516
 //   4096 x 14336   76 -> (63)    187 -> 172    998 -> 614    1254 -> 1179  3719 -> 3568
-//   28672 x 4096 (activation)  97.9 -> 86.5  371 -> 347  1386 -> 1238  2406 -> 2225  8058 -> 7182
-//   16384 x 2048 (activation)  38.1 -> 28.8  114 -> 97.8  435 -> 363   803 -> 644    2559 -> 2104
+//   28672 x 4096 (activation)  97.9 -> 86.5  371 -> 356  1386 -> 1241  2406 -> 2256  8058 -> 7353
+//   16384 x 2048 (activation)  38.1 -> 28.8  114 -> 97.8  435 -> 371   803 -> 663    2559 -> 2158
 // Left: with all of W and A in L2 it would be 1.62 to 1.67 (its fabric's power), with
 // no loads at all 2.0.  Products of 32 x 32, groups of 2 or 8 tiles along the rows
 // instead of 4, starts at other stages (against channels in step), non-temporal stores

@@ -1414,6 +1414,46 @@ def test_short_gemm_few_rows(ext, M, N, K, glu):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + err + 1e-30).all()
 
 
+@pytest.mark.parametrize("M", [3, 700])
+def test_gates_far_from_zero(ext, M):
+    """Gates whose 1 + e^-z is beyond 2^126, the largest number with a normal
+    reciprocal, in every kernel that applies one to numbers given to it: the
+    quotient is a normal number and comes out as one."""
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    from quickstart_streaming_agents_amd.ops import lm_ext
+    N, K = 256, 512
+    z = torch.tensor([-87.0, -87.5, -88.0, -88.5]).repeat(N // 4).bfloat16()
+    up = torch.full((N,), 2.0 ** 100).bfloat16()
+    silu = z.double() / (1 + torch.exp(-z.double()))
+    want = (silu * up.double()).expand(M, N)
+
+    def close(got, want=want):
+        # the exponential's argument times log2(e), rounded: 2^-17 at 88; the
+        # factor and the result rounded to bf16
+        err = (got.cpu().double() - want).abs()
+        assert (err <= 2.0 ** -8 * want.abs()).all()
+
+    rows = [t.expand(M, N).contiguous().to(dev()) for t in (z, up)]
+    close(ext.swiglu(*rows))
+    close(D.glu(*rows))
+    # products: the first column of W is the gate's and the factor's row
+    x = torch.zeros(M, K).bfloat16()
+    x[:, 0] = 1
+    w = torch.zeros(2 * N, K).bfloat16()
+    w[:, 0] = torch.cat((z, up))
+    x, w = x.to(dev()), w.to(dev())
+    close(ext.short_gemm(x, w, True))
+    close(lm_ext().rows_glu(x, w, False, False))
+    close(lm_ext().wide_gemm(x, w, 0, 3))
+    # a convolution of one tap: the result itself is as small
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=dev())
+    y = D.conv_silu(rows[0], torch.ones(1, N, device=dev()),
+                    torch.zeros(N, device=dev()),
+                    torch.zeros(M, 0, N, device=dev()).bfloat16(), None, None,
+                    None, i32(*[5] * M), None, i32(*range(M)))
+    close(y, silu.expand(M, N))
+
+
 def test_mean_rows(ext):
     lens = [1, 3, 4, 5, 700]
     x = torch.randn(sum(lens), 520, device=dev()).bfloat16()
