@@ -92,17 +92,16 @@ class EmbeddingEncoder:
         """x W^T (`parts`: for the residual's norm), with glu silu(gate) * up of
         it, w = [gate; up] (GPU).  Few tiles are short_gemm's
         (ops/hip/short_gemm.hip: 384 x 512 at 400 rows 3.6 us, 4.5 in rows_gemm,
-        5.5 in the library; of long K while its blocks are few: 384 x 1536 at 130
-        rows 5.8, 6.8 in rows_gemm), the others rows_gemm's or wide_gemm's: at 8800 rows
+        5.5 in the library; of long K up to 32 rows: beyond, rows_gemm's shares of K,
+        which the norm adds, are sooner, 384 x 1536 with its norm at 33 / 130 / 320
+        rows 6.4 / 6.7 / 7.2, 7.6 / 8.0 / 8.8 here), the others rows_gemm's or
+        wide_gemm's: at 8800 rows
         1536 x 384 takes 16.5 us (short_gemm 20.7, the library 18.3), 3072 x 384
         with the activation 30 (34, 72 with a pass of its own), 384 x 512 7.4
         (10.5, 10.7), 384 x 1536 14.1 (23.4, 17.2)."""
         n, k = w.shape
         if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
-                n % 32 == 0 and \
-                (k <= 512 or x.shape[0] <= 32 or (
-                    k <= 2048 and not glu and
-                    -(-x.shape[0] // 32) * (n // 16) <= 256)) and \
+                n % 32 == 0 and (k <= 512 or x.shape[0] <= 32) and \
                 -(-x.shape[0] // 32) * -(-n // 64) <= 192:
             return D.ext().short_gemm(x, w, glu)
         if not glu:

@@ -275,7 +275,7 @@ static void short_go(ShortArgs p, int glu, hipStream_t st) {
 // 2.92, of 130, 480 blocks, 3.30 / 4.06; 384 x 1536 of 15 rows 7.2 / 4.7, of 250, 192
 // blocks, 7.4 / 5.9, of 400, 312 blocks, 7.4 / 9.8; gated 1536 x 384 of 15 rows 3.31 /
 // 3.00, of 60, 96 blocks, 3.34 / 3.36, of 130, 240 blocks, 3.37 / 3.46).
-extern "C" bool qsa_few_gemm_takes(long long M, long long N, bool glu) {
+static bool few_takes(long long M, long long N, bool glu) {
   return (M + 31) / 32 * (N / (glu ? 32 : 16)) <= (glu ? 128 : 256);
 }
 
@@ -292,7 +292,7 @@ extern "C" void qsa_short_gemm_launch(const bf16_t* A, const bf16_t* W,
   auto blocks = [&](int b) {
     return (long long)((M + b - 1) / b) * ((N + b - 1) / b);
   };
-  if (qsa_few_gemm_takes(M, N, glu)) {
+  if (few_takes(M, N, glu)) {
     if (K <= 512) few_go<1>(p, glu, st); else few_go<3>(p, glu, st);
     return;
   }

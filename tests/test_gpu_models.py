@@ -675,3 +675,29 @@ def test_encoder_layers_at_once():
     before = res.clone()
     assert enc._native_layers(res, *maps) is None
     assert torch.equal(res, before)
+
+
+@pytest.mark.parametrize("rows", [32, 33, 130, 320])
+def test_encoder_down_product(rows):
+    """The feed-forward's second product and the norm that adds it: beyond 32
+    rows in shares of K, which it adds sooner than a product is finished; either
+    way rounded once, as it would be stored, before the residual is."""
+    from quickstart_streaming_agents_amd.models.encoder import (
+        EmbeddingEncoder, EncoderConfig)
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    enc = EmbeddingEncoder(EncoderConfig(n_layers=1), device="cuda:0", seed=4)
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, 1536, generator=g).bfloat16().to("cuda:0")
+    w = enc.layers[0]["wdown"]
+    y = enc._linear(x, w, parts=True)
+    assert y.dim() == (2 if rows <= 32 else 3) and \
+        y.dtype == (torch.bfloat16 if rows <= 32 else torch.float32)
+    res = torch.randn(rows, 384, generator=g).bfloat16().to("cuda:0")
+    old = res.double()
+    D.rmsnorm_residual(y, res, enc.final_norm, 1e-5)
+    want = x.double() @ w.double().T
+    err = 1536 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    # half an ulp of bf16 is up to 2^-8: of the product, and of the sum, which may
+    # be larger by the product's
+    assert ((res.double() - old - want).abs() <= 2.0 ** -8 * (
+        1.01 * want.abs() + (old + want).abs()) + 1.01 * err).all()
