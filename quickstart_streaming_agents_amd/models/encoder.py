@@ -100,9 +100,8 @@ class EmbeddingEncoder:
         with the activation 30 (34, 72 with a pass of its own), 384 x 512 7.4
         (10.5, 10.7), 384 x 1536 14.1 (23.4, 17.2)."""
         n, k = w.shape
-        if x.dtype == w.dtype == torch.bfloat16 and k % 64 == 0 and \
-                n % 32 == 0 and (k <= 512 or x.shape[0] <= 32) and \
-                -(-x.shape[0] // 32) * -(-n // 64) <= 192:
+        if x.dtype == w.dtype == torch.bfloat16 and \
+                D.ext().short_gemm_takes(x.shape[0], n, k):
             return D.ext().short_gemm(x, w, glu)
         if not glu:
             return D.linear_parts(x, w) if parts else D.linear(x, w)
@@ -147,9 +146,11 @@ class EmbeddingEncoder:
 
     def _native_layers(self, res, qb_item, qb_pos0, off, lens):
         """All layers as one call that launches the kernels of _layers_by_call, or
-        None where it does not take them."""
+        None where it does not take them, or where a product is not _linear's."""
         if not have_lm_ext() or type(res) is not torch.Tensor or \
-                torch.compiler.is_compiling():
+                torch.compiler.is_compiling() or \
+                getattr(self._project, "__func__", None) is not \
+                EmbeddingEncoder._linear:
             return None
         c = self.cfg
         weights = [Ly[k] for Ly in self.layers for k in

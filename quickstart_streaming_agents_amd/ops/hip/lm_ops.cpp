@@ -49,6 +49,7 @@ extern "C" void qsa_rmsnorm_launch(const bf16_t*, const bf16_t*, bf16_t*, bf16_t
     long long, int, float, hipStream_t);
 extern "C" void qsa_short_gemm_launch(const bf16_t*, const bf16_t*, bf16_t*, int, int,
     int, long long, int, hipStream_t);
+extern "C" bool qsa_short_gemm_takes(long long, long long, long long);
 extern "C" void qsa_encoder_attn_launch(const bf16_t*, const float*, const float*, int,
     const int*, const int*, const int*, const int*, bf16_t*, int, int, int, float,
     hipStream_t);
@@ -1318,8 +1319,7 @@ struct EncoderProduct {
     if (!gemm_takes(a, w, glu)) return false;
     const int64_t m = a.size(0), n = w.size(0), k = w.size(1);
     M = (int)m, N = (int)n, K = (int)k, act = glu ? 3 : 0;
-    brief = n % 32 == 0 && n < 1 << 20 && (k <= 512 || m <= 32) &&
-            (m + 31) / 32 * ((n + 63) / 64) <= 192;
+    brief = qsa_short_gemm_takes(m, n, k);
     if (brief) return true;
     if (!gemm_sizes(m, n, k, a.stride(0), glu)) return false;
     plan = gemm_choice(m, n, k, a.stride(0), act, parts);

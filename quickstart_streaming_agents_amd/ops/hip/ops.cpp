@@ -116,6 +116,7 @@ extern "C" void qsa_hash_probe_launch(const long long*,
                                       const unsigned long long*, int*, int,
                                       unsigned int, long long, int,
                                       hipStream_t);
+extern "C" bool qsa_short_gemm_takes(long long, long long, long long);
 extern "C" void qsa_short_gemm_launch(const unsigned short*,
                                       const unsigned short*, unsigned short*,
                                       int, int, int, long long, int,
@@ -997,6 +998,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("encoder_attn", &encoder_attn,
         "rotation and bidirectional attention of projection rows");
   m.def("short_gemm", &short_gemm, "GEMM of a short K, optionally gated");
+  m.def("short_gemm_takes", &qsa_short_gemm_takes,
+        "whether the encoder's product [M, N, K] is short_gemm's");
   m.def("mean_rows", &mean_rows, "mean of each item's rows (f32)");
   m.def("kv_scatter", &kv_scatter, "scatter prefill k/v by slot ids");
   m.def("pack_weight_frag", &pack_weight_frag,

@@ -279,6 +279,14 @@ static bool few_takes(long long M, long long N, bool glu) {
   return (M + 31) / 32 * (N / (glu ? 32 : 16)) <= (glu ? 128 : 256);
 }
 
+// Which of the encoder's products are this file's where rows_gemm.hip and wide_gemm.hip
+// are there too: while the tiles of 32 x 64 leave CUs idle, K being short or the rows
+// few (the figures above and at the encoder's products).
+extern "C" bool qsa_short_gemm_takes(long long M, long long N, long long K) {
+  return K % 64 == 0 && N % 32 == 0 && N < 1 << 20 && (K <= 512 || M <= 32) &&
+         (M + 31) / 32 * ((N + 63) / 64) <= 192;
+}
+
 // Tiles of 128 x 128 once two rounds of blocks are left, 64 x 64 while they
 // make half a round, 32 x 64 below (384 x 512 at 400 rows: 8.2 / 4.5 / 3.7 us;
 // 1536 x 384 at 1600: 7.9 / 6.8 / 8.0, at 8800: 20.9 / 23.0 / 28.4; 3072 x 384

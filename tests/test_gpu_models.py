@@ -701,3 +701,27 @@ def test_encoder_down_product(rows):
     # be larger by the product's
     assert ((res.double() - old - want).abs() <= 2.0 ** -8 * (
         1.01 * want.abs() + (old + want).abs()) + 1.01 * err).all()
+
+
+def test_encoder_products_of_another(monkeypatch):
+    """A product that is replaced, in a subclass or an object, is the one that
+    runs, for every layer."""
+    from quickstart_streaming_agents_amd.models.encoder import (
+        EmbeddingEncoder, EncoderConfig)
+
+    class Counted(EmbeddingEncoder):
+        def _linear(self, x, w, glu=False, parts=False):
+            calls.append(w.shape)
+            return super()._linear(x, w, glu)
+
+    calls, cfg, text = [], EncoderConfig(n_layers=2), ["water and light"]
+    plain = EmbeddingEncoder(cfg, device="cuda:0", seed=4)
+    want = plain.embed_batch(text)
+    assert np.abs(Counted(cfg, device="cuda:0", seed=4).embed_batch(text) -
+                  want).max() <= 0.02 * np.abs(want).max()
+    assert len(calls) == 9                  # and the projection
+    linear = plain._linear
+    monkeypatch.setattr(plain, "_linear", lambda *a, **k: calls.append(0) or
+                        linear(*a, **k))
+    assert np.array_equal(plain.embed_batch(text), want)
+    assert len(calls) == 18
