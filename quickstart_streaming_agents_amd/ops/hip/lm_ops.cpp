@@ -34,6 +34,12 @@ static inline void chk_rows(const Tensor& t, const char* name) {
   TORCH_CHECK(t.dim() == 2 && t.stride(1) == 1, name,
               " must be 2-D with contiguous rows");
 }
+// a kernel given a host tensor's pointer would read the host's memory
+template <typename... Ts>
+static inline void chk_there(const Tensor& like, const Ts&... t) {
+  TORCH_CHECK(((t.device() == like.device()) && ...), "operands must be on ",
+              like.device());
+}
 static inline const bf16_t* u16(const Tensor& t) {
   return reinterpret_cast<const bf16_t*>(t.data_ptr());
 }
@@ -911,6 +917,9 @@ Tensor ssd_step(Tensor x, Tensor qw, Tensor qtails, Tensor cos_t, Tensor sin_t,
   CHK_F32(state); CHK_F32(bias); CHK_F32(A); CHK_F32(dt_bias); CHK_F32(D);
   CHK_F32(norm); CHK_SAME(u, x); CHK_SAME(u, out);
   CHK_DEV(u); chk_rows(u, "u"); chk_rows(out, "out");
+  chk_there(u, x, qw, qtails, cache_slots, kc, vc, w, bias, tails, A, dt_bias, D,
+            state, norm, out, slots, seq_lens);
+  if (rot) chk_there(u, cos_t, sin_t);
   TORCH_CHECK(u.scalar_type() == at::kBFloat16, "bf16 storage");
   TORCH_CHECK(state.dim() == 4, "state [slots, H, N, P]");
   const int SH = (int)state.size(1), N = (int)state.size(2),
@@ -1386,6 +1395,7 @@ OptTensor encoder_layers(Tensor res, std::vector<Tensor> weights, Tensor final_n
   if (!norm_ok(final_norm) || !layer_ok(0)) return c10::nullopt;
   CHK_F32(cos_t); CHK_F32(sin_t);
   CHK_I32(qb_item); CHK_I32(qb_t0); CHK_I32(off); CHK_I32(len);
+  chk_there(res, cos_t, sin_t, qb_item, qb_t0, off, len);
   TORCH_CHECK(cos_t.dim() == 2 && cos_t.size(0) >= 1 && cos_t.size(1) == D / 2 &&
                   sin_t.sizes() == cos_t.sizes(), "cos/sin [positions, D/2]");
   TORCH_CHECK(qb_item.numel() == qb_t0.numel() && off.numel() == len.numel(), "maps");

@@ -394,6 +394,8 @@ torch::Tensor paged_attn_prefill(torch::Tensor q, torch::Tensor kc,
     TORCH_CHECK(cos_t->dim() == 2 && cos_t->size(1) == D / 2 &&
                     cos_t->size(0) > 0 && sin_t->sizes() == cos_t->sizes(),
                 "cos/sin [positions, D/2]");
+    TORCH_CHECK(cos_t->device() == q.device() && sin_t->device() == q.device(),
+                "cos and sin must be where q is");
     TORCH_CHECK(((reinterpret_cast<uintptr_t>(cos_t->data_ptr()) |
                   reinterpret_cast<uintptr_t>(sin_t->data_ptr())) & 15) == 0,
                 "cos and sin must be 16-byte aligned");

@@ -1312,6 +1312,22 @@ def test_prefill_rotates_queries(ext, D, QH, KVH, rows, scale):
     assert err.abs().max() <= 2 ** -7 * vc.abs().max()
 
 
+def test_prefill_refuses_host_angles(ext):
+    """Rotation tables whose memory is the host's are an error, not a launch."""
+    mk = lambda *x: torch.tensor(x, dtype=torch.int32, device=dev())
+    q = torch.randn(5, 4, 64).bfloat16().to(dev())
+    kc = torch.randn(1, 1, 8, 64, 8).bfloat16().to(dev())
+    vc = torch.randn(1, 1, 64, 64).bfloat16().to(dev())
+    args = (q, kc, vc, mk(0).view(1, 1), mk(0), mk(0), mk(0), mk(0), mk(5),
+            0.125, True, 16)
+    t = torch.ones(64, 32)
+    assert torch.isfinite(
+        ext.paged_attn_prefill(*args, t.to(dev()), t.to(dev()))).all()
+    for angles in ((t, t.to(dev())), (t.to(dev()), t)):
+        with pytest.raises(RuntimeError, match="must be where q is"):
+            ext.paged_attn_prefill(*args, *angles)
+
+
 @pytest.mark.parametrize("D,H", [(64, 8), (128, 4)])
 @pytest.mark.parametrize("lens", [[1], [64, 63, 65, 1, 130], [512, 3, 128]])
 def test_encoder_attn(ext, lens, D, H):

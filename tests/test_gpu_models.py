@@ -725,3 +725,24 @@ def test_encoder_products_of_another(monkeypatch):
                         linear(*a, **k))
     assert np.array_equal(plain.embed_batch(text), want)
     assert len(calls) == 18
+
+
+@pytest.mark.parametrize("which", ["cos", "sin", 0, 1, 2, 3])
+def test_encoder_layers_refuses_host_operands(which):
+    """Tables and maps whose memory is the host's: an error before anything is
+    launched."""
+    from quickstart_streaming_agents_amd.models.encoder import (
+        EmbeddingEncoder, EncoderConfig)
+    enc = EmbeddingEncoder(EncoderConfig(n_layers=1), device="cuda:0", seed=4)
+    maps = [torch.tensor(x, dtype=torch.int32, device="cuda:0")
+            for x in ([0], [0], [0], [7])]
+    if which in ("cos", "sin"):
+        name = "rope_" + which
+        setattr(enc, name, getattr(enc, name).cpu())
+    else:
+        maps[which] = maps[which].cpu()
+    res = torch.randn(7, 384).bfloat16().to("cuda:0")
+    before = res.clone()
+    with pytest.raises(RuntimeError, match="operands must be on"):
+        enc._native_layers(res, *maps)
+    assert torch.equal(res, before)

@@ -589,6 +589,30 @@ def test_ssd_step_refuses(case):
     assert not D.ssd_step_ok(*case)
 
 
+def test_ssd_step_refuses_host_operands():
+    """Each operand whose memory is the host's is an error, not a launch."""
+    g, B, H, N, P, G, QH, KG, Dm, E = gen(1), 3, 4, 64, 128, 4, 2, 1, 8, 8
+    inner, C, qc = H * P, H * P + 2 * G * N, (QH + KG) * Dm + KG * E
+    rope = RopeTable(8, 1e4, DEV)
+    rope.ensure(10)
+    args = [rnd(g, B, qc, dtype=BF).to(DEV), rnd(g, 4, qc).to(DEV),
+            rnd(g, B, 3, qc, dtype=BF).to(DEV), rope.cos, rope.sin, 8,
+            i32(0, 64, 128), rnd(g, 3, KG, 64, Dm, dtype=BF).to(DEV),
+            rnd(g, 3, KG, 64, E, dtype=BF).to(DEV), QH,
+            rnd(g, B, inner + C + H, dtype=BF).to(DEV),
+            rnd(g, 4, C).to(DEV), rnd(g, C).to(DEV),
+            rnd(g, B, 3, C, dtype=BF).to(DEV), rnd(g, H).to(DEV),
+            rnd(g, H).to(DEV), rnd(g, H).to(DEV), rnd(g, B, H, N, P).to(DEV), G,
+            rnd(g, inner).to(DEV), 1e-5,
+            torch.zeros(B, inner, device=DEV, dtype=BF), i32(0, 1, 2),
+            i32(1, 5, 9)]
+    assert torch.isfinite(D.ssd_step(*args)).all()
+    for i, t in enumerate(args):
+        if isinstance(t, torch.Tensor):
+            with pytest.raises(RuntimeError):
+                D.lm_ext().ssd_step(*args[:i], t.cpu(), *args[i + 1:])
+
+
 # ---- the model through the framework ----------------------------------------
 
 @pytest.fixture(scope="module")
