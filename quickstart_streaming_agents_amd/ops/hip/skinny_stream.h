@@ -205,12 +205,14 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
 
   const rsrc rf = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, 0x7fffffff,
                                                     0x00027000);
+  // from nowhere: just beyond what a descriptor covers, whatever the step adds to it
+  constexpr unsigned NOWHERE = 0x80000000u;
   auto load = [&](Group& g, int base) {
     if constexpr (LITTLE)
 #pragma unroll
       for (int j = 0; j < AL; ++j)
         g.few[j] = __builtin_amdgcn_raw_buffer_load_b128(
-              rf, base + am[j] < steps ? ao[j] : 0xffffffffu, base * 128, 0);
+              rf, base + am[j] < steps ? ao[j] : NOWHERE, base * 128, 0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = base + u * WAVES;

@@ -776,6 +776,43 @@ def test_skinny_fp8_steps(M, K):
     close(new, old.double() + h @ W.t())
 
 
+@pytest.mark.parametrize("K", [256, 768, 1280, 4096, 7168])
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 17])
+def test_skinny_fp8_rows_apart(M, K):
+    """A row of NaN or of infinities, and such rows before and behind those given,
+    change no bit of the others: what is read beyond the last step is zero for
+    every row, in all forms."""
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    from quickstart_streaming_agents_amd.ops import ext
+    g = torch.Generator(device="cuda").manual_seed(K + M)
+    N = 128
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16() * 0.05
+    packed = D.pack_weight_fp8(w)
+    ids = torch.arange(M, device="cuda")
+    ones = torch.ones(max(N, K), device="cuda").bfloat16()
+    rows = torch.randn(M + 2, K, generator=g, device="cuda").bfloat16()
+    old = torch.randn(M, N, generator=g, device="cuda").bfloat16()
+
+    def run(bad, value):
+        t = rows.clone()
+        t[0] = t[-1] = float("nan")
+        if value is not None:
+            t[1 + bad] = value
+        x = t[1:-1]
+        out = [ext().skinny_gemm_fp8(x, *packed, N, K)]
+        _, step, ss = D.embed_rows(x.contiguous(), ids, ones[:K])
+        out.append(D.norm_linear_fp8(step, ss, 1, M, 1e-5, packed, N, K))
+        out.append(old.clone())
+        D.linear_residual_fp8(step, packed, N, K, out[-1], ones[:N])
+        return [torch.cat((o[:bad], o[bad + 1:])) for o in out]
+
+    for bad in (0, M - 1):
+        want = run(bad, None)
+        assert all(torch.isfinite(t).all() for t in want)
+        for value in (float("nan"), float("inf")):
+            assert all(map(torch.equal, run(bad, value), want))
+
+
 def test_skinny_gemm_fp8_gpu_pack_matches_cpu_pack():
     """CPU and GPU packs agree in VALUE (the f32->e4m3 cast may round
     ties differently across backends; one e4m3 quantum of slack)."""
