@@ -80,6 +80,16 @@ CONFIGS = {
                                                            1), 64, 1.0, 1.0),
                   par(left(1, 1, 16, 32, 2, 2, 0.5), right(1, 8, 8, 1, 2, 1),
                       72, 1.0, 1.0), scale=1.0),
+    # single tokens in one launch: norm parts that are the groups, columns and
+    # states that its threads divide, two, four and eight rows of state each; an
+    # odd head count
+    "groups": model(160, 128, 40,
+                    par(left(4, 2, 32, 24, 4, 16, 0.2, 500.0, STRETCH),
+                        right(4, 64, 128, 2, 4, 2), 96, 0.7, 0.9),
+                    par(left(2, 1, 20, 36, 2, 8, 0.3),
+                        right(1, 64, 128, 1, 3, 1), 72),
+                    par(left(3, 3, 16, 16, 1, 0, 0.3),
+                        right(2, 128, 128, 1, 1, 1), 80, 1.2, 0.6)),
     # wide heads and states, more query heads per key head than one tile has
     "wide": model(200, 256, 40,
                   par(left(17, 1, 256, 136, 4, 128, 0.05, 1e6),

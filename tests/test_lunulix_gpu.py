@@ -623,6 +623,14 @@ def cases():
 NAMES = pytest.mark.parametrize("name", list(C.CONFIGS))
 
 
+def test_steps_in_one_launch(cases):
+    """Which models' single tokens take the one launch: those of "groups", stored
+    in bf16, in every layer."""
+    for (name, dtype), case in cases.items():
+        whole = [L.mixer.whole for L in case.model.layers]
+        assert all(whole) if (name, dtype) == ("groups", BF) else not any(whole)
+
+
 @BOTH
 @NAMES
 def test_residual_after_every_layer(cases, name, dtype):
@@ -680,17 +688,18 @@ def test_long_prompt_and_long_decoding(cases, dtype):
 @BOTH
 @pytest.mark.parametrize("chunk", [None, 24])
 @pytest.mark.parametrize("graph", [True, False])
-@pytest.mark.parametrize("name", ["odd", "tiles"])
+@pytest.mark.parametrize("name", ["odd", "tiles", "groups"])
 def test_generation(cases, name, chunk, graph, dtype):
     C.scenario_generate(cases[name, dtype], use_graph=graph,
                         chunk_tokens=chunk)
 
 
 @BOTH
-def test_graph_replays_match_eager_steps(cases, dtype):
+@pytest.mark.parametrize("name", ["tiles", "groups"])
+def test_graph_replays_match_eager_steps(cases, name, dtype):
     """Captured decode runs, several in a row with eager work between them,
     against eager decoding of the same prompts."""
-    case = cases["tiles", dtype]
+    case = cases[name, dtype]
     prompts = [case.tokens(n, seed=n) for n in (70, 3, 129)]
     eng = case.engine(1024)
     ref = case.engine(1024)
@@ -707,8 +716,9 @@ def test_graph_replays_match_eager_steps(cases, dtype):
 
 
 @BOTH
-def test_conversations_reuse_the_snapshot(cases, dtype):
-    C.scenario_conversation(cases["tiles", dtype])
+@pytest.mark.parametrize("name", ["tiles", "groups"])
+def test_conversations_reuse_the_snapshot(cases, name, dtype):
+    C.scenario_conversation(cases[name, dtype])
 
 
 def test_preset_on_engine():
