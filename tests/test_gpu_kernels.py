@@ -1010,16 +1010,21 @@ def test_paged_attn_step(ext, B, QH, KVH, D, longest):
         assert torch.equal(_from_step_rows(step, B), out.view(B, -1))
 
 
+# rows that read ahead: more than four, up to 64 with their key heads, none split
+@pytest.mark.parametrize("lens", [
+    [300, 0, 65, 64], [300, 0, 65, 1, 700],
+    [5, 300, 0, 65, 1, 128, 64, 9, 0, 700, 63, 2, 90, 1000, 3, 31],
+    [300, 0, 65, 1, 128, 64, 9, 10, 700, 63, 2, 90, 1000, 3, 31, 33, 17]])
 @pytest.mark.parametrize("sizes", [(16,), (16 * 4097, 40), (1 << 20, 3),
                                    (25 << 20, 16), (9, 7)])
-def test_paged_attn_step_reads_ahead(ext, sizes):
+def test_paged_attn_step_reads_ahead(ext, sizes, lens):
     """What idle blocks read, ends included, changes nothing."""
     g = torch.Generator().manual_seed(len(sizes))
-    lens = [300, 0, 65]
-    kc, vc, bt = _make_paged_kv(3, 4, 64, lens, 8)
-    rot = torch.rand(301, 32, generator=g)
-    qkv = torch.randn(3, 24 * 64, generator=g).bfloat16().to(dev())
-    q, k, v = (t.view(3, -1, 64) for t in qkv.split([1024, 256, 256], 1))
+    B = len(lens)
+    kc, vc, bt = _make_paged_kv(B, 4, 64, lens, sum(-(-n // 64) for n in lens))
+    rot = torch.rand(1001, 32, generator=g)
+    qkv = torch.randn(B, 24 * 64, generator=g).bfloat16().to(dev())
+    q, k, v = (t.view(B, -1, 64) for t in qkv.split([1024, 256, 256], 1))
     warm = [torch.ones(n, dtype=torch.uint8, device=dev()) for n in sizes]
 
     def run(**more):
