@@ -1451,6 +1451,16 @@ def test_short_gemm(ext, M, N, K, glu):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + err + 1e-30).all()
 
 
+@pytest.mark.parametrize("M,N,glu", [(33, 3072, True), (1000, 400, False)])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 11, 12, 24])
+def test_short_gemm_steps(ext, M, N, glu, steps):
+    """The tiles of 32 x 64 with every number of steps behind the last six that
+    are under way together."""
+    assert -(-M // 32) * (N // (32 if glu else 16)) > (128 if glu else 256)
+    assert -(-M // 64) * -(-N // 64) < 128
+    test_short_gemm(ext, M, N, 64 * steps, glu)
+
+
 @pytest.mark.parametrize("M,N,K,glu", [
     (1, 32, 64, False), (32, 384, 1536, False), (40, 96, 1088, False),
     (17, 48, 576, False), (250, 512, 1600, False), (31, 64, 2112, True),
