@@ -93,7 +93,11 @@ __device__ __forceinline__ void qsa_warm(const u32x4_v* at, long long n,
   }
 }
 
-// rotate elements k0.. and k0 + D/2.. of a row held in two fragments
+// Rotate elements k0.. and k0 + D/2.. of a row held in two fragments.  Which product is
+// fused is not left to the compiler, who decides it for each kernel, so that a query has
+// the same bits whether it is turned on its way into the attention or before it: the
+// cosine's, but SIN in the second half of a prompt's keys.
+template <bool SIN = false>
 __device__ __forceinline__ void rotate_pair(bf16x8_a& a, bf16x8_a& b,
                                             const float* c, const float* s) {
   u32x4_v u = __builtin_bit_cast(u32x4_v, a), v = __builtin_bit_cast(u32x4_v, b);
@@ -102,8 +106,9 @@ __device__ __forceinline__ void rotate_pair(bf16x8_a& a, bf16x8_a& b,
     const float2 x = bf16x2_to_f32x2(u[e]), y = bf16x2_to_f32x2(v[e]);
     const float c0 = c[2 * e], c1 = c[2 * e + 1];
     const float s0 = s[2 * e], s1 = s[2 * e + 1];
-    u[e] = cvt_bf16x2(x.x * c0 - y.x * s0, x.y * c1 - y.y * s1);
-    v[e] = cvt_bf16x2(x.x * s0 + y.x * c0, x.y * s1 + y.y * c1);
+    u[e] = cvt_bf16x2(fmaf(x.x, c0, -(y.x * s0)), fmaf(x.y, c1, -(y.y * s1)));
+    v[e] = SIN ? cvt_bf16x2(fmaf(x.x, s0, y.x * c0), fmaf(x.y, s1, y.y * c1))
+               : cvt_bf16x2(fmaf(y.x, c0, x.x * s0), fmaf(y.y, c1, x.y * s1));
   }
   a = __builtin_bit_cast(bf16x8_a, u);
   b = __builtin_bit_cast(bf16x8_a, v);
@@ -815,7 +820,7 @@ qsa_rope_kv_scatter(unsigned short* __restrict__ q,        // [T, QH, D] strided
           *reinterpret_cast<bf16x8_a*>(qp + j * D + D / 2) = y[j];
         }
     }
-    rotate_pair(kx, ky, c, s);
+    rotate_pair<true>(kx, ky, c, s);
     if (slot >= 0) {
       const long long tile =
           ((long long)(slot / QSA_PAGE) * KVH + g) * D * QSA_PAGE;

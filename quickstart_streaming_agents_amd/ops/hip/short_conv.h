@@ -254,9 +254,11 @@ __device__ __forceinline__ void conv_qkv_unit(const ConvQkv& p, int chunk,
     if (turn) {
 #pragma unroll
       for (int i = 0; i < VEC; ++i) {
+        // fused here, not as the compiler likes, so that every form of a step
+        // leaves the same bits
         const float u0 = a[0][i], v0 = a[1][i];
-        a[0][i] = u0 * r.c[i] - v0 * r.s[i];
-        a[1][i] = v0 * r.c[i] + u0 * r.s[i];
+        a[0][i] = fmaf(u0, r.c[i], -(v0 * r.s[i]));
+        a[1][i] = fmaf(u0, r.s[i], v0 * r.c[i]);
       }
     }
     if (!query && r.slot < 0) return;

@@ -255,6 +255,38 @@ def test_conv_chunks_shared_or_whole(taps, dtype):
     assert torch.equal(tails[4], t[4])
 
 
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 6])
+@pytest.mark.parametrize("n", [1, 3, 40, 1500])
+def test_conv_qkv_turns_alike(taps, n):
+    """The rotation's sums to the last bit in every form of a step: a token alone,
+    few and many chunks, any filter.  A filter that passes its token through leaves
+    f32 inputs as they are, and f64 holds a product of two of them whole."""
+    g = gen(taps)
+    H, G, Dm, rot = 2, 1, 24, 16
+    c = (H + G) * Dm + G * Dm
+    x, w = rnd(g, n, c), torch.zeros(taps, c)
+    w[-1] = 1
+    rope = RopeTable(rot, 500.0, DEV)
+    rope.ensure(n)
+    item, t0, off, start, lens, slots = _steps([n], [0])
+    if n == 1:
+        steps = (None, None, None, lens, None, slots)
+    else:
+        steps = (item, t0, off, start, lens, slots)
+    kc = torch.zeros(n // 64 + 1, G, 64, Dm, device=DEV)
+    vc = torch.zeros_like(kc)
+    q = D.conv_qkv(x.to(DEV), w.to(DEV), torch.zeros(5, taps - 1, c, device=DEV),
+                   rope.cos, rope.sin, rot, i32(*range(n)), kc, vc, H, *steps)
+    cos, sin = (t[:n, None].cpu().double() for t in (rope.cos, rope.sin))
+    qk = x[:, :(H + G) * Dm].view(n, H + G, Dm).double()
+    a, b = qk[..., :rot // 2], qk[..., rot // 2:rot]
+    want = torch.cat([a * cos - (b * sin).float().double(),
+                      a * sin + (b * cos).float().double(), qk[..., rot:]], -1)
+    assert torch.equal(q.cpu().view(n, H, Dm), want[:, :H].float())
+    assert torch.equal(kc[:, 0].reshape(-1, Dm)[:n].cpu(), want[:, H].float())
+    assert torch.equal(vc[:, 0].reshape(-1, Dm)[:n].cpu(), x[:, -Dm:])
+
+
 # ---- attention --------------------------------------------------------------
 
 @BOTH
