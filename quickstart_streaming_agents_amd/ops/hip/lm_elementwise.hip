@@ -184,8 +184,9 @@ qsa_residual_norm(float* __restrict__ res, const T* __restrict__ y,
 // is waited for, what is absent (a null pointer) is read from the residual and
 // not used, since a branch would wait for the loads ahead of it, and each sum
 // has its own slots and so one barrier.  Sums and roundings are those of the
-// kernel above.  A 64-row step with 16 of them (2048 wide, shares of K) takes
-// 641 us instead of 652, one row 345 instead of 354.
+// kernel above, which its branches keep from being fused: a row has the same bits
+// among 256 and among 257.  A 64-row step with 16 of them (2048 wide, shares of K)
+// takes 641 us instead of 652, one row 345 instead of 354.
 template <typename T, int VEC, bool LAYER, bool POST, bool SHARES>
 __global__ void __launch_bounds__(1024)
 qsa_residual_norm_once(float* __restrict__ res, const T* __restrict__ y,
@@ -241,6 +242,7 @@ qsa_residual_norm_once(float* __restrict__ res, const T* __restrict__ y,
         1.f / sqrtf(block_sum(ss, scratch[0]) / (float)W + eps);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
+#pragma clang fp contract(off)
       v[j] *= pinv * p[j];
       if (!init) v[j] += r[j];
     }
@@ -284,6 +286,7 @@ qsa_residual_norm_once(float* __restrict__ res, const T* __restrict__ y,
   const float inv = 1.f / sqrtf(ms + eps);
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
+#pragma clang fp contract(off)
     v[j] = (v[j] - mean) * inv * g[j];
     if (b) v[j] += h[j];
   }

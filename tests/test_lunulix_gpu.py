@@ -967,6 +967,30 @@ def test_residual_norm_few_rows_or_many(W, dtype):
             close(got, want[:256].cpu(), dtype)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("W", [4, 260, 1024])
+def test_residual_norm_bits_of_few_or_many(W, dtype):
+    """Widths that one group a thread covers either way: not a bit of a row depends
+    on how many there are."""
+    g, T = gen(W), 257
+    res, y = rnd(g, T, W).to(DEV), rnd(g, T, W, dtype=dtype).to(DEV)
+    w, b, vec, post = (rnd(g, W, dtype=dtype).to(DEV) for _ in range(4))
+    table, ids = rnd(g, 9, W, dtype=dtype).to(DEV), torch.arange(T, device=DEV) % 9
+    for kw in ({}, {"vec": vec}, {"post": post}, {"post": post, "init": True},
+               {"post": post, "vec": vec, "table": table, "tscale": .5}):
+        for layer, weight, bias in ((True, w, b), (True, w, None),
+                                    (False, w, b), (False, w, None),
+                                    (False, None, None)):
+            out = []
+            for n in (T, T - 1):
+                r = res[:n].clone()
+                k = {**kw, "ids": ids[:n]} if "table" in kw else kw
+                out.append((r, D.residual_norm(r, y[:n], weight, bias, 1e-4,
+                                               layer=layer, **k)))
+            (many, a), (few, c) = out
+            assert torch.equal(many[:-1], few) and torch.equal(a[:-1], c)
+
+
 def test_product_in_shares():
     """What is left in shares adds up to the product."""
     g = gen(3)
