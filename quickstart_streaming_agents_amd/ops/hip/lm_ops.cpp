@@ -1034,8 +1034,9 @@ Tensor skinny_gemm(Tensor a, Tensor wf, long N, long K, bool far) {
   TORCH_CHECK(M >= 1 && M <= 32 && a.size(1) == K, "M in [1, 32], K");
   TORCH_CHECK(K % 256 == 0 && N % 16 == 0 && wf.numel() == N * K, "W packing");
   TORCH_CHECK(a.stride(0) % 8 == 0 && aligned(a, 16), "a alignment");
-  // the kernel's offsets are 32 bits
+  // the kernel reads by descriptors: 32-bit offsets of whole 16 bytes
   if (M * a.stride(0) >= 1ll << 30) a = a.clone(at::MemoryFormat::Contiguous);
+  if (!aligned(wf, 16)) wf = wf.clone(at::MemoryFormat::Contiguous);
   auto out = torch::empty({M, (long long)N}, a.options());
   qsa_skinny_gemm_launch(u16(a), u16(wf), u16m(out), M, (int)N, K,
                          a.stride(0), far, cur_stream());

@@ -506,6 +506,18 @@ torch::Tensor pack_weight_frag(torch::Tensor w) {
       .permute({0, 2, 1, 3}).contiguous();
 }
 
+// What the weight streams (skinny_stream.h) read by descriptors of 32-bit offsets, in
+// whole 16 bytes: a copy where a tensor does not start on one, or its rows are not that
+// or too far apart.
+static torch::Tensor whole16(torch::Tensor t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) & 15
+             ? t.clone(at::MemoryFormat::Contiguous) : t;
+}
+static torch::Tensor stream_rows(torch::Tensor a) {
+  return a.stride(0) % 8 || a.size(0) * a.stride(0) >= 1ll << 30
+             ? a.clone(at::MemoryFormat::Contiguous) : whole16(a);
+}
+
 torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor wf, long N, long K) {
   // C[M,N] = a[M,K] @ W^T with W pre-packed by pack_weight_frag.
   CHK_DEV(a); CHK_BF16(a); CHK_BF16(wf); CHK_CONT(wf);
@@ -515,6 +527,8 @@ torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor wf, long N, long K) {
   TORCH_CHECK(a.size(1) == K, "K mismatch");
   TORCH_CHECK(K % 256 == 0 && N % 16 == 0, "K%256==0, N%16==0");
   TORCH_CHECK(wf.numel() == (long long)N * K, "wf size");
+  a = stream_rows(a);
+  wf = whole16(wf);
   auto out = torch::empty({M, (long long)N}, a.options());
   qsa_skinny_gemm_launch(u16(a), u16(wf), u16m(out), M, (int)N, K,
                          a.stride(0), false, cur_stream());
@@ -528,6 +542,8 @@ torch::Tensor skinny_gemm_probe(torch::Tensor a, torch::Tensor wf, long N,
   TORCH_CHECK(M >= 1 && M <= 32 && N % (16 * tiles) == 0 && K % 64 == 0 &&
                   wf.numel() == (long long)N * K && a.size(1) == K,
               "skinny_gemm_probe: shapes");
+  a = stream_rows(a);
+  wf = whole16(wf);
   auto out = torch::empty({M, (long long)N}, a.options());
   TORCH_CHECK(qsa_skinny_gemm_probe_launch(u16(a), u16(wf), u16m(out), M,
                                            (int)N, K, a.stride(0), (int)waves,
@@ -641,10 +657,8 @@ torch::Tensor skinny_gemm_fp8(torch::Tensor a, torch::Tensor qf,
   // C[M,N] = a @ (scale[N] * dequant(Q))^T; Q pre-packed fp8 e4m3 in the
   // fragment-pair-major stream layout (skinny_gemm_fp8.hip header).
   const int M = chk_skinny_fp8(a, qf, scale, N, K);
-  // the kernel's offsets are 32 bits of whole 16 bytes
-  if ((reinterpret_cast<uintptr_t>(a.data_ptr()) & 15) || a.stride(0) % 8 ||
-      a.stride(0) < 0 || M * a.stride(0) >= 1ll << 30)
-    a = a.clone(at::MemoryFormat::Contiguous);
+  a = stream_rows(a);
+  qf = whole16(qf);
   auto out = torch::empty({M, (long long)N}, a.options());
   qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
                              scale.data_ptr<float>(), u16m(out), nullptr, M,
@@ -676,6 +690,8 @@ torch::Tensor skinny_gemm_fp8_norm(torch::Tensor a, torch::Tensor ss,
   TORCH_CHECK(parts >= 1 && ss.numel() == 32 * ((parts + 3) & ~3L),
               "sums of squares [32, parts4]");
   TORCH_CHECK(!glu || N % 64 == 0, "gate and up: N % 64 == 0");
+  a = whole16(a);
+  qf = whole16(qf);
   auto out = glu ? step_rows(M, N / 2, a.options())
                  : torch::empty({(long long)M, (long long)N}, a.options());
   qsa_skinny_gemm_fp8_launch(u16(a), qf.data_ptr<unsigned char>(),
@@ -711,6 +727,8 @@ std::vector<torch::Tensor> skinny_gemm_fp8_residual(
   chk_fp8_weight(qf, scale, N, K);
   CHK_DEV(w); CHK_BF16(w); CHK_CONT(w);
   TORCH_CHECK(w.numel() == N && N % 32 == 0, "norm weight [N], N % 32 == 0");
+  a = whole16(a);
+  qf = whole16(qf);
   auto next = step_rows(M, N, a.options());
   auto ss = torch::empty({32, (skinny_gemm_fp8_parts(M, N, K) + 3) & ~3L},
                          a.options().dtype(at::kFloat));
@@ -757,6 +775,8 @@ torch::Tensor skinny_gemm_fp8_probe(torch::Tensor a, torch::Tensor qf,
   TORCH_CHECK(M >= 1 && M <= 32 && N % (16 * tiles) == 0 &&
                   a.numel() == (pack ? (M <= 16 ? 16 : 32) : M) * (long long)K,
               "skinny_gemm_fp8_probe: shapes");
+  a = whole16(a);
+  qf = whole16(qf);
   auto out = torch::empty({(long long)M, (long long)N}, a.options());
   TORCH_CHECK(qsa_skinny_gemm_fp8_probe_launch(
                   u16(a), qf.data_ptr<unsigned char>(),

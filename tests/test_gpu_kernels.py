@@ -776,6 +776,52 @@ def test_skinny_fp8_steps(M, K):
     close(new, old.double() + h @ W.t())
 
 
+def test_skinny_rows_and_weights_anywhere(ext):
+    """Rows off the 16 bytes that a load takes, an odd number of elements or some
+    2^31 bytes apart, and weights off their 16 bytes, give the bits of a copy."""
+    from quickstart_streaming_agents_amd.ops import dispatch as D
+    from quickstart_streaming_agents_amd.ops import lm_ext
+    M, N, K = 3, 64, 512
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    wf, (qf, scale) = ext.pack_weight_frag(w), D.pack_weight_fp8(w)
+
+    def moved(t, by):
+        flat = t.new_empty(t.numel() + by)[by:]
+        return flat.copy_(t.reshape(-1)).view(t.shape)
+
+    def strided(step):
+        flat = x.new_empty((M - 1) * step + K)
+        return flat.as_strided((M, K), (step, 1)).copy_(x)
+
+    far = 1 << 29
+    rows = [moved(x, 3), strided(K + 5), strided(far)]
+    calls = [(ext.skinny_gemm, (wf,)), (ext.skinny_gemm_fp8, (qf, scale))]
+    for call, (packed, *more) in calls:
+        want = call(x, packed, *more, N, K)
+        for a in rows:
+            assert torch.equal(call(a, packed, *more, N, K), want)
+        assert torch.equal(call(x, moved(packed, 1), *more, N, K), want)
+    want = lm_ext().skinny_gemm(x, wf, N, K, False)
+    for a, b in ((strided(far), wf), (x, moved(wf, 1))):
+        assert torch.equal(lm_ext().skinny_gemm(a, b, N, K, False), want)
+    # rows of a step
+    embed, ids = x, torch.arange(M, device="cuda")
+    ones = torch.ones(K, device="cuda").bfloat16()
+    old = torch.randn(M, N, generator=g, device="cuda").bfloat16()
+    _, step, ss = D.embed_rows(embed, ids, ones)
+
+    def both(step, qf):
+        res = old.clone()
+        D.linear_residual_fp8(step, (qf, scale), N, K, res, ones[:N])
+        return D.norm_linear_fp8(step, ss, 1, M, 1e-5, (qf, scale), N, K), res
+
+    want = both(step, qf)
+    for a, b in ((moved(step, 1), qf), (step, moved(qf, 1))):
+        assert all(map(torch.equal, both(a, b), want))
+
+
 @pytest.mark.parametrize("K", [256, 768, 1280, 4096, 7168])
 @pytest.mark.parametrize("M", [2, 3, 4, 5, 17])
 def test_skinny_fp8_rows_apart(M, K):
