@@ -306,8 +306,14 @@ static void residual_norm_go(float* res, const void* y, long long ystride,
   const int most = rows <= 256 ? 1024 : 256;
   threads = threads > most ? most : threads;
   auto kernel = qsa_residual_norm<T, VEC, LAYER, POST, SHARES>;
-  // up to 256 rows a CU has one block at most and nothing hides its waits; with
-  // more the other blocks do, and reading what is absent would be extra traffic
+  // Up to 256 rows a CU has one block at most and nothing hides its waits; with
+  // more the other blocks do, and reading what is absent would be extra traffic.
+  // us, above / so: steps of four layers 4096 wide, one row 450 / 446, 16 524 / 515,
+  // 128 947 / 938, 200 1247 / 1225 (Lunulix), 336 / 333, 382 / 374, 665 / 655, 859 /
+  // 850 (Luzalorn).  Launches alone, all of their operands in L2: layer norms of 1024 to
+  // 4096 columns 2.8 to 5.8 / 2.3 to 4.9 for 1 to 256 rows, rms norms with a post norm
+  // 3.0 to 5.6 / 2.4 to 5.0, those of shares 6.6 / 6.4 for 256 rows of 4096, but 3.3 /
+  // 3.5 for one, whose absent operands are loads that no wait hides.
   if constexpr (VEC == 4) {
     if (rows <= 256 && W <= most * VEC)
       kernel = qsa_residual_norm_once<T, VEC, LAYER, POST, SHARES>;

@@ -1363,8 +1363,10 @@ struct EncoderProduct {
 // there is no result and nothing has changed.  Up to some 2000 rows a call is as long as
 // the host takes for its launches: 84 calls from Python at 5 us each, products planned
 // each time; here they are planned once, and operands lie in the same places in every
-// layer (texts embedded in one call, us: one of 15 tokens 543 -> 400, 8 of some 50 584 ->
-// 503, from some 1000 tokens on level).
+// layer (texts embedded in one call, us: one of 15 tokens 520 -> 393, 8 of some 50 574 ->
+// 503, from some 1000 tokens on level).  The price is that nothing takes another's place
+// meanwhile: beside res 2 H + 4 A + F numbers of 16 bits a row, and the largest shares,
+// 9 KB a row for the widths of EncoderConfig.
 OptTensor encoder_layers(Tensor res, std::vector<Tensor> weights, Tensor final_norm,
                          Tensor cos_t, Tensor sin_t, Tensor qb_item, Tensor qb_t0,
                          Tensor off, Tensor len, int64_t heads, double scale,
