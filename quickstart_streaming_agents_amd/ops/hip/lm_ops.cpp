@@ -65,9 +65,9 @@ extern "C" void qsa_glu_launch(const void*, const float*, int, const void*,
     const long long*,
     void*, long long, long long, long long, long long, long long, int, int,
     int, hipStream_t);
-extern "C" void qsa_conv_qkv_launch(ConvQkv, int, int, int, hipStream_t);
+extern "C" void qsa_conv_qkv_launch(ConvQkv, long long, int, int, int, hipStream_t);
 extern "C" void qsa_conv_silu_launch(const void*, long long, const float*,
-    const float*, int, void*, ConvStep, int, void*, int, int, int,
+    const float*, int, void*, ConvStep, long long, int, void*, int, int, int,
     hipStream_t);
 extern "C" void qsa_gqa_rows_launch(const void*, const void*, const void*,
     const int*, int, const int*, const int*, const float*, const void*,
@@ -660,7 +660,7 @@ Tensor conv_qkv(Tensor x, Tensor w, Tensor tails, Tensor cos_t, Tensor sin_t,
   if (x.size(0) == 0) return q;
   const int chunks = conv_step(p.step, item, t0, off, start, len, slots,
                                x.size(0));
-  qsa_conv_qkv_launch(p, chunks, is_f32(x), v4, cur_stream());
+  qsa_conv_qkv_launch(p, x.size(0), chunks, is_f32(x), v4, cur_stream());
   return q;
 }
 
@@ -680,8 +680,8 @@ Tensor conv_silu(Tensor x, Tensor w, Tensor bias, Tensor tails,
                  aligned(x, is_f32(x) ? 16 : 8);
   qsa_conv_silu_launch(x.data_ptr(), x.stride(0), w.data_ptr<float>(),
                        bias.data_ptr<float>(), (int)w.size(0),
-                       tails.data_ptr(), st, chunks, out.data_ptr(), (int)C,
-                       is_f32(x), v4, cur_stream());
+                       tails.data_ptr(), st, x.size(0), chunks,
+                       out.data_ptr(), (int)C, is_f32(x), v4, cur_stream());
   return out;
 }
 

@@ -37,15 +37,28 @@ __device__ __forceinline__ ConvSpan conv_span(const ConvStep& st, int c,
 
 // NP (1 or 2) groups of VEC channels, c0.. and c1..; TAPS 0: `taps` of them,
 // through memory.  pre(t) loads what emit(t, values, .) wants besides.
-template <typename T, int TAPS, int VEC, int NP, typename Pre, typename Emit>
+// SINGLE: tokens one by one, which takes fewer registers (conv_single, short_conv.hip).
+template <typename T, int TAPS, int VEC, int NP, bool SINGLE, typename Pre,
+          typename Emit>
 __device__ __forceinline__ void conv_rows(
     const T* x, long long xstride, T* tail, int C, int c0, int c1,
     const float* w, const float* bias, int taps, const ConvSpan& s, Pre pre,
     Emit emit) {
   const int NT = (TAPS ? TAPS : taps) - 1;
   auto ch = [&](int p) { return p == 0 ? c0 : c1; };
-  // chosen by address: a branch for each would wait for each
+  // few blocks: chosen by address, as a branch for each would wait for each
   auto load = [&](int t, int p, float* v) {
+    if constexpr (SINGLE) {
+      if (t >= 0) {
+        ldv<T, VEC>(x + (long long)(s.r0 + t) * xstride + ch(p), v);
+      } else if (s.p0 + t >= 0) {
+        ldv<T, VEC>((const T*)tail + (long long)(NT + t) * C + ch(p), v);
+      } else {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) v[i] = 0.f;
+      }
+      return;
+    }
     const T* at = t >= 0 ? x + (long long)(s.r0 + t) * xstride
                          : (const T*)tail + (long long)(NT + t) * C;
     ldv<T, VEC>(at + ch(p), v);
@@ -80,6 +93,23 @@ __device__ __forceinline__ void conv_rows(
     // token waited for memory by itself.  4096 channels with four taps, to pages / with
     // silu, us: 60 tokens 15.2 / 10.8 -> 9.9 / 7.7, 7500 35.4 / 40.0 -> 36.9 / 32.7 (to
     // pages two and four tokens ahead were 13.2 and 10.6, 48 and 40).
+    auto step = [&](int t, const float (&u)[NP][VEC], const auto& aux) {
+      float a[NP][VEC];
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+          a[p][i] = b[p][i];
+#pragma unroll
+          for (int k = 0; k < TAPS - 1; ++k)
+            a[p][i] = fmaf(wt[p][k][i], win[p][k][i], a[p][i]);
+          a[p][i] = fmaf(wt[p][TAPS - 1][i], u[p][i], a[p][i]);
+#pragma unroll
+          for (int k = 0; k + 2 < TAPS; ++k) win[p][k][i] = win[p][k + 1][i];
+          win[p][K - 1][i] = u[p][i];
+        }
+      emit(t, a, aux);
+    };
     auto walk = [&](auto ahead) {
       constexpr int AHEAD = ahead.value;
       for (int t0 = s.t0; t0 < s.t1; t0 += AHEAD) {
@@ -96,25 +126,21 @@ __device__ __forceinline__ void conv_rows(
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
           if (t0 + j >= s.t1) break;              // uniform over the block
-          float a[NP][VEC];
-#pragma unroll
-          for (int p = 0; p < NP; ++p)
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) {
-              a[p][i] = b[p][i];
-#pragma unroll
-              for (int k = 0; k < TAPS - 1; ++k)
-                a[p][i] = fmaf(wt[p][k][i], win[p][k][i], a[p][i]);
-              a[p][i] = fmaf(wt[p][TAPS - 1][i], u[j][p][i], a[p][i]);
-#pragma unroll
-              for (int k = 0; k + 2 < TAPS; ++k) win[p][k][i] = win[p][k + 1][i];
-              win[p][K - 1][i] = u[j][p][i];
-            }
-          emit(t0 + j, a, aux[j]);
+          step(t0 + j, u[j], aux[j]);
         }
       }
     };
-    if (s.t1 - s.t0 == 1) walk(std::integral_constant<int, 1>{});
+    if constexpr (SINGLE) {
+#pragma unroll 4
+      for (int t = s.t0; t < s.t1; ++t) {
+        const auto aux = pre(t);
+        float u[NP][VEC];
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+          ldv<T, VEC>(x + (long long)(s.r0 + t) * xstride + ch(p), u[p]);
+        step(t, u, aux);
+      }
+    } else if (s.t1 - s.t0 == 1) walk(std::integral_constant<int, 1>{});
     else if (s.t1 - s.t0 <= CONV_ROWS / CONV_PARTS)
       walk(std::integral_constant<int, CONV_ROWS / CONV_PARTS>{});
     else walk(std::integral_constant<int, NP == 1 && sizeof(T) == 2 ? 16 : 8>{});
@@ -167,8 +193,8 @@ __device__ __forceinline__ void conv_rows(
 }
 
 #define CONV_CASE(T, TAPS, VEC, NP)                                          \
-  conv_rows<T, TAPS, VEC, NP>(x, xstride, tail, C, c0, c1, w, bias, taps, s, \
-                              pre, emit)
+  conv_rows<T, TAPS, VEC, NP, SINGLE>(x, xstride, tail, C, c0, c1, w, bias,  \
+                                      taps, s, pre, emit)
 #define CONV_DISPATCH(T, VEC, NP)              \
   switch (taps) {                              \
     case 1: CONV_CASE(T, 1, VEC, NP); break;   \
@@ -196,7 +222,7 @@ __host__ __device__ inline int conv_qkv_units(const ConvQkv& p, int vec) {
 
 // ONE: the step has one token per row and filters of up to CONV_ONE_TAPS taps
 #define CONV_ONE_TAPS 4
-template <typename T, int VEC, bool ONE = false>
+template <typename T, int VEC, bool ONE = false, bool SINGLE = false>
 __device__ __forceinline__ void conv_qkv_unit(const ConvQkv& p, int chunk,
                                               int u, int part = 0,
                                               int parts = 1) {

@@ -255,6 +255,44 @@ def test_conv_chunks_shared_or_whole(taps, dtype):
     assert torch.equal(tails[4], t[4])
 
 
+@BOTH
+@pytest.mark.parametrize("taps", [1, 3, 4, 6])
+def test_conv_one_by_one_or_ahead(taps, dtype):
+    """More waves than the chip holds take their tokens one by one, a part of them
+    several ahead, and so do portions of three and of four: not a bit differs."""
+    g = gen(taps)
+    H, G, Dm, rot, n = 40, 8, 24, 8, 8300
+    c = (H + 2 * G) * Dm
+    x, w, b = rnd(g, n, c, dtype=dtype).to(DEV), rnd(g, taps, c).to(DEV), \
+        rnd(g, c).to(DEV)
+    rope = RopeTable(rot, 500.0, DEV)
+    rope.ensure(n)
+    pages = torch.arange(n, dtype=torch.int32, device=DEV)
+
+    def run(cuts):
+        tails = [torch.zeros(5, taps - 1, c, dtype=dtype, device=DEV)
+                 for _ in range(2)]
+        kc = torch.zeros(n // 64 + 1, G, 64, Dm, dtype=dtype, device=DEV)
+        vc, out, at = torch.zeros_like(kc), [], 0
+        for m in cuts:
+            item, t0, off, start, lens, slots = _steps([m], [at])
+            steps = item, t0, off, start, lens, slots
+            rows = slice(at, at + m)
+            out.append(torch.cat([
+                D.conv_qkv(x[rows], w, tails[0], rope.cos, rope.sin, rot,
+                           pages[rows], kc, vc, H, *steps),
+                D.conv_silu(x[rows], w, b, tails[1], *steps)], 1))
+            at += m
+        assert at == n
+        return [torch.cat(out), kc, vc, *tails]
+
+    # 168 threads' worth of channels: four waves for each 16 tokens
+    assert n / 16 * 4 > 2048 > n / 32 * 4
+    whole = run([n])
+    for cuts in ([n // 2, n // 2], [n // 2 - 7, 3, 4, n // 2]):
+        assert all(map(torch.equal, run(cuts), whole))
+
+
 @pytest.mark.parametrize("taps", [1, 2, 3, 4, 6])
 @pytest.mark.parametrize("n", [1, 3, 40, 1500])
 def test_conv_qkv_turns_alike(taps, n):
