@@ -26,8 +26,9 @@ struct ShortArgs {
   long long lda;
 };
 
-// 4 waves as 2 x 2; a wave has MT x NT tiles of 16 x 16
-template <int MT, int NT, bool GLU>
+// 4 waves as 2 x 2; a wave has MT x NT tiles of 16 x 16; PF steps of K are in registers
+// or under way besides the two in LDS
+template <int MT, int NT, int PF, bool GLU>
 __global__ void __launch_bounds__(256, 2)
 qsa_short_gemm(ShortArgs p) {
   constexpr int BM = 32 * MT, BN = 32 * NT;
@@ -74,8 +75,6 @@ qsa_short_gemm(ShortArgs p) {
     return (((row >> 4) * 2 + half) * 64 + h * 16 +
             ((row & 15) ^ (h << 1 | half << 3))) * 8;
   };
-  // PF steps of K are in registers or under way besides the two in LDS
-  constexpr int PF = MT == 1 ? 6 : 1;  // (384 x 1536 of 15 rows 7.2 -> 6.2 us)
   u32x4_v ar[PF][AL], br[PF][BL];
   const int steps = p.K >> 6;
   auto load = [&](int q, int step) {   // beyond the end: the last one again
@@ -257,16 +256,16 @@ static void few_go(const ShortArgs& p, int glu, hipStream_t st) {
     hipLaunchKernelGGL((qsa_few_gemm<U, false>), grid, dim3(512), 0, st, p);
 }
 
-template <int MT, int NT>
+template <int MT, int NT, int PF = 1>
 static void short_go(ShortArgs p, int glu, hipStream_t st) {
   p.NB = (p.N + 32 * NT - 1) / (32 * NT);
   const int mb = (p.M + 32 * MT - 1) / (32 * MT);
   const dim3 grid((unsigned)((mb < 8 ? mb : (mb + 7) / 8 * 8) * p.NB));
   if (glu)
-    hipLaunchKernelGGL((qsa_short_gemm<MT, NT, true>), grid, dim3(256), 0, st,
+    hipLaunchKernelGGL((qsa_short_gemm<MT, NT, PF, true>), grid, dim3(256), 0, st,
                        p);
   else
-    hipLaunchKernelGGL((qsa_short_gemm<MT, NT, false>), grid, dim3(256), 0, st,
+    hipLaunchKernelGGL((qsa_short_gemm<MT, NT, PF, false>), grid, dim3(256), 0, st,
                        p);
 }
 
@@ -290,7 +289,11 @@ extern "C" bool qsa_short_gemm_takes(long long M, long long N, long long K) {
 // Tiles of 128 x 128 once two rounds of blocks are left, 64 x 64 while they
 // make half a round, 32 x 64 below (384 x 512 at 400 rows: 8.2 / 4.5 / 3.7 us;
 // 1536 x 384 at 1600: 7.9 / 6.8 / 8.0, at 8800: 20.9 / 23.0 / 28.4; 3072 x 384
-// with the activation at 16,000: 58 with 128 x 128, 94 with 32 x 64).
+// with the activation at 16,000: 58 with 128 x 128, 94 with 32 x 64).  Six steps of K
+// ahead pay where K is long (384 x 1536 of 15 rows 7.2 -> 6.2 us); a few are over by
+// then, and as many more are read in vain (one ahead / six: 1536 x 384 at 130 and 320
+// rows 3.57 / 3.69, 4.41 / 5.02, 3072 x 384 gated at 100 3.76 / 3.94, 384 x 128 at 600
+// 2.76 / 3.10; K 512 level).
 extern "C" void qsa_short_gemm_launch(const bf16_t* A, const bf16_t* W,
                                       bf16_t* C, int M, int N, int K,
                                       long long lda, int glu,
@@ -306,5 +309,6 @@ extern "C" void qsa_short_gemm_launch(const bf16_t* A, const bf16_t* W,
   }
   if (blocks(128) >= 512) short_go<4, 4>(p, glu, st);
   else if (blocks(64) >= 128) short_go<2, 2>(p, glu, st);
-  else short_go<1, 2>(p, glu, st);
+  else if (K <= 512) short_go<1, 2>(p, glu, st);
+  else short_go<1, 2, 6>(p, glu, st);
 }

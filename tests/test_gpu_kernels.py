@@ -1493,10 +1493,10 @@ def test_short_gemm(ext, M, N, K, glu):
 
 
 @pytest.mark.parametrize("M,N,glu", [(33, 3072, True), (1000, 400, False)])
-@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 11, 12, 24])
+@pytest.mark.parametrize("steps", [1, 2, 3, 7, 8, 9, 10, 11, 12, 13, 14, 24])
 def test_short_gemm_steps(ext, M, N, glu, steps):
-    """The tiles of 32 x 64 with every number of steps behind the last six that
-    are under way together."""
+    """The tiles of 32 x 64, up to eight steps with one ahead, beyond with every
+    number of them behind the last six that are under way together."""
     assert -(-M // 32) * (N // (32 if glu else 16)) > (128 if glu else 256)
     assert -(-M // 64) * -(-N // 64) < 128
     test_short_gemm(ext, M, N, 64 * steps, glu)
