@@ -286,13 +286,8 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
   load(g0, wave);
   load(g1, wave + ROUND);
   if constexpr (NORM) {
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
+    auto factor = [&](int i) {
       const int row = wave + i * WAVES;
-      // Rows that do not exist cost a wave 86 instructions each before its first
-      // product (16 layers of width 2048, a step of one row 509 -> 494 us; 8 layers, 4
-      // rows 293 -> 281).
-      if (row >= p.M) break;                      // uniform over the wave
       float s = 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) s += lane * 4 + e < p.parts ? sv[i][e] : 0.f;
@@ -300,6 +295,22 @@ __device__ __forceinline__ void skinny_stream(const SkinnyArgs& p) {
         s += p.ss_in[row * p4 + k];
       s = wave_reduce_sum(s);
       if (lane == 0) inv_s[row] = rsqrtf(s / (float)p.K + p.eps);
+    };
+    // Rows that do not exist cost a wave 86 instructions each before its first
+    // product (16 layers of width 2048, a step of one row 509 -> 494 us; 8 layers, 4
+    // rows 293 -> 281).  Where all 16 do, the chains of a wave's rows lie beside each
+    // other, without a look at each (us, looks / none: 16 rows of 2048 x 2048 3.93 /
+    // 3.61, of 1024 x 768 3.79 / 3.58, of 512 x 256 3.72 / 3.56, 28,672 x 4096 gated
+    // 23.7 / 23.3; of two tiles 32 rows of 16,384 x 2048 gated 7.9 / 8.3).
+    if (MT == 1 && p.M == 16) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) factor(i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        if (wave + i * WAVES >= p.M) break;       // uniform over the wave
+        factor(i);
+      }
     }
   }
   // both groups are always loaded again, so that the waits in the loop are for one
