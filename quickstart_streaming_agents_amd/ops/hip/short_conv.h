@@ -88,11 +88,6 @@ __device__ __forceinline__ void conv_rows(
       for (int j = 0; j < TAPS - 1; ++j)
         load(s.t0 - (TAPS - 1) + j, p, win[p][j]);
     }
-    // All loads of AHEAD tokens go out before the first of them is used: a store may
-    // write what a later load reads, as far as the compiler knows, so in one loop each
-    // token waited for memory by itself.  4096 channels with four taps, to pages / with
-    // silu, us: 60 tokens 15.2 / 10.8 -> 9.9 / 7.7, 7500 35.4 / 40.0 -> 36.9 / 32.7 (to
-    // pages two and four tokens ahead were 13.2 and 10.6, 48 and 40).
     auto step = [&](int t, const float (&u)[NP][VEC], const auto& aux) {
       float a[NP][VEC];
 #pragma unroll
@@ -110,6 +105,11 @@ __device__ __forceinline__ void conv_rows(
         }
       emit(t, a, aux);
     };
+    // All loads of AHEAD tokens go out before the first of them is used: a store may
+    // write what a later load reads, as far as the compiler knows, so in one loop each
+    // token waited for memory by itself.  4096 channels with four taps, to pages / with
+    // silu, us: 60 tokens 15.2 / 10.8 -> 9.9 / 7.7 (to pages two and four tokens ahead
+    // were 13.2 and 10.6), 7500 with silu 40.2 -> 33.8.
     auto walk = [&](auto ahead) {
       constexpr int AHEAD = ahead.value;
       for (int t0 = s.t0; t0 < s.t1; t0 += AHEAD) {
